@@ -226,7 +226,8 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
 // exactness   q, k, v are bf16 already.  What enters the state (the weighted values) meets k as three bf16 terms, 24 bits: the state's sums are
 //             those of fp32 operands at the rate of bf16 matrix instructions.  What is read out of it for the output (S, the weights of
 //             the keys) meets q and v as two terms, 16 bits.  n is carried in fp32, each wave half of it.
-// loads       k of a chunk is requested at its head, q and v of the next one as soon as both waves have read this one's.
+// loads       k of a chunk is requested at its head, once both waves are through with the last one's, q and v of the next one as soon as
+//             both waves have read this one's.
 // operands    an accumulator tile of v_mfma_f32_32x32x16_bf16 (lane = column, registers = rows 8 (v / 4) + 4 (lane / 32) + v % 4) is, as it
 //             lies, an operand of the next product over those rows when the other operand takes its sixteen k in the same order:
 //               scores^T = K Q^T        lane = query, registers = keys   -> left operand of   P V     (V out of LDS transposed)
@@ -424,6 +425,10 @@ __global__ __launch_bounds__( 128, 1 ) void mlstm_chunk_kernel( float* __restric
   for ( uint32_t t0 = 0; t0 < st.n_tokens; t0 += CHUNK ) {
     const uint32_t rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
     const __bf16* first = in.main.data + ( row_first + t0 ) * in.main.stride;
+    if ( t0 > 0 ) {
+      // k of the last chunk is read up to its end, by both waves in whole: neither may have its half replaced before the other is through
+      asm volatile( "s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory" );
+    }
     fetch( s_k, first + in.col.k + h * s.dim, rows, s.dim / 8, swizzle_row, std::integral_constant<uint32_t, RB> {} );
     if ( t0 == 0 ) {
       fetch_qv( 0 );

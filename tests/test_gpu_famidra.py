@@ -398,6 +398,31 @@ def test_mlstm_extreme_gates(dtype):
             at += c
 
 
+@pytest.mark.parametrize("d,dv,T", [(64, 64, 320), (128, 192, 257), (256, 512, 512)])
+def test_mlstm_same_bits_twice(d, dv, T):
+    """The chunks of a prompt share their LDS tiles: with enough work-groups for the waves of one to drift apart, the same inputs give the
+    same bits, outputs and state."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    H, width, batch = 8, 64, 8
+    m = GhMlstm(H, d, dv, 15.0, 1e-5)
+    rows, _ = ops.mlstm_weight_rows(m)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, w = (torch.randn(n, width, generator=gen, device="cuda").to(torch.bfloat16) for n in (batch * T, rows))
+    w *= width ** -0.5
+    zeros, ones = torch.zeros(H, dtype=torch.bfloat16, device="cuda"), torch.ones(H * dv, dtype=torch.bfloat16, device="cuda")
+    start = torch.zeros(batch, dtype=torch.int32, device="cuda")
+    first = None
+    for _ in range(4):
+        state = torch.zeros((batch, ops.mlstm_state_bytes(m) // 4), device="cuda")
+        table = ops.row_table([state[i].data_ptr() for i in range(batch)])
+        out = ops.mlstm_forward(x, w, m, zeros, zeros, ones, table, start, T)
+        got = (out.cpu(), state.cpu())
+        first = first or got
+        assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1])
+
+
 # ---- whole models ---------------------------------------------------------------------------------
 @pytest.fixture(scope="module")
 def models(tmp_path_factory):
