@@ -9,7 +9,7 @@
 // contiguous elements at row + h*head_size, the V head at row + kv_dim + h*head_size.
 //
 // Three kernels produce the same partial format:
-//   generic  any head_size <= 256, any gqa, f16/f32 storage; one wave per (context, query head, split)
+//   generic  any head_size <= 256, any gqa, f16/f32 storage; one work-group per (context, query head, split)
 //   valu     f16, head_size 128: one wave per (context, kv head, split); 16 lanes share a token's
 //            256-byte head row (one 16-byte load per lane), dot products with v_dot2_f32_f16,
 //            16-lane DPP reductions, four independent online-softmax streams per wave
@@ -49,28 +49,38 @@ struct Partials
 
 // =================================================================================================
 // generic kernel
+//
+// Work-group = (query head, split, context), its W waves take the split's keys in turns of U and add their parts up in LDS.  Bound by
+// latency, not by bytes: a wave's lanes are the dims of a key, so a key is one short load and one reduction over the wave, and what
+// counts is how many are under way at once.  A turn requests U keys and values before the first use and its U reductions overlap.
+// Whole 15M model, 4 contexts of up to 256 keys (24 work-groups): 90 us a layer with one wave that walked key by key, 7 with 16 waves.
+// NK: 64-lane pieces of a head (head_size <= 64 NK)
 // =================================================================================================
-template<typename T>
-__global__ __launch_bounds__( 64 ) void attn_decode_generic_kernel( const T* __restrict__ q,
-                                                                    const T* const* __restrict__ layer_rows,
-                                                                    const uint32_t* __restrict__ pos,
-                                                                    Partials part,
-                                                                    T* __restrict__ xb,
-                                                                    uint32_t n_kv_heads,
-                                                                    uint32_t gqa,
-                                                                    uint32_t head_size,
-                                                                    uint32_t chunk,
-                                                                    uint32_t max_splits,
-                                                                    float scale_log2e )
+template<typename T, int NK, int W>
+__global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T* __restrict__ q,
+                                                                       const T* const* __restrict__ layer_rows,
+                                                                       const uint32_t* __restrict__ pos,
+                                                                       Partials part,
+                                                                       T* __restrict__ xb,
+                                                                       uint32_t n_kv_heads,
+                                                                       uint32_t gqa,
+                                                                       uint32_t head_size,
+                                                                       uint32_t chunk,
+                                                                       uint32_t max_splits,
+                                                                       float scale_log2e )
 {
+  constexpr int U = 8 / NK; // keys per turn
+  __shared__ float s_out[W][NK * 64];
+  __shared__ float s_m[W], s_l[W];
   const uint32_t head = blockIdx.x;
   const uint32_t split = blockIdx.y;
   const uint32_t ctx = blockIdx.z;
   const T* base = layer_rows[ctx];
+  const uint32_t last = pos[ctx]; // read before the branch on `base`: one round trip for the two
   if ( base == nullptr ) {
     return;
   }
-  const uint32_t n_tok = min( pos[ctx] + 1, max_splits * chunk ); // never beyond what the host sized the grid and the partials for
+  const uint32_t n_tok = min( last + 1, max_splits * chunk ); // never beyond what the host sized the grid and the partials for
   const uint32_t t_begin = split * chunk;
   if ( t_begin >= n_tok ) {
     return;
@@ -78,53 +88,107 @@ __global__ __launch_bounds__( 64 ) void attn_decode_generic_kernel( const T* __r
   const uint32_t t_end = min( n_tok, t_begin + chunk );
   const uint32_t n_heads = n_kv_heads * gqa;
   const uint32_t h = head / gqa;
-  const uint32_t lane = threadIdx.x;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint64_t row_elems = 2ull * n_kv_heads * head_size;
 
-  float qd[4], acc[4];
+  float qd[NK], acc[NK];
+  uint32_t dim[NK]; // a lane past the head reads its last element against a query of zero and stores nothing
   const T* qh = q + ( (uint64_t)ctx * n_heads + head ) * head_size;
 #pragma unroll
-  for ( int k = 0; k < 4; k++ ) {
+  for ( int k = 0; k < NK; k++ ) {
     const uint32_t d = lane + 64 * k;
-    qd[k] = d < head_size ? to_f32( qh[d] ) : 0.0f;
+    dim[k] = min( d, head_size - 1 );
+    qd[k] = d < head_size ? to_f32( qh[dim[k]] ) : 0.0f;
     acc[k] = 0.0f;
   }
   float m = -INFINITY, l = 0.0f;
   const T* kbase = base + (uint64_t)h * head_size;
   const T* vbase = kbase + (uint64_t)n_kv_heads * head_size;
 
-  for ( uint32_t t = t_begin; t < t_end; t++ ) {
-    const T* kr = kbase + (uint64_t)t * row_elems;
-    const T* vr = vbase + (uint64_t)t * row_elems;
-    float partial = 0.0f;
-    float vd[4];
+  for ( uint32_t t0 = t_begin + wave * U; t0 < t_end; t0 += W * U ) {
+    T kd[U][NK], vd[U][NK];
 #pragma unroll
-    for ( int k = 0; k < 4; k++ ) {
-      const uint32_t d = lane + 64 * k;
-      if ( d < head_size ) {
-        partial += to_f32( kr[d] ) * qd[k];
-        vd[k] = to_f32( vr[d] );
-      } else {
-        vd[k] = 0.0f;
+    for ( int u = 0; u < U; u++ ) {
+      const uint64_t at = (uint64_t)min( t0 + u, t_end - 1 ) * row_elems; // a key past the end repeats the last one and is not counted
+#pragma unroll
+      for ( int k = 0; k < NK; k++ ) {
+        kd[u][k] = kbase[at + dim[k]];
+        vd[u][k] = vbase[at + dim[k]];
       }
     }
-    const float s = wave_sum( partial ) * scale_log2e;
-    const float m_new = fmaxf( m, s );
-    const float alpha = fast_exp2( m - m_new );
-    const float p = fast_exp2( s - m_new );
-    l = l * alpha + p;
+    float s[U];
+    float m_new = m;
 #pragma unroll
-    for ( int k = 0; k < 4; k++ ) {
-      acc[k] = acc[k] * alpha + p * vd[k];
+    for ( int u = 0; u < U; u++ ) {
+      float partial = 0.0f;
+#pragma unroll
+      for ( int k = 0; k < NK; k++ ) {
+        partial += ( lane + 64 * k < head_size ? to_f32( kd[u][k] ) : 0.0f ) * qd[k];
+      }
+      s[u] = wave_sum( partial ) * scale_log2e;
+      m_new = t0 + u < t_end ? fmaxf( m_new, s[u] ) : m_new;
+    }
+    const float alpha = fast_exp2( m - m_new );
+    l *= alpha;
+#pragma unroll
+    for ( int k = 0; k < NK; k++ ) {
+      acc[k] *= alpha;
+    }
+#pragma unroll
+    for ( int u = 0; u < U; u++ ) {
+      if ( t0 + u < t_end ) { // uniform
+        const float p = fast_exp2( s[u] - m_new );
+        l += p;
+#pragma unroll
+        for ( int k = 0; k < NK; k++ ) {
+          acc[k] += p * to_f32( vd[u][k] );
+        }
+      }
     }
     m = m_new;
+  }
+
+  if constexpr ( W > 1 ) {
+#pragma unroll
+    for ( int k = 0; k < NK; k++ ) {
+      s_out[wave][lane + 64 * k] = acc[k];
+    }
+    if ( lane == 0 ) {
+      s_m[wave] = m;
+      s_l[wave] = l;
+    }
+    __syncthreads();
+    if ( wave != 0 ) {
+      return;
+    }
+    float m_all = m; // wave 0 always has a key
+#pragma unroll
+    for ( int w = 1; w < W; w++ ) {
+      m_all = fmaxf( m_all, s_m[w] );
+    }
+    l = 0.0f;
+#pragma unroll
+    for ( int k = 0; k < NK; k++ ) {
+      acc[k] = 0.0f;
+    }
+    for ( int w = 0; w < W; w++ ) {
+      if ( t_begin + w * U < t_end ) { // uniform; a wave without keys adds nothing
+        const float f = fast_exp2( s_m[w] - m_all );
+        l += s_l[w] * f;
+#pragma unroll
+        for ( int k = 0; k < NK; k++ ) {
+          acc[k] += s_out[w][lane + 64 * k] * f;
+        }
+      }
+    }
+    m = m_all;
   }
 
   if ( max_splits == 1 ) {
     const float inv = 1.0f / l;
     T* o = xb + ( (uint64_t)ctx * n_heads + head ) * head_size;
 #pragma unroll
-    for ( int k = 0; k < 4; k++ ) {
+    for ( int k = 0; k < NK; k++ ) {
       const uint32_t d = lane + 64 * k;
       if ( d < head_size ) {
         o[d] = from_f32<T>( acc[k] * inv );
@@ -134,7 +198,7 @@ __global__ __launch_bounds__( 64 ) void attn_decode_generic_kernel( const T* __r
     const uint64_t slot = ( (uint64_t)ctx * n_heads + head ) * max_splits + split;
     float* o = part.out + slot * head_size;
 #pragma unroll
-    for ( int k = 0; k < 4; k++ ) {
+    for ( int k = 0; k < NK; k++ ) {
       const uint32_t d = lane + 64 * k;
       if ( d < head_size ) {
         o[d] = acc[k];
@@ -1259,6 +1323,43 @@ uint64_t partial_floats( uint64_t batch, const gh_shape* s, uint32_t max_splits 
   return batch * s->n_heads * (uint64_t)max_splits * ( s->head_size + 2ull );
 }
 
+// Waves per work-group of the generic kernel: as many as find keys, 16 while that leaves no CU with a second work-group to wait for, 4
+// beyond (long contexts of many heads: the waves of four work-groups on a CU cover each other's latency).
+template<typename T, int NK, int W>
+void launch_generic_waves( hipStream_t st, const void* q, const void* const* layer_rows_dev, const uint32_t* pos_dev, Partials part, void* xb, uint64_t batch,
+                           const gh_shape* s, const Plan& plan, float scale )
+{
+  attn_decode_generic_kernel<T, NK, W><<<dim3( s->n_heads, plan.max_splits, (unsigned)batch ), 64 * W, 0, st>>>(
+    static_cast<const T*>( q ), reinterpret_cast<const T* const*>( layer_rows_dev ), pos_dev, part, static_cast<T*>( xb ), s->n_kv_heads, s->gqa_size, s->head_size,
+    plan.chunk, plan.max_splits, scale );
+}
+template<typename T, int NK>
+void launch_generic_head( hipStream_t st, const void* q, const void* const* layer_rows_dev, const uint32_t* pos_dev, Partials part, void* xb, uint64_t batch,
+                          uint32_t max_pos, const gh_shape* s, const Plan& plan, float scale )
+{
+  const uint32_t turns = ( std::min( plan.chunk, max_pos + 1 ) + 8 / NK - 1 ) / ( 8 / NK );
+  const uint64_t groups = batch * s->n_heads * plan.max_splits;
+  if ( turns <= 1 ) {
+    launch_generic_waves<T, NK, 1>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+  } else if ( turns <= 4 || groups > (uint64_t)cu_count() ) {
+    launch_generic_waves<T, NK, 4>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+  } else {
+    launch_generic_waves<T, NK, 16>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+  }
+}
+template<typename T>
+void launch_generic( hipStream_t st, const void* q, const void* const* layer_rows_dev, const uint32_t* pos_dev, Partials part, void* xb, uint64_t batch,
+                     uint32_t max_pos, const gh_shape* s, const Plan& plan, float scale )
+{
+  if ( s->head_size <= 64 ) {
+    launch_generic_head<T, 1>( st, q, layer_rows_dev, pos_dev, part, xb, batch, max_pos, s, plan, scale );
+  } else if ( s->head_size <= 128 ) {
+    launch_generic_head<T, 2>( st, q, layer_rows_dev, pos_dev, part, xb, batch, max_pos, s, plan, scale );
+  } else {
+    launch_generic_head<T, 4>( st, q, layer_rows_dev, pos_dev, part, xb, batch, max_pos, s, plan, scale );
+  }
+}
+
 template<int G>
 void launch_valu( dim3 grid, hipStream_t st, const void* q, const void* const* rows, const uint32_t* pos, Partials part, void* xb,
                   const gh_shape* s, const Plan& p, float scale )
@@ -1496,15 +1597,10 @@ static int attn_decode_run( const char* who, const void* q, const void* const* l
   }
 
   if ( plan.variant == GH_ATTN_GENERIC ) {
-    const dim3 grid( shape->n_heads, plan.max_splits, (unsigned)batch );
     if ( dt == GH_F16 ) {
-      attn_decode_generic_kernel<__half><<<grid, 64, 0, st>>>( static_cast<const __half*>( q ), reinterpret_cast<const __half* const*>( layer_rows_dev ),
-                                                              pos_dev, part, static_cast<__half*>( xb ), shape->n_kv_heads, shape->gqa_size,
-                                                              shape->head_size, plan.chunk, plan.max_splits, scale );
+      launch_generic<__half>( st, q, layer_rows_dev, pos_dev, part, xb, batch, max_pos, shape, plan, scale );
     } else {
-      attn_decode_generic_kernel<float><<<grid, 64, 0, st>>>( static_cast<const float*>( q ), reinterpret_cast<const float* const*>( layer_rows_dev ),
-                                                             pos_dev, part, static_cast<float*>( xb ), shape->n_kv_heads, shape->gqa_size,
-                                                             shape->head_size, plan.chunk, plan.max_splits, scale );
+      launch_generic<float>( st, q, layer_rows_dev, pos_dev, part, xb, batch, max_pos, shape, plan, scale );
     }
   } else if ( joined ) {
     const uint32_t heads_per_group = join / plan.max_splits;
