@@ -142,31 +142,51 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
 }
 
 // ---- argmax: one block per row, first index of the maximum --------------------------------------
-template<typename T>
-__global__ __launch_bounds__( EW_THREADS ) void argmax_kernel( uint32_t* __restrict__ out, const T* __restrict__ v, uint32_t n )
+// Bound by latency: a row of 32000 values is one work-group's, so a thread asks for ARG_AHEAD pieces of it before it compares the first.  4 fp32
+// rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  As a loop over the row would have it: the lowest index
+// of equal values, NaN never beats anything but stays where the row begins with it.
+constexpr int ARG_THREADS = 1024, ARG_AHEAD = 8;
+__device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float v, uint32_t i )
 {
-  __shared__ float s_val[EW_THREADS / WAVE];
-  __shared__ uint32_t s_idx[EW_THREADS / WAVE];
+  const bool take = v > best || ( v == best && i < best_i );
+  best = take ? v : best;
+  best_i = take ? i : best_i;
+}
+// V: values per load, n % V == 0 and rows aligned to V values
+template<typename T, int V>
+__global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __restrict__ out, const T* __restrict__ v, uint32_t n )
+{
+  __shared__ float s_val[ARG_THREADS / WAVE];
+  __shared__ uint32_t s_idx[ARG_THREADS / WAVE];
   const T* row = v + (uint64_t)blockIdx.x * n;
-
+  struct alignas( sizeof( T ) * V ) Piece
+  {
+    T e[V];
+  };
+  const Piece* pieces = reinterpret_cast<const Piece*>( row );
+  const uint32_t n_pieces = n / V;
   float best = -INFINITY;
   uint32_t best_i = 0xffffffffu;
-  // ascending indices per thread, strict '>' keeps the lowest index of equal values
-  for ( uint32_t i = threadIdx.x; i < n; i += blockDim.x ) {
-    const float f = to_f32( row[i] );
-    if ( f > best || best_i == 0xffffffffu ) {
-      best = f;
-      best_i = i;
+  for ( uint64_t p0 = threadIdx.x; p0 < n_pieces; p0 += ARG_THREADS * ARG_AHEAD ) {
+    Piece x[ARG_AHEAD];
+#pragma unroll
+    for ( int u = 0; u < ARG_AHEAD; u++ ) {
+      x[u] = pieces[min( p0 + u * ARG_THREADS, (uint64_t)n_pieces - 1 )]; // past the end: the last one again, which changes nothing
+    }
+#pragma unroll
+    for ( int u = 0; u < ARG_AHEAD; u++ ) {
+      const uint32_t i0 = (uint32_t)min( p0 + u * ARG_THREADS, (uint64_t)n_pieces - 1 ) * V;
+#pragma unroll
+      for ( int e = 0; e < V; e++ ) {
+        arg_better( best, best_i, to_f32( x[u].e[e] ), i0 + e );
+      }
     }
   }
 #pragma unroll
   for ( int off = 32; off > 0; off >>= 1 ) {
     const float o_val = __shfl_xor( best, off, WAVE );
     const uint32_t o_idx = __shfl_xor( best_i, off, WAVE );
-    if ( o_idx != 0xffffffffu && ( best_i == 0xffffffffu || o_val > best || ( o_val == best && o_idx < best_i ) ) ) {
-      best = o_val;
-      best_i = o_idx;
-    }
+    arg_better( best, best_i, o_val, o_idx );
   }
   const int wave = threadIdx.x / WAVE;
   if ( threadIdx.x % WAVE == 0 ) {
@@ -175,15 +195,11 @@ __global__ __launch_bounds__( EW_THREADS ) void argmax_kernel( uint32_t* __restr
   }
   __syncthreads();
   if ( threadIdx.x == 0 ) {
-    for ( int w = 1; w < (int)( blockDim.x / WAVE ); w++ ) {
-      const float o_val = s_val[w];
-      const uint32_t o_idx = s_idx[w];
-      if ( o_idx != 0xffffffffu && ( best_i == 0xffffffffu || o_val > best || ( o_val == best && o_idx < best_i ) ) ) {
-        best = o_val;
-        best_i = o_idx;
-      }
+    for ( int w = 1; w < ARG_THREADS / WAVE; w++ ) {
+      arg_better( best, best_i, s_val[w], s_idx[w] );
     }
-    out[blockIdx.x] = best_i;
+    const float first = to_f32( row[0] );
+    out[blockIdx.x] = first != first || best_i == 0xffffffffu ? 0u : best_i;
   }
 }
 
@@ -393,7 +409,11 @@ int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n,
   }
   GH_REQUIRE( out_dev && v, "gh_argmax: NULL pointer" );
   GH_REQUIRE( n > 0 && n <= 0xfffffffeull && batch <= 0x7fffffffull, "gh_argmax: bad shape" );
-  GH_DISPATCH_DT( dt, argmax_kernel<T><<<(unsigned)batch, EW_THREADS, 0, as_stream( stream )>>>( out_dev, static_cast<const T*>( v ), (uint32_t)n ) );
+  if ( n * dtype_size( dt ) % 16 == 0 && ( reinterpret_cast<uintptr_t>( v ) & 15u ) == 0 ) {
+    GH_DISPATCH_DT( dt, argmax_kernel<T, 16 / sizeof( T )><<<(unsigned)batch, ARG_THREADS, 0, as_stream( stream )>>>( out_dev, static_cast<const T*>( v ), (uint32_t)n ) );
+  } else {
+    GH_DISPATCH_DT( dt, argmax_kernel<T, 1><<<(unsigned)batch, ARG_THREADS, 0, as_stream( stream )>>>( out_dev, static_cast<const T*>( v ), (uint32_t)n ) );
+  }
   GH_LAUNCH_CHECK();
   if ( out_host ) {
     GH_HIP( hipMemcpyAsync( out_host, out_dev, batch * sizeof( uint32_t ), hipMemcpyDeviceToHost, as_stream( stream ) ) );
