@@ -8,7 +8,7 @@
 // wave (v_mfma_f32_16x16x32_f16 / _bf16).  When r / 64 is too small to fill the chip K is split across
 // work-groups and an fp32 partial buffer is reduced by a second kernel.
 //
-// f32: plain wave-per-row kernel (only the tiny fp32 configuration uses it).
+// f32: gh_gemm_f32.hip.
 #include "gh_common.h"
 
 #include <cstdlib>
@@ -42,6 +42,8 @@ void gemm_tile_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits_out, u
 template<typename E>
 int gemm_tile_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, uint32_t splits, uint32_t k_per_split,
                       hipStream_t st );
+// fp32 (gh_gemm_f32.hip)
+int gemm_f32( float* out, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 
 namespace {
 
@@ -275,28 +277,6 @@ __global__ __launch_bounds__( 256 ) void gemm_skinny_kernel( float* __restrict__
   }
 }
 
-// f32: one wave per weight row, batch columns looped
-__global__ __launch_bounds__( 256 ) void gemm_f32_kernel( float* __restrict__ xout, const float* __restrict__ x, const float* __restrict__ w, uint32_t s, uint32_t r, uint32_t b )
-{
-  const uint32_t row = blockIdx.x * 4 + ( threadIdx.x >> 6 );
-  if ( row >= r ) {
-    return;
-  }
-  const uint32_t lane = threadIdx.x & 63;
-  const float* wr = w + (uint64_t)row * s;
-  for ( uint32_t col = 0; col < b; col++ ) {
-    const float* xc = x + (uint64_t)col * s;
-    float sum = 0.0f;
-    for ( uint32_t p = lane; p < s; p += 64 ) {
-      sum += wr[p] * xc[p];
-    }
-    sum = wave_sum( sum );
-    if ( lane == 0 ) {
-      xout[(uint64_t)col * r + row] = sum;
-    }
-  }
-}
-
 } // namespace
 } // namespace gh
 
@@ -479,10 +459,7 @@ int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_
       *partial_out = dst;
       *splits_out = 1;
     }
-    gemm_f32_kernel<<<(unsigned)( ( r + 3 ) / 4 ), 256, 0, st>>>( dst, static_cast<const float*>( x ), static_cast<const float*>( w ), (uint32_t)s, (uint32_t)r,
-                                                                 (uint32_t)b );
-    GH_LAUNCH_CHECK();
-    return GH_OK;
+    return gemm_f32( dst, static_cast<const float*>( x ), static_cast<const float*>( w ), s, r, b, st );
   }
   GH_REQUIRE( is_half_type( dt ), "gh_matmul: unsupported dtype %d", (int)dt );
   return with_half_type( dt, [&]( auto* e ) {

@@ -15,6 +15,11 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
 bool gemm_tile_epilogue_applicable( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
 int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, int epilogue, hipStream_t st,
                                bool* done );
+// fp32: the product and what follows it in one kernel (gh_gemm_f32.hip)
+int gemm_f32_accum( float* residual, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
+int gemm_f32_gate( float* hb, const float* x, const float* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
+int gemm_f32_qkv( float* q, float* kv_out, const float* x, const float* wqkv, uint64_t s, uint64_t b, const uint32_t* pos, const float* freq_real, const float* freq_imag,
+                  void* const* token_rows, uint32_t dim, uint32_t kv_dim, uint32_t head_size, hipStream_t st );
 
 namespace {
 
@@ -444,6 +449,12 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   GH_REQUIRE( residual != nullptr, "gh_matmul_accum: NULL residual" );
   GH_REQUIRE( ( norm_out == nullptr ) == ( norm_weight == nullptr ), "gh_matmul_accum: norm_out and norm_weight go together" );
   hipStream_t st = as_stream( stream );
+  if ( dt == GH_F32 ) {
+    if ( int rc = gemm_f32_accum( static_cast<float*>( residual ), static_cast<const float*>( x ), static_cast<const float*>( w ), s, r, b, st ) ) {
+      return rc;
+    }
+    return norm_out != nullptr ? gh_rmsnorm( norm_out, residual, norm_weight, r, b, dt, stream ) : GH_OK;
+  }
   bool done = false;
   // many rows (prompt tokens), the product by the vendor's library where the dispatcher sends plain products there: the rounded
   // product, then the reference's own next ops on it (accum, rmsnorm) -- the same roundings as fused
@@ -496,12 +507,9 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   if ( dt == GH_F16 && r % 4 == 0 && r <= 2 * 4 * EPI_THREADS && rows_8byte ) {
     epi_accum_norm_row8k_kernel<<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<__half*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
                                                                      static_cast<__half*>( norm_out ), static_cast<const __half*>( norm_weight ) );
-  } else if ( dt == GH_F16 ) {
+  } else {
     epi_accum_norm_kernel<__half><<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<__half*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
                                                                static_cast<__half*>( norm_out ), static_cast<const __half*>( norm_weight ) );
-  } else {
-    epi_accum_norm_kernel<float><<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<float*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
-                                                              static_cast<float*>( norm_out ), static_cast<const float*>( norm_weight ) );
   }
   GH_LAUNCH_CHECK();
   return GH_OK;
@@ -520,6 +528,9 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   }
   GH_REQUIRE( hb != nullptr, "gh_matmul_silu_gate: NULL output" );
   hipStream_t st = as_stream( stream );
+  if ( dt == GH_F32 ) {
+    return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), static_cast<const float*>( w13 ), s, hidden_dim, b, st );
+  }
   bool done = false;
   if ( int rc = gemm_gate_one_launch( hb, hidden_dim, x, w13, s, hidden_dim, b, dt, st, &done ) ) {
     return rc;
@@ -569,11 +580,7 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   }
   const uint64_t total = b * hidden_dim;
   const unsigned blocks = (unsigned)std::min<uint64_t>( ( total + 255 ) / 256, 8192 );
-  if ( dt == GH_F16 ) {
-    epi_silu_gate_kernel<__half><<<blocks, 256, 0, st>>>( static_cast<__half*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
-  } else {
-    epi_silu_gate_kernel<float><<<blocks, 256, 0, st>>>( static_cast<float*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
-  }
+  epi_silu_gate_kernel<__half><<<blocks, 256, 0, st>>>( static_cast<__half*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
   GH_LAUNCH_CHECK();
   return GH_OK;
 }
@@ -597,21 +604,19 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   }
   GH_REQUIRE( q && pos_dev && freq_real && freq_imag && token_rows_dev, "gh_matmul_qkv_rope_append: NULL pointer" );
   hipStream_t st = as_stream( stream );
+  if ( dt == GH_F32 ) {
+    return gemm_f32_qkv( static_cast<float*>( q ), static_cast<float*>( kv_out ), static_cast<const float*>( x ), static_cast<const float*>( wqkv ), s, b, pos_dev,
+                         static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size, st );
+  }
   float* partial = nullptr;
   uint32_t splits = 0;
   if ( int rc = gemm_partials( nullptr, x, wqkv, s, r, b, dt, st, true, &partial, &splits ) ) {
     return rc;
   }
   const dim3 grid( (unsigned)( ( r / 2 + 255 ) / 256 ), (unsigned)b );
-  if ( dt == GH_F16 ) {
-    epi_qkv_kernel<__half><<<grid, 256, 0, st>>>( static_cast<__half*>( q ), static_cast<__half*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
-                                                 static_cast<const __half*>( freq_real ), static_cast<const __half*>( freq_imag ), token_rows_dev, (uint32_t)dim,
-                                                 (uint32_t)kv_dim, head_size );
-  } else {
-    epi_qkv_kernel<float><<<grid, 256, 0, st>>>( static_cast<float*>( q ), static_cast<float*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
-                                                static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim,
-                                                (uint32_t)kv_dim, head_size );
-  }
+  epi_qkv_kernel<__half><<<grid, 256, 0, st>>>( static_cast<__half*>( q ), static_cast<__half*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
+                                               static_cast<const __half*>( freq_real ), static_cast<const __half*>( freq_imag ), token_rows_dev, (uint32_t)dim,
+                                               (uint32_t)kv_dim, head_size );
   GH_LAUNCH_CHECK();
   return GH_OK;
 }

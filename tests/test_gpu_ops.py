@@ -108,6 +108,36 @@ def test_argmax_bit_exact(dt):
     assert ops.argmax(torch.from_numpy(small).cuda()) == O.argmax(small).tolist()
 
 
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("n", [1, 7, 8, 4099, 8192, 70001])
+def test_argmax_edges(dt, n):
+    """Rows that begin with NaN, hold one, hold nothing but the lowest value or minus infinity; the maximum at either end."""
+    rng = np.random.default_rng(n)
+    v = rng.standard_normal((7, n)).astype(ndt(dt))
+    v[0, 0] = np.nan
+    v[1, n // 2] = np.nan
+    v[2, :] = -np.inf
+    v[3, :] = np.finfo(ndt(dt)).min
+    v[4, n - 1] = np.inf
+    v[5, :] = -np.inf
+    v[5, n - 1] = np.finfo(ndt(dt)).min
+    assert ops.argmax(torch.from_numpy(v).cuda()) == O.argmax(v).tolist()
+
+
+# rows that do and do not fill the pieces a wave asks for at once, with and without whole 16-byte loads, 1 to 9 activation rows at a time and
+# more than a grid row of them, two and four weight rows a wave
+@pytest.mark.parametrize("b", [1, 4, 5, 9, 67])
+@pytest.mark.parametrize("s,r", [(1, 3), (3, 7), (256, 5), (260, 64), (1027, 33), (2052, 130), (512, 4097), (96, 8195)])
+def test_matmul_f32(b, s, r):
+    rng = np.random.default_rng(61)
+    x, w = rng.standard_normal((b, s)).astype(np.float32), rng.standard_normal((r, s)).astype(np.float32)
+    got = ops.matmul(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()).cpu().numpy()
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    # a lane adds s / 64 products one after the other, the wave then 6 times two lanes' sums: at most that many roundings of the sum of magnitudes
+    bound = (s / 64 + 8) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    assert (np.abs(got - want) <= bound + 1e-30).all()
+
+
 def test_soft_sample_only_touches_warm_rows():
     rng = np.random.default_rng(5)
     v = rng.standard_normal((3, 1000)).astype(np.float32)
@@ -707,6 +737,19 @@ def test_fused_generic(dt, shape, chunk):
     got, want = run_fused_case(shape, dt, GH_ATTN_GENERIC, pos, present, chunk)
     if dt == "f32":
         np.testing.assert_allclose(got[:-1], want[:-1], rtol=1e-4, atol=2e-5)
+
+
+# head sizes of two and four pieces of 64 lanes; one key, a turn of keys and one more, the last key; few and many work-groups (16, 4 waves)
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("contexts", [5, 90])
+@pytest.mark.parametrize("heads,kv_heads,head_size", [(6, 3, 48), (3, 1, 72), (4, 4, 128), (4, 2, 160), (3, 3, 256)])
+def test_fused_generic_head_sizes(dt, contexts, heads, kv_heads, head_size):
+    shape = Shape(dim=heads * head_size, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, hidden_dim=64, seq_len=150)
+    pos = ([0, 8, 149, 1, 64] * contexts)[:contexts]
+    got, want = run_fused_case(shape, dt, GH_ATTN_GENERIC, pos, [i != 3 for i in range(contexts)], 0)
+    if dt == "f32":
+        live = [i for i in range(contexts) if i != 3]
+        np.testing.assert_allclose(got[live], want[live], rtol=1e-4, atol=2e-5)
 
 
 @pytest.mark.parametrize("shape", [MHA128, MHA128_ODD, GQA2, GQA4, GQA8], ids=["mha", "mha6", "gqa2", "gqa4", "gqa8"])
