@@ -9,7 +9,7 @@
 // work-groups and an fp32 partial buffer is reduced by a second kernel.
 //
 // f32: gh_gemm_f32.hip.
-#include "gh_common.h"
+#include "gh_product.h"
 
 #include <cstdlib>
 #include <mutex>
@@ -17,7 +17,7 @@
 
 namespace gh {
 
-// streaming decode kernel (gh_gemm_stream.hip)
+// weights through registers, on request only (gh_gemm_stream.hip)
 bool gemm_stream_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
 void gemm_stream_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits_out, uint32_t* k_per_split_out, uint32_t* rows_per_wg_out );
 template<typename E>
@@ -25,6 +25,7 @@ int gemm_stream_launch( E* xout, float* partial, const E* x, const E* w, uint64_
                         uint32_t k_per_split, uint32_t rows_per_wg, bool write_partials, hipStream_t st );
 void gemm_stream_tuning( int target_wgs, int depth );
 void gemm_stream_gate_waves( int waves );
+int gemm_stream_gate_waves();
 bool gemm_stream_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const void* x, const void* w13, const void* hb, uint64_t hb_stride );
 template<typename E>
 int gemm_stream_gate_launch( E* hb, uint64_t hb_stride, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
@@ -36,12 +37,15 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
 uint64_t gemm_tile256_token_split( uint64_t s, uint64_t r, uint64_t b );
 void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, uint32_t* splits, uint32_t* k_len );
 void gemm_tile256_tuning( int rows );
-// large-batch (prefill) kernel (gh_gemm_tile.hip)
-bool gemm_tile_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
-void gemm_tile_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits_out, uint32_t* k_per_split_out );
+// up to some hundred rows (gh_gemm_ring.hip)
+bool gemm_ring_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
+uint32_t gemm_ring_splits( uint64_t s, uint64_t r, uint64_t b, double* ns );
 template<typename E>
-int gemm_tile_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, uint32_t splits, uint32_t k_per_split,
-                      hipStream_t st );
+int gemm_ring_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
+bool gemm_ring_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const void* x, const void* w13, const void* hb, uint64_t hb_stride );
+template<typename E>
+int gemm_ring_gate_launch( E* hb, const GateRows& gate, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
+void gemm_ring_tuning( int target_wgs );
 // fp32 (gh_gemm_f32.hip)
 int gemm_f32( float* out, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 
@@ -55,7 +59,7 @@ int with_half_type( gh_dtype dt, F&& run )
 }
 inline bool is_half_type( gh_dtype dt ) { return dt == GH_F16 || dt == GH_BF16; }
 
-int g_force_kernel = 0; // 0 auto, 1 small tiled kernel of this file, 2 streaming kernel, 3 large tile kernel
+int g_force_kernel = 0; // 0 auto, 1 small tiled kernel of this file, 2 streaming kernel, 3 ring kernel (b > 64), 4 256-token tile kernel
 // GLINT_LIBRARY_ROWS in the environment overrides the default (for the command-line profilers, which have no other way in)
 uint64_t library_rows_default()
 {
@@ -285,19 +289,32 @@ namespace gh {
 // Runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums
 // `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue;
 // otherwise the kernel may store DType results straight into `xout` (*splits_out == 0 then).
-// w1, w3 and the SiLU gate in one launch of the streaming kernel, where gemm_partials() would pick that
-// kernel without a K split.  *done = false: nothing was launched, the caller takes the two-kernel route.
-int gemm_gate_one_launch( void* hb, uint64_t hb_stride, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
+
+int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
                           bool* done )
 {
   *done = false;
-  if ( !is_half_type( dt ) || ( g_force_kernel != 0 && g_force_kernel != 2 ) || b > 64 || !gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, hb_stride ) ) {
+  if ( !is_half_type( dt ) ) {
+    return GH_OK;
+  }
+  const bool stream = ( g_force_kernel == 2 || ( g_force_kernel == 0 && gemm_stream_gate_waves() != 0 ) ) && b <= 64
+                      && gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
+  // From 192 rows on the 256-token tiles with the gate's kernel behind them, where they are enough (70B, 256 rows: 235 us, here 264);
+  // the vendor's library where it is asked for.  An exact caller's other route there is one product with the matrices next to w13.
+  const bool others = b >= 192 && ( gate.exact || gemm_tile256_applicable( s, 2 * hidden, b, x, w13, hb ) );
+  const bool library = b > 64 && ( gemm_library_wanted_wide( s, 2 * hidden, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden, b, dt, x, w13, hb ) );
+  const bool ring = !stream && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) && !others && !library
+                    && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
+  if ( !stream && !ring ) {
     return GH_OK;
   }
   *done = true;
   return with_half_type( dt, [&]( auto* e ) {
     using E = std::remove_pointer_t<decltype( e )>;
-    return gemm_stream_gate_launch<E>( static_cast<E*>( hb ), hb_stride, static_cast<const E*>( x ), static_cast<const E*>( w13 ), s, hidden, b, st );
+    E* out = static_cast<E*>( hb );
+    const E *in = static_cast<const E*>( x ), *mat = static_cast<const E*>( w13 );
+    return stream ? gemm_stream_gate_launch<E>( out, gate.stride, in, mat, s, hidden, b, st )
+                  : gemm_ring_gate_launch<E>( out, gate, in, mat, s, hidden, b, st );
   } );
 }
 
@@ -351,7 +368,7 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     GH_LAUNCH_CHECK();
     return GH_OK;
   }
-  // many tokens at once (prefill): the MFMA-bound tile kernel; few (decode): the weight-streaming one
+  // many tokens at once (prefill): the MFMA-bound tile kernel; few (decode): the ring kernel
   if ( ( g_force_kernel == 0 || g_force_kernel == 4 ) && gemm_tile256_applicable( s, r, b, x, w, xout ? xout : x ) ) {
     float* ws = nullptr;
     if ( want_partials ) {
@@ -363,10 +380,15 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     }
     return gemm_tile256_launch( xout, ws, x, w, s, r, b, 0, st, 1, 0 );
   }
+  const bool ring = gemm_ring_applicable( s, r, b, x, w, xout ? xout : x );
+  double ring_ns = 0.0;
+  const uint32_t ring_splits = ring ? gemm_ring_splits( s, r, b, &ring_ns ) : 0;
   if ( g_force_kernel == 0 || g_force_kernel == 4 ) { // some hundred rows and few tiles: the same kernel with the K range split
     uint32_t splits = 0, k_len = 0;
     gemm_tile256_split_plan( s, r, b, x, w, &splits, &k_len );
-    if ( splits > 1 ) {
+    // a step of 64 k takes a tile 1.7 us, the sums as in the ring kernel's plan (512 rows: 70B wo 75 us, ring 84; 13B w2 128 and 94)
+    const double tile_ns = 3000.0 + 1700.0 * k_len / 64 + (double)( splits * b * r ) * 8.0 / 5000.0;
+    if ( splits > 1 && ( g_force_kernel == 4 || !ring || tile_ns < ring_ns ) ) {
       float* ws = nullptr;
       if ( int rc = ensure_workspace( (uint64_t)splits * b * r * sizeof( float ), &ws, st ) ) {
         return rc;
@@ -377,22 +399,20 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     }
   }
   GH_REQUIRE( g_force_kernel != 4, "gh_matmul: the 256 x 256 tile kernel needs b >= 192, at least 192 tiles with a last round that is not mostly empty, s %% 64 == 0 and 16-byte aligned operands" );
-  if ( ( g_force_kernel == 0 || g_force_kernel == 3 ) && gemm_tile_applicable( s, r, b, x, w, xout ? xout : x ) ) {
-    uint32_t splits = 1, k_per_split = 0;
-    gemm_tile_plan( s, r, b, &splits, &k_per_split );
+  if ( ring && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) ) {
     float* ws = nullptr;
-    if ( want_partials || splits > 1 ) {
-      if ( int rc = ensure_workspace( (uint64_t)splits * b * r * sizeof( float ), &ws, st ) ) {
+    if ( want_partials || ring_splits > 1 ) {
+      if ( int rc = ensure_workspace( (uint64_t)ring_splits * b * r * sizeof( float ), &ws, st ) ) {
         return rc;
       }
       *partial_out = ws;
-      *splits_out = splits;
+      *splits_out = ring_splits;
     }
-    return gemm_tile_launch( xout, ws, x, w, s, r, b, splits, k_per_split, st );
+    return gemm_ring_launch( xout, ws, x, w, s, r, b, st );
   }
-  GH_REQUIRE( g_force_kernel != 3, "gh_matmul: the tile kernel needs b > 64, s %% 8 == 0 and 16-byte aligned operands" );
+  GH_REQUIRE( g_force_kernel != 3, "gh_matmul: the ring kernel needs b > 64 (when forced), s %% 8 == 0 and 16-byte aligned operands" );
 
-  if ( g_force_kernel != 1 && gemm_stream_applicable( s, r, b, x, w, xout ? xout : x ) ) {
+  if ( g_force_kernel == 2 && gemm_stream_applicable( s, r, b, x, w, xout ? xout : x ) ) {
     uint32_t splits = 1, k_per_split = 0, rows_per_wg = 0;
     gemm_stream_plan( s, r, b, &splits, &k_per_split, &rows_per_wg );
     float* ws = nullptr;
@@ -501,6 +521,7 @@ int gh_gemm_set_tuning( int kernel, int target_workgroups, int tile_rows )
 {
   g_force_kernel = kernel;
   gemm_stream_tuning( target_workgroups, 0 );
+  gemm_ring_tuning( target_workgroups );
   gemm_tile256_tuning( tile_rows );
   return GH_OK;
 }

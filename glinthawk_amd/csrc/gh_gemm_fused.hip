@@ -4,13 +4,11 @@
 // are a single launch when no K split is needed), so a layer needs 9 launches instead of 21.
 // Rounding points are those of the unfused sequence: every matmul result is rounded to DType first
 // (the reference stores it), later math is fp32 with one rounding per store.
-#include "gh_common.h"
+#include "gh_product.h"
 
 namespace gh {
 
-int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, hipStream_t st, bool want_partials,
-                   float** partial_out, uint32_t* splits_out );
-int gemm_gate_one_launch( void* hb, uint64_t hb_stride, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st, bool* done );
+int gemm_gate_one_launch( void* hb, uint64_t hb_stride, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, bool exact, hipStream_t st, bool* done );
 uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
 bool gemm_tile_epilogue_applicable( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
 int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, int epilogue, hipStream_t st,
@@ -532,7 +530,7 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
     return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), static_cast<const float*>( w13 ), s, hidden_dim, b, st );
   }
   bool done = false;
-  if ( int rc = gemm_gate_one_launch( hb, hidden_dim, x, w13, s, hidden_dim, b, dt, st, &done ) ) {
+  if ( int rc = gemm_gate_one_launch( hb, GateRows { hidden_dim }, x, w13, s, hidden_dim, b, dt, st, &done ) ) {
     return rc;
   }
   if ( done ) {
@@ -560,7 +558,7 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   // Some hundred rows and more with enough tiles for the large tile kernel: both factors in one launch of it, stored as DType whole
   // row segments (the second factor into a scratch buffer), then the gate as the element-wise kernel.  The fp32 sums that the
   // route below leaves for its gate kernel are stored from the accumulator registers, 16 bytes to each of 32 lines per
-  // instruction, and are twice the bytes: at 256 rows of the 70B shape 277 + 19 us against 257 + 12.  Same roundings either way
+  // instruction, and are twice the bytes (256 rows of the 70B shape: 224 + 9 us here; with sums 20 + 7 us more).  Same roundings either way
   // (each factor to DType, then the gate).
   if ( dt == GH_F16 && hidden_dim % 8 == 0
        && ( gemm_tile_epilogue_applicable( s, 2 * hidden_dim, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden_dim, b, dt, x, w13, hb ) ) ) {

@@ -1,4 +1,5 @@
-// Weight-streaming GEMM for decode: xout(b, r) = sum_p w(r, p) * x(b, p) with a small batch
+// Weight-streaming GEMM through registers, run on request only (gh_gemm_set_tuning, gh_gemm_set_gate_waves; gh_gemm_stream_plan tells its
+// plan): the ring kernel (gh_gemm_ring.hip) was faster at every shape measured.  xout(b, r) = sum_p w(r, p) * x(b, p) with a small batch
 // (64 columns per column slab), f16 or bf16 storage, fp32 accumulate.  Every weight element is read from HBM
 // exactly once, so the kernel is built like a streaming read:
 //
@@ -477,6 +478,8 @@ void gemm_stream_tuning( int target_wgs, int depth )
   }
   (void)depth;
 }
+
+int gemm_stream_gate_waves() { return g_gate_waves; }
 
 void gemm_stream_gate_waves( int waves ) { g_gate_waves = waves == 4 || waves == 8 ? waves : 0; }
 

@@ -476,7 +476,7 @@ void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, const void* x,
   }
   const uint64_t steps = s / TKS;
   // Very few tiles and a short K (70B wo at 256 rows: 32 tiles, 8 splits of 16 steps, fp32 sums half the size of the weights):
-  // the 128 x 128 kernel with two work-groups per CU hides more of such a short work-group's start-up (60 against 73 us).
+  // the ring kernel's smaller tiles need fewer and hide more of a short work-group's start-up (55 against 73 us with the sums).
   if ( tiles * 8 <= cus && steps <= 128 ) {
     return;
   }

@@ -14,9 +14,6 @@
 
 namespace gh {
 
-// gh_gemm.hip: gate, up and SiLU in one launch where the streaming kernel runs without a K split; *done = false: nothing was launched
-int gemm_gate_one_launch( void* hb, uint64_t hb_stride, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st, bool* done );
-
 namespace {
 
 struct ParallelCols
@@ -256,7 +253,8 @@ int gh_matmul_parallel( void* q, float* head_gates, void* hidden, uint64_t hidde
   hipStream_t st = as_stream( stream );
   if ( ff > 0 && dt == GH_BF16 && activation == GH_ACT_SILU ) {
     bool done = false;
-    if ( int rc = gemm_gate_one_launch( hidden, hidden_stride, x, static_cast<const __bf16*>( w ) + cols.ff * width, width, ff, rows, dt, st, &done ) ) {
+    const GateRows gate { hidden_stride, true, const_cast<const void* const*>( context_rows_dev ), n_tokens };
+    if ( int rc = gemm_gate_one_launch( hidden, gate, x, static_cast<const __bf16*>( w ) + cols.ff * width, width, ff, rows, dt, st, &done ) ) {
       return rc;
     }
     if ( done ) {

@@ -10,6 +10,17 @@ namespace gh {
 int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, hipStream_t st, bool want_partials,
                    float** partial_out, uint32_t* splits_out );
 
+// Rows of a gated feed-forward that its product stores itself: DType(silu(y1) * y3).
+struct GateRows
+{
+  uint64_t stride { 0 };                       // elements from row to row
+  bool exact { false };                        // the gate over the fp32 sums; else y1 and y3 rounded to DType first, as two products would leave them
+  const void* const* context_rows { nullptr }; // n_tokens rows of each context; those of a context without an entry are not written
+  uint32_t n_tokens { 1 };
+};
+// w1, w3 and the gate in one launch; *done = false: nothing was launched, the caller takes its other route
+int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st, bool* done );
+
 struct Product
 {
   const void* data { nullptr };

@@ -153,12 +153,12 @@ int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_
 int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::matmul<s,r> / untemplated_matmul  arch/amd64/common/ops.hh:74-93,212-271 :
  * xout(b, r) = sum_p w(r, p) * x(b, p); w row-major (r, s); fp32 accumulate */
-/* tuning hook: kernel 0 auto / 1 small tiled / 2 streaming (decode) / 3 128x128 tile / 4 256-token tile (many rows); the number of compute units the
- * streaming kernel's K split is balanced for (<= 0 keeps the current value; the default is the device's own count); `tile_rows` non-zero: a
+/* tuning hook: kernel 0 auto / 1 small tiled / 2 streaming through registers / 3 ring (more than 64 rows) / 4 256-token tile (many rows); the number of
+ * compute units the streaming and the ring kernel's plans are balanced for (<= 0 keeps the current value; the default is the device's own count); `tile_rows` non-zero: a
  * product is never cut in two along the tokens */
 int gh_gemm_set_tuning( int kernel, int target_workgroups, int tile_rows );
-/* measurement / test hook: waves per work-group of the decode product that computes w1 and w3 in one launch and applies the SiLU gate itself
- * (gh_matmul_silu_gate at up to 64 rows without a K split): 4, 8, or 0 = the library's choice (8 where work-groups of 4 would come two to a CU) */
+/* measurement / test hook: w1 and w3 with the SiLU gate in one launch (gh_matmul_silu_gate) by the streaming kernel in work-groups of 4 or 8
+ * waves, at up to 64 rows where that kernel would not split K; 0: the library's choice, the ring kernel */
 int gh_gemm_set_gate_waves( int waves );
 /* Opt-in: plain f16 products (gh_matmul, the two of gh_matmul_pair, the product inside gh_matmul_accum and gh_matmul_silu_gate where no
  * kernel of this library fuses it) of `rows` activation rows and more go to the vendor's GEMM library, as every product of the

@@ -332,6 +332,26 @@ def test_matmul_streaming_kernel_sweep(b, s, r):
     assert err.max().item() < 2e-2 and (err.mean() / want.abs().mean()).item() < 1e-3
 
 
+# the ring kernel's edges: K ranges that end inside a step of 64, fewer steps than stages, odd row counts, each width of the activation
+# tile and the first beyond it, several slabs of activation rows, both heights of the weight tile, K splits
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,s,r", [(1, 8, 4), (16, 72, 20), (32, 4104, 1030), (33, 8192, 10240), (96, 1000, 517), (97, 4096, 256), (129, 2056, 12),
+                                   (192, 640, 3000), (191, 1472, 5000), (257, 1096, 300), (700, 520, 1001), (5, 28672, 8192), (128, 8192, 14336)])
+def test_matmul_ring_edges(dt, b, s, r):
+    """One-hot activations: every output is one weight, bit for bit.  A random product: fp32 sums, so off by the result's own rounding
+    (half an ulp, relative 2^-11 or 2^-8) and by the order of the sums (s terms of about s^-1/2: far below 1e-4 of their scale)."""
+    g = torch.Generator(device="cuda").manual_seed(b * 13 + r)
+    w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+    hot = torch.zeros((b, s), dtype=dt, device="cuda")
+    cols = torch.tensor([(7919 * i + 3) % s for i in range(b)], device="cuda")
+    hot[torch.arange(b, device="cuda"), cols] = 1
+    x = torch.randn((b, s), generator=g, device="cuda").to(dt)
+    assert torch.equal(ops.matmul(hot, w), w[:, cols].t().contiguous())
+    want = x.double() @ w.double().t()
+    bound = want.abs() * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 1e-4
+    assert ((ops.matmul(x, w).double() - want).abs() <= bound).all()
+
+
 # some hundred rows (the decode step of a large slot arena): whatever the dispatcher picks at each batch size (streaming kernel up
 # to 64 rows, 128 x 128 tiles with or without a K split, 256-token tiles with the K range split over work-groups when the tiles are
 # few), ragged edges in rows, tokens and K steps.  One-hot activations: every output is one weight, bit for bit.
