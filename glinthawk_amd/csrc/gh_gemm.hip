@@ -30,12 +30,15 @@ bool gemm_stream_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const
 template<typename E>
 int gemm_stream_gate_launch( E* hb, uint64_t hb_stride, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
 // 256 x 256 tile kernel for products with enough tiles (gh_gemm_tile256.hip)
-bool gemm_tile256_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
+bool gemm_tile256_takes( uint64_t s, uint64_t b, const void* x, const void* w, const void* xout );
+bool gemm_tile256_fills( uint64_t r, uint64_t b );
+double gemm_tile256_ns( uint64_t s, uint64_t r, uint64_t b );
 template<typename E>
 int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, int epilogue, hipStream_t st,
                          uint32_t splits, uint32_t k_len, E* xout2 = nullptr, uint64_t r_first = 0 );
-uint64_t gemm_tile256_token_split( uint64_t s, uint64_t r, uint64_t b );
-void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, uint32_t* splits, uint32_t* k_len );
+uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b );
+uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds );
+void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns );
 void gemm_tile256_tuning( int rows );
 // up to some hundred rows (gh_gemm_ring.hip)
 bool gemm_ring_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
@@ -290,6 +293,25 @@ namespace gh {
 // `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue;
 // otherwise the kernel may store DType results straight into `xout` (*splits_out == 0 then).
 
+// Many rows without whole tiles of 256 x 256: the ring kernel, or those tiles with the K range split, and the kernel that adds the sums.
+static double other_tiles_ns( uint64_t s, uint64_t r, uint64_t b )
+{
+  double ring = 0.0, tiles = 0.0;
+  uint32_t splits = 0, k_len = 0;
+  ring += gemm_ring_splits( s, r, b, &ring ) > 1 ? 4500.0 : 0.0;
+  gemm_tile256_split_plan( s, r, b, &splits, &k_len, &tiles );
+  return splits > 1 ? std::min( ring, tiles + 4500.0 ) : ring;
+}
+
+// Whether a product runs as whole tiles of 256 x 256 (what is left of it once gemm_token_split() has cut it).
+static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout )
+{
+  if ( !gemm_tile256_takes( s, b, x, w, xout ) ) {
+    return false;
+  }
+  return g_force_kernel == 4 ? gemm_tile256_fills( r, b ) : g_force_kernel == 0 && gemm_tile256_ns( s, r, b ) <= other_tiles_ns( s, r, b );
+}
+
 int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
                           bool* done )
 {
@@ -301,7 +323,7 @@ int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const v
                       && gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
   // From 192 rows on the 256-token tiles with the gate's kernel behind them, where they are enough (70B, 256 rows: 235 us, here 264);
   // the vendor's library where it is asked for.  An exact caller's other route there is one product with the matrices next to w13.
-  const bool others = b >= 192 && ( gate.exact || gemm_tile256_applicable( s, 2 * hidden, b, x, w13, hb ) );
+  const bool others = b >= 192 && ( gate.exact || tile256_wanted( s, 2 * hidden, b, x, w13, hb ) );
   const bool library = b > 64 && ( gemm_library_wanted_wide( s, 2 * hidden, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden, b, dt, x, w13, hb ) );
   const bool ring = !stream && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) && !others && !library
                     && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
@@ -318,15 +340,29 @@ int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const v
   } );
 }
 
-// Tokens of the first part when a many-row product is better run as two products along the tokens (see
-// gemm_tile256_token_split), 0 otherwise.
+// Tokens of the first part when a many-row product is better run as two products along the tokens, 0 otherwise.
 uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout )
 {
-  if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_applicable( s, r, b, x, w, xout ) ) {
+  if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
     return 0;
   }
-  const uint64_t b1 = gemm_tile256_token_split( s, r, b );
-  return b1 != 0 && gemm_tile256_applicable( s, r, b1, x, w, xout ) && ( b1 * r * 2 ) % 16 == 0 && ( b1 * s * 2 ) % 16 == 0 ? b1 : 0;
+  const double whole = gemm_tile256_ns( s, r, b );
+  double best = std::min( whole, other_tiles_ns( s, r, b ) );
+  uint64_t best_b1 = 0;
+  const uint64_t rounds = gemm_tile256_rounds( r, b );
+  for ( uint64_t n = 1; n < 3 && n < rounds; n++ ) { // the first part one round shorter, or two
+    const uint64_t b1 = gemm_tile256_tokens( r, b, rounds - n );
+    if ( b1 < 192 || ( b1 * r * 2 ) % 16 != 0 ) {
+      break;
+    }
+    // a second launch, and 2 % for what the estimates don't know
+    const double cost = ( gemm_tile256_ns( s, r, b1 ) + other_tiles_ns( s, r, b - b1 ) + 2000.0 ) * 1.02;
+    if ( cost < best ) {
+      best = cost;
+      best_b1 = b1;
+    }
+  }
+  return best_b1;
 }
 
 // Many rows: the large tile kernel with the op that follows the product in its epilogue, 1 = xout += product
@@ -334,7 +370,7 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
 // its other route.
 bool gemm_tile_epilogue_applicable( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout )
 {
-  return is_half_type( dt ) && r % 8 == 0 && ( g_force_kernel == 0 || g_force_kernel == 4 ) && gemm_tile256_applicable( s, r, b, x, w, xout );
+  return is_half_type( dt ) && r % 8 == 0 && tile256_wanted( s, r, b, x, w, xout );
 }
 
 int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, int epilogue, hipStream_t st,
@@ -369,7 +405,7 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     return GH_OK;
   }
   // many tokens at once (prefill): the MFMA-bound tile kernel; few (decode): the ring kernel
-  if ( ( g_force_kernel == 0 || g_force_kernel == 4 ) && gemm_tile256_applicable( s, r, b, x, w, xout ? xout : x ) ) {
+  if ( tile256_wanted( s, r, b, x, w, xout ? xout : x ) ) {
     float* ws = nullptr;
     if ( want_partials ) {
       if ( int rc = ensure_workspace( b * r * sizeof( float ), &ws, st ) ) {
@@ -385,9 +421,10 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
   const uint32_t ring_splits = ring ? gemm_ring_splits( s, r, b, &ring_ns ) : 0;
   if ( g_force_kernel == 0 || g_force_kernel == 4 ) { // some hundred rows and few tiles: the same kernel with the K range split
     uint32_t splits = 0, k_len = 0;
-    gemm_tile256_split_plan( s, r, b, x, w, &splits, &k_len );
-    // a step of 64 k takes a tile 1.7 us, the sums as in the ring kernel's plan (512 rows: 70B wo 75 us, ring 84; 13B w2 128 and 94)
-    const double tile_ns = 3000.0 + 1700.0 * k_len / 64 + (double)( splits * b * r ) * 8.0 / 5000.0;
+    double tile_ns = 0.0;
+    if ( gemm_tile256_takes( s, b, x, w, x ) ) {
+      gemm_tile256_split_plan( s, r, b, &splits, &k_len, &tile_ns );
+    }
     if ( splits > 1 && ( g_force_kernel == 4 || !ring || tile_ns < ring_ns ) ) {
       float* ws = nullptr;
       if ( int rc = ensure_workspace( (uint64_t)splits * b * r * sizeof( float ), &ws, st ) ) {
@@ -544,7 +581,10 @@ uint64_t gh_gemm_library_rows( void ) { return g_library_rows; }
 int gh_matmul_fuses_many_rows( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
 {
   static const char aligned[16] __attribute__( ( aligned( 16 ) ) ) = { 0 };
-  return gemm_tile_epilogue_applicable( s, r, b, dt, aligned, aligned, aligned ) ? 1 : 0;
+  return gemm_tile_epilogue_applicable( s, r, b, dt, aligned, aligned, aligned )
+             || ( r % 8 == 0 && gemm_token_split( s, r, b, dt, aligned, aligned, aligned ) != 0 )
+           ? 1
+           : 0;
 }
 
 int gh_gemm_stream_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_per_split, uint32_t* rows_per_workgroup )
@@ -577,7 +617,7 @@ int gh_matmul_pair( void* xout_a, void* xout_b, const void* x, const void* w, ui
   }
   // many rows: one launch of the large tile kernel whose work-groups store to the matrix their rows belong to, so that the two
   // products fill their rounds together (a product of 2048 rows alone leaves most of the chip idle)
-  if ( is_half_type( dt ) && g_force_kernel == 0 && r_a > 0 && r_b > 0 && r_a % 8 == 0 && r_b % 8 == 0 && gemm_tile256_applicable( s, r, b, x, w, xout_a )
+  if ( is_half_type( dt ) && g_force_kernel == 0 && r_a > 0 && r_b > 0 && r_a % 8 == 0 && r_b % 8 == 0 && gemm_tile256_takes( s, b, x, w, xout_a )
        && ( reinterpret_cast<uintptr_t>( xout_b ) & 15u ) == 0 ) {
     if ( const uint64_t b1 = gemm_token_split( s, r, b, dt, x, w, xout_a ) ) {
       if ( ( b1 * r_a * elem ) % 16 == 0 && ( b1 * r_b * elem ) % 16 == 0 ) {
@@ -588,11 +628,13 @@ int gh_matmul_pair( void* xout_a, void* xout_b, const void* x, const void* w, ui
                                static_cast<const char*>( x ) + b1 * s * elem, w, s, r_a, r_b, b - b1, dt, stream );
       }
     }
-    return with_half_type( dt, [&]( auto* e ) {
-      using E = std::remove_pointer_t<decltype( e )>;
-      return gemm_tile256_launch<E>( static_cast<E*>( xout_a ), nullptr, static_cast<const E*>( x ), static_cast<const E*>( w ), s, r, b, 0, as_stream( stream ), 1,
-                                     0, static_cast<E*>( xout_b ), r_a );
-    } );
+    if ( tile256_wanted( s, r, b, x, w, xout_a ) ) {
+      return with_half_type( dt, [&]( auto* e ) {
+        using E = std::remove_pointer_t<decltype( e )>;
+        return gemm_tile256_launch<E>( static_cast<E*>( xout_a ), nullptr, static_cast<const E*>( x ), static_cast<const E*>( w ), s, r, b, 0, as_stream( stream ),
+                                       1, 0, static_cast<E*>( xout_b ), r_a );
+      } );
+    }
   }
   if ( int rc = gh_matmul( xout_a, x, w, s, r_a, b, dt, stream ) ) {
     return rc;

@@ -6,8 +6,9 @@
 //               lane, no registers); S - 1 steps are requested ahead.  One barrier a step: behind it this step's stage has landed for
 //               all waves, and the stage of the step before is free and is refilled at once.
 //   math        v_mfma_f32_16x16x32, the waves as RG groups of weight rows by TG groups of activation rows
-//   k order     a work-group starts a long K range at a step of its own and wraps around: rows are a power of two apart in memory, and
-//               work-groups in lock step on one column range would meet on few channels (7B w1 + w3 at 8 rows: 35 us, rotated 29)
+//   k order     with one slab of activation rows, a work-group starts a long K range at a step of its own and wraps around: rows are a power of two apart in memory, and
+//               work-groups in lock step on one column range would meet on few channels (7B w1 + w3 at 8 rows: 35 us, rotated 29).  Several slabs read the same
+//               weights and keep step, so that L2 serves all but one (7B wo at 1800 rows: 71 us, rotated 100)
 //   XCDs        neighbouring work-groups of one K range on one XCD, whose L2 then holds that range of the activations
 //
 // Measured, cold weights (the streaming kernel, or from 65 rows on a register-staged 128 x 128 tile kernel with two work-groups a CU,
@@ -93,7 +94,7 @@ __global__ __launch_bounds__( RING_THREADS, 1 ) void gemm_ring_kernel( void* __r
   const uint32_t col0 = slab * cut.cols, n_cols = min( cut.cols, b - col0 );
   const uint32_t all_steps = ( s + RING_K - 1 ) / RING_K;
   const uint32_t step0 = split * cut.steps, n_steps = min( cut.steps, all_steps - step0 );
-  const uint32_t start = n_steps < RING_TURN_STEPS ? 0 : unit % n_steps;
+  const uint32_t start = n_steps < RING_TURN_STEPS || cut.slabs > 1 ? 0 : unit % n_steps;
   // RING_GATE: 16-row tiles of w1 and w3 in turn, so that the factors of an output meet in one lane; a wave loads from one of the two
   const uint64_t w_row0 = first + ( MODE == RING_GATE ? ( ( wave >> 1 ) & 1 ) * (uint64_t)r : 0 );
   const char* w_base = reinterpret_cast<const char*>( w + w_row0 * s );
@@ -318,10 +319,11 @@ int ring_launch( int mode, void* out, const E* x, const E* w, uint64_t s, uint64
 int g_ring_cus = 0; // tuning override of the CU count the plan balances for (0: the device's)
 
 // The tile, the rows of a work-group and the K split.  A CU takes one work-group at a time, so a launch is as slow as its rounds of
-// work-groups.  Fitted to timings of the 7B, 13B and 70B shapes with cold weights, 1 to 512 rows: a step costs its weights at the CU's
-// share of the memory's rate (4.7 ns a row; less where slabs share them in L2) and its activations at what L2 delivers to a CU (2 ns a
-// row), but no less than a load's time in flight (1.9 us) over the steps requested ahead; a round costs what it takes to fill the ring,
-// and a split the fp32 sums that are written and read again.
+// work-groups.  Fitted to timings of the 7B, 13B and 70B shapes, up to 256 rows with cold weights, and 300 to 7000.  A step costs its
+// weights at the CU's share of the memory's rate (4.7 ns a row) and its activations at what L2 delivers to a CU (2 ns a row), but no
+// less than a load's time in flight (1.9 us) over the steps requested ahead.  With several slabs the weights come from L2 and the
+// matrix units set the pace; wide slabs slow each other down.  A round costs what it takes to fill the ring, and a split the fp32 sums
+// that are written and read again.
 RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
 {
   constexpr uint32_t XS[] = { 32, 64, 96, 128, 192, 256 };
@@ -347,10 +349,11 @@ RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
           const uint64_t rows = std::min<uint64_t>( most, std::max<uint64_t>( 16, ( ( r + blocks - 1 ) / blocks + 3 ) / 4 * 4 ) );
           const uint64_t row_blocks = ( r + rows - 1 ) / rows;
           const double real_rounds = (double)( ( row_blocks * slabs * splits + n_cu - 1 ) / n_cu );
-          const double step_ns = std::max( ( slabs == 1 ? 4.7 : 2.7 ) * (double)( gate ? 2 * rows : rows ) + 2.0 * (double)std::min<uint64_t>( cols, b ),
-                                           1900.0 / ( ring_stages( w, x ) - 1 ) );
+          const double w_rows = (double)( gate ? 2 * rows : rows ), x_rows = (double)std::min<uint64_t>( cols, b );
+          const double step_ns = slabs == 1 ? std::max( 4.7 * w_rows + 2.0 * x_rows, 1900.0 / ( ring_stages( w, x ) - 1 ) )
+                                            : 1.05 * ( 2.9 * w_rows + 1.05 * ( x_rows + x ) + ( x > 128 ? 20.0 + 7.0 * (double)slabs : 40.0 ) );
           const double sums_ns = splits > 1 ? (double)( splits * b * r ) * 8.0 / 5000.0 : 0.0;
-          const double cost = real_rounds * ( 2000.0 + (double)per * step_ns ) + sums_ns;
+          const double cost = real_rounds * ( ( slabs == 1 ? 2000.0 : 3000.0 ) + (double)per * step_ns ) + sums_ns;
           if ( best.w == 0 || cost < best.ns ) {
             best = RingPlan { w, x, RingCut { (uint32_t)rows, (uint32_t)cols, (uint32_t)row_blocks, (uint32_t)slabs, (uint32_t)splits, (uint32_t)per }, cost };
           }

@@ -419,74 +419,71 @@ uint64_t rounds_per_xcd( uint64_t r, uint64_t b )
 
 void gemm_tile256_tuning( int rows ) { g_tile_rows = rows; }
 
-// Worth it when the 256 x 256 tiles alone fill the chip (no K split here) and the last round of them
-// is not mostly empty (measured against the 128 x 128 kernel: 15-40 % faster from 192 tiles up, except
-// at 258-260 tiles, where the second round runs 4 tiles on 256 CUs).
-bool gemm_tile256_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout )
+bool gemm_tile256_takes( uint64_t s, uint64_t b, const void* x, const void* w, const void* xout )
 {
-  const uint64_t tiles = ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 );
-  // one work-group per CU: a last round that leaves more than 40 % of the chip idle goes to the 128 x 128 kernel instead
-  const uint64_t cus = (uint64_t)cu_count();
-  const uint64_t rounds = ( tiles + cus - 1 ) / cus;
-  const bool enough = 4 * tiles >= 3 * cus && 10 * tiles >= 6 * rounds * cus;
-  return b >= 192 && enough && s % TKS == 0 && s >= 2 * TKS && s < ( 1u << 22 )
+  return b >= 192 && s % TKS == 0 && s >= 2 * TKS && s < ( 1u << 22 )
          && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) | reinterpret_cast<uintptr_t>( xout ) ) & 15u ) == 0;
 }
 
-// A launch is as slow as its number of rounds (one work-group per CU), so a product whose tiles leave the last round mostly
-// empty pays for a whole round there: 8192 rows x 4480 tokens are 576 tiles of 256 x 256, 2.25 rounds, and take 3.  Such a product
-// is cut in two along the tokens: the first part a number of tokens whose tiles fill their rounds, the rest a product of a few
-// hundred tokens that goes its own way (smaller tiles, or this kernel with the K range split).  Returns the tokens of the first
-// part, 0 to leave the product whole.  Costs in percent of a round.
-uint64_t gemm_tile256_token_split( uint64_t s, uint64_t r, uint64_t b )
+// Enough tiles to fill the chip without a K split, and no last round that is mostly empty: what the forced kernel takes.
+bool gemm_tile256_fills( uint64_t r, uint64_t b )
 {
-  if ( g_tile_rows != 0 || b < 3 * TN2 ) {
-    return 0;
-  }
-  auto cost = [&]( uint64_t tokens ) { return 100 * rounds_per_xcd( r, tokens ); };
-  const uint64_t whole = cost( b );
-  uint64_t best = whole, best_b1 = 0;
-  const uint64_t token_tiles = b / TN2;
-  for ( uint64_t t = token_tiles; t + 8 >= token_tiles && t >= 2; t-- ) {
-    const uint64_t b1 = t * TN2;
-    if ( b1 >= b ) {
-      continue;
-    }
-    // the rest: its flops in rounds of this kernel, at 60 % of this kernel's rate, plus a start-up
-    const uint64_t rest = 100 * ( b - b1 ) * r / ( (uint64_t)TM2 * TN2 * (uint64_t)cu_count() ) * 10 / 6 + 15;
-    const uint64_t c = cost( b1 ) + rest;
-    if ( c < best ) {
-      best = c;
-      best_b1 = b1;
-    }
-  }
-  return 100 * best < 92 * whole ? best_b1 : 0;
+  const uint64_t tiles = ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 );
+  const uint64_t cus = (uint64_t)cu_count(), rounds = ( tiles + cus - 1 ) / cus;
+  return 4 * tiles >= 3 * cus && 10 * tiles >= 6 * rounds * cus;
 }
 
-// Few tiles (a decode step of some hundred rows, or a narrow product): the K range is split over several work-groups per tile so
-// that the chip is full in one round, and the fp32 sums of each split go to partial[split].  *splits = 0: not for this shape.
-void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, uint32_t* splits, uint32_t* k_len )
+// `rounds` of one work-group per CU, `units` work-groups in all.  A step of 64 k takes 1 us while few CUs multiply and 1.37 when all do and
+// the clock drops (70B w2, 448 steps: 200 tokens 483 us, 1024 511, 2048 616, 3328 in two rounds 1155), a round's ends 3.5.
+static double rounds_ns( uint64_t rounds, uint64_t units, uint64_t steps, double step_ns )
+{
+  const double busy = (double)units / (double)( rounds * (uint64_t)cu_count() );
+  return (double)rounds * ( (double)steps * std::max( step_ns, 1000.0 + 370.0 * busy * busy ) + 3500.0 );
+}
+double gemm_tile256_ns( uint64_t s, uint64_t r, uint64_t b )
+{
+  return rounds_ns( rounds_per_xcd( r, b ), ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 ), s / TKS, 0.0 );
+}
+
+// A launch is as slow as its number of rounds, so a product whose tiles leave the last round partly empty pays for a whole round there:
+// 8192 rows x 3328 tokens are 416 tiles, 1.6 rounds, and take 2.  Such a product may be cut in two along the tokens: the first part as
+// many tokens as fill `rounds` rounds, the rest a product of its own (the K range split over work-groups, or smaller tiles).  Returns
+// those tokens, 0 if there are none.
+uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds )
+{
+  for ( uint64_t t = ( b - 1 ) / TN2; g_tile_rows == 0 && t >= 1; t-- ) {
+    if ( rounds_per_xcd( r, t * TN2 ) <= rounds ) {
+      return t * TN2;
+    }
+  }
+  return 0;
+}
+uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b ) { return rounds_per_xcd( r, b ); }
+
+// The K range of each tile split over several work-groups, the fp32 sums of each split to partial[split].  *splits = 0: not for this
+// shape.  With a single row of tiles a step takes 2 us (the weights are then read for one tile each); the sums are written and read.
+void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns )
 {
   *splits = 0;
   *k_len = 0;
-  const uint64_t tiles = ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 );
-  const uint64_t cus = (uint64_t)cu_count();
-  if ( b < 192 || tiles * 2 > cus || s % TKS != 0 || s >= ( 1u << 22 ) || ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) ) & 15u ) != 0 ) {
+  *ns = 0.0;
+  const uint64_t token_tiles = ( b + TN2 - 1 ) / TN2, tiles = ( ( r + TM2 - 1 ) / TM2 ) * token_tiles;
+  const uint64_t cus = (uint64_t)cu_count(), steps = s / TKS;
+  if ( b < 192 || tiles > 2 * cus || s % TKS != 0 || s >= ( 1u << 22 ) ) {
     return;
   }
-  const uint64_t steps = s / TKS;
-  // Very few tiles and a short K (70B wo at 256 rows: 32 tiles, 8 splits of 16 steps, fp32 sums half the size of the weights):
-  // the ring kernel's smaller tiles need fewer and hide more of a short work-group's start-up (55 against 73 us with the sums).
-  if ( tiles * 8 <= cus && steps <= 128 ) {
-    return;
+  for ( uint64_t want = 2; want <= 16; want++ ) {
+    const uint64_t per = ( steps + want - 1 ) / want, n = ( steps + per - 1 ) / per;
+    if ( per < 12 || n != want ) {
+      continue;
+    }
+    const double cost = rounds_ns( ( tiles * n + cus - 1 ) / cus, tiles * n, per, token_tiles == 1 ? 2000.0 : 0.0 ) + (double)( n * b * r ) * 8.0 / 5000.0;
+    if ( *splits == 0 || cost < *ns ) {
+      *splits = (uint32_t)n;
+      *k_len = (uint32_t)( per * TKS );
+      *ns = cost;
+    }
   }
-  uint64_t n = std::min<uint64_t>( cus / tiles, steps / 16 ); // at least 16 steps of 64 k per split
-  if ( n < 2 ) {
-    return;
-  }
-  const uint64_t steps_per_split = ( steps + n - 1 ) / n;
-  *k_len = (uint32_t)( steps_per_split * TKS );
-  *splits = (uint32_t)( ( steps + steps_per_split - 1 ) / steps_per_split );
 }
 
 // `partial` != nullptr: fp32 sums (splits, b, r) instead of xout; else `epilogue` 0 stores, 1 accumulates into xout (needs r % 8 == 0).
@@ -513,9 +510,9 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   ord.token_tiles = (uint32_t)( ( b + TN2 - 1 ) / TN2 );
   // Whole row tiles per XCD, the weights of each read into one L2 only, where that takes no more rounds of the XCD's 32 CUs than an even
   // share of all tiles (13824 x 5120 at 16384 tokens, 54 row tiles: 14 either way, 1 % faster); else the row tiles beyond a multiple
-  // of 8 are shared out (20 row tiles: 5 rounds against 6).
+  // of 8 are shared out (20 row tiles: 5 rounds against 6; with 4 splits of 3 token tiles 32 work-groups per XCD against 36, 110 us against 149).
   const uint64_t tokens = ord.token_tiles, even = ( row_tiles / 8 ) * tokens + ( ( row_tiles % 8 ) * tokens + 7 ) / 8, whole = ( row_tiles + 7 ) / 8 * tokens;
-  ord.rest_rows = ( whole + 31 ) / 32 <= ( even + 31 ) / 32 ? 0 : row_tiles % 8;
+  ord.rest_rows = ( whole * splits + 31 ) / 32 <= ( even * splits + 31 ) / 32 ? 0 : row_tiles % 8;
   ord.owned = row_tiles - ord.rest_rows;
   // The 32 tiles an XCD works on at a time read gm + gn operand strips into its L2: strips of equal height, at most 6 row tiles, and
   // patches of equal width that make 32 tiles with that (6 x 5: 11 strips; heights of 4 and 2 with patches 8 wide: 12 and 18).

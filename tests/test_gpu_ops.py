@@ -352,6 +352,18 @@ def test_matmul_ring_edges(dt, b, s, r):
     assert ((ops.matmul(x, w).double() - want).abs() <= bound).all()
 
 
+# whole rounds of tiles and a rest with its K range split; K splits over row tiles that are no multiple of the XCDs; several slabs of the
+# ring kernel over a long K range (all keep step), over one that ends inside a step; one-hot activations, every output is one weight
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,s,r", [(3328, 3072, 8192), (640, 6144, 5120), (1800, 4096, 4096), (2900, 2304, 4104), (700, 2056, 6152), (1111, 1536, 2050)])
+def test_matmul_rounds_and_rests_one_hot(dt, b, s, r):
+    w = torch.arange(r * s, dtype=torch.float32, device="cuda").reshape(r, s).remainder(251).to(dt)
+    x = torch.zeros((b, s), dtype=dt, device="cuda")
+    cols = torch.tensor([(7919 * i + 3) % s for i in range(b)], device="cuda")
+    x[torch.arange(b, device="cuda"), cols] = 1
+    assert torch.equal(ops.matmul(x, w), w[:, cols].t().contiguous())
+
+
 # some hundred rows (the decode step of a large slot arena): whatever the dispatcher picks at each batch size (streaming kernel up
 # to 64 rows, 128 x 128 tiles with or without a K split, 256-token tiles with the K range split over work-groups when the tiles are
 # few), ragged edges in rows, tokens and K steps.  One-hot activations: every output is one weight, bit for bit.
