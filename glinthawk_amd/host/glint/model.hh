@@ -387,18 +387,30 @@ public:
     DType* pxb = pf_xb_.get();
     DType* pq = pf_q_.get();
     DType* phb = pf_hb_.get();
-    // Many tokens arriving from and leaving for the host: the rows are cut into four runs, and the copies of a run go over a
-    // stream of their own, so that the first layer's projections of run c (row-wise work: norm, wq, wkv, append, RoPE) overlap the
-    // upload of run c + 1 and the download of run c overlaps the last layer's w2 product of run c + 1.  Everything in between
-    // (attention needs all rows of a context) runs on all rows at once.
-    const bool pipelined = n >= 8192 && !( first_layer == 0 && token_ids != nullptr ) && ( acts_in_host != nullptr );
+    // Many tokens arriving from and leaving for the host: the rows are cut into runs, and the copies of a run go over a stream of their
+    // own, so that the first layer's projections of a run (row-wise work: norm, wq, wkv, append, RoPE) overlap the upload of the next,
+    // and the last layer's feed-forward of a run overlaps the download of the one before.  Everything in between (attention needs all
+    // rows of a context) runs on all rows at once.  What stays exposed is the first layer's work on the last run and that run's
+    // download, so the runs get shorter (70B, 3328 tokens, 2 layers: 9.73 ms as 2048 + 768 + 512, 10.93 in one; 13B, 14000 tokens,
+    // 4 layers: 31.2 and 35.2); below 1024 tokens a copy is shorter than what the cuts cost.
+    const bool pipelined = n >= 1024 && !( first_layer == 0 && token_ids != nullptr ) && ( acts_in_host != nullptr );
     std::vector<std::pair<uint64_t, uint64_t>> chunks; // (first row, rows)
     if ( pipelined ) {
       ensure_copy_stream();
-      const uint64_t per = ( ( n + N_CHUNKS - 1 ) / N_CHUNKS + 255 ) / 256 * 256;
-      for ( uint64_t r0 = 0; r0 < n; r0 += per ) {
-        chunks.emplace_back( r0, std::min( per, n - r0 ) );
+      // A run's download may take as long as the next run's feed-forward: about 3 x hidden_dim multiply-adds a value at 650 T/s against
+      // 2 bytes at 55 GB/s, so each run is that much shorter than the one before.
+      const double rate = 3.0 * Config::hidden_dim * 55e9 / ( 650e12 * sizeof( DType ) );
+      const double part = std::clamp( 1.0 - 1.0 / rate, 0.3, 0.6 );
+      uint64_t r0 = 0;
+      while ( n - r0 > std::max<uint64_t>( 768, n / 8 ) && chunks.size() + 1 < N_CHUNKS ) {
+        const uint64_t rows = std::max<uint64_t>( 1, static_cast<uint64_t>( part * static_cast<double>( n - r0 ) / 256.0 + 0.5 ) ) * 256; // whole tiles
+        if ( r0 + rows >= n ) {
+          break;
+        }
+        chunks.emplace_back( r0, rows );
+        r0 += rows;
       }
+      chunks.emplace_back( r0, n - r0 );
     } else {
       chunks.emplace_back( 0, n );
     }
@@ -431,8 +443,8 @@ public:
       const auto& w = layers_[run[k]];
       // one table entry per (context, token) for this layer's rows
       GLINT_GH( gh_prefill_tables( layer_rows_dev( k ), pos_dev(), batch, n_tokens, row_bytes, nullptr, pf_token_rows(), pf_pos(), ops_.stream() ) );
-      if ( n < 128 ) {
-        // few tokens: the weight-streaming GEMM with fused follow-up ops, as in decode
+      if ( n <= PREFILL_FUSED_ROWS ) {
+        // few tokens: products bound by their weights, with the follow-up ops fused, as in decode
         ops_.matmul_qkv_rope_append( pq, pxb, w.wq, n, pf_pos(), base_.freq_cis_real, base_.freq_cis_imag, pf_token_rows() );
         GLINT_GH( gh_attn_prefill( pq, layer_rows_dev( k ), pos_dev(), pxb, batch, n_tokens, max_start, &shape, hip::gh_type<DType>(), pf_attn_ws_.get(),
                                    pf_attn_ws_bytes_, GH_ATTN_AUTO, ops_.stream() ) );
@@ -476,17 +488,22 @@ public:
           ops_.template accum<Config::dim>( px, pxb2, n );
           ops_.template rmsnorm<Config::dim>( pxb, px, reinterpret_cast<float32_t*>( temp_ ), w.rms_ffn_weight, n );
         }
-        ops_.template matmul<Config::dim, Config::hidden_dim>( phb, pxb, w.w1, n );
-        ops_.template matmul<Config::dim, Config::hidden_dim>( phb2, pxb, w.w3, n );
-        ops_.template silu<Config::hidden_dim>( phb, phb2, n );
         const DType* next_norm = k + 1 < run.size() ? layers_[run[k + 1]].rms_att_weight : nullptr;
-        // the last product of the call run by run when its result leaves for the host, each run's download behind it
+        // the feed-forward of the last layer run by run when its result leaves for the host, each run's download behind it
         const bool out_by_run = pipelined && k + 1 == run.size() && acts_out_host != nullptr;
         for ( size_t c = 0; c < ( out_by_run ? chunks.size() : 1 ); c++ ) {
           const uint64_t r0 = out_by_run ? chunks[c].first : 0, rows = out_by_run ? chunks[c].second : n;
           DType* cx = px + r0 * Config::dim;
           DType* cxb = pxb + r0 * Config::dim;
-          const DType* chb = phb + r0 * Config::hidden_dim;
+          DType* chb = phb + r0 * Config::hidden_dim;
+          DType* chb2 = phb2 + r0 * Config::hidden_dim;
+          if ( rows <= 65535 && w.w3 == w.w1 + (uint64_t)Config::dim * Config::hidden_dim ) { // w3 lies behind w1: one launch, and the gate with it
+            ops_.matmul_silu_gate( chb, cxb, w.w1, rows );
+          } else {
+            ops_.template matmul<Config::dim, Config::hidden_dim>( chb, cxb, w.w1, rows );
+            ops_.template matmul<Config::dim, Config::hidden_dim>( chb2, cxb, w.w3, rows );
+            ops_.template silu<Config::hidden_dim>( chb, chb2, rows );
+          }
           // whether the residual add rides in the product's epilogue is a property of the shape, so it is asked per run
           if ( rows <= 65535 && gh_matmul_fuses_many_rows( Config::hidden_dim, Config::dim, rows, hip::gh_type<DType>() ) == 1 ) {
             ops_.template matmul_accum<Config::hidden_dim, Config::dim>( cx, chb, w.w2, rows, next_norm ? cxb : nullptr, next_norm );
@@ -971,8 +988,11 @@ private:
     pf_attn_ws_ = ops_.device_allocate( std::max<uint64_t>( pf_attn_ws_bytes_, 16 ) );
     pf_capacity_ = n;
   }
+  // Tokens up to which a prefill's products carry their follow-up ops: the ring kernel takes them at once and the fp32 sums stay small
+  // (70B, 132 tokens, 2 layers: 983 us, as separate ops 1056; 7B, 150 tokens, 4 layers: 746 and 952).
+  static constexpr uint64_t PREFILL_FUSED_ROWS = 256;
   // the stream and events of the pipelined prefill, created on first use and kept for the life of the model
-  static constexpr size_t N_CHUNKS = 4;
+  static constexpr size_t N_CHUNKS = 8;
   struct CopyLane
   {
     gh_stream stream { nullptr };

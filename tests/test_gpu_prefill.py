@@ -297,6 +297,28 @@ def test_stage_prefill_copies_overlapped_with_compute_equal_plain_call():
     b.close()
 
 
+@pytest.mark.parametrize("hosted,batch,T", [(1, 2, 550),      # one layer, the first and the last at once; a last run that is no multiple of 256
+                                            (2, 4, 257)])     # 1028 tokens: just cut
+def test_stage_prefill_short_runs_equal_plain_calls(hosted, batch, T):
+    """A call whose rows are cut into runs of falling length against calls of one context each, too short to be cut: the same outputs
+    but for the order of fp32 sums (the products are split differently), so to a rounding of f16 here and there."""
+    first, dim = 8, 4096
+    a, b = (S.Stage("llama2-7b", "f16", first, hosted, batch, batch, seed=3, weight_std=0.02) for _ in range(2))
+    x, y = ops.pinned_empty((batch * T, dim), np.float16), ops.pinned_empty((batch * T, dim), np.float16)
+    x[:] = np.random.default_rng(6).standard_normal(x.shape).astype(np.float16)
+    ids = [40 + i for i in range(batch)]
+    assert a.prefill(ids, [0] * batch, T, first, activations=x, out=y) is not None
+    want = np.zeros_like(y)
+    for i in range(batch):
+        rows = slice(i * T, (i + 1) * T)
+        assert b.prefill(ids[i:i + 1], [0], T, first, activations=x[rows], out=want[rows]) is not None
+    assert np.all(np.isfinite(y.astype(np.float32)))
+    assert (y.view(np.uint16) != want.view(np.uint16)).mean() < 0.05
+    np.testing.assert_allclose(y.astype(np.float32), want.astype(np.float32), rtol=4e-3, atol=4e-3)
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("shape", [MHA, GQA4], ids=["mha", "gqa4"])
 def test_prefill_one_key_stands_out(shape):
     """A key whose score lies far above all others, at each place of a 16-key group in turn: whichever lane of the wave holds it, the
