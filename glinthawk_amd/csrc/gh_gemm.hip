@@ -35,7 +35,7 @@ bool gemm_tile256_fills( uint64_t r, uint64_t b );
 double gemm_tile256_ns( uint64_t s, uint64_t r, uint64_t b );
 template<typename E>
 int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, int epilogue, hipStream_t st,
-                         uint32_t splits, uint32_t k_len, E* xout2 = nullptr, uint64_t r_first = 0 );
+                         uint32_t splits, uint32_t k_len, E* xout2 = nullptr, uint64_t r_first = 0, const GateRows* gate = nullptr );
 uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b );
 uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds );
 void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns );
@@ -312,6 +312,8 @@ static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, c
   return g_force_kernel == 4 ? gemm_tile256_fills( r, b ) : g_force_kernel == 0 && gemm_tile256_ns( s, r, b ) <= other_tiles_ns( s, r, b );
 }
 
+uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
+
 int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
                           bool* done )
 {
@@ -319,15 +321,34 @@ int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const v
   if ( !is_half_type( dt ) ) {
     return GH_OK;
   }
+  const bool plain_silu = gate.activation == GH_ACT_SILU && gate.bias == nullptr;
+  if ( !plain_silu && b >= 192 ) { // the tiles' epilogue has no room for it
+    return GH_OK;
+  }
   const bool stream = ( g_force_kernel == 2 || ( g_force_kernel == 0 && gemm_stream_gate_waves() != 0 ) ) && b <= 64
+                      && plain_silu
                       && gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
-  // From 192 rows on the 256-token tiles with the gate's kernel behind them, where they are enough (70B, 256 rows: 235 us, here 264);
-  // the vendor's library where it is asked for.  An exact caller's other route there is one product with the matrices next to w13.
-  const bool others = b >= 192 && ( gate.exact || tile256_wanted( s, 2 * hidden, b, x, w13, hb ) );
   const bool library = b > 64 && ( gemm_library_wanted_wide( s, 2 * hidden, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden, b, dt, x, w13, hb ) );
-  const bool ring = !stream && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) && !others && !library
+  const bool takes_tiles = !stream && !library && gate.stride % 8 == 0 && hidden % 8 == 0;
+  if ( takes_tiles && gate.context_rows == nullptr ) { // (rows of contexts are counted from the first)
+    if ( const uint64_t b1 = gemm_token_split( s, 2 * hidden, b, dt, x, w13, hb ) ) {
+      char* rest = static_cast<char*>( hb ) + b1 * gate.stride * 2;
+      const char* rest_x = static_cast<const char*>( x ) + b1 * s * 2;
+      if ( gemm_ring_gate_applicable( s, hidden, b - b1, rest_x, w13, rest, gate.stride ) || tile256_wanted( s, 2 * hidden, b - b1, rest_x, w13, rest ) ) {
+        if ( int rc = gemm_gate_one_launch( hb, gate, x, w13, s, hidden, b1, dt, st, done ) ) {
+          return rc;
+        }
+        if ( *done ) {
+          return gemm_gate_one_launch( rest, gate, rest_x, w13, s, hidden, b - b1, dt, st, done );
+        }
+      }
+    }
+  }
+  // From 192 rows on the 256 x 256 tiles where they are enough (70B, 256 rows: 235 us with the gate behind them, the ring kernel 264).
+  const bool tiles = takes_tiles && tile256_wanted( s, 2 * hidden, b, x, w13, hb );
+  const bool ring = !stream && !tiles && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) && !library
                     && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
-  if ( !stream && !ring ) {
+  if ( !stream && !ring && !tiles ) {
     return GH_OK;
   }
   *done = true;
@@ -335,8 +356,9 @@ int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const v
     using E = std::remove_pointer_t<decltype( e )>;
     E* out = static_cast<E*>( hb );
     const E *in = static_cast<const E*>( x ), *mat = static_cast<const E*>( w13 );
-    return stream ? gemm_stream_gate_launch<E>( out, gate.stride, in, mat, s, hidden, b, st )
-                  : gemm_ring_gate_launch<E>( out, gate, in, mat, s, hidden, b, st );
+    return stream  ? gemm_stream_gate_launch<E>( out, gate.stride, in, mat, s, hidden, b, st )
+           : tiles ? gemm_tile256_launch<E>( out, nullptr, in, mat, s, hidden, b, 2, st, 1, 0, nullptr, 0, &gate )
+                   : gemm_ring_gate_launch<E>( out, gate, in, mat, s, hidden, b, st );
   } );
 }
 

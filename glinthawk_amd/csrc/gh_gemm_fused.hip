@@ -555,13 +555,8 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
       return GH_OK;
     }
   }
-  // Some hundred rows and more with enough tiles for the large tile kernel: both factors in one launch of it, stored as DType whole
-  // row segments (the second factor into a scratch buffer), then the gate as the element-wise kernel.  The fp32 sums that the
-  // route below leaves for its gate kernel are stored from the accumulator registers, 16 bytes to each of 32 lines per
-  // instruction, and are twice the bytes (256 rows of the 70B shape: 224 + 9 us here; with sums 20 + 7 us more).  Same roundings either way
-  // (each factor to DType, then the gate).
-  if ( dt == GH_F16 && hidden_dim % 8 == 0
-       && ( gemm_tile_epilogue_applicable( s, 2 * hidden_dim, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden_dim, b, dt, x, w13, hb ) ) ) {
+  // the factors as two products of the vendor's library, then the gate; the same roundings
+  if ( hidden_dim % 8 == 0 && gemm_library_wanted( s, hidden_dim, b, dt, x, w13, hb ) ) {
     void* factor = nullptr;
     if ( int rc = stream_scratch( st, SCRATCH_GATE_FACTOR, b * hidden_dim * sizeof( __half ), 16ull << 20, &factor ) ) {
       return rc;

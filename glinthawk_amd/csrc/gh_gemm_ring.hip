@@ -213,9 +213,7 @@ __global__ __launch_bounds__( RING_THREADS, 1 ) void gemm_ring_kernel( void* __r
         } y;
 #pragma unroll
         for ( int v = 0; v < 4; v++ ) {
-          const float y1 = gate.exact ? acc[i][c][v] : to_f32<E>( from_f32<E>( acc[i][c][v] ) );
-          const float y3 = gate.exact ? acc[i + 1][c][v] : to_f32<E>( from_f32<E>( acc[i + 1][c][v] ) );
-          y.h[v] = from_f32<E>( y1 / ( 1.0f + __expf( -y1 ) ) * y3 );
+          y.h[v] = gated<E>( gate, acc[i][c][v], acc[i + 1][c][v], min( first + row + v, r - 1 ), r );
         }
         if ( row < n_rows ) { // r % 4 == 0: all four
           *reinterpret_cast<uint2*>( static_cast<E*>( out ) + ( col0 + col ) * gate.stride + first + row ) = y.raw;

@@ -27,7 +27,7 @@
 //               (1.14), 8192 x 28672 at 3328 (1.6 rounds) 1.33 (1.13).  Of that: reads in front of the loads of a part 1 %; tile after
 //               tile without draining 1-2 %; the output's addresses once a tile instead of once a store 3 %.  Not kept: raised wave
 //               priority around the MFMAs (-2 %), the loads between the MFMAs (-3 %), four loads in either phase instead of 2 and 6 (0).
-#include "gh_common.h"
+#include "gh_product.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -82,16 +82,19 @@ __device__ __forceinline__ bool tile_of_index( const TileOrder& ord, uint32_t xc
 
 // What a work-group does with its sums: xout = DType(sum); the reference's next op on top of that,
 // xout = DType(float(xout) + float(DType(sum))) (accum; only with r % 8 == 0); or the fp32 sums, (splits, b, r).
-// (The SiLU gate was tried here as well: with one work-group per CU nothing hides the epilogue's
-// divisions and exponentials, and the separate element-wise kernel is faster.)
-constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_PARTIAL = 3;
+// Or the SiLU gate over two products, w = [w1 rows | w3 rows], as GateRows says (gh_product.h), without a bias: a tile is 128 rows of w1 and the same 128 of
+// w3, whose sums a lane holds side by side; half as many stores, and no kernel that reads both factors
+// again (13B, 16384 tokens: 271 us a layer; the pass of four 36.9 -> 35.5 ms).  With one work-group per CU nothing hides the epilogue, so a
+// gate that takes longer stays a kernel of its own (tanh and biases here, 8192 rows of 2 x 11008: 2 % of the pass slower).
+constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3;
 
 struct TileOut
 {
   void* xout;      // rows [0, r_first), a (b, r_first) matrix
   void* xout2;     // rows from r_first on, as rows 0.. of a (b, r - r_first) matrix; r_first == r: one output
   float* partial;  // EPI_PARTIAL
-  uint32_t r, b, r_first;
+  uint32_t r, b, r_first; // EPI_GATE: r rows of each factor
+  GateRows gate;
 };
 
 // LDS slot (16 bytes) of a chunk: rows of 8 chunks.  A wave's 16-byte reads are served in four passes of 16 lanes (0-3, 12-15, 20-23, 24-27 first);
@@ -100,7 +103,7 @@ __device__ __forceinline__ uint32_t x_swizzle( uint32_t row ) { return ( row >> 
 __device__ __forceinline__ uint32_t w_swizzle( uint32_t row ) { return ( ( row >> 1 ) & 1 ) | ( ( row >> 2 ) & 6 ); } // rows 8 (m / 4) + m % 4 (+ 4), m < 16
 
 // acc[a][h][i][j][v]: row 128 a + 64 group + 32 (i / 2) + 8 (lane / 16) + 4 (i % 2) + v, token 128 h + 32 wave + 16 j + lane % 16.
-// Returns whether the tile left by exactly 16 stores of this wave behind its last load (not EPI_PARTIAL).
+// Returns whether the tile left by exactly 16 (EPI_GATE: 8) stores of this wave behind its last load (not EPI_PARTIAL).
 template<typename E, int EPI>
 __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2], const TileOut& o, uint32_t tile_row0, uint32_t tile_col0, uint32_t group, uint32_t wave,
                                             uint32_t lane, uint32_t split )
@@ -145,6 +148,31 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
       }
     }
     return false;
+  }
+  if constexpr ( EPI == EPI_GATE ) { // tile_row0: of the output
+    auto values = [&]( int h, int i, int j ) __attribute__( ( always_inline ) ) {
+      Chunk y;
+#pragma unroll
+      for ( int e = 0; e < 8; e++ ) {
+        const float a1 = acc[0][h][2 * i + ( e >> 2 )][j][e & 3], a3 = acc[1][h][2 * i + ( e >> 2 )][j][e & 3];
+        const float y1 = o.gate.exact ? a1 : to_f32<E>( from_f32<E>( a1 ) ), y3 = o.gate.exact ? a3 : to_f32<E>( from_f32<E>( a3 ) );
+        y.h[e] = from_f32<E>( y1 / ( 1.0f + __expf( -y1 ) ) * y3 );
+      }
+      return y;
+    };
+    const bool whole = tile_row0 + TM2 / 2 <= o.r && tile_col0 + TN2 <= o.b && o.gate.context_rows == nullptr;
+    E* base = static_cast<E*>( o.xout ) + (uint64_t)col0 * o.gate.stride + row0;
+#pragma unroll
+    for ( int n = 0; n < 8; n++ ) {
+      const int h = n >> 2, j = ( n >> 1 ) & 1, i = n & 1;
+      const uint32_t col = col0 + 128 * h + 16 * j;
+      const Chunk y = values( h, i, j );
+      if ( whole
+           || ( row0 + 32 * i < o.r && col < o.b && ( o.gate.context_rows == nullptr || o.gate.context_rows[col / o.gate.n_tokens] != nullptr ) ) ) {
+        *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * o.gate.stride + 32 * i ) = y.raw; // r % 8 == 0: eight rows
+      }
+    }
+    return whole;
   }
   // two products that share their activations in one launch: a tile of one of them, or of both
   const bool second = tile_row0 >= o.r_first;
@@ -233,6 +261,8 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
     w_off[i] = ( row + 64 * i ) * ld_bytes + ( slot ^ w_swizzle( row ) ) * 16;
     x_off[i] = ( row + 64 * i ) * ld_bytes + ( slot ^ x_swizzle( row ) ) * 16;
   }
+  constexpr uint32_t ROWS = EPI == EPI_GATE ? TM2 / 2 : TM2; // output rows of a tile
+  const uint64_t w3_bytes = (uint64_t)out.r * ld_bytes;      // EPI_GATE: from a row of w1 to its row of w3
   struct Operands // of a tile: first byte of this split's k range and bytes from there to the end of its last row
   {
     const char *w, *x;
@@ -240,9 +270,9 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   };
   auto operands_of = [&]( uint32_t rt, uint32_t tt ) __attribute__( ( always_inline ) ) {
     Operands p;
-    p.w = reinterpret_cast<const char*>( w + (uint64_t)rt * TM2 * s + k0 );
+    p.w = reinterpret_cast<const char*>( w + (uint64_t)rt * ROWS * s + k0 );
     p.x = reinterpret_cast<const char*>( x + (uint64_t)tt * TN2 * s + k0 );
-    p.w_bytes = min( (uint32_t)TM2, out.r - rt * TM2 ) * ld_bytes - k0 * 2;
+    p.w_bytes = min( ROWS, out.r - rt * ROWS ) * ld_bytes - k0 * 2;
     p.x_bytes = min( (uint32_t)TN2, out.b - tt * TN2 ) * ld_bytes - k0 * 2;
     return p;
   };
@@ -255,10 +285,12 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   };
   auto fetch_w = [&]( uint4* tile, int half, uint32_t step ) __attribute__( ( always_inline ) ) {
     const Operands& p = WALK && step >= n_steps ? next : cur;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<char*>( p.w ), 0, (int)p.w_bytes, 0x00020000 );
+    const char* base = EPI == EPI_GATE && half == 1 ? p.w + w3_bytes : p.w;
+    const int row = EPI == EPI_GATE ? 0 : 2 * half;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<char*>( base ), 0, (int)p.w_bytes, 0x00020000 );
     const uint32_t kb = k_bytes( step );
-    __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + 64 * all_waves ), 16, w_off[2 * half], kb, 0, 0 );
-    __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + 64 * 8 + 64 * all_waves ), 16, w_off[2 * half + 1], kb, 0, 0 );
+    __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + 64 * all_waves ), 16, w_off[row], kb, 0, 0 );
+    __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + 64 * 8 + 64 * all_waves ), 16, w_off[row + 1], kb, 0, 0 );
   };
   auto fetch_x = [&]( uint4* tile, int half, uint32_t step ) __attribute__( ( always_inline ) ) {
     const Operands& p = WALK && step >= n_steps ? next : cur;
@@ -315,7 +347,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   };
   // The end of a memory part: this wave's reads are here, and all of its loads but the youngest 8, which leaves what the next part reads
   // in LDS (the barrier makes that all waves').  `stores`: the last tile's stores are still counted behind the loads this waits for.
-  constexpr int STORES = 16;
+  constexpr int STORES = EPI == EPI_GATE ? 8 : 16;
   auto arrive = [&]( bool stores ) __attribute__( ( always_inline ) ) {
     __builtin_amdgcn_sched_barrier( 0 );
     if ( stores ) {
@@ -380,7 +412,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
       if ( !more ) {
         __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): no load-to-LDS outlives the work-group
       }
-      stores = store_tile<E, EPI>( acc, out, row_tile * TM2, token_tile * TN2, group, wave, lane, 0 );
+      stores = store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, 0 );
       if ( !more ) {
         break;
       }
@@ -398,7 +430,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
       step( s_wa0, s_wb0, s_x0, s_wb1, j, false );
     }
     __builtin_amdgcn_s_waitcnt( 0x0F70 );
-    store_tile<E, EPI>( acc, out, row_tile * TM2, token_tile * TN2, group, wave, lane, blockIdx.y );
+    store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, blockIdx.y );
   }
   if ( group == 0 ) {
     barrier();
@@ -486,11 +518,12 @@ void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* spli
   }
 }
 
-// `partial` != nullptr: fp32 sums (splits, b, r) instead of xout; else `epilogue` 0 stores, 1 accumulates into xout (needs r % 8 == 0).
+// `partial` != nullptr: fp32 sums (splits, b, r) instead of xout; else `epilogue` 0 stores, 1 accumulates into xout (needs r % 8 == 0), 2 gates
+// (2 r weight rows, `gate`).
 // splits > 1 (from gemm_tile256_split_plan, with its k_len) needs `partial`.
 template<typename E>
 int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, int epilogue, hipStream_t st, uint32_t splits,
-                         uint32_t k_len, E* xout2, uint64_t r_first )
+                         uint32_t k_len, E* xout2, uint64_t r_first, const GateRows* gate )
 {
   if ( xout2 == nullptr ) {
     r_first = r;
@@ -503,9 +536,11 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
     k_len = (uint32_t)s;
   }
   const int epi = partial != nullptr ? EPI_PARTIAL : epilogue;
-  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL, "gh_matmul: unknown tile epilogue %d", epi );
+  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL || ( epi == EPI_GATE && gate != nullptr && gate->activation == GH_ACT_SILU && gate->bias == nullptr && r % 8 == 0 && gate->stride % 8 == 0 ),
+              "gh_matmul: unknown tile epilogue %d", epi );
   GH_REQUIRE( epi != EPI_ACCUM || r % 8 == 0, "gh_matmul: the accumulating tile epilogue needs r %% 8 == 0" );
-  const uint32_t row_tiles = (uint32_t)( ( r + TM2 - 1 ) / TM2 );
+  const uint64_t tile_rows = epi == EPI_GATE ? TM2 / 2 : TM2;
+  const uint32_t row_tiles = (uint32_t)( ( r + tile_rows - 1 ) / tile_rows );
   TileOrder ord;
   ord.token_tiles = (uint32_t)( ( b + TN2 - 1 ) / TN2 );
   // Whole row tiles per XCD, the weights of each read into one L2 only, where that takes no more rounds of the XCD's 32 CUs than an even
@@ -523,7 +558,7 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   ord.rest_share = (uint32_t)( ( (uint64_t)ord.rest_rows * tokens + 7 ) / 8 );
   const uint64_t per_xcd = ord.rest_rows == 0 ? whole : even; // the longest list
   GH_REQUIRE( 8 * per_xcd < ( 1ull << 31 ), "gh_matmul: grid too large" );
-  const TileOut out { xout, xout2, partial, (uint32_t)r, (uint32_t)b, (uint32_t)r_first };
+  const TileOut out { xout, xout2, partial, (uint32_t)r, (uint32_t)b, (uint32_t)r_first, gate != nullptr ? *gate : GateRows {} };
   const uint64_t per_cu = std::max<uint64_t>( 1, (uint64_t)cu_count() / 8 );
   const bool walk = per_xcd > per_cu && epi != EPI_PARTIAL && s % ( 2 * TKS ) == 0;
   const dim3 grid( (unsigned)( 8 * ( walk ? per_cu : per_xcd ) ), splits );
@@ -531,6 +566,7 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   switch ( epi ) {
     case EPI_STORE: walk ? GH_TILE256( EPI_STORE, true ) : GH_TILE256( EPI_STORE, false ); break;
     case EPI_ACCUM: walk ? GH_TILE256( EPI_ACCUM, true ) : GH_TILE256( EPI_ACCUM, false ); break;
+    case EPI_GATE: walk ? GH_TILE256( EPI_GATE, true ) : GH_TILE256( EPI_GATE, false ); break;
     default: GH_TILE256( EPI_PARTIAL, false ); break;
   }
 #undef GH_TILE256
@@ -539,8 +575,8 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
 }
 
 template int gemm_tile256_launch<__half>( __half*, float*, const __half*, const __half*, uint64_t, uint64_t, uint64_t, int, hipStream_t, uint32_t, uint32_t,
-                                          __half*, uint64_t );
+                                          __half*, uint64_t, const GateRows* );
 template int gemm_tile256_launch<__bf16>( __bf16*, float*, const __bf16*, const __bf16*, uint64_t, uint64_t, uint64_t, int, hipStream_t, uint32_t, uint32_t,
-                                          __bf16*, uint64_t );
+                                          __bf16*, uint64_t, const GateRows* );
 
 } // namespace gh

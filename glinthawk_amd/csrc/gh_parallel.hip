@@ -251,9 +251,9 @@ int gh_matmul_parallel( void* q, float* head_gates, void* hidden, uint64_t hidde
   const WindowShape s = window_shape( a );
   ParallelCols cols = parallel_cols( a, head_gates != nullptr, ff );
   hipStream_t st = as_stream( stream );
-  if ( ff > 0 && dt == GH_BF16 && activation == GH_ACT_SILU ) {
+  if ( ff > 0 && dt == GH_BF16 ) {
     bool done = false;
-    const GateRows gate { hidden_stride, true, const_cast<const void* const*>( context_rows_dev ), n_tokens };
+    const GateRows gate { hidden_stride, true, const_cast<const void* const*>( context_rows_dev ), n_tokens, activation };
     if ( int rc = gemm_gate_one_launch( hidden, gate, x, static_cast<const __bf16*>( w ) + cols.ff * width, width, ff, rows, dt, st, &done ) ) {
       return rc;
     }

@@ -10,16 +10,44 @@ namespace gh {
 int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, hipStream_t st, bool want_partials,
                    float** partial_out, uint32_t* splits_out );
 
-// Rows of a gated feed-forward that its product stores itself: DType(silu(y1) * y3).
+// Rows of a gated feed-forward that its product stores itself: DType(activation(y1 + bias1) * (y3 + bias3)).
 struct GateRows
 {
   uint64_t stride { 0 };                       // elements from row to row
   bool exact { false };                        // the gate over the fp32 sums; else y1 and y3 rounded to DType first, as two products would leave them
   const void* const* context_rows { nullptr }; // n_tokens rows of each context; those of a context without an entry are not written
   uint32_t n_tokens { 1 };
+  int activation { GH_ACT_SILU };
+  const void* bias { nullptr }; // of DType, for w1's rows then w3's; with it the factors stay fp32 sums
 };
 // w1, w3 and the gate in one launch; *done = false: nothing was launched, the caller takes its other route
 int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st, bool* done );
+
+// activation of a gated feed-forward, for storage type E
+template<typename E>
+__device__ __forceinline__ float activate( float z, int act )
+{
+  if ( act == GH_ACT_GELU_TANH ) {
+    const float u = 0.7978845608028654f * ( z + 0.044715f * z * z * z );
+    // 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)); the fp32 build takes the library's tanh
+    return sizeof( E ) == 4 ? 0.5f * z * ( 1.0f + tanhf( u ) ) : z / ( 1.0f + __expf( -2.0f * u ) );
+  }
+  return z / ( 1.0f + ( sizeof( E ) == 4 ? expf( -z ) : __expf( -z ) ) );
+}
+
+// the stored value of one output, y1 and y3 the fp32 sums of its factors; rows: of each factor
+template<typename E>
+__device__ __forceinline__ E gated( const GateRows& gate, float y1, float y3, uint32_t row, uint32_t rows )
+{
+  if ( !gate.exact ) {
+    y1 = to_f32<E>( from_f32<E>( y1 ) ), y3 = to_f32<E>( from_f32<E>( y3 ) );
+  }
+  if ( gate.bias != nullptr ) {
+    const E* bias = static_cast<const E*>( gate.bias );
+    y1 += to_f32<E>( bias[row] ), y3 += to_f32<E>( bias[rows + row] );
+  }
+  return from_f32<E>( activate<E>( y1, gate.activation ) * y3 );
+}
 
 struct Product
 {
@@ -141,18 +169,6 @@ struct ProductView
     }
   }
 };
-
-// activation of a gated feed-forward, for storage type E
-template<typename E>
-__device__ __forceinline__ float activate( float z, int act )
-{
-  if ( act == GH_ACT_GELU_TANH ) {
-    const float u = 0.7978845608028654f * ( z + 0.044715f * z * z * z );
-    // 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)); the fp32 build takes the library's tanh
-    return sizeof( E ) == 4 ? 0.5f * z * ( 1.0f + tanhf( u ) ) : z / ( 1.0f + __expf( -2.0f * u ) );
-  }
-  return z / ( 1.0f + ( sizeof( E ) == 4 ? expf( -z ) : __expf( -z ) ) );
-}
 
 // run( storage tag, view ): the follow-up kernel of a product, instantiated for bf16 and fp32 storage
 template<typename F>

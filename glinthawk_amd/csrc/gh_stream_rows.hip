@@ -442,6 +442,16 @@ int gh_matmul_gate( void* hb, const void* x, const void* w_gate_up, const void* 
   GH_REQUIRE( dt == GH_BF16 || dt == GH_F32, "gh_matmul_gate: unsupported dtype %d", (int)dt );
   GH_REQUIRE( activation == GH_ACT_SILU || activation == GH_ACT_GELU_TANH, "gh_matmul_gate: unknown activation %d", activation );
   hipStream_t st = as_stream( stream );
+  if ( dt == GH_BF16 ) { // the product stores the gated values itself
+    bool done = false;
+    const GateRows gate { hidden, true, nullptr, 1, activation, bias };
+    if ( int rc = gemm_gate_one_launch( hb, gate, x, w_gate_up, s, hidden, rows, dt, st, &done ) ) {
+      return rc;
+    }
+    if ( done ) {
+      return GH_OK;
+    }
+  }
   Product y;
   if ( int rc = make_product( x, w_gate_up, s, 2 * hidden, rows, dt, false, st, &y ) ) {
     return rc;

@@ -96,6 +96,28 @@ def check_matmul_silu_gate(dt, b, s, hidden, product_route):
     product_route.check(plain + (1 if wide else 0))
 
 
+# the gate in the product's own epilogue: whole 256 x 256 tiles that leave whole and ragged, walked and not, an odd number of steps, a rest
+# of tokens on the ring kernel, and the ring kernel alone with ragged rows and columns
+@pytest.mark.parametrize("activation", [ops.GH_ACT_SILU, ops.GH_ACT_GELU_TANH])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("b,s,hidden", [(4096, 256, 8192), (2300, 576, 4104), (2100, 640, 6152), (300, 4096, 12544), (77, 520, 2052), (200, 512, 16404), (5, 4096, 11008)])
+def test_matmul_gate_in_epilogue(b, s, hidden, bias, activation):
+    """Against 64 bits, bf16.  One rounding of the result, off by 2^-8 of it; from 192 rows on the factors may be rounded as well, before
+    the bias is added: off by 2^-8 of the plain product each, which reaches the output times the other factor (and times the activation's
+    slope, at most 1.13).  1 % for the second order; 1e-3 for fp32 sums and the fast exponential."""
+    g = torch.Generator(device="cuda").manual_seed(b + hidden)
+    x = torch.randn((b, s), generator=g, device="cuda").bfloat16()
+    w = (torch.randn((2 * hidden, s), generator=g, device="cuda") / s ** 0.5).bfloat16()
+    add = torch.randn(2 * hidden, generator=g, device="cuda").bfloat16() if bias else None
+    got = ops.matmul_gate(x, w, add, activation).double()
+    raw = x.double() @ w.double().t()
+    y = raw + (add.double() if bias else 0.0)
+    a, u = y[:, :hidden], y[:, hidden:]
+    act = a * torch.sigmoid(a) if activation == ops.GH_ACT_SILU else torch.nn.functional.gelu(a, approximate="tanh")
+    bound = 1.01 * 2.0 ** -8 * ((act * u).abs() + 1.13 * (raw[:, :hidden] * u).abs() + (act * raw[:, hidden:]).abs()) + 1e-3
+    assert ((got - act * u).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [Shape(dim=32, n_layers=1, n_heads=4, n_kv_heads=2, hidden_dim=48, seq_len=16),
                                    Shape(dim=288, n_layers=1, n_heads=6, n_kv_heads=6, hidden_dim=768, seq_len=256),
