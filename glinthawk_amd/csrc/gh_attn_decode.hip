@@ -128,7 +128,8 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
       s[u] = wave_sum( partial ) * scale_log2e;
       m_new = t0 + u < t_end ? fmaxf( m_new, s[u] ) : m_new;
     }
-    const float alpha = fast_exp2( m - m_new );
+    // A score of -inf weighs 0, also where no finite one came before it (the difference of the two infinities would be NaN).
+    const float alpha = m == -INFINITY ? 0.0f : fast_exp2( m - m_new );
     l *= alpha;
 #pragma unroll
     for ( int k = 0; k < NK; k++ ) {
@@ -137,7 +138,7 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
 #pragma unroll
     for ( int u = 0; u < U; u++ ) {
       if ( t0 + u < t_end ) { // uniform
-        const float p = fast_exp2( s[u] - m_new );
+        const float p = s[u] == -INFINITY ? 0.0f : fast_exp2( s[u] - m_new );
         l += p;
 #pragma unroll
         for ( int k = 0; k < NK; k++ ) {
@@ -173,7 +174,7 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
     }
     for ( int w = 0; w < W; w++ ) {
       if ( t_begin + w * U < t_end ) { // uniform; a wave without keys adds nothing
-        const float f = fast_exp2( s_m[w] - m_all );
+        const float f = s_m[w] == -INFINITY ? 0.0f : fast_exp2( s_m[w] - m_all );
         l += s_l[w] * f;
 #pragma unroll
         for ( int k = 0; k < NK; k++ ) {

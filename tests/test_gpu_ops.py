@@ -784,6 +784,38 @@ def test_fused_generic_head_sizes(dt, contexts, heads, kv_heads, head_size):
         np.testing.assert_allclose(got[live], want[live], rtol=1e-4, atol=2e-5)
 
 
+# scores of -inf: the last key, the only one of a wave; the first; a wave's whole first turn; several waves' keys; all but one; a whole split
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("chunk", [0, 32])
+@pytest.mark.parametrize("heads,kv_heads,head_size", [(6, 3, 48), (3, 1, 72), (3, 3, 256)])
+def test_fused_generic_scores_of_minus_infinity(dt, chunk, heads, kv_heads, head_size):
+    """Such keys weigh nothing, as in a softmax over all of them; a NaN among the scores still reaches the output."""
+    keys = [9, 9, 64, 150, 150, 150, 150]
+    gone = [[8], [0], range(8), range(5, 140), [i for i in range(150) if i != 77], range(32, 64), []]
+    g = torch.Generator(device="cuda").manual_seed(head_size)
+    cache = torch.randn((len(keys), 150, 2, kv_heads, head_size), generator=g, device="cuda").to(dt)
+    q = torch.randn((len(keys), heads, head_size), generator=g, device="cuda").to(dt)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    for i, which in enumerate(gone):
+        cache[i, list(which), 0, :, 0] = -torch.inf
+    cache[6, 100, 0, :, 0] = torch.nan
+    shape = Shape(dim=heads * head_size, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, hidden_dim=64, seq_len=150)
+    out = torch.zeros((len(keys), heads * head_size), dtype=dt, device="cuda")
+    ops.attn_set_chunk(chunk)
+    try:
+        ops.attn_decode(q.flatten(1), ops.row_table([cache[i].data_ptr() for i in range(len(keys))]),
+                        torch.tensor([n - 1 for n in keys], dtype=torch.int32, device="cuda"), out, 149, shape, variant=GH_ATTN_GENERIC)
+    finally:
+        ops.attn_set_chunk(0)
+    assert out[6].isnan().all()
+    for i, n in enumerate(keys[:6]):
+        k, v = (cache[i, :n, part].double().repeat_interleave(heads // kv_heads, 1) for part in (0, 1))
+        want = ((q[i].double() * k).sum(-1) * head_size ** -0.5).softmax(0)[:, :, None].mul(v).sum(0)
+        # fp32 sums of at most 256 terms of about 1; the stored value's own rounding
+        bound = 2e-5 + want.abs() * (2.0 ** -11 if dt == torch.float16 else 0.0)
+        assert ((out[i].view(heads, head_size).double() - want).abs() <= bound).all(), i
+
+
 @pytest.mark.parametrize("shape", [MHA128, MHA128_ODD, GQA2, GQA4, GQA8], ids=["mha", "mha6", "gqa2", "gqa4", "gqa8"])
 @pytest.mark.parametrize("chunk", [0, 16, 80, 256])
 def test_fused_valu(shape, chunk):
