@@ -447,7 +447,10 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   GH_REQUIRE( residual != nullptr, "gh_matmul_accum: NULL residual" );
   GH_REQUIRE( ( norm_out == nullptr ) == ( norm_weight == nullptr ), "gh_matmul_accum: norm_out and norm_weight go together" );
   hipStream_t st = as_stream( stream );
-  if ( dt == GH_F32 ) {
+  // gh_rmsnorm takes 16-byte aligned buffers only: other ones go through fp32 sums and the row kernel, which reads them element by element
+  const bool norm_kernel = norm_out == nullptr
+                           || ( ( reinterpret_cast<uintptr_t>( residual ) | reinterpret_cast<uintptr_t>( norm_out ) | reinterpret_cast<uintptr_t>( norm_weight ) ) & 15u ) == 0;
+  if ( dt == GH_F32 && norm_kernel ) {
     if ( int rc = gemm_f32_accum( static_cast<float*>( residual ), static_cast<const float*>( x ), static_cast<const float*>( w ), s, r, b, st ) ) {
       return rc;
     }
@@ -490,8 +493,10 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   // many rows: the residual is added in the tile kernel's epilogue, no fp32 partials;
   // the norm of the new residual, when asked for, is the plain row kernel
   done = false;
-  if ( int rc = gemm_tile_epilogue_launch( residual, x, w, s, r, b, dt, 1, st, &done ) ) {
-    return rc;
+  if ( norm_kernel ) {
+    if ( int rc = gemm_tile_epilogue_launch( residual, x, w, s, r, b, dt, 1, st, &done ) ) {
+      return rc;
+    }
   }
   if ( done ) {
     return norm_out != nullptr ? gh_rmsnorm( norm_out, residual, norm_weight, r, b, dt, stream ) : GH_OK;
@@ -505,9 +510,12 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   if ( dt == GH_F16 && r % 4 == 0 && r <= 2 * 4 * EPI_THREADS && rows_8byte ) {
     epi_accum_norm_row8k_kernel<<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<__half*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
                                                                      static_cast<__half*>( norm_out ), static_cast<const __half*>( norm_weight ) );
-  } else {
+  } else if ( dt == GH_F16 ) {
     epi_accum_norm_kernel<__half><<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<__half*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
                                                                static_cast<__half*>( norm_out ), static_cast<const __half*>( norm_weight ) );
+  } else {
+    epi_accum_norm_kernel<float><<<(unsigned)b, EPI_THREADS, 0, st>>>( static_cast<float*>( residual ), partial, (uint32_t)r, (uint32_t)b, splits,
+                                                              static_cast<float*>( norm_out ), static_cast<const float*>( norm_weight ) );
   }
   GH_LAUNCH_CHECK();
   return GH_OK;

@@ -52,6 +52,32 @@ def test_matmul_accum_and_norm(dt, b, s, r, product_route):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("b,s,r", [(4, 288, 288), (3, 100, 37), (70, 512, 1000),
+                                   (2048, 512, 6152)])          # f16: enough tiles for the residual add in the tile kernel's epilogue
+@pytest.mark.parametrize("at", ["residual", "norm_out", "norm_weight"])
+def test_matmul_accum_norm_of_unaligned_rows(dt, b, s, r, at):
+    """A buffer that starts one element past a 16-byte boundary gives what aligned ones give, up to the order of the norm's sum."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn((b, s), generator=g, device="cuda").to(dt)
+    w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+    res = torch.randn((b, r), generator=g, device="cuda").to(dt)
+    nw = (1 + 0.1 * torch.randn(r, generator=g, device="cuda")).to(dt)
+
+    def place(t, shifted):
+        buffer = torch.zeros(t.numel() + 1, dtype=dt, device="cuda")
+        view = buffer[1:] if shifted else buffer[:-1]
+        return view.view(t.shape).copy_(t)
+
+    want_res = res.clone()
+    want_norm = ops.matmul_accum(want_res, x, w, nw)
+    got_res, got_norm, weight = place(res, at == "residual"), place(torch.zeros_like(res), at == "norm_out"), place(nw, at == "norm_weight")
+    _lib.check(_lib.lib().gh_matmul_accum(ops._p(got_res), ops._p(x), ops._p(w), s, r, b, ops._p(got_norm), ops._p(weight), ops._dt(x), ops._stream()))
+    tol = 2e-3 if dt == torch.float16 else 3e-6
+    assert torch.allclose(got_res.float(), want_res.float(), rtol=tol, atol=tol)
+    assert torch.allclose(got_norm.float(), want_norm.float(), rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
                                         # enough row tiles for one launch without a K split: both factors in one kernel
                                         (64, 512, 16384), (5, 256, 16404), (33, 1024, 28672),
