@@ -49,6 +49,7 @@ bool gemm_ring_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const v
 template<typename E>
 int gemm_ring_gate_launch( E* hb, const GateRows& gate, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
 void gemm_ring_tuning( int target_wgs );
+int gemm_ring_cut( uint64_t s, uint64_t r, uint64_t b, bool gate, uint32_t* plan );
 // fp32 (gh_gemm_f32.hip)
 int gemm_f32( float* out, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 
@@ -615,6 +616,15 @@ int gh_gemm_stream_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, u
   GH_REQUIRE( s >= 256 && s % 256 == 0 && r > 0 && b > 0, "gh_gemm_stream_plan: the streaming kernel takes s %% 256 == 0, r > 0, b > 0" );
   gemm_stream_plan( s, r, b, splits, k_per_split, rows_per_workgroup );
   return GH_OK;
+}
+
+int gh_gemm_ring_plan( uint64_t s, uint64_t r, uint64_t b, int gated, uint32_t* plan )
+{
+  static const char aligned[16] __attribute__( ( aligned( 16 ) ) ) = { 0 };
+  GH_REQUIRE( plan != nullptr, "gh_gemm_ring_plan: NULL output" );
+  GH_REQUIRE( s > 0 && r > 0 && b > 0 && gemm_ring_applicable( s, gated ? 2 * r : r, b, aligned, aligned, aligned ) && ( !gated || r % 4 == 0 ),
+              "gh_gemm_ring_plan: the ring kernel takes s %% 8 == 0 up to 2^21, r > 0 (a multiple of 4 with the gate), b > 0" );
+  return gemm_ring_cut( s, r, b, gated != 0, plan );
 }
 
 int gh_matmul_pair( void* xout_a, void* xout_b, const void* x, const void* w, uint64_t s, uint64_t r_a, uint64_t r_b, uint64_t b, gh_dtype dt,

@@ -22,6 +22,7 @@
 #include "gh_product.h"
 
 #include <algorithm>
+#include <iterator>
 #include <type_traits>
 
 namespace gh {
@@ -322,15 +323,14 @@ int g_ring_cus = 0; // tuning override of the CU count the plan balances for (0:
 // less than a load's time in flight (1.9 us) over the steps requested ahead.  With several slabs the weights come from L2 and the
 // matrix units set the pace; wide slabs slow each other down.  A round costs what it takes to fill the ring, and a split the fp32 sums
 // that are written and read again.
-RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
+RingPlan find_ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate, uint64_t n_cu )
 {
   constexpr uint32_t XS[] = { 32, 64, 96, 128, 192, 256 };
-  const uint64_t n_cu = g_ring_cus > 0 ? (uint64_t)g_ring_cus : (uint64_t)cu_count();
   const uint64_t steps = ( s + RING_K - 1 ) / RING_K;
   RingPlan best {};
   for ( uint32_t x : XS ) {
-    if ( b <= 256 ? x < b : x < 128 ) {
-      continue; // up to 256 activation rows: the narrowest tile that takes them at once
+    if ( b <= 256 ? x < b || best.w != 0 : x < 128 ) {
+      continue; // up to 256 activation rows: the narrowest tile that takes them at once (a wider one has no more stages)
     }
     const uint64_t slabs = ( b + x - 1 ) / x, cols = ( ( b + slabs - 1 ) / slabs + 15 ) / 16 * 16;
     for ( uint32_t w = 128; w <= ( x <= 128 ? 256u : 128u ); w += 128 ) {
@@ -360,6 +360,27 @@ RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
     }
   }
   return best;
+}
+
+// The plan of a product, asked for by the dispatch and again by the launch, and of the same products in every layer and step: the search
+// (1 us up to 256 rows, 1.8 beyond) runs only when another product of this thread took the slot in between.  With a search at every call, of
+// all widths (5 to 7 us up to 64 rows), the host needed 17 us for a product of 8 rows, 13 so.
+RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
+{
+  struct Slot
+  {
+    uint64_t s, r, b, n_cu;
+    bool gate;
+    RingPlan plan;
+  };
+  static thread_local Slot slots[64] {};
+  const uint64_t n_cu = g_ring_cus > 0 ? (uint64_t)g_ring_cus : (uint64_t)cu_count();
+  const uint64_t mixed = ( ( s * 31 + r ) * 31 + b ) * 2 + ( gate ? 1 : 0 );
+  Slot& slot = slots[( mixed * 0x9e3779b97f4a7c15ull ) >> 58];
+  if ( slot.s != s || slot.r != r || slot.b != b || slot.n_cu != n_cu || slot.gate != gate ) { // (s > 0: an empty slot is no product's)
+    slot = Slot { s, r, b, n_cu, gate, find_ring_plan( s, r, b, gate, n_cu ) };
+  }
+  return slot.plan;
 }
 
 } // namespace
@@ -406,6 +427,14 @@ void gemm_ring_tuning( int target_wgs )
   if ( target_wgs > 0 ) {
     g_ring_cus = target_wgs;
   }
+}
+
+int gemm_ring_cut( uint64_t s, uint64_t r, uint64_t b, bool gate, uint32_t* plan )
+{
+  const RingPlan p = ring_plan( s, r, b, gate );
+  const uint32_t out[] = { p.w, p.x, p.cut.rows, p.cut.cols, p.cut.splits, p.cut.steps };
+  std::copy( std::begin( out ), std::end( out ), plan );
+  return GH_OK;
 }
 
 template int gemm_ring_launch<__half>( __half*, float*, const __half*, const __half*, uint64_t, uint64_t, uint64_t, hipStream_t );

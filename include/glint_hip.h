@@ -176,6 +176,9 @@ int gh_matmul_fuses_many_rows( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
 /* host-only query: how the weight-streaming kernel would cut an (r x s) . (b x s)^T product for the initialised device (256 compute
  * units before initialisation): number of K ranges, k per range (a multiple of 256), weight rows per work-group */
 int gh_gemm_stream_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_per_split, uint32_t* rows_per_workgroup );
+/* host-only query: how the ring kernel would cut a product, or with `gated` one of r rows of w1 and r of w3: weight rows and activation rows of the tile,
+ * (output) rows and activation rows of a work-group, K ranges, 64-k steps of a range */
+int gh_gemm_ring_plan( uint64_t s, uint64_t r, uint64_t b, int gated, uint32_t plan[6] );
 int gh_matmul( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, gh_stream stream );
 /* Two products that share their activations, their weights one behind the other ((r_a + r_b, s) row-major, as the reference lays out
  * wq and wkv, models/llama2/base.hh:410-433): xout_a = x . w[0:r_a]^T (b, r_a), xout_b = x . w[r_a:]^T (b, r_b).  The same results as

@@ -1,7 +1,8 @@
-"""The weight-streaming GEMM's plan (K split and row tile) is host logic: properties every plan must
-have, and the plans of the shapes the benchmark configurations use (256 compute units, the value
-the library assumes before a device is initialised)."""
+"""The GEMM kernels' plans are host logic: properties every plan must have, and the plans of the shapes the benchmark configurations use
+(256 compute units, the value the library assumes before a device is initialised).  gh_gemm_ring_plan is of the kernel that products of up
+to some hundred rows run on, gh_gemm_stream_plan of the one that runs on request."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -45,3 +46,68 @@ def test_rejects_what_the_kernel_does_not_take():
     splits, kps, rows = C.c_uint32(0), C.c_uint32(0), C.c_uint32(0)
     rc = _lib.lib().gh_gemm_stream_plan(100, 64, 1, C.byref(splits), C.byref(kps), C.byref(rows))
     assert rc != 0 and b"256" in _lib.lib().gh_last_error()
+
+
+def ring_plan(s, r, b, gated=False):
+    out = (C.c_uint32 * 6)()
+    _lib.check(_lib.lib().gh_gemm_ring_plan(s, r, b, int(gated), out))
+    return tuple(out)
+
+
+def some_shapes(n, seed):
+    rng = np.random.default_rng(seed)
+    size = lambda lo, hi: int(np.exp(rng.uniform(np.log(lo), np.log(hi))))
+    return [(8 * size(1, 4000), 4 * size(1, 20000), size(1, 3000 if i % 3 else 70), bool(i % 2)) for i in range(n)]
+
+
+def test_every_ring_plan_covers_the_product_once():
+    for s, r, b, gated in [(8, 1, 1, False), (8, 4, 1, True), (1 << 21, 128, 3, False), (288, 32000, 7000, False)] + some_shapes(500, 6):
+        w, x, rows, cols, splits, steps = ring_plan(s, r, b, gated)
+        assert (w, x) in [(128, 32), (256, 32), (128, 64), (256, 64), (128, 96), (256, 96), (128, 128), (256, 128), (128, 192), (128, 256)]
+        assert rows % 4 == 0 and 16 <= rows <= (w // 2 if gated else w) and 1 <= cols <= x and (b > 256 or x >= b)
+        total = -(-s // 64)
+        assert 1 <= splits <= 16 and steps * (splits - 1) < total <= steps * splits      # no empty range, nothing left over
+        assert splits == 1 or (steps >= 4 and not gated)
+        assert -(-b // cols) * cols >= b and (cols % 16 == 0 or cols >= b)
+
+
+@pytest.mark.parametrize("name,s,r,b,gated,want", [
+    ("70B wo", 8192, 8192, 64, False, (128, 64, 128, 64, 4, 32)),
+    ("70B w2", 28672, 8192, 64, False, (256, 64, 256, 64, 8, 56)),
+    ("70B w1 and w3", 8192, 28672, 64, True, (256, 64, 112, 64, 1, 128)),
+    ("7B wq and wkv", 4096, 12288, 32, False, (128, 32, 96, 32, 2, 32)),
+    ("7B w1 and w3, a prompt", 4096, 11008, 77, True, (128, 96, 44, 80, 1, 64)),
+])
+def test_ring_plans_of_the_benchmark_shapes(name, s, r, b, gated, want):
+    assert ring_plan(s, r, b, gated) == want, name
+
+
+def test_a_kept_ring_plan_is_that_of_its_product():
+    """More shapes than a thread keeps plans of, asked for again and again, from several threads, and with the units to balance for changed in
+    between: every answer is the first one's."""
+    shapes = some_shapes(400, 7)
+    first = [ring_plan(*c) for c in shapes]
+    wrong = []
+
+    def ask():
+        for _ in range(3):
+            wrong.extend(c for c, want in zip(shapes, first) if ring_plan(*c) != want)
+
+    threads = [threading.Thread(target=ask) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    try:
+        _lib.check(_lib.lib().gh_gemm_set_tuning(0, 64, 0))
+        assert sum(ring_plan(*c) != want for c, want in zip(shapes, first)) > 100
+    finally:
+        _lib.check(_lib.lib().gh_gemm_set_tuning(0, 256, 0))
+    assert [ring_plan(*c) for c in shapes] == first
+
+
+def test_ring_plan_rejects_what_the_kernel_does_not_take():
+    out = (C.c_uint32 * 6)()
+    for s, r, b, gated in [(100, 64, 1, 0), ((1 << 21) + 8, 64, 1, 0), (64, 0, 1, 0), (64, 64, 0, 0), (64, 66, 1, 1)]:
+        assert _lib.lib().gh_gemm_ring_plan(s, r, b, gated, out) != 0 and b"ring" in _lib.lib().gh_last_error()
