@@ -89,7 +89,7 @@ def build_tools() -> list[str]:
 
 
 # kernels of the run-time sized designs and what they stand on: all that the trace runner needs
-TRACE_KERNELS = ("gh_runtime", "gh_elementwise", "gh_gemm", "gh_gemm_f32", "gh_gemm_lib", "gh_gemm_ring", "gh_gemm_stream", "gh_gemm_tile256",
+TRACE_KERNELS = ("gh_runtime", "gh_elementwise", "gh_gemm", "gh_gemm_f32", "gh_gemm_lib", "gh_gemm_ring", "gh_gemm_stream", "gh_gemm_tile", "gh_gemm_tile256",
                  "gh_stream_rows", "gh_attn_window", "gh_parallel", "gh_mlstm")
 
 

@@ -40,11 +40,18 @@ uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b );
 uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds );
 void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns );
 void gemm_tile256_tuning( int rows );
+// 128 x 128 tiles, two work-groups a CU (gh_gemm_tile.hip)
+bool gemm_tile_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
+void gemm_tile_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits_out, uint32_t* k_per_split_out );
+double gemm_tile_ns( uint64_t s, uint64_t r, uint64_t b );
+template<typename E>
+int gemm_tile_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, uint32_t splits, uint32_t k_per_split, hipStream_t st );
 // up to some hundred rows (gh_gemm_ring.hip)
 bool gemm_ring_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout );
 uint32_t gemm_ring_splits( uint64_t s, uint64_t r, uint64_t b, double* ns );
 template<typename E>
 int gemm_ring_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
+double gemm_ring_gate_ns( uint64_t s, uint64_t hidden, uint64_t b );
 bool gemm_ring_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const void* x, const void* w13, const void* hb, uint64_t hb_stride );
 template<typename E>
 int gemm_ring_gate_launch( E* hb, const GateRows& gate, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
@@ -63,7 +70,7 @@ int with_half_type( gh_dtype dt, F&& run )
 }
 inline bool is_half_type( gh_dtype dt ) { return dt == GH_F16 || dt == GH_BF16; }
 
-int g_force_kernel = 0; // 0 auto, 1 small tiled kernel of this file, 2 streaming kernel, 3 ring kernel (b > 64), 4 256-token tile kernel
+int g_force_kernel = 0; // 0 auto, 1 small tiled kernel of this file, 2 streaming kernel, 3 128 x 128 tiles (b > 64), 4 256 x 256 tiles, 5 ring kernel
 // GLINT_LIBRARY_ROWS in the environment overrides the default (for the command-line profilers, which have no other way in)
 uint64_t library_rows_default()
 {
@@ -294,14 +301,51 @@ namespace gh {
 // `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue;
 // otherwise the kernel may store DType results straight into `xout` (*splits_out == 0 then).
 
-// Many rows without whole tiles of 256 x 256: the ring kernel, or those tiles with the K range split, and the kernel that adds the sums.
-static double other_tiles_ns( uint64_t s, uint64_t r, uint64_t b )
+// The stores of the ring kernel, 8 bytes a lane with nothing to hide them; what the steps of a long K range are priced at covers part of it
+// (32000 x 64 at 7000 rows: 400 us, of which the one step is 20).
+static double ring_stores_ns( uint64_t s, uint64_t r, uint64_t b ) { return (double)( b * r ) / 1000.0 * std::min( 1.0, 1024.0 / (double)s ); }
+
+// Which kernel takes a 16-bit product that all of them can take (s % 8 == 0, 16-byte aligned operands), by what each is estimated to need:
+// the estimates are fitted to timings of 65 shapes of 64 to 11008 k and 288 to 32000 weight rows at 17 row counts from 65 to 7000, where the
+// choice is 1 % off the fastest on average.  The same whether the rounded result is wanted or, for the kernel that follows, its fp32 sums: both
+// calls give the same bits.
+enum class HalfKernel { ring, tile128, tile256, tile256_split };
+struct HalfPlan
 {
-  double ring = 0.0, tiles = 0.0;
-  uint32_t splits = 0, k_len = 0;
-  ring += gemm_ring_splits( s, r, b, &ring ) > 1 ? 4500.0 : 0.0;
-  gemm_tile256_split_plan( s, r, b, &splits, &k_len, &tiles );
-  return splits > 1 ? std::min( ring, tiles + 4500.0 ) : ring;
+  HalfKernel kernel { HalfKernel::ring };
+  uint32_t splits { 1 }, k_len { 0 };
+  double ns { 0.0 };      // to the rounded result
+  double sums_ns { 0.0 }; // to the fp32 sums, the reading of them included
+};
+static HalfPlan half_plan( uint64_t s, uint64_t r, uint64_t b, bool whole_tiles )
+{
+  const double plane_ns = (double)( b * r ) * 8.0 / 5000.0; // fp32 sums of one K range written and read
+  auto priced = [&]( HalfKernel kernel, uint32_t splits, uint32_t k_len, double kernel_ns, double store_ns ) {
+    const double sums_ns = kernel_ns + splits * plane_ns;
+    return HalfPlan { kernel, splits, k_len, splits > 1 ? sums_ns + GEMM_REDUCE_NS : kernel_ns + store_ns, sums_ns };
+  };
+  double ns = 0.0;
+  uint32_t splits = gemm_ring_splits( s, r, b, &ns ), k_len = 0;
+  HalfPlan best = priced( HalfKernel::ring, splits, 0, ns, ring_stores_ns( s, r, b ) );
+  auto better = [&]( const HalfPlan& plan ) {
+    if ( plan.ns <= best.ns ) {
+      best = plan;
+    }
+  };
+  if ( b > 64 ) {
+    gemm_tile_plan( s, r, b, &splits, &k_len );
+    better( priced( HalfKernel::tile128, splits, k_len, gemm_tile_ns( s, r, b ), 0.0 ) );
+  }
+  if ( gemm_tile256_takes( s, b, nullptr, nullptr, nullptr ) ) {
+    gemm_tile256_split_plan( s, r, b, &splits, &k_len, &ns );
+    if ( splits > 1 ) {
+      better( priced( HalfKernel::tile256_split, splits, k_len, ns - splits * plane_ns, 0.0 ) );
+    }
+    if ( whole_tiles ) {
+      better( priced( HalfKernel::tile256, 1, 0, gemm_tile256_ns( s, r, b ), 0.0 ) );
+    }
+  }
+  return best;
 }
 
 // Whether a product runs as whole tiles of 256 x 256 (what is left of it once gemm_token_split() has cut it).
@@ -310,67 +354,14 @@ static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, c
   if ( !gemm_tile256_takes( s, b, x, w, xout ) ) {
     return false;
   }
-  return g_force_kernel == 4 ? gemm_tile256_fills( r, b ) : g_force_kernel == 0 && gemm_tile256_ns( s, r, b ) <= other_tiles_ns( s, r, b );
+  return g_force_kernel == 4 ? gemm_tile256_fills( r, b ) : g_force_kernel == 0 && half_plan( s, r, b, true ).kernel == HalfKernel::tile256;
 }
 
-uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
-
-int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
-                          bool* done )
+// Tokens of the first part when a product, `whole_ns` in one, is better run as whole rounds of 256 x 256 tiles and a rest, rest_ns( tokens ); 0 otherwise.
+template<typename F>
+static uint64_t cut_tokens( uint64_t s, uint64_t r, uint64_t b, double whole_ns, F&& rest_ns )
 {
-  *done = false;
-  if ( !is_half_type( dt ) ) {
-    return GH_OK;
-  }
-  const bool plain_silu = gate.activation == GH_ACT_SILU && gate.bias == nullptr;
-  if ( !plain_silu && b >= 192 ) { // the tiles' epilogue has no room for it
-    return GH_OK;
-  }
-  const bool stream = ( g_force_kernel == 2 || ( g_force_kernel == 0 && gemm_stream_gate_waves() != 0 ) ) && b <= 64
-                      && plain_silu
-                      && gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
-  const bool library = b > 64 && ( gemm_library_wanted_wide( s, 2 * hidden, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden, b, dt, x, w13, hb ) );
-  const bool takes_tiles = !stream && !library && gate.stride % 8 == 0 && hidden % 8 == 0;
-  if ( takes_tiles && gate.context_rows == nullptr ) { // (rows of contexts are counted from the first)
-    if ( const uint64_t b1 = gemm_token_split( s, 2 * hidden, b, dt, x, w13, hb ) ) {
-      char* rest = static_cast<char*>( hb ) + b1 * gate.stride * 2;
-      const char* rest_x = static_cast<const char*>( x ) + b1 * s * 2;
-      if ( gemm_ring_gate_applicable( s, hidden, b - b1, rest_x, w13, rest, gate.stride ) || tile256_wanted( s, 2 * hidden, b - b1, rest_x, w13, rest ) ) {
-        if ( int rc = gemm_gate_one_launch( hb, gate, x, w13, s, hidden, b1, dt, st, done ) ) {
-          return rc;
-        }
-        if ( *done ) {
-          return gemm_gate_one_launch( rest, gate, rest_x, w13, s, hidden, b - b1, dt, st, done );
-        }
-      }
-    }
-  }
-  // From 192 rows on the 256 x 256 tiles where they are enough (70B, 256 rows: 235 us with the gate behind them, the ring kernel 264).
-  const bool tiles = takes_tiles && tile256_wanted( s, 2 * hidden, b, x, w13, hb );
-  const bool ring = !stream && !tiles && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) && !library
-                    && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride );
-  if ( !stream && !ring && !tiles ) {
-    return GH_OK;
-  }
-  *done = true;
-  return with_half_type( dt, [&]( auto* e ) {
-    using E = std::remove_pointer_t<decltype( e )>;
-    E* out = static_cast<E*>( hb );
-    const E *in = static_cast<const E*>( x ), *mat = static_cast<const E*>( w13 );
-    return stream  ? gemm_stream_gate_launch<E>( out, gate.stride, in, mat, s, hidden, b, st )
-           : tiles ? gemm_tile256_launch<E>( out, nullptr, in, mat, s, hidden, b, 2, st, 1, 0, nullptr, 0, &gate )
-                   : gemm_ring_gate_launch<E>( out, gate, in, mat, s, hidden, b, st );
-  } );
-}
-
-// Tokens of the first part when a many-row product is better run as two products along the tokens, 0 otherwise.
-uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout )
-{
-  if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
-    return 0;
-  }
-  const double whole = gemm_tile256_ns( s, r, b );
-  double best = std::min( whole, other_tiles_ns( s, r, b ) );
+  double best = whole_ns;
   uint64_t best_b1 = 0;
   const uint64_t rounds = gemm_tile256_rounds( r, b );
   for ( uint64_t n = 1; n < 3 && n < rounds; n++ ) { // the first part one round shorter, or two
@@ -379,7 +370,7 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
       break;
     }
     // a second launch, and 2 % for what the estimates don't know
-    const double cost = ( gemm_tile256_ns( s, r, b1 ) + other_tiles_ns( s, r, b - b1 ) + 2000.0 ) * 1.02;
+    const double cost = ( gemm_tile256_ns( s, r, b1 ) + rest_ns( b - b1 ) + 2000.0 ) * 1.02;
     if ( cost < best ) {
       best = cost;
       best_b1 = b1;
@@ -388,12 +379,114 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
   return best_b1;
 }
 
+uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout )
+{
+  if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
+    return 0;
+  }
+  return cut_tokens( s, r, b, half_plan( s, r, b, true ).ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
+}
+
+// Which kernel takes w1, w3 and the gate in one launch (what is left of it once gemm_token_split() has cut it); none: two launches.
+enum class GateKernel { none, stream, ring, tiles };
+static GateKernel gate_kernel( const void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, double* ns )
+{
+  *ns = 0.0;
+  const bool plain_silu = gate.activation == GH_ACT_SILU && gate.bias == nullptr;
+  if ( !is_half_type( dt ) || ( !plain_silu && b >= 192 ) ) { // the tiles' epilogue has no room for more than the plain SiLU gate
+    return GateKernel::none;
+  }
+  if ( ( g_force_kernel == 2 || ( g_force_kernel == 0 && gemm_stream_gate_waves() != 0 ) ) && b <= 64 && plain_silu
+       && gemm_stream_gate_applicable( s, hidden, b, x, w13, hb, gate.stride ) ) {
+    return GateKernel::stream;
+  }
+  if ( b > 64 && ( gemm_library_wanted_wide( s, 2 * hidden, b, dt, x, w13, hb ) || gemm_library_wanted( s, hidden, b, dt, x, w13, hb ) ) ) {
+    return GateKernel::none;
+  }
+  const bool rows_of_eight = gate.stride % 8 == 0 && hidden % 8 == 0;
+  if ( g_force_kernel != 0 ) {
+    return g_force_kernel == 4 && rows_of_eight && tile256_wanted( s, 2 * hidden, b, x, w13, hb ) ? GateKernel::tiles
+           : g_force_kernel == 5 && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride )
+             ? GateKernel::ring
+             : GateKernel::none;
+  }
+  if ( !gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride ) ) {
+    return GateKernel::none;
+  }
+  // From 192 rows on 256 x 256 tiles where they are enough (70B, 256 rows: 235 us with the gate behind them, the ring kernel 264).  The ring kernel
+  // splits no K range here: where too few rows fill the chip (2 x 1024 of 2048 k at 8 rows: 10.5 us) the split of the plain product with the
+  // gate's kernel behind it (about 4.5 us) is faster (9), and so are 128 x 128 tiles where the K range is short (2 x 1376 of 512 k at 224
+  // rows: 20 us, 16), but those would leave rounded factors to a gate over the fp32 sums of many rows.
+  const bool keeps_sums = gate.exact && b >= PRODUCT_ROUNDED_ROWS;
+  const double ring_ns = gemm_ring_gate_ns( s, hidden, b ) + ring_stores_ns( s, hidden, b );
+  double two_ns = 0.0;
+  if ( keeps_sums ) {
+    const uint32_t splits = gemm_ring_splits( s, 2 * hidden, b, &two_ns );
+    two_ns = splits > 1 ? two_ns + splits * (double)( 2 * b * hidden ) * 8.0 / 5000.0 + 4500.0 : 1e30;
+  } else {
+    two_ns = half_plan( s, 2 * hidden, b, false ).sums_ns + 4500.0;
+  }
+  if ( rows_of_eight && gemm_tile256_takes( s, b, x, w13, hb ) && gemm_tile256_ns( s, 2 * hidden, b ) <= std::min( ring_ns, two_ns ) ) {
+    *ns = gemm_tile256_ns( s, 2 * hidden, b );
+    return GateKernel::tiles;
+  }
+  *ns = std::min( ring_ns, two_ns );
+  return ring_ns <= two_ns ? GateKernel::ring : GateKernel::none;
+}
+
+int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st,
+                          bool* done )
+{
+  *done = false;
+  double ns = 0.0;
+  const GateKernel kernel = gate_kernel( hb, gate, x, w13, s, hidden, b, dt, &ns );
+  if ( kernel == GateKernel::none ) {
+    return GH_OK;
+  }
+  if ( g_force_kernel == 0 && kernel != GateKernel::stream && gate.context_rows == nullptr // (rows of contexts are counted from the first)
+       && gate.stride % 8 == 0 && hidden % 8 == 0 && gemm_tile256_takes( s, b, x, w13, hb ) ) {
+    // `rest` tokens after those of the first part; only if the gate rides in both launches
+    auto rest_ns = [&]( uint64_t rest ) {
+      double first_ns = 0.0, last_ns = 0.0;
+      const GateKernel first = gate_kernel( hb, gate, x, w13, s, hidden, b - rest, dt, &first_ns ), last = gate_kernel( hb, gate, x, w13, s, hidden, rest, dt, &last_ns );
+      return first != GateKernel::none && last != GateKernel::none ? last_ns : 1e30;
+    };
+    if ( const uint64_t b1 = cut_tokens( s, 2 * hidden, b, ns, rest_ns ) ) {
+      if ( int rc = gemm_gate_one_launch( hb, gate, x, w13, s, hidden, b1, dt, st, done ) ) {
+        return rc;
+      }
+      return gemm_gate_one_launch( static_cast<char*>( hb ) + b1 * gate.stride * 2, gate, static_cast<const char*>( x ) + b1 * s * 2, w13, s, hidden, b - b1, dt, st,
+                                   done );
+    }
+  }
+  *done = true;
+  return with_half_type( dt, [&]( auto* e ) {
+    using E = std::remove_pointer_t<decltype( e )>;
+    E* out = static_cast<E*>( hb );
+    const E *in = static_cast<const E*>( x ), *mat = static_cast<const E*>( w13 );
+    switch ( kernel ) {
+      case GateKernel::stream: return gemm_stream_gate_launch<E>( out, gate.stride, in, mat, s, hidden, b, st );
+      case GateKernel::tiles: return gemm_tile256_launch<E>( out, nullptr, in, mat, s, hidden, b, 2, st, 1, 0, nullptr, 0, &gate );
+      default: return gemm_ring_gate_launch<E>( out, gate, in, mat, s, hidden, b, st );
+    }
+  } );
+}
+
 // Many rows: the large tile kernel with the op that follows the product in its epilogue, 1 = xout += product
 // (accum).  *done = false: nothing was launched (shape or alignment not for that kernel), the caller takes
 // its other route.
 bool gemm_tile_epilogue_applicable( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout )
 {
-  return is_half_type( dt ) && r % 8 == 0 && tile256_wanted( s, r, b, x, w, xout );
+  if ( !is_half_type( dt ) || r % 8 != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
+    return false;
+  }
+  if ( g_force_kernel != 0 ) {
+    return tile256_wanted( s, r, b, x, w, xout );
+  }
+  // Unsplit 128 x 128 tiles sum in the same order, but would leave fp32 sums here (1024 x 1024, 7000 rows with the norm: 46 us so, 67 with them).
+  const HalfPlan plan = half_plan( s, r, b, true );
+  return plan.kernel == HalfKernel::tile256
+         || ( plan.kernel == HalfKernel::tile128 && plan.splits == 1 && gemm_tile256_ns( s, r, b ) <= plan.sums_ns );
 }
 
 int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, int epilogue, hipStream_t st,
@@ -427,50 +520,57 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     GH_LAUNCH_CHECK();
     return GH_OK;
   }
-  // many tokens at once (prefill): the MFMA-bound tile kernel; few (decode): the ring kernel
-  if ( tile256_wanted( s, r, b, x, w, xout ? xout : x ) ) {
-    float* ws = nullptr;
-    if ( want_partials ) {
-      if ( int rc = ensure_workspace( b * r * sizeof( float ), &ws, st ) ) {
-        return rc;
-      }
-      *partial_out = ws;
-      *splits_out = 1;
+  auto planes = [&]( uint32_t n, float** ws ) { // room for the fp32 sums of n K ranges
+    *partial_out = nullptr;
+    if ( int rc = ensure_workspace( (uint64_t)n * b * r * sizeof( float ), ws, st ) ) {
+      return rc;
     }
-    return gemm_tile256_launch( xout, ws, x, w, s, r, b, 0, st, 1, 0 );
+    *partial_out = *ws;
+    *splits_out = n;
+    return (int)GH_OK;
+  };
+  const void* out = xout ? static_cast<const void*>( xout ) : x;
+  HalfPlan plan;
+  bool taken = false; // by one of the kernels for aligned operands
+  if ( g_force_kernel == 0 ) {
+    taken = gemm_ring_applicable( s, r, b, x, w, out );
+    if ( taken ) {
+      plan = half_plan( s, r, b, true );
+    }
+  } else if ( g_force_kernel == 3 ) {
+    taken = gemm_tile_applicable( s, r, b, x, w, out );
+    GH_REQUIRE( taken, "gh_matmul: the 128 x 128 tile kernel needs b > 64, s %% 8 == 0 and 16-byte aligned operands" );
+    plan.kernel = HalfKernel::tile128;
+    gemm_tile_plan( s, r, b, &plan.splits, &plan.k_len );
+  } else if ( g_force_kernel == 4 ) {
+    plan.kernel = HalfKernel::tile256;
+    taken = tile256_wanted( s, r, b, x, w, out );
+    if ( !taken && gemm_tile256_takes( s, b, x, w, x ) ) {
+      plan.kernel = HalfKernel::tile256_split;
+      gemm_tile256_split_plan( s, r, b, &plan.splits, &plan.k_len, &plan.ns );
+      taken = plan.splits > 1;
+    }
+    GH_REQUIRE( taken, "gh_matmul: the 256 x 256 tile kernel needs b >= 192, at least 192 tiles with a last round that is not mostly empty, s %% 64 == 0 and 16-byte aligned operands" );
+  } else if ( g_force_kernel == 5 ) {
+    taken = gemm_ring_applicable( s, r, b, x, w, out );
+    GH_REQUIRE( taken, "gh_matmul: the ring kernel needs s %% 8 == 0 and 16-byte aligned operands" );
+    plan.splits = gemm_ring_splits( s, r, b, &plan.ns );
   }
-  const bool ring = gemm_ring_applicable( s, r, b, x, w, xout ? xout : x );
-  double ring_ns = 0.0;
-  const uint32_t ring_splits = ring ? gemm_ring_splits( s, r, b, &ring_ns ) : 0;
-  if ( g_force_kernel == 0 || g_force_kernel == 4 ) { // some hundred rows and few tiles: the same kernel with the K range split
-    uint32_t splits = 0, k_len = 0;
-    double tile_ns = 0.0;
-    if ( gemm_tile256_takes( s, b, x, w, x ) ) {
-      gemm_tile256_split_plan( s, r, b, &splits, &k_len, &tile_ns );
-    }
-    if ( splits > 1 && ( g_force_kernel == 4 || !ring || tile_ns < ring_ns ) ) {
-      float* ws = nullptr;
-      if ( int rc = ensure_workspace( (uint64_t)splits * b * r * sizeof( float ), &ws, st ) ) {
-        return rc;
-      }
-      *partial_out = ws;
-      *splits_out = splits;
-      return gemm_tile256_launch<E>( nullptr, ws, x, w, s, r, b, 0, st, splits, k_len );
-    }
-  }
-  GH_REQUIRE( g_force_kernel != 4, "gh_matmul: the 256 x 256 tile kernel needs b >= 192, at least 192 tiles with a last round that is not mostly empty, s %% 64 == 0 and 16-byte aligned operands" );
-  if ( ring && ( g_force_kernel == 0 || ( g_force_kernel == 3 && b > 64 ) ) ) {
+  if ( taken ) {
     float* ws = nullptr;
-    if ( want_partials || ring_splits > 1 ) {
-      if ( int rc = ensure_workspace( (uint64_t)ring_splits * b * r * sizeof( float ), &ws, st ) ) {
+    if ( want_partials || plan.splits > 1 ) {
+      if ( int rc = planes( plan.splits, &ws ) ) {
         return rc;
       }
-      *partial_out = ws;
-      *splits_out = ring_splits;
+    }
+    switch ( plan.kernel ) {
+      case HalfKernel::tile128: return gemm_tile_launch( xout, ws, x, w, s, r, b, plan.splits, plan.k_len, st );
+      case HalfKernel::tile256: return gemm_tile256_launch( xout, ws, x, w, s, r, b, 0, st, 1, 0 );
+      case HalfKernel::tile256_split: return gemm_tile256_launch<E>( nullptr, ws, x, w, s, r, b, 0, st, plan.splits, plan.k_len );
+      case HalfKernel::ring: break;
     }
     return gemm_ring_launch( xout, ws, x, w, s, r, b, st );
   }
-  GH_REQUIRE( g_force_kernel != 3, "gh_matmul: the ring kernel needs b > 64 (when forced), s %% 8 == 0 and 16-byte aligned operands" );
 
   if ( g_force_kernel == 2 && gemm_stream_applicable( s, r, b, x, w, xout ? xout : x ) ) {
     uint32_t splits = 1, k_per_split = 0, rows_per_wg = 0;

@@ -35,6 +35,10 @@ constexpr int RING_THREADS = 512;
 // Steps of a K range from which on a work-group starts at one of its own: a short range is over before the channels matter (7B wo, 8 to 16
 // steps: 8.6 and 9.4 us either way), and all of its rows are summed in the one order whichever product they are part of.
 [[maybe_unused]] constexpr uint32_t RING_TURN_STEPS = 17;
+// What a K split costs beside its sums, in ns.  Products of a layer leave sums to the kernel that follows in any case, plain ones only with a split, for
+// GEMM_REDUCE_NS, and the plan is the same for both, so that both give the same bits.  This keeps 512 k in one range up to 64 rows (512 x 512,
+// plain: 9 us instead of 12) and cuts longer ones; with 2.6 us 2048 x 2048 at 512 rows would stay whole, 25.6 us with its norm instead of 21.8.
+constexpr double RING_SPLIT_NS = 1600.0;
 constexpr int RING_K = 64; // k a step: 8 chunks of 8 halves
 [[maybe_unused]] constexpr uint32_t RING_PAST_ROW = 0x80000000u;  // lane offset of a row that is not there
 [[maybe_unused]] constexpr uint32_t RING_PAST_STEP = 0x40000000u; // scalar offset of a step that is not there: no descriptor is longer
@@ -322,7 +326,8 @@ int g_ring_cus = 0; // tuning override of the CU count the plan balances for (0:
 // weights at the CU's share of the memory's rate (4.7 ns a row) and its activations at what L2 delivers to a CU (2 ns a row), but no
 // less than a load's time in flight (1.9 us) over the steps requested ahead.  With several slabs the weights come from L2 and the
 // matrix units set the pace; wide slabs slow each other down.  A round costs what it takes to fill the ring, and a split the fp32 sums
-// that are written and read again.
+// that are written and read again, and RING_SPLIT_NS.  A work-group that fills three wide stages
+// first starts later (4096 x 512 at 256 rows: 16 us for 8 steps), of which the steps of a long range are priced to cover a part.
 RingPlan find_ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate, uint64_t n_cu )
 {
   constexpr uint32_t XS[] = { 32, 64, 96, 128, 192, 256 };
@@ -350,8 +355,9 @@ RingPlan find_ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate, uint64_t
           const double w_rows = (double)( gate ? 2 * rows : rows ), x_rows = (double)std::min<uint64_t>( cols, b );
           const double step_ns = slabs == 1 ? std::max( 4.7 * w_rows + 2.0 * x_rows, 1900.0 / ( ring_stages( w, x ) - 1 ) )
                                             : 1.05 * ( 2.9 * w_rows + 1.05 * ( x_rows + x ) + ( x > 128 ? 20.0 + 7.0 * (double)slabs : 40.0 ) );
-          const double sums_ns = splits > 1 ? (double)( splits * b * r ) * 8.0 / 5000.0 : 0.0;
-          const double cost = real_rounds * ( ( slabs == 1 ? 2000.0 : 3000.0 ) + (double)per * step_ns ) + sums_ns;
+          const double start_ns = slabs > 1 ? 3000.0 : x < 192 ? 2000.0 : 2000.0 + 4000.0 * std::min( 1.0, 16.0 / (double)per );
+          const double sums_ns = splits > 1 ? (double)( splits * b * r ) * 8.0 / 5000.0 + RING_SPLIT_NS : 0.0;
+          const double cost = real_rounds * ( start_ns + (double)per * step_ns ) + sums_ns;
           if ( best.w == 0 || cost < best.ns ) {
             best = RingPlan { w, x, RingCut { (uint32_t)rows, (uint32_t)cols, (uint32_t)row_blocks, (uint32_t)slabs, (uint32_t)splits, (uint32_t)per }, cost };
           }
@@ -392,10 +398,11 @@ bool gemm_ring_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, co
          && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) | reinterpret_cast<uintptr_t>( xout ) ) & 15u ) == 0;
 }
 
+// *ns: the estimate without the sums of a split
 uint32_t gemm_ring_splits( uint64_t s, uint64_t r, uint64_t b, double* ns )
 {
   const RingPlan plan = ring_plan( s, r, b, false );
-  *ns = plan.ns;
+  *ns = plan.cut.splits > 1 ? plan.ns - (double)( plan.cut.splits * b * r ) * 8.0 / 5000.0 - RING_SPLIT_NS : plan.ns;
   return plan.cut.splits;
 }
 
@@ -408,13 +415,12 @@ int gemm_ring_launch( E* xout, float* partial, const E* x, const E* w, uint64_t 
   return ring_launch<E>( partial ? RING_PARTIAL : RING_STORE, partial ? (void*)partial : (void*)xout, x, w, s, r, b, GateRows {}, plan, st );
 }
 
-// hb(b, hidden) = DType(silu(y1) * y3), y1 = x . w1^T, y3 = x . w3^T, w13 = w1 rows then w3 rows, in one launch.  Where too few rows fill the chip (2 x 1024 of 2048 k at 8 rows: 10.5 us) the K split
-// of the plain product with the gate's kernel behind it (about 4.5 us) is faster: 9.
+// hb(b, hidden) = DType(silu(y1) * y3), y1 = x . w1^T, y3 = x . w3^T, w13 = w1 rows then w3 rows, in one launch
 bool gemm_ring_gate_applicable( uint64_t s, uint64_t hidden, uint64_t b, const void* x, const void* w13, const void* hb, uint64_t hb_stride )
 {
-  return hidden % 4 == 0 && hb_stride % 4 == 0 && gemm_ring_applicable( s, 2 * hidden, b, x, w13, hb )
-         && ring_plan( s, hidden, b, true ).ns <= ring_plan( s, 2 * hidden, b, false ).ns + 4500.0;
+  return hidden % 4 == 0 && hb_stride % 4 == 0 && gemm_ring_applicable( s, 2 * hidden, b, x, w13, hb );
 }
+double gemm_ring_gate_ns( uint64_t s, uint64_t hidden, uint64_t b ) { return ring_plan( s, hidden, b, true ).ns; }
 
 template<typename E>
 int gemm_ring_gate_launch( E* hb, const GateRows& gate, const E* x, const E* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st )

@@ -466,15 +466,20 @@ bool gemm_tile256_fills( uint64_t r, uint64_t b )
 }
 
 // `rounds` of one work-group per CU, `units` work-groups in all.  A step of 64 k takes 1 us while few CUs multiply and 1.37 when all do and
-// the clock drops (70B w2, 448 steps: 200 tokens 483 us, 1024 511, 2048 616, 3328 in two rounds 1155), a round's ends 3.5.
-static double rounds_ns( uint64_t rounds, uint64_t units, uint64_t steps, double step_ns )
+// the clock drops (70B w2, 448 steps: 200 tokens 483 us, 1024 511, 2048 616, 3328 in two rounds 1155), a round's ends 3.5, and up to 3 more that a
+// long K range hides (14 rounds of 2, 8, 16 and 32 steps, 32000 rows at 7000 tokens: 126, 248, 383 and 667 us).  With a single row of
+// token tiles no work-group shares its weights and all of them come from memory at once: 2 us when all CUs ask (256 tokens of 57344 x 8192,
+// 224 tiles, 128 steps: 1.83 us a step; 32000 x 8192, 125 tiles: 1.48; 10240 x 8192, 40: 1.1), less with fewer tokens beside them (28672 x 8192, 112
+// tiles: 1.47 at 256 tokens, 1.41 at 224, 1.27 at 192), but not where a K split asks in several places (8192 x 28672 in 8 at 192 tokens: 1.9).
+static double rounds_ns( uint64_t rounds, uint64_t units, uint64_t steps, uint64_t b, bool split )
 {
   const double busy = (double)units / (double)( rounds * (uint64_t)cu_count() );
-  return (double)rounds * ( (double)steps * std::max( step_ns, 1000.0 + 370.0 * busy * busy ) + 3500.0 );
+  const double step_ns = b > TN2 ? 1000.0 + 370.0 * busy * busy : 1000.0 + busy * ( split ? 1000.0 : 1800.0 * (double)b / TN2 - 800.0 );
+  return (double)rounds * ( (double)steps * step_ns + 3500.0 + 3000.0 * std::min( 1.0, 16.0 / (double)steps ) ) + 1000.0;
 }
 double gemm_tile256_ns( uint64_t s, uint64_t r, uint64_t b )
 {
-  return rounds_ns( rounds_per_xcd( r, b ), ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 ), s / TKS, 0.0 );
+  return rounds_ns( rounds_per_xcd( r, b ), ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 ), s / TKS, b, false );
 }
 
 // A launch is as slow as its number of rounds, so a product whose tiles leave the last round partly empty pays for a whole round there:
@@ -493,13 +498,13 @@ uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds )
 uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b ) { return rounds_per_xcd( r, b ); }
 
 // The K range of each tile split over several work-groups, the fp32 sums of each split to partial[split].  *splits = 0: not for this
-// shape.  With a single row of tiles a step takes 2 us (the weights are then read for one tile each); the sums are written and read.
+// shape.  The sums are written and read.
 void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns )
 {
   *splits = 0;
   *k_len = 0;
   *ns = 0.0;
-  const uint64_t token_tiles = ( b + TN2 - 1 ) / TN2, tiles = ( ( r + TM2 - 1 ) / TM2 ) * token_tiles;
+  const uint64_t tiles = ( ( r + TM2 - 1 ) / TM2 ) * ( ( b + TN2 - 1 ) / TN2 );
   const uint64_t cus = (uint64_t)cu_count(), steps = s / TKS;
   if ( b < 192 || tiles > 2 * cus || s % TKS != 0 || s >= ( 1u << 22 ) ) {
     return;
@@ -509,7 +514,7 @@ void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* spli
     if ( per < 12 || n != want ) {
       continue;
     }
-    const double cost = rounds_ns( ( tiles * n + cus - 1 ) / cus, tiles * n, per, token_tiles == 1 ? 2000.0 : 0.0 ) + (double)( n * b * r ) * 8.0 / 5000.0;
+    const double cost = rounds_ns( ( tiles * n + cus - 1 ) / cus, tiles * n, per, b, true ) + (double)( n * b * r ) * 8.0 / 5000.0;
     if ( *splits == 0 || cost < *ns ) {
       *splits = (uint32_t)n;
       *k_len = (uint32_t)( per * TKS );

@@ -10,6 +10,9 @@ namespace gh {
 int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, hipStream_t st, bool want_partials,
                    float** partial_out, uint32_t* splits_out );
 
+// The kernel that rounds the sums of a K split, with the gap in front of it, in ns
+constexpr double GEMM_REDUCE_NS = 3000.0;
+
 // Rows of a gated feed-forward that its product stores itself: DType(activation(y1 + bias1) * (y3 + bias3)).
 struct GateRows
 {

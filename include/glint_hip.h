@@ -153,7 +153,7 @@ int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_
 int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::matmul<s,r> / untemplated_matmul  arch/amd64/common/ops.hh:74-93,212-271 :
  * xout(b, r) = sum_p w(r, p) * x(b, p); w row-major (r, s); fp32 accumulate */
-/* tuning hook: kernel 0 auto / 1 small tiled / 2 streaming through registers / 3 ring (more than 64 rows) / 4 256-token tile (many rows); the number of
+/* tuning hook: kernel 0 auto / 1 small tiled / 2 streaming through registers / 3 128 x 128 tiles (more than 64 rows) / 4 256 x 256 tiles (many rows) / 5 ring; the number of
  * compute units the streaming and the ring kernel's plans are balanced for (<= 0 keeps the current value; the default is the device's own count); `tile_rows` non-zero: a
  * product is never cut in two along the tokens */
 int gh_gemm_set_tuning( int kernel, int target_workgroups, int tile_rows );

@@ -352,6 +352,47 @@ def test_matmul_ring_edges(dt, b, s, r):
     assert ((ops.matmul(x, w).double() - want).abs() <= bound).all()
 
 
+# the 128 x 128 tile kernel: K ranges that end inside a step, of one step and of several K splits; rows that leave whole 16-byte chunks, four at a time
+# and one by one, rounded and as fp32 sums; ragged tiles in both directions
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,s,r", [(65, 8, 3), (128, 64, 128), (129, 72, 132), (300, 288, 1030), (257, 1024, 520), (200, 4104, 516), (130, 2056, 261), (1000, 520, 4100)])
+def test_matmul_tiles_128_edges(dt, b, s, r):
+    """As for the ring kernel; the residual add of the same product gives its sums the same bits."""
+    from glinthawk_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(b * 17 + r)
+    w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+    hot = torch.zeros((b, s), dtype=dt, device="cuda")
+    cols = torch.tensor([(7919 * i + 3) % s for i in range(b)], device="cuda")
+    hot[torch.arange(b, device="cuda"), cols] = 1
+    x = torch.randn((b, s), generator=g, device="cuda").to(dt)
+    _lib.check(_lib.lib().gh_gemm_set_tuning(3, 0, 0))
+    try:
+        assert torch.equal(ops.matmul(hot, w), w[:, cols].t().contiguous())
+        got = ops.matmul(x, w)
+        if dt == torch.float16:
+            residual = torch.zeros_like(got)
+            ops.matmul_accum(residual, x, w)
+            assert torch.equal(residual, got)
+    finally:
+        _lib.check(_lib.lib().gh_gemm_set_tuning(0, 0, 0))
+    want = x.double() @ w.double().t()
+    bound = want.abs() * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 1e-4
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+# rows and K ranges at which the dispatch changes kernels: the product that the residual add carries gives the bits of the plain one and an add
+@pytest.mark.parametrize("b,s,r", [(64, 512, 512), (65, 288, 4096), (192, 768, 4096), (256, 512, 4096), (256, 8192, 5000), (700, 2048, 2048), (7000, 1024, 1024), (4096, 768, 2048)])
+def test_matmul_accum_has_the_bits_of_the_product(b, s, r):
+    g = torch.Generator(device="cuda").manual_seed(b + s + r)
+    x = torch.randn((b, s), generator=g, device="cuda").half()
+    w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).half()
+    residual = torch.randn((b, r), generator=g, device="cuda").half()
+    want = residual.clone()
+    ops.accum(want, ops.matmul(x, w))
+    ops.matmul_accum(residual, x, w)
+    assert torch.equal(residual, want)
+
+
 # whole rounds of tiles and a rest with its K range split; K splits over row tiles that are no multiple of the XCDs; several slabs of the
 # ring kernel over a long K range (all keep step), over one that ends inside a step; one-hot activations, every output is one weight
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
