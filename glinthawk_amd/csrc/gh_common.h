@@ -91,6 +91,13 @@ public:
 // shares one.  Growing waits for that stream only.  `min_bytes` is the size of the first allocation.
 enum { SCRATCH_GEMM_PARTIALS = 0, SCRATCH_CONVERT = 1, SCRATCH_ATTN_PV = 2, SCRATCH_GATE_FACTOR = 3, SCRATCH_LIBRARY = 4, SCRATCH_PRODUCT = 5, SCRATCH_MIXER = 6 };
 int stream_scratch( hipStream_t stream, int which, uint64_t bytes, uint64_t min_bytes, void** out );
+// Whether two buffers share memory: an op that stores its output while its other work-groups still read the input must not take such a pair.
+inline bool overlap( const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes )
+{
+  const uintptr_t p = reinterpret_cast<uintptr_t>( a ), q = reinterpret_cast<uintptr_t>( b );
+  return a != nullptr && b != nullptr && p < q + b_bytes && q < p + a_bytes;
+}
+
 // gh_gemm_lib.hip: a plain f16 product through the vendor's GEMM library; *done = false: declined, nothing queued
 int gemm_library( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st, bool* done );
 bool gemm_library_available( uint64_t s, uint64_t r, uint64_t b );

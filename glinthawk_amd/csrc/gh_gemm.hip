@@ -438,6 +438,9 @@ int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const v
                           bool* done )
 {
   *done = false;
+  if ( !is_half_type( dt ) || overlap( hb, ( ( b - 1 ) * gate.stride + hidden ) * 2, x, b * s * 2 ) ) {
+    return GH_OK;
+  }
   double ns = 0.0;
   const GateKernel kernel = gate_kernel( hb, gate, x, w13, s, hidden, b, dt, &ns );
   if ( kernel == GateKernel::none ) {

@@ -450,7 +450,9 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   // gh_rmsnorm takes 16-byte aligned buffers only: other ones go through fp32 sums and the row kernel, which reads them element by element
   const bool norm_kernel = norm_out == nullptr
                            || ( ( reinterpret_cast<uintptr_t>( residual ) | reinterpret_cast<uintptr_t>( norm_out ) | reinterpret_cast<uintptr_t>( norm_weight ) ) & 15u ) == 0;
-  if ( dt == GH_F32 && norm_kernel ) {
+  // a residual that lies over the activations gets its product through fp32 sums: every row of them is read before the first is stored
+  const bool apart = !overlap( residual, b * r * dtype_size( dt ), x, b * s * dtype_size( dt ) );
+  if ( dt == GH_F32 && norm_kernel && apart ) {
     if ( int rc = gemm_f32_accum( static_cast<float*>( residual ), static_cast<const float*>( x ), static_cast<const float*>( w ), s, r, b, st ) ) {
       return rc;
     }
@@ -482,7 +484,7 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
       return norm_out != nullptr ? gh_rmsnorm( norm_out, residual, norm_weight, r, b, dt, stream ) : GH_OK;
     }
   }
-  if ( const uint64_t b1 = gemm_token_split( s, r, b, dt, x, w, residual ) ) { // two products along the tokens (rows are independent)
+  if ( const uint64_t b1 = apart ? gemm_token_split( s, r, b, dt, x, w, residual ) : 0 ) { // two products along the tokens (rows are independent)
     const uint64_t elem = 2;
     if ( int rc = gh_matmul_accum( residual, x, w, s, r, b1, norm_out, norm_weight, dt, stream ) ) {
       return rc;
@@ -493,7 +495,7 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   // many rows: the residual is added in the tile kernel's epilogue, no fp32 partials;
   // the norm of the new residual, when asked for, is the plain row kernel
   done = false;
-  if ( norm_kernel ) {
+  if ( norm_kernel && apart ) {
     if ( int rc = gemm_tile_epilogue_launch( residual, x, w, s, r, b, dt, 1, st, &done ) ) {
       return rc;
     }
@@ -534,7 +536,8 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   }
   GH_REQUIRE( hb != nullptr, "gh_matmul_silu_gate: NULL output" );
   hipStream_t st = as_stream( stream );
-  if ( dt == GH_F32 ) {
+  const bool apart = !overlap( hb, b * hidden_dim * dtype_size( dt ), x, b * s * dtype_size( dt ) ); // else through fp32 sums, as in gh_matmul_accum
+  if ( dt == GH_F32 && apart ) {
     return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), static_cast<const float*>( w13 ), s, hidden_dim, b, st );
   }
   bool done = false;
@@ -564,7 +567,7 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
     }
   }
   // the factors as two products of the vendor's library, then the gate; the same roundings
-  if ( hidden_dim % 8 == 0 && gemm_library_wanted( s, hidden_dim, b, dt, x, w13, hb ) ) {
+  if ( apart && hidden_dim % 8 == 0 && gemm_library_wanted( s, hidden_dim, b, dt, x, w13, hb ) ) {
     void* factor = nullptr;
     if ( int rc = stream_scratch( st, SCRATCH_GATE_FACTOR, b * hidden_dim * sizeof( __half ), 16ull << 20, &factor ) ) {
       return rc;
@@ -581,7 +584,11 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   }
   const uint64_t total = b * hidden_dim;
   const unsigned blocks = (unsigned)std::min<uint64_t>( ( total + 255 ) / 256, 8192 );
-  epi_silu_gate_kernel<__half><<<blocks, 256, 0, st>>>( static_cast<__half*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
+  if ( dt == GH_F16 ) {
+    epi_silu_gate_kernel<__half><<<blocks, 256, 0, st>>>( static_cast<__half*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
+  } else {
+    epi_silu_gate_kernel<float><<<blocks, 256, 0, st>>>( static_cast<float*>( hb ), partial, (uint32_t)hidden_dim, (uint32_t)b, splits );
+  }
   GH_LAUNCH_CHECK();
   return GH_OK;
 }
@@ -605,7 +612,8 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   }
   GH_REQUIRE( q && pos_dev && freq_real && freq_imag && token_rows_dev, "gh_matmul_qkv_rope_append: NULL pointer" );
   hipStream_t st = as_stream( stream );
-  if ( dt == GH_F32 ) {
+  const uint64_t x_bytes = b * s * dtype_size( dt );
+  if ( dt == GH_F32 && !overlap( q, b * dim * sizeof( float ), x, x_bytes ) && !overlap( kv_out, b * 2 * kv_dim * sizeof( float ), x, x_bytes ) ) {
     return gemm_f32_qkv( static_cast<float*>( q ), static_cast<float*>( kv_out ), static_cast<const float*>( x ), static_cast<const float*>( wqkv ), s, b, pos_dev,
                          static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size, st );
   }
@@ -615,9 +623,15 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
     return rc;
   }
   const dim3 grid( (unsigned)( ( r / 2 + 255 ) / 256 ), (unsigned)b );
-  epi_qkv_kernel<__half><<<grid, 256, 0, st>>>( static_cast<__half*>( q ), static_cast<__half*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
-                                               static_cast<const __half*>( freq_real ), static_cast<const __half*>( freq_imag ), token_rows_dev, (uint32_t)dim,
-                                               (uint32_t)kv_dim, head_size );
+  if ( dt == GH_F16 ) {
+    epi_qkv_kernel<__half><<<grid, 256, 0, st>>>( static_cast<__half*>( q ), static_cast<__half*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
+                                                 static_cast<const __half*>( freq_real ), static_cast<const __half*>( freq_imag ), token_rows_dev, (uint32_t)dim,
+                                                 (uint32_t)kv_dim, head_size );
+  } else {
+    epi_qkv_kernel<float><<<grid, 256, 0, st>>>( static_cast<float*>( q ), static_cast<float*>( kv_out ), partial, (uint32_t)b, splits, pos_dev,
+                                                static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim,
+                                                (uint32_t)kv_dim, head_size );
+  }
   GH_LAUNCH_CHECK();
   return GH_OK;
 }

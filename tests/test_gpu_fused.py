@@ -77,6 +77,41 @@ def test_matmul_accum_norm_of_unaligned_rows(dt, b, s, r, at):
     assert torch.allclose(got_norm.float(), want_norm.float(), rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,s", [(3, 512), (70, 1024), (300, 4096)])
+def test_outputs_over_their_activations(dt, b, s):
+    """An output buffer that lies over the activations gives what one of its own gives (the order of fp32 sums may differ: a rounding)."""
+    if dt != torch.float32 and b == 300:
+        b = 2304                                        # enough tiles for the epilogues of the large tile kernel
+    g = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, s), generator=g, device="cuda").to(dt)
+    w = (torch.randn((3 * s, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+    tol = dict(rtol=1e-5, atol=1e-5) if dt == torch.float32 else dict(rtol=2e-2, atol=2e-2) if dt == torch.bfloat16 else dict(rtol=4e-3, atol=4e-3)
+    lib, p, shape, st = _lib.lib(), ops._p, Shape(dim=s, n_layers=1, n_heads=s // 64, n_kv_heads=s // 64, hidden_dim=s, seq_len=8), ops._stream()
+    half = w[:s].contiguous()                           # w1 and w3 of half as many rows
+    got, spare = x.clone(), torch.empty((b, s // 2), dtype=dt, device="cuda")
+    if dt == torch.bfloat16:
+        _lib.check(lib.gh_matmul_gate(p(spare), p(x), p(half), None, s, s // 2, b, ops.GH_ACT_SILU, ops._dt(x), st))
+        _lib.check(lib.gh_matmul_gate(p(got), p(got), p(half), None, s, s // 2, b, ops.GH_ACT_SILU, ops._dt(x), st))
+        assert torch.allclose(got.flatten()[: spare.numel()].float(), spare.flatten().float(), **tol)
+        return
+    _lib.check(lib.gh_matmul_silu_gate(p(spare), p(x), p(half), s, s // 2, b, ops._dt(x), st))
+    _lib.check(lib.gh_matmul_silu_gate(p(got), p(got), p(half), s, s // 2, b, ops._dt(x), st))
+    assert torch.allclose(got.flatten()[: spare.numel()].float(), spare.flatten().float(), **tol)
+    residual, got = x.clone(), x.clone()
+    ops.matmul_accum(residual, x, half)
+    _lib.check(lib.gh_matmul_accum(p(got), p(got), p(half), s, s, b, None, None, ops._dt(x), st))
+    assert torch.allclose(got.float(), residual.float(), **tol)
+    pos = torch.arange(b, dtype=torch.int32, device="cuda") % 8
+    re, im = (torch.randn((8, 32), generator=g, device="cuda").to(dt) for _ in range(2))
+    cache, over = (torch.zeros((b, 2 * s), dtype=dt, device="cuda") for _ in range(2))
+    q, _ = ops.matmul_qkv_rope_append(x, w, pos, re, im, ops.row_table([cache[i].data_ptr() for i in range(b)]), shape)
+    got = x.clone()
+    _lib.check(lib.gh_matmul_qkv_rope_append(p(got), None, p(got), p(w), s, b, p(pos), p(re), p(im), p(ops.row_table([over[i].data_ptr() for i in range(b)])),
+                                             shape.n_kv_heads, shape.gqa_size, shape.head_size, ops._dt(x), st))
+    assert torch.allclose(got.float(), q.float(), **tol) and torch.allclose(over.float(), cache.float(), **tol)
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
                                         # enough row tiles for one launch without a K split: both factors in one kernel
