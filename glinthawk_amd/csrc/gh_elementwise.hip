@@ -3,6 +3,7 @@
 // following the reference's CPU path (arch/amd64/common/ops.hh).
 #include "gh_common.h"
 
+#include <type_traits>
 #include <vector>
 
 namespace gh {
@@ -143,9 +144,10 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
 
 // ---- argmax: one block per row, first index of the maximum --------------------------------------
 // Bound by latency: a row of 32000 values is one work-group's, so a thread asks for ARG_AHEAD pieces of it before it compares the first.  4 fp32
-// rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  As a loop over the row would have it: the lowest index
+// rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  256 threads where they ask for all of a row at once (1024 rows of
+// 4096: 10.2 us, with 1024 threads 17.8), else 1024.  As a loop over the row would have it: the lowest index
 // of equal values, NaN never beats anything but stays where the row begins with it.
-constexpr int ARG_THREADS = 1024, ARG_AHEAD = 8;
+constexpr int ARG_AHEAD = 8;
 __device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float v, uint32_t i )
 {
   const bool take = v > best || ( v == best && i < best_i );
@@ -153,7 +155,7 @@ __device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float
   best_i = take ? i : best_i;
 }
 // V: values per load, n % V == 0 and rows aligned to V values
-template<typename T, int V>
+template<typename T, int V, int ARG_THREADS>
 __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __restrict__ out, const T* __restrict__ v, uint32_t n )
 {
   __shared__ float s_val[ARG_THREADS / WAVE];
@@ -409,11 +411,19 @@ int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n,
   }
   GH_REQUIRE( out_dev && v, "gh_argmax: NULL pointer" );
   GH_REQUIRE( n > 0 && n <= 0xfffffffeull && batch <= 0x7fffffffull, "gh_argmax: bad shape" );
-  if ( n * dtype_size( dt ) % 16 == 0 && ( reinterpret_cast<uintptr_t>( v ) & 15u ) == 0 ) {
-    GH_DISPATCH_DT( dt, argmax_kernel<T, 16 / sizeof( T )><<<(unsigned)batch, ARG_THREADS, 0, as_stream( stream )>>>( out_dev, static_cast<const T*>( v ), (uint32_t)n ) );
-  } else {
-    GH_DISPATCH_DT( dt, argmax_kernel<T, 1><<<(unsigned)batch, ARG_THREADS, 0, as_stream( stream )>>>( out_dev, static_cast<const T*>( v ), (uint32_t)n ) );
-  }
+  const bool whole = n * dtype_size( dt ) % 16 == 0 && ( reinterpret_cast<uintptr_t>( v ) & 15u ) == 0;
+  auto launch = [&]( auto* e, auto per_load ) {
+    using T = std::remove_pointer_t<decltype( e )>;
+    constexpr int V = decltype( per_load )::value;
+    const T* rows = static_cast<const T*>( v );
+    if ( n <= 256ull * ARG_AHEAD * V ) {
+      argmax_kernel<T, V, 256><<<(unsigned)batch, 256, 0, as_stream( stream )>>>( out_dev, rows, (uint32_t)n );
+    } else {
+      argmax_kernel<T, V, 1024><<<(unsigned)batch, 1024, 0, as_stream( stream )>>>( out_dev, rows, (uint32_t)n );
+    }
+  };
+  GH_DISPATCH_DT( dt, whole ? launch( static_cast<T*>( nullptr ), std::integral_constant<int, 16 / sizeof( T )> {} )
+                            : launch( static_cast<T*>( nullptr ), std::integral_constant<int, 1> {} ) );
   GH_LAUNCH_CHECK();
   if ( out_host ) {
     GH_HIP( hipMemcpyAsync( out_host, out_dev, batch * sizeof( uint32_t ), hipMemcpyDeviceToHost, as_stream( stream ) ) );
