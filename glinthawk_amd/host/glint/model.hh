@@ -392,8 +392,10 @@ public:
     // and the last layer's feed-forward of a run overlaps the download of the one before.  Everything in between (attention needs all
     // rows of a context) runs on all rows at once.  What stays exposed is the first layer's work on the last run and that run's
     // download, so the runs get shorter (70B, 3328 tokens, 2 layers: 9.73 ms as 2048 + 768 + 512, 10.93 in one; 13B, 14000 tokens,
-    // 4 layers: 31.2 and 35.2); below 1024 tokens a copy is shorter than what the cuts cost.
-    const bool pipelined = n >= 1024 && !( first_layer == 0 && token_ids != nullptr ) && ( acts_in_host != nullptr );
+    // 4 layers: 31.2 and 35.2).  Below 1024 tokens or 10 MB a copy is shorter than what the cuts cost (7B, 1 layer: 1040 tokens 833 us in one,
+    // 864 in two; 1500 tokens 1151 and 1024).
+    const bool pipelined
+      = n >= 1024 && n * Config::dim * sizeof( DType ) >= 10'000'000 && !( first_layer == 0 && token_ids != nullptr ) && ( acts_in_host != nullptr );
     std::vector<std::pair<uint64_t, uint64_t>> chunks; // (first row, rows)
     if ( pipelined ) {
       ensure_copy_stream();
@@ -401,9 +403,13 @@ public:
       // 2 bytes at 55 GB/s, so each run is that much shorter than the one before.
       const double rate = 3.0 * Config::hidden_dim * 55e9 / ( 650e12 * sizeof( DType ) );
       const double part = std::clamp( 1.0 - 1.0 / rate, 0.3, 0.6 );
+      // The products of a few hundred rows run at half their rate: a smaller model's runs are no shorter than some 1000 rows (7B, 1 layer, 2400
+      // tokens: 1759 us as 768 + 512 + 512 + 608, 1645 in one, 1515 as 1536 + 864; 4400 tokens: 2656, 2835 and as 2560 + 1024 + 816 2363).
+      const uint64_t last = part < 0.5 ? 1280 : 768;
       uint64_t r0 = 0;
-      while ( n - r0 > std::max<uint64_t>( 768, n / 8 ) && chunks.size() + 1 < N_CHUNKS ) {
-        const uint64_t rows = std::max<uint64_t>( 1, static_cast<uint64_t>( part * static_cast<double>( n - r0 ) / 256.0 + 0.5 ) ) * 256; // whole tiles
+      while ( ( r0 == 0 || n - r0 > std::max<uint64_t>( last, n / 8 ) ) && chunks.size() + 1 < N_CHUNKS ) {
+        const double rest = static_cast<double>( n - r0 ), this_part = std::max( part, std::min( 0.6, 2600.0 / rest ) );
+        const uint64_t rows = std::max<uint64_t>( 1, static_cast<uint64_t>( this_part * rest / 256.0 + 0.5 ) ) * 256; // whole tiles
         if ( r0 + rows >= n ) {
           break;
         }
@@ -422,13 +428,7 @@ public:
       }
     } else {
       GLINT_CHECK( acts_in_host != nullptr );
-      if ( pipelined ) {
-        for ( size_t c = 0; c < chunks.size(); c++ ) {
-          const uint64_t off = chunks[c].first * Config::dim;
-          GLINT_GH( gh_memcpy( px + off, acts_in_host + off, chunks[c].second * Config::dim * sizeof( DType ), GH_HOST_TO_DEVICE, 1, copy_lane_->stream ) );
-          GLINT_GH( gh_event_record( copy_lane_->in[c], copy_lane_->stream ) );
-        }
-      } else {
+      if ( !pipelined ) {
         ops_.copy( px, acts_in_host, n * Config::dim * sizeof( DType ), CopyType::HostToDevice, true );
       }
     }
@@ -463,6 +463,9 @@ public:
         for ( size_t c = 0; c < ( by_run ? chunks.size() : 1 ); c++ ) {
           const uint64_t r0 = by_run ? chunks[c].first : 0, rows = by_run ? chunks[c].second : n;
           if ( by_run ) {
+            // a copy of memory that is not page-locked keeps the host: the work on the runs before it is queued by then
+            GLINT_GH( gh_memcpy( px + r0 * Config::dim, acts_in_host + r0 * Config::dim, rows * Config::dim * sizeof( DType ), GH_HOST_TO_DEVICE, 1, copy_lane_->stream ) );
+            GLINT_GH( gh_event_record( copy_lane_->in[c], copy_lane_->stream ) );
             GLINT_GH( gh_stream_wait_event( ops_.stream(), copy_lane_->in[c] ) );
             ops_.template rmsnorm<Config::dim>( pxb + r0 * Config::dim, px + r0 * Config::dim, reinterpret_cast<float32_t*>( temp_ ), w.rms_att_weight, rows );
           }
@@ -516,16 +519,19 @@ public:
           }
           if ( out_by_run ) {
             GLINT_GH( gh_event_record( copy_lane_->out[c], ops_.stream() ) );
-            GLINT_GH( gh_stream_wait_event( copy_lane_->stream, copy_lane_->out[c] ) );
-            GLINT_GH( gh_memcpy( acts_out_host + r0 * Config::dim, cx, rows * Config::dim * sizeof( DType ), GH_DEVICE_TO_HOST, 1, copy_lane_->stream ) );
           }
         }
       }
     }
 
     if ( acts_out_host != nullptr ) {
-      if ( pipelined ) {
-        GLINT_GH( gh_sync( copy_lane_->stream ) ); // the downloads queued behind the last layer
+      if ( pipelined ) { // (all work is queued by now: see the uploads)
+        for ( size_t c = 0; c < chunks.size(); c++ ) {
+          const uint64_t off = chunks[c].first * Config::dim;
+          GLINT_GH( gh_stream_wait_event( copy_lane_->stream, copy_lane_->out[c] ) );
+          GLINT_GH( gh_memcpy( acts_out_host + off, px + off, chunks[c].second * Config::dim * sizeof( DType ), GH_DEVICE_TO_HOST, 1, copy_lane_->stream ) );
+        }
+        GLINT_GH( gh_sync( copy_lane_->stream ) );
       } else {
         ops_.copy( acts_out_host, px, n * Config::dim * sizeof( DType ), CopyType::DeviceToHost );
       }
@@ -965,6 +971,9 @@ private:
   ModelOptions options_;
   LlamaOperations ops_;
 
+  // Tokens up to which a prefill's products carry their follow-up ops: the ring kernel takes them at once and the fp32 sums stay small
+  // (70B, 132 tokens, 2 layers: 983 us, as separate ops 1056; 7B, 150 tokens, 4 layers: 746 and 952).
+  static constexpr uint64_t PREFILL_FUSED_ROWS = 256;
   // prefill scratch: activations for `pf_capacity_` tokens, grown on demand
   void ensure_prefill_scratch( const uint64_t n )
   {
@@ -976,7 +985,7 @@ private:
     pf_xb_ = ops_.device_allocate( n * Config::dim * sizeof( DType ) );
     pf_q_ = ops_.device_allocate( n * Config::dim * sizeof( DType ) );
     pf_hb_ = ops_.device_allocate( n * Config::hidden_dim * sizeof( DType ) );
-    if ( n >= 128 ) {
+    if ( n > PREFILL_FUSED_ROWS ) {
       pf_hb2_ = ops_.device_allocate( n * Config::hidden_dim * sizeof( DType ) );
       pf_xb2_ = ops_.device_allocate( n * Config::dim * sizeof( DType ) );
       pf_kv_ = ops_.device_allocate( n * Config::kv_dim * 2 * sizeof( DType ) );
@@ -988,9 +997,6 @@ private:
     pf_attn_ws_ = ops_.device_allocate( std::max<uint64_t>( pf_attn_ws_bytes_, 16 ) );
     pf_capacity_ = n;
   }
-  // Tokens up to which a prefill's products carry their follow-up ops: the ring kernel takes them at once and the fp32 sums stay small
-  // (70B, 132 tokens, 2 layers: 983 us, as separate ops 1056; 7B, 150 tokens, 4 layers: 746 and 952).
-  static constexpr uint64_t PREFILL_FUSED_ROWS = 256;
   // the stream and events of the pipelined prefill, created on first use and kept for the life of the model
   static constexpr size_t N_CHUNKS = 8;
   struct CopyLane

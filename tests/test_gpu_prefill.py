@@ -297,14 +297,17 @@ def test_stage_prefill_copies_overlapped_with_compute_equal_plain_call():
     b.close()
 
 
-@pytest.mark.parametrize("hosted,batch,T", [(1, 2, 550),      # one layer, the first and the last at once; a last run that is no multiple of 256
-                                            (2, 4, 257)])     # 1028 tokens: just cut
-def test_stage_prefill_short_runs_equal_plain_calls(hosted, batch, T):
+@pytest.mark.parametrize("buffers", [ops.pinned_empty, np.empty], ids=["page-locked", "pageable"])
+@pytest.mark.parametrize("hosted,batch,T", [(1, 2, 550), (2, 4, 257),     # not cut: too short a copy
+                                            (1, 2, 650),      # one layer, the first and the last at once; a last run that is no multiple of 256
+                                            (2, 5, 257),      # 1285 tokens: just cut
+                                            (1, 4, 1100)])    # three runs
+def test_stage_prefill_short_runs_equal_plain_calls(hosted, batch, T, buffers):
     """A call whose rows are cut into runs of falling length against calls of one context each, too short to be cut: the same outputs
     but for the order of fp32 sums (the products are split differently), so to a rounding of f16 here and there."""
     first, dim = 8, 4096
     a, b = (S.Stage("llama2-7b", "f16", first, hosted, batch, batch, seed=3, weight_std=0.02) for _ in range(2))
-    x, y = ops.pinned_empty((batch * T, dim), np.float16), ops.pinned_empty((batch * T, dim), np.float16)
+    x, y = buffers((batch * T, dim), np.float16), buffers((batch * T, dim), np.float16)
     x[:] = np.random.default_rng(6).standard_normal(x.shape).astype(np.float16)
     ids = [40 + i for i in range(batch)]
     assert a.prefill(ids, [0] * batch, T, first, activations=x, out=y) is not None
