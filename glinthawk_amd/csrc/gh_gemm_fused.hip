@@ -447,9 +447,11 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
   GH_REQUIRE( residual != nullptr, "gh_matmul_accum: NULL residual" );
   GH_REQUIRE( ( norm_out == nullptr ) == ( norm_weight == nullptr ), "gh_matmul_accum: norm_out and norm_weight go together" );
   hipStream_t st = as_stream( stream );
-  // gh_rmsnorm takes 16-byte aligned buffers only: other ones go through fp32 sums and the row kernel, which reads them element by element
+  // gh_rmsnorm takes 16-byte aligned buffers only: other ones go through fp32 sums and the row kernel, which reads them element by element.  So do fp32
+  // rows beyond 8192, which that kernel's 1024 threads take faster (4 x 32000: 20, with gh_rmsnorm 29).
   const bool norm_kernel = norm_out == nullptr
-                           || ( ( reinterpret_cast<uintptr_t>( residual ) | reinterpret_cast<uintptr_t>( norm_out ) | reinterpret_cast<uintptr_t>( norm_weight ) ) & 15u ) == 0;
+                           || ( ( dt != GH_F32 || r <= 8192 )
+                                && ( ( reinterpret_cast<uintptr_t>( residual ) | reinterpret_cast<uintptr_t>( norm_out ) | reinterpret_cast<uintptr_t>( norm_weight ) ) & 15u ) == 0 );
   // a residual that lies over the activations gets its product through fp32 sums: every row of them is read before the first is stored
   const bool apart = !overlap( residual, b * r * dtype_size( dt ), x, b * s * dtype_size( dt ) );
   if ( dt == GH_F32 && norm_kernel && apart ) {
