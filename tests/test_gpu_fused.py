@@ -19,7 +19,7 @@ def _init():
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("b,s,r", [(4, 288, 288), (64, 1024, 512), (5, 768, 1000), (3, 100, 36),
-                                   # more rows than one streaming slab: the tile kernels write the partials
+                                   # more than 64 rows: any of the kernels leaves the partial sums
                                    (100, 512, 260), (256, 1024, 512), (300, 4096, 1000),
                                    # enough 256-token tiles: the residual is added in the large tile kernel's epilogue (f16, r % 8 == 0)
                                    (768, 8192, 16384), (2048, 512, 6152), (3000, 1024, 6144), (2300, 512, 8192),
@@ -163,9 +163,9 @@ def check_matmul_silu_gate(dt, b, s, hidden, product_route):
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("b,s,hidden", [(4096, 256, 8192), (2300, 576, 4104), (2100, 640, 6152), (300, 4096, 12544), (77, 520, 2052), (200, 512, 16404), (5, 4096, 11008)])
 def test_matmul_gate_in_epilogue(b, s, hidden, bias, activation):
-    """Against 64 bits, bf16.  One rounding of the result, off by 2^-8 of it; from 192 rows on the factors may be rounded as well, before
-    the bias is added: off by 2^-8 of the plain product each, which reaches the output times the other factor (and times the activation's
-    slope, at most 1.13).  1 % for the second order; 1e-3 for fp32 sums and the fast exponential."""
+    """Against 64 bits, bf16.  The gate works on the fp32 sums: one rounding, off by 2^-8 of the result, and 1e-4 for the sums and the fast
+    exponential.  From 192 rows on the tanh gate and biases are a kernel of their own over rounded factors: off by 2^-8 of the plain product
+    each, which reaches the output times the other factor (and times the activation's slope, at most 1.13), 1 % for the second order."""
     g = torch.Generator(device="cuda").manual_seed(b + hidden)
     x = torch.randn((b, s), generator=g, device="cuda").bfloat16()
     w = (torch.randn((2 * hidden, s), generator=g, device="cuda") / s ** 0.5).bfloat16()
@@ -175,7 +175,9 @@ def test_matmul_gate_in_epilogue(b, s, hidden, bias, activation):
     y = raw + (add.double() if bias else 0.0)
     a, u = y[:, :hidden], y[:, hidden:]
     act = a * torch.sigmoid(a) if activation == ops.GH_ACT_SILU else torch.nn.functional.gelu(a, approximate="tanh")
-    bound = 1.01 * 2.0 ** -8 * ((act * u).abs() + 1.13 * (raw[:, :hidden] * u).abs() + (act * raw[:, hidden:]).abs()) + 1e-3
+    bound = 2.0 ** -8 * (act * u).abs() + 1e-4
+    if b >= 192 and (bias or activation != ops.GH_ACT_SILU):
+        bound = 1.01 * (bound + 2.0 ** -8 * (1.13 * (raw[:, :hidden] * u).abs() + (act * raw[:, hidden:]).abs())) + 1e-3
     assert ((got - act * u).abs() <= bound).all()
 
 

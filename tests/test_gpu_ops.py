@@ -186,7 +186,7 @@ def test_matmul(dt, b, s, r):
         np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-5)
 
 
-# many rows of x at once (prompt tokens): the MFMA tile kernel, ragged edges in both dimensions
+# many rows of x at once (prompt tokens), whichever kernel takes them: ragged edges in both dimensions
 @pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("b,s,r", [(128, 64, 128), (130, 512, 200), (257, 288, 288), (300, 72, 37), (512, 1024, 130),
                                    (1000, 776, 514), (129, 100, 64)])
@@ -200,20 +200,16 @@ def test_matmul_many_rows(dt, b, s, r):
     assert_close(got, want, what=f"matmul {dt} {b}x{s}x{r}")
 
 
-# enough 256-token tiles for the second tile kernel (forced with 256 and with 384 rows per work-group, and
-# whatever the dispatcher picks), ragged edges; the row counts leave 4, 0 and 6 (256) / 3, 6 and 7 (384)
-# row tiles beyond a multiple of 8, the part of the tile order that is cut into equal runs per XCD
-@pytest.mark.parametrize("force,rows", [(4, 256), (4, 384), (4, 128), (4, 129), (4, 0), (0, 0)])
+# enough 256 x 256 tiles for the large tile kernel, forced and as the dispatcher has it, ragged edges; the row counts leave 1, 0 and 7 row tiles
+# beyond a multiple of 8, the part of the tile order that is cut into equal runs per XCD; an odd number of steps in the last
+@pytest.mark.parametrize("force", [4, 0])
 @pytest.mark.parametrize("b,s,r", [(3000, 8192, 4100), (8200, 128, 8190), (700, 8256, 18000)])
-def test_matmul_256_tiles(force, rows, b, s, r):
+def test_matmul_256_tiles(force, b, s, r):
     from glinthawk_amd import _lib
-    if rows in (128, 129) and s % 128:
-        pytest.skip("the four-wave kernel (tile rows 128: one tile per work-group, 129: equal shares of all steps) takes K ranges of an even "
-                    "number of 64-k steps; the dispatcher takes the eight-wave one here")
     rng = np.random.default_rng(26)
     x = rng.standard_normal((b, s)).astype(np.float16)
     w = (rng.standard_normal((r, s)) / np.sqrt(s)).astype(np.float16)
-    _lib.lib().gh_gemm_set_tuning(force, 0, rows)
+    _lib.lib().gh_gemm_set_tuning(force, 0, 0)
     try:
         got = ops.matmul(torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda())
     finally:
@@ -226,18 +222,17 @@ def test_matmul_256_tiles(force, rows, b, s, r):
     assert_close(got[:8].cpu().numpy(), want_cpu, what=f"matmul 256-tile {b}x{s}x{r}")
 
 
-@pytest.mark.parametrize("rows", [256, 384, 128, 129])
-@pytest.mark.parametrize("s,r,b", [(8192, 12544, 1030),    # 49 / 33 row tiles x 5: one left-over row tile
-                                   (1024, 5000, 16390),    # 20 / 14 row tiles x 65: 4 / 6 left over, ragged last token tile
-                                   (256, 1700, 9000)])     # 7 / 5 row tiles: left-over tiles only
-def test_matmul_256_tile_one_hot_layout(rows, s, r, b):
+@pytest.mark.parametrize("s,r,b", [(8192, 12544, 1030),    # 49 row tiles x 5: one left-over row tile
+                                   (1024, 5000, 16390),    # 20 row tiles x 65: 4 left over, ragged last token tile
+                                   (256, 1700, 9000)])     # 7 row tiles: left-over tiles only
+def test_matmul_256_tile_one_hot_layout(s, r, b):
     """One-hot activations: every output is one weight, so each tile of the order must land bit for bit."""
     from glinthawk_amd import _lib
     w = torch.arange(r * s, dtype=torch.float32, device="cuda").reshape(r, s).remainder(1000).half()
     x = torch.zeros((b, s), dtype=torch.float16, device="cuda")
     cols = [(7919 * i + 3) % s for i in range(b)]
     x[torch.arange(b), torch.tensor(cols)] = 1
-    _lib.lib().gh_gemm_set_tuning(4, 0, rows)
+    _lib.lib().gh_gemm_set_tuning(4, 0, 0)
     try:
         got = ops.matmul(x, w)
     finally:
@@ -246,12 +241,12 @@ def test_matmul_256_tile_one_hot_layout(rows, s, r, b):
 
 
 @pytest.mark.parametrize("epilogue", ["store", "accum", "pair"])
-def test_matmul_equal_shares_of_all_steps(epilogue):
-    """The four-wave kernel over equal shares of all 64-k steps (tile rows 129): shares that end inside tiles leave pieces that a
-    second kernel adds in a fixed order.  Ragged tiles in both directions, shares shorter and longer than a tile, all three outputs
+def test_matmul_256_tiles_walked(epilogue):
+    """More tiles than CUs, so that a work-group takes one after the other without draining (an even number of steps), the same with a
+    work-group for each tile (an odd number), and a single round.  Ragged tiles in both directions behind whole ones, all three outputs
     (plain, residual add, two matrices); one-hot activations bit for bit, a random product twice with identical bits."""
     from glinthawk_amd import _lib
-    for b, s, r in [(3000, 1280, 4104), (1100, 2560, 15880), (2300, 768, 8968)]:     # 204, 315 and 324 tiles of 20, 40 and 12 steps; shares of 16, 50 and 16
+    for b, s, r in [(3000, 1280, 4104), (1100, 2560, 15880), (2300, 1536, 8968), (2300, 1600, 8968)]:     # 204, 315, 324 and 324 tiles of 20, 40, 24 and 25 steps
         w = torch.arange(r * s, dtype=torch.float32, device="cuda").reshape(r, s).remainder(1000).half()
         hot = torch.zeros((b, s), dtype=torch.float16, device="cuda")
         cols = torch.tensor([(7919 * i + 3) % s for i in range(b)], device="cuda")
@@ -260,7 +255,7 @@ def test_matmul_equal_shares_of_all_steps(epilogue):
         x = torch.randn((b, s), generator=g, device="cuda").half()
         wr = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).half()
         res = torch.randn((b, r), generator=g, device="cuda").half()
-        _lib.lib().gh_gemm_set_tuning(4 if epilogue == "store" else 0, 0, 129)
+        _lib.lib().gh_gemm_set_tuning(0 if epilogue == "pair" else 4, 0, 1)     # two matrices: the dispatcher's choice, which is this kernel; no cut along b
         try:
             if epilogue == "store":
                 got_hot, first, again = ops.matmul(hot, w), ops.matmul(x, wr), ops.matmul(x, wr)
@@ -340,16 +335,22 @@ def test_matmul_streaming_kernel_sweep(b, s, r):
 def test_matmul_ring_edges(dt, b, s, r):
     """One-hot activations: every output is one weight, bit for bit.  A random product: fp32 sums, so off by the result's own rounding
     (half an ulp, relative 2^-11 or 2^-8) and by the order of the sums (s terms of about s^-1/2: far below 1e-4 of their scale)."""
+    from glinthawk_amd import _lib
     g = torch.Generator(device="cuda").manual_seed(b * 13 + r)
     w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).to(dt)
     hot = torch.zeros((b, s), dtype=dt, device="cuda")
     cols = torch.tensor([(7919 * i + 3) % s for i in range(b)], device="cuda")
     hot[torch.arange(b, device="cuda"), cols] = 1
     x = torch.randn((b, s), generator=g, device="cuda").to(dt)
-    assert torch.equal(ops.matmul(hot, w), w[:, cols].t().contiguous())
+    _lib.check(_lib.lib().gh_gemm_set_tuning(5, 0, 0))
+    try:
+        got_hot, got = ops.matmul(hot, w), ops.matmul(x, w)
+    finally:
+        _lib.check(_lib.lib().gh_gemm_set_tuning(0, 0, 0))
+    assert torch.equal(got_hot, w[:, cols].t().contiguous())
     want = x.double() @ w.double().t()
     bound = want.abs() * (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 1e-4
-    assert ((ops.matmul(x, w).double() - want).abs() <= bound).all()
+    assert ((got.double() - want).abs() <= bound).all()
 
 
 # the 128 x 128 tile kernel: K ranges that end inside a step, of one step and of several K splits; rows that leave whole 16-byte chunks, four at a time
@@ -405,9 +406,8 @@ def test_matmul_rounds_and_rests_one_hot(dt, b, s, r):
     assert torch.equal(ops.matmul(x, w), w[:, cols].t().contiguous())
 
 
-# some hundred rows (the decode step of a large slot arena): whatever the dispatcher picks at each batch size (streaming kernel up
-# to 64 rows, 128 x 128 tiles with or without a K split, 256-token tiles with the K range split over work-groups when the tiles are
-# few), ragged edges in rows, tokens and K steps.  One-hot activations: every output is one weight, bit for bit.
+# some hundred rows (the decode step of a large slot arena): whatever the dispatcher picks at each batch size (the ring kernel, 128 x 128
+# tiles, 256 x 256 tiles with the K range split over work-groups when the tiles are few), ragged edges in rows, tokens and K steps.  One-hot activations: every output is one weight, bit for bit.
 @pytest.mark.parametrize("b", [65, 128, 192, 256, 300, 512])
 @pytest.mark.parametrize("s,r", [(2048, 1024), (2112, 1000), (8192, 2560), (4096, 516)])
 def test_matmul_some_hundred_rows(b, s, r):
