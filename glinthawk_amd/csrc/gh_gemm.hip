@@ -1,14 +1,13 @@
-// Dense projection GEMM of the stage: xout(b, r) = sum_p w(r, p) * x(b, p), w row-major (r, s),
-// fp32 accumulate (Operations::matmul / untemplated_matmul, arch/amd64/common/ops.hh:74-93,212-271).
+// Dense projection GEMM of the stage: xout(b, r) = sum_p w(r, p) * x(b, p), w row-major (r, s), fp32 accumulate
+// (Operations::matmul / untemplated_matmul, arch/amd64/common/ops.hh:74-93,212-271): which kernel takes a product, and the entry points.
 //
-// f16, bf16: MFMA kernel.  The weight matrix is the streamed operand (read exactly once), the
-// activations are the small operand.  A work-group owns a 64-row slab of w and a 64-column slab of
-// the batch, walks K in steps of 128, stages both tiles in LDS with 16-byte chunks XOR-swizzled so
-// that the MFMA-operand reads are bank-conflict free, and keeps 4 x (16x16) fp32 accumulators per
-// wave (v_mfma_f32_16x16x32_f16 / _bf16).  When r / 64 is too small to fill the chip K is split across
-// work-groups and an fp32 partial buffer is reduced by a second kernel.
-//
-// f32: gh_gemm_f32.hip.
+//   f16, bf16   s % 8 == 0 and 16-byte aligned operands: the ring kernel (gh_gemm_ring.hip), 128 x 128 tiles (gh_gemm_tile.hip) or 256 x 256 tiles
+//               (gh_gemm_tile256.hip), by estimated time: half_plan()
+//   otherwise   the kernel of this file.  A work-group owns a 64-row slab of w and a 64-column slab of the batch, walks K in steps of 128,
+//               stages both tiles in LDS with 16-byte chunks XOR-swizzled so that the MFMA-operand reads are bank-conflict free, and keeps
+//               4 x (16x16) fp32 accumulators per wave (v_mfma_f32_16x16x32_f16 / _bf16).  Where r / 64 is too small to fill the chip K is
+//               split across work-groups and an fp32 partial buffer is reduced by a second kernel.
+//   f32         gh_gemm_f32.hip
 #include "gh_product.h"
 
 #include <cstdlib>
@@ -297,10 +296,6 @@ __global__ __launch_bounds__( 256 ) void gemm_skinny_kernel( float* __restrict__
 
 namespace gh {
 
-// Runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums
-// `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue;
-// otherwise the kernel may store DType results straight into `xout` (*splits_out == 0 then).
-
 // The stores of the ring kernel, 8 bytes a lane with nothing to hide them; what the steps of a long K range are priced at covers part of it
 // (32000 x 64 at 7000 rows: 400 us, of which the one step is 20).
 static double ring_stores_ns( uint64_t s, uint64_t r, uint64_t b ) { return (double)( b * r ) / 1000.0 * std::min( 1.0, 1024.0 / (double)s ); }
@@ -506,7 +501,9 @@ int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_
   } );
 }
 
-// the 16-bit part of gemm_partials()
+// The 16-bit part of gemm_partials(): runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums
+// `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue; otherwise the kernel may store
+// DType results straight into `xout` (*splits_out == 0 then).
 template<typename E>
 int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st, bool want_partials, float** partial_out,
                         uint32_t* splits_out )
@@ -523,15 +520,6 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
     GH_LAUNCH_CHECK();
     return GH_OK;
   }
-  auto planes = [&]( uint32_t n, float** ws ) { // room for the fp32 sums of n K ranges
-    *partial_out = nullptr;
-    if ( int rc = ensure_workspace( (uint64_t)n * b * r * sizeof( float ), ws, st ) ) {
-      return rc;
-    }
-    *partial_out = *ws;
-    *splits_out = n;
-    return (int)GH_OK;
-  };
   const void* out = xout ? static_cast<const void*>( xout ) : x;
   HalfPlan plan;
   bool taken = false; // by one of the kernels for aligned operands
@@ -562,9 +550,11 @@ int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r,
   if ( taken ) {
     float* ws = nullptr;
     if ( want_partials || plan.splits > 1 ) {
-      if ( int rc = planes( plan.splits, &ws ) ) {
+      if ( int rc = ensure_workspace( (uint64_t)plan.splits * b * r * sizeof( float ), &ws, st ) ) {
         return rc;
       }
+      *partial_out = ws;
+      *splits_out = plan.splits;
     }
     switch ( plan.kernel ) {
       case HalfKernel::tile128: return gemm_tile_launch( xout, ws, x, w, s, r, b, plan.splits, plan.k_len, st );

@@ -439,12 +439,14 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
 
 int g_tile_rows = 0; // tuning hook: non-zero leaves every product whole (no cut along the tokens)
 
-// Rounds of one work-group per CU that an XCD (32 CUs) runs for its share of the tiles.
+uint64_t cus_per_xcd() { return std::max<uint64_t>( 1, (uint64_t)cu_count() / 8 ); } // 32
+
+// Rounds of one work-group per CU that an XCD runs for its share of the tiles.
 uint64_t rounds_per_xcd( uint64_t r, uint64_t b )
 {
   const uint64_t row_tiles = ( r + TM2 - 1 ) / TM2, token_tiles = ( b + TN2 - 1 ) / TN2;
   const uint64_t tiles = ( row_tiles / 8 ) * token_tiles + ( ( row_tiles % 8 ) * token_tiles + 7 ) / 8;
-  return ( tiles + 31 ) / 32;
+  return ( tiles + cus_per_xcd() - 1 ) / cus_per_xcd();
 }
 
 } // namespace
@@ -552,7 +554,8 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   // share of all tiles (13824 x 5120 at 16384 tokens, 54 row tiles: 14 either way, 1 % faster); else the row tiles beyond a multiple
   // of 8 are shared out (20 row tiles: 5 rounds against 6; with 4 splits of 3 token tiles 32 work-groups per XCD against 36, 110 us against 149).
   const uint64_t tokens = ord.token_tiles, even = ( row_tiles / 8 ) * tokens + ( ( row_tiles % 8 ) * tokens + 7 ) / 8, whole = ( row_tiles + 7 ) / 8 * tokens;
-  ord.rest_rows = ( whole * splits + 31 ) / 32 <= ( even * splits + 31 ) / 32 ? 0 : row_tiles % 8;
+  const uint64_t per_cu = cus_per_xcd();
+  ord.rest_rows = ( whole * splits + per_cu - 1 ) / per_cu <= ( even * splits + per_cu - 1 ) / per_cu ? 0 : row_tiles % 8;
   ord.owned = row_tiles - ord.rest_rows;
   // The 32 tiles an XCD works on at a time read gm + gn operand strips into its L2: strips of equal height, at most 6 row tiles, and
   // patches of equal width that make 32 tiles with that (6 x 5: 11 strips; heights of 4 and 2 with patches 8 wide: 12 and 18).
@@ -564,7 +567,6 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   const uint64_t per_xcd = ord.rest_rows == 0 ? whole : even; // the longest list
   GH_REQUIRE( 8 * per_xcd < ( 1ull << 31 ), "gh_matmul: grid too large" );
   const TileOut out { xout, xout2, partial, (uint32_t)r, (uint32_t)b, (uint32_t)r_first, gate != nullptr ? *gate : GateRows {} };
-  const uint64_t per_cu = std::max<uint64_t>( 1, (uint64_t)cu_count() / 8 );
   const bool walk = per_xcd > per_cu && epi != EPI_PARTIAL && s % ( 2 * TKS ) == 0;
   const dim3 grid( (unsigned)( 8 * ( walk ? per_cu : per_xcd ) ), splits );
 #define GH_TILE256( EP, WALK ) gemm_tile256_kernel<E, EP, WALK><<<grid, T256_THREADS, 0, st>>>( x, w, (uint32_t)s, k_len, out, ord )
