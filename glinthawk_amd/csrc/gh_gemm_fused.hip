@@ -485,8 +485,10 @@ int gh_matmul_accum( void* residual, const void* x, const void* w, uint64_t s, u
       return norm_out != nullptr ? gh_rmsnorm( norm_out, residual, norm_weight, r, b, dt, stream ) : GH_OK;
     }
   }
-  if ( const uint64_t b1 = apart ? gemm_token_split( s, r, b, dt, x, w, residual ) : 0 ) { // two products along the tokens (rows are independent)
-    const uint64_t elem = 2;
+  // Two products along the tokens (rows are independent), unless norms of the first part lie over activations that the second reads: rows of x as
+  // long as the normed ones, in one buffer, do not.
+  const uint64_t elem = 2, b1 = apart ? gemm_token_split( s, r, b, dt, x, w, residual ) : 0;
+  if ( b1 != 0 && !overlap( norm_out, b1 * r * elem, static_cast<const char*>( x ) + b1 * s * elem, ( b - b1 ) * s * elem ) ) {
     if ( int rc = gh_matmul_accum( residual, x, w, s, r, b1, norm_out, norm_weight, dt, stream ) ) {
       return rc;
     }

@@ -112,6 +112,24 @@ def test_outputs_over_their_activations(dt, b, s):
     assert torch.allclose(got.float(), q.float(), **tol) and torch.allclose(over.float(), cache.float(), **tol)
 
 
+@pytest.mark.parametrize("b,s,r", [(2080, 1024, 8192), (3080, 2048, 5120)])
+def test_norm_over_activations_of_shorter_rows(b, s, r):
+    """The norm's rows in the buffer of the activations, whose rows are shorter, where the product is better run in two parts along the tokens: norms
+    of the first must not land on activations of the second.  The parts may sum in another order: a rounding of f16."""
+    g = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, s), generator=g, device="cuda").half()
+    w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).half()
+    res = torch.randn((b, r), generator=g, device="cuda").half()
+    nw = (1 + 0.1 * torch.randn(r, generator=g, device="cuda")).half()
+    want_res = res.clone()
+    want_norm = ops.matmul_accum(want_res, x, w, nw)
+    both = torch.empty((b, r), dtype=torch.float16, device="cuda")
+    both.flatten()[: x.numel()] = x.flatten()
+    _lib.check(_lib.lib().gh_matmul_accum(ops._p(res), ops._p(both), ops._p(w), s, r, b, ops._p(both), ops._p(nw), ops._dt(x), ops._stream()))
+    assert torch.allclose(res.float(), want_res.float(), rtol=4e-3, atol=4e-3)
+    assert torch.allclose(both.float(), want_norm.float(), rtol=4e-3, atol=4e-3)
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
                                         # enough row tiles for one launch without a K split: both factors in one kernel
