@@ -251,10 +251,10 @@ def test_stage_prefill_middle_stage_and_chunks():
 
 
 def test_stage_prefill_copies_overlapped_with_compute_equal_plain_call():
-    """From 8192 tokens on, a prefill that takes activations from the host cuts the rows into four runs whose copies overlap the
-    first and the last row-wise products.  Same contexts in one such call (4 x 2048 tokens) and in two plain calls (2 x 2048
-    each): the outputs and the cache rows agree (the products of the runs may be split differently, so to rounding).  Then a
-    second chunk of 2048 tokens per context from position 2048 on, without activations out (only the upload is cut into runs)."""
+    """A long prefill that takes activations from the host cuts the rows into runs whose copies overlap the first and the last row-wise
+    products.  Same contexts in one such call (4 x 2048 tokens) and in plain calls (512 tokens of one context each, too few to be cut):
+    the outputs and the cache rows agree (the products may be split differently, so to rounding).  Then a second chunk of 2048 tokens
+    per context from position 2048 on, without activations out (only the upload is cut into runs)."""
     first, hosted, batch, T = 8, 2, 4, 2048
     a = S.Stage("llama2-13b-4k", "f16", first, hosted, batch, batch, seed=3, weight_std=0.02)
     b = S.Stage("llama2-13b-4k", "f16", first, hosted, batch, batch, seed=3, weight_std=0.02)
@@ -270,10 +270,10 @@ def test_stage_prefill_copies_overlapped_with_compute_equal_plain_call():
         res = a.prefill(ids, [start] * batch, T, first, activations=x, out=ya if want_out else None, want_activations=want_out)
         assert res is not None and (res[0] is ya) == want_out
         yb = np.zeros((batch * T, dim), np.float16)
-        for half in range(2):
-            rows = slice(half * 2 * T, (half + 1) * 2 * T)
-            res = b.prefill(ids[2 * half:2 * half + 2], [start, start], T, first, activations=x[rows], out=yb[rows])
-            assert res is not None
+        for i in range(batch):
+            for t in range(0, T, 512):
+                rows = slice(i * T + t, i * T + t + 512)
+                assert b.prefill(ids[i:i + 1], [start + t], 512, first, activations=x[rows], out=yb[rows]) is not None
         return yb
 
     yb = both(0, True)
