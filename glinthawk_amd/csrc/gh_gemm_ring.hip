@@ -324,7 +324,8 @@ int g_ring_cus = 0; // tuning override of the CU count the plan balances for (0:
 // The tile, the rows of a work-group and the K split.  A CU takes one work-group at a time, so a launch is as slow as its rounds of
 // work-groups.  Fitted to timings of the 7B, 13B and 70B shapes, up to 256 rows with cold weights, and 300 to 7000.  A step costs its
 // weights at the CU's share of the memory's rate (4.7 ns a row) and its activations at what L2 delivers to a CU (2 ns a row), but no
-// less than a load's time in flight (1.9 us) over the steps requested ahead.  With several slabs the weights come from L2 and the
+// less than a load's time in flight (1.9 us) over the steps requested ahead; 1.5 us with the gate in wide tiles, whose ring_plan() is weighed against two
+// launches (2 x 11008 of 4096 k at 77 rows: 37 us so, 43 as two, for which 1.9 us spoke; 2 x 5632 of 2048 at 65: 18 and 23).  With several slabs the weights come from L2 and the
 // matrix units set the pace; wide slabs slow each other down.  A round costs what it takes to fill the ring, and a split the fp32 sums
 // that are written and read again, and RING_SPLIT_NS.  A work-group that fills three wide stages
 // first starts later (4096 x 512 at 256 rows: 16 us for 8 steps), of which the steps of a long range are priced to cover a part.
@@ -353,7 +354,8 @@ RingPlan find_ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate, uint64_t
           const uint64_t row_blocks = ( r + rows - 1 ) / rows;
           const double real_rounds = (double)( ( row_blocks * slabs * splits + n_cu - 1 ) / n_cu );
           const double w_rows = (double)( gate ? 2 * rows : rows ), x_rows = (double)std::min<uint64_t>( cols, b );
-          const double step_ns = slabs == 1 ? std::max( 4.7 * w_rows + 2.0 * x_rows, 1900.0 / ( ring_stages( w, x ) - 1 ) )
+          const double flight_ns = gate && ring_stages( w, x ) < 6 ? 1500.0 : 1900.0;
+          const double step_ns = slabs == 1 ? std::max( 4.7 * w_rows + 2.0 * x_rows, flight_ns / ( ring_stages( w, x ) - 1 ) )
                                             : 1.05 * ( 2.9 * w_rows + 1.05 * ( x_rows + x ) + ( x > 128 ? 20.0 + 7.0 * (double)slabs : 40.0 ) );
           const double start_ns = slabs > 1 ? 3000.0 : x < 192 ? 2000.0 : 2000.0 + 4000.0 * std::min( 1.0, 16.0 / (double)per );
           const double sums_ns = splits > 1 ? (double)( splits * b * r ) * 8.0 / 5000.0 + RING_SPLIT_NS : 0.0;
