@@ -381,6 +381,22 @@ def test_matmul_tiles_128_edges(dt, b, s, r):
     assert ((got.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("b", [1000, 1500])
+def test_matmul_256_tiles_with_split_k_where_faster(b):
+    """20 row tiles of 256 under four and six token tiles, a third of a round: with the K range split they were timed a tenth and more faster than the
+    ring kernel, so the default gives their bits."""
+    from glinthawk_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, 5120), generator=g, device="cuda").half()
+    w = (torch.randn((5120, 5120), generator=g, device="cuda") / 5120 ** 0.5).half()
+    got = ops.matmul(x, w)
+    _lib.check(_lib.lib().gh_gemm_set_tuning(4, 0, 0))
+    try:
+        assert torch.equal(got, ops.matmul(x, w))
+    finally:
+        _lib.check(_lib.lib().gh_gemm_set_tuning(0, 0, 0))
+
+
 # rows and K ranges at which the dispatch changes kernels: the product that the residual add carries gives the bits of the plain one and an add
 @pytest.mark.parametrize("b,s,r", [(64, 512, 512), (65, 288, 4096), (192, 768, 4096), (256, 512, 4096), (256, 8192, 5000), (700, 2048, 2048), (7000, 1024, 1024), (4096, 768, 2048)])
 def test_matmul_accum_has_the_bits_of_the_product(b, s, r):
