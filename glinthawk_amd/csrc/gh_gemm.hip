@@ -408,10 +408,10 @@ static GateKernel gate_kernel( const void* hb, const GateRows& gate, const void*
   if ( !gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride ) ) {
     return GateKernel::none;
   }
-  // From 192 rows on 256 x 256 tiles where they are enough (70B, 256 rows: 235 us with the gate behind them, the ring kernel 264).  The ring kernel
-  // splits no K range here: where too few rows fill the chip (2 x 1024 of 2048 k at 8 rows: 10.5 us) the split of the plain product with the
-  // gate's kernel behind it (about 4.5 us) is faster (9), and so are 128 x 128 tiles where the K range is short (2 x 1376 of 512 k at 224
-  // rows: 20 us, 16), but those would leave rounded factors to a gate over the fp32 sums of many rows.
+  // From 192 rows on 256 x 256 tiles where they are enough (70B, 256 rows: 221 us with the gate behind them, the ring kernel 270).  The ring kernel
+  // splits no K range here: where too few rows fill the chip (2 x 1024 of 2048 k at 8 rows: 11.6 us) the split of the plain product with the
+  // gate's kernel behind it (about 4.5 us) is faster (8.2).  A gate over the fp32 sums of many rows takes such a split only: unsplit products of so
+  // many rows leave rounded factors.
   const bool keeps_sums = gate.exact && b >= PRODUCT_ROUNDED_ROWS;
   const double ring_ns = gemm_ring_gate_ns( s, hidden, b ) + ring_stores_ns( s, hidden, b );
   double two_ns = 0.0;

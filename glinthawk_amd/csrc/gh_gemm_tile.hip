@@ -298,13 +298,14 @@ void gemm_tile_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits_out, u
 }
 
 // Without the writing and reading of sums.  Two work-groups on each CU at a time take 1.9 us and 1.23 a step of 64 k (32000 weight rows, 7000
-// tokens, 1 to 32 steps: within 4 %), and the weights leave memory at 2.9 TB/s (28672 x 8192 at 65 to 128 rows: 3.1 to 3.4).
+// tokens, 1 to 32 steps: within 4 %), the XCDs with one row tile more than others the longest (1536 x 512 at 7000 tokens, 12 row tiles: 26 us, 256 x
+// 256 tiles 20), and the weights leave memory at 2.9 TB/s (28672 x 8192 at 65 to 128 rows: 3.1 to 3.4).
 double gemm_tile_ns( uint64_t s, uint64_t r, uint64_t b )
 {
   uint32_t splits = 1, k_per_split = 0;
   gemm_tile_plan( s, r, b, &splits, &k_per_split );
-  const double groups = (double)( ( ( r + TM - 1 ) / TM ) * ( ( b + TN - 1 ) / TN ) * splits );
-  const double rounds = std::max( 1.0, groups / ( 2.0 * (double)cu_count() ) );
+  const double xcd_groups = (double)( ( ( r + TM - 1 ) / TM + 7 ) / 8 * ( ( b + TN - 1 ) / TN ) * splits );
+  const double rounds = std::max( 1.0, xcd_groups * 4.0 / (double)cu_count() );
   return std::max( rounds * ( 1900.0 + 1230.0 * (double)( k_per_split / TK ) ), 1900.0 + (double)( r * s ) * 2.0 / 2900.0 );
 }
 
