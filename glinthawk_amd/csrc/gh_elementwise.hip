@@ -143,11 +143,10 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
 }
 
 // ---- argmax: one block per row, first index of the maximum --------------------------------------
-// Bound by latency: a row of 32000 values is one work-group's, so a thread asks for ARG_AHEAD pieces of it before it compares the first.  4 fp32
-// rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  256 threads where they ask for all of a row at once (1024 rows of
-// 4096: 10.2 us, with 1024 threads 17.8), else 1024.  As a loop over the row would have it: the lowest index
-// of equal values, NaN never beats anything but stays where the row begins with it.
-constexpr int ARG_AHEAD = 8;
+// Bound by latency: a row of 32000 values is one work-group's, so a thread asks for AHEAD pieces of it before it compares the first.  4 fp32
+// rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  256 threads where they ask for all of a row at once, with the fewest
+// pieces that do (1024 f16 rows of 1000: 4.1 us, 7.5 with eight each; of 4096: 5.0, 9.3, with 1024 threads 17.6), else 1024.  As a loop over the row
+// would have it: the lowest index of equal values, NaN never beats anything but stays where the row begins with it.
 __device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float v, uint32_t i )
 {
   const bool take = v > best || ( v == best && i < best_i );
@@ -155,7 +154,7 @@ __device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float
   best_i = take ? i : best_i;
 }
 // V: values per load, n % V == 0 and rows aligned to V values
-template<typename T, int V, int ARG_THREADS>
+template<typename T, int V, int ARG_THREADS, int AHEAD>
 __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __restrict__ out, const T* __restrict__ v, uint32_t n )
 {
   __shared__ float s_val[ARG_THREADS / WAVE];
@@ -165,18 +164,19 @@ __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __rest
   {
     T e[V];
   };
+  const float first = to_f32( row[0] );
   const Piece* pieces = reinterpret_cast<const Piece*>( row );
   const uint32_t n_pieces = n / V;
   float best = -INFINITY;
   uint32_t best_i = 0xffffffffu;
-  for ( uint64_t p0 = threadIdx.x; p0 < n_pieces; p0 += ARG_THREADS * ARG_AHEAD ) {
-    Piece x[ARG_AHEAD];
+  for ( uint64_t p0 = threadIdx.x; p0 < n_pieces; p0 += ARG_THREADS * AHEAD ) {
+    Piece x[AHEAD];
 #pragma unroll
-    for ( int u = 0; u < ARG_AHEAD; u++ ) {
+    for ( int u = 0; u < AHEAD; u++ ) {
       x[u] = pieces[min( p0 + u * ARG_THREADS, (uint64_t)n_pieces - 1 )]; // past the end: the last one again, which changes nothing
     }
 #pragma unroll
-    for ( int u = 0; u < ARG_AHEAD; u++ ) {
+    for ( int u = 0; u < AHEAD; u++ ) {
       const uint32_t i0 = (uint32_t)min( p0 + u * ARG_THREADS, (uint64_t)n_pieces - 1 ) * V;
 #pragma unroll
       for ( int e = 0; e < V; e++ ) {
@@ -200,7 +200,6 @@ __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __rest
     for ( int w = 1; w < ARG_THREADS / WAVE; w++ ) {
       arg_better( best, best_i, s_val[w], s_idx[w] );
     }
-    const float first = to_f32( row[0] );
     out[blockIdx.x] = first != first || best_i == 0xffffffffu ? 0u : best_i;
   }
 }
@@ -416,10 +415,25 @@ int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n,
     using T = std::remove_pointer_t<decltype( e )>;
     constexpr int V = decltype( per_load )::value;
     const T* rows = static_cast<const T*>( v );
-    if ( n <= 256ull * ARG_AHEAD * V ) {
-      argmax_kernel<T, V, 256><<<(unsigned)batch, 256, 0, as_stream( stream )>>>( out_dev, rows, (uint32_t)n );
+    auto go = [&]( auto threads, auto ahead ) {
+      constexpr int N = decltype( threads )::value, A = decltype( ahead )::value;
+      argmax_kernel<T, V, N, A><<<(unsigned)batch, N, 0, as_stream( stream )>>>( out_dev, rows, (uint32_t)n );
+    };
+    const uint64_t pieces = n / V;
+    const std::integral_constant<int, 256> few {};
+    const std::integral_constant<int, 1024> many {};
+    if ( pieces <= 256 ) {
+      go( few, std::integral_constant<int, 1> {} );
+    } else if ( pieces <= 512 ) {
+      go( few, std::integral_constant<int, 2> {} );
+    } else if ( pieces <= 1024 ) {
+      go( few, std::integral_constant<int, 4> {} );
+    } else if ( pieces <= 2048 ) {
+      go( few, std::integral_constant<int, 8> {} );
+    } else if ( pieces <= 4096 ) {
+      go( many, std::integral_constant<int, 4> {} );
     } else {
-      argmax_kernel<T, V, 1024><<<(unsigned)batch, 1024, 0, as_stream( stream )>>>( out_dev, rows, (uint32_t)n );
+      go( many, std::integral_constant<int, 8> {} );
     }
   };
   GH_DISPATCH_DT( dt, whole ? launch( static_cast<T*>( nullptr ), std::integral_constant<int, 16 / sizeof( T )> {} )

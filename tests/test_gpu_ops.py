@@ -109,7 +109,7 @@ def test_argmax_bit_exact(dt):
 
 
 @pytest.mark.parametrize("dt", ["f16", "f32"])
-@pytest.mark.parametrize("n", [1, 7, 8, 2048, 2049, 4099, 8192, 8196, 16384, 16392, 70001])
+@pytest.mark.parametrize("n", [1, 7, 8, 256, 257, 513, 1024, 1025, 1028, 2048, 2049, 2052, 2056, 4096, 4099, 4100, 4104, 8192, 8196, 8200, 16384, 16388, 16392, 32768, 32776, 70001])
 def test_argmax_edges(dt, n):
     """Rows that begin with NaN, hold one, hold nothing but the lowest value or minus infinity; the maximum at either end."""
     rng = np.random.default_rng(n)
