@@ -128,8 +128,9 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
       s[u] = wave_sum( partial ) * scale_log2e;
       m_new = t0 + u < t_end ? fmaxf( m_new, s[u] ) : m_new;
     }
-    // A score of -inf weighs 0, also where no finite one came before it (the difference of the two infinities would be NaN).
-    const float alpha = m == -INFINITY ? 0.0f : fast_exp2( m - m_new );
+    // A score of -inf weighs 0, also where no finite one came before it: then against 0, as the difference of the two infinities would be NaN.
+    const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+    const float alpha = fast_exp2( m - m_ref );
     l *= alpha;
 #pragma unroll
     for ( int k = 0; k < NK; k++ ) {
@@ -138,7 +139,7 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
 #pragma unroll
     for ( int u = 0; u < U; u++ ) {
       if ( t0 + u < t_end ) { // uniform
-        const float p = s[u] == -INFINITY ? 0.0f : fast_exp2( s[u] - m_new );
+        const float p = fast_exp2( s[u] - m_ref );
         l += p;
 #pragma unroll
         for ( int k = 0; k < NK; k++ ) {
@@ -174,7 +175,7 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
     }
     for ( int w = 0; w < W; w++ ) {
       if ( t_begin + w * U < t_end ) { // uniform; a wave without keys adds nothing
-        const float f = s_m[w] == -INFINITY ? 0.0f : fast_exp2( s_m[w] - m_all );
+        const float f = fast_exp2( s_m[w] - ( m_all == -INFINITY ? 0.0f : m_all ) );
         l += s_l[w] * f;
 #pragma unroll
         for ( int k = 0; k < NK; k++ ) {
