@@ -131,7 +131,7 @@ def test_norm_over_activations_of_shorter_rows(b, s, r):
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
-@pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
+@pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (1, 288, 768), (1, 260, 2050), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
                                         # enough row tiles for one launch without a K split: both factors in one kernel
                                         (64, 512, 16384), (5, 256, 16404), (33, 1024, 28672),
                                         (5, 256, 16386)])     # rows not a multiple of 4: the two-kernel route
