@@ -18,7 +18,7 @@ def _init():
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
-@pytest.mark.parametrize("b,s,r", [(4, 288, 288), (64, 1024, 512), (5, 768, 1000), (3, 100, 36),
+@pytest.mark.parametrize("b,s,r", [(4, 288, 288), (1, 288, 288), (1, 260, 4100), (64, 1024, 512), (5, 768, 1000), (3, 100, 36),
                                    # more than 64 rows: any of the kernels leaves the partial sums
                                    (100, 512, 260), (256, 1024, 512), (300, 4096, 1000),
                                    # enough 256-token tiles: the residual is added in the large tile kernel's epilogue (f16, r % 8 == 0)
