@@ -89,7 +89,7 @@ public:
 // ---- library-owned device scratch ---------------------------------------------------------------
 // Grow-only buffer for purpose `which`, private to `stream`: work queued on different streams never
 // shares one.  Growing waits for that stream only.  `min_bytes` is the size of the first allocation.
-enum { SCRATCH_GEMM_PARTIALS = 0, SCRATCH_CONVERT = 1, SCRATCH_ATTN_PV = 2, SCRATCH_GATE_FACTOR = 3, SCRATCH_LIBRARY = 4, SCRATCH_PRODUCT = 5, SCRATCH_MIXER = 6 };
+enum { SCRATCH_GEMM_PARTIALS = 0, SCRATCH_CONVERT = 1, SCRATCH_ATTN_PV = 2, SCRATCH_GATE_FACTOR = 3, SCRATCH_LIBRARY = 4, SCRATCH_PRODUCT = 5, SCRATCH_MIXER = 6, SCRATCH_NORM = 7 };
 int stream_scratch( hipStream_t stream, int which, uint64_t bytes, uint64_t min_bytes, void** out );
 // Whether two buffers share memory: an op that stores its output while its other work-groups still read the input must not take such a pair.
 inline bool overlap( const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes )

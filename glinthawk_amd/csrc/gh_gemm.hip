@@ -57,7 +57,7 @@ int gemm_ring_gate_launch( E* hb, const GateRows& gate, const E* x, const E* w13
 void gemm_ring_tuning( int target_wgs );
 int gemm_ring_cut( uint64_t s, uint64_t r, uint64_t b, bool gate, uint32_t* plan );
 // fp32 (gh_gemm_f32.hip)
-int gemm_f32( float* out, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
+int gemm_f32( float* out, const float* x, const float* norm, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 
 namespace {
 
@@ -632,7 +632,7 @@ int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_
       *partial_out = dst;
       *splits_out = 1;
     }
-    return gemm_f32( dst, static_cast<const float*>( x ), static_cast<const float*>( w ), s, r, b, st );
+    return gemm_f32( dst, static_cast<const float*>( x ), nullptr, static_cast<const float*>( w ), s, r, b, st );
   }
   GH_REQUIRE( is_half_type( dt ), "gh_matmul: unsupported dtype %d", (int)dt );
   return with_half_type( dt, [&]( auto* e ) {

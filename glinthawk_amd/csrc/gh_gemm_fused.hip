@@ -14,9 +14,11 @@ int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_
                                bool* done );
 // fp32: the product and what follows it in one kernel (gh_gemm_f32.hip)
 int gemm_f32_accum( float* residual, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
-int gemm_f32_gate( float* hb, const float* x, const float* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
-int gemm_f32_qkv( float* q, float* kv_out, const float* x, const float* wqkv, uint64_t s, uint64_t b, const uint32_t* pos, const float* freq_real, const float* freq_imag,
-                  void* const* token_rows, uint32_t dim, uint32_t kv_dim, uint32_t head_size, hipStream_t st );
+int gemm_f32( float* out, const float* x, const float* norm, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
+int gemm_f32_gate( float* hb, const float* x, const float* norm, const float* w13, uint64_t s, uint64_t hidden, uint64_t b, hipStream_t st );
+int gemm_f32_qkv( float* q, float* kv_out, const float* x, const float* norm, const float* wqkv, uint64_t s, uint64_t b, const uint32_t* pos, const float* freq_real,
+                  const float* freq_imag, void* const* token_rows, uint32_t dim, uint32_t kv_dim, uint32_t head_size, hipStream_t st );
+bool gemm_f32_norm_fits( uint64_t s, uint64_t r, const void* x, const void* norm, const void* w );
 
 namespace {
 
@@ -424,6 +426,15 @@ int check_common( const void* x, const void* w, uint64_t s, uint64_t r, uint64_t
   return GH_OK;
 }
 
+// The norm in front of a product that does not take it into its own launch: normed rows in a buffer of the stream's.
+int normed_rows( const void* x, const void* norm_weight, uint64_t s, uint64_t b, gh_dtype dt, gh_stream stream, void** out )
+{
+  if ( int rc = stream_scratch( as_stream( stream ), SCRATCH_NORM, b * s * dtype_size( dt ), 1ull << 20, out ) ) {
+    return rc;
+  }
+  return gh_rmsnorm( *out, x, norm_weight, s, b, dt, stream );
+}
+
 } // namespace
 } // namespace gh
 
@@ -541,7 +552,7 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
   hipStream_t st = as_stream( stream );
   const bool apart = !overlap( hb, b * hidden_dim * dtype_size( dt ), x, b * s * dtype_size( dt ) ); // else through fp32 sums, as in gh_matmul_accum
   if ( dt == GH_F32 && apart ) {
-    return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), static_cast<const float*>( w13 ), s, hidden_dim, b, st );
+    return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), nullptr, static_cast<const float*>( w13 ), s, hidden_dim, b, st );
   }
   bool done = false;
   if ( int rc = gemm_gate_one_launch( hb, GateRows { hidden_dim }, x, w13, s, hidden_dim, b, dt, st, &done ) ) {
@@ -617,7 +628,7 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   hipStream_t st = as_stream( stream );
   const uint64_t x_bytes = b * s * dtype_size( dt );
   if ( dt == GH_F32 && !overlap( q, b * dim * sizeof( float ), x, x_bytes ) && !overlap( kv_out, b * 2 * kv_dim * sizeof( float ), x, x_bytes ) ) {
-    return gemm_f32_qkv( static_cast<float*>( q ), static_cast<float*>( kv_out ), static_cast<const float*>( x ), static_cast<const float*>( wqkv ), s, b, pos_dev,
+    return gemm_f32_qkv( static_cast<float*>( q ), static_cast<float*>( kv_out ), static_cast<const float*>( x ), nullptr, static_cast<const float*>( wqkv ), s, b, pos_dev,
                          static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size, st );
   }
   float* partial = nullptr;
@@ -637,6 +648,89 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   }
   GH_LAUNCH_CHECK();
   return GH_OK;
+}
+
+// Norm and product in one launch: worth it while what every wave norms again takes less than the launch it saves, i.e. for few and short rows; a product of
+// many weight rows has more waves than the chip holds at once and pays for each.  Two launches / one, us, in a graph: 2304 x 768 at 8 rows 7.0 / 6.5, at 16
+// 8.2 / 8.2, 2 x 2048 with the gate 9.5 / 10.1; 2 x 768 x 288 at 16 rows 7.1 / 6.6, at 32 8.4 / 8.6; 32000 x 288 at 8 rows 13.9 / 13.1, at 16 21.6 / 22.0;
+// 32000 x 512 at 4 14.1 / 12.9, at 8 15.7 / 16.3.
+int gh_rmsnorm_rides( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
+{
+  return dt == GH_F32 && b <= 16 && s * b <= ( r <= 4096 ? 6144 : 2304 ) && gemm_f32_norm_fits( s, r, nullptr, nullptr, nullptr ) ? 1 : 0;
+}
+
+int gh_rmsnorm_matmul( void* xout, const void* x, const void* norm_weight, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( b == 0 || r == 0 ) {
+    return GH_OK;
+  }
+  GH_REQUIRE( xout && x && norm_weight && w, "gh_rmsnorm_matmul: NULL pointer" );
+  GH_REQUIRE( dt == GH_F16 || dt == GH_F32, "gh_rmsnorm_matmul: unsupported dtype %d", (int)dt );
+  GH_REQUIRE( s > 0 && s <= 0x7fffffffull && r <= 0x7fffffffull && b <= 0x7fffffffull, "gh_rmsnorm_matmul: bad shape" );
+  if ( dt == GH_F32 && gemm_f32_norm_fits( s, r, x, norm_weight, w ) && !overlap( xout, b * r * sizeof( float ), x, b * s * sizeof( float ) ) ) {
+    return gemm_f32( static_cast<float*>( xout ), static_cast<const float*>( x ), static_cast<const float*>( norm_weight ), static_cast<const float*>( w ), s, r, b,
+                     as_stream( stream ) );
+  }
+  void* normed = nullptr;
+  if ( int rc = normed_rows( x, norm_weight, s, b, dt, stream, &normed ) ) {
+    return rc;
+  }
+  return gh_matmul( xout, normed, w, s, r, b, dt, stream );
+}
+
+int gh_rmsnorm_matmul_silu_gate( void* hb, const void* x, const void* norm_weight, const void* w13, uint64_t s, uint64_t hidden_dim, uint64_t b, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( b == 0 ) {
+    return GH_OK;
+  }
+  if ( int rc = check_common( x, w13, s, 2 * hidden_dim, b, dt, "gh_rmsnorm_matmul_silu_gate" ) ) {
+    return rc;
+  }
+  GH_REQUIRE( hb && norm_weight, "gh_rmsnorm_matmul_silu_gate: NULL pointer" );
+  if ( dt == GH_F32 && gemm_f32_norm_fits( s, 2 * hidden_dim, x, norm_weight, w13 )
+       && !overlap( hb, b * hidden_dim * sizeof( float ), x, b * s * sizeof( float ) ) ) {
+    return gemm_f32_gate( static_cast<float*>( hb ), static_cast<const float*>( x ), static_cast<const float*>( norm_weight ), static_cast<const float*>( w13 ), s,
+                          hidden_dim, b, as_stream( stream ) );
+  }
+  void* normed = nullptr;
+  if ( int rc = normed_rows( x, norm_weight, s, b, dt, stream, &normed ) ) {
+    return rc;
+  }
+  return gh_matmul_silu_gate( hb, normed, w13, s, hidden_dim, b, dt, stream );
+}
+
+int gh_rmsnorm_matmul_qkv_rope_append( void* q, const void* x, const void* norm_weight, const void* wqkv, uint64_t s, uint64_t b, const uint32_t* pos_dev,
+                                       const void* freq_real, const void* freq_imag, void* const* token_rows_dev, uint32_t n_kv_heads, uint32_t gqa_size,
+                                       uint32_t head_size, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( b == 0 ) {
+    return GH_OK;
+  }
+  GH_REQUIRE( n_kv_heads > 0 && gqa_size > 0 && head_size > 0 && head_size % 2 == 0, "gh_rmsnorm_matmul_qkv_rope_append: bad head shape" );
+  const uint64_t kv_dim = (uint64_t)n_kv_heads * head_size, dim = kv_dim * gqa_size;
+  if ( int rc = check_common( x, wqkv, s, dim + 2 * kv_dim, b, dt, "gh_rmsnorm_matmul_qkv_rope_append" ) ) {
+    return rc;
+  }
+  GH_REQUIRE( q && norm_weight && pos_dev && freq_real && freq_imag && token_rows_dev, "gh_rmsnorm_matmul_qkv_rope_append: NULL pointer" );
+  if ( dt == GH_F32 && gemm_f32_norm_fits( s, dim + 2 * kv_dim, x, norm_weight, wqkv ) && !overlap( q, b * dim * sizeof( float ), x, b * s * sizeof( float ) ) ) {
+    return gemm_f32_qkv( static_cast<float*>( q ), nullptr, static_cast<const float*>( x ), static_cast<const float*>( norm_weight ), static_cast<const float*>( wqkv ), s, b,
+                         pos_dev, static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim,
+                         head_size, as_stream( stream ) );
+  }
+  void* normed = nullptr;
+  if ( int rc = normed_rows( x, norm_weight, s, b, dt, stream, &normed ) ) {
+    return rc;
+  }
+  return gh_matmul_qkv_rope_append( q, nullptr, normed, wqkv, s, b, pos_dev, freq_real, freq_imag, token_rows_dev, n_kv_heads, gqa_size, head_size, dt, stream );
 }
 
 } // extern "C"

@@ -392,6 +392,31 @@ public:
                                          Config::n_kv_heads, Config::gqa_size, Config::head_size, gh_type<DType>(), this->stream_ ) );
   }
 
+  // The same over rows that are normed first; norm_rides( r ): whether the norm goes into the product's launch (r weight rows)
+  static bool norm_rides( const uint64_t r, const uint64_t batch_size ) { return gh_rmsnorm_rides( Config::dim, r, batch_size, gh_type<DType>() ) == 1; }
+  template<uint64_t r>
+  void rmsnorm_matmul( DType* xo, const DType* x, const DType* norm_weight, const DType* w, const uint64_t batch_size ) const
+  {
+    GLINT_GH( gh_rmsnorm_matmul( xo, x, norm_weight, w, Config::dim, r, batch_size, gh_type<DType>(), this->stream_ ) );
+  }
+  void rmsnorm_matmul_silu_gate( DType* hb, const DType* x, const DType* norm_weight, const DType* w13, const uint64_t batch_size ) const
+  {
+    GLINT_GH( gh_rmsnorm_matmul_silu_gate( hb, x, norm_weight, w13, Config::dim, Config::hidden_dim, batch_size, gh_type<DType>(), this->stream_ ) );
+  }
+  void rmsnorm_matmul_qkv_rope_append( DType* q,
+                                       const DType* x,
+                                       const DType* norm_weight,
+                                       const DType* wqkv,
+                                       const uint64_t batch_size,
+                                       const uint32_t* token_positions_dev,
+                                       const DType* freq_cis_real,
+                                       const DType* freq_cis_imag,
+                                       void* const* token_rows_dev ) const
+  {
+    GLINT_GH( gh_rmsnorm_matmul_qkv_rope_append( q, x, norm_weight, wqkv, Config::dim, batch_size, token_positions_dev, freq_cis_real, freq_cis_imag, token_rows_dev,
+                                                 Config::n_kv_heads, Config::gqa_size, Config::head_size, gh_type<DType>(), this->stream_ ) );
+  }
+
 private:
   // TokenContext / LayerContext are a single pointer each, so an array of them is a pointer table
   static_assert( sizeof( typename ContextType::TokenContextType ) == sizeof( void* ) );

@@ -223,7 +223,10 @@ public:
 
     spans_.mark( 0, ops_.stream() ); // the activations and the tables are queued: from here to the copy back it is kernels only
     const bool fused_layers = options_.fused_attention && options_.fused_projections;
-    if ( fused_layers && !run.empty() ) {
+    // the norms of a layer in the launches of the products behind them, or at the end of those in front of them
+    const bool norms_ride = fused_layers && LlamaOperations::norm_rides( Config::dim + 2 * Config::kv_dim, batch_ )
+                            && LlamaOperations::norm_rides( 2 * Config::hidden_dim, batch_ );
+    if ( fused_layers && !run.empty() && !norms_ride ) {
       // the first attention norm stands alone; every later one rides on the epilogue of the previous w2
       ops_.template rmsnorm<Config::dim>( xb_, x_, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, batch_ );
     }
@@ -232,7 +235,7 @@ public:
       GLINT_CHECK( settings_.hosts( l, InferenceStage::Attention ) && settings_.hosts( l, InferenceStage::PostAttention ) );
       if ( fused_layers ) {
         const DType* next_norm = k + 1 < run.size() ? layers_[run[k + 1]].rms_att_weight : nullptr;
-        fused_layer_ops( l, k, next_norm );
+        norms_ride ? normed_layer_ops( l, k ) : fused_layer_ops( l, k, next_norm );
       } else {
         for ( size_t i = 0; i < contexts.size(); i++ ) {
           layer_contexts_[i] = contexts[i]->layer( l );
@@ -640,8 +643,23 @@ private:
     ops_.template matmul_accum<Config::hidden_dim, Config::dim>( x_, hb_, w.w2, batch_, next_att_norm ? xb_ : nullptr, next_att_norm );
   }
 
+  // The same with the norms in the launches of the products that read them: 5 launches, x_ all that passes from layer to layer.
+  void normed_layer_ops( const size_t layer, const size_t table_index )
+  {
+    const auto& w = layers_[layer];
+    ops_.rmsnorm_matmul_qkv_rope_append( q_, x_, w.rms_att_weight, w.wq, batch_, pos_dev(), base_.freq_cis_real, base_.freq_cis_imag, token_rows_dev( table_index ) );
+    fused_attention( table_index );
+    ops_.template matmul_accum<Config::dim, Config::dim>( x_, xb_, w.wo, batch_ );
+    ops_.rmsnorm_matmul_silu_gate( hb_, x_, w.rms_ffn_weight, w.w1, batch_ );
+    ops_.template matmul_accum<Config::hidden_dim, Config::dim>( x_, hb_, w.w2, batch_ );
+  }
+
   void classify_ops()
   {
+    if ( options_.fused_projections && LlamaOperations::norm_rides( Config::vocab_size, batch_ ) ) {
+      ops_.template rmsnorm_matmul<Config::vocab_size>( logits_, x_, base_.rms_final_weight, base_.wcls, batch_ );
+      return;
+    }
     ops_.template rmsnorm<Config::dim>( x_, x_, reinterpret_cast<float32_t*>( temp_ ), base_.rms_final_weight, batch_ );
     ops_.template matmul<Config::dim, Config::vocab_size>( logits_, x_, base_.wcls, batch_ );
   }

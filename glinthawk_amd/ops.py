@@ -143,6 +143,35 @@ def matmul_qkv_rope_append(x: torch.Tensor, wqkv: torch.Tensor, pos: torch.Tenso
     return q, kv
 
 
+def rmsnorm_rides(s: int, r: int, b: int, dtype: torch.dtype) -> bool:
+    return lib().gh_rmsnorm_rides(s, r, b, GH_F32 if dtype == torch.float32 else GH_F16) == 1
+
+
+def rmsnorm_matmul(x: torch.Tensor, norm_weight: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    b, s = x.shape
+    out = torch.empty((b, w.shape[0]), dtype=x.dtype, device=x.device)
+    check(lib().gh_rmsnorm_matmul(_p(out), _p(x), _p(norm_weight), _p(w), s, w.shape[0], b, _dt(x), _stream()), "gh_rmsnorm_matmul")
+    return out
+
+
+def rmsnorm_matmul_silu_gate(x: torch.Tensor, norm_weight: torch.Tensor, w13: torch.Tensor) -> torch.Tensor:
+    b, s = x.shape
+    hidden = w13.shape[0] // 2
+    hb = torch.empty((b, hidden), dtype=x.dtype, device=x.device)
+    check(lib().gh_rmsnorm_matmul_silu_gate(_p(hb), _p(x), _p(norm_weight), _p(w13), s, hidden, b, _dt(x), _stream()), "gh_rmsnorm_matmul_silu_gate")
+    return hb
+
+
+def rmsnorm_matmul_qkv_rope_append(x: torch.Tensor, norm_weight: torch.Tensor, wqkv: torch.Tensor, pos: torch.Tensor, freq_real, freq_imag,
+                                   token_rows: torch.Tensor, shape: Shape) -> torch.Tensor:
+    b, s = x.shape
+    q = torch.empty((b, shape.dim), dtype=x.dtype, device=x.device)
+    check(lib().gh_rmsnorm_matmul_qkv_rope_append(_p(q), _p(x), _p(norm_weight), _p(wqkv), s, b, _p(pos), _p(freq_real), _p(freq_imag), _p(token_rows),
+                                                  shape.n_kv_heads, shape.gqa_size, shape.head_size, _dt(x), _stream()),
+          "gh_rmsnorm_matmul_qkv_rope_append")
+    return q
+
+
 def soft_sample(v: torch.Tensor, temperatures: Sequence[float], seed: int = 0) -> None:
     batch, vocab = v.shape
     temps = (C.c_float * batch)(*[float(t) for t in temperatures])

@@ -203,6 +203,16 @@ int gh_matmul_silu_gate( void* hb, const void* x, const void* w13, uint64_t s, u
 int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void* wqkv, uint64_t s, uint64_t b, const uint32_t* pos_dev, const void* freq_real,
                                const void* freq_imag, void* const* token_rows_dev, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, gh_dtype dt,
                                gh_stream stream );
+/* rmsnorm + one of the products above over its rows (x itself is left as it is): one launch for fp32 rows short enough to be held by a wave (16-byte
+ * aligned operands, no output over x), the two calls one after the other otherwise.  gh_rmsnorm_rides, host-only: 1 where the one launch is what a
+ * caller wants for a product of r weight rows (w1 and w3 together) */
+int gh_rmsnorm_rides( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt );
+int gh_rmsnorm_matmul( void* xout, const void* x, const void* norm_weight, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, gh_stream stream );
+int gh_rmsnorm_matmul_silu_gate( void* hb, const void* x, const void* norm_weight, const void* w13, uint64_t s, uint64_t hidden_dim, uint64_t b, gh_dtype dt,
+                                 gh_stream stream );
+int gh_rmsnorm_matmul_qkv_rope_append( void* q, const void* x, const void* norm_weight, const void* wqkv, uint64_t s, uint64_t b, const uint32_t* pos_dev,
+                                       const void* freq_real, const void* freq_imag, void* const* token_rows_dev, uint32_t n_kv_heads, uint32_t gqa_size,
+                                       uint32_t head_size, gh_dtype dt, gh_stream stream );
 /* Operations::soft_sample   arch/amd64/common/ops.hh:97-107,273-283 : rows with temperature > 0 get
  * v / T - log(-log(u)), u from a counter-based generator keyed by (seed, row, column).
  * `temperatures` is a HOST array (batch floats), as in the reference. */

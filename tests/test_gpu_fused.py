@@ -130,6 +130,63 @@ def test_norm_over_activations_of_shorter_rows(b, s, r):
     assert torch.allclose(both.float(), want_norm.float(), rtol=4e-3, atol=4e-3)
 
 
+# rows that a wave requests in one go (the norm in the product's launch): one piece and a bit, the most that two and four weight rows a wave leave
+# room for, and one element more; s % 4 != 0; f16: two launches
+@pytest.mark.parametrize("dt,s", [(torch.float32, 4), (torch.float32, 256), (torch.float32, 288), (torch.float32, 512), (torch.float32, 516), (torch.float32, 1024),
+                                  (torch.float32, 1028), (torch.float32, 290), (torch.float16, 288)])
+@pytest.mark.parametrize("b", [1, 2, 4, 5, 9, 17, 67])
+def test_products_of_normed_rows(dt, s, b):
+    """Against 64 bits.  fp32: an element of the normed row is off by some 4 roundings of 2^-24, and the sum of s products by at most s of them, of the sum
+    of magnitudes; f16: the rounding of the normed row, 2^-11 of the magnitudes, and of the result."""
+    g = torch.Generator(device="cuda").manual_seed(s * 31 + b)
+    shape = Shape(dim=48, n_layers=1, n_heads=6, n_kv_heads=2, hidden_dim=s, seq_len=8)
+    x = (3 * torch.randn((b, s), generator=g, device="cuda")).to(dt)
+    nw = (1 + 0.1 * torch.randn(s, generator=g, device="cuda")).to(dt)
+    normed = x.double() / torch.sqrt((x.double() ** 2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    unit = (s + 8) * 2.0 ** -24 if dt == torch.float32 else 2.0 ** -10
+
+    def bound(w):
+        return unit * (normed.abs() @ w.double().abs().T) + 2.0 ** (-24 if dt == torch.float32 else -11) * (normed @ w.double().T).abs() + 1e-6
+
+    for r in (1, 37, 4096, 4100):
+        w = (torch.randn((r, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+        got = ops.rmsnorm_matmul(x, nw, w)
+        assert ((got.double() - normed @ w.double().T).abs() <= bound(w)).all()
+    for hidden in (3, 768, 2050):
+        w = (torch.randn((2 * hidden, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+        y = normed @ w.double().T
+        y1, y3, slack = y[:, :hidden], y[:, hidden:], bound(w)
+        got = ops.rmsnorm_matmul_silu_gate(x, nw, w).double()
+        # the gate's slope in y1 is at most 1.1 |y3|; the fast exponential and the rounding of the factors and the result on top
+        want = y1 * torch.sigmoid(y1) * y3
+        rounding = 2e-6 if dt == torch.float32 else 2.0 ** -9
+        assert ((got - want).abs() <= 1.1 * slack[:, :hidden] * y3.abs() + slack[:, hidden:] * y1.abs() + rounding * (1 + want.abs())).all()
+    w = (torch.randn((80, s), generator=g, device="cuda") / s ** 0.5).to(dt)
+    pos = torch.arange(b, dtype=torch.int32, device="cuda") % 8
+    angle = torch.rand((8, 4), generator=g, device="cuda") * 6
+    re, im = torch.cos(angle).to(dt), torch.sin(angle).to(dt)
+    caches = [torch.full((b, 32), 5.0, dtype=dt, device="cuda") for _ in range(2)]
+    rows = [ops.row_table([0 if i == 1 else c[i].data_ptr() for i in range(b)]) for c in caches]
+    got = ops.rmsnorm_matmul_qkv_rope_append(x, nw, w, pos, re, im, rows[0], shape)
+    want, _ = ops.matmul_qkv_rope_append(ops.rmsnorm(x, nw), w, pos, re, im, rows[1], shape)
+    tol = dict(rtol=1e-5, atol=1e-5) if dt == torch.float32 else dict(rtol=4e-3, atol=4e-3)     # another order of the norm's sum; a rotation adds two products
+    assert torch.allclose(got.float(), want.float(), **tol) and torch.allclose(caches[0].float(), caches[1].float(), **tol)
+
+
+def test_norm_over_the_rows_it_reads():
+    """An output that lies over the activations, and weights or rows that start off a 16-byte boundary, go through two launches: the same values."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((4, 288), generator=g, device="cuda")
+    nw, w = 1 + 0.1 * torch.randn(288, generator=g, device="cuda"), torch.randn((288, 288), generator=g, device="cuda") / 17
+    want, lib, p, st = ops.rmsnorm_matmul(x, nw, w), _lib.lib(), ops._p, ops._stream()
+    got = x.clone()
+    _lib.check(lib.gh_rmsnorm_matmul(p(got), p(got), p(nw), p(w), 288, 288, 4, ops._dt(x), st))
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
+    shifted = torch.empty(w.numel() + 1, device="cuda")[1:].view(288, 288).copy_(w)
+    _lib.check(lib.gh_rmsnorm_matmul(p(got), p(x), p(nw), p(shifted), 288, 288, 4, ops._dt(x), st))
+    assert torch.allclose(got, want, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("b,s,hidden", [(4, 288, 768), (1, 288, 768), (1, 260, 2050), (64, 512, 1536), (3, 100, 50), (130, 512, 1536), (512, 8192, 12544),
                                         # enough row tiles for one launch without a K split: both factors in one kernel
