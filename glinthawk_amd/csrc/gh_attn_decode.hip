@@ -50,13 +50,21 @@ struct Partials
 // =================================================================================================
 // generic kernel
 //
-// Work-group = (query head, split, context), its W waves take the split's keys in turns of U and add their parts up in LDS.  Bound by
-// latency, not by bytes: a wave's lanes are the dims of a key, so a key is one short load and one reduction over the wave, and what
-// counts is how many are under way at once.  A turn requests U keys and values before the first use and its U reductions overlap.
-// Whole 15M model, 4 contexts of up to 256 keys (24 work-groups): 90 us a layer with one wave that walked key by key, 7 with 16 waves.
-// NK: 64-lane pieces of a head (head_size <= 64 NK)
+// Work-group = (query head, split, context), its W waves take the split's keys in turns and add their parts up in LDS.  Bound by latency, not by
+// bytes, so what counts is how many memory round trips, reductions and instructions lie one behind the other.  Lane (r = lane / 16, c = lane % 16)
+// holds the pieces c, c + 16, ... of four elements of key 4 u + r of a turn: a turn requests 4 U keys and values at once, a key's score is a
+// reduction over 16 lanes, and the four rows of lanes share one running maximum, so that their outputs add up at the end.
+// Whole 15M model, 4 contexts of up to 256 keys (24 work-groups): 90 us a layer with one wave that walked key by key, 7.0 with 16 waves of one key a
+// wave-wide reduction, 4.4 so; 64 contexts x 12 heads of 64, 256 keys, f16: 19.2 and 11.6.  NP: pieces of a head a lane holds (head_size <= 64 NP)
 // =================================================================================================
-template<typename T, int NK, int W>
+template<typename T>
+struct alignas( 4 * sizeof( T ) ) HeadPiece
+{
+  T e[4];
+};
+
+// U: keys of a lane per turn
+template<typename T, int NP, int U, int W>
 __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T* __restrict__ q,
                                                                        const T* const* __restrict__ layer_rows,
                                                                        const uint32_t* __restrict__ pos,
@@ -69,8 +77,7 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
                                                                        uint32_t max_splits,
                                                                        float scale_log2e )
 {
-  constexpr int U = 8 / NK; // keys per turn
-  __shared__ float s_out[W][NK * 64];
+  __shared__ float s_out[W][NP * 64];
   __shared__ float s_m[W], s_l[W];
   const uint32_t head = blockIdx.x;
   const uint32_t split = blockIdx.y;
@@ -88,72 +95,119 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
   const uint32_t t_end = min( n_tok, t_begin + chunk );
   const uint32_t n_heads = n_kv_heads * gqa;
   const uint32_t h = head / gqa;
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane >> 4, c = lane & 15;
   const uint64_t row_elems = 2ull * n_kv_heads * head_size;
-
-  float qd[NK], acc[NK];
-  uint32_t dim[NK]; // a lane past the head reads its last element against a query of zero and stores nothing
   const T* qh = q + ( (uint64_t)ctx * n_heads + head ) * head_size;
-#pragma unroll
-  for ( int k = 0; k < NK; k++ ) {
-    const uint32_t d = lane + 64 * k;
-    dim[k] = min( d, head_size - 1 );
-    qd[k] = d < head_size ? to_f32( qh[dim[k]] ) : 0.0f;
-    acc[k] = 0.0f;
-  }
-  float m = -INFINITY, l = 0.0f;
   const T* kbase = base + (uint64_t)h * head_size;
   const T* vbase = kbase + (uint64_t)n_kv_heads * head_size;
+  // whole pieces where head and rows are made of them (the rows' addresses are known here only), else element by element
+  const bool whole = head_size % 4 == 0 && ( ( reinterpret_cast<uintptr_t>( q ) | reinterpret_cast<uintptr_t>( base ) ) & ( 4 * sizeof( T ) - 1 ) ) == 0;
 
-  for ( uint32_t t0 = t_begin + wave * U; t0 < t_end; t0 += W * U ) {
-    T kd[U][NK], vd[U][NK];
+  float acc[NP][4];
 #pragma unroll
-    for ( int u = 0; u < U; u++ ) {
-      const uint64_t at = (uint64_t)min( t0 + u, t_end - 1 ) * row_elems; // a key past the end repeats the last one and is not counted
+  for ( int k = 0; k < NP; k++ ) {
 #pragma unroll
-      for ( int k = 0; k < NK; k++ ) {
-        kd[u][k] = kbase[at + dim[k]];
-        vd[u][k] = vbase[at + dim[k]];
-      }
+    for ( int e = 0; e < 4; e++ ) {
+      acc[k][e] = 0.0f;
     }
-    float s[U];
-    float m_new = m;
+  }
+  float m = -INFINITY, l = 0.0f; // m: of the wave; l: of this lane's keys
+
+  auto walk = [&]( auto pieces ) __attribute__( ( always_inline ) ) {
+    // past the head's end: its last elements again, as zeros
+    auto load = [&]( const T* row, HeadPiece<T>( &out )[NP] ) __attribute__( ( always_inline ) ) {
 #pragma unroll
-    for ( int u = 0; u < U; u++ ) {
-      float partial = 0.0f;
+      for ( int k = 0; k < NP; k++ ) {
+        const uint32_t d = 4 * ( c + 16 * k );
+        if constexpr ( pieces.value ) {
+          out[k] = *reinterpret_cast<const HeadPiece<T>*>( row + min( d, head_size - 4 ) );
+        } else {
 #pragma unroll
-      for ( int k = 0; k < NK; k++ ) {
-        partial += ( lane + 64 * k < head_size ? to_f32( kd[u][k] ) : 0.0f ) * qd[k];
-      }
-      s[u] = wave_sum( partial ) * scale_log2e;
-      m_new = t0 + u < t_end ? fmaxf( m_new, s[u] ) : m_new;
-    }
-    // A score of -inf weighs 0, also where no finite one came before it: then against 0, as the difference of the two infinities would be NaN.
-    const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
-    const float alpha = fast_exp2( m - m_ref );
-    l *= alpha;
-#pragma unroll
-    for ( int k = 0; k < NK; k++ ) {
-      acc[k] *= alpha;
-    }
-#pragma unroll
-    for ( int u = 0; u < U; u++ ) {
-      if ( t0 + u < t_end ) { // uniform
-        const float p = fast_exp2( s[u] - m_ref );
-        l += p;
-#pragma unroll
-        for ( int k = 0; k < NK; k++ ) {
-          acc[k] += p * to_f32( vd[u][k] );
+          for ( int e = 0; e < 4; e++ ) {
+            out[k].e[e] = row[min( d + e, head_size - 1 )];
+          }
         }
       }
+    };
+    auto value = [&]( const HeadPiece<T>& p, int k, int e ) __attribute__( ( always_inline ) ) {
+      return 4 * ( c + 16 * k ) + ( pieces.value ? 0 : e ) < head_size ? to_f32( p.e[e] ) : 0.0f;
+    };
+    HeadPiece<T> qp[NP];
+    load( qh, qp );
+    float qd[NP][4];
+#pragma unroll
+    for ( int k = 0; k < NP; k++ ) {
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        qd[k][e] = value( qp[k], k, e );
+      }
     }
-    m = m_new;
+    for ( uint32_t t0 = t_begin + wave * ( 4 * U ); t0 < t_end; t0 += W * 4 * U ) {
+      HeadPiece<T> kp[U][NP], vp[U][NP];
+#pragma unroll
+      for ( int u = 0; u < U; u++ ) {
+        const uint64_t at = (uint64_t)min( t0 + 4 * u + r, t_end - 1 ) * row_elems; // a key past the end repeats the last one and is not counted
+        load( kbase + at, kp[u] );
+        load( vbase + at, vp[u] );
+      }
+      float s[U], most = -INFINITY;
+#pragma unroll
+      for ( int u = 0; u < U; u++ ) {
+        float partial = 0.0f;
+#pragma unroll
+        for ( int k = 0; k < NP; k++ ) {
+#pragma unroll
+          for ( int e = 0; e < 4; e++ ) {
+            partial += value( kp[u][k], k, e ) * qd[k][e];
+          }
+        }
+        s[u] = row16_sum( partial ) * scale_log2e;
+        most = t0 + 4 * u + r < t_end ? fmaxf( most, s[u] ) : most;
+      }
+      const float m_new = fmaxf( m, fmaxf( fmaxf( lane_value( most, 0 ), lane_value( most, 16 ) ), fmaxf( lane_value( most, 32 ), lane_value( most, 48 ) ) ) );
+      // A score of -inf weighs 0, also where no finite one came before it: then against 0, as the difference of the two infinities would be NaN.
+      const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = fast_exp2( m - m_ref );
+      l *= alpha;
+#pragma unroll
+      for ( int k = 0; k < NP; k++ ) {
+#pragma unroll
+        for ( int e = 0; e < 4; e++ ) {
+          acc[k][e] *= alpha;
+        }
+      }
+#pragma unroll
+      for ( int u = 0; u < U; u++ ) {
+        const bool in = t0 + 4 * u + r < t_end;
+        const float p = in ? fast_exp2( s[u] - m_ref ) : 0.0f;
+        l += p;
+#pragma unroll
+        for ( int k = 0; k < NP; k++ ) {
+#pragma unroll
+          for ( int e = 0; e < 4; e++ ) {
+            acc[k][e] += in ? p * to_f32( vp[u][k].e[e] ) : 0.0f;
+          }
+        }
+      }
+      m = m_new;
+    }
+  };
+  whole ? walk( std::true_type {} ) : walk( std::false_type {} );
+
+  // the rows of lanes added up: lane (r, c) ends up with element 4 (c + 16 k) + r
+  float out[NP];
+  uint32_t dim[NP];
+#pragma unroll
+  for ( int k = 0; k < NP; k++ ) {
+    out[k] = sum_rows( sum_halves( acc[k][0], acc[k][2] ), sum_halves( acc[k][1], acc[k][3] ) );
+    dim[k] = 4 * ( c + 16 * k ) + r;
   }
+  l = ( lane_value( l, 0 ) + lane_value( l, 16 ) ) + ( lane_value( l, 32 ) + lane_value( l, 48 ) );
 
   if constexpr ( W > 1 ) {
 #pragma unroll
-    for ( int k = 0; k < NK; k++ ) {
-      s_out[wave][lane + 64 * k] = acc[k];
+    for ( int k = 0; k < NP; k++ ) {
+      s_out[wave][lane + 64 * k] = out[k];
     }
     if ( lane == 0 ) {
       s_m[wave] = m;
@@ -163,24 +217,24 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
     if ( wave != 0 ) {
       return;
     }
-    float m_all = m; // wave 0 always has a key
+    float m_all = m;
 #pragma unroll
     for ( int w = 1; w < W; w++ ) {
       m_all = fmaxf( m_all, s_m[w] );
     }
+    const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
     l = 0.0f;
 #pragma unroll
-    for ( int k = 0; k < NK; k++ ) {
-      acc[k] = 0.0f;
+    for ( int k = 0; k < NP; k++ ) {
+      out[k] = 0.0f;
     }
-    for ( int w = 0; w < W; w++ ) {
-      if ( t_begin + w * U < t_end ) { // uniform; a wave without keys adds nothing
-        const float f = fast_exp2( s_m[w] - ( m_all == -INFINITY ? 0.0f : m_all ) );
-        l += s_l[w] * f;
 #pragma unroll
-        for ( int k = 0; k < NK; k++ ) {
-          acc[k] += s_out[w][lane + 64 * k] * f;
-        }
+    for ( int w = 0; w < W; w++ ) { // a wave without keys: maximum -inf, sums of zero
+      const float f = fast_exp2( s_m[w] - m_ref );
+      l += s_l[w] * f;
+#pragma unroll
+      for ( int k = 0; k < NP; k++ ) {
+        out[k] += s_out[w][lane + 64 * k] * f;
       }
     }
     m = m_all;
@@ -190,20 +244,18 @@ __global__ __launch_bounds__( 64 * W ) void attn_decode_generic_kernel( const T*
     const float inv = 1.0f / l;
     T* o = xb + ( (uint64_t)ctx * n_heads + head ) * head_size;
 #pragma unroll
-    for ( int k = 0; k < NK; k++ ) {
-      const uint32_t d = lane + 64 * k;
-      if ( d < head_size ) {
-        o[d] = from_f32<T>( acc[k] * inv );
+    for ( int k = 0; k < NP; k++ ) {
+      if ( dim[k] < head_size ) {
+        o[dim[k]] = from_f32<T>( out[k] * inv );
       }
     }
   } else {
     const uint64_t slot = ( (uint64_t)ctx * n_heads + head ) * max_splits + split;
     float* o = part.out + slot * head_size;
 #pragma unroll
-    for ( int k = 0; k < NK; k++ ) {
-      const uint32_t d = lane + 64 * k;
-      if ( d < head_size ) {
-        o[d] = acc[k];
+    for ( int k = 0; k < NP; k++ ) {
+      if ( dim[k] < head_size ) {
+        o[dim[k]] = out[k];
       }
     }
     if ( lane == 0 ) {
@@ -1326,27 +1378,32 @@ uint64_t partial_floats( uint64_t batch, const gh_shape* s, uint32_t max_splits 
 }
 
 // Waves per work-group of the generic kernel: as many as find keys, 16 while that leaves no CU with a second work-group to wait for, 4
-// beyond (long contexts of many heads: the waves of four work-groups on a CU cover each other's latency).
-template<typename T, int NK, int W>
+// beyond (long contexts of many heads: the waves of four work-groups on a CU cover each other's latency).  One wave for a turn of keys, and for two where
+// a turn's pieces fill the registers that four waves would compete for (64 contexts x 32 heads of 128, 9 keys, f16: 6.4 us with four, 5.4 with one).
+template<typename T, int NP, int U, int W>
 void launch_generic_waves( hipStream_t st, const void* q, const void* const* layer_rows_dev, const uint32_t* pos_dev, Partials part, void* xb, uint64_t batch,
                            const gh_shape* s, const Plan& plan, float scale )
 {
-  attn_decode_generic_kernel<T, NK, W><<<dim3( s->n_heads, plan.max_splits, (unsigned)batch ), 64 * W, 0, st>>>(
+  attn_decode_generic_kernel<T, NP, U, W><<<dim3( s->n_heads, plan.max_splits, (unsigned)batch ), 64 * W, 0, st>>>(
     static_cast<const T*>( q ), reinterpret_cast<const T* const*>( layer_rows_dev ), pos_dev, part, static_cast<T*>( xb ), s->n_kv_heads, s->gqa_size, s->head_size,
     plan.chunk, plan.max_splits, scale );
 }
-template<typename T, int NK>
+template<typename T, int NP>
 void launch_generic_head( hipStream_t st, const void* q, const void* const* layer_rows_dev, const uint32_t* pos_dev, Partials part, void* xb, uint64_t batch,
                           uint32_t max_pos, const gh_shape* s, const Plan& plan, float scale )
 {
-  const uint32_t turns = ( std::min( plan.chunk, max_pos + 1 ) + 8 / NK - 1 ) / ( 8 / NK );
+  constexpr int U = 4 / NP;
+  const uint32_t keys = std::min( plan.chunk, max_pos + 1 );
+  const uint32_t turns = ( keys + 4 * U - 1 ) / ( 4 * U );
   const uint64_t groups = batch * s->n_heads * plan.max_splits;
-  if ( turns <= 1 ) {
-    launch_generic_waves<T, NK, 1>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+  if ( keys <= 4 ) {
+    launch_generic_waves<T, NP, 1, 1>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+  } else if ( turns <= ( NP > 1 ? 2 : 1 ) ) {
+    launch_generic_waves<T, NP, U, 1>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
   } else if ( turns <= 4 || groups > (uint64_t)cu_count() ) {
-    launch_generic_waves<T, NK, 4>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+    launch_generic_waves<T, NP, U, 4>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
   } else {
-    launch_generic_waves<T, NK, 16>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
+    launch_generic_waves<T, NP, U, 16>( st, q, layer_rows_dev, pos_dev, part, xb, batch, s, plan, scale );
   }
 }
 template<typename T>

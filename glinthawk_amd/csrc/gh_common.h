@@ -178,6 +178,21 @@ __device__ __forceinline__ float half_wave_max( float v )
   return fmaxf( __builtin_bit_cast( float, low ), __builtin_bit_cast( float, high ) );
 }
 
+// Two sums in one go, by lanes that change places in the vector ALU: of a lane's value and that 32 lanes further on, of `a` in the lower half of the
+// wave and of `b` in the upper; and of the values of two neighbouring rows of 16 lanes, of `a` in the even rows and of `b` in the odd.
+__device__ __forceinline__ float sum_halves( float a, float b )
+{
+  const auto r = __builtin_amdgcn_permlane32_swap( __builtin_bit_cast( unsigned, a ), __builtin_bit_cast( unsigned, b ), false, false );
+  const unsigned r0 = r[0], r1 = r[1];
+  return __builtin_bit_cast( float, r0 ) + __builtin_bit_cast( float, r1 );
+}
+__device__ __forceinline__ float sum_rows( float a, float b )
+{
+  const auto r = __builtin_amdgcn_permlane16_swap( __builtin_bit_cast( unsigned, a ), __builtin_bit_cast( unsigned, b ), false, false );
+  const unsigned r0 = r[0], r1 = r[1];
+  return __builtin_bit_cast( float, r0 ) + __builtin_bit_cast( float, r1 );
+}
+
 template<typename T>
 __device__ __forceinline__ float to_f32( T v );
 template<>

@@ -141,20 +141,6 @@ __device__ __forceinline__ uint32_t column_of_lane( uint32_t lane )
 {
   return COLS == 1 ? 0 : COLS == 4 ? lane >> 4 : ( lane >> 4 ) + ( ( lane >> 3 ) & 1 ) * 4;
 }
-// a in the lower half of the wave, b in the upper
-__device__ __forceinline__ float sum_halves( float a, float b )
-{
-  const auto r = __builtin_amdgcn_permlane32_swap( __builtin_bit_cast( unsigned, a ), __builtin_bit_cast( unsigned, b ), false, false );
-  const unsigned r0 = r[0], r1 = r[1];
-  return __builtin_bit_cast( float, r0 ) + __builtin_bit_cast( float, r1 );
-}
-// a in the even rows of 16 lanes, b in the odd
-__device__ __forceinline__ float sum_rows( float a, float b )
-{
-  const auto r = __builtin_amdgcn_permlane16_swap( __builtin_bit_cast( unsigned, a ), __builtin_bit_cast( unsigned, b ), false, false );
-  const unsigned r0 = r[0], r1 = r[1];
-  return __builtin_bit_cast( float, r0 ) + __builtin_bit_cast( float, r1 );
-}
 template<int COLS>
 __device__ __forceinline__ float column_sum( const float ( &v )[COLS], uint32_t lane )
 {

@@ -841,6 +841,28 @@ def test_fused_generic_head_sizes(dt, contexts, heads, kv_heads, head_size):
         np.testing.assert_allclose(got[live], want[live], rtol=1e-4, atol=2e-5)
 
 
+# element by element: heads that are no whole pieces of four, and rows that start between two pieces; keys at the edges of a turn and of the waves that share
+# them out (one, four, sixteen)
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+@pytest.mark.parametrize("keys", [1, 4, 5, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("heads,kv_heads,head_size,shift", [(2, 1, 18, 0), (3, 3, 66, 0), (2, 2, 130, 0), (2, 1, 48, 2), (2, 2, 128, 1), (1, 1, 256, 3)])
+def test_fused_generic_unaligned(dt, keys, heads, kv_heads, head_size, shift):
+    g = torch.Generator(device="cuda").manual_seed(keys * 7 + head_size)
+    flat = torch.randn(2 * keys * 2 * kv_heads * head_size + 8, generator=g, device="cuda").to(dt)
+    cache = flat[shift: shift + 2 * keys * 2 * kv_heads * head_size].view(2, keys, 2, kv_heads, head_size)
+    q = torch.randn((2, heads, head_size), generator=g, device="cuda").to(dt)
+    shape = Shape(dim=heads * head_size, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, hidden_dim=64, seq_len=keys)
+    out = torch.zeros((2, heads * head_size), dtype=dt, device="cuda")
+    ops.attn_decode(q.flatten(1), ops.row_table([cache[i].data_ptr() for i in range(2)]), torch.tensor([keys - 1, keys // 2], dtype=torch.int32, device="cuda"), out,
+                    keys - 1, shape, variant=GH_ATTN_GENERIC)
+    for i, n in enumerate((keys, keys // 2 + 1)):
+        k, v = (cache[i, :n, part].double().repeat_interleave(heads // kv_heads, 1) for part in (0, 1))
+        want = ((q[i].double() * k).sum(-1) * head_size ** -0.5).softmax(0)[:, :, None].mul(v).sum(0)
+        # fp32 sums of at most 256 terms of about 1; the stored value's own rounding
+        bound = 2e-5 + want.abs() * (2.0 ** -11 if dt == torch.float16 else 0.0)
+        assert ((out[i].view(heads, head_size).double() - want).abs() <= bound).all(), i
+
+
 # scores of -inf: the last key, the only one of a wave; the first; a wave's whole first turn; several waves' keys; all but one; a whole split
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("chunk", [0, 32])
