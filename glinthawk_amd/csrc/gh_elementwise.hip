@@ -142,6 +142,20 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
   }
 }
 
+// ---- rows of a table by index: one block per row, bytes as they are -------------------------------
+template<typename P>
+__global__ __launch_bounds__( EW_THREADS ) void embed_rows_kernel( P* __restrict__ x, const uint32_t* __restrict__ tokens, const P* __restrict__ table, uint32_t width,
+                                                                  uint32_t vocab )
+{
+  const uint64_t token = tokens[blockIdx.x];
+  if ( token >= vocab ) {
+    return; // a row without a token stays as it is
+  }
+  for ( uint32_t c = threadIdx.x; c < width; c += blockDim.x ) {
+    x[(uint64_t)blockIdx.x * width + c] = table[token * width + c];
+  }
+}
+
 // ---- argmax: one block per row, first index of the maximum --------------------------------------
 // Bound by latency: a row of 32000 values is one work-group's, so a thread asks for AHEAD pieces of it before it compares the first.  4 fp32
 // rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  256 threads where they ask for all of a row at once, with the fewest
@@ -396,6 +410,27 @@ int gh_rmsnorm( void* out, const void* x, const void* weight, uint64_t size, uin
   GH_REQUIRE( aligned16( out ) && aligned16( x ) && aligned16( weight ), "gh_rmsnorm: buffers must be 16-byte aligned" );
   GH_DISPATCH_DT( dt, rmsnorm_kernel<T><<<(unsigned)batch, EW_THREADS, 0, as_stream( stream )>>>(
                         static_cast<T*>( out ), static_cast<const T*>( x ), static_cast<const T*>( weight ), (uint32_t)size ) );
+  GH_LAUNCH_CHECK();
+  return GH_OK;
+}
+
+int gh_embed_rows( void* x, const uint32_t* tokens_dev, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( batch == 0 || width == 0 ) {
+    return GH_OK;
+  }
+  GH_REQUIRE( x && tokens_dev && table, "gh_embed_rows: NULL pointer" );
+  GH_REQUIRE( width <= 0x7fffffffull && vocab <= 0xffffffffull && batch <= 0x7fffffffull, "gh_embed_rows: shape too large" );
+  const uint64_t bytes = width * dtype_size( dt );
+  auto launch = [&]( auto piece ) {
+    using P = decltype( piece );
+    embed_rows_kernel<P><<<(unsigned)batch, EW_THREADS, 0, as_stream( stream )>>>( static_cast<P*>( x ), tokens_dev, static_cast<const P*>( table ),
+                                                                                   (uint32_t)( bytes / sizeof( P ) ), (uint32_t)vocab );
+  };
+  bytes % 16 == 0 && aligned16( x ) && aligned16( table ) ? launch( uint4 {} ) : launch( uint16_t {} );
   GH_LAUNCH_CHECK();
   return GH_OK;
 }

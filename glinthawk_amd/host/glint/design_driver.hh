@@ -321,6 +321,7 @@ protected:
     WeightCursor<DType> placing( weights_.get(), tensors_ );
     lay_out( placing );
     grow_tables( settings_.concurrency_limit, settings_.concurrency_limit, 0 );
+    argmax_ = hip::pinned_array<uint32_t>( std::max<uint64_t>( settings_.concurrency_limit, LOGIT_ROWS ) ); // rows of a step that are sampled at once
     if ( settings_.randomize_parameters ) {
       uint64_t seed = options_.seed * 1000003ull;
       for ( const auto& t : tensors_ ) {
@@ -361,8 +362,6 @@ protected:
       ops_.synchronize();
       logits_ = logit_ops_.device_allocate( logit_rows * sizes_.vocab * sizeof( float ) );
       picked_x_ = logit_ops_.device_allocate( logit_rows * sizes_.width * sizeof( float ) );
-      argmax_dev_ = logit_ops_.device_allocate( logit_rows * sizeof( uint32_t ) );
-      argmax_.resize( logit_rows );
       logit_rows_ = logit_rows;
     }
   }
@@ -437,10 +436,11 @@ protected:
       logit_ops_.copy( out + run * rows * sizes_.width, x_.get(), rows * sizes_.width * sizeof( float ), CopyType::DeviceToHost );
     }
   }
-  // greedy token of the first n rows of the logits, on the host
+  // greedy token of the first n rows of the logits, on the host: the kernel writes them there itself
   void sample( const uint64_t n )
   {
-    GLINT_GH( gh_argmax( argmax_.data(), reinterpret_cast<uint32_t*>( argmax_dev_.get() ), logits_.get(), sizes_.vocab, n, GH_F32, ops_.stream() ) );
+    GLINT_GH( gh_argmax( nullptr, argmax_.get(), logits_.get(), sizes_.vocab, n, GH_F32, ops_.stream() ) );
+    ops_.synchronize();
   }
 
   Sizes sizes_;
@@ -455,9 +455,9 @@ protected:
   DType* final_norm_ {}; // set by lay_out()
 
   typename Operations::DeviceUniquePtr h_ {}, tables_dev_ {};
-  hip::Operations<float>::DeviceUniquePtr x_ {}, logits_ {}, picked_x_ {}, argmax_dev_ {};
+  hip::Operations<float>::DeviceUniquePtr x_ {}, logits_ {}, picked_x_ {};
   uint64_t rows_ { 0 }, logit_rows_ { 0 };
-  std::vector<uint32_t> argmax_ {};
+  hip::PinnedArray<uint32_t> argmax_ {};
   uint8_t* tables_host_ { nullptr };
   uint64_t tables_bytes_ { 0 }, t_batch_ { 0 }, t_rows_ { 0 }, t_picked_ { 0 };
   uint32_t max_start_ { 0 };

@@ -69,6 +69,21 @@ inline void use_pinned_state_buffers()
   (void)installed;
 }
 
+// page-locked host memory, which kernels write and read as well
+struct PinnedFree
+{
+  void operator()( void* p ) const { (void)gh_host_free( p ); }
+};
+template<typename T>
+using PinnedArray = std::unique_ptr<T[], PinnedFree>;
+template<typename T>
+PinnedArray<T> pinned_array( const uint64_t n )
+{
+  void* p = nullptr;
+  GLINT_GH( gh_host_malloc( &p, n * sizeof( T ) ) );
+  return PinnedArray<T> { static_cast<T*>( p ) };
+}
+
 template<typename DType>
 class Operations
 {
@@ -116,6 +131,20 @@ public:
   void argmax( uint32_t* output, const DType* v, DType* temp, const uint64_t batch_size ) const
   {
     GLINT_GH( gh_argmax( output, reinterpret_cast<uint32_t*>( temp ), v, n, batch_size, gh_type<DType>(), stream_ ) );
+  }
+
+  // The same into page-locked host memory, which the kernel writes itself: there when the stream has been waited for
+  template<uint64_t n>
+  void argmax_pinned( uint32_t* output, const DType* v, const uint64_t batch_size ) const
+  {
+    GLINT_GH( gh_argmax( nullptr, output, v, n, batch_size, gh_type<DType>(), stream_ ) );
+  }
+
+  // x(i) = table(tokens_dev[i]); a row whose token is not below vocab stays as it is
+  template<uint64_t width, uint64_t vocab>
+  void embed_rows( DType* x, const uint32_t* tokens_dev, const DType* table, const uint64_t batch_size ) const
+  {
+    GLINT_GH( gh_embed_rows( x, tokens_dev, table, width, vocab, batch_size, gh_type<DType>(), stream_ ) );
   }
 
   template<uint64_t hidden_dim>

@@ -201,10 +201,11 @@ public:
       token_positions_[i] = states.token_pos( i );
     }
 
-    if ( first == 0 ) {
-      load_embedding( states );
-    } else {
+    const bool embed = first == 0;
+    if ( !embed ) {
       ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
+    } else if ( !options_.fused_attention ) {
+      load_embedding( states );
     }
 
     size_t last = Config::n_layers;
@@ -218,7 +219,10 @@ public:
       }
     }
     if ( options_.fused_attention ) {
-      upload_tables( contexts, run );
+      upload_tables( contexts, run, true, embed ? &states : nullptr );
+      if ( embed ) {
+        ops_.template embed_rows<Config::dim, Config::vocab_size>( x_, tokens_dev(), base_.token_embedding_table, batch_ );
+      }
     }
 
     spans_.mark( 0, ops_.stream() ); // the activations and the tables are queued: from here to the copy back it is kernels only
@@ -547,7 +551,8 @@ public:
                    true );
       }
       classify_ops();
-      ops_.template argmax<Config::vocab_size>( argmax_pos_, logits_, temp_, batch );
+      ops_.template argmax_pinned<Config::vocab_size>( argmax_pos_.get(), logits_, batch );
+      ops_.synchronize();
       for ( size_t i = 0; i < batch; i++ ) {
         next_tokens[i] = argmax_pos_[i];
       }
@@ -564,7 +569,7 @@ public:
   DType* scratch_q() const { return q_; }
   DType* scratch_kv() const { return kv_; }
   DType* scratch_logits() const { return logits_; }
-  const uint32_t* argmax_pos() const { return argmax_pos_; }
+  const uint32_t* argmax_pos() const { return argmax_pos_.get(); }
 
 private:
   // ---- ops of one layer ----------------------------------------------------------------------
@@ -736,7 +741,8 @@ private:
         temps.push_back( states.temperature( i ) );
       }
       ops_.soft_sample( logits_, temps, Config::vocab_size );
-      ops_.template argmax<Config::vocab_size>( argmax_pos_, logits_, temp_, temps.size() );
+      ops_.template argmax_pinned<Config::vocab_size>( argmax_pos_.get(), logits_, temps.size() );
+      ops_.synchronize();
 
       states.deallocate_activations();
       states.deallocate_queries();
@@ -767,10 +773,12 @@ private:
   }
 
   // ---- device-side tables of the fused path --------------------------------------------------
-  // layout of one upload: pos[cap] (u32) | for each layer of the run: layer_rows[cap], token_rows[cap] (pointers)
+  // layout of one upload: pos[cap], tokens[cap] (u32) | for each layer of the run: layer_rows[cap], token_rows[cap] (pointers)
   size_t table_stride() const { return settings_.concurrency_limit; }
   const uint32_t* pos_dev() const { return reinterpret_cast<const uint32_t*>( tables_dev_.get() ); }
-  uint8_t* ptr_tables( uint8_t* base ) const { return base + ( ( table_stride() * sizeof( uint32_t ) + 15 ) / 16 * 16 ); }
+  const uint32_t* tokens_dev() const { return pos_dev() + table_stride(); }
+  static size_t ptr_tables_offset( const size_t cap ) { return ( 2 * cap * sizeof( uint32_t ) + 15 ) / 16 * 16; }
+  uint8_t* ptr_tables( uint8_t* base ) const { return base + ptr_tables_offset( table_stride() ); }
   const void* const* layer_rows_dev( size_t k ) const
   {
     return reinterpret_cast<const void* const*>( ptr_tables( reinterpret_cast<uint8_t*>( tables_dev_.get() ) ) ) + ( 2 * k ) * table_stride();
@@ -780,8 +788,9 @@ private:
     return reinterpret_cast<void* const*>( ptr_tables( reinterpret_cast<uint8_t*>( tables_dev_.get() ) ) ) + ( 2 * k + 1 ) * table_stride();
   }
 
-  // `decode`: the positions are those of one new token per context (a batched prefill attends from many)
-  void upload_tables( const ContextVector& contexts, const std::vector<size_t>& run, const bool decode = true )
+  // `decode`: the positions are those of one new token per context (a batched prefill attends from many).  `tokens`: whose tokens are embedded
+  // (a row that is not active gets none), or nullptr
+  void upload_tables( const ContextVector& contexts, const std::vector<size_t>& run, const bool decode = true, const StateType* tokens = nullptr )
   {
     // The previous upload reads the pinned buffer asynchronously: it has to be over before the buffer is rewritten.  A step
     // ends with a blocking copy of its results, which is such a wait already; only without one since the last upload is
@@ -795,6 +804,10 @@ private:
     uint64_t keys = 0, live = 0;
     for ( size_t i = 0; i < batch_; i++ ) {
       pos[i] = token_positions_[i];
+      if ( tokens != nullptr ) {
+        GLINT_CHECK( !tokens->active( i ) || tokens->token( i ) < Config::vocab_size );
+        pos[table_stride() + i] = tokens->active( i ) ? tokens->token( i ) : UINT32_MAX;
+      }
       if ( !contexts[i]->empty() ) {
         GLINT_CHECK( token_positions_[i] < Config::seq_len );
         max_pos_ = std::max( max_pos_, token_positions_[i] );
@@ -922,6 +935,7 @@ private:
     att_ = carve( cur, att_elems );
     logits_ = carve( cur, cls ? cap * Config::vocab_size : 0 );
     temp_ = carve( cur, temp_elems );
+    argmax_pos_ = hip::pinned_array<uint32_t>( cap );
 
     if ( options_.fused_attention ) {
       const gh_shape s = LlamaOperations::shape();
@@ -933,7 +947,7 @@ private:
         attn_bal_ws_ = ops_.device_allocate( std::max<uint64_t>( attn_bal_ws_bytes_, 16 ) );
       }
       const size_t n_run = std::max<size_t>( 1, settings_.num_attention_layers_hosted() );
-      const size_t bytes = ( cap * sizeof( uint32_t ) + 15 ) / 16 * 16 + n_run * 2 * cap * sizeof( void* );
+      const size_t bytes = ptr_tables_offset( cap ) + n_run * 2 * cap * sizeof( void* );
       tables_dev_ = ops_.device_allocate( bytes );
       void* pinned = nullptr;
       GLINT_GH( gh_host_malloc( &pinned, bytes ) );
@@ -1069,7 +1083,7 @@ private:
   // ... and host arrays (models/llama2/base.hh:196-202)
   uint64_t batch_ { 1 };
   uint32_t max_pos_ { 0 };
-  uint32_t argmax_pos_[MAX_BATCH_SIZE] {};
+  hip::PinnedArray<uint32_t> argmax_pos_ {}; // one per slot of a batch, written by the kernel
   uint32_t token_positions_[MAX_BATCH_SIZE] {};
   typename Context::LayerContextType layer_contexts_[MAX_BATCH_SIZE] {};
   typename Context::TokenContextType token_contexts_[MAX_BATCH_SIZE] {};

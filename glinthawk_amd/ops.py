@@ -85,6 +85,11 @@ def silu(hb: torch.Tensor, hb2: torch.Tensor) -> None:
     check(lib().gh_silu(_p(hb), _p(hb2), hidden, batch, _dt(hb), _stream()), "gh_silu")
 
 
+def embed_rows(x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> None:
+    batch, width = x.shape
+    check(lib().gh_embed_rows(_p(x), _p(tokens), _p(table), width, table.shape[0], batch, _dt(x), _stream()), "gh_embed_rows")
+
+
 def argmax(v: torch.Tensor, to_host: bool = True):
     batch, n = v.shape
     out_dev = torch.empty(batch, dtype=torch.int32, device=v.device)

@@ -147,8 +147,10 @@ int gh_accum( void* a, const void* b, uint64_t size, uint64_t batch, gh_dtype dt
 int gh_rmsnorm( void* out, const void* x, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::silu<hidden>   arch/amd64/common/ops.hh:194-210 : hb = DType(x / (1 + exp(-x)) * hb2) */
 int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_dtype dt, gh_stream stream );
+/* x(i) = table(tokens_dev[i]), (vocab, width) rows; a token that is not below vocab leaves its row as it is */
+int gh_embed_rows( void* x, const uint32_t* tokens_dev, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::argmax<n>      arch/amd64/common/ops.hh:171-192 : first index of the row maximum.
- * `out_dev` (batch uint32, device) receives the indices; if `out_host` is non-NULL they are also
+ * `out_dev` (batch uint32, device memory or page-locked host memory) receives the indices; if `out_host` is non-NULL they are also
  * copied there and the call synchronises (the reference writes a host array: arch/cuda/common/ops.cuh:646-650) */
 int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::matmul<s,r> / untemplated_matmul  arch/amd64/common/ops.hh:74-93,212-271 :

@@ -109,6 +109,21 @@ def test_argmax_bit_exact(dt):
 
 
 @pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("batch,width,shift", [(1, 1, 0), (3, 7, 0), (5, 288, 0), (4, 8, 1), (2, 8192, 0), (70, 4096, 0)])
+def test_embed_rows(dt, batch, width, shift):
+    """Rows of a table by index, bit for bit; an index past the table leaves its row as it is.  Whole pieces of 16 bytes and element by element."""
+    g = torch.Generator(device="cuda").manual_seed(width)
+    table = torch.randn(11 * width + shift, generator=g, device="cuda").to(tdt(dt))[shift:].view(11, width)
+    x = torch.full((batch, width), 5.0, dtype=tdt(dt), device="cuda")
+    tokens = torch.randint(0, 11, (batch,), generator=g, device="cuda", dtype=torch.int32)
+    tokens[batch // 2] = -1
+    ops.embed_rows(x, tokens, table)
+    want = table[tokens.clamp(min=0).long()].clone()
+    want[batch // 2] = 5.0
+    assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("n", [1, 7, 8, 256, 257, 513, 1024, 1025, 1028, 2048, 2049, 2052, 2056, 4096, 4099, 4100, 4104, 8192, 8196, 8200, 16384, 16388, 16392, 32768, 32776, 70001])
 def test_argmax_edges(dt, n):
     """Rows that begin with NaN, hold one, hold nothing but the lowest value or minus infinity; the maximum at either end."""
