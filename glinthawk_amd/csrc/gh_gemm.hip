@@ -34,7 +34,8 @@ bool gemm_tile256_fills( uint64_t r, uint64_t b );
 double gemm_tile256_ns( uint64_t s, uint64_t r, uint64_t b );
 template<typename E>
 int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, int epilogue, hipStream_t st,
-                         uint32_t splits, uint32_t k_len, E* xout2 = nullptr, uint64_t r_first = 0, const GateRows* gate = nullptr );
+                         uint32_t splits, uint32_t k_len, E* xout2 = nullptr, uint64_t r_first = 0, const GateRows* gate = nullptr, const QkvRows* qkv = nullptr );
+bool gemm_tile256_qkv_fits( const QkvRows& q );
 uint64_t gemm_tile256_rounds( uint64_t r, uint64_t b );
 uint64_t gemm_tile256_tokens( uint64_t r, uint64_t b, uint64_t rounds );
 void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_len, double* ns );
@@ -501,6 +502,19 @@ int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_
   } );
 }
 
+// Many rows of q, k and v in one launch that rotates and appends them (f16); *done = false: nothing was launched.
+bool gemm_tile_qkv_applicable( uint64_t s, uint64_t b, gh_dtype dt, const void* x, const void* wqkv, const void* q, const QkvRows& rows )
+{
+  return dt == GH_F16 && gemm_tile256_qkv_fits( rows ) && gemm_tile_epilogue_applicable( s, rows.dim + 2ull * rows.kv_dim, b, dt, x, wqkv, q );
+}
+int gemm_tile_qkv_launch( void* q, const void* x, const void* wqkv, uint64_t s, uint64_t b, gh_dtype dt, const QkvRows& rows, hipStream_t st, bool* done )
+{
+  *done = gemm_tile_qkv_applicable( s, b, dt, x, wqkv, q, rows );
+  return *done ? gemm_tile256_launch<__half>( static_cast<__half*>( q ), nullptr, static_cast<const __half*>( x ), static_cast<const __half*>( wqkv ), s,
+                                              rows.dim + 2ull * rows.kv_dim, b, 4, st, 1, 0, nullptr, 0, nullptr, &rows )
+               : GH_OK;
+}
+
 // The 16-bit part of gemm_partials(): runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums
 // `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue; otherwise the kernel may store
 // DType results straight into `xout` (*splits_out == 0 then).
@@ -699,6 +713,22 @@ int gh_matmul_fuses_many_rows( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
   static const char aligned[16] __attribute__( ( aligned( 16 ) ) ) = { 0 };
   return gemm_tile_epilogue_applicable( s, r, b, dt, aligned, aligned, aligned )
              || ( r % 8 == 0 && gemm_token_split( s, r, b, dt, aligned, aligned, aligned ) != 0 )
+           ? 1
+           : 0;
+}
+
+int gh_matmul_qkv_fuses_many_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt )
+{
+  static const char aligned[16] __attribute__( ( aligned( 16 ) ) ) = { 0 };
+  QkvRows rows;
+  rows.kv_dim = n_kv_heads * head_size;
+  rows.dim = rows.kv_dim * gqa_size;
+  rows.head_size = head_size;
+  if ( gemm_library_wanted( s, rows.dim, b, dt, aligned, aligned, aligned ) || gemm_library_wanted( s, 2ull * rows.kv_dim, b, dt, aligned, aligned, aligned ) ) {
+    return 0;
+  }
+  return gemm_tile_qkv_applicable( s, b, dt, aligned, aligned, aligned, rows )
+             || ( dt == GH_F16 && gemm_tile256_qkv_fits( rows ) && gemm_token_split( s, rows.dim + 2ull * rows.kv_dim, b, dt, aligned, aligned, aligned ) != 0 )
            ? 1
            : 0;
 }

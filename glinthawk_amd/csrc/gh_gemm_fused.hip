@@ -12,6 +12,8 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
 bool gemm_tile_epilogue_applicable( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, const void* x, const void* w, const void* xout );
 int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, int epilogue, hipStream_t st,
                                bool* done );
+int gemm_tile_qkv_launch( void* q, const void* x, const void* wqkv, uint64_t s, uint64_t b, gh_dtype dt, const QkvRows& rows, hipStream_t st, bool* done );
+bool gemm_tile256_qkv_fits( const QkvRows& q );
 // fp32: the product and what follows it in one kernel (gh_gemm_f32.hip)
 int gemm_f32_accum( float* residual, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 int gemm_f32( float* out, const float* x, const float* norm, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
@@ -630,6 +632,24 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   if ( dt == GH_F32 && !overlap( q, b * dim * sizeof( float ), x, x_bytes ) && !overlap( kv_out, b * 2 * kv_dim * sizeof( float ), x, x_bytes ) ) {
     return gemm_f32_qkv( static_cast<float*>( q ), static_cast<float*>( kv_out ), static_cast<const float*>( x ), nullptr, static_cast<const float*>( wqkv ), s, b, pos_dev,
                          static_cast<const float*>( freq_real ), static_cast<const float*>( freq_imag ), token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size, st );
+  }
+  // many rows: rotated and appended in the tile kernel's epilogue, no fp32 sums; whole rounds of tiles and a rest where that is faster
+  const QkvRows rows { pos_dev, freq_real, freq_imag, token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size };
+  if ( dt == GH_F16 && kv_out == nullptr && gemm_tile256_qkv_fits( rows ) && !overlap( q, b * dim * 2, x, x_bytes ) ) {
+    if ( const uint64_t b1 = gemm_token_split( s, r, b, dt, x, wqkv, q ) ) {
+      if ( int rc = gh_matmul_qkv_rope_append( q, nullptr, x, wqkv, s, b1, pos_dev, freq_real, freq_imag, token_rows_dev, n_kv_heads, gqa_size, head_size, dt, stream ) ) {
+        return rc;
+      }
+      return gh_matmul_qkv_rope_append( static_cast<__half*>( q ) + b1 * dim, nullptr, static_cast<const __half*>( x ) + b1 * s, wqkv, s, b - b1, pos_dev + b1, freq_real,
+                                        freq_imag, token_rows_dev + b1, n_kv_heads, gqa_size, head_size, dt, stream );
+    }
+    bool done = false;
+    if ( int rc = gemm_tile_qkv_launch( q, x, wqkv, s, b, dt, rows, st, &done ) ) {
+      return rc;
+    }
+    if ( done ) {
+      return GH_OK;
+    }
   }
   float* partial = nullptr;
   uint32_t splits = 0;

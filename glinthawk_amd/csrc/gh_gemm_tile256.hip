@@ -86,7 +86,9 @@ __device__ __forceinline__ bool tile_of_index( const TileOrder& ord, uint32_t xc
 // w3, whose sums a lane holds side by side; half as many stores, and no kernel that reads both factors
 // again (13B, 16384 tokens: 271 us a layer; the pass of four 36.9 -> 35.5 ms).  With one work-group per CU nothing hides the epilogue, so a
 // gate that takes longer stays a kernel of its own (tanh and biases here, 8192 rows of 2 x 11008: 2 % of the pass slower).
-constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3;
+// Or q, k and v as QkvRows says, 16-byte pieces of a token's heads to its query and its cache row: the two kernels that read the product again, append and
+// rotate took 260 us a layer at 13B and 16384 tokens (3 x 5120 rows of 5120), this epilogue 55 of the product's 1785 (1730 with plain stores).
+constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3, EPI_QKV = 4;
 
 struct TileOut
 {
@@ -95,6 +97,7 @@ struct TileOut
   float* partial;  // EPI_PARTIAL
   uint32_t r, b, r_first; // EPI_GATE: r rows of each factor
   GateRows gate;
+  QkvRows qkv;
 };
 
 // LDS slot (16 bytes) of a chunk: rows of 8 chunks.  A wave's 16-byte reads are served in four passes of 16 lanes (0-3, 12-15, 20-23, 24-27 first);
@@ -102,11 +105,16 @@ struct TileOut
 __device__ __forceinline__ uint32_t x_swizzle( uint32_t row ) { return ( row >> 1 ) & 7; }                           // 16 neighbouring rows
 __device__ __forceinline__ uint32_t w_swizzle( uint32_t row ) { return ( ( row >> 1 ) & 1 ) | ( ( row >> 2 ) & 6 ); } // rows 8 (m / 4) + m % 4 (+ 4), m < 16
 
+__device__ __forceinline__ void drain_loads_and_stores() { __builtin_amdgcn_s_waitcnt( 0x0F70 ); } // vmcnt(0)
+
 // acc[a][h][i][j][v]: row 128 a + 64 group + 32 (i / 2) + 8 (lane / 16) + 4 (i % 2) + v, token 128 h + 32 wave + 16 j + lane % 16.
-// Returns whether the tile left by exactly 16 (EPI_GATE: 8) stores of this wave behind its last load (not EPI_PARTIAL).
+// Returns whether the tile left by exactly 16 (EPI_GATE: 8) stores of this wave behind its last load (not EPI_PARTIAL); else nothing is outstanding, so that
+// also the compiler, which waits before it reads what loads leave in LDS, may count those stores: with one path of fewer stores it has the next
+// tile's second reads wait for nearly all of them (4096 x 1024 at 8192 tokens 61 -> 59 us, 2 x 11008 x 4096 with the gate 1 %).
+// tokens: LDS, EPI_QKV: the cache rows of the tile's 256 tokens, then their positions; those past the last hold the last one's
 template<typename E, int EPI>
 __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2], const TileOut& o, uint32_t tile_row0, uint32_t tile_col0, uint32_t group, uint32_t wave,
-                                            uint32_t lane, uint32_t split )
+                                            uint32_t lane, uint32_t split, const uint32_t* tokens )
 {
   const uint32_t row0 = tile_row0 + 64 * group + 8 * ( lane >> 4 ), col0 = tile_col0 + 32 * wave + ( lane & 15 );
   union Chunk
@@ -160,43 +168,111 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
       }
       return y;
     };
-    const bool whole = tile_row0 + TM2 / 2 <= o.r && tile_col0 + TN2 <= o.b && o.gate.context_rows == nullptr;
     E* base = static_cast<E*>( o.xout ) + (uint64_t)col0 * o.gate.stride + row0;
+    auto store = [&]( auto all ) __attribute__( ( always_inline ) ) {
 #pragma unroll
-    for ( int n = 0; n < 8; n++ ) {
-      const int h = n >> 2, j = ( n >> 1 ) & 1, i = n & 1;
-      const uint32_t col = col0 + 128 * h + 16 * j;
-      const Chunk y = values( h, i, j );
-      if ( whole
-           || ( row0 + 32 * i < o.r && col < o.b && ( o.gate.context_rows == nullptr || o.gate.context_rows[col / o.gate.n_tokens] != nullptr ) ) ) {
-        *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * o.gate.stride + 32 * i ) = y.raw; // r % 8 == 0: eight rows
+      for ( int n = 0; n < 8; n++ ) {
+        const int h = n >> 2, j = ( n >> 1 ) & 1, i = n & 1;
+        const uint32_t col = col0 + 128 * h + 16 * j;
+        const Chunk y = values( h, i, j );
+        if ( all.value
+             || ( row0 + 32 * i < o.r && col < o.b && ( o.gate.context_rows == nullptr || o.gate.context_rows[col / o.gate.n_tokens] != nullptr ) ) ) {
+          *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * o.gate.stride + 32 * i ) = y.raw; // r % 8 == 0: eight rows
+        }
       }
+    };
+    if ( ( tile_row0 + TM2 / 2 <= o.r ) & ( tile_col0 + TN2 <= o.b ) & ( o.gate.context_rows == nullptr ) ) {
+      store( std::true_type {} );
+      return true;
     }
-    return whole;
+    store( std::false_type {} );
+    drain_loads_and_stores();
+    return false;
+  }
+  if constexpr ( EPI == EPI_QKV ) { // a tile's rows are all of q, of k or of v, and 128 rows of whole heads: the angles of rows 128 further on are the same
+    const bool to_q = tile_row0 < o.qkv.dim, turn = tile_row0 < o.qkv.dim + o.qkv.kv_dim;
+    const E *re = static_cast<const E*>( o.qkv.freq_real ), *im = static_cast<const E*>( o.qkv.freq_imag );
+    auto cache_of = [&]( int h, int j ) __attribute__( ( always_inline ) ) {
+      return reinterpret_cast<E*>( reinterpret_cast<const uint64_t*>( tokens )[128 * h + 32 * wave + 16 * j + ( lane & 15 )] );
+    };
+    auto takes_pieces = []( const void* cache ) __attribute__( ( always_inline ) ) { return ( cache != nullptr ) & ( ( reinterpret_cast<uintptr_t>( cache ) & 15u ) == 0 ); };
+    // every store of the tile unconditional: all tokens are there, and all their rows take 16 bytes at a time
+    const bool aligned = takes_pieces( cache_of( 0, 0 ) ) & takes_pieces( cache_of( 0, 1 ) ) & takes_pieces( cache_of( 1, 0 ) ) & takes_pieces( cache_of( 1, 1 ) );
+    const bool whole = ( tile_col0 + TN2 <= o.b ) & ( to_q | (bool)__all( aligned ) );
+    union Angles
+    {
+      uint2 raw;
+      E h[4];
+    };
+    auto store = [&]( auto turned, auto all ) __attribute__( ( always_inline ) ) {
+      Angles cs[2][2][2], sn[2][2][2]; // [token half][token][32 rows]
+      if constexpr ( turned.value ) {
+#pragma unroll
+        for ( int n = 0; n < 8; n++ ) {
+          const int h = n >> 2, j = ( n >> 1 ) & 1, i = n & 1;
+          const uint32_t at = cache_of( h, j ) != nullptr ? tokens[2 * TN2 + 128 * h + 32 * wave + 16 * j + ( lane & 15 )] : 0;
+          const uint64_t k = (uint64_t)at * ( o.qkv.head_size / 2 ) + ( ( row0 + 32 * i ) % o.qkv.head_size ) / 2;
+          cs[h][j][i].raw = *reinterpret_cast<const uint2*>( re + k );
+          sn[h][j][i].raw = *reinterpret_cast<const uint2*>( im + k );
+        }
+      }
+#pragma unroll
+      for ( int n = 0; n < 16; n++ ) {
+        const int h = n >> 3, j = ( n >> 2 ) & 1, a = ( n >> 1 ) & 1, i = n & 1;
+        const uint32_t row = row0 + 128 * a + 32 * i, col = col0 + 128 * h + 16 * j;
+        E* const own = cache_of( h, j );
+        Chunk y = rounded( a, h, i, j );
+        if ( turned.value && own != nullptr ) {
+#pragma unroll
+          for ( int e = 0; e < 4; e++ ) {
+            const float c = to_f32<E>( cs[h][j][i].h[e] ), s = to_f32<E>( sn[h][j][i].h[e] ), y0 = to_f32<E>( y.h[2 * e] ), y1 = to_f32<E>( y.h[2 * e + 1] );
+            y.h[2 * e] = from_f32<E>( y0 * c - y1 * s );
+            y.h[2 * e + 1] = from_f32<E>( y0 * s + y1 * c );
+          }
+        }
+        E* dst = to_q ? static_cast<E*>( o.xout ) + (uint64_t)col * o.qkv.dim + row : own + ( row - o.qkv.dim );
+        if ( all.value || ( col < o.b && ( to_q || takes_pieces( own ) ) ) ) {
+          *reinterpret_cast<uint4*>( dst ) = y.raw;
+        } else if ( col < o.b && own != nullptr ) {
+#pragma unroll
+          for ( int e = 0; e < 8; e++ ) {
+            dst[e] = y.h[e];
+          }
+        }
+      }
+    };
+    if ( whole & turn ) {
+      store( std::true_type {}, std::true_type {} );
+      return true;
+    }
+    if ( whole ) {
+      store( std::false_type {}, std::true_type {} );
+      return true;
+    }
+    turn ? store( std::true_type {}, std::false_type {} ) : store( std::false_type {}, std::false_type {} );
+    drain_loads_and_stores();
+    return false;
   }
   // two products that share their activations in one launch: a tile of one of them, or of both
   const bool second = tile_row0 >= o.r_first;
-  if ( tile_row0 + TM2 <= o.r && tile_col0 + TN2 <= o.b && ( o.r & 7 ) == 0 && ( second || tile_row0 + TM2 <= o.r_first ) ) {
+  if ( ( tile_row0 + TM2 <= o.r ) & ( tile_col0 + TN2 <= o.b ) & ( ( o.r & 7 ) == 0 ) & ( second | ( tile_row0 + TM2 <= o.r_first ) ) ) {
     const uint64_t ld = second ? o.r - o.r_first : o.r_first;
     E* base = static_cast<E*>( second ? o.xout2 : o.xout ) + (uint64_t)col0 * ld + ( row0 - ( second ? o.r_first : 0 ) );
+    Chunk old[EPI == EPI_ACCUM ? 16 : 1]; // all of them before the first store, which a load behind it would wait for
+    if constexpr ( EPI == EPI_ACCUM ) {
 #pragma unroll
-    for ( int h = 0; h < 2; h++ ) {
-      Chunk old[8];
-      if ( EPI == EPI_ACCUM ) {
-#pragma unroll
-        for ( int n = 0; n < 8; n++ ) {
-          old[n].raw = *reinterpret_cast<const uint4*>( base + ( 128 * h + 16 * ( n >> 2 ) ) * ld + 128 * ( ( n >> 1 ) & 1 ) + 32 * ( n & 1 ) );
-        }
+      for ( int n = 0; n < 16; n++ ) {
+        old[n].raw = *reinterpret_cast<const uint4*>( base + ( 128 * ( n >> 3 ) + 16 * ( ( n >> 2 ) & 1 ) ) * ld + 128 * ( ( n >> 1 ) & 1 ) + 32 * ( n & 1 ) );
       }
+    }
 #pragma unroll
-      for ( int n = 0; n < 8; n++ ) {
-        const int j = n >> 2, a = ( n >> 1 ) & 1, i = n & 1;
-        Chunk y = rounded( a, h, i, j );
-        if ( EPI == EPI_ACCUM ) {
-          y = added( y, old[n] );
-        }
-        *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * ld + 128 * a + 32 * i ) = y.raw;
+    for ( int n = 0; n < 16; n++ ) {
+      const int h = n >> 3, j = ( n >> 2 ) & 1, a = ( n >> 1 ) & 1, i = n & 1;
+      Chunk y = rounded( a, h, i, j );
+      if constexpr ( EPI == EPI_ACCUM ) {
+        y = added( y, old[n] );
       }
+      *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * ld + 128 * a + 32 * i ) = y.raw;
     }
     return true;
   }
@@ -227,6 +303,7 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
       }
     }
   }
+  drain_loads_and_stores();
   return false;
 }
 
@@ -239,6 +316,9 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   // Separate arrays: the compiler keeps an LDS read behind the loads into its own array only.  W: the weight rows' halves, X: all tokens.
   __shared__ uint4 s_wa0[128 * 8], s_wb0[128 * 8], s_x0[256 * 8];
   __shared__ uint4 s_wa1[128 * 8], s_wb1[128 * 8], s_x1[256 * 8];
+  // EPI_QKV: cache rows and positions of a tile's tokens, left here at the end of the tile before: read where they are needed they would be one more round
+  // trip a tile with nothing beside it.  Two of them, as a wave may be through with a tile while others still store it.
+  __shared__ uint32_t s_tokens[2][EPI == EPI_QKV ? 3 * TN2 : 1];
   typedef typename Mfma<E>::x8 x8;
   const uint32_t xcd = blockIdx.x & 7; // work-groups go to the XCDs in turn
   uint32_t idx = blockIdx.x >> 3;
@@ -376,6 +456,28 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
     multiply( lower, 0 );
     barrier();
   };
+  // (no branch around loads and stores: what the compiler cannot count it waits for)
+  struct Token
+  {
+    uint64_t row;
+    uint32_t pos;
+  };
+  auto token_of = [&]( uint32_t tt ) __attribute__( ( always_inline ) ) {
+    Token token { 0, 0 };
+    if constexpr ( EPI == EPI_QKV ) {
+      const uint32_t col = min( tt * TN2 + ( threadIdx.x & ( TN2 - 1 ) ), out.b - 1 );
+      token.row = reinterpret_cast<const uint64_t*>( out.qkv.token_rows )[col];
+      token.pos = out.qkv.pos[col];
+    }
+    return token;
+  };
+  auto keep_token = [&]( uint32_t* tokens, const Token& token ) __attribute__( ( always_inline ) ) {
+    if constexpr ( EPI == EPI_QKV ) { // (by two threads each)
+      reinterpret_cast<uint64_t*>( tokens )[threadIdx.x & ( TN2 - 1 )] = token.row;
+      tokens[2 * TN2 + ( threadIdx.x & ( TN2 - 1 ) )] = token.pos;
+    }
+  };
+  keep_token( s_tokens[0], token_of( token_tile ) );
   fetch_w( s_wa0, 0, 0 );
   fetch_x( s_x0, 0, 0 );
   fetch_x( s_x0, 1, 0 );
@@ -383,7 +485,9 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   fetch_w( s_wa1, 0, 1 );
   fetch_x( s_x1, 0, 1 );
   fetch_x( s_x1, 1, 1 );
-  __builtin_amdgcn_s_waitcnt( 0x0F78 ); // vmcnt(8): step 0 up to its second half of weight rows
+  // vmcnt(8): step 0 up to its second half of weight rows.  WALK: vmcnt(0), as what is outstanding here is what the compiler, which waits before it reads
+  // what loads leave in LDS, allows for in every tile: the first reads of the second and later ones would wait for the stores in between.
+  __builtin_amdgcn_s_waitcnt( WALK ? 0x0F70 : 0x0F78 );
   barrier();
   if ( group == 1 ) {
     barrier();
@@ -397,7 +501,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   uint32_t j = 0;
   if constexpr ( WALK ) {
     bool stores = false;
-    while ( true ) {
+    for ( uint32_t tile = 0;; tile++ ) {
       uint32_t next_row = 0, next_token = 0;
       idx += gridDim.x >> 3;
       more = tile_of_index( ord, xcd, idx, next_row, next_token );
@@ -405,14 +509,18 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
         next = operands_of( next_row, next_token );
       }
       clear();
-      for ( j = 0; j < n_steps; j += 2 ) {
+      j = 0;
+      do { // (an even number of steps)
         step( s_wa0, s_wb0, s_x0, s_wb1, j, stores && j == 0 );
         step( s_wa1, s_wb1, s_x1, s_wb0, j + 1, false );
-      }
+        j += 2;
+      } while ( j < n_steps );
       if ( !more ) {
         __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): no load-to-LDS outlives the work-group
       }
-      stores = store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, 0 );
+      const Token token = token_of( more ? next_token : token_tile );
+      stores = store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, 0, s_tokens[tile & 1] );
+      keep_token( s_tokens[( tile + 1 ) & 1], token );
       if ( !more ) {
         break;
       }
@@ -430,7 +538,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
       step( s_wa0, s_wb0, s_x0, s_wb1, j, false );
     }
     __builtin_amdgcn_s_waitcnt( 0x0F70 );
-    store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, blockIdx.y );
+    store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, blockIdx.y, s_tokens[0] );
   }
   if ( group == 0 ) {
     barrier();
@@ -528,12 +636,19 @@ void gemm_tile256_split_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* spli
   }
 }
 
+// Tiles that lie in one of q, k and v, whole heads in 128 rows, angles that are read four at a time.
+bool gemm_tile256_qkv_fits( const QkvRows& q )
+{
+  return q.dim % TM2 == 0 && q.kv_dim % TM2 == 0 && q.head_size >= 8 && 128 % q.head_size == 0
+         && ( ( reinterpret_cast<uintptr_t>( q.freq_real ) | reinterpret_cast<uintptr_t>( q.freq_imag ) ) & 7u ) == 0;
+}
+
 // `partial` != nullptr: fp32 sums (splits, b, r) instead of xout; else `epilogue` 0 stores, 1 accumulates into xout (needs r % 8 == 0), 2 gates
-// (2 r weight rows, `gate`).
+// (2 r weight rows, `gate`), 4 rotates and appends (`qkv`; xout: q).
 // splits > 1 (from gemm_tile256_split_plan, with its k_len) needs `partial`.
 template<typename E>
 int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, int epilogue, hipStream_t st, uint32_t splits,
-                         uint32_t k_len, E* xout2, uint64_t r_first, const GateRows* gate )
+                         uint32_t k_len, E* xout2, uint64_t r_first, const GateRows* gate, const QkvRows* qkv )
 {
   if ( xout2 == nullptr ) {
     r_first = r;
@@ -546,7 +661,7 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
     k_len = (uint32_t)s;
   }
   const int epi = partial != nullptr ? EPI_PARTIAL : epilogue;
-  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL || ( epi == EPI_GATE && gate != nullptr && gate->activation == GH_ACT_SILU && gate->bias == nullptr && r % 8 == 0 && gate->stride % 8 == 0 ),
+  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL || ( epi == EPI_QKV && qkv != nullptr && gemm_tile256_qkv_fits( *qkv ) ) || ( epi == EPI_GATE && gate != nullptr && gate->activation == GH_ACT_SILU && gate->bias == nullptr && r % 8 == 0 && gate->stride % 8 == 0 ),
               "gh_matmul: unknown tile epilogue %d", epi );
   GH_REQUIRE( epi != EPI_ACCUM || r % 8 == 0, "gh_matmul: the accumulating tile epilogue needs r %% 8 == 0" );
   const uint64_t tile_rows = epi == EPI_GATE ? TM2 / 2 : TM2;
@@ -569,7 +684,7 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   ord.rest_share = (uint32_t)( ( (uint64_t)ord.rest_rows * tokens + 7 ) / 8 );
   const uint64_t per_xcd = ord.rest_rows == 0 ? whole : even; // the longest list
   GH_REQUIRE( 8 * per_xcd < ( 1ull << 31 ), "gh_matmul: grid too large" );
-  const TileOut out { xout, xout2, partial, (uint32_t)r, (uint32_t)b, (uint32_t)r_first, gate != nullptr ? *gate : GateRows {} };
+  const TileOut out { xout, xout2, partial, (uint32_t)r, (uint32_t)b, (uint32_t)r_first, gate != nullptr ? *gate : GateRows {}, qkv != nullptr ? *qkv : QkvRows {} };
   const bool walk = per_xcd > per_cu && epi != EPI_PARTIAL && s % ( 2 * TKS ) == 0;
   const dim3 grid( (unsigned)( 8 * ( walk ? per_cu : per_xcd ) ), splits );
 #define GH_TILE256( EP, WALK ) gemm_tile256_kernel<E, EP, WALK><<<grid, T256_THREADS, 0, st>>>( x, w, (uint32_t)s, k_len, out, ord )
@@ -577,6 +692,11 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
     case EPI_STORE: walk ? GH_TILE256( EPI_STORE, true ) : GH_TILE256( EPI_STORE, false ); break;
     case EPI_ACCUM: walk ? GH_TILE256( EPI_ACCUM, true ) : GH_TILE256( EPI_ACCUM, false ); break;
     case EPI_GATE: walk ? GH_TILE256( EPI_GATE, true ) : GH_TILE256( EPI_GATE, false ); break;
+    case EPI_QKV:
+      if constexpr ( std::is_same_v<E, __half> ) {
+        walk ? GH_TILE256( EPI_QKV, true ) : GH_TILE256( EPI_QKV, false );
+      }
+      break;
     default: GH_TILE256( EPI_PARTIAL, false ); break;
   }
 #undef GH_TILE256
@@ -585,8 +705,8 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
 }
 
 template int gemm_tile256_launch<__half>( __half*, float*, const __half*, const __half*, uint64_t, uint64_t, uint64_t, int, hipStream_t, uint32_t, uint32_t,
-                                          __half*, uint64_t, const GateRows* );
+                                          __half*, uint64_t, const GateRows*, const QkvRows* );
 template int gemm_tile256_launch<__bf16>( __bf16*, float*, const __bf16*, const __bf16*, uint64_t, uint64_t, uint64_t, int, hipStream_t, uint32_t, uint32_t,
-                                          __bf16*, uint64_t, const GateRows* );
+                                          __bf16*, uint64_t, const GateRows*, const QkvRows* );
 
 } // namespace gh

@@ -23,6 +23,15 @@ struct GateRows
   int activation { GH_ACT_SILU };
   const void* bias { nullptr }; // of DType, for w1's rows then w3's; with it the factors stay fp32 sums
 };
+// Rows of q, k and v that their product rotates and appends itself, f16: q(b, dim) = rope(DType(q)), cache row = [rope(DType(k)) | DType(v)]; a context without
+// a row keeps its query unrotated.
+struct QkvRows
+{
+  const uint32_t* pos { nullptr };
+  const void *freq_real { nullptr }, *freq_imag { nullptr }; // (positions, head_size / 2)
+  void* const* token_rows { nullptr };
+  uint32_t dim { 0 }, kv_dim { 0 }, head_size { 0 };
+};
 // w1, w3 and the gate in one launch; *done = false: nothing was launched, the caller takes its other route
 int gemm_gate_one_launch( void* hb, const GateRows& gate, const void* x, const void* w13, uint64_t s, uint64_t hidden, uint64_t b, gh_dtype dt, hipStream_t st, bool* done );
 

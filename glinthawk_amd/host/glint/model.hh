@@ -476,7 +476,15 @@ public:
             GLINT_GH( gh_stream_wait_event( ops_.stream(), copy_lane_->in[c] ) );
             ops_.template rmsnorm<Config::dim>( pxb + r0 * Config::dim, px + r0 * Config::dim, reinterpret_cast<float32_t*>( temp_ ), w.rms_att_weight, rows );
           }
-          if ( w.wkv == w.wq + (uint64_t)Config::dim * Config::dim ) { // wkv lies behind wq: one launch for the two products
+          const bool together = w.wkv == w.wq + (uint64_t)Config::dim * Config::dim; // wkv lies behind wq: one launch for the two products
+          if ( together && rows <= 65535
+               && gh_matmul_qkv_fuses_many_rows( Config::dim, Config::n_kv_heads, Config::gqa_size, Config::head_size, rows, hip::gh_type<DType>() ) == 1 ) {
+            // ... that rotates and appends as well
+            ops_.matmul_qkv_rope_append( pq + r0 * Config::dim, pxb + r0 * Config::dim, w.wq, rows, pf_pos() + r0, base_.freq_cis_real, base_.freq_cis_imag,
+                                         pf_token_rows() + r0 );
+            continue;
+          }
+          if ( together ) {
             ops_.template matmul_pair<Config::dim, Config::dim, Config::kv_dim * 2>( pq + r0 * Config::dim, pkv + r0 * Config::kv_dim * 2, pxb + r0 * Config::dim,
                                                                                       w.wq, rows );
           } else {

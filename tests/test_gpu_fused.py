@@ -318,6 +318,34 @@ def test_matmul_qkv_rope_append(dt, shape):
     assert torch.equal(arena_b.dev[mask], before[mask])
 
 
+# tokens that end on a tile, behind one, with a rest that is a product of its own; steps that are walked (even) and not; heads of 128, 64 and 32
+@pytest.mark.parametrize("s,kv_heads,gqa,head_size,b", [(1024, 4, 2, 128, 7168), (2048, 4, 4, 128, 3328), (2048, 4, 4, 128, 4100), (1024, 8, 4, 64, 5000), (576, 2, 8, 128, 7000),
+                                                        (640, 16, 2, 32, 9000), (8192, 8, 8, 128, 3328)])
+def test_many_rows_of_qkv_rotated_and_appended(s, kv_heads, gqa, head_size, b):
+    """Against product, append and rotation one by one.  The product may sum in another order (a rounding of f16), and a rotation adds two products.  Empty
+    contexts keep their query unrotated; the rows around an appended one stay as they are; cache rows off a 16-byte boundary."""
+    dim, kv_dim = kv_heads * gqa * head_size, kv_heads * head_size
+    assert _lib.lib().gh_matmul_qkv_fuses_many_rows(s, kv_heads, gqa, head_size, b, 0) == 1
+    shape = Shape(dim=dim, n_layers=1, n_heads=kv_heads * gqa, n_kv_heads=kv_heads, hidden_dim=64, seq_len=64)
+    g = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, s), generator=g, device="cuda").half()
+    w = (torch.randn((dim + 2 * kv_dim, s), generator=g, device="cuda") / s ** 0.5).half()
+    pos = torch.randint(0, 64, (b,), generator=g, device="cuda", dtype=torch.int32)
+    angle = torch.rand((64, head_size // 2), generator=g, device="cuda") * 6
+    re, im = torch.cos(angle).half(), torch.sin(angle).half()
+    for shift in (0, 4):
+        flat = [torch.full((2 * b * 2 * kv_dim + 8,), 5.0, dtype=torch.float16, device="cuda") for _ in range(2)]
+        caches = [f[shift: shift + 2 * b * 2 * kv_dim].view(b, 2, 2 * kv_dim) for f in flat]         # a row is appended, the next stays
+        rows = [ops.row_table([0 if i % 97 == 5 else c[i].data_ptr() for i in range(b)]) for c in caches]
+        q = ops.matmul(x, w[:dim].contiguous())
+        ops.kv_append(rows[0], ops.matmul(x, w[dim:].contiguous()), kv_dim)
+        ops.rope(pos, re, im, q, rows[0], shape)
+        got, _ = ops.matmul_qkv_rope_append(x, w, pos, re, im, rows[1], shape)
+        assert torch.allclose(got.float(), q.float(), rtol=4e-3, atol=4e-3)
+        assert torch.allclose(flat[1].float(), flat[0].float(), rtol=4e-3, atol=4e-3)
+        assert (caches[1][:, 1] == 5.0).all() and (caches[1][5] == 5.0).all()
+
+
 @pytest.mark.parametrize("name,dtype", [("test-gqa4", "f16"), ("stories15m", "f32"), ("test-tiny", "f32")])
 def test_stage_with_and_without_fused_projections(name, dtype):
     cfg = SHAPES[name]
