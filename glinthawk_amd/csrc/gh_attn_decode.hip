@@ -330,6 +330,91 @@ __global__ __launch_bounds__( 256 ) void attn_merge_kernel( Partials part,
   }
 }
 
+// More than 8 splits: G groups of `dims` threads take every G-th split, eight of them requested at once, and add their parts up in LDS.  One memory round
+// trip up to 8 G splits, where the kernel above takes one for every split beyond its eight (70B, one context of 4096 keys in 32 splits: 20.6 us, so 14.8).
+constexpr uint32_t MERGE_GROUPS = 8;
+template<typename T>
+__global__ __launch_bounds__( 1024 ) void attn_merge_many_kernel( Partials part,
+                                                                  const void* const* __restrict__ layer_rows,
+                                                                  const uint32_t* __restrict__ pos,
+                                                                  T* __restrict__ xb,
+                                                                  uint32_t n_heads,
+                                                                  uint32_t head_size,
+                                                                  uint32_t chunk,
+                                                                  uint32_t max_splits,
+                                                                  uint32_t dims )
+{
+  constexpr uint32_t G = MERGE_GROUPS, BATCH = 8;
+  __shared__ float s_m[G], s_l[G], s_out[G][128];
+  const uint32_t head = blockIdx.x;
+  const uint32_t ctx = blockIdx.y;
+  const void* const rows = layer_rows[ctx];
+  const uint32_t last = pos[ctx]; // read before the branch on `rows`: one round trip for the two
+  if ( rows == nullptr ) {
+    return;
+  }
+  const uint32_t n_splits = min( ( last + chunk ) / chunk, max_splits ); // as above
+  const uint64_t slot0 = ( (uint64_t)ctx * n_heads + head ) * max_splits;
+  const float2* ml = reinterpret_cast<const float2*>( part.ml ) + slot0;
+  const uint32_t group = threadIdx.x / dims, in_group = threadIdx.x % dims;
+  for ( uint32_t d0 = 0; d0 < head_size; d0 += dims ) {
+    const uint32_t d = d0 + in_group, dl = min( d, head_size - 1 );
+    float m = -INFINITY, l = 0.0f, acc = 0.0f;
+    for ( uint32_t first = group; first < n_splits; first += G * BATCH ) { // (uniform in a wave)
+      float2 st[BATCH];
+      float o[BATCH];
+#pragma unroll
+      for ( uint32_t u = 0; u < BATCH; u++ ) { // a split past the last reads the last again and weighs nothing
+        const uint32_t sp = min( first + u * G, n_splits - 1 );
+        st[u] = ml[sp];
+        o[u] = part.out[( slot0 + sp ) * head_size + dl];
+      }
+      float m_new = m;
+#pragma unroll
+      for ( uint32_t u = 0; u < BATCH; u++ ) {
+        m_new = first + u * G < n_splits ? fmaxf( m_new, st[u].x ) : m_new;
+      }
+      const float m_ref = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = fast_exp2( m - m_ref );
+      l *= alpha;
+      acc *= alpha;
+#pragma unroll
+      for ( uint32_t u = 0; u < BATCH; u++ ) {
+        const float wgt = first + u * G < n_splits ? fast_exp2( st[u].x - m_ref ) : 0.0f;
+        l += st[u].y * wgt;
+        acc += first + u * G < n_splits ? o[u] * wgt : 0.0f;
+      }
+      m = m_new;
+    }
+    if ( d0 > 0 ) {
+      __syncthreads(); // the last dims' parts have been read
+    }
+    s_out[group][in_group] = acc;
+    if ( in_group == 0 ) {
+      s_m[group] = m;
+      s_l[group] = l;
+    }
+    __syncthreads();
+    if ( group == 0 && d < head_size ) {
+      float m_all = -INFINITY;
+#pragma unroll
+      for ( uint32_t g = 0; g < G; g++ ) {
+        m_all = fmaxf( m_all, s_m[g] );
+      }
+      const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
+      l = 0.0f;
+      acc = 0.0f;
+#pragma unroll
+      for ( uint32_t g = 0; g < G; g++ ) { // a group without splits: maximum -inf, sums of zero
+        const float wgt = fast_exp2( s_m[g] - m_ref );
+        l += s_l[g] * wgt;
+        acc += s_out[g][in_group] * wgt;
+      }
+      xb[( (uint64_t)ctx * n_heads + head ) * head_size + d] = from_f32<T>( acc * ( 1.0f / l ) );
+    }
+  }
+}
+
 // =================================================================================================
 // joined splits: the splits of a (context, kv head) stream are the waves of ONE work-group, which adds them up itself
 //
@@ -1303,6 +1388,26 @@ JoinChoice join_choice( uint64_t streams, int variant, uint32_t n_tok )
   return c;
 }
 
+// Few streams of few keys: a wave's keys are a chain (20 us for 256 of them, 10 for 64), and most CUs have none, so splits go below the 256 keys that the
+// rules for a full chip keep.  Up to about 800 waves of the MFMA kernel and 1536 of the VALU kernel, at least four splits; at least 64 keys, 32 where that is a
+// share of up to 256.  Only while they stay short, as longer ones come out even with or behind the plan they replace (7B, 4 contexts of 2048 keys: 26.6 us, in
+// splits of 192 28.9), and where there are keys enough for the streams that many waves pay for a merge kernel (70B, 48 contexts of 128 keys: one split 11.4,
+// four and a merge 14.8).  us, the fused op with splits of 256 or joined / so; 70B shape, contexts x keys:
+//   1 x 300: 19.5 / 9.3   1 x 1537: 19.8 / 11.3   1 x 4096: 20.9 / 12.3   4 x 1025: 19.6 / 12.2   9 x 512: 20.0 / 11.7   16 x 768: 21.8 / 17.0
+//   32 x 300: 22.4 / 14.8   48 x 768: 36.2 / 32.9
+// 7B shape: 1 x 1025: 19.7 / 11.4   4 x 512: 22.2 / 12.1   9 x 300: 23.4 / 13.8   16 x 300: 25.3 / 18.6   16 x 768: 38.8 / 36.5
+// Splits per stream of such a plan at most, 0: none.
+uint64_t short_splits( uint64_t streams, const gh_shape* s, int variant )
+{
+  const bool mfma = variant == GH_ATTN_MFMA;
+  if ( streams == 0 || streams > ( mfma ? 384u : 512u ) || variant == GH_ATTN_GENERIC ) {
+    return 0;
+  }
+  const uint64_t splits = std::clamp<uint64_t>( ( mfma ? 800 : 1536 ) / streams, 4, 64 );
+  // what gh_attn_decode_static holds: a call that it took is not refused for being cut finer
+  return streams * splits * s->gqa_size * ( s->head_size + 2ull ) * sizeof( float ) <= STATIC_SCRATCH_BYTES ? splits : 0;
+}
+
 bool fast_ok( const gh_shape* s, gh_dtype dt ) { return dt == GH_F16 && s->head_size == HS; }
 bool valu_gqa_ok( uint32_t g ) { return g == 1 || g == 2 || g == 4 || g == 8; }
 bool mfma_gqa_ok( uint32_t g ) { return g == 2 || g == 4 || g == 8 || g == 16; }
@@ -1346,8 +1451,17 @@ Plan make_plan( uint64_t batch, uint32_t max_pos, const gh_shape* s, gh_dtype dt
       chunk = 256;
     }
     split_cap = std::min<uint64_t>( splits, ( n_tok + 255 ) / 256 );
+    bool short_plan = false;
+    if ( const uint64_t most = short_splits( streams, s, p.variant ) ) {
+      const uint64_t keys = std::max<uint64_t>( ( ( n_tok + most - 1 ) / most + 15 ) / 16 * 16, n_tok <= 256 ? 32 : 64 );
+      short_plan = ( keys <= 160 || ( keys <= 192 && n_tok <= 768 ) ) && 10ull * n_tok >= ( p.variant == GH_ATTN_MFMA ? 7 : 5 ) * streams;
+      if ( short_plan ) {
+        chunk = (uint32_t)keys;
+      }
+      split_cap = std::max( split_cap, std::min<uint64_t>( most, ( n_tok + 31 ) / 32 ) );
+    }
     // the joined route where it pays: never more splits than the rule above gives, so the workspace bound holds either way
-    if ( g_split_join != 0 && p.variant != GH_ATTN_GENERIC ) {
+    if ( !short_plan && g_split_join != 0 && p.variant != GH_ATTN_GENERIC ) {
       const JoinChoice c = join_choice( streams, p.variant, n_tok );
       if ( c.waves != 0 && c.splits <= splits ) {
         chunk = ( n_tok + c.splits - 1 ) / c.splits;
@@ -1710,14 +1824,18 @@ static int attn_decode_run( const char* who, const void* q, const void* const* l
 
   if ( plan.max_splits > 1 && !joined ) {
     const dim3 grid( shape->n_heads, (unsigned)batch );
-    const unsigned threads = shape->head_size <= 64 ? 64 : ( shape->head_size <= 128 ? 128 : 256 );
-    if ( dt == GH_F16 ) {
-      attn_merge_kernel<__half><<<grid, threads, 0, st>>>( part, layer_rows_dev, pos_dev, static_cast<__half*>( xb ), shape->n_heads,
-                                                          shape->head_size, plan.chunk, plan.max_splits );
-    } else {
-      attn_merge_kernel<float><<<grid, threads, 0, st>>>( part, layer_rows_dev, pos_dev, static_cast<float*>( xb ), shape->n_heads,
-                                                         shape->head_size, plan.chunk, plan.max_splits );
-    }
+    auto merge = [&]( auto* out ) {
+      // (more work-groups of 1024 threads than the chip holds at once wait for each other: 70B, 16 contexts of 1025 keys in 9 splits 20.9 us with the one
+      // kernel, 25.7 with the other)
+      if ( plan.max_splits > 8 && grid.x * batch <= 2ull * cu_count() ) {
+        const unsigned dims = shape->head_size <= 64 ? 64 : 128;
+        attn_merge_many_kernel<<<grid, MERGE_GROUPS * dims, 0, st>>>( part, layer_rows_dev, pos_dev, out, shape->n_heads, shape->head_size, plan.chunk, plan.max_splits, dims );
+      } else {
+        const unsigned threads = shape->head_size <= 64 ? 64 : ( shape->head_size <= 128 ? 128 : 256 );
+        attn_merge_kernel<<<grid, threads, 0, st>>>( part, layer_rows_dev, pos_dev, out, shape->n_heads, shape->head_size, plan.chunk, plan.max_splits );
+      }
+    };
+    dt == GH_F16 ? merge( static_cast<__half*>( xb ) ) : merge( static_cast<float*>( xb ) );
     GH_LAUNCH_CHECK();
   }
   return timed ? timer_mark( st, &timer, 2 ) : GH_OK;
