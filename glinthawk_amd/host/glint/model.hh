@@ -446,13 +446,14 @@ public:
     if ( !pipelined ) {
       ops_.template rmsnorm<Config::dim>( pxb, px, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, n );
     }
+    // one table entry per (context, token) for the rows of every layer
+    GLINT_GH( gh_prefill_layer_tables( layer_rows_dev( 0 ), 2 * table_stride(), run.size(), pos_dev(), batch, n_tokens, row_bytes, pf_token_rows(), pf_pos(), ops_.stream() ) );
     for ( size_t k = 0; k < run.size(); k++ ) {
       const auto& w = layers_[run[k]];
-      // one table entry per (context, token) for this layer's rows
-      GLINT_GH( gh_prefill_tables( layer_rows_dev( k ), pos_dev(), batch, n_tokens, row_bytes, nullptr, pf_token_rows(), pf_pos(), ops_.stream() ) );
+      void** const token_rows = pf_token_rows() + k * n;
       if ( n <= PREFILL_FUSED_ROWS ) {
         // few tokens: products bound by their weights, with the follow-up ops fused, as in decode
-        ops_.matmul_qkv_rope_append( pq, pxb, w.wq, n, pf_pos(), base_.freq_cis_real, base_.freq_cis_imag, pf_token_rows() );
+        ops_.matmul_qkv_rope_append( pq, pxb, w.wq, n, pf_pos(), base_.freq_cis_real, base_.freq_cis_imag, token_rows );
         GLINT_GH( gh_attn_prefill( pq, layer_rows_dev( k ), pos_dev(), pxb, batch, n_tokens, max_start, &shape, hip::gh_type<DType>(), pf_attn_ws_.get(),
                                    pf_attn_ws_bytes_, GH_ATTN_AUTO, ops_.stream() ) );
         ops_.template matmul_accum<Config::dim, Config::dim>( px, pxb, w.wo, n, pxb, w.rms_ffn_weight );
@@ -481,7 +482,7 @@ public:
                && gh_matmul_qkv_fuses_many_rows( Config::dim, Config::n_kv_heads, Config::gqa_size, Config::head_size, rows, hip::gh_type<DType>() ) == 1 ) {
             // ... that rotates and appends as well
             ops_.matmul_qkv_rope_append( pq + r0 * Config::dim, pxb + r0 * Config::dim, w.wq, rows, pf_pos() + r0, base_.freq_cis_real, base_.freq_cis_imag,
-                                         pf_token_rows() + r0 );
+                                         token_rows + r0 );
             continue;
           }
           if ( together ) {
@@ -491,8 +492,8 @@ public:
             ops_.template matmul<Config::dim, Config::dim>( pq + r0 * Config::dim, pxb + r0 * Config::dim, w.wq, rows );
             ops_.template matmul<Config::dim, Config::kv_dim * 2>( pkv + r0 * Config::kv_dim * 2, pxb + r0 * Config::dim, w.wkv, rows );
           }
-          GLINT_GH( gh_kv_append( pf_token_rows() + r0, pkv + r0 * Config::kv_dim * 2, rows, Config::kv_dim, hip::gh_type<DType>(), ops_.stream() ) );
-          GLINT_GH( gh_rope( rows, pf_pos() + r0, base_.freq_cis_real, base_.freq_cis_imag, pq + r0 * Config::dim, pf_token_rows() + r0, Config::n_kv_heads,
+          GLINT_GH( gh_kv_append( token_rows + r0, pkv + r0 * Config::kv_dim * 2, rows, Config::kv_dim, hip::gh_type<DType>(), ops_.stream() ) );
+          GLINT_GH( gh_rope( rows, pf_pos() + r0, base_.freq_cis_real, base_.freq_cis_imag, pq + r0 * Config::dim, token_rows + r0, Config::n_kv_heads,
                              Config::gqa_size, Config::head_size, hip::gh_type<DType>(), ops_.stream() ) );
         }
         GLINT_GH( gh_attn_prefill( pq, layer_rows_dev( k ), pos_dev(), pxb, batch, n_tokens, max_start, &shape, hip::gh_type<DType>(), pf_attn_ws_.get(),
@@ -1030,7 +1031,7 @@ private:
       pf_xb2_ = ops_.device_allocate( n * Config::dim * sizeof( DType ) );
       pf_kv_ = ops_.device_allocate( n * Config::kv_dim * 2 * sizeof( DType ) );
     }
-    pf_tables_ = ops_.device_allocate( n * ( sizeof( void* ) + sizeof( uint32_t ) ) + 64 );
+    pf_tables_ = ops_.device_allocate( n * ( pf_layers() * sizeof( void* ) + sizeof( uint32_t ) ) + 64 );
     const gh_shape shape = LlamaOperations::shape();
     // sized for the widest call: every context contributes all n tokens
     pf_attn_ws_bytes_ = gh_attn_prefill_workspace( 1, static_cast<uint32_t>( n ), &shape );
@@ -1069,7 +1070,8 @@ private:
     }
   }
   void** pf_token_rows() const { return reinterpret_cast<void**>( pf_tables_.get() ); }
-  uint32_t* pf_pos() const { return reinterpret_cast<uint32_t*>( pf_token_rows() + pf_capacity_ ); }
+  uint64_t pf_layers() const { return std::max<uint64_t>( 1, settings_.num_attention_layers_hosted() ); }
+  uint32_t* pf_pos() const { return reinterpret_cast<uint32_t*>( pf_token_rows() + pf_layers() * pf_capacity_ ); }
 
   DevicePtr base_storage_ {}, layer_storage_ {}, scratch_storage_ {}, attn_ws_ {}, tables_dev_ {};
   DevicePtr pf_x_ {}, pf_xb_ {}, pf_q_ {}, pf_hb_ {}, pf_hb2_ {}, pf_xb2_ {}, pf_kv_ {}, pf_tables_ {}, pf_attn_ws_ {};

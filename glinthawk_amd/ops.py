@@ -317,6 +317,16 @@ def prefill_tables(layer_rows: torch.Tensor, start_pos: torch.Tensor, n_tokens: 
     return rows, trows, pos
 
 
+def prefill_layer_tables(layer_rows: torch.Tensor, start_pos: torch.Tensor, n_tokens: int, row_bytes: int):
+    """layer_rows: (layers, batch or more) table of which the entries of start_pos are used; (rows of every token in every layer, positions)."""
+    layers, batch = layer_rows.shape[0], start_pos.numel()
+    trows = torch.empty((layers, batch * n_tokens), dtype=torch.int64, device=layer_rows.device)
+    pos = torch.empty(batch * n_tokens, dtype=torch.int32, device=layer_rows.device)
+    check(lib().gh_prefill_layer_tables(_p(layer_rows), layer_rows.shape[1], layers, _p(start_pos), batch, n_tokens, row_bytes, _p(trows), _p(pos), _stream()),
+          "gh_prefill_layer_tables")
+    return trows, pos
+
+
 def attn_prefill(q, layer_rows: torch.Tensor, start_pos: torch.Tensor, xb, n_tokens: int, max_start_pos: int, shape: Shape,
                  variant: int = GH_ATTN_AUTO) -> None:
     s = shape.c()

@@ -329,6 +329,10 @@ int gh_attn_decode_host( const void* q, const void* const* layer_rows_host, cons
  *   pos_out[i*T+t] = start_i + t.  Any output may be NULL. */
 int gh_prefill_tables( const void* const* layer_rows_dev, const uint32_t* start_pos_dev, uint64_t batch, uint32_t n_tokens, uint64_t row_bytes,
                        const void** layer_rows_out, void** token_rows_out, uint32_t* pos_out, gh_stream stream );
+/* The cache rows for all of `layers` layers in one launch: layer k's table begins layer_stride entries behind that of k - 1, its rows go to
+ * token_rows_out[k * batch * n_tokens + ...] */
+int gh_prefill_layer_tables( const void* const* layer_rows_dev, uint64_t layer_stride, uint64_t layers, const uint32_t* start_pos_dev, uint64_t batch, uint32_t n_tokens,
+                             uint64_t row_bytes, void** token_rows_out, uint32_t* pos_out, gh_stream stream );
 /* Causal attention of the new tokens over the cache (their rows already appended and rotated):
  * query token t of context i attends keys [0, start_i + t].  f16 / head size 128 runs a tiled MFMA
  * kernel; other shapes run the decode kernels on expanded tables (workspace needed, see

@@ -345,3 +345,17 @@ def test_prefill_one_key_stands_out(shape):
         got = xb.float().cpu().numpy()
         assert np.isfinite(got).all(), f"key {j}"
         assert_close(got, want, mean_rel=4e-3, what=f"key {j}")
+
+
+@pytest.mark.parametrize("layers,batch,n_tokens,spare", [(1, 1, 1, 0), (3, 2, 77, 3), (2, 5, 256, 0), (4, 3, 300, 1)])
+def test_tables_of_all_layers(layers, batch, n_tokens, spare):
+    """Rows of every layer from one call, as a call per layer gives them; an empty context has none."""
+    g = torch.Generator().manual_seed(n_tokens)
+    table = torch.randint(1, 1 << 40, (layers, batch + spare), generator=g).cuda()
+    table[:, batch // 2] = 0
+    start = torch.randint(0, 1000, (batch,), generator=g, dtype=torch.int32).cuda()
+    rows, pos = ops.prefill_layer_tables(table, start, n_tokens, 4096)
+    want_pos = (start[:, None] + torch.arange(n_tokens, dtype=torch.int32, device="cuda")).flatten()
+    assert torch.equal(pos, want_pos)
+    base = table[:, :batch].repeat_interleave(n_tokens, 1)
+    assert torch.equal(rows, torch.where(base == 0, 0, base + want_pos.long() * 4096))
