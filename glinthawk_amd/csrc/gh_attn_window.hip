@@ -317,12 +317,12 @@ __host__ __device__ inline uint64_t partial_stride( const WindowShape& s ) { ret
 
 // The results of a work-group's NW waves for the query heads h0 .. h0 + nh - 1 of a row, wave w's for head h at
 // lds[(w * hq + h) * (vpad + 2)]: added up and stored, as the output or as the partial result of a split.
-template<typename E, int NW>
+template<typename E, int NW, int THREADS = 64 * NW>
 __device__ __forceinline__ void finish_split( const WindowOut<E>& out, float* partial, const float* lds, uint32_t hq, uint32_t nh, uint64_t row, uint32_t h0, uint32_t split,
                                               uint32_t splits, const WindowShape& s )
 {
   const uint32_t stride = s.vpad + 2;
-  for ( uint32_t i = threadIdx.x; i < nh * s.vpad; i += 64 * NW ) {
+  for ( uint32_t i = threadIdx.x; i < nh * s.vpad; i += THREADS ) {
     const uint32_t h = i / s.vpad, e = i % s.vpad;
     float m = NO_KEY;
 #pragma unroll
@@ -511,7 +511,8 @@ __global__ __launch_bounds__( 256 ) void window_rows_kernel( WindowOut<E> out,
   finish_split<E, 4>( out, partial, lds, HQ, nh, row, h0, split, splits, s );
 }
 
-// one wave per (row, head)
+// One wave per (row, head): lane k holds maximum and sum of split k (at most 64), and eight splits' values are requested at once (one row of 32 heads, 1025
+// keys: 16.5 us with the attention, with a split after the other 18.6).
 template<typename E>
 __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, const float* __restrict__ partial, WindowRows wr, WindowShape s, uint32_t splits,
                                                               uint64_t pairs )
@@ -522,21 +523,26 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
   }
   const uint32_t lane = threadIdx.x & 63, stride = s.vpad + 2;
   const float* src = partial + pair * splits * stride;
-  float m = NO_KEY;
-  for ( uint32_t k = 0; k < splits; k++ ) {
-    m = fmaxf( m, src[k * stride + s.vpad + 1] );
-  }
+  const float* own = src + min( lane, splits - 1 ) * stride + s.vpad;
+  const float own_sum = own[0], own_max = own[1];
   const uint64_t row = pair / s.heads;
   const uint32_t head = (uint32_t)( pair % s.heads );
   const float gate = out.gate( row, head );
-  float sm = 0.0f;
-  for ( uint32_t k = 0; k < splits; k++ ) {
-    sm += src[k * stride + s.vpad] * __expf( src[k * stride + s.vpad + 1] - m );
-  }
+  const float m = wave_max( own_max ); // (the last split's repeated in the lanes beyond)
+  const float weight = lane < splits ? __expf( own_max - m ) : 0.0f;
+  const float sm = wave_sum( lane < splits ? own_sum * weight : 0.0f );
   for ( uint32_t e = lane; e < s.vdim; e += 64 ) {
     float a = 0.0f;
-    for ( uint32_t k = 0; k < splits; k++ ) {
-      a += src[k * stride + e] * __expf( src[k * stride + s.vpad + 1] - m );
+    for ( uint32_t k0 = 0; k0 < splits; k0 += 8 ) {
+      float v[8];
+#pragma unroll
+      for ( uint32_t u = 0; u < 8; u++ ) { // a split past the last reads the last again and is not added
+        v[u] = src[min( k0 + u, splits - 1 ) * stride + e];
+      }
+#pragma unroll
+      for ( uint32_t u = 0; u < 8; u++ ) {
+        a += k0 + u < splits ? v[u] * lane_value( weight, min( k0 + u, splits - 1 ) ) : 0.0f;
+      }
     }
     out.out[row * out.stride + head * s.vdim + e] = from_f32<E>( a / sm * gate );
   }
@@ -873,8 +879,8 @@ __device__ __forceinline__ float column_max( float v )
   return half_wave_max( fmaxf( __builtin_bit_cast( float, even ), __builtin_bit_cast( float, odd ) ) );
 }
 
-// D: head size up to which the kernel goes; NW waves
-template<int D, bool SHARED, int NW>
+// D: head size up to which the kernel goes; NW waves, HB blocks of head_cols heads side by side, NW / HB waves on the keys of each
+template<int D, bool SHARED, int NW, int HB>
 __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kernel( WindowOut<__bf16> out,
                                                                                          float* __restrict__ partial,
                                                                                          const __bf16* __restrict__ q,
@@ -887,7 +893,7 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
 {
   constexpr int KS = D / 32, VB = D / 16; // steps of 32 of the query/key size, blocks of 16 of the value size
   __shared__ uint4 tiles[step_lds( NW, SHARED )]; // K and V of each wave, 256 bytes a key
-  const uint32_t head_blocks = s.heads / head_cols;
+  const uint32_t head_blocks = s.heads / ( head_cols * HB );
   const uint32_t hb = blockIdx.x % head_blocks, split = blockIdx.x / head_blocks % splits;
   const uint64_t row = blockIdx.x / head_blocks / splits;
   const uint32_t ctx = (uint32_t)( row / wr.n_tokens ), tok = (uint32_t)( row % wr.n_tokens );
@@ -896,11 +902,11 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
     return;
   }
   const __bf16* cache = reinterpret_cast<const __bf16*>( base + wr.offset );
-  const uint32_t h0 = hb * head_cols, g = h0 / s.group;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), block = wave % HB, turn = wave / HB;
+  const uint32_t h0 = ( hb * HB + block ) * head_cols, g = h0 / s.group;
   const uint32_t pos = wr.start_pos[ctx] + tok;
   const Visible vis = visible_keys( pos, s );
   const uint32_t k_begin = split * keys_per_split, k_end = min( vis.count, k_begin + keys_per_split );
-  const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
   const uint32_t lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
   const uint32_t hc = min( r, head_cols - 1 ); // columns beyond do as the last one and are not stored
   uint4* s_k = tiles + wave * STEP_KEYS * ( SHARED ? 16 : 32 );
@@ -972,11 +978,11 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
     acc[vb] = mfma_f32x4 { 0.0f, 0.0f, 0.0f, 0.0f };
   }
   float m = NO_KEY, l = 0.0f;
-  uint32_t i0 = k_begin + wave * STEP_KEYS;
+  uint32_t i0 = k_begin + turn * STEP_KEYS;
   if ( i0 < k_end ) {
     load( i0 );
   }
-  for ( ; i0 < k_end; i0 += NW * STEP_KEYS ) {
+  for ( ; i0 < k_end; i0 += NW / HB * STEP_KEYS ) {
     uint32_t w_lane = w_home, k_lane = k_home, v_lane = v_home;
     asm( "" : "+v"( w_lane ), "+v"( k_lane ), "+v"( v_lane ) ); // the addresses beside these are made where they are used, not kept in registers
 #pragma unroll
@@ -990,8 +996,8 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
     if ( SHARED && lane < STEP_KEYS ) {
       s_factor[lane] = rf * scale_log2e;
     }
-    if ( i0 + NW * STEP_KEYS < k_end ) {
-      load( i0 + NW * STEP_KEYS );
+    if ( i0 + NW / HB * STEP_KEYS < k_end ) {
+      load( i0 + NW / HB * STEP_KEYS );
     }
     __builtin_amdgcn_fence( __ATOMIC_RELEASE, "wavefront" );
     float st[8]; // of key i0 + 16 (e / 4) + 4 g4 + e % 4
@@ -1091,7 +1097,7 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
     }
   }
   __syncthreads();
-  finish_split<__bf16, NW>( out, partial, results, head_cols, head_cols, row, h0, split, splits, s );
+  finish_split<__bf16, NW / HB, 64 * NW>( out, partial, results, HB * head_cols, HB * head_cols, row, hb * HB * head_cols, split, splits, s );
 }
 
 template<typename E, int NC, bool SHARED>
@@ -1159,31 +1165,36 @@ int attend_decode( const WindowOut<__bf16>& out, const __bf16* q, const float* b
   while ( head_cols > STEP_COLS || s.group % head_cols != 0 ) {
     head_cols--;
   }
-  const uint64_t head_blocks = s.heads / head_cols;
-  // keys of a row over eight waves where work-groups of four would leave room on the CUs and each wave still has a few tiles
-  const bool wide = s.values_are_keys && rows * head_blocks < 4ull * cu_count() && max_pos >= 16 * STEP_KEYS;
+  const uint64_t blocks = s.heads / head_cols, groups = rows * blocks, most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
+  // Eight waves on the keys of a row where work-groups of four would leave room on the CUs and each wave still has a tile or more; with K and V apart a CU
+  // holds one such work-group, which pays only while they are few.  us, 32 heads of 128, rows x keys, four waves / eight.  Values that are keys: 1 x 300
+  // 11.0 / 7.6, 8 x 300 13.8 / 9.2, 24 x 300 15.7 / 17.6, 1 x 2048 26 / 18, 32 x 1025 49.4 / 46.9, 48 x 1025 69.2 / 65.0.  Both: 1 x 1025 18.9 / 16.5, 4 x 1025
+  // 24.8 / 26.8, 8 x 300 17.5 / 13.1, 16 x 300 20.3 / 24.0.
+  const bool wide = s.values_are_keys ? ( groups < 16ull * cu_count() && most >= 16 * STEP_KEYS ) || ( groups <= (uint64_t)cu_count() && most >= 4 * STEP_KEYS )
+                                      : most >= 4 * STEP_KEYS && ( 4 * groups <= (uint64_t)cu_count() || ( groups <= (uint64_t)cu_count() && most <= 16 * STEP_KEYS ) );
+  // Two heads a work-group where there are more work-groups than the CUs hold and few keys to each: half as many starts (32 x 64 15.2 -> 12.0, 32 x 300
+  // 36.2 -> 32.8; 32 x 1025 92 -> 93).
+  const bool pair = !s.values_are_keys && !wide && blocks % 2 == 0 && groups >= 3ull * cu_count() && most <= 16 * STEP_KEYS;
+  const uint64_t head_blocks = pair ? blocks / 2 : blocks;
   SplitPlan plan;
-  if ( int rc = plan_splits( s, rows, head_blocks, max_pos, ( wide ? 8 : 4 ) * STEP_KEYS, st, &plan ) ) {
+  if ( int rc = plan_splits( s, rows, head_blocks, max_pos, ( wide ? 8 : pair ? 2 : 4 ) * STEP_KEYS, st, &plan ) ) {
     return rc;
   }
   const uint64_t grid = rows * head_blocks * plan.splits;
   GH_REQUIRE( grid < ( 1ull << 31 ), "gh_attn_window: grid too large" );
-#define GH_WINDOW_DECODE( D, SHARED, NW ) \
-  window_decode_kernel<D, SHARED, NW><<<(unsigned)grid, 64 * NW, 0, st>>>( out, plan.partial, q, bias, wr, s, head_cols, plan.keys, plan.splits )
-  const bool small = s.dpad <= 64 && s.vpad <= 64;
-  if ( !s.values_are_keys && small ) {
-    GH_WINDOW_DECODE( 64, false, 4 );
-  } else if ( !s.values_are_keys ) {
-    GH_WINDOW_DECODE( 128, false, 4 );
-  } else if ( small && wide ) {
-    GH_WINDOW_DECODE( 64, true, 8 );
-  } else if ( small ) {
-    GH_WINDOW_DECODE( 64, true, 4 );
-  } else if ( wide ) {
-    GH_WINDOW_DECODE( 128, true, 8 );
-  } else {
-    GH_WINDOW_DECODE( 128, true, 4 );
-  }
+#define GH_WINDOW_DECODE( D, SHARED, NW, HB ) \
+  window_decode_kernel<D, SHARED, NW, HB><<<(unsigned)grid, 64 * NW, 0, st>>>( out, plan.partial, q, bias, wr, s, head_cols, plan.keys, plan.splits )
+  auto launch = [&]( auto size ) {
+    constexpr int D = decltype( size )::value;
+    if ( s.values_are_keys ) {
+      wide ? GH_WINDOW_DECODE( D, true, 8, 1 ) : GH_WINDOW_DECODE( D, true, 4, 1 );
+    } else if ( pair ) {
+      GH_WINDOW_DECODE( D, false, 4, 2 );
+    } else {
+      wide ? GH_WINDOW_DECODE( D, false, 8, 1 ) : GH_WINDOW_DECODE( D, false, 4, 1 );
+    }
+  };
+  s.dpad <= 64 && s.vpad <= 64 ? launch( std::integral_constant<int, 64> {} ) : launch( std::integral_constant<int, 128> {} );
 #undef GH_WINDOW_DECODE
   GH_LAUNCH_CHECK();
   return merge_splits( out, plan, wr, s, rows, st );

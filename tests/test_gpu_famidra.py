@@ -211,6 +211,19 @@ def test_windowed_attention(name, dtype):
         assert_rows(attend(shape, q, k, v, rel, [p, p], 1, dtype)[:, 0].reshape(2, -1), w.reshape(2, -1), tol, f"token {p}")
 
 
+# more work-groups than the CUs hold (two blocks of heads each, where their number is even), as many as they hold and few (eight waves on a row's keys)
+@pytest.mark.parametrize("contexts", [400, 40, 3])
+@pytest.mark.parametrize("name", ["grouped", "matrix", "own", "open"])
+def test_windowed_attention_of_many_contexts(name, contexts):
+    """Single tokens at another position in every context, an uneven number of keys to every wave."""
+    T = 150
+    shape, q, k, v, rel, want = attention_case(name, T, 5, n_seq=2)
+    start = [(37 * i + 11) % T for i in range(contexts)]
+    pick = [i % 2 for i in range(contexts)]
+    got = attend(shape, [q[i] for i in pick], [k[i] for i in pick], [v[i] for i in pick], rel, start, 1, "bf16")
+    assert_rows(got[:, 0].reshape(contexts, -1), np.stack([want[i][s] for i, s in zip(pick, start)]).reshape(contexts, -1), 8e-3, "tokens")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["grouped", "matrix", "ten", "own"])
 def test_one_key_stands_out(name, dtype):
