@@ -115,7 +115,9 @@ SIGNATURES = {
     "gh_accum": (_i, [_vp, _vp, _u64, _u64, _i, _vp]),
     "gh_rmsnorm": (_i, [_vp, _vp, _vp, _u64, _u64, _i, _vp]),
     "gh_silu": (_i, [_vp, _vp, _u64, _u64, _i, _vp]),
-    "gh_embed_rows": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _i, _vp]),
+    "gh_rows_in": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _vp, _vp, _u64, _i, _vp]),
+    "gh_rows_out": (_i, [_vp, _vp, _u64, _vp]),
+    "gh_embed_rows": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _vp, _vp, _u64, _i, _vp]),
     "gh_argmax": (_i, [_vp, _vp, _vp, _u64, _u64, _i, _vp]),
     "gh_gemm_set_tuning": (_i, [_i, _i, _i]),
     "gh_gemm_set_gate_waves": (_i, [_i]),

@@ -142,11 +142,104 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
   }
 }
 
+// ---- rows that arrive in page-locked host memory -------------------------------------------------
+// The first kernel of a step reads them where the host left them: they go to the device and, normed, to the first product, and the step's tables come along
+// in work-groups of their own.  As copies in front of rmsnorm_kernel each is a launch and a hand-over between engines more.  Bound by the bus.
+// The copy engine is the faster way over it for 2 MB and more: beyond 1.5 MiB the rows are copied (f16 with norm, tables and a wait, copied and in place:
+// 32 rows of 4096 28.1 and 19.6 us, 64 of 8192 43.4 and 36.8, 128 61.7 and 61.9, 256 99 and 109).
+constexpr uint64_t ROWS_IN_BYTES = 3ull << 19;
+// The sums as rmsnorm_kernel takes them, from registers: a second pass would cross the bus again.  16-byte pieces; PIECES: a thread's.
+template<typename T, int PIECES>
+__global__ __launch_bounds__( EW_THREADS ) void rows_in_kernel( T* __restrict__ x,
+                                                               T* __restrict__ normed,
+                                                               const T* __restrict__ host,
+                                                               const T* __restrict__ weight,
+                                                               uint32_t size,
+                                                               uint32_t rows,
+                                                               uint4* __restrict__ table,
+                                                               const uint4* __restrict__ host_table,
+                                                               uint32_t table_pieces )
+{
+  __shared__ float smem[EW_THREADS / WAVE];
+  if ( blockIdx.x >= rows ) {
+    const uint32_t i = ( blockIdx.x - rows ) * EW_THREADS + threadIdx.x;
+    if ( i < table_pieces ) {
+      table[i] = host_table[i];
+    }
+    return;
+  }
+  constexpr int N = Vec16<T>::N;
+  const uint32_t n_vec = size / N;
+  const uint64_t first = (uint64_t)blockIdx.x * n_vec;
+  Vec16<T> v[PIECES], w[PIECES];
+#pragma unroll
+  for ( int p = 0; p < PIECES; p++ ) { // a piece past the row's end is the first again and counts nothing
+    const uint32_t i = p * EW_THREADS + threadIdx.x, at = i < n_vec ? i : 0;
+    v[p].raw = reinterpret_cast<const uint4*>( host )[first + at];
+    w[p].raw = reinterpret_cast<const uint4*>( weight )[at];
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for ( int p = 0; p < PIECES; p++ ) {
+    const bool in = p * EW_THREADS + threadIdx.x < n_vec;
+#pragma unroll
+    for ( int k = 0; k < N; k++ ) {
+      const float f = to_f32( v[p].v[k] );
+      ss += in ? f * f : 0.0f;
+    }
+  }
+  ss = block_sum( ss, smem );
+  ss = ss / (float)size + 1e-5f;
+  const float inv = 1.0f / sqrtf( ss );
+#pragma unroll
+  for ( int p = 0; p < PIECES; p++ ) {
+    const uint32_t i = p * EW_THREADS + threadIdx.x;
+    if ( i < n_vec ) {
+      reinterpret_cast<uint4*>( x )[first + i] = v[p].raw;
+#pragma unroll
+      for ( int k = 0; k < N; k++ ) {
+        v[p].v[k] = from_f32<T>( to_f32( w[p].v[k] ) * ( inv * to_f32( v[p].v[k] ) ) );
+      }
+      reinterpret_cast<uint4*>( normed )[first + i] = v[p].raw;
+    }
+  }
+}
+
+// Rows to page-locked memory, bound by the bus; no size at which the copy engine is faster was found (f16 with the wait, copied and so: 1 row of 8192 16.2 and
+// 15.9 us, 32 of 4096 28.4 and 20.8, 64 of 8192 42.2 and 34.8, 256 99 and 92).
+__global__ __launch_bounds__( EW_THREADS ) void copy_pieces_kernel( uint4* __restrict__ dst, const uint4* __restrict__ src, uint64_t n )
+{
+  const uint64_t stride = (uint64_t)gridDim.x * EW_THREADS;
+  for ( uint64_t i = (uint64_t)blockIdx.x * EW_THREADS + threadIdx.x; i < n; i += stride ) {
+    dst[i] = src[i];
+  }
+}
+
+// Whether kernels can read and write this host memory, i.e. it was allocated page-locked.
+bool page_locked( const void* p )
+{
+  hipPointerAttribute_t a {};
+  const bool known = hipPointerGetAttributes( &a, p ) == hipSuccess;
+  if ( !known ) {
+    (void)hipGetLastError(); // memory the runtime has not heard of: not an error of the next launch
+  }
+  return known && a.type == hipMemoryTypeHost && a.devicePointer == p;
+}
+
 // ---- rows of a table by index: one block per row, bytes as they are -------------------------------
+// (with a step's table in work-groups of its own, as above)
 template<typename P>
 __global__ __launch_bounds__( EW_THREADS ) void embed_rows_kernel( P* __restrict__ x, const uint32_t* __restrict__ tokens, const P* __restrict__ table, uint32_t width,
-                                                                  uint32_t vocab )
+                                                                  uint32_t vocab, uint32_t rows, uint4* __restrict__ step, const uint4* __restrict__ host_step,
+                                                                  uint32_t step_pieces )
 {
+  if ( blockIdx.x >= rows ) {
+    const uint32_t i = ( blockIdx.x - rows ) * EW_THREADS + threadIdx.x;
+    if ( i < step_pieces ) {
+      step[i] = host_step[i];
+    }
+    return;
+  }
   const uint64_t token = tokens[blockIdx.x];
   if ( token >= vocab ) {
     return; // a row without a token stays as it is
@@ -414,21 +507,95 @@ int gh_rmsnorm( void* out, const void* x, const void* weight, uint64_t size, uin
   return GH_OK;
 }
 
-int gh_embed_rows( void* x, const uint32_t* tokens_dev, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, gh_dtype dt, gh_stream stream )
+int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, void* table_dev, const void* table_host, uint64_t table_bytes,
+                gh_dtype dt, gh_stream stream )
 {
   if ( int rc = ensure_init() ) {
     return rc;
   }
-  if ( batch == 0 || width == 0 ) {
+  if ( size == 0 ) {
+    batch = 0;
+  }
+  if ( batch == 0 ) {
+    dt = GH_F16; // a table alone: bytes as they are
+  }
+  GH_REQUIRE( batch == 0 || ( x && normed && host && weight ), "gh_rows_in: NULL pointer" );
+  GH_REQUIRE( table_bytes == 0 || ( table_dev && table_host ), "gh_rows_in: NULL table" );
+  GH_REQUIRE( size <= 0xffffffffull && batch <= 0x7fffffffull && table_bytes <= ( 1ull << 34 ), "gh_rows_in: shape too large" );
+  const uint64_t bytes = size * dtype_size( dt ), pieces = ( bytes / 16 + EW_THREADS - 1 ) / EW_THREADS;
+  if ( table_bytes % 16 != 0 || !aligned16( table_dev ) || !aligned16( table_host ) || ( table_bytes > 0 && !page_locked( table_host ) ) ) {
+    GH_HIP( hipMemcpyAsync( table_dev, table_host, table_bytes, hipMemcpyHostToDevice, as_stream( stream ) ) );
+    table_bytes = 0;
+  }
+  const uint64_t table_groups = ( table_bytes / 16 + EW_THREADS - 1 ) / EW_THREADS;
+  const bool in_place = batch > 0 && batch * bytes <= ROWS_IN_BYTES && bytes % 16 == 0 && pieces <= 4 && aligned16( x ) && aligned16( normed ) && aligned16( host )
+                        && aligned16( weight ) && page_locked( host );
+  const uint64_t rows = in_place ? batch : 0;
+  if ( rows + table_groups > 0 ) {
+    auto launch = [&]( auto* e, auto count ) {
+      using T = std::remove_pointer_t<decltype( e )>;
+      rows_in_kernel<T, decltype( count )::value><<<(unsigned)( rows + table_groups ), EW_THREADS, 0, as_stream( stream )>>>(
+        static_cast<T*>( x ), static_cast<T*>( normed ), static_cast<const T*>( host ), static_cast<const T*>( weight ), (uint32_t)size, (uint32_t)rows,
+        static_cast<uint4*>( table_dev ), static_cast<const uint4*>( table_host ), (uint32_t)( table_bytes / 16 ) );
+    };
+    GH_DISPATCH_DT( dt, pieces <= 2 ? launch( static_cast<T*>( nullptr ), std::integral_constant<int, 2> {} )
+                                    : launch( static_cast<T*>( nullptr ), std::integral_constant<int, 4> {} ) );
+    GH_LAUNCH_CHECK();
+  }
+  if ( batch == 0 || in_place ) {
     return GH_OK;
   }
-  GH_REQUIRE( x && tokens_dev && table, "gh_embed_rows: NULL pointer" );
-  GH_REQUIRE( width <= 0x7fffffffull && vocab <= 0xffffffffull && batch <= 0x7fffffffull, "gh_embed_rows: shape too large" );
-  const uint64_t bytes = width * dtype_size( dt );
+  GH_HIP( hipMemcpyAsync( x, host, batch * bytes, hipMemcpyHostToDevice, as_stream( stream ) ) );
+  return gh_rmsnorm( normed, x, weight, size, batch, dt, stream );
+}
+
+int gh_rows_out( void* host, const void* x, uint64_t bytes, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( bytes == 0 ) {
+    return GH_OK;
+  }
+  GH_REQUIRE( host && x, "gh_rows_out: NULL pointer" );
+  if ( bytes % 16 == 0 && aligned16( host ) && aligned16( x ) && page_locked( host ) ) {
+    const uint64_t n = bytes / 16;
+    copy_pieces_kernel<<<(unsigned)std::min<uint64_t>( ( n + EW_THREADS - 1 ) / EW_THREADS, 1024 ), EW_THREADS, 0, as_stream( stream )>>>(
+      static_cast<uint4*>( host ), static_cast<const uint4*>( x ), n );
+    GH_LAUNCH_CHECK();
+  } else {
+    GH_HIP( hipMemcpyAsync( host, x, bytes, hipMemcpyDeviceToHost, as_stream( stream ) ) );
+  }
+  GH_HIP( hipStreamSynchronize( as_stream( stream ) ) );
+  return GH_OK;
+}
+
+int gh_embed_rows( void* x, const uint32_t* tokens, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, void* table_dev, const void* table_host,
+                   uint64_t table_bytes, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( width == 0 ) {
+    batch = 0;
+  }
+  GH_REQUIRE( batch == 0 || ( x && tokens && table ), "gh_embed_rows: NULL pointer" );
+  GH_REQUIRE( table_bytes == 0 || ( table_dev && table_host ), "gh_embed_rows: NULL table" );
+  GH_REQUIRE( width <= 0x7fffffffull && vocab <= 0xffffffffull && batch <= 0x3fffffffull && table_bytes <= ( 1ull << 34 ), "gh_embed_rows: shape too large" );
+  if ( table_bytes % 16 != 0 || !aligned16( table_dev ) || !aligned16( table_host ) || ( table_bytes > 0 && !page_locked( table_host ) ) ) {
+    GH_HIP( hipMemcpyAsync( table_dev, table_host, table_bytes, hipMemcpyHostToDevice, as_stream( stream ) ) );
+    table_bytes = 0;
+  }
+  const uint64_t bytes = width * dtype_size( dt ), groups = batch + ( table_bytes / 16 + EW_THREADS - 1 ) / EW_THREADS;
+  if ( groups == 0 ) {
+    return GH_OK;
+  }
   auto launch = [&]( auto piece ) {
     using P = decltype( piece );
-    embed_rows_kernel<P><<<(unsigned)batch, EW_THREADS, 0, as_stream( stream )>>>( static_cast<P*>( x ), tokens_dev, static_cast<const P*>( table ),
-                                                                                   (uint32_t)( bytes / sizeof( P ) ), (uint32_t)vocab );
+    embed_rows_kernel<P><<<(unsigned)groups, EW_THREADS, 0, as_stream( stream )>>>( static_cast<P*>( x ), tokens, static_cast<const P*>( table ),
+                                                                                    (uint32_t)( bytes / sizeof( P ) ), (uint32_t)vocab, (uint32_t)batch,
+                                                                                    static_cast<uint4*>( table_dev ), static_cast<const uint4*>( table_host ),
+                                                                                    (uint32_t)( table_bytes / 16 ) );
   };
   bytes % 16 == 0 && aligned16( x ) && aligned16( table ) ? launch( uint4 {} ) : launch( uint16_t {} );
   GH_LAUNCH_CHECK();

@@ -406,7 +406,8 @@ protected:
   }
   void upload_tables()
   {
-    GLINT_GH( gh_memcpy( tables_dev_.get(), tables_host_, picked_off() + t_picked_ * sizeof( uint32_t ), GH_HOST_TO_DEVICE, 1, ops_.stream() ) );
+    const uint64_t bytes = ( picked_off() + t_picked_ * sizeof( uint32_t ) + 15 ) / 16 * 16; // (there is room: grow_tables)
+    GLINT_GH( gh_rows_in( nullptr, nullptr, nullptr, nullptr, 0, 0, tables_dev_.get(), tables_host_, bytes, DT, ops_.stream() ) );
   }
   const uint8_t* dev() const { return reinterpret_cast<const uint8_t*>( tables_dev_.get() ); }
   void* const* contexts_dev() const { return reinterpret_cast<void* const*>( tables_dev_.get() ); }

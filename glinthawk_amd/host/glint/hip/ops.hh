@@ -140,11 +140,23 @@ public:
     GLINT_GH( gh_argmax( nullptr, output, v, n, batch_size, gh_type<DType>(), stream_ ) );
   }
 
-  // x(i) = table(tokens_dev[i]); a row whose token is not below vocab stays as it is
-  template<uint64_t width, uint64_t vocab>
-  void embed_rows( DType* x, const uint32_t* tokens_dev, const DType* table, const uint64_t batch_size ) const
+  // What a step begins and ends with: rows from host memory with their norm and the step's table, or rows of a table by the tokens in host memory (a row whose
+  // token is not below vocab stays as it is); rows to host memory, there on return.
+  template<uint64_t size>
+  void rows_in( DType* x, DType* normed, const DType* host, const DType* weight, const uint64_t batch_size, void* table_dev, const void* table_host,
+                const uint64_t table_bytes ) const
   {
-    GLINT_GH( gh_embed_rows( x, tokens_dev, table, width, vocab, batch_size, gh_type<DType>(), stream_ ) );
+    GLINT_GH( gh_rows_in( x, normed, host, weight, size, batch_size, table_dev, table_host, table_bytes, gh_type<DType>(), stream_ ) );
+  }
+  template<uint64_t width, uint64_t vocab>
+  void embed_rows( DType* x, const uint32_t* tokens, const DType* table, const uint64_t batch_size, void* table_dev, const void* table_host, const uint64_t table_bytes ) const
+  {
+    GLINT_GH( gh_embed_rows( x, tokens, table, width, vocab, batch_size, table_dev, table_host, table_bytes, gh_type<DType>(), stream_ ) );
+  }
+  void rows_out( DType* host, const DType* x, const uint64_t size_bytes ) const
+  {
+    GLINT_GH( gh_rows_out( host, x, size_bytes, stream_ ) );
+    drains_++;
   }
 
   template<uint64_t hidden_dim>

@@ -201,13 +201,6 @@ public:
       token_positions_[i] = states.token_pos( i );
     }
 
-    const bool embed = first == 0;
-    if ( !embed ) {
-      ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
-    } else if ( !options_.fused_attention ) {
-      load_embedding( states );
-    }
-
     size_t last = Config::n_layers;
     std::vector<size_t> run;
     for ( size_t l = first; l < Config::n_layers && settings_.hosts( l, InferenceStage::PreAttention ); l++ ) {
@@ -218,20 +211,33 @@ public:
         GLINT_CHECK( contexts[i]->prepare( l, states.token_pos( i ), false ) );
       }
     }
-    if ( options_.fused_attention ) {
-      upload_tables( contexts, run, true, embed ? &states : nullptr );
-      if ( embed ) {
-        ops_.template embed_rows<Config::dim, Config::vocab_size>( x_, tokens_dev(), base_.token_embedding_table, batch_ );
-      }
-    }
-
-    spans_.mark( 0, ops_.stream() ); // the activations and the tables are queued: from here to the copy back it is kernels only
-    const bool fused_layers = options_.fused_attention && options_.fused_projections;
+    const bool fused_layers = options_.fused_attention && options_.fused_projections, embed = first == 0;
     // the norms of a layer in the launches of the products behind them, or at the end of those in front of them
     const bool norms_ride = fused_layers && LlamaOperations::norm_rides( Config::dim + 2 * Config::kv_dim, batch_ )
                             && LlamaOperations::norm_rides( 2 * Config::hidden_dim, batch_ );
-    if ( fused_layers && !run.empty() && !norms_ride ) {
-      // the first attention norm stands alone; every later one rides on the epilogue of the previous w2
+    // the first attention norm comes with the activations, or stands alone; every later one rides on the epilogue of the previous w2
+    bool normed = !fused_layers || run.empty() || norms_ride;
+    if ( options_.fused_attention ) {
+      const size_t table_bytes = fill_tables( contexts, run, true, embed ? &states : nullptr );
+      if ( embed ) {
+        ops_.template embed_rows<Config::dim, Config::vocab_size>( x_, tokens_host(), base_.token_embedding_table, batch_, tables_dev_.get(), tables_host_, table_bytes );
+      } else if ( !normed && states.activations().len() == batch_ * Config::dim * sizeof( DType ) ) {
+        ops_.template rows_in<Config::dim>( x_, xb_, reinterpret_cast<const DType*>( states.activations().data() ), layers_[run[0]].rms_att_weight, batch_,
+                                            tables_dev_.get(), tables_host_, table_bytes );
+        normed = true;
+      } else {
+        ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
+        send_tables( table_bytes );
+      }
+      balance_step();
+    } else if ( embed ) {
+      load_embedding( states );
+    } else {
+      ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
+    }
+
+    spans_.mark( 0, ops_.stream() ); // the activations and the tables are there: from here to the copy back it is kernels only
+    if ( !normed ) {
       ops_.template rmsnorm<Config::dim>( xb_, x_, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, batch_ );
     }
     for ( size_t k = 0; k < run.size(); k++ ) {
@@ -388,7 +394,7 @@ public:
                                            k == 0 && start_pos[i] == 0 && settings_.first_layer_served == first_layer ) );
       }
     }
-    upload_tables( contexts, run, false ); // per-context tables: pos = start positions, layer bases per layer
+    const size_t table_bytes = fill_tables( contexts, run, false ); // per-context tables: pos = start positions, layer bases per layer
 
     DType* px = pf_x_.get();
     DType* pxb = pf_xb_.get();
@@ -433,19 +439,20 @@ public:
         ops_.copy( px + r * Config::dim, base_.token_embedding_table + (uint64_t)token_ids[r] * Config::dim, Config::dim * sizeof( DType ),
                    CopyType::DeviceToDevice, true );
       }
+    }
+    if ( pipelined || ( first_layer == 0 && token_ids != nullptr ) ) {
+      send_tables( table_bytes );
+      if ( !pipelined ) {
+        ops_.template rmsnorm<Config::dim>( pxb, px, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, n );
+      }
     } else {
       GLINT_CHECK( acts_in_host != nullptr );
-      if ( !pipelined ) {
-        ops_.copy( px, acts_in_host, n * Config::dim * sizeof( DType ), CopyType::HostToDevice, true );
-      }
+      ops_.template rows_in<Config::dim>( px, pxb, acts_in_host, layers_[run[0]].rms_att_weight, n, tables_dev_.get(), tables_host_, table_bytes );
     }
 
     const gh_shape shape = LlamaOperations::shape();
     const uint64_t row_bytes = 2ull * Config::kv_dim * sizeof( DType );
     const bool fuse_wo = n <= 65535 && gh_matmul_fuses_many_rows( Config::dim, Config::dim, n, hip::gh_type<DType>() ) == 1;
-    if ( !pipelined ) {
-      ops_.template rmsnorm<Config::dim>( pxb, px, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, n );
-    }
     // one table entry per (context, token) for the rows of every layer
     GLINT_GH( gh_prefill_layer_tables( layer_rows_dev( 0 ), 2 * table_stride(), run.size(), pos_dev(), batch, n_tokens, row_bytes, pf_token_rows(), pf_pos(), ops_.stream() ) );
     for ( size_t k = 0; k < run.size(); k++ ) {
@@ -549,7 +556,7 @@ public:
         }
         GLINT_GH( gh_sync( copy_lane_->stream ) );
       } else {
-        ops_.copy( acts_out_host, px, n * Config::dim * sizeof( DType ), CopyType::DeviceToHost );
+        ops_.rows_out( acts_out_host, px, n * Config::dim * sizeof( DType ) );
       }
     }
     const size_t last = run.back();
@@ -771,7 +778,7 @@ private:
       states.allocate_activations();
       states.deallocate_queries();
       states.deallocate_kvs();
-      ops_.copy( reinterpret_cast<DType*>( states.activations().data() ), x_, states.batch_size() * Config::dim * sizeof( DType ), CopyType::DeviceToHost );
+      ops_.rows_out( reinterpret_cast<DType*>( states.activations().data() ), x_, states.batch_size() * Config::dim * sizeof( DType ) );
       if ( most_recent_layer == Config::n_layers - 1 ) {
         states.set_next_stage( InferenceStage::Classification );
       } else {
@@ -785,7 +792,7 @@ private:
   // layout of one upload: pos[cap], tokens[cap] (u32) | for each layer of the run: layer_rows[cap], token_rows[cap] (pointers)
   size_t table_stride() const { return settings_.concurrency_limit; }
   const uint32_t* pos_dev() const { return reinterpret_cast<const uint32_t*>( tables_dev_.get() ); }
-  const uint32_t* tokens_dev() const { return pos_dev() + table_stride(); }
+  const uint32_t* tokens_host() const { return reinterpret_cast<const uint32_t*>( tables_host_ ) + table_stride(); }
   static size_t ptr_tables_offset( const size_t cap ) { return ( 2 * cap * sizeof( uint32_t ) + 15 ) / 16 * 16; }
   uint8_t* ptr_tables( uint8_t* base ) const { return base + ptr_tables_offset( table_stride() ); }
   const void* const* layer_rows_dev( size_t k ) const
@@ -799,7 +806,8 @@ private:
 
   // `decode`: the positions are those of one new token per context (a batched prefill attends from many).  `tokens`: whose tokens are embedded
   // (a row that is not active gets none), or nullptr
-  void upload_tables( const ContextVector& contexts, const std::vector<size_t>& run, const bool decode = true, const StateType* tokens = nullptr )
+  // Returns the bytes that go to the device, which the caller sends, alone or with what else a step begins with; then balance_step().
+  size_t fill_tables( const ContextVector& contexts, const std::vector<size_t>& run, const bool decode = true, const StateType* tokens = nullptr )
   {
     // The previous upload reads the pinned buffer asynchronously: it has to be over before the buffer is rewritten.  A step
     // ends with a blocking copy of its results, which is such a wait already; only without one since the last upload is
@@ -833,10 +841,23 @@ private:
         ptrs[( 2 * k + 1 ) * table_stride() + i] = layer.token( token_positions_[i] ).key();
       }
     }
-    const size_t bytes = ( ptr_tables( tables_host_ ) - tables_host_ ) + run.size() * 2 * table_stride() * sizeof( void* );
-    GLINT_GH( gh_memcpy( tables_dev_.get(), tables_host_, bytes, GH_HOST_TO_DEVICE, 1, ops_.stream() ) );
+    const size_t bytes = ( ptr_tables( tables_host_ ) - tables_host_ ) + run.size() * 2 * table_stride() * sizeof( void* ); // a multiple of 16
     tables_uploaded_ = true;
     tables_drain_count_ = ops_.drain_count();
+    return bytes;
+  }
+  void send_tables( const size_t bytes )
+  {
+    ops_.template rows_in<Config::dim>( nullptr, nullptr, nullptr, nullptr, 0, tables_dev_.get(), tables_host_, bytes );
+  }
+  void upload_tables( const ContextVector& contexts, const std::vector<size_t>& run, const bool decode = true )
+  {
+    send_tables( fill_tables( contexts, run, decode ) );
+    balance_step();
+  }
+  // the cuts of a step over equal runs of keys, from the tables on the device
+  void balance_step()
+  {
     if ( balanced_step_ ) {
       const gh_shape s = LlamaOperations::shape();
       GLINT_GH( gh_attn_balance( layer_rows_dev( 0 ), pos_dev(), batch_, max_pos_, &s, attn_bal_ws_.get(), attn_bal_ws_bytes_, ops_.stream() ) );

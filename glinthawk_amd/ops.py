@@ -85,9 +85,21 @@ def silu(hb: torch.Tensor, hb2: torch.Tensor) -> None:
     check(lib().gh_silu(_p(hb), _p(hb2), hidden, batch, _dt(hb), _stream()), "gh_silu")
 
 
+def rows_in(x: torch.Tensor, normed: torch.Tensor, host, weight: torch.Tensor, table: Optional[torch.Tensor] = None, host_table=None) -> None:
+    """`host`, `host_table`: arrays in host memory, page-locked (pinned_empty) or not."""
+    batch, size = x.shape
+    bytes_ = 0 if table is None else host_table.nbytes
+    check(lib().gh_rows_in(_p(x), _p(normed), host.ctypes.data, _p(weight), size, batch, _p(table), None if table is None else host_table.ctypes.data, bytes_, _dt(x), _stream()),
+          "gh_rows_in")
+
+
+def rows_out(host, x: torch.Tensor) -> None:
+    check(lib().gh_rows_out(host.ctypes.data, _p(x), x.numel() * x.element_size(), _stream()), "gh_rows_out")
+
+
 def embed_rows(x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> None:
     batch, width = x.shape
-    check(lib().gh_embed_rows(_p(x), _p(tokens), _p(table), width, table.shape[0], batch, _dt(x), _stream()), "gh_embed_rows")
+    check(lib().gh_embed_rows(_p(x), _p(tokens), _p(table), width, table.shape[0], batch, None, None, 0, _dt(x), _stream()), "gh_embed_rows")
 
 
 def argmax(v: torch.Tensor, to_host: bool = True):

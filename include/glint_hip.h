@@ -147,8 +147,17 @@ int gh_accum( void* a, const void* b, uint64_t size, uint64_t batch, gh_dtype dt
 int gh_rmsnorm( void* out, const void* x, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::silu<hidden>   arch/amd64/common/ops.hh:194-210 : hb = DType(x / (1 + exp(-x)) * hb2) */
 int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_dtype dt, gh_stream stream );
-/* x(i) = table(tokens_dev[i]), (vocab, width) rows; a token that is not below vocab leaves its row as it is */
-int gh_embed_rows( void* x, const uint32_t* tokens_dev, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, gh_dtype dt, gh_stream stream );
+/* What a step begins with: x(batch, size) from host memory, its rmsnorm in `normed`, and a table of the step's (table_bytes from table_host to table_dev) with it.
+ * One launch that reads page-locked memory in place (16-byte aligned, multiples of 16 bytes, rows of up to 16 KiB, up to 1.5 MiB), else copies and
+ * gh_rmsnorm.  Without rows (batch 0) the table alone.  The host buffers may be changed again once the stream has been waited for. */
+int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, void* table_dev, const void* table_host, uint64_t table_bytes,
+                gh_dtype dt, gh_stream stream );
+/* What it ends with: `bytes` of x to host memory, there when the call returns; by a kernel where that memory is page-locked */
+int gh_rows_out( void* host, const void* x, uint64_t bytes, gh_stream stream );
+/* x(i) = table(tokens[i]), (vocab, width) rows; a token that is not below vocab leaves its row as it is.  tokens: device or page-locked host memory; a table
+ * of the step's goes along as in gh_rows_in */
+int gh_embed_rows( void* x, const uint32_t* tokens, const void* table, uint64_t width, uint64_t vocab, uint64_t batch, void* table_dev, const void* table_host,
+                   uint64_t table_bytes, gh_dtype dt, gh_stream stream );
 /* Operations::argmax<n>      arch/amd64/common/ops.hh:171-192 : first index of the row maximum.
  * `out_dev` (batch uint32, device memory or page-locked host memory) receives the indices; if `out_host` is non-NULL they are also
  * copied there and the call synchronises (the reference writes a host array: arch/cuda/common/ops.cuh:646-650) */

@@ -124,6 +124,37 @@ def test_embed_rows(dt, batch, width, shift):
 
 
 @pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("batch,width,table,locked,shift", [(1, 8, 0, True, 0), (3, 288, 12, True, 0), (5, 1000, 512, True, 0), (2, 4104, 4112, True, 0), (2, 8192, 16, True, 0),
+                                                            (1, 8200, 16, True, 0), (4, 7, 20, True, 0), (4, 2048, 4096, True, 4), (4, 2048, 48, False, 0), (92, 4096, 4080, True, 0),
+                                                            (200, 4096, 4080, True, 0), (0, 64, 1040, True, 0)])
+def test_rows_in_and_out(dt, batch, width, table, locked, shift):
+    """Rows, their norm and a table from page-locked or pageable memory, and rows back: in place at the edges of a thread's pieces, and copied (rows that are too
+    long, too many, ragged or not aligned).  Rows and tables bit for bit; the norm within a rounding of the result and 64 roundings of its sum in 32 bits."""
+    rng = np.random.default_rng(width + batch)
+    host_memory = (lambda shape, dtype: ops.pinned_empty(shape, dtype)) if locked else np.empty
+    rows = host_memory((max(batch, 1) * width + shift,), ndt(dt))
+    rows[:] = rng.standard_normal(rows.shape).astype(ndt(dt)) * 3
+    host = rows[shift:shift + batch * width].reshape(batch, width)
+    step = host_memory((max(table, 1),), np.uint8)
+    step[:] = rng.integers(0, 256, step.shape)
+    x = torch.full((batch, width), 5.0, dtype=tdt(dt), device="cuda")
+    normed, weight = torch.zeros_like(x), torch.from_numpy(rng.standard_normal(width).astype(ndt(dt))).cuda()
+    step_dev = torch.zeros(table + 16, dtype=torch.uint8, device="cuda")
+    ops.rows_in(x, normed, host, weight, step_dev if table else None, step if table else None)
+    assert np.array_equal(x.cpu().numpy(), host)
+    assert np.array_equal(step_dev.cpu().numpy()[:table], step[:table]) and not step_dev[table:].any()
+    want = torch.from_numpy(np.asarray(host)).double()
+    want = weight.cpu().double() * want / torch.sqrt((want * want).mean(dim=1, keepdim=True) + 1e-5)
+    tol = (2.0 ** (-11 if dt == "f16" else -24) + 64 * 2.0 ** -24) * want.abs() + 2.0 ** -25
+    assert ((normed.cpu().double() - want).abs() <= tol).all()
+    back = host_memory((batch * width + 8,), ndt(dt))
+    back[:] = 7
+    ops.rows_out(back[shift:], normed)
+    assert np.array_equal(back[shift:shift + batch * width].reshape(batch, width), normed.cpu().numpy())
+    assert (back[:shift] == 7).all() and (back[shift + batch * width:] == 7).all()
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("n", [1, 7, 8, 256, 257, 513, 1024, 1025, 1028, 2048, 2049, 2052, 2056, 4096, 4099, 4100, 4104, 8192, 8196, 8200, 16384, 16388, 16392, 32768, 32776, 70001])
 def test_argmax_edges(dt, n):
     """Rows that begin with NaN, hold one, hold nothing but the lowest value or minus infinity; the maximum at either end."""
