@@ -389,7 +389,9 @@ static GateKernel gate_kernel( const void* hb, const GateRows& gate, const void*
 {
   *ns = 0.0;
   const bool plain_silu = gate.activation == GH_ACT_SILU && gate.bias == nullptr;
-  if ( !is_half_type( dt ) || ( !plain_silu && b >= 192 ) ) { // the tiles' epilogue has no room for more than the plain SiLU gate
+  // other gates of many rows: only the tiles have a variant for them, bf16 and over the fp32 sums
+  const bool tiles_only = !plain_silu && b >= 192;
+  if ( !is_half_type( dt ) || ( tiles_only && ( dt != GH_BF16 || !gate.exact ) ) ) {
     return GateKernel::none;
   }
   if ( ( g_force_kernel == 2 || ( g_force_kernel == 0 && gemm_stream_gate_waves() != 0 ) ) && b <= 64 && plain_silu
@@ -402,7 +404,7 @@ static GateKernel gate_kernel( const void* hb, const GateRows& gate, const void*
   const bool rows_of_eight = gate.stride % 8 == 0 && hidden % 8 == 0;
   if ( g_force_kernel != 0 ) {
     return g_force_kernel == 4 && rows_of_eight && tile256_wanted( s, 2 * hidden, b, x, w13, hb ) ? GateKernel::tiles
-           : g_force_kernel == 5 && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride )
+           : g_force_kernel == 5 && !tiles_only && gemm_ring_gate_applicable( s, hidden, b, x, w13, hb, gate.stride )
              ? GateKernel::ring
              : GateKernel::none;
   }
@@ -413,6 +415,11 @@ static GateKernel gate_kernel( const void* hb, const GateRows& gate, const void*
   // splits no K range here: where too few rows fill the chip (2 x 1024 of 2048 k at 8 rows: 11.6 us) the split of the plain product with the
   // gate's kernel behind it (about 4.5 us) is faster (8.2).  A gate over the fp32 sums of many rows takes such a split only: unsplit products of so
   // many rows leave rounded factors.
+  if ( tiles_only ) { // against a product of rounded factors and the gate's kernel, which reads them once more
+    const double tile_ns = gemm_tile256_ns( s, 2 * hidden, b ), two_ns = half_plan( s, 2 * hidden, b, false ).ns + 3000.0 + (double)( 3 * b * hidden ) * 2.0 / 5000.0;
+    *ns = std::min( tile_ns, two_ns );
+    return rows_of_eight && gemm_tile256_takes( s, b, x, w13, hb ) && tile_ns <= two_ns ? GateKernel::tiles : GateKernel::none;
+  }
   const bool keeps_sums = gate.exact && b >= PRODUCT_ROUNDED_ROWS;
   const double ring_ns = gemm_ring_gate_ns( s, hidden, b ) + ring_stores_ns( s, hidden, b );
   double two_ns = 0.0;

@@ -85,17 +85,18 @@ __device__ __forceinline__ bool tile_of_index( const TileOrder& ord, uint32_t xc
 // Or the SiLU gate over two products, w = [w1 rows | w3 rows], as GateRows says (gh_product.h), without a bias: a tile is 128 rows of w1 and the same 128 of
 // w3, whose sums a lane holds side by side; half as many stores, and no kernel that reads both factors
 // again (13B, 16384 tokens: 271 us a layer; the pass of four 36.9 -> 35.5 ms).  With one work-group per CU nothing hides the epilogue, so a
-// gate that takes longer stays a kernel of its own (tanh and biases here, 8192 rows of 2 x 11008: 2 % of the pass slower).
+// gate that takes longer is a variant of its own, bf16: the tanh gate, and biases, kept in LDS since the tile before (8192 rows, 2 x 11008 of
+// 4096 k: 1083 us as a rounded product and a kernel behind it, 984 so; 1024 rows of 2 x 2816 of 1024 k 33.8 and 26.1).
 // Or q, k and v as QkvRows says, 16-byte pieces of a token's heads to its query and its cache row: the two kernels that read the product again, append and
 // rotate took 260 us a layer at 13B and 16384 tokens (3 x 5120 rows of 5120), this epilogue 55 of the product's 1785 (1730 with plain stores).
-constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3, EPI_QKV = 4;
+constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3, EPI_QKV = 4, EPI_BIAS_GATE = 5;
 
 struct TileOut
 {
   void* xout;      // rows [0, r_first), a (b, r_first) matrix
   void* xout2;     // rows from r_first on, as rows 0.. of a (b, r - r_first) matrix; r_first == r: one output
   float* partial;  // EPI_PARTIAL
-  uint32_t r, b, r_first; // EPI_GATE: r rows of each factor
+  uint32_t r, b, r_first; // the gates: r rows of each factor
   GateRows gate;
   QkvRows qkv;
 };
@@ -108,10 +109,11 @@ __device__ __forceinline__ uint32_t w_swizzle( uint32_t row ) { return ( ( row >
 __device__ __forceinline__ void drain_loads_and_stores() { __builtin_amdgcn_s_waitcnt( 0x0F70 ); } // vmcnt(0)
 
 // acc[a][h][i][j][v]: row 128 a + 64 group + 32 (i / 2) + 8 (lane / 16) + 4 (i % 2) + v, token 128 h + 32 wave + 16 j + lane % 16.
-// Returns whether the tile left by exactly 16 (EPI_GATE: 8) stores of this wave behind its last load (not EPI_PARTIAL); else nothing is outstanding, so that
+// Returns whether the tile left by exactly 16 (the gates: 8) stores of this wave behind its last load (not EPI_PARTIAL); else nothing is outstanding, so that
 // also the compiler, which waits before it reads what loads leave in LDS, may count those stores: with one path of fewer stores it has the next
 // tile's second reads wait for nearly all of them (4096 x 1024 at 8192 tokens 61 -> 59 us, 2 x 11008 x 4096 with the gate 1 %).
-// tokens: LDS, EPI_QKV: the cache rows of the tile's 256 tokens, then their positions; those past the last hold the last one's
+// tokens: LDS, EPI_QKV: the cache rows of the tile's 256 tokens, then their positions; those past the last hold the last one's.
+// EPI_BIAS_GATE: the biases (float) of the tile's 128 rows of w1, then those of w3
 template<typename E, int EPI>
 __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2], const TileOut& o, uint32_t tile_row0, uint32_t tile_col0, uint32_t group, uint32_t wave,
                                             uint32_t lane, uint32_t split, const uint32_t* tokens )
@@ -157,24 +159,30 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
     }
     return false;
   }
-  if constexpr ( EPI == EPI_GATE ) { // tile_row0: of the output
-    auto values = [&]( int h, int i, int j ) __attribute__( ( always_inline ) ) {
+  if constexpr ( EPI == EPI_GATE || EPI == EPI_BIAS_GATE ) { // tile_row0: of the output
+    constexpr bool BIAS = EPI == EPI_BIAS_GATE;
+    auto values = [&]( int h, int i, int j, auto act ) __attribute__( ( always_inline ) ) {
       Chunk y;
 #pragma unroll
       for ( int e = 0; e < 8; e++ ) {
         const float a1 = acc[0][h][2 * i + ( e >> 2 )][j][e & 3], a3 = acc[1][h][2 * i + ( e >> 2 )][j][e & 3];
-        const float y1 = o.gate.exact ? a1 : to_f32<E>( from_f32<E>( a1 ) ), y3 = o.gate.exact ? a3 : to_f32<E>( from_f32<E>( a3 ) );
-        y.h[e] = from_f32<E>( y1 / ( 1.0f + __expf( -y1 ) ) * y3 );
+        if constexpr ( BIAS ) {
+          const float* bias = reinterpret_cast<const float*>( tokens ) + 64 * group + 8 * ( lane >> 4 ) + 32 * i + e;
+          y.h[e] = from_f32<E>( activate<E>( a1 + bias[0], act ) * ( a3 + bias[TM2 / 2] ) );
+        } else {
+          const float y1 = o.gate.exact ? a1 : to_f32<E>( from_f32<E>( a1 ) ), y3 = o.gate.exact ? a3 : to_f32<E>( from_f32<E>( a3 ) );
+          y.h[e] = from_f32<E>( y1 / ( 1.0f + __expf( -y1 ) ) * y3 );
+        }
       }
       return y;
     };
     E* base = static_cast<E*>( o.xout ) + (uint64_t)col0 * o.gate.stride + row0;
-    auto store = [&]( auto all ) __attribute__( ( always_inline ) ) {
+    auto store = [&]( auto all, auto act ) __attribute__( ( always_inline ) ) {
 #pragma unroll
-      for ( int n = 0; n < 8; n++ ) {
-        const int h = n >> 2, j = ( n >> 1 ) & 1, i = n & 1;
+      for ( int n = 0; n < 8; n++ ) { // (with biases the four outputs of a row in turn)
+        const int h = BIAS ? ( n >> 1 ) & 1 : n >> 2, j = BIAS ? n & 1 : ( n >> 1 ) & 1, i = BIAS ? n >> 2 : n & 1;
         const uint32_t col = col0 + 128 * h + 16 * j;
-        const Chunk y = values( h, i, j );
+        const Chunk y = values( h, i, j, act );
         if ( all.value
              || ( row0 + 32 * i < o.r && col < o.b && ( o.gate.context_rows == nullptr || o.gate.context_rows[col / o.gate.n_tokens] != nullptr ) ) ) {
           *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * o.gate.stride + 32 * i ) = y.raw; // r % 8 == 0: eight rows
@@ -182,10 +190,14 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
       }
     };
     if ( ( tile_row0 + TM2 / 2 <= o.r ) & ( tile_col0 + TN2 <= o.b ) & ( o.gate.context_rows == nullptr ) ) {
-      store( std::true_type {} );
+      if ( BIAS && o.gate.activation == GH_ACT_GELU_TANH ) {
+        store( std::true_type {}, std::integral_constant<int, GH_ACT_GELU_TANH> {} );
+      } else {
+        store( std::true_type {}, std::integral_constant<int, GH_ACT_SILU> {} );
+      }
       return true;
     }
-    store( std::false_type {} );
+    store( std::false_type {}, o.gate.activation );
     drain_loads_and_stores();
     return false;
   }
@@ -318,7 +330,9 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   __shared__ uint4 s_wa1[128 * 8], s_wb1[128 * 8], s_x1[256 * 8];
   // EPI_QKV: cache rows and positions of a tile's tokens, left here at the end of the tile before: read where they are needed they would be one more round
   // trip a tile with nothing beside it.  Two of them, as a wave may be through with a tile while others still store it.
-  __shared__ uint32_t s_tokens[2][EPI == EPI_QKV ? 3 * TN2 : 1];
+  // EPI_BIAS_GATE: its biases, likewise.
+  __shared__ __align__( 16 ) uint32_t s_tokens[2][EPI == EPI_QKV ? 3 * TN2 : EPI == EPI_BIAS_GATE ? TM2 : 1];
+  constexpr bool GATE = EPI == EPI_GATE || EPI == EPI_BIAS_GATE;
   typedef typename Mfma<E>::x8 x8;
   const uint32_t xcd = blockIdx.x & 7; // work-groups go to the XCDs in turn
   uint32_t idx = blockIdx.x >> 3;
@@ -341,8 +355,8 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
     w_off[i] = ( row + 64 * i ) * ld_bytes + ( slot ^ w_swizzle( row ) ) * 16;
     x_off[i] = ( row + 64 * i ) * ld_bytes + ( slot ^ x_swizzle( row ) ) * 16;
   }
-  constexpr uint32_t ROWS = EPI == EPI_GATE ? TM2 / 2 : TM2; // output rows of a tile
-  const uint64_t w3_bytes = (uint64_t)out.r * ld_bytes;      // EPI_GATE: from a row of w1 to its row of w3
+  constexpr uint32_t ROWS = GATE ? TM2 / 2 : TM2; // output rows of a tile
+  const uint64_t w3_bytes = (uint64_t)out.r * ld_bytes;      // the gates: from a row of w1 to its row of w3
   struct Operands // of a tile: first byte of this split's k range and bytes from there to the end of its last row
   {
     const char *w, *x;
@@ -365,8 +379,8 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   };
   auto fetch_w = [&]( uint4* tile, int half, uint32_t step ) __attribute__( ( always_inline ) ) {
     const Operands& p = WALK && step >= n_steps ? next : cur;
-    const char* base = EPI == EPI_GATE && half == 1 ? p.w + w3_bytes : p.w;
-    const int row = EPI == EPI_GATE ? 0 : 2 * half;
+    const char* base = GATE && half == 1 ? p.w + w3_bytes : p.w;
+    const int row = GATE ? 0 : 2 * half;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<char*>( base ), 0, (int)p.w_bytes, 0x00020000 );
     const uint32_t kb = k_bytes( step );
     __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + 64 * all_waves ), 16, w_off[row], kb, 0, 0 );
@@ -427,7 +441,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   };
   // The end of a memory part: this wave's reads are here, and all of its loads but the youngest 8, which leaves what the next part reads
   // in LDS (the barrier makes that all waves').  `stores`: the last tile's stores are still counted behind the loads this waits for.
-  constexpr int STORES = EPI == EPI_GATE ? 8 : 16;
+  constexpr int STORES = GATE ? 8 : 16;
   auto arrive = [&]( bool stores ) __attribute__( ( always_inline ) ) {
     __builtin_amdgcn_sched_barrier( 0 );
     if ( stores ) {
@@ -461,13 +475,20 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
   {
     uint64_t row;
     uint32_t pos;
+    float bias;
   };
-  auto token_of = [&]( uint32_t tt ) __attribute__( ( always_inline ) ) {
-    Token token { 0, 0 };
+  auto token_of = [&]( uint32_t rt, uint32_t tt ) __attribute__( ( always_inline ) ) {
+    Token token { 0, 0, 0.0f };
     if constexpr ( EPI == EPI_QKV ) {
       const uint32_t col = min( tt * TN2 + ( threadIdx.x & ( TN2 - 1 ) ), out.b - 1 );
       token.row = reinterpret_cast<const uint64_t*>( out.qkv.token_rows )[col];
       token.pos = out.qkv.pos[col];
+    }
+    if constexpr ( EPI == EPI_BIAS_GATE ) { // (without biases any value that can be read)
+      const uint32_t row = min( rt * ROWS + ( threadIdx.x & ( ROWS - 1 ) ), out.r - 1 );
+      const E* bias = out.gate.bias != nullptr ? static_cast<const E*>( out.gate.bias ) : w;
+      const float value = to_f32<E>( bias[( threadIdx.x & ROWS ) != 0 ? (uint64_t)out.r + row : row] );
+      token.bias = out.gate.bias != nullptr ? value : 0.0f;
     }
     return token;
   };
@@ -476,8 +497,11 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
       reinterpret_cast<uint64_t*>( tokens )[threadIdx.x & ( TN2 - 1 )] = token.row;
       tokens[2 * TN2 + ( threadIdx.x & ( TN2 - 1 ) )] = token.pos;
     }
+    if constexpr ( EPI == EPI_BIAS_GATE ) {
+      reinterpret_cast<float*>( tokens )[threadIdx.x & ( TM2 - 1 )] = token.bias;
+    }
   };
-  keep_token( s_tokens[0], token_of( token_tile ) );
+  keep_token( s_tokens[0], token_of( row_tile, token_tile ) );
   fetch_w( s_wa0, 0, 0 );
   fetch_x( s_x0, 0, 0 );
   fetch_x( s_x0, 1, 0 );
@@ -518,7 +542,7 @@ __global__ __launch_bounds__( T256_THREADS, 1 ) void gemm_tile256_kernel( const 
       if ( !more ) {
         __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): no load-to-LDS outlives the work-group
       }
-      const Token token = token_of( more ? next_token : token_tile );
+      const Token token = token_of( more ? next_row : row_tile, more ? next_token : token_tile );
       stores = store_tile<E, EPI>( acc, out, row_tile * ROWS, token_tile * TN2, group, wave, lane, 0, s_tokens[tile & 1] );
       keep_token( s_tokens[( tile + 1 ) & 1], token );
       if ( !more ) {
@@ -660,11 +684,13 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
   if ( splits == 1 ) {
     k_len = (uint32_t)s;
   }
-  const int epi = partial != nullptr ? EPI_PARTIAL : epilogue;
-  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL || ( epi == EPI_QKV && qkv != nullptr && gemm_tile256_qkv_fits( *qkv ) ) || ( epi == EPI_GATE && gate != nullptr && gate->activation == GH_ACT_SILU && gate->bias == nullptr && r % 8 == 0 && gate->stride % 8 == 0 ),
+  const bool plain_gate = gate != nullptr && gate->activation == GH_ACT_SILU && gate->bias == nullptr;
+  const int epi = partial != nullptr ? EPI_PARTIAL : epilogue == EPI_GATE && !plain_gate ? EPI_BIAS_GATE : epilogue;
+  GH_REQUIRE( epi == EPI_STORE || epi == EPI_ACCUM || epi == EPI_PARTIAL || ( epi == EPI_QKV && qkv != nullptr && gemm_tile256_qkv_fits( *qkv ) )
+                || ( ( epi == EPI_GATE || ( epi == EPI_BIAS_GATE && gate != nullptr && gate->exact && std::is_same_v<E, __bf16> ) ) && r % 8 == 0 && gate->stride % 8 == 0 ),
               "gh_matmul: unknown tile epilogue %d", epi );
   GH_REQUIRE( epi != EPI_ACCUM || r % 8 == 0, "gh_matmul: the accumulating tile epilogue needs r %% 8 == 0" );
-  const uint64_t tile_rows = epi == EPI_GATE ? TM2 / 2 : TM2;
+  const uint64_t tile_rows = epi == EPI_GATE || epi == EPI_BIAS_GATE ? TM2 / 2 : TM2;
   const uint32_t row_tiles = (uint32_t)( ( r + tile_rows - 1 ) / tile_rows );
   TileOrder ord;
   ord.token_tiles = (uint32_t)( ( b + TN2 - 1 ) / TN2 );
@@ -692,6 +718,11 @@ int gemm_tile256_launch( E* xout, float* partial, const E* x, const E* w, uint64
     case EPI_STORE: walk ? GH_TILE256( EPI_STORE, true ) : GH_TILE256( EPI_STORE, false ); break;
     case EPI_ACCUM: walk ? GH_TILE256( EPI_ACCUM, true ) : GH_TILE256( EPI_ACCUM, false ); break;
     case EPI_GATE: walk ? GH_TILE256( EPI_GATE, true ) : GH_TILE256( EPI_GATE, false ); break;
+    case EPI_BIAS_GATE:
+      if constexpr ( std::is_same_v<E, __bf16> ) {
+        walk ? GH_TILE256( EPI_BIAS_GATE, true ) : GH_TILE256( EPI_BIAS_GATE, false );
+      }
+      break;
     case EPI_QKV:
       if constexpr ( std::is_same_v<E, __half> ) {
         walk ? GH_TILE256( EPI_QKV, true ) : GH_TILE256( EPI_QKV, false );

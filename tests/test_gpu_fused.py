@@ -271,6 +271,34 @@ def test_matmul_gate_in_epilogue(b, s, hidden, bias, activation):
     assert ((got - act * u).abs() <= bound).all()
 
 
+# tiles that walk over row tiles and token tiles, whole and ragged; a work-group each; an odd number of steps
+@pytest.mark.parametrize("activation", [ops.GH_ACT_SILU, ops.GH_ACT_GELU_TANH])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("b,s,hidden", [(4096, 256, 8192), (4100, 256, 8200), (2304, 640, 8192), (2300, 576, 8200), (512, 128, 16384)])
+def test_matmul_gate_of_whole_tiles(b, s, hidden, bias, activation):
+    """The gate with tanh or biases in the tiles' epilogue, against 64 bits: on the fp32 sums, one rounding to bf16, off by 2^-8 of the result, and 1e-4 for the
+    sums and the fast exponential.  Each bias once in a thousand is far off the rest, so that a wrong row's would show."""
+    if activation == ops.GH_ACT_SILU and not bias:
+        pytest.skip("the plain gate")
+    g = torch.Generator(device="cuda").manual_seed(b + hidden)
+    x = torch.randn((b, s), generator=g, device="cuda").bfloat16()
+    w = (torch.randn((2 * hidden, s), generator=g, device="cuda") / s ** 0.5).bfloat16()
+    add = torch.randn(2 * hidden, generator=g, device="cuda") if bias else None
+    if bias:
+        add[::997] += 20.0
+        add = add.bfloat16()
+    lib = _lib.lib()
+    _lib.check(lib.gh_gemm_set_tuning(4, 0, 0))
+    try:
+        got = ops.matmul_gate(x, w, add, activation).double()
+    finally:
+        _lib.check(lib.gh_gemm_set_tuning(0, 0, 0))
+    y = x.double() @ w.double().t() + (add.double() if bias else 0.0)
+    a, u = y[:, :hidden], y[:, hidden:]
+    want = (a * torch.sigmoid(a) if activation == ops.GH_ACT_SILU else torch.nn.functional.gelu(a, approximate="tanh")) * u
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * (1.0 + want.abs().sqrt())).all()
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [Shape(dim=32, n_layers=1, n_heads=4, n_kv_heads=2, hidden_dim=48, seq_len=16),
                                    Shape(dim=288, n_layers=1, n_heads=6, n_kv_heads=6, hidden_dim=768, seq_len=256),
