@@ -145,9 +145,8 @@ __global__ __launch_bounds__( EW_THREADS ) void rmsnorm_kernel( T* __restrict__ 
 // ---- rows that arrive in page-locked host memory -------------------------------------------------
 // The first kernel of a step reads them where the host left them: they go to the device and, normed, to the first product, and the step's tables come along
 // in work-groups of their own.  As copies in front of rmsnorm_kernel each is a launch and a hand-over between engines more.  Bound by the bus.
-// The copy engine is the faster way over it for 2 MB and more: beyond 1.5 MiB the rows are copied (f16 with norm, tables and a wait, copied and in place:
+// The copy engine is the faster way over it for 2 MB and more: beyond GH_ROWS_IN_BYTES the rows are copied (f16 with norm, tables and a wait, copied and in place:
 // 32 rows of 4096 28.1 and 19.6 us, 64 of 8192 43.4 and 36.8, 128 61.7 and 61.9, 256 99 and 109).
-constexpr uint64_t ROWS_IN_BYTES = 3ull << 19;
 // The sums as rmsnorm_kernel takes them, from registers: a second pass would cross the bus again.  16-byte pieces; PIECES: a thread's.
 template<typename T, int PIECES>
 __global__ __launch_bounds__( EW_THREADS ) void rows_in_kernel( T* __restrict__ x,
@@ -528,7 +527,7 @@ int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uin
     table_bytes = 0;
   }
   const uint64_t table_groups = ( table_bytes / 16 + EW_THREADS - 1 ) / EW_THREADS;
-  const bool in_place = batch > 0 && batch * bytes <= ROWS_IN_BYTES && bytes % 16 == 0 && pieces <= 4 && aligned16( x ) && aligned16( normed ) && aligned16( host )
+  const bool in_place = batch > 0 && batch * bytes <= GH_ROWS_IN_BYTES && bytes % 16 == 0 && pieces <= 4 && aligned16( x ) && aligned16( normed ) && aligned16( host )
                         && aligned16( weight ) && page_locked( host );
   const uint64_t rows = in_place ? batch : 0;
   if ( rows + table_groups > 0 ) {

@@ -206,38 +206,39 @@ public:
     for ( size_t l = first; l < Config::n_layers && settings_.hosts( l, InferenceStage::PreAttention ); l++ ) {
       run.push_back( l );
     }
+    const bool fused_layers = options_.fused_attention && options_.fused_projections, embed = first == 0;
+    // the norms of a layer in the launches of the products behind them, or at the end of those in front of them
+    const bool norms_ride = fused_layers && LlamaOperations::norm_rides( Config::dim + 2 * Config::kv_dim, batch_ )
+                            && LlamaOperations::norm_rides( 2 * Config::hidden_dim, batch_ );
+    // The first attention norm comes with the activations, or stands alone; every later one rides on the epilogue of the previous w2.  Activations that are
+    // copied go first: the copy runs beside the host's work on the tables.
+    const uint64_t rows_bytes = batch_ * Config::dim * sizeof( DType );
+    const bool in_place = !embed && fused_layers && !norms_ride && !run.empty() && states.activations().len() == rows_bytes && rows_bytes <= GH_ROWS_IN_BYTES;
+    if ( !embed && !in_place ) {
+      ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
+    } else if ( !options_.fused_attention ) {
+      load_embedding( states );
+    }
     for ( size_t l : run ) {
       for ( size_t i = 0; i < contexts.size(); i++ ) {
         GLINT_CHECK( contexts[i]->prepare( l, states.token_pos( i ), false ) );
       }
     }
-    const bool fused_layers = options_.fused_attention && options_.fused_projections, embed = first == 0;
-    // the norms of a layer in the launches of the products behind them, or at the end of those in front of them
-    const bool norms_ride = fused_layers && LlamaOperations::norm_rides( Config::dim + 2 * Config::kv_dim, batch_ )
-                            && LlamaOperations::norm_rides( 2 * Config::hidden_dim, batch_ );
-    // the first attention norm comes with the activations, or stands alone; every later one rides on the epilogue of the previous w2
-    bool normed = !fused_layers || run.empty() || norms_ride;
     if ( options_.fused_attention ) {
       const size_t table_bytes = fill_tables( contexts, run, true, embed ? &states : nullptr );
       if ( embed ) {
         ops_.template embed_rows<Config::dim, Config::vocab_size>( x_, tokens_host(), base_.token_embedding_table, batch_, tables_dev_.get(), tables_host_, table_bytes );
-      } else if ( !normed && states.activations().len() == batch_ * Config::dim * sizeof( DType ) ) {
+      } else if ( in_place ) {
         ops_.template rows_in<Config::dim>( x_, xb_, reinterpret_cast<const DType*>( states.activations().data() ), layers_[run[0]].rms_att_weight, batch_,
                                             tables_dev_.get(), tables_host_, table_bytes );
-        normed = true;
       } else {
-        ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
         send_tables( table_bytes );
       }
       balance_step();
-    } else if ( embed ) {
-      load_embedding( states );
-    } else {
-      ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
     }
 
     spans_.mark( 0, ops_.stream() ); // the activations and the tables are there: from here to the copy back it is kernels only
-    if ( !normed ) {
+    if ( fused_layers && !run.empty() && !norms_ride && !in_place ) {
       ops_.template rmsnorm<Config::dim>( xb_, x_, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, batch_ );
     }
     for ( size_t k = 0; k < run.size(); k++ ) {

@@ -147,8 +147,9 @@ int gh_accum( void* a, const void* b, uint64_t size, uint64_t batch, gh_dtype dt
 int gh_rmsnorm( void* out, const void* x, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt, gh_stream stream );
 /* Operations::silu<hidden>   arch/amd64/common/ops.hh:194-210 : hb = DType(x / (1 + exp(-x)) * hb2) */
 int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_dtype dt, gh_stream stream );
+#define GH_ROWS_IN_BYTES ( 3u << 19 ) /* of rows, up to which gh_rows_in reads them in place */
 /* What a step begins with: x(batch, size) from host memory, its rmsnorm in `normed`, and a table of the step's (table_bytes from table_host to table_dev) with it.
- * One launch that reads page-locked memory in place (16-byte aligned, multiples of 16 bytes, rows of up to 16 KiB, up to 1.5 MiB), else copies and
+ * One launch that reads page-locked memory in place (16-byte aligned, multiples of 16 bytes, rows of up to 16 KiB, GH_ROWS_IN_BYTES in all), else copies and
  * gh_rmsnorm.  Without rows (batch 0) the table alone.  The host buffers may be changed again once the stream has been waited for. */
 int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, void* table_dev, const void* table_host, uint64_t table_bytes,
                 gh_dtype dt, gh_stream stream );
