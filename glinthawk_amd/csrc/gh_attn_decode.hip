@@ -863,12 +863,13 @@ __device__ __forceinline__ void mfma_stream_range( const __half* __restrict__ q,
     }
     mt = fmaxf( mt, __shfl_xor( mt, 16, WAVE ) );
     mt = fmaxf( mt, __shfl_xor( mt, 32, WAVE ) );
-    const float m_new = fmaxf( m, mt ); // finite: the first token of every tile is inside the range
-    const float alpha = fast_exp2( m - m_new );
+    const float m_new = fmaxf( m, mt );
+    const float m_safe = m_new == -INFINITY ? 0.0f : m_new; // a head that has seen scores of -inf only, which weigh nothing
+    const float alpha = fast_exp2( m - m_safe );
     float p[4];
 #pragma unroll
     for ( int i = 0; i < 4; i++ ) {
-      p[i] = fast_exp2( s[i] - m_new );
+      p[i] = fast_exp2( s[i] - m_safe );
     }
     l = l * alpha + ( p[0] + p[1] ) + ( p[2] + p[3] );
     m = m_new;

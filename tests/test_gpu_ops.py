@@ -941,6 +941,55 @@ def test_fused_generic_scores_of_minus_infinity(dt, chunk, heads, kv_heads, head
         assert ((out[i].view(heads, head_size).double() - want).abs() <= bound).all(), i
 
 
+# the fp16 kernels walk tiles of 16 keys from a tile that differs from split to split: every other tile of -inf (either half of them) is each split's first one
+# in one context or the other; a whole split; all keys but one; the keys that are the second tile of the short plan's second split
+@pytest.mark.parametrize("variant", [GH_ATTN_VALU, GH_ATTN_MFMA])
+@pytest.mark.parametrize("route,chunk", [("short", 0), ("joined", 80), ("merged", 32), ("whole", 304), ("balanced", 0)])
+@pytest.mark.parametrize("kv_heads,gqa", [(2, 4), (1, 8)])
+def test_fused_fp16_scores_of_minus_infinity(variant, route, chunk, kv_heads, gqa):
+    """Such keys weigh nothing wherever they stand, whether a split holds others or not."""
+    if route == "balanced" and variant == GH_ATTN_VALU:
+        pytest.skip("the balanced kernel has one walk per head count")
+    keys, heads = 300, kv_heads * gqa
+    gone = [[t for t in range(keys) if t // 16 % 2 == 0], [t for t in range(keys) if t // 16 % 2 == 1], range(64, 160), [t for t in range(keys) if t != 77], range(80, 96)]
+    n = len(gone)
+    g = torch.Generator(device="cuda").manual_seed(gqa)
+    cache = torch.randn((n, keys, 2, kv_heads, 128), generator=g, device="cuda").half()
+    q = torch.randn((n, heads, 128), generator=g, device="cuda").half()
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    for i, which in enumerate(gone):
+        cache[i, list(which), 0, :, 0] = -torch.inf
+    shape = Shape(dim=heads * 128, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, hidden_dim=64, seq_len=keys)
+    rows, pos = ops.row_table([cache[i].data_ptr() for i in range(n)]), torch.full((n,), keys - 1, dtype=torch.int32, device="cuda")
+    out = torch.zeros((n, heads * 128), dtype=torch.float16, device="cuda")
+    ops.attn_set_chunk(chunk)
+    ops.attn_set_split_join(0 if route == "merged" else 1)
+    try:
+        if route == "balanced":
+            ws = torch.empty(ops.attn_balanced_workspace(n, shape), dtype=torch.uint8, device="cuda")
+            ops.attn_balance(rows, pos, keys - 1, shape, ws)
+            ops.attn_decode_balanced(q.flatten(1), rows, out, keys - 1, shape, ws)
+        else:
+            c_shape, per_split, splits = shape.c(), C.c_uint32(0), C.c_uint32(0)
+            _lib.check(_lib.lib().gh_attn_decode_plan(n, keys - 1, C.byref(c_shape), _lib.GH_F16, variant, C.byref(per_split), C.byref(splits), None))
+            joined = ops.attn_decode_join_waves(n, keys - 1, shape, variant=variant)
+            assert (splits.value, joined) == {"short": (5, 0), "joined": (4, 8), "merged": (10, 0), "whole": (1, 0)}[route]
+            ops.attn_decode(q.flatten(1), rows, pos, out, keys - 1, shape, variant=variant)
+    finally:
+        ops.attn_set_chunk(0)
+        ops.attn_set_split_join(1)
+    for i in range(n):
+        k, v = (cache[i, :, part].double().repeat_interleave(gqa, 1) for part in (0, 1))
+        p = ((q[i].double() * k).sum(-1) * 128 ** -0.5).softmax(0)[:, :, None]
+        want = (p * v).sum(0)
+        # fp32 sums of 300 terms of about 1 and the stored value's own rounding; the MFMA kernel multiplies weights of fp16: their rounding, or half the
+        # smallest step of a subnormal one
+        bound = 2e-5 + 2.0 ** -11 * want.abs()
+        if variant == GH_ATTN_MFMA:
+            bound += 2.0 ** -11 * (p * v.abs()).sum(0) + 2.0 ** -25 * v.abs().sum(0)
+        assert ((out[i].view(heads, 128).double() - want).abs() <= bound).all(), i
+
+
 @pytest.mark.parametrize("shape", [MHA128, MHA128_ODD, GQA2, GQA4, GQA8], ids=["mha", "mha6", "gqa2", "gqa4", "gqa8"])
 @pytest.mark.parametrize("chunk", [0, 16, 80, 256])
 def test_fused_valu(shape, chunk):
