@@ -1680,14 +1680,19 @@ uint64_t gh_attn_decode_workspace( uint64_t batch, uint32_t max_pos, const gh_sh
   if ( shape == nullptr || batch == 0 ) {
     return 0;
   }
-  // A smaller batch gets more splits per context, and batch * splits does not grow with the batch:
-  // the buffer has to hold the largest need of any batch in [1, batch].  The generic kernel splits
-  // per query head and may use more splits than the fast ones; size for the larger of the two.
+  // A smaller batch gets more splits per context, and batch * splits does not grow with the batch: the buffer has to hold the largest need of any
+  // batch in [1, batch].  The kernels cut differently (the generic one per query head, the other two for different numbers of waves) and a caller may
+  // ask for any that takes the shape, so it is sized for the largest of them, whatever GH_ATTN_AUTO stands for at the moment.
   uint64_t floats = 0;
   for ( uint64_t b = 1; b <= batch; b++ ) {
-    const Plan fast = make_plan( b, max_pos, shape, GH_F16, GH_ATTN_AUTO );
-    const Plan generic = make_plan( b, max_pos, shape, GH_F32, GH_ATTN_GENERIC );
-    floats = std::max( floats, partial_floats( b, shape, std::max( fast.split_bound, generic.split_bound ) ) );
+    uint32_t splits = make_plan( b, max_pos, shape, GH_F32, GH_ATTN_GENERIC ).split_bound;
+    if ( fast_ok( shape, GH_F16 ) && valu_gqa_ok( shape->gqa_size ) ) {
+      splits = std::max( splits, make_plan( b, max_pos, shape, GH_F16, GH_ATTN_VALU ).split_bound );
+    }
+    if ( fast_ok( shape, GH_F16 ) && mfma_gqa_ok( shape->gqa_size ) ) {
+      splits = std::max( splits, make_plan( b, max_pos, shape, GH_F16, GH_ATTN_MFMA ).split_bound );
+    }
+    floats = std::max( floats, partial_floats( b, shape, splits ) );
   }
   return floats * sizeof( float ) + 256;
 }

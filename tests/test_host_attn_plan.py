@@ -6,14 +6,23 @@ import ctypes as C
 import pytest
 
 from glinthawk_amd import _lib
-from glinthawk_amd._lib import GH_ATTN_AUTO, GH_ATTN_GENERIC, Shape
+from glinthawk_amd._lib import GH_ATTN_AUTO, GH_ATTN_GENERIC, GH_ATTN_MFMA, GH_ATTN_VALU, Shape
 
 SHAPES = {
     "7B": Shape(dim=4096, n_layers=1, n_heads=32, n_kv_heads=32, hidden_dim=11008, seq_len=2048),
     "13B": Shape(dim=5120, n_layers=1, n_heads=40, n_kv_heads=40, hidden_dim=13824, seq_len=4096),
     "70B": Shape(dim=8192, n_layers=1, n_heads=64, n_kv_heads=8, hidden_dim=28672, seq_len=4096),
     "tiny": Shape(dim=288, n_layers=1, n_heads=6, n_kv_heads=6, hidden_dim=768, seq_len=256),
+    "gqa2": Shape(dim=1024, n_layers=1, n_heads=8, n_kv_heads=4, hidden_dim=64, seq_len=4096),
+    "gqa4": Shape(dim=4096, n_layers=1, n_heads=32, n_kv_heads=8, hidden_dim=64, seq_len=4096),
+    "gqa16": Shape(dim=4096, n_layers=1, n_heads=32, n_kv_heads=2, hidden_dim=64, seq_len=4096),
 }
+
+
+def variants(shape):
+    """(type, kernel) of every call that gh_attn_decode takes for this shape."""
+    gqa, fast = shape.n_heads // shape.n_kv_heads, shape.dim // shape.n_heads == 128
+    return [(0, GH_ATTN_AUTO), (0, GH_ATTN_GENERIC), (1, GH_ATTN_AUTO)] + [(0, GH_ATTN_VALU)] * (fast and gqa <= 8) + [(0, GH_ATTN_MFMA)] * (fast and gqa >= 2)
 
 
 def plan(batch, max_pos, shape, dt, variant):
@@ -29,18 +38,42 @@ def workspace(batch, max_pos, shape):
 
 
 @pytest.mark.parametrize("name", sorted(SHAPES))
-@pytest.mark.parametrize("cap", [1, 8, 32, 64, 128, 256])
+@pytest.mark.parametrize("cap", [1, 2, 3, 8, 32, 64, 128, 256])
 def test_workspace_of_the_limit_serves_every_smaller_batch(name, cap):
     shape = SHAPES[name]
     have = workspace(cap, shape.seq_len - 1, shape)
     positions = sorted({0, 1, 15, 16, 255, 256, 257, 511, 1000, shape.seq_len // 2, shape.seq_len - 2, shape.seq_len - 1} & set(range(shape.seq_len)))
     for batch in range(1, cap + 1):
         for max_pos in positions:
-            for dt, variant in ((0, GH_ATTN_AUTO), (0, GH_ATTN_GENERIC), (1, GH_ATTN_AUTO)):
+            for dt, variant in variants(shape):
                 chunk, splits, need = plan(batch, max_pos, shape, dt, variant)
                 assert need <= have, (name, cap, batch, max_pos, dt, variant, need, have)
                 assert chunk % 16 == 0 and splits >= 1
                 assert (splits - 1) * chunk < max_pos + 1 <= splits * chunk          # every key in exactly one split
+
+
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_workspace_of_a_call_serves_it_with_any_kernel(name):
+    shape = SHAPES[name]
+    for batch in list(range(1, 18)) + [24, 31, 32, 48, 49, 64, 65]:
+        for keys in list(range(1, shape.seq_len, 97)) + [shape.seq_len]:
+            have = workspace(batch, keys - 1, shape)
+            for dt, variant in variants(shape):
+                assert plan(batch, keys - 1, shape, dt, variant)[2] <= have, (name, batch, keys, dt, variant)
+
+
+def test_workspace_does_not_hang_on_the_kernel_that_auto_stands_for():
+    L, shape = _lib.lib(), SHAPES["70B"]
+    have = workspace(8, shape.seq_len - 1, shape)
+    for variant in (GH_ATTN_VALU, GH_ATTN_MFMA, GH_ATTN_GENERIC):
+        _lib.check(L.gh_attn_set_auto_variant(variant))
+        try:
+            assert workspace(8, shape.seq_len - 1, shape) == have
+            for batch in range(1, 9):
+                for keys in range(256, shape.seq_len + 1, 256):
+                    assert plan(batch, keys - 1, shape, 0, GH_ATTN_AUTO)[2] <= have
+        finally:
+            _lib.check(L.gh_attn_set_auto_variant(GH_ATTN_AUTO))
 
 
 def test_the_case_that_used_to_overflow():
