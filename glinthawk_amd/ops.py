@@ -93,6 +93,11 @@ def rows_in(x: torch.Tensor, normed: torch.Tensor, host, weight: torch.Tensor, t
           "gh_rows_in")
 
 
+def host_in_place(host: int, dev: int, nbytes: int) -> bool:
+    """Addresses of host and device memory."""
+    return lib().gh_host_in_place(host, dev, nbytes) == 1
+
+
 def rows_out(host, x: torch.Tensor) -> None:
     check(lib().gh_rows_out(host.ctypes.data, _p(x), x.numel() * x.element_size(), _stream()), "gh_rows_out")
 

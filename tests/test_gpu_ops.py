@@ -123,6 +123,27 @@ def test_embed_rows(dt, batch, width, shift):
     assert torch.equal(x, want)
 
 
+@pytest.mark.parametrize("source", ["library", "torch"])
+def test_host_memory_in_place(source):
+    """Kernels read host memory where it is only if every byte they are to read lies in one page-locked allocation.  A question only: nothing is launched."""
+    size = 1 << 20
+    if source == "library":
+        keep = ops.pinned_empty((size,), np.uint8)
+        at = keep.ctypes.data
+    else:       # torch rounds its blocks up to powers of two
+        keep = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+        at = keep.data_ptr()
+    dev = torch.empty(size, dtype=torch.uint8, device="cuda").data_ptr()
+    for first, n in ((0, 16), (0, size), (16, size - 16), (size - 16, 16), (4096, 65536), (size // 2, size // 2)):
+        assert ops.host_in_place(at + first, dev, n)
+    for first, n in ((0, size + 16), (16, size), (size - 16, 32), (size // 2, 16 * size), (0, 1 << 40)):
+        assert not ops.host_in_place(at + first, dev, n)
+    assert not ops.host_in_place(at + 4, dev, 16) and not ops.host_in_place(at, dev + 8, 16) and not ops.host_in_place(at, dev, 24)
+    pageable = np.empty(4096 + 16, np.uint8)
+    assert not ops.host_in_place((pageable.ctypes.data + 15) // 16 * 16, dev, 4096)
+    assert not ops.host_in_place(dev, dev, 16)      # device memory is no host memory
+
+
 @pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("batch,width,table,locked,shift", [(1, 8, 0, True, 0), (3, 288, 12, True, 0), (5, 1000, 512, True, 0), (2, 4104, 4112, True, 0), (2, 8192, 16, True, 0),
                                                             (1, 8200, 16, True, 0), (4, 7, 20, True, 0), (4, 2048, 4096, True, 4), (4, 2048, 48, False, 0), (92, 4096, 4080, True, 0),
