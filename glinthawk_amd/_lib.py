@@ -116,6 +116,7 @@ SIGNATURES = {
     "gh_rmsnorm": (_i, [_vp, _vp, _vp, _u64, _u64, _i, _vp]),
     "gh_silu": (_i, [_vp, _vp, _u64, _u64, _i, _vp]),
     "gh_rows_in": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _vp, _vp, _u64, _i, _vp]),
+    "gh_rows_in_place": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _i]),
     "gh_host_in_place": (_i, [_vp, _vp, _u64]),
     "gh_rows_out": (_i, [_vp, _vp, _u64, _vp]),
     "gh_embed_rows": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _vp, _vp, _u64, _i, _vp]),

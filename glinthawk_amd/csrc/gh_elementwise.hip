@@ -439,6 +439,13 @@ bool pieces_in_place( const void* host, const void* dev, uint64_t bytes )
 {
   return bytes % 16 == 0 && aligned16( host ) && aligned16( dev ) && page_locked( host, bytes );
 }
+// the rows of gh_rows_in: at most four pieces a thread
+bool rows_in_place( const void* x, const void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt )
+{
+  const uint64_t bytes = size * dtype_size( dt );
+  return bytes % 16 == 0 && bytes <= 4 * 16 * EW_THREADS && batch * bytes <= GH_ROWS_IN_BYTES && aligned16( normed ) && aligned16( weight )
+         && pieces_in_place( host, x, batch * bytes );
+}
 
 } // namespace
 } // namespace gh
@@ -543,8 +550,7 @@ int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uin
     table_bytes = 0;
   }
   const uint64_t table_groups = ( table_bytes / 16 + EW_THREADS - 1 ) / EW_THREADS;
-  const bool in_place = batch > 0 && batch * bytes <= GH_ROWS_IN_BYTES && bytes % 16 == 0 && pieces <= 4 && aligned16( normed ) && aligned16( weight )
-                        && pieces_in_place( host, x, batch * bytes );
+  const bool in_place = batch > 0 && rows_in_place( x, normed, host, weight, size, batch, dt );
   const uint64_t rows = in_place ? batch : 0;
   if ( rows + table_groups > 0 ) {
     auto launch = [&]( auto* e, auto count ) {
@@ -562,6 +568,14 @@ int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uin
   }
   GH_HIP( hipMemcpyAsync( x, host, batch * bytes, hipMemcpyHostToDevice, as_stream( stream ) ) );
   return gh_rmsnorm( normed, x, weight, size, batch, dt, stream );
+}
+
+int gh_rows_in_place( const void* x, const void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt )
+{
+  if ( ensure_init() != GH_OK || host == nullptr || size == 0 || size > 0xffffffffull || batch == 0 || batch > 0x7fffffffull || ( dt != GH_F16 && dt != GH_F32 ) ) {
+    return 0;
+  }
+  return rows_in_place( x, normed, host, weight, size, batch, dt ) ? 1 : 0;
 }
 
 int gh_host_in_place( const void* host, const void* dev, uint64_t bytes )

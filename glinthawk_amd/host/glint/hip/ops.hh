@@ -148,6 +148,12 @@ public:
   {
     GLINT_GH( gh_rows_in( x, normed, host, weight, size, batch_size, table_dev, table_host, table_bytes, gh_type<DType>(), stream_ ) );
   }
+  // whether rows_in reads these rows where they are
+  template<uint64_t size>
+  bool rows_in_place( const DType* x, const DType* normed, const DType* host, const DType* weight, const uint64_t batch_size ) const
+  {
+    return gh_rows_in_place( x, normed, host, weight, size, batch_size, gh_type<DType>() ) == 1;
+  }
   template<uint64_t width, uint64_t vocab>
   void embed_rows( DType* x, const uint32_t* tokens, const DType* table, const uint64_t batch_size, void* table_dev, const void* table_host, const uint64_t table_bytes ) const
   {

@@ -212,10 +212,11 @@ public:
                             && LlamaOperations::norm_rides( 2 * Config::hidden_dim, batch_ );
     // The first attention norm comes with the activations, or stands alone; every later one rides on the epilogue of the previous w2.  Activations that are
     // copied go first: the copy runs beside the host's work on the tables.
-    const uint64_t rows_bytes = batch_ * Config::dim * sizeof( DType );
-    const bool in_place = !embed && fused_layers && !norms_ride && !run.empty() && states.activations().len() == rows_bytes && rows_bytes <= GH_ROWS_IN_BYTES;
+    const DType* const acts = reinterpret_cast<const DType*>( states.activations().data() );
+    const bool in_place = !embed && fused_layers && !norms_ride && !run.empty() && states.activations().len() == batch_ * Config::dim * sizeof( DType )
+                          && ops_.template rows_in_place<Config::dim>( x_, xb_, acts, layers_[run[0]].rms_att_weight, batch_ );
     if ( !embed && !in_place ) {
-      ops_.copy( x_, reinterpret_cast<const DType*>( states.activations().data() ), states.activations().len(), CopyType::HostToDevice, true );
+      ops_.copy( x_, acts, states.activations().len(), CopyType::HostToDevice, true );
     } else if ( !options_.fused_attention ) {
       load_embedding( states );
     }
@@ -229,8 +230,7 @@ public:
       if ( embed ) {
         ops_.template embed_rows<Config::dim, Config::vocab_size>( x_, tokens_host(), base_.token_embedding_table, batch_, tables_dev_.get(), tables_host_, table_bytes );
       } else if ( in_place ) {
-        ops_.template rows_in<Config::dim>( x_, xb_, reinterpret_cast<const DType*>( states.activations().data() ), layers_[run[0]].rms_att_weight, batch_,
-                                            tables_dev_.get(), tables_host_, table_bytes );
+        ops_.template rows_in<Config::dim>( x_, xb_, acts, layers_[run[0]].rms_att_weight, batch_, tables_dev_.get(), tables_host_, table_bytes );
       } else {
         send_tables( table_bytes );
       }

@@ -93,6 +93,11 @@ def rows_in(x: torch.Tensor, normed: torch.Tensor, host, weight: torch.Tensor, t
           "gh_rows_in")
 
 
+def rows_in_place(x: torch.Tensor, normed: torch.Tensor, host, weight: torch.Tensor) -> bool:
+    batch, size = x.shape
+    return lib().gh_rows_in_place(_p(x), _p(normed), host.ctypes.data, _p(weight), size, batch, _dt(x)) == 1
+
+
 def host_in_place(host: int, dev: int, nbytes: int) -> bool:
     """Addresses of host and device memory."""
     return lib().gh_host_in_place(host, dev, nbytes) == 1

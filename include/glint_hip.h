@@ -153,6 +153,8 @@ int gh_silu( void* hb, const void* hb2, uint64_t hidden_dim, uint64_t batch, gh_
  * gh_rmsnorm.  Without rows (batch 0) the table alone.  The host buffers may be changed again once the stream has been waited for. */
 int gh_rows_in( void* x, void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, void* table_dev, const void* table_host, uint64_t table_bytes,
                 gh_dtype dt, gh_stream stream );
+/* host-only query: 1 when gh_rows_in reads these rows where they are: a caller whose rows are copied does better to queue the copy before it makes its tables */
+int gh_rows_in_place( const void* x, const void* normed, const void* host, const void* weight, uint64_t size, uint64_t batch, gh_dtype dt );
 /* host-only query: 1 when these calls move `bytes` between this host memory and `dev` by a kernel that reads or writes the host memory where it is: all of it
  * inside one page-locked allocation, both addresses and the size multiples of 16 */
 int gh_host_in_place( const void* host, const void* dev, uint64_t bytes );

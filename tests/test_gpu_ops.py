@@ -145,7 +145,7 @@ def test_host_memory_in_place(source):
 
 
 @pytest.mark.parametrize("dt", ["f16", "f32"])
-@pytest.mark.parametrize("batch,width,table,locked,shift", [(1, 8, 0, True, 0), (3, 288, 12, True, 0), (5, 1000, 512, True, 0), (2, 4104, 4112, True, 0), (2, 8192, 16, True, 0),
+@pytest.mark.parametrize("batch,width,table,locked,shift", [(1, 8, 0, True, 0), (3, 288, 12, True, 0), (4, 1024, 64, True, 1), (5, 1000, 512, True, 0), (2, 4104, 4112, True, 0), (2, 8192, 16, True, 0),
                                                             (1, 8200, 16, True, 0), (4, 7, 20, True, 0), (4, 2048, 4096, True, 4), (4, 2048, 48, False, 0), (92, 4096, 4080, True, 0),
                                                             (200, 4096, 4080, True, 0), (0, 64, 1040, True, 0)])
 def test_rows_in_and_out(dt, batch, width, table, locked, shift):
@@ -161,6 +161,10 @@ def test_rows_in_and_out(dt, batch, width, table, locked, shift):
     x = torch.full((batch, width), 5.0, dtype=tdt(dt), device="cuda")
     normed, weight = torch.zeros_like(x), torch.from_numpy(rng.standard_normal(width).astype(ndt(dt))).cuda()
     step_dev = torch.zeros(table + 16, dtype=torch.uint8, device="cuda")
+    # the route: whole pieces of 16 bytes, rows of up to 16 KiB, 1.5 MiB in all, page-locked
+    row = width * x.element_size()
+    assert ops.rows_in_place(x, normed, host, weight) == (batch > 0 and locked and row % 16 == 0 and shift * x.element_size() % 16 == 0 and row <= 16384
+                                                          and batch * row <= 3 << 19)
     ops.rows_in(x, normed, host, weight, step_dev if table else None, step if table else None)
     assert np.array_equal(x.cpu().numpy(), host)
     assert np.array_equal(step_dev.cpu().numpy()[:table], step[:table]) and not step_dev[table:].any()
