@@ -107,9 +107,12 @@ def rows_out(host, x: torch.Tensor) -> None:
     check(lib().gh_rows_out(host.ctypes.data, _p(x), x.numel() * x.element_size(), _stream()), "gh_rows_out")
 
 
-def embed_rows(x: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor) -> None:
+def embed_rows(x: torch.Tensor, tokens, table: torch.Tensor, step: Optional[torch.Tensor] = None, host_step=None) -> None:
+    """`tokens`: a tensor on the device or an array in page-locked memory; `host_step`: a step's table in host memory, page-locked or not, that goes to `step`."""
     batch, width = x.shape
-    check(lib().gh_embed_rows(_p(x), _p(tokens), _p(table), width, table.shape[0], batch, None, None, 0, _dt(x), _stream()), "gh_embed_rows")
+    at = _p(tokens) if isinstance(tokens, torch.Tensor) else tokens.ctypes.data
+    check(lib().gh_embed_rows(_p(x), at, _p(table), width, table.shape[0], batch, _p(step), None if step is None else host_step.ctypes.data,
+                              0 if step is None else host_step.nbytes, _dt(x), _stream()), "gh_embed_rows")
 
 
 def argmax(v: torch.Tensor, to_host: bool = True):

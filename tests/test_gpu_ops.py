@@ -123,6 +123,54 @@ def test_embed_rows(dt, batch, width, shift):
     assert torch.equal(x, want)
 
 
+# a step's table beside the rows: whole work-groups of pieces and one more, a ragged one, one off a 16-byte boundary, one in pageable memory, one alone
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("batch,nbytes,shift,locked", [(3, 16, 0, True), (5, 4096, 0, True), (5, 4112, 0, True), (300, 65536, 0, True), (3, 20, 0, True), (3, 64, 4, True),
+                                                       (3, 4096, 0, False), (0, 1040, 0, True)])
+def test_embed_rows_with_a_table_of_the_step(dt, batch, nbytes, shift, locked):
+    """Tokens in page-locked memory and the table's bytes as they are; what lies behind the table stays.  The route: in place where the table is whole pieces in
+    page-locked memory."""
+    width, vocab = 24, 50
+    rng = np.random.default_rng(nbytes + batch)
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    table = torch.randn((vocab, width), generator=g, device="cuda").to(tdt(dt))
+    x = torch.full((batch, width), 5.0, dtype=tdt(dt), device="cuda")
+    tokens = ops.pinned_empty((max(batch, 1),), np.uint32)
+    tokens[:] = rng.integers(0, vocab, tokens.shape)
+    tokens[batch // 2] = 0xffffffff if batch > 1 else 0
+    memory = ops.pinned_empty((nbytes + shift,), np.uint8) if locked else np.empty(nbytes + shift, np.uint8)
+    memory[:] = rng.integers(0, 256, memory.shape)
+    host = memory[shift:]
+    step = torch.zeros(nbytes + 16, dtype=torch.uint8, device="cuda")
+    assert ops.host_in_place(host.ctypes.data, step.data_ptr(), nbytes) == (locked and nbytes % 16 == 0 and shift == 0)
+    ops.embed_rows(x, tokens, table, step, host)
+    ops.sync()
+    assert np.array_equal(step.cpu().numpy()[:nbytes], host) and not step[nbytes:].any()
+    ids = torch.from_numpy(tokens[:batch].astype(np.int64)).cuda()
+    want = torch.where((ids < vocab)[:, None], table[ids.clamp(max=vocab - 1)], torch.full_like(x, 5.0))
+    assert torch.equal(x, want)
+
+
+def test_rows_in_captured():
+    """A recorded call reads the rows and the table of the moment it is replayed."""
+    rng = np.random.default_rng(5)
+    host, step = ops.pinned_empty((4, 512), np.float16), ops.pinned_empty((96,), np.uint8)
+    x, step_dev = torch.empty((4, 512), dtype=torch.float16, device="cuda"), torch.empty(96, dtype=torch.uint8, device="cuda")
+    normed, weight = torch.empty_like(x), torch.from_numpy(rng.standard_normal(512).astype(np.float16)).cuda()
+    assert ops.rows_in_place(x, normed, host, weight)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.rows_in(x, normed, host, weight, step_dev, step)
+    for _ in range(3):
+        host[:], step[:] = rng.standard_normal(host.shape).astype(np.float16), rng.integers(0, 256, step.shape)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = normed.clone()
+        assert np.array_equal(x.cpu().numpy(), host) and np.array_equal(step_dev.cpu().numpy(), step)
+        ops.rows_in(x, normed, host, weight)
+        assert torch.equal(got, normed)
+
+
 @pytest.mark.parametrize("source", ["library", "torch"])
 def test_host_memory_in_place(source):
     """Kernels read host memory where it is only if every byte they are to read lies in one page-locked allocation.  A question only: nothing is launched."""
@@ -165,6 +213,7 @@ def test_rows_in_and_out(dt, batch, width, table, locked, shift):
     row = width * x.element_size()
     assert ops.rows_in_place(x, normed, host, weight) == (batch > 0 and locked and row % 16 == 0 and shift * x.element_size() % 16 == 0 and row <= 16384
                                                           and batch * row <= 3 << 19)
+    assert table == 0 or ops.host_in_place(step.ctypes.data, step_dev.data_ptr(), table) == (locked and table % 16 == 0)
     ops.rows_in(x, normed, host, weight, step_dev if table else None, step if table else None)
     assert np.array_equal(x.cpu().numpy(), host)
     assert np.array_equal(step_dev.cpu().numpy()[:table], step[:table]) and not step_dev[table:].any()
@@ -174,6 +223,8 @@ def test_rows_in_and_out(dt, batch, width, table, locked, shift):
     assert ((normed.cpu().double() - want).abs() <= tol).all()
     back = host_memory((batch * width + 8,), ndt(dt))
     back[:] = 7
+    if batch > 0:
+        assert ops.host_in_place(back[shift:].ctypes.data, normed.data_ptr(), batch * row) == (locked and batch * row % 16 == 0 and shift * x.element_size() % 16 == 0)
     ops.rows_out(back[shift:], normed)
     assert np.array_equal(back[shift:shift + batch * width].reshape(batch, width), normed.cpu().numpy())
     assert (back[:shift] == 7).all() and (back[shift + batch * width:] == 7).all()
@@ -1013,6 +1064,40 @@ def test_fused_fp16_scores_of_minus_infinity(variant, route, chunk, kv_heads, gq
         if variant == GH_ATTN_MFMA:
             bound += 2.0 ** -11 * (p * v.abs()).sum(0) + 2.0 ** -25 * v.abs().sum(0)
         assert ((out[i].view(heads, 128).double() - want).abs() <= bound).all(), i
+
+
+# the merge of more than 8 splits: one more than that, one turn of its groups (64) and one more, and enough for three; heads of one turn over the dims and of two
+@pytest.mark.parametrize("keys", [144, 1024, 1040, 2100])
+@pytest.mark.parametrize("variant,dt,heads,kv_heads,head_size", [(GH_ATTN_GENERIC, torch.float32, 2, 1, 48), (GH_ATTN_GENERIC, torch.float16, 3, 3, 160),
+                                                                 (GH_ATTN_GENERIC, torch.float32, 2, 2, 200), (GH_ATTN_GENERIC, torch.float32, 4, 2, 256),
+                                                                 (GH_ATTN_VALU, torch.float16, 2, 2, 128), (GH_ATTN_MFMA, torch.float16, 8, 2, 128)])
+def test_fused_merge_of_many_splits(keys, variant, dt, heads, kv_heads, head_size):
+    """Contexts of every length between one key and all, so that groups of the merge have many splits, one or none."""
+    lengths = [keys, keys - 1, keys // 2 + 3, 129, 128, 17, 16, 1]
+    n = len(lengths)
+    g = torch.Generator(device="cuda").manual_seed(keys + head_size)
+    cache = torch.randn((n, keys, 2, kv_heads, head_size), generator=g, device="cuda").to(dt)
+    q = torch.randn((n, heads, head_size), generator=g, device="cuda").to(dt)
+    shape = Shape(dim=heads * head_size, n_layers=1, n_heads=heads, n_kv_heads=kv_heads, hidden_dim=64, seq_len=keys)
+    out = torch.zeros((n, heads * head_size), dtype=dt, device="cuda")
+    ops.attn_set_chunk(16)
+    try:
+        c_shape, per_split, splits = shape.c(), C.c_uint32(0), C.c_uint32(0)
+        _lib.check(_lib.lib().gh_attn_decode_plan(n, keys - 1, C.byref(c_shape), ops._dt(q), variant, C.byref(per_split), C.byref(splits), None))
+        assert (per_split.value, splits.value) == (16, -(-keys // 16))
+        ops.attn_decode(q.flatten(1), ops.row_table([cache[i].data_ptr() for i in range(n)]), torch.tensor([k - 1 for k in lengths], dtype=torch.int32, device="cuda"), out,
+                        keys - 1, shape, variant=variant)
+    finally:
+        ops.attn_set_chunk(0)
+    for i, k_n in enumerate(lengths):
+        k, v = (cache[i, :k_n, part].double().repeat_interleave(heads // kv_heads, 1) for part in (0, 1))
+        p = ((q[i].double() * k).sum(-1) * head_size ** -0.5).softmax(0)[:, :, None]
+        want = (p * v).sum(0)
+        # fp32 sums of terms of about 1 whose weights add up to 1; the stored value's own rounding; the MFMA kernel's weights of fp16, as above
+        bound = 2e-5 + want.abs() * (2.0 ** -11 if dt == torch.float16 else 0.0)
+        if variant == GH_ATTN_MFMA:
+            bound += 2.0 ** -11 * (p * v.abs()).sum(0) + 2.0 ** -25 * v.abs().sum(0) * p.max(0).values
+        assert ((out[i].view(heads, head_size).double() - want).abs() <= bound).all(), i
 
 
 @pytest.mark.parametrize("shape", [MHA128, MHA128_ODD, GQA2, GQA4, GQA8], ids=["mha", "mha6", "gqa2", "gqa4", "gqa8"])

@@ -144,18 +144,21 @@ def test_joined_plans_of_the_benchmark_shapes():
     assert both(32, 2047, SHAPES["13B"])[0] == 0
 
 
-@pytest.mark.parametrize("name", ["7B", "13B", "70B"])
+@pytest.mark.parametrize("name", ["7B", "13B", "70B", "gqa2", "gqa4", "gqa16"])
 def test_short_splits_stay_inside_what_the_fixed_array_holds(name):
     """Plans of few streams and few keys cut below 256 keys; never so fine that a call which fitted the fixed array of gh_attn_decode_static with
-    splits of 256 keys would not fit any more."""
+    splits of 256 keys would not fit any more, whichever kernel is asked for."""
     shape = SHAPES[name]
-    short = 0
-    for batch in range(1, 70):
-        for keys in list(range(1, 300, 7)) + list(range(300, shape.seq_len, 61)):
-            chunk, splits, need = plan(batch, keys - 1, shape, 0, GH_ATTN_AUTO)
-            short += chunk < 256 and splits > 1
-            whole = batch * shape.n_heads * ((keys + 255) // 256) * 130 * 4
-            assert need <= 16 << 20 or whole > 16 << 20 or chunk >= 256
-            assert splits <= 64 or chunk >= 256
-            assert chunk >= (32 if keys <= 256 else 64)
-    assert short > 100
+    for dt, variant in variants(shape):
+        if dt == 1 or variant == GH_ATTN_GENERIC:
+            continue
+        short = 0
+        for batch in range(1, 70):
+            for keys in list(range(1, 300, 7)) + list(range(300, shape.seq_len, 61)):
+                chunk, splits, need = plan(batch, keys - 1, shape, dt, variant)
+                short += chunk < 256 and splits > 1
+                whole = batch * shape.n_heads * ((keys + 255) // 256) * 130 * 4
+                assert need <= 16 << 20 or whole > 16 << 20 or chunk >= 256
+                assert splits <= 64 or chunk >= 256
+                assert chunk >= (32 if keys <= 256 else 64)
+        assert short > 100
