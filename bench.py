@@ -17,7 +17,8 @@ Prints ONE JSON line:
                events run right after them and are reported as ms_per_step_with_attn_events
   *_resident   the same step between two events, after its activations and tables are queued and before the copy
                back: what the stage costs with its inputs resident in HBM (ms_per_step goes through the host
-               state buffers on both sides, as the reference's forward() does)
+               state buffers on both sides, as the reference's forward() does).  Activations of up to 1.5 MiB
+               are read and normed by one kernel, so that the step's first norm lies in front of these events
   cpu_baseline the CPU oracle (a port of the reference's fp32 OpenMP path) timed on a bounded sample:
                one hosted layer on the very weights, cache rows and activations the GPU stage ran on
   concept_path the same stage driven through the reference's own op sequence only (unfused attention

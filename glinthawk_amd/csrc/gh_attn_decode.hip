@@ -331,7 +331,8 @@ __global__ __launch_bounds__( 256 ) void attn_merge_kernel( Partials part,
 }
 
 // More than 8 splits: G groups of `dims` threads take every G-th split, eight of them requested at once, and add their parts up in LDS.  One memory round
-// trip up to 8 G splits, where the kernel above takes one for every split beyond its eight (70B, one context of 4096 keys in 32 splits: 20.6 us, so 14.8).
+// trip up to 8 G splits, where the kernel above takes one for every split beyond its eight (70B, one context of 4096 keys in 32 splits of 128, attention and
+// merge in a graph: 20.4 us, so 14.8).
 constexpr uint32_t MERGE_GROUPS = 8;
 template<typename T>
 __global__ __launch_bounds__( 1024 ) void attn_merge_many_kernel( Partials part,
@@ -1393,8 +1394,9 @@ JoinChoice join_choice( uint64_t streams, int variant, uint32_t n_tok )
 // rules for a full chip keep.  Up to about 800 waves of the MFMA kernel and 1536 of the VALU kernel, at least four splits; at least 64 keys, 32 where that is a
 // share of up to 256.  Only while they stay short, as longer ones come out even with or behind the plan they replace (7B, 4 contexts of 2048 keys: 26.6 us, in
 // splits of 192 28.9), and where there are keys enough for the streams that many waves pay for a merge kernel (70B, 48 contexts of 128 keys: one split 11.4,
-// four and a merge 14.8).  us, the fused op with splits of 256 or joined / so; 70B shape, contexts x keys:
-//   1 x 300: 19.5 / 9.3   1 x 1537: 19.8 / 11.3   1 x 4096: 20.9 / 12.3   4 x 1025: 19.6 / 12.2   9 x 512: 20.0 / 11.7   16 x 768: 21.8 / 17.0
+// four and a merge 14.8).  us, the fused op with splits of 256 or joined / so (more than 8 splits merged by attn_merge_many_kernel on
+// either side); 70B shape, contexts x keys:
+//   1 x 300: 19.5 / 9.3   1 x 1537: 19.8 / 11.3   1 x 4096: 21.4 / 12.1   4 x 1025: 19.6 / 12.2   9 x 512: 20.0 / 11.7   16 x 768: 21.8 / 17.0
 //   32 x 300: 22.4 / 14.8   48 x 768: 36.2 / 32.9
 // 7B shape: 1 x 1025: 19.7 / 11.4   4 x 512: 22.2 / 12.1   9 x 300: 23.4 / 13.8   16 x 300: 25.3 / 18.6   16 x 768: 38.8 / 36.5
 // Splits per stream of such a plan at most, 0: none.

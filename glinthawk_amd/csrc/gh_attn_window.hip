@@ -1166,8 +1166,8 @@ int attend_decode( const WindowOut<__bf16>& out, const __bf16* q, const float* b
     head_cols--;
   }
   const uint64_t blocks = s.heads / head_cols, groups = rows * blocks, most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
-  // Eight waves on the keys of a row where work-groups of four would leave room on the CUs and each wave still has a tile or more; with K and V apart a CU
-  // holds one such work-group, which pays only while they are few.  us, 32 heads of 128, rows x keys, four waves / eight.  Values that are keys: 1 x 300
+  // Eight waves on the keys of a row where work-groups of four would leave room on the CUs and a row has four tiles or more (below eight tiles some of the
+  // waves have none); with K and V apart a CU holds one such work-group, which pays only while they are few.  us, 32 heads of 128, rows x keys, four waves / eight.  Values that are keys: 1 x 300
   // 11.0 / 7.6, 8 x 300 13.8 / 9.2, 24 x 300 15.7 / 17.6, 1 x 2048 26 / 18, 32 x 1025 49.4 / 46.9, 48 x 1025 69.2 / 65.0.  Both: 1 x 1025 18.9 / 16.5, 4 x 1025
   // 24.8 / 26.8, 8 x 300 17.5 / 13.1, 16 x 300 20.3 / 24.0.
   const bool wide = s.values_are_keys ? ( groups < 16ull * cu_count() && most >= 16 * STEP_KEYS ) || ( groups <= (uint64_t)cu_count() && most >= 4 * STEP_KEYS )

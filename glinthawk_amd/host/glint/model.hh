@@ -237,7 +237,9 @@ public:
       balance_step();
     }
 
-    spans_.mark( 0, ops_.stream() ); // the activations and the tables are there: from here to the copy back it is kernels only
+    // The activations and the tables are there: from here to the copy back it is kernels only.  The first norm is one of them unless the activations were
+    // read in place: then it is part of the kernel that brought them, and lies outside the span.
+    spans_.mark( 0, ops_.stream() );
     if ( fused_layers && !run.empty() && !norms_ride && !in_place ) {
       ops_.template rmsnorm<Config::dim>( xb_, x_, reinterpret_cast<float32_t*>( temp_ ), layers_[run[0]].rms_att_weight, batch_ );
     }
@@ -605,8 +607,8 @@ private:
     }
   }
 
-  // the fused decode attention of one layer: over equal runs of keys where upload_tables() found the lengths of this
-  // step's contexts far apart (the cuts are made there, once for all layers), else one wave per (context, kv head, split)
+  // the fused decode attention of one layer: over equal runs of keys where fill_tables() found the lengths of this
+  // step's contexts far apart (balance_step() makes the cuts, once for all layers), else one wave per (context, kv head, split)
   void fused_attention( const size_t table_index )
   {
     if ( balanced_step_ ) {

@@ -292,8 +292,8 @@ int gh_attn_set_chunk( uint32_t tokens_per_split );
 int gh_attn_set_split_join( int on );
 /* measurement hook: which kernel GH_ATTN_AUTO picks where the shape permits it (GH_ATTN_AUTO restores the library's choice) */
 int gh_attn_set_auto_variant( int variant );
-/* bytes that serve every call with at most `batch` rows and positions up to `max_pos` (a smaller batch is cut into more splits per context, so the
- * largest need over all batch sizes in [1, batch] is returned) */
+/* bytes that serve every call with at most `batch` rows and positions up to `max_pos`, whichever kernel it asks for (a smaller batch is cut into more splits
+ * per context, so the largest need over all batch sizes in [1, batch] is returned) */
 uint64_t gh_attn_decode_workspace( uint64_t batch, uint32_t max_pos, const gh_shape* shape );
 /* host-only query: how gh_attn_decode would cut this call (tokens per split, splits of the longest context) and the workspace bytes it would use
  * (0 for a plan whose splits are added up inside the work-groups) */
