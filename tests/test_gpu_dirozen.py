@@ -102,6 +102,34 @@ def test_projections_with_a_large_feed_forward(n_tokens):
     assert_rows(back(region[:at].view(torch.bfloat16)).reshape(-1, kv * d)[4:4 + n_tokens], y[:, 256:384], 1e-2, "keys")
 
 
+# whole tiles and ragged ones in both directions
+@pytest.mark.parametrize("n_tokens,ff", [(768, 8192), (700, 8200), (1365, 5632)])
+def test_feed_forward_of_many_rows_with_tanh(n_tokens, ff):
+    """The gate with tanh in the tiles' epilogue, on the fp32 sums (rounded factors would be further off than this allows), into rows that lie apart: one rounding to
+    bf16, 2^-8 of the result, and 1e-4 for the sums and the fast exponential.  A context without an entry gets no row, and nothing beside the hidden values is written."""
+    import torch
+    from glinthawk_amd import ops
+    heads, kv, d, width = 4, 2, 64, 256
+    a = ops.window_attn(heads, kv, d, d, 1.0, values_are_keys=True)
+    rows, ff_row = ops.parallel_weight_rows(a, True, ff)
+    g = torch.Generator().manual_seed(n_tokens)
+    w = (torch.randn((rows, width), generator=g) / 16).cuda().bfloat16()
+    x = torch.randn((3 * n_tokens, width), generator=g).cuda().bfloat16()
+    keys = -(-n_tokens // 32) * 32
+    at = keys * kv * d * 2
+    regions = [torch.zeros(at + keys * kv * 4, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    wide = torch.full((3 * n_tokens, ff + 48), 5.0, dtype=torch.bfloat16, device="cuda")
+    ops.matmul_parallel(x, w, a, ops.row_table([regions[0].data_ptr(), 0, regions[1].data_ptr()]), positions([0, 0, 0]), n_tokens, 1e-3, 0.5, 8, True, wide[:, 40:40 + ff],
+                        ops.GH_ACT_GELU_TANH, factor_offset=at)
+    y = x.double() @ w[ff_row:ff_row + 2 * ff].double().T
+    want = torch.nn.functional.gelu(y[:, :ff], approximate="tanh") * y[:, ff:]
+    got = wide[:, 40:40 + ff].double()
+    live = torch.ones(3 * n_tokens, dtype=torch.bool, device="cuda")
+    live[n_tokens:2 * n_tokens] = False
+    assert ((got - want).abs()[live] <= (2.0 ** -8 * want.abs() + 1e-4 * (1.0 + want.abs().sqrt()))[live]).all()
+    assert bool((wide[~live] == 5).all()) and bool((wide[:, :40] == 5).all()) and bool((wide[:, 40 + ff:] == 5).all())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n_tokens", [1, 4, 250, 600])
 @pytest.mark.parametrize("heads,kv,d,ff,gated,every", [(6, 3, 20, 44, True, 7), (4, 1, 64, 0, True, 1), (5, 5, 96, 72, False, 33), (3, 1, 136, 21, True, 64), (2, 2, 300, 40, True, 0),

@@ -346,9 +346,10 @@ def test_matmul_qkv_rope_append(dt, shape):
     assert torch.equal(arena_b.dev[mask], before[mask])
 
 
-# tokens that end on a tile, behind one, with a rest that is a product of its own; steps that are walked (even) and not; heads of 128, 64 and 32
+# tokens that end on a tile, behind one, with a rest that is a product of its own; steps that are walked (even) and not; heads of 128 to 8
 @pytest.mark.parametrize("s,kv_heads,gqa,head_size,b", [(1024, 4, 2, 128, 7168), (2048, 4, 4, 128, 3328), (2048, 4, 4, 128, 4100), (1024, 8, 4, 64, 5000), (576, 2, 8, 128, 7000),
-                                                        (640, 16, 2, 32, 9000), (8192, 8, 8, 128, 3328)])
+                                                        (640, 16, 2, 32, 9000), (512, 32, 4, 16, 9000), (576, 32, 4, 8, 9100),
+                                                        (8192, 8, 8, 128, 3328)])
 def test_many_rows_of_qkv_rotated_and_appended(s, kv_heads, gqa, head_size, b):
     """Against product, append and rotation one by one.  The product may sum in another order (a rounding of f16), and a rotation adds two products.  Empty
     contexts keep their query unrotated; the rows around an appended one stay as they are; cache rows off a 16-byte boundary."""
