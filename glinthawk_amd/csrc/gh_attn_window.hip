@@ -531,7 +531,9 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
   const float m = wave_max( own_max ); // (the last split's repeated in the lanes beyond)
   const float weight = lane < splits ? __expf( own_max - m ) : 0.0f;
   const float sm = wave_sum( lane < splits ? own_sum * weight : 0.0f );
-  for ( uint32_t e = lane; e < s.vdim; e += 64 ) {
+  // No lane leaves before the end: each holds a split's weight, and what makes it may move into a loop that only the lanes with a value enter.
+  for ( uint32_t e0 = 0; e0 < s.vdim; e0 += 64 ) {
+    const uint32_t e = min( e0 + lane, s.vdim - 1 );
     float a = 0.0f;
     for ( uint32_t k0 = 0; k0 < splits; k0 += 8 ) {
       float v[8];
@@ -544,7 +546,9 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
         a += k0 + u < splits ? v[u] * lane_value( weight, min( k0 + u, splits - 1 ) ) : 0.0f;
       }
     }
-    out.out[row * out.stride + head * s.vdim + e] = from_f32<E>( a / sm * gate );
+    if ( e0 + lane < s.vdim ) {
+      out.out[row * out.stride + head * s.vdim + e] = from_f32<E>( a / sm * gate );
+    }
   }
 }
 

@@ -280,6 +280,23 @@ def test_attention_over_keys_that_are_values(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["small", "ten", "matrix", "own", "deep"])
+def test_attention_over_many_splits(name, dtype):
+    """Single tokens behind thousands of keys, in more splits than their merge takes at once (64 at most), or than a head has values; contexts that end in the first of
+    them and in the middle."""
+    T, eps, scale = 5000, 1e-3, 2.0 / ATTENTIONS[name][2] ** 0.5
+    heads, kv, d = shape = ATTENTIONS[name]
+    rng = np.random.default_rng(8)
+    start = [T - 1, 40, 2600]
+    q = [M.to_bf16(rng.standard_normal((T, heads, d))) for _ in start]
+    k = [M.to_bf16(rng.standard_normal((T, kv, d)) * np.exp(rng.standard_normal((T, kv, 1)))) for _ in start]
+    want = np.stack([[P.read_keys(qq[s, h].astype(np.float64), kk[: s + 1, h // (heads // kv)].astype(np.float64), eps, scale) for h in range(heads)] for qq, kk, s in zip(q, k, start)])
+    tol = 1e-5 if dtype == "f32" else 8e-3
+    assert_rows(attend(shape, q, k, start, 1, dtype, eps, scale).reshape(3, -1), want.reshape(3, -1), tol, "three contexts")
+    assert_rows(attend(shape, q[:1], k[:1], start[:1], 1, dtype, eps, scale).reshape(1, -1), want[:1].reshape(1, -1), tol, "one")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["small", "matrix", "ten", "own", "between", "deep"])
 def test_one_key_stands_out(name, dtype):
     """Every key in turn made the one its queries' scores pick, among hundreds: read from its own position on by every later query, near or

@@ -225,6 +225,29 @@ def test_windowed_attention_of_many_contexts(name, contexts):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_windowed_attention_over_many_splits(dtype):
+    """Single tokens behind thousands of keys, in more splits than their merge takes at once (64 at most), and than a head has values; contexts that end in
+    the first of them and in the middle."""
+    T = 5000
+    heads, kv, d, dv, _, _, rows, bias_max = shape = ATTENTIONS["open"]
+    rng = np.random.default_rng(9)
+    start = [T - 1, 40, 2600]
+    q, k, v = ([M.to_bf16(rng.standard_normal((T, n, e))) for _ in start] for n, e in ((heads, d), (kv, d), (kv, dv)))
+    rel = rng.standard_normal((rows, heads)).astype(np.float32)
+    want = np.zeros((3, heads, dv))
+    for i, s in enumerate(start):
+        bias = rel[[P.distance_bucket(s - j, rows, bias_max) for j in range(s + 1)]].astype(np.float64)
+        for h in range(heads):
+            score = (k[i][: s + 1, h // (heads // kv)].astype(np.float64) @ q[i][s, h]) * d ** -0.5 + bias[:, h]
+            p = np.exp(score - score.max())
+            want[i, h] = p / p.sum() @ v[i][: s + 1, h // (heads // kv)].astype(np.float64)
+    tol = 1e-5 if dtype == "f32" else 8e-3
+    for n in (3, 1):
+        got = attend(shape, q[:n], k[:n], v[:n], rel, start[:n], 1, dtype)
+        assert_rows(got.reshape(n, -1), want[:n].reshape(n, -1), tol, f"{n} contexts")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["grouped", "matrix", "ten", "own"])
 def test_one_key_stands_out(name, dtype):
     """Every key in turn made the one that its query's score picks: seen exactly where the window or the kept tokens show it, and just
