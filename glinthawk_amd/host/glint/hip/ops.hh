@@ -464,6 +464,28 @@ public:
                                                  Config::n_kv_heads, Config::gqa_size, Config::head_size, gh_type<DType>(), this->stream_ ) );
   }
 
+  // All of a layer up to its attention in one launch; attention_rides( batch_size ): whether there is one
+  static bool attention_rides( const uint64_t batch_size )
+  {
+    const gh_shape s = shape();
+    return gh_rmsnorm_qkv_attn_rides( batch_size, &s, gh_type<DType>() ) == 1;
+  }
+  void rmsnorm_qkv_attention( DType* xb,
+                              const DType* x,
+                              const DType* norm_weight,
+                              const DType* wqkv,
+                              const uint64_t batch_size,
+                              const uint32_t* token_positions_dev,
+                              const DType* freq_cis_real,
+                              const DType* freq_cis_imag,
+                              const void* const* layer_rows_dev,
+                              void* const* token_rows_dev ) const
+  {
+    const gh_shape s = shape();
+    GLINT_GH( gh_rmsnorm_qkv_attn( xb, x, norm_weight, wqkv, batch_size, token_positions_dev, freq_cis_real, freq_cis_imag, layer_rows_dev, token_rows_dev, &s,
+                                   gh_type<DType>(), this->stream_ ) );
+  }
+
 private:
   // TokenContext / LayerContext are a single pointer each, so an array of them is a pointer table
   static_assert( sizeof( typename ContextType::TokenContextType ) == sizeof( void* ) );

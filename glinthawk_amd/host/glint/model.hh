@@ -667,12 +667,18 @@ private:
     ops_.template matmul_accum<Config::hidden_dim, Config::dim>( x_, hb_, w.w2, batch_, next_att_norm ? xb_ : nullptr, next_att_norm );
   }
 
-  // The same with the norms in the launches of the products that read them: 5 launches, x_ all that passes from layer to layer.
+  // The same with the norms in the launches of the products that read them: 5 launches, 4 where the attention is in that of its projections; x_ is all
+  // that passes from layer to layer.
   void normed_layer_ops( const size_t layer, const size_t table_index )
   {
     const auto& w = layers_[layer];
-    ops_.rmsnorm_matmul_qkv_rope_append( q_, x_, w.rms_att_weight, w.wq, batch_, pos_dev(), base_.freq_cis_real, base_.freq_cis_imag, token_rows_dev( table_index ) );
-    fused_attention( table_index );
+    if ( !balanced_step_ && LlamaOperations::attention_rides( batch_ ) ) {
+      ops_.rmsnorm_qkv_attention( xb_, x_, w.rms_att_weight, w.wq, batch_, pos_dev(), base_.freq_cis_real, base_.freq_cis_imag, layer_rows_dev( table_index ),
+                                  token_rows_dev( table_index ) );
+    } else {
+      ops_.rmsnorm_matmul_qkv_rope_append( q_, x_, w.rms_att_weight, w.wq, batch_, pos_dev(), base_.freq_cis_real, base_.freq_cis_imag, token_rows_dev( table_index ) );
+      fused_attention( table_index );
+    }
     ops_.template matmul_accum<Config::dim, Config::dim>( x_, xb_, w.wo, batch_ );
     ops_.rmsnorm_matmul_silu_gate( hb_, x_, w.rms_ffn_weight, w.w1, batch_ );
     ops_.template matmul_accum<Config::hidden_dim, Config::dim>( x_, hb_, w.w2, batch_ );

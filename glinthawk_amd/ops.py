@@ -202,6 +202,15 @@ def rmsnorm_matmul_qkv_rope_append(x: torch.Tensor, norm_weight: torch.Tensor, w
     return q
 
 
+def rmsnorm_qkv_attn(x: torch.Tensor, norm_weight: torch.Tensor, wqkv: torch.Tensor, pos: torch.Tensor, freq_real, freq_imag, layer_rows: torch.Tensor,
+                     token_rows: torch.Tensor, shape: Shape) -> torch.Tensor:
+    b = x.shape[0]
+    xb = torch.zeros((b, shape.dim), dtype=x.dtype, device=x.device)
+    check(lib().gh_rmsnorm_qkv_attn(_p(xb), _p(x), _p(norm_weight), _p(wqkv), b, _p(pos), _p(freq_real), _p(freq_imag), _p(layer_rows), _p(token_rows),
+                                    C.byref(shape.c()), _dt(x), _stream()), "gh_rmsnorm_qkv_attn")
+    return xb
+
+
 def soft_sample(v: torch.Tensor, temperatures: Sequence[float], seed: int = 0) -> None:
     batch, vocab = v.shape
     temps = (C.c_float * batch)(*[float(t) for t in temperatures])

@@ -1,5 +1,7 @@
 """Projections fused with their follow-up ops against the same ops issued one by one (bit-exact where
 the arithmetic is element-wise, tolerance where a reduction order differs) and against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -413,3 +415,53 @@ def test_stage_with_and_without_fused_projections(name, dtype):
             a.set_prompt(i, i, tokens[i], step + 1)
     a.close()
     b.close()
+
+
+# widths and heads of the smallest and the largest the launch takes, groups of query heads, heads that leave rows of lanes idle; more keys than one turn
+@pytest.mark.parametrize("kv_heads,gqa,head_size,batch", [(6, 1, 48, 4), (2, 2, 8, 7), (5, 1, 64, 3), (2, 4, 40, 6), (1, 1, 4, 8), (4, 1, 20, 64), (3, 2, 44, 8)])
+def test_attention_in_the_launch_of_its_projections(kv_heads, gqa, head_size, batch):
+    """Against 64 bits: rounding is that of fp32 sums of up to 320 products and 600 weights, some 1e-6; a wrong key, row or rotation is far beyond.  Cache rows on
+    and off a 16-byte boundary, an empty context, a key whose scores are infinite, rows around the appended one."""
+    shape = Shape(dim=kv_heads * gqa * head_size, n_layers=1, n_heads=kv_heads * gqa, n_kv_heads=kv_heads, hidden_dim=64, seq_len=600)
+    dim, kv_dim = shape.dim, shape.kv_dim
+    g = torch.Generator(device="cuda").manual_seed(head_size)
+    x, nw = torch.randn((batch, dim), generator=g, device="cuda"), torch.randn((dim,), generator=g, device="cuda")
+    w = torch.randn((dim + 2 * kv_dim, dim), generator=g, device="cuda") / dim ** 0.5
+    angle = torch.rand((600, head_size // 2), generator=g, device="cuda") * 6
+    re, im = torch.cos(angle), torch.sin(angle)
+    pos = ([0, 1, 255, 256, 599, 31, 257, 300] * 8)[:batch]
+    dpos = torch.tensor(pos, dtype=torch.int32, device="cuda")
+    assert _lib.lib().gh_rmsnorm_qkv_attn_rides(batch, ctypes.byref(shape.c()), _lib.GH_F32) == 1
+    for shift in (0, 1):
+        flat = torch.randn((batch * 600 * 2 * kv_dim + 1,), generator=g, device="cuda")
+        cache = flat[shift: shift + batch * 600 * 2 * kv_dim].view(batch, 600, 2 * kv_dim)
+        cache[2, 7, 0] = -float("inf")
+        before = cache.clone()
+        rows = ops.row_table([0 if i == 1 and batch > 4 else cache[i].data_ptr() for i in range(batch)])
+        ends = ops.row_table([0 if i == 1 and batch > 4 else cache[i, pos[i]].data_ptr() for i in range(batch)])
+        got = ops.rmsnorm_qkv_attn(x, nw, w, dpos, re, im, rows, ends, shape)
+        xd = x.double()
+        y = (xd / torch.sqrt((xd * xd).mean(1, keepdim=True) + 1e-5) * nw.double()) @ w.double().t()
+        for i in range(batch):
+            if i == 1 and batch > 4:
+                assert (got[i] == 0).all() and torch.equal(cache[i], before[i])
+                continue
+            p = pos[i]
+            a, b = re[p].double(), im[p].double()
+
+            def turned(v):
+                v = v.view(-1, head_size // 2, 2)
+                return torch.stack([v[..., 0] * a - v[..., 1] * b, v[..., 0] * b + v[..., 1] * a], -1).view(-1, head_size)
+
+            q, k, v = turned(y[i, :dim]), turned(y[i, dim: dim + kv_dim]), y[i, dim + kv_dim:].view(-1, head_size)
+            old = before[i, :p].double().view(p, 2, kv_heads, head_size)
+            keys, values = torch.cat([old[:, 0], k[None]]), torch.cat([old[:, 1], v[None]])
+            want = torch.empty((gqa * kv_heads, head_size), dtype=torch.float64, device="cuda")
+            for h in range(gqa * kv_heads):
+                want[h] = torch.softmax(keys[:, h // gqa].contiguous() @ q[h] * head_size ** -0.5, 0) @ values[:, h // gqa].contiguous()
+            for have, should in ((got[i], want.view(-1)), (cache[i, p], torch.cat([k.view(-1), v.view(-1)]))):
+                fine = ~should.isnan()
+                assert torch.equal(have.isnan(), ~fine)
+                assert (have.double() - should)[fine].norm() <= 5e-6 * should[fine].norm() + 1e-12
+            keep = torch.arange(600, device="cuda") != p
+            assert torch.equal(cache[i][keep], before[i][keep])
