@@ -170,6 +170,8 @@ SIGNATURES = {
     "gh_attn_set_prefill_tiles": (_i, [_i]),
     "gh_attn_prefill_workspace": (_u64, [_u64, _u32, _shp]),
     "gh_attn_prefill": (_i, [_vp, _vp, _vp, _vp, _u64, _u32, _u32, _shp, _i, _vp, _u64, _i, _vp]),
+    "gh_embed_step": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _u64, _u32, _vp, _vp, _u64, _u64, _u64, _vp, _u64, _step, _i, _vp]),
+    "gh_matmul_scaled_argmax": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _u64, _f, _i, _vp]),
     "gh_embed_positions": (_i, [_vp, _vp, _vp, _u64, _u32, _vp, _vp, _u64, _u64, _u64, _vp, _u64, _i, _vp]),
     "gh_matmul_stream": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _step, _i, _vp]),
     "gh_stream_out": (_i, [_vp, _u64, _u64, _step, _i, _vp]),

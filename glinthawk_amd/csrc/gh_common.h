@@ -193,6 +193,37 @@ __device__ __forceinline__ float sum_rows( float a, float b )
   return __builtin_bit_cast( float, r0 ) + __builtin_bit_cast( float, r1 );
 }
 
+// the lower index of equal values; NaN never beats anything
+__device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float v, uint32_t i )
+{
+  const bool take = v > best || ( v == best && i < best_i );
+  best = take ? v : best;
+  best_i = take ? i : best_i;
+}
+// Over a work-group of THREADS: true in thread 0, which has the result.
+template<int THREADS>
+__device__ __forceinline__ bool block_arg( float& best, uint32_t& best_i, float* s_val, uint32_t* s_idx )
+{
+#pragma unroll
+  for ( int off = 32; off > 0; off >>= 1 ) {
+    const float o_val = __shfl_xor( best, off, WAVE );
+    const uint32_t o_idx = __shfl_xor( best_i, off, WAVE );
+    arg_better( best, best_i, o_val, o_idx );
+  }
+  if ( threadIdx.x % WAVE == 0 ) {
+    s_val[threadIdx.x / WAVE] = best;
+    s_idx[threadIdx.x / WAVE] = best_i;
+  }
+  __syncthreads();
+  if ( threadIdx.x != 0 ) {
+    return false;
+  }
+  for ( int w = 1; w < THREADS / WAVE; w++ ) {
+    arg_better( best, best_i, s_val[w], s_idx[w] );
+  }
+  return true;
+}
+
 template<typename T>
 __device__ __forceinline__ float to_f32( T v );
 template<>

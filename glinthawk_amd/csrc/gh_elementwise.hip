@@ -242,12 +242,6 @@ __global__ __launch_bounds__( EW_THREADS ) void embed_rows_kernel( P* __restrict
 // rows of 32000: 36.8 us with 256 threads that went value by value, 6.1 so.  256 threads where they ask for all of a row at once, with the fewest
 // pieces that do (1024 f16 rows of 1000: 4.1 us, 7.5 with eight each; of 4096: 5.0, 9.3, with 1024 threads 17.6), else 1024.  As a loop over the row
 // would have it: the lowest index of equal values, NaN never beats anything but stays where the row begins with it.
-__device__ __forceinline__ void arg_better( float& best, uint32_t& best_i, float v, uint32_t i )
-{
-  const bool take = v > best || ( v == best && i < best_i );
-  best = take ? v : best;
-  best_i = take ? i : best_i;
-}
 // V: values per load, n % V == 0 and rows aligned to V values
 template<typename T, int V, int ARG_THREADS, int AHEAD>
 __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __restrict__ out, const T* __restrict__ v, uint32_t n )
@@ -279,22 +273,7 @@ __global__ __launch_bounds__( ARG_THREADS ) void argmax_kernel( uint32_t* __rest
       }
     }
   }
-#pragma unroll
-  for ( int off = 32; off > 0; off >>= 1 ) {
-    const float o_val = __shfl_xor( best, off, WAVE );
-    const uint32_t o_idx = __shfl_xor( best_i, off, WAVE );
-    arg_better( best, best_i, o_val, o_idx );
-  }
-  const int wave = threadIdx.x / WAVE;
-  if ( threadIdx.x % WAVE == 0 ) {
-    s_val[wave] = best;
-    s_idx[wave] = best_i;
-  }
-  __syncthreads();
-  if ( threadIdx.x == 0 ) {
-    for ( int w = 1; w < ARG_THREADS / WAVE; w++ ) {
-      arg_better( best, best_i, s_val[w], s_idx[w] );
-    }
+  if ( block_arg<ARG_THREADS>( best, best_i, s_val, s_idx ) ) {
     out[blockIdx.x] = first != first || best_i == 0xffffffffu ? 0u : best_i;
   }
 }

@@ -93,6 +93,50 @@ __device__ __forceinline__ float4 load4_e( const void* p, uint32_t c )
   return ProductView<E>::load4( static_cast<const E*>( p ) + c );
 }
 
+// what a step leaves for the next product: the row, normed where there is a norm
+template<typename E, int NV>
+__device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_t ( &col )[NV], const bool ( &live )[NV], uint64_t row, uint32_t width, const StepPtrs& p, float* s_next )
+{
+  if ( p.out == nullptr ) {
+    return;
+  }
+  float inv = 1.0f;
+  if ( p.next_norm != nullptr ) {
+    float ss = 0.0f;
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) {
+      ss += live[g] ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
+    }
+    inv = 1.0f / sqrtf( row_sum( ss, s_next ) / (float)width + p.eps );
+  }
+  E* out = static_cast<E*>( p.out ) + row * p.out_stride;
+#pragma unroll
+  for ( int g = 0; g < NV; g++ ) {
+    float4 w = make_float4( 1.0f, 1.0f, 1.0f, 1.0f );
+    if ( p.next_norm != nullptr ) {
+      w = load4_e<E>( p.next_norm, col[g] );
+      w = make_float4( p.norm_base + w.x, p.norm_base + w.y, p.norm_base + w.z, p.norm_base + w.w );
+    }
+    union
+    {
+      E e[4];
+      uint2 half;
+      uint4 full;
+    } o;
+    o.e[0] = from_f32<E>( v[g].x * inv * w.x );
+    o.e[1] = from_f32<E>( v[g].y * inv * w.y );
+    o.e[2] = from_f32<E>( v[g].z * inv * w.z );
+    o.e[3] = from_f32<E>( v[g].w * inv * w.w );
+    if ( live[g] ) {
+      if constexpr ( sizeof( E ) == 2 ) {
+        *reinterpret_cast<uint2*>( out + col[g] ) = o.half;
+      } else {
+        *reinterpret_cast<uint4*>( out + col[g] ) = o.full;
+      }
+    }
+  }
+}
+
 // A thread owns NV groups of four columns.  A group past the row's end reads group 0 and stores nothing: no load sits under a branch.
 template<typename E, typename View, bool PRODUCT, int NV>
 __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict__ x, View y, uint32_t width, StepPtrs p )
@@ -155,44 +199,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
       v[g] = old[g];
     }
   }
-  if ( p.out == nullptr ) {
-    return;
-  }
-  float inv = 1.0f;
-  if ( p.next_norm != nullptr ) {
-    float ss = 0.0f;
-#pragma unroll
-    for ( int g = 0; g < NV; g++ ) {
-      ss += live[g] ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
-    }
-    inv = 1.0f / sqrtf( row_sum( ss, s_next ) / (float)width + p.eps );
-  }
-  E* out = static_cast<E*>( p.out ) + row * p.out_stride;
-#pragma unroll
-  for ( int g = 0; g < NV; g++ ) {
-    float4 w = make_float4( 1.0f, 1.0f, 1.0f, 1.0f );
-    if ( p.next_norm != nullptr ) {
-      w = load4_e<E>( p.next_norm, col[g] );
-      w = make_float4( p.norm_base + w.x, p.norm_base + w.y, p.norm_base + w.z, p.norm_base + w.w );
-    }
-    union
-    {
-      E e[4];
-      uint2 half;
-      uint4 full;
-    } o;
-    o.e[0] = from_f32<E>( v[g].x * inv * w.x );
-    o.e[1] = from_f32<E>( v[g].y * inv * w.y );
-    o.e[2] = from_f32<E>( v[g].z * inv * w.z );
-    o.e[3] = from_f32<E>( v[g].w * inv * w.w );
-    if ( live[g] ) {
-      if constexpr ( sizeof( E ) == 2 ) {
-        *reinterpret_cast<uint2*>( out + col[g] ) = o.half;
-      } else {
-        *reinterpret_cast<uint4*>( out + col[g] ) = o.full;
-      }
-    }
-  }
+  step_out<E, NV>( v, col, live, row, width, p, s_next );
 }
 
 // any width: the row goes through memory between the passes (each thread re-reads only what it wrote)
@@ -243,6 +250,81 @@ __global__ __launch_bounds__( 256 ) void stream_step_any_kernel( float* __restri
   }
 }
 
+// The start of a step in one launch: embedding, the norm behind it and, in work-groups of their own, the step's tables, which lie in page-locked memory
+// and of which the rows read their token and position there.  Each was a launch before, at the head of a chain that the host is only just ahead of: 32 rows of
+// 4096 with a wait behind them 34.0 us, 20.8 so; 512 (tables uploaded first) 34.0 and 24.7; 8192 74.4 and 51.9, a pass over the rows less.
+template<typename E, int NV>
+__global__ __launch_bounds__( 1024 ) void embed_step_kernel( float* __restrict__ x, const uint32_t* __restrict__ tokens, const uint32_t* __restrict__ start_pos, uint32_t n_tokens,
+                                                             const E* __restrict__ embed, const E* __restrict__ pos_table, uint32_t width, uint32_t vocab, uint32_t max_pos,
+                                                             E* __restrict__ copy, uint64_t copy_stride, StepPtrs p, uint32_t rows, uint4* __restrict__ table,
+                                                             const uint4* __restrict__ host_table, uint32_t table_pieces )
+{
+  __shared__ float s_next[16];
+  if ( blockIdx.x >= rows ) {
+    const uint32_t i = ( blockIdx.x - rows ) * blockDim.x + threadIdx.x;
+    if ( i < table_pieces ) {
+      table[i] = host_table[i];
+    }
+    return;
+  }
+  const uint64_t row = blockIdx.x;
+  const uint64_t token = min( tokens[row], vocab - 1 ); // rows without a context may hold anything
+  const E* e = embed + token * width;
+  const E* at = pos_table != nullptr ? pos_table + (uint64_t)min( start_pos[row / n_tokens] + (uint32_t)( row % n_tokens ), max_pos - 1 ) * width : nullptr;
+  uint32_t col[NV];
+  bool live[NV];
+  float4 v[NV];
+#pragma unroll
+  for ( int g = 0; g < NV; g++ ) { // a group past the row's end reads group 0 and stores nothing
+    const uint32_t c = ( g * blockDim.x + threadIdx.x ) * 4;
+    live[g] = c < width;
+    col[g] = live[g] ? c : 0;
+    v[g] = load4_e<E>( e, col[g] );
+  }
+  if ( at != nullptr ) {
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) {
+      const float4 a = load4_e<E>( at, col[g] );
+      v[g] = make_float4( v[g].x + a.x, v[g].y + a.y, v[g].z + a.z, v[g].w + a.w );
+    }
+  }
+#pragma unroll
+  for ( int g = 0; g < NV; g++ ) {
+    if ( live[g] ) {
+      *reinterpret_cast<float4*>( x + row * width + col[g] ) = v[g];
+      if ( copy != nullptr ) {
+        struct alignas( 4 * sizeof( E ) ) Four
+        {
+          E e[4];
+        };
+        *reinterpret_cast<Four*>( copy + row * copy_stride + col[g] ) = Four { { from_f32<E>( v[g].x ), from_f32<E>( v[g].y ), from_f32<E>( v[g].z ), from_f32<E>( v[g].w ) } };
+      }
+    }
+  }
+  step_out<E, NV>( v, col, live, row, width, p, s_next );
+}
+
+// Threads to a row of `groups` groups of four columns: many rows, fewer threads with more of the row each; few rows, the row over as many threads as it has groups.
+uint32_t step_threads( uint32_t groups, uint64_t rows )
+{
+  const uint32_t want = rows >= 1024 ? ( groups + 3 ) / 4 : groups;
+  return std::min<uint32_t>( 1024, std::max<uint32_t>( 64, ( want + 63 ) / 64 * 64 ) );
+}
+// go( NV ): the groups of a thread, at most 8
+template<typename F>
+void with_groups( uint32_t nv, F&& go )
+{
+  if ( nv <= 1 ) {
+    go( std::integral_constant<int, 1> {} );
+  } else if ( nv <= 2 ) {
+    go( std::integral_constant<int, 2> {} );
+  } else if ( nv <= 4 ) {
+    go( std::integral_constant<int, 4> {} );
+  } else {
+    go( std::integral_constant<int, 8> {} );
+  }
+}
+
 template<typename E, bool PRODUCT, typename View>
 int launch_step( float* x, const View& y, uint64_t width, uint64_t rows, const StepPtrs& p, hipStream_t st )
 {
@@ -255,19 +337,10 @@ int launch_step( float* x, const View& y, uint64_t width, uint64_t rows, const S
     return GH_OK;
   }
   const uint32_t groups = w / 4;
-  // many rows: fewer threads with more of the row each; few rows: the row over as many threads as it has groups
-  const uint32_t want = rows >= 1024 ? ( groups + 3 ) / 4 : groups;
-  uint32_t threads = std::min<uint32_t>( 1024, std::max<uint32_t>( 64, ( want + 63 ) / 64 * 64 ) );
-  const uint32_t nv = ( groups + threads - 1 ) / threads;
-  if ( nv <= 1 ) {
-    stream_step_kernel<E, View, PRODUCT, 1><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
-  } else if ( nv <= 2 ) {
-    stream_step_kernel<E, View, PRODUCT, 2><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
-  } else if ( nv <= 4 ) {
-    stream_step_kernel<E, View, PRODUCT, 4><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
-  } else {
-    stream_step_kernel<E, View, PRODUCT, 8><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
-  }
+  const uint32_t threads = step_threads( groups, rows );
+  with_groups( ( groups + threads - 1 ) / threads, [&]( auto nv ) {
+    stream_step_kernel<E, View, PRODUCT, decltype( nv )::value><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
+  } );
   GH_LAUNCH_CHECK();
   return GH_OK;
 }
@@ -341,6 +414,40 @@ __global__ __launch_bounds__( 256 ) void scale_rows_kernel( float* __restrict__ 
   }
 }
 
+// The same with the index of each row's maximum (the lowest of equal ones; 0 where the row begins with NaN, as in gh_argmax), one work-group a row.
+// Bound by latency; with a launch between the two 32 rows of 4096 took 4.7 + 4.1 us.  r % 4 == 0, 16-byte aligned rows
+__global__ __launch_bounds__( 1024 ) void scale_rows_argmax_kernel( float* __restrict__ out, uint32_t* __restrict__ best_out, ProductView<float> y, uint32_t r, float scale )
+{
+  __shared__ float s_val[1024 / WAVE];
+  __shared__ uint32_t s_idx[1024 / WAVE];
+  const uint64_t row = blockIdx.x;
+  const uint32_t pieces = r / 4;
+  float best = -INFINITY;
+  uint32_t best_i = 0xffffffffu;
+  bool unordered = false;
+  for ( uint32_t p0 = threadIdx.x; p0 < pieces; p0 += 2048 ) {
+    float4 v[2];
+#pragma unroll
+    for ( int u = 0; u < 2; u++ ) { // past the end: the last piece again, which changes nothing
+      v[u] = y.at4( row, 4 * min( p0 + 1024 * u, pieces - 1 ) );
+    }
+#pragma unroll
+    for ( int u = 0; u < 2; u++ ) {
+      const uint32_t c = 4 * min( p0 + 1024 * u, pieces - 1 );
+      const float s[4] = { v[u].x * scale, v[u].y * scale, v[u].z * scale, v[u].w * scale };
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        arg_better( best, best_i, s[e], c + e );
+      }
+      unordered |= c == 0 && s[0] != s[0];
+      *reinterpret_cast<float4*>( out + row * r + c ) = make_float4( s[0], s[1], s[2], s[3] );
+    }
+  }
+  if ( block_arg<1024>( best, best_i, s_val, s_idx ) ) {
+    best_out[row] = unordered || best_i == 0xffffffffu ? 0u : best_i;
+  }
+}
+
 unsigned grid_for( uint64_t items ) { return (unsigned)std::min<uint64_t>( std::max<uint64_t>( 1, ( items + 255 ) / 256 ), 16384 ); }
 
 // ---- gather of rows ----------------------------------------------------------------------------
@@ -380,6 +487,63 @@ int gh_embed_positions( float* x, const uint32_t* tokens_dev, const uint32_t* st
     const uint32_t threads = vec ? (uint32_t)std::min<uint64_t>( 256, ( width / 4 + 63 ) / 64 * 64 ) : 256;
     ( vec ? embed_positions4_kernel<E> : embed_positions_kernel<E> )<<<(unsigned)rows, threads, 0, as_stream( stream )>>>(
       x, tokens_dev, start_pos_dev, n_tokens, e, p, (uint32_t)width, (uint32_t)vocab, (uint32_t)max_pos, static_cast<E*>( copy ), copy_stride );
+  };
+  if ( dt == GH_F32 ) {
+    launch( float {} );
+  } else {
+    launch( __bf16 {} );
+  }
+  GH_LAUNCH_CHECK();
+  return GH_OK;
+}
+
+// Rows up to which the embedding reads its tokens and positions over the bus: one launch instead of an upload and another.  Beyond, each row's work-group waits
+// for the bus while the upload is a small part of the step.
+constexpr uint64_t EMBED_IN_PLACE_ROWS = 256;
+
+int gh_embed_step( float* x, void* table_dev, const void* table_host, uint64_t table_bytes, uint64_t tokens_at, uint64_t pos_at, uint64_t batch, uint32_t n_tokens,
+                   const void* embed, const void* pos_table, uint64_t width, uint64_t vocab, uint64_t max_pos, void* copy, uint64_t copy_stride,
+                   const gh_stream_step* step, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  const uint64_t rows = batch * n_tokens;
+  GH_REQUIRE( table_dev && table_host && tokens_at % 4 == 0 && pos_at % 4 == 0 && tokens_at + rows * 4 <= table_bytes && pos_at + batch * 4 <= table_bytes,
+              "gh_embed_step: the tables do not hold the step" );
+  GH_REQUIRE( dt == GH_BF16 || dt == GH_F32, "gh_embed_step: unsupported dtype %d", (int)dt );
+  if ( rows == 0 ) {
+    return gh_rows_in( nullptr, nullptr, nullptr, nullptr, 0, 0, table_dev, table_host, table_bytes, dt, stream );
+  }
+  GH_REQUIRE( x && embed && step && step->out && width > 0 && vocab > 0 && max_pos > 0, "gh_embed_step: bad argument" );
+  GH_REQUIRE( rows < ( 1ull << 31 ) && width < ( 1ull << 31 ), "gh_embed_step: too large" );
+  const StepPtrs p = step_ptrs( step );
+  const bool vec = width % 4 == 0 && width <= 32768 && p.out_stride % 4 == 0 && aligned16( x ) && aligned16( embed ) && aligned16( pos_table ) && aligned16( p.out )
+                   && aligned16( p.next_norm ) && copy_stride % 4 == 0 && aligned16( copy );
+  const bool in_place = vec && rows <= EMBED_IN_PLACE_ROWS && table_bytes <= ( 1ull << 20 ) && gh_host_in_place( table_host, table_dev, table_bytes ) == 1;
+  if ( !in_place ) {
+    if ( int rc = gh_rows_in( nullptr, nullptr, nullptr, nullptr, 0, 0, table_dev, table_host, table_bytes, dt, stream ) ) {
+      return rc;
+    }
+  }
+  const char* from = static_cast<const char*>( in_place ? table_host : table_dev );
+  const uint32_t *tokens = reinterpret_cast<const uint32_t*>( from + tokens_at ), *start_pos = reinterpret_cast<const uint32_t*>( from + pos_at );
+  if ( !vec ) {
+    if ( int rc = gh_embed_positions( x, tokens, start_pos, batch, n_tokens, embed, pos_table, width, vocab, max_pos, copy, copy_stride, dt, stream ) ) {
+      return rc;
+    }
+    return gh_stream_out( x, width, rows, step, dt, stream );
+  }
+  const uint32_t groups = (uint32_t)width / 4, threads = step_threads( groups, rows );
+  const uint32_t table_pieces = in_place ? (uint32_t)( table_bytes / 16 ) : 0;
+  const unsigned grid = (unsigned)( rows + ( table_pieces + threads - 1 ) / threads );
+  auto launch = [&]( auto tag ) {
+    using E = decltype( tag );
+    with_groups( ( groups + threads - 1 ) / threads, [&]( auto nv ) {
+      embed_step_kernel<E, decltype( nv )::value><<<grid, threads, 0, as_stream( stream )>>>(
+        x, tokens, start_pos, n_tokens, static_cast<const E*>( embed ), static_cast<const E*>( pos_table ), (uint32_t)width, (uint32_t)vocab, (uint32_t)max_pos,
+        static_cast<E*>( copy ), copy_stride, p, (uint32_t)rows, static_cast<uint4*>( table_dev ), static_cast<const uint4*>( table_host ), table_pieces );
+    } );
   };
   if ( dt == GH_F32 ) {
     launch( float {} );
@@ -500,6 +664,33 @@ int gh_matmul_scaled( float* out, const void* x, const void* w, uint64_t s, uint
   }
   const ProductView<float> view( y );
   scale_rows_kernel<<<grid_for( rows * r ), 256, 0, st>>>( out, view, (uint32_t)r, rows, scale );
+  GH_LAUNCH_CHECK();
+  return GH_OK;
+}
+
+int gh_matmul_scaled_argmax( float* out, uint32_t* argmax, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t rows, float scale, gh_dtype dt, gh_stream stream )
+{
+  if ( int rc = ensure_init() ) {
+    return rc;
+  }
+  if ( rows == 0 ) {
+    return GH_OK;
+  }
+  GH_REQUIRE( out && argmax && x && w, "gh_matmul_scaled_argmax: NULL pointer" );
+  GH_REQUIRE( s > 0 && s < ( 1ull << 31 ) && r > 0 && r < ( 1ull << 31 ) && rows < ( 1ull << 31 ), "gh_matmul_scaled_argmax: bad shape" );
+  GH_REQUIRE( dt == GH_BF16 || dt == GH_F32, "gh_matmul_scaled_argmax: unsupported dtype %d", (int)dt );
+  if ( r % 4 != 0 || !aligned16( out ) ) {
+    if ( int rc = gh_matmul_scaled( out, x, w, s, r, rows, scale, dt, stream ) ) {
+      return rc;
+    }
+    return gh_argmax( nullptr, argmax, out, r, rows, GH_F32, stream );
+  }
+  hipStream_t st = as_stream( stream );
+  Product y;
+  if ( int rc = make_product( x, w, s, r, rows, dt, true, st, &y ) ) {
+    return rc;
+  }
+  scale_rows_argmax_kernel<<<(unsigned)rows, 1024, 0, st>>>( out, argmax, ProductView<float>( y ), (uint32_t)r, scale );
   GH_LAUNCH_CHECK();
   return GH_OK;
 }

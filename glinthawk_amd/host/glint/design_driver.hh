@@ -195,20 +195,20 @@ public:
       put_context( i, *contexts[i], live ? states.token_pos( i ) : 0, 1 );
       table_tokens()[i] = live ? states.token( i ) : 0;
     }
-    upload_tables();
-    spans_.mark( 0, ops_.stream() );
-    run_layers( batch, 1, true, nullptr );
-    classify( batch );
-    spans_.mark( 1, ops_.stream() );
-
     std::vector<float> temperatures;
     for ( size_t i = 0; i < batch; i++ ) {
       temperatures.push_back( states.temperature( i ) );
     }
-    if ( std::any_of( temperatures.begin(), temperatures.end(), []( float t ) { return t > 0; } ) ) {
+    const bool greedy = std::none_of( temperatures.begin(), temperatures.end(), []( float t ) { return t > 0; } );
+    spans_.mark( 0, ops_.stream() );
+    run_layers( batch, 1, true, nullptr );
+    classify( batch, greedy );
+    spans_.mark( 1, ops_.stream() );
+    if ( !greedy ) {
       logit_ops_.soft_sample( logits_.get(), temperatures, sizes_.vocab );
+      sample( batch );
     }
-    sample( batch );
+    ops_.synchronize();
     spans_.close();
     states.set_next_layer( 0 );
     states.set_next_stage( InferenceStage::PreAttention );
@@ -262,7 +262,6 @@ public:
       GLINT_CHECK( picked[k] < rows );
       table_picked()[k] = picked[k];
     }
-    upload_tables();
     run_layers( batch, n_tokens, false, residuals_out );
     // the wanted rows, at most LOGIT_ROWS of them at a time
     for ( size_t k = 0; k < picked.size(); k += LOGIT_ROWS ) {
@@ -271,13 +270,13 @@ public:
       gh_stream_step step = no_step();
       lead_out( step );
       GLINT_GH( gh_stream_out( picked_x_.get(), sizes_.width, n, &step, DT, ops_.stream() ) );
-      classify( n );
+      classify( n, k + n > want.size() );
       const size_t plain = k < want.size() ? std::min( n, want.size() - k ) : 0;
       if ( plain > 0 ) {
         logit_ops_.copy( logits_out + k * sizes_.vocab, logits_.get(), plain * sizes_.vocab * sizeof( float ), CopyType::DeviceToHost );
       }
       if ( plain < n ) {
-        sample( n );
+        ops_.synchronize();
         for ( size_t j = plain; j < n; j++ ) {
           next_tokens[k + j - want.size()] = argmax_[j];
         }
@@ -339,11 +338,11 @@ protected:
   virtual void lay_out( WeightCursor<DType>& cursor ) = 0;
   // scratch of the layers for steps of up to `rows` rows; the device is idle
   virtual void allocate_layer_scratch( uint64_t rows ) = 0;
-  // embedding and all layers, over the tables of this step; `all_rows_classified`: the output's norm of every row ends up in h.
+  // embedding (start_step) and all layers, over the tables of this step; `all_rows_classified`: the output's norm of every row ends up in h.
   // residuals_out as prefill()'s
   virtual void run_layers( uint64_t batch, uint32_t n_tokens, bool all_rows_classified, float* residuals_out ) = 0;
-  // logits of the first n rows of h
-  virtual void classify( uint64_t n ) = 0;
+  // the output's matrix and what its product is scaled with
+  virtual std::pair<const DType*, float> head() const = 0;
   // tensors that are not copied as they are
   virtual std::string load_tables( const SafeTensors& ) { return {}; }
   virtual void randomize_tables( uint64_t ) {}
@@ -404,10 +403,23 @@ protected:
     reinterpret_cast<uint32_t*>( tables_host_ + pos_off() )[i] = pos;
     max_start_ = std::max( max_start_, pos );
   }
-  void upload_tables()
+  // the step's tables to the device, its embeddings to the stream and, by `first`, to what the first product reads
+  void start_step( const uint64_t batch, const uint32_t n_tokens, const DType* embed, const DType* positions, const uint64_t max_positions, DType* copy,
+                   const uint64_t copy_stride, const gh_stream_step& first )
   {
     const uint64_t bytes = ( picked_off() + t_picked_ * sizeof( uint32_t ) + 15 ) / 16 * 16; // (there is room: grow_tables)
-    GLINT_GH( gh_rows_in( nullptr, nullptr, nullptr, nullptr, 0, 0, tables_dev_.get(), tables_host_, bytes, DT, ops_.stream() ) );
+    GLINT_GH( gh_embed_step( x_.get(), tables_dev_.get(), tables_host_, bytes, tokens_off(), pos_off(), batch, n_tokens, embed, positions, sizes_.width, sizes_.vocab,
+                             max_positions, copy, copy_stride, &first, DT, ops_.stream() ) );
+  }
+  // logits of the first n rows of h; `greedy`: each row's likeliest token with them, to the host (there once the stream is done)
+  void classify( const uint64_t n, const bool greedy )
+  {
+    const auto [weights, scale] = head();
+    if ( greedy ) {
+      GLINT_GH( gh_matmul_scaled_argmax( logits_.get(), argmax_.get(), h_.get(), weights, sizes_.width, sizes_.vocab, n, scale, DT, ops_.stream() ) );
+    } else {
+      GLINT_GH( gh_matmul_scaled( logits_.get(), h_.get(), weights, sizes_.width, sizes_.vocab, n, scale, DT, ops_.stream() ) );
+    }
   }
   const uint8_t* dev() const { return reinterpret_cast<const uint8_t*>( tables_dev_.get() ); }
   void* const* contexts_dev() const { return reinterpret_cast<void* const*>( tables_dev_.get() ); }
@@ -437,12 +449,8 @@ protected:
       logit_ops_.copy( out + run * rows * sizes_.width, x_.get(), rows * sizes_.width * sizeof( float ), CopyType::DeviceToHost );
     }
   }
-  // greedy token of the first n rows of the logits, on the host: the kernel writes them there itself
-  void sample( const uint64_t n )
-  {
-    GLINT_GH( gh_argmax( nullptr, argmax_.get(), logits_.get(), sizes_.vocab, n, GH_F32, ops_.stream() ) );
-    ops_.synchronize();
-  }
+  // greedy token of the first n rows of the logits as they are now, likewise
+  void sample( const uint64_t n ) { GLINT_GH( gh_argmax( nullptr, argmax_.get(), logits_.get(), sizes_.vocab, n, GH_F32, ops_.stream() ) ); }
 
   Sizes sizes_;
   SettingsType settings_;

@@ -125,11 +125,10 @@ private:
   {
     const uint64_t rows = batch * n_tokens, width = config_.width;
     const gh_stream stream = ops_.stream();
-    GLINT_GH( gh_embed_positions( x_.get(), tokens_dev(), pos_dev(), batch, n_tokens, embed_, nullptr, width, config_.vocab, 1, nullptr, 0, DT, stream ) );
     {
       gh_stream_step first = no_step();
       lead_to( first, layers_[0].norm1 );
-      GLINT_GH( gh_stream_out( x_.get(), width, rows, &first, DT, stream ) );
+      this->start_step( batch, n_tokens, embed_, nullptr, 1, nullptr, 0, first );
     }
     for ( size_t l = 0; l < layers_.size(); l++ ) {
       const auto& w = layers_[l];
@@ -150,10 +149,7 @@ private:
     }
   }
 
-  void classify( const uint64_t n ) override
-  {
-    GLINT_GH( gh_matmul_scaled( this->logits_.get(), h_.get(), head_, config_.width, config_.vocab, n, 1.0f, DT, ops_.stream() ) );
-  }
+  std::pair<const DType*, float> head() const override { return { head_, 1.0f }; }
 
   DirozenConfig config_;
   std::vector<Layer> layers_ {};

@@ -233,12 +233,10 @@ private:
     const uint64_t rows = batch * n_tokens, width = config_.width;
     const gh_stream stream = ops_.stream();
     DType* x0 = config_.looped ? cat_.get() + width : nullptr;
-    GLINT_GH( gh_embed_positions( x_.get(), tokens_dev(), pos_dev(), batch, n_tokens, embed_, pos_, width, config_.vocab, config_.max_positions, x0, 2 * width, DT,
-                                  stream ) );
     {
       gh_stream_step first = no_step();
       lead_into( first, 0, all_rows_classified );
-      GLINT_GH( gh_stream_out( x_.get(), width, rows, &first, DT, stream ) );
+      this->start_step( batch, n_tokens, embed_, pos_, config_.max_positions, x0, 2 * width, first );
     }
     for ( size_t k = 0; k < runs_.size(); k++ ) {
       const auto& run = runs_[k];
@@ -283,10 +281,7 @@ private:
     }
   }
 
-  void classify( const uint64_t n ) override
-  {
-    GLINT_GH( gh_matmul_scaled( this->logits_.get(), h_.get(), embed_, config_.width, config_.vocab, n, config_.logit_scale, DT, ops_.stream() ) );
-  }
+  std::pair<const DType*, float> head() const override { return { embed_, config_.logit_scale }; }
 
   FamidraConfig config_;
   std::vector<FamidraConfig::Run> runs_;

@@ -465,6 +465,24 @@ def matmul_scaled(x, w, scale: float):
     return out
 
 
+def embed_step(table_dev, table_host, tokens_at: int, pos_at: int, batch: int, n_tokens: int, embed, out, pos_table=None, copy=None, next_norm=None,
+               eps: float = 1e-5, norm_base: float = 0.0):
+    """table_host: the step's tables as bytes (pinned_empty: read in place), uploaded to table_dev.  Returns the stream; `out` receives the rows normed."""
+    s = _stream_step(eps, next_norm=next_norm, out=out, norm_base=norm_base)
+    x = torch.empty((batch * n_tokens, embed.shape[1]), dtype=torch.float32, device=embed.device)
+    check(lib().gh_embed_step(_p(x), _p(table_dev), table_host.ctypes.data, table_host.nbytes, tokens_at, pos_at, batch, n_tokens, _p(embed), _p(pos_table),
+                              embed.shape[1], embed.shape[0], 1 if pos_table is None else pos_table.shape[0], None if copy is None else copy.data_ptr(),
+                              0 if copy is None else copy.stride(0), C.byref(s), _dt(embed), _stream()), "gh_embed_step")
+    return x
+
+
+def matmul_scaled_argmax(x, w, scale: float):
+    out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
+    best = torch.empty((x.shape[0],), dtype=torch.int32, device=x.device)
+    check(lib().gh_matmul_scaled_argmax(_p(out), _p(best), _p(x), _p(w), x.shape[1], w.shape[0], x.shape[0], scale, _dt(x), _stream()), "gh_matmul_scaled_argmax")
+    return out, best
+
+
 def window_attn(heads, kv_heads, dim, vdim, scale, window=0, keep_first=0, n_dist=0, values_are_keys=False) -> GhWindowAttn:
     return GhWindowAttn(heads, kv_heads, dim, vdim, window, keep_first, n_dist, scale, int(values_are_keys))
 

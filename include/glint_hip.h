@@ -398,6 +398,11 @@ typedef struct gh_stream_step
   int accumulate;
   float norm_base;
 } gh_stream_step;
+/* gh_rows_in of a step's tables (page-locked, read where they lie for few rows), gh_embed_positions with the tokens at byte tokens_at and the start positions at
+ * byte pos_at of them, gh_stream_out of the rows: the same results in one or two launches */
+int gh_embed_step( float* x, void* table_dev, const void* table_host, uint64_t table_bytes, uint64_t tokens_at, uint64_t pos_at, uint64_t batch, uint32_t n_tokens,
+                   const void* embed, const void* pos_table, uint64_t width, uint64_t vocab, uint64_t max_pos, void* copy, uint64_t copy_stride,
+                   const gh_stream_step* step, gh_dtype dt, gh_stream stream );
 /* y = in (rows, s) . w (width, s)^T */
 int gh_matmul_stream( float* x, const void* in, const void* w, uint64_t s, uint64_t width, uint64_t rows, const gh_stream_step* step, gh_dtype dt,
                       gh_stream stream );
@@ -408,6 +413,9 @@ int gh_matmul_gate( void* hb, const void* x, const void* w_gate_up, const void* 
                     gh_stream stream );
 /* out (fp32) = (x . w^T) * scale */
 int gh_matmul_scaled( float* out, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t rows, float scale, gh_dtype dt, gh_stream stream );
+/* the same, with the index of each row's maximum as gh_argmax gives it; argmax (rows) may be page-locked host memory */
+int gh_matmul_scaled_argmax( float* out, uint32_t* argmax, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t rows, float scale, gh_dtype dt,
+                             gh_stream stream );
 /* out(i) = x(rows_dev[i]), n rows out of n_rows */
 int gh_gather_rows( float* out, const float* x, const uint32_t* rows_dev, uint64_t n, uint64_t n_rows, uint64_t width, gh_stream stream );
 

@@ -130,6 +130,55 @@ def test_embedding():
     assert np.array_equal(x.cpu().numpy().reshape(2, 5, 20), want) and np.array_equal(copy[:, 20:].cpu().numpy(), x.cpu().numpy())
 
 
+# threads of a row with one, two, four and eight groups of columns, a row that ends inside them, widths that are not of fours; read in place, uploaded, or pageable
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,batch,n_tokens,pinned", [(4096, 3, 1, True), (288, 5, 1, True), (4100, 2, 7, True), (16388, 1, 2, True), (32768, 2, 1, False), (30, 4, 1, True),
+                                                         (64, 256, 1, True), (64, 257, 1, True), (1028, 2, 600, True)])
+def test_start_of_a_step(dtype, width, batch, n_tokens, pinned):
+    """As the upload, the embedding and the norm one by one: the same bits but for the norm, whose sums of squares may be contracted otherwise (some 2^-22)."""
+    import torch
+    from glinthawk_amd import ops
+    g, rows = torch.Generator(device="cuda").manual_seed(width), batch * n_tokens
+    e, p, nw = (torch.randn(s, generator=g, device="cuda").to(torch_dtype(dtype)) for s in ((50, width), (700, width), (width,)))
+    size = (rows + batch) * 4 + 12
+    host = ops.pinned_empty((size // 16 * 16,), np.uint8) if pinned else np.empty((size // 16 * 16,), np.uint8)
+    words, rng = host.view(np.int32), np.random.default_rng(width)
+    words[:] = 0
+    words[:batch], words[batch: batch + rows] = rng.integers(0, 80, batch), rng.integers(0, 50, rows)
+    words[batch] = 1000                      # a row without a context may hold anything
+    for pos, copied, norm, base in ((p, True, nw, 0.0), (None, False, nw, 1.0), (p, True, None, 0.0)):
+        copies = [torch.zeros((rows, 2 * width), device="cuda", dtype=torch_dtype(dtype)) for _ in range(2)]
+        outs = [torch.zeros((rows, width), device="cuda", dtype=torch_dtype(dtype)) for _ in range(2)]
+        table = torch.zeros(host.shape, dtype=torch.uint8, device="cuda")
+        got = ops.embed_step(table, host, 4 * batch, 0, batch, n_tokens, e, outs[0], pos, copies[0][:, width:] if copied else None, norm, 1e-5, base)
+        torch.cuda.synchronize()
+        assert np.array_equal(table.cpu().numpy(), host)
+        on_device = torch.from_numpy(words.copy()).cuda()
+        want = ops.embed_positions(on_device[batch: batch + rows].contiguous(), on_device[:batch].contiguous(), n_tokens, e, pos, copies[1][:, width:] if copied else None)
+        ops.stream_out(want, outs[1], norm, 1e-5, base)
+        assert torch.equal(got, want) and torch.equal(copies[0], copies[1])
+        tol = 2.0 ** -8 if dtype == "bf16" else 1e-6    # one unit in the last place of bf16
+        assert torch.allclose(outs[0].float(), outs[1].float(), rtol=tol, atol=0.0)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,s,r", [(32, 4096, 4096), (1, 64, 4), (3, 100, 36), (5, 256, 8196), (2, 64, 32000), (200, 128, 1000), (4, 64, 30)])
+def test_scaled_product_with_its_argmax(dtype, rows, s, r):
+    """The same bits as the product and the argmax one after the other: ties, NaN first and elsewhere, rows of -inf."""
+    import torch
+    from glinthawk_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(r)
+    x, w = (torch.randn(shape, generator=g, device="cuda").to(torch_dtype(dtype)) for shape in ((rows, s), (r, s)))
+    w[r // 2] = w[r - 1]
+    if rows > 2:
+        w[0, 0], x[0, 0], x[1, 1:], x[2] = float("inf"), 0.0, 0.0, -float("inf")   # NaN at column 0; +-inf or 0; -inf, inf and NaN
+        w[r // 3, 0] = float("inf")
+    logits, best = ops.matmul_scaled_argmax(x, w, 0.5)
+    want = ops.matmul_scaled(x, w, 0.5)
+    assert torch.equal(logits.view(torch.int32), want.view(torch.int32))
+    assert best.tolist() == ops.argmax(want)
+
+
 ATTENTIONS = {
     # heads, kv heads, dim, vdim, window, kept, table rows, bias_max
     "grouped": (6, 2, 24, 16, 11, 3, 10, 40),
