@@ -13,6 +13,7 @@
 #include "gh_window.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace gh {
 namespace {
@@ -1104,6 +1105,196 @@ __global__ __launch_bounds__( 64 * NW, SHARED ? 4 : 2 ) void window_decode_kerne
   finish_split<__bf16, NW / HB, 64 * NW>( out, partial, results, HB * head_cols, HB * head_cols, row, hb * HB * head_cols, split, splits, s );
 }
 
+// ---- few tokens of heads that share their keys with no other: dot products in the vector ALU -------------------------------------
+//
+// With one query head to a kv head the matrix cores above would multiply one column of sixteen, and a tile's way there is through LDS.  Here 16 lanes hold one
+// key, eight elements a lane, straight from memory, and the vector ALU keeps up with it.  A wave walks a range of the visible keys in tiles of
+// 4 U, from one of its own on (work-groups in step on rows a power of two apart meet on few channels), the next tile under way; lane c of a row of lanes owns the
+// score of key c % U, so that a tile is one exponential.  Scores, weights and sums are fp32, and the weights enter the sums whole.
+// Bound by memory, and by the vector ALU next: with the products of the scores unpacked to fp32, where v_dot2_f32_bf16 takes two at a time, values that are keys
+// took 49.5 us instead of 43.5 at 32 contexts x 32 heads x 1025 keys (6.2 TB/s; 46.6 by the kernel above), K and V apart 87.2 instead of 84.9 (6.3; 92.2).
+typedef __bf16 bf16x2_t __attribute__( ( ext_vector_type( 2 ) ) );
+template<bool SHARED, int NW, int HB>
+__global__ __launch_bounds__( 64 * NW, 4 ) void window_dot_kernel( WindowOut<__bf16> out,
+                                                                   float* __restrict__ partial,
+                                                                   const __bf16* __restrict__ q,
+                                                                   const float* __restrict__ bias,
+                                                                   WindowRows wr,
+                                                                   WindowShape s,
+                                                                   uint32_t keys_per_split,
+                                                                   uint32_t splits )
+{
+  constexpr int U = SHARED ? 8 : 4; // keys of a row of lanes in a tile: 8 KB of a wave either way
+  constexpr uint32_t TILE = 4 * U;
+  __shared__ float results[NW * ( 128 + 2 )];
+  const uint32_t head_blocks = s.heads / HB, hb = blockIdx.x % head_blocks, split = blockIdx.x / head_blocks % splits;
+  const uint64_t row = blockIdx.x / head_blocks / splits;
+  const uint32_t ctx = (uint32_t)( row / wr.n_tokens ), tok = (uint32_t)( row % wr.n_tokens );
+  const uint8_t* base = static_cast<const uint8_t*>( wr.rows[ctx] );
+  const uint32_t pos = wr.start_pos[ctx] + tok; // (read before the branch: one round trip for the two)
+  if ( base == nullptr ) {
+    return;
+  }
+  const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63, r = lane >> 4, c = lane & 15;
+  const uint32_t head = hb * HB + wave % HB, turn = wave / HB;
+  const Visible vis = visible_keys( pos, s );
+  const uint32_t s_begin = split * keys_per_split, s_end = min( vis.count, s_begin + keys_per_split );
+  const uint32_t s_keys = s_end > s_begin ? s_end - s_begin : 0;
+  const uint32_t per_wave = ( s_keys + NW / HB * TILE - 1 ) / ( NW / HB * TILE ) * TILE;
+  const uint32_t k_begin = s_begin + turn * per_wave, k_end = min( s_end, k_begin + per_wave );
+
+  const char* cache = reinterpret_cast<const char*>( base + wr.offset );
+  const uint32_t row_bytes = s.row_elems() * sizeof( __bf16 );
+  const bool k_chunk = c * 8 < s.dpad, v_chunk = c * 8 < s.vpad;
+  const uint32_t at_k = ( head * s.dpad + c * 8 ) * sizeof( __bf16 ), at_v = ( s.k_elems() + head * s.vpad + c * 8 ) * sizeof( __bf16 );
+  const float* factors = reinterpret_cast<const float*>( base + wr.factors );
+  u32x4_t qr = { 0, 0, 0, 0 };
+  if ( k_chunk ) {
+    qr = *(global_u32x4_t*)( q + ( row * s.heads + head ) * s.dpad + c * 8 );
+  }
+
+  u32x4_t kn[U], vn[SHARED ? 1 : U]; // chunks beyond a head's size stay zero
+#pragma unroll
+  for ( int j = 0; j < U; j++ ) {
+    kn[j] = u32x4_t { 0, 0, 0, 0 };
+    vn[SHARED ? 0 : j] = u32x4_t { 0, 0, 0, 0 };
+  }
+  float fn = 0.0f;
+  const uint32_t own = 4 * ( c % U ) + r; // key of the tile whose score is this lane's
+  auto load_row = [&]( int j, const char* key_row, uint32_t off ) __attribute__( ( always_inline ) ) {
+    if ( k_chunk ) {
+      kn[j] = __builtin_nontemporal_load( (global_u32x4_t*)( key_row + ( off + at_k ) ) );
+    }
+    if constexpr ( !SHARED ) {
+      if ( v_chunk ) {
+        vn[j] = __builtin_nontemporal_load( (global_u32x4_t*)( key_row + ( off + at_v ) ) );
+      }
+    }
+  };
+  auto load = [&]( uint32_t i0 ) __attribute__( ( always_inline ) ) {
+    if constexpr ( SHARED ) {
+      fn = factors[factor_index( vis.key( min( i0 + own, k_end - 1 ) ), head, s.kv_heads )];
+    }
+    if ( i0 + TILE <= k_end && ( i0 >= vis.kept || i0 + TILE <= vis.kept ) ) { // neighbouring rows: one address for the wave
+      const char* tile = cache + (uint64_t)vis.key( i0 ) * row_bytes;
+#pragma unroll
+      for ( int j = 0; j < U; j++ ) {
+        load_row( j, tile + 4 * j * row_bytes, r * row_bytes );
+      }
+    } else {
+#pragma unroll
+      for ( int j = 0; j < U; j++ ) { // past the end: the last key again, without weight
+        load_row( j, cache + (uint64_t)vis.key( min( i0 + 4 * j + r, k_end - 1 ) ) * row_bytes, 0 );
+      }
+    }
+  };
+  const float scale_log2e = s.scale * LOG2E;
+  const float* my_bias = bias != nullptr ? bias + (uint64_t)head * s.n_dist : nullptr;
+  const float far_bias = bias != nullptr ? my_bias[s.n_dist - 1] * LOG2E : 0.0f;
+
+  float acc[8];
+#pragma unroll
+  for ( int e = 0; e < 8; e++ ) {
+    acc[e] = 0.0f;
+  }
+  float m = NO_KEY, l = 0.0f; // m: of a row of lanes; l: of this lane's keys
+  const uint32_t n_tiles = k_begin < k_end ? ( k_end - k_begin + TILE - 1 ) / TILE : 0;
+  uint32_t i0 = n_tiles > 0 ? k_begin + (uint32_t)( ( row * 5 + turn * 3 ) * 7 ) % n_tiles * TILE : 0;
+  if ( n_tiles > 0 ) {
+    load( i0 );
+  }
+  for ( uint32_t n = 0; n < n_tiles; n++ ) {
+    const uint32_t next = i0 + TILE < k_end ? i0 + TILE : k_begin;
+    u32x4_t kc[U], vc[SHARED ? 1 : U];
+#pragma unroll
+    for ( int j = 0; j < U; j++ ) {
+      kc[j] = kn[j];
+      vc[SHARED ? 0 : j] = vn[SHARED ? 0 : j];
+    }
+    const float f = SHARED ? fn * scale_log2e : scale_log2e;
+    if ( n + 1 < n_tiles ) {
+      load( next );
+    }
+    auto unpacked = []( u32x4_t raw, float( &v )[8] ) __attribute__( ( always_inline ) ) {
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        v[2 * e] = __builtin_bit_cast( float, raw[e] << 16 );
+        v[2 * e + 1] = __builtin_bit_cast( float, raw[e] & 0xffff0000u );
+      }
+    };
+    float sc = 0.0f;
+#pragma unroll
+    for ( int j = 0; j < U; j++ ) {
+      float dot = 0.0f;
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        const uint32_t kw = kc[j][e], qw = qr[e];
+        dot = __builtin_amdgcn_fdot2_f32_bf16( __builtin_bit_cast( bf16x2_t, kw ), __builtin_bit_cast( bf16x2_t, qw ), dot, false );
+      }
+      dot = row16_sum( dot );
+      sc = j == 0 || c % U == (uint32_t)j ? dot : sc;
+    }
+    sc *= f;
+    if ( bias != nullptr ) {
+      // every distance of the tile in the bias table's last row?
+      const uint32_t nearest = vis.key( min( i0 + TILE, k_end ) - 1 );
+      sc += pos - nearest >= s.n_dist - 1 ? far_bias : my_bias[min( pos - vis.key( min( i0 + own, k_end - 1 ) ), s.n_dist - 1 )] * LOG2E;
+    }
+    sc = i0 + own < k_end ? sc : -INFINITY;
+    const float mx = row16_max( sc );
+    if ( __builtin_amdgcn_ballot_w64( mx > m + LAZY ) != 0 ) {
+      const float m_new = fmaxf( m, mx );
+      const float alpha = __builtin_amdgcn_exp2f( m - m_new );
+      m = m_new;
+      l *= alpha;
+#pragma unroll
+      for ( int e = 0; e < 8; e++ ) {
+        acc[e] *= alpha;
+      }
+    }
+    const float p = __builtin_amdgcn_exp2f( sc - m );
+    l += c < U ? p : 0.0f;
+    auto add = [&]( auto j ) __attribute__( ( always_inline ) ) {
+      constexpr int J = decltype( j )::value;
+      float v8[8];
+      unpacked( SHARED ? kc[J] : vc[SHARED ? 0 : J], v8 );
+      const float pj = __builtin_bit_cast( float, __builtin_amdgcn_update_dpp( 0, __builtin_bit_cast( int, p ), 0x150 + J, 0xF, 0xF, true ) ); // lane J of the row
+#pragma unroll
+      for ( int e = 0; e < 8; e++ ) {
+        acc[e] += pj * v8[e];
+      }
+    };
+    add( std::integral_constant<int, 0> {} ), add( std::integral_constant<int, 1> {} ), add( std::integral_constant<int, 2> {} ), add( std::integral_constant<int, 3> {} );
+    if constexpr ( U == 8 ) {
+      add( std::integral_constant<int, 4> {} ), add( std::integral_constant<int, 5> {} ), add( std::integral_constant<int, 6> {} ), add( std::integral_constant<int, 7> {} );
+    }
+    i0 = next;
+  }
+  // the rows of lanes added up against the wave's maximum: lane (r, c) ends up with elements 8 c + r and 8 c + 4 + r
+  const float m_all = column_max( m ), f = __builtin_amdgcn_exp2f( m - m_all );
+  l = row16_sum( l ) * f;
+  l = ( lane_value( l, 0 ) + lane_value( l, 16 ) ) + ( lane_value( l, 32 ) + lane_value( l, 48 ) );
+#pragma unroll
+  for ( int e = 0; e < 8; e++ ) {
+    acc[e] *= f;
+  }
+  float* mine = results + wave * ( s.vpad + 2 );
+#pragma unroll
+  for ( int k = 0; k < 2; k++ ) {
+    const float sum = sum_rows( sum_halves( acc[4 * k], acc[4 * k + 2] ), sum_halves( acc[4 * k + 1], acc[4 * k + 3] ) );
+    const uint32_t d = 8 * c + 4 * k + r;
+    if ( d < s.vpad ) {
+      mine[d] = sum;
+    }
+  }
+  if ( lane == 0 ) {
+    mine[s.vpad] = l;
+    mine[s.vpad + 1] = m_all * ( 1.0f / LOG2E ); // the sums are joined in natural units
+  }
+  __syncthreads();
+  finish_split<__bf16, NW / HB, 64 * NW>( out, partial, results, HB, HB, row, hb * HB, split, splits, s );
+}
+
 template<typename E, int NC, bool SHARED>
 void launch_rows( int hq, dim3 grid, hipStream_t st, const WindowOut<E>& out, float* partial, const E* q, const float* bias, const WindowRows& wr, const WindowShape& s,
                   uint32_t keys_per_split, uint32_t splits )
@@ -1135,11 +1326,8 @@ struct SplitPlan
   uint32_t keys { 0 }, splits { 1 };
   float* partial { nullptr };
 };
-int plan_splits( const WindowShape& s, uint64_t rows, uint64_t head_blocks, uint32_t max_pos, uint64_t least, hipStream_t st, SplitPlan* plan )
+int cut_keys( const WindowShape& s, uint64_t rows, uint64_t most, uint64_t splits, hipStream_t st, SplitPlan* plan )
 {
-  const uint64_t most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
-  uint64_t splits = std::max<uint64_t>( 1, 2ull * cu_count() / std::max<uint64_t>( 1, rows * head_blocks ) );
-  splits = std::min( { splits, std::max<uint64_t>( 1, most / least ), (uint64_t)64 } );
   plan->keys = (uint32_t)( ( ( most + splits - 1 ) / splits + 31 ) / 32 * 32 );
   plan->splits = (uint32_t)( ( most + plan->keys - 1 ) / plan->keys );
   if ( plan->splits > 1 ) {
@@ -1150,6 +1338,12 @@ int plan_splits( const WindowShape& s, uint64_t rows, uint64_t head_blocks, uint
     plan->partial = static_cast<float*>( p );
   }
   return GH_OK;
+}
+int plan_splits( const WindowShape& s, uint64_t rows, uint64_t head_blocks, uint32_t max_pos, uint64_t least, hipStream_t st, SplitPlan* plan )
+{
+  const uint64_t most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
+  const uint64_t splits = std::max<uint64_t>( 1, 2ull * cu_count() / std::max<uint64_t>( 1, rows * head_blocks ) );
+  return cut_keys( s, rows, most, std::min( { splits, std::max<uint64_t>( 1, most / least ), (uint64_t)64 } ), st, plan );
 }
 template<typename E>
 int merge_splits( const WindowOut<E>& out, const SplitPlan& plan, const WindowRows& wr, const WindowShape& s, uint64_t rows, hipStream_t st )
@@ -1162,9 +1356,66 @@ int merge_splits( const WindowOut<E>& out, const SplitPlan& plan, const WindowRo
   return GH_OK;
 }
 
+// Few rows of bf16 whose query heads have a kv head each, of 65 to 128.  us, 32 heads of 128, against window_decode_kernel, K and V apart | values that are keys:
+//   1 row    1025 keys 13.9 -> 11.7, 4097 25.7 -> 18.5 | 11.7 -> 10.1, 16.5 -> 14.0
+//   8 rows    300 13.4 -> 10.9, 1025 31.9 -> 25.4, 4097 91 -> 85 | 9.5 -> 8.6, 20.6 -> 15.1, 52 -> 46
+//   16 rows  1025 50 -> 45, 4097 170 -> 158 | 26.7 -> 24.8, 88 -> 81
+//   32 rows    64 10.7 -> 9.2, 1025 91 -> 84, 4097 325 -> 317 | 8.2 -> 6.8, 45.5 -> 44.4, 169 -> 164
+//   48 rows   300 48.5 -> 38.5, 1025 129 -> 122 | 25.1 -> 22.2, 65 -> 64
+// What counts is the waves on the chip, some 4 to 8 a CU, and that work-groups come out even over the CUs; beyond that neighbouring heads in a work-group, which read
+// neighbouring pieces of a cache row.  So eight waves, on one head while there are no more streams of keys than CUs (cut further where that leaves CUs idle and a stream
+// is long: the merge is a launch), on two heads up to twice as many and on four up to four times.
+int attend_dot( const WindowOut<__bf16>& out, const __bf16* q, const float* bias, const WindowRows& wr, const WindowShape& s, uint64_t rows, uint32_t max_pos, hipStream_t st )
+{
+  const uint64_t most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
+  const uint64_t streams = rows * s.heads, cus = (uint64_t)cu_count();
+  uint32_t waves = 8, heads = streams <= cus ? 1 : streams <= 2 * cus ? 2 : streams <= 4 * cus ? 4 : 2;
+  // (16 rows of 4097 keys 163 | 84.7 us with four ranges of a head's keys, 158 | 81.1 with two; 48 rows of 64 13.4 | 9.7 and 11.3 | 7.6)
+  if ( heads == 2 && ( streams <= 2 * cus ? most > 3072 : most <= 192 ) ) {
+    waves = 4;
+  }
+  while ( s.heads % heads != 0 ) {
+    heads /= 2;
+  }
+  uint64_t splits = 1;
+  if ( const uint64_t idle = cus / streams; idle >= 2 && most * ( s.values_are_keys ? 1 : 2 ) >= ( idle >= 4 ? 1024u : 2048u ) ) {
+    splits = std::min( { idle, most / 64, (uint64_t)64 } );
+  }
+  SplitPlan plan;
+  if ( int rc = cut_keys( s, rows, most, splits, st, &plan ) ) {
+    return rc;
+  }
+  const uint64_t grid = streams / heads * plan.splits;
+  GH_REQUIRE( grid < ( 1ull << 31 ), "gh_attn_window: grid too large" );
+  auto launch = [&]( auto nw, auto hb ) {
+    constexpr int NW = decltype( nw )::value, HB = decltype( hb )::value;
+    if ( s.values_are_keys ) {
+      window_dot_kernel<true, NW, HB><<<(unsigned)grid, 64 * NW, 0, st>>>( out, plan.partial, q, bias, wr, s, plan.keys, plan.splits );
+    } else {
+      window_dot_kernel<false, NW, HB><<<(unsigned)grid, 64 * NW, 0, st>>>( out, plan.partial, q, bias, wr, s, plan.keys, plan.splits );
+    }
+  };
+  const std::integral_constant<int, 4> four {};
+  const std::integral_constant<int, 8> eight {};
+  const std::integral_constant<int, 2> two {};
+  const std::integral_constant<int, 1> one {};
+  if ( heads == 4 ) {
+    launch( eight, four );
+  } else if ( heads == 2 ) {
+    waves == 4 ? launch( four, two ) : launch( eight, two );
+  } else {
+    launch( eight, one );
+  }
+  GH_LAUNCH_CHECK();
+  return merge_splits( out, plan, wr, s, rows, st );
+}
+
 // few rows of bf16 with heads of up to 128
 int attend_decode( const WindowOut<__bf16>& out, const __bf16* q, const float* bias, const WindowRows& wr, const WindowShape& s, uint64_t rows, uint32_t max_pos, hipStream_t st )
 {
+  if ( s.group == 1 && std::max( s.dpad, s.vpad ) > 64 ) {
+    return attend_dot( out, q, bias, wr, s, rows, max_pos, st );
+  }
   uint32_t head_cols = s.group; // the largest divisor of the group that fits
   while ( head_cols > STEP_COLS || s.group % head_cols != 0 ) {
     head_cols--;

@@ -191,6 +191,61 @@ ATTENTIONS = {
 }
 
 
+# streams of keys (rows x heads) up to the CUs, cut into splits and not; up to two, four times as many and more; short and long; heads that do not divide by
+# two or four; head sizes that leave lanes idle
+@pytest.mark.parametrize("shared", [False, True])
+@pytest.mark.parametrize("heads,dim,vdim,rows,keys", [(4, 128, 128, 1, 1500), (2, 72, 128, 40, 2100), (3, 96, 96, 5, 40), (32, 128, 128, 1, 64), (8, 128, 104, 40, 250),
+                                                      (4, 72, 72, 70, 3100), (4, 128, 128, 150, 70), (6, 80, 72, 100, 33), (4, 128, 128, 300, 150), (4, 72, 128, 300, 250),
+                                                      (5, 128, 128, 240, 200)])
+def test_decode_of_heads_with_keys_of_their_own(heads, dim, vdim, rows, keys, shared):
+    """Against 64 bits: a rounding to bf16 and fp32 sums.  Contexts of all lengths and none, a window with kept keys, a bias by distance, keys whose scores are -inf."""
+    import torch
+    from glinthawk_amd import ops
+    vdim = dim if shared else vdim
+    window, keep, n_dist = (keys // 2 + 1, 5, 0) if heads % 4 == 0 else (0, 0, 0 if shared else 17)
+    a = ops.window_attn(heads, heads, dim, vdim, dim ** -0.5, window, keep, n_dist, shared)
+    g = torch.Generator(device="cuda").manual_seed(rows + keys)
+    row = heads * (dim if shared else dim + vdim)
+    cache = torch.randn((rows, keys, row), generator=g, device="cuda").bfloat16()
+    groups = -(-keys // 32)                                           # GH_WINDOW_FACTOR_GROUP keys side by side
+    factors = torch.rand((rows, groups, heads, 32), generator=g, device="cuda") + 0.5
+    memory = torch.cat([cache.view(rows, -1).view(torch.uint8), factors.view(rows, -1).view(torch.uint8)], 1).contiguous()
+    lengths = torch.randint(1, keys + 1, (rows,), generator=g, device="cuda")
+    lengths[-1], lengths[0] = 1, keys
+    missing = rows // 2 if rows > 2 else -1
+    table = ops.row_table([0 if i == missing else memory[i].data_ptr() for i in range(rows)])
+    q = torch.randn((rows, heads, dim), generator=g, device="cuda").bfloat16()
+    bias = torch.randn((heads, n_dist), generator=g, device="cuda") if n_dist else None
+    if rows > 2:
+        memory[0].view(torch.bfloat16)[3 * row] = -float("inf")            # a key of the first head: -inf or inf by the query's sign
+        q[0, 0, 0] = 1.0
+        cache[0, 3, 0] = -float("inf")
+    got = ops.attn_window(q.view(rows, -1), a, table, (lengths - 1).int(), 1, keys - 1, bias, 0, cache[0].numel() * 2).double().view(rows, heads, vdim)
+    j = torch.arange(keys, device="cuda")
+    for i in range(rows):
+        if i == missing:
+            assert (got[i] == 0).all()
+            continue
+        p = int(lengths[i]) - 1
+        k = cache[i, :p + 1, :heads * dim].view(p + 1, heads, dim).double()
+        v = k if shared else cache[i, :p + 1, heads * dim:].view(p + 1, heads, vdim).double()
+        score = (k * q[i].double()).sum(-1) * dim ** -0.5
+        if shared:
+            score = score * factors[i].permute(0, 2, 1).reshape(-1, heads)[:p + 1].double()
+        if bias is not None:
+            score = score + bias.double().T[(p - j[:p + 1]).clamp(max=n_dist - 1)]
+        hidden = (p - j[:p + 1] >= window) & (j[:p + 1] >= keep) if window else torch.zeros(p + 1, dtype=torch.bool, device="cuda")
+        weight = score.masked_fill(hidden[:, None], -float("inf")).softmax(0)
+        if shared and i == 0:
+            v = v.clone()
+            v[v.isinf()] = 0.0
+            got[0, 0, 0] = 0.0                                             # 0 x inf
+        want = (weight[:, :, None] * v).sum(0)
+        if shared and i == 0:
+            want[0, 0] = 0.0
+        assert ((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), i
+
+
 class Cache:
     """One attention layer's cache rows of a few contexts, filled by hand (heads padded to 8 elements with zeros)."""
 
