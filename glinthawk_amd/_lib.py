@@ -128,6 +128,7 @@ SIGNATURES = {
     "gh_gemm_library_calls": (_u64, []),
     "gh_matmul_fuses_many_rows": (_i, [_u64, _u64, _u64, _i]),
     "gh_matmul_qkv_fuses_many_rows": (_i, [_u64, _u32, _u32, _u32, _u64, _i]),
+    "gh_matmul_qkv_fuses_few_rows": (_i, [_u64, _u32, _u32, _u32, _u64, _i]),
     "gh_gemm_stream_plan": (_i, [_u64, _u64, _u64, _vp, _vp, _vp]),
     "gh_gemm_ring_plan": (_i, [_u64, _u64, _u64, _i, _vp]),
     "gh_matmul": (_i, [_vp, _vp, _vp, _u64, _u64, _u64, _i, _vp]),

@@ -14,6 +14,8 @@ int gemm_tile_epilogue_launch( void* xout, const void* x, const void* w, uint64_
                                bool* done );
 int gemm_tile_qkv_launch( void* q, const void* x, const void* wqkv, uint64_t s, uint64_t b, gh_dtype dt, const QkvRows& rows, hipStream_t st, bool* done );
 bool gemm_tile256_qkv_fits( const QkvRows& q );
+bool gemm_qkv_applicable( uint64_t s, uint64_t b, const void* x, const void* w, const void* q, const QkvRows& rows );
+int gemm_qkv_launch( void* q, const void* x, const void* w, uint64_t s, uint64_t b, const QkvRows& rows, hipStream_t st );
 // fp32: the product and what follows it in one kernel (gh_gemm_f32.hip)
 int gemm_f32_accum( float* residual, const float* x, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
 int gemm_f32( float* out, const float* x, const float* norm, const float* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st );
@@ -635,6 +637,10 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   }
   // many rows: rotated and appended in the tile kernel's epilogue, no fp32 sums; whole rounds of tiles and a rest where that is faster
   const QkvRows rows { pos_dev, freq_real, freq_imag, token_rows_dev, (uint32_t)dim, (uint32_t)kv_dim, head_size };
+  // few rows: rotated and appended where the sums are, each work-group over the whole K range
+  if ( dt == GH_F16 && kv_out == nullptr && !overlap( q, b * dim * 2, x, x_bytes ) && gemm_qkv_applicable( s, b, x, wqkv, q, rows ) ) {
+    return gemm_qkv_launch( q, x, wqkv, s, b, rows, st );
+  }
   if ( dt == GH_F16 && kv_out == nullptr && gemm_tile256_qkv_fits( rows ) && !overlap( q, b * dim * 2, x, x_bytes ) ) {
     if ( const uint64_t b1 = gemm_token_split( s, r, b, dt, x, wqkv, q ) ) {
       if ( int rc = gh_matmul_qkv_rope_append( q, nullptr, x, wqkv, s, b1, pos_dev, freq_real, freq_imag, token_rows_dev, n_kv_heads, gqa_size, head_size, dt, stream ) ) {
@@ -668,6 +674,15 @@ int gh_matmul_qkv_rope_append( void* q, void* kv_out, const void* x, const void*
   }
   GH_LAUNCH_CHECK();
   return GH_OK;
+}
+
+int gh_matmul_qkv_fuses_few_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt )
+{
+  QkvRows rows;
+  rows.kv_dim = n_kv_heads * head_size;
+  rows.dim = rows.kv_dim * gqa_size;
+  rows.head_size = head_size;
+  return s > 0 && rows.dim > 0 && dt == GH_F16 && gemm_qkv_applicable( s, b, nullptr, nullptr, nullptr, rows ) ? 1 : 0;
 }
 
 // Norm and product in one launch: worth it while what every wave norms again takes less than the launch it saves, i.e. for few and short rows; a product of

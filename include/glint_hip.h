@@ -193,6 +193,8 @@ int gh_matmul_fuses_many_rows( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
 /* host-only query: 1 when gh_matmul_qkv_rope_append (no kv_out, 16-byte aligned operands) rotates and appends the rows of this many tokens, all or all but a
  * rest of them, in the large tile kernel's epilogue: the caller's test for taking the fused call on many rows */
 int gh_matmul_qkv_fuses_many_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt );
+/* host-only query: 1 when it does so for few tokens, in the epilogue of a product whose work-groups take their weight rows over the whole K range */
+int gh_matmul_qkv_fuses_few_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt );
 /* host-only query: how the weight-streaming kernel would cut an (r x s) . (b x s)^T product for the initialised device (256 compute
  * units before initialisation): number of K ranges, k per range (a multiple of 256), weight rows per work-group */
 int gh_gemm_stream_plan( uint64_t s, uint64_t r, uint64_t b, uint32_t* splits, uint32_t* k_per_split, uint32_t* rows_per_workgroup );

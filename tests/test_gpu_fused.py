@@ -417,6 +417,45 @@ def test_stage_with_and_without_fused_projections(name, dtype):
     b.close()
 
 
+# every width of the activation tile and the row it ends on; shares of 32 to 64 rows of the CUs, work-groups with a part of a share; K that ends inside a step, that is
+# shorter than the ring, one step; heads of 8
+@pytest.mark.parametrize("s,kv_heads,gqa,head_size,b", [(4096, 32, 1, 128, 1), (4096, 32, 1, 128, 32), (1024, 16, 4, 128, 33), (1024, 32, 2, 64, 64), (520, 32, 2, 128, 48),
+                                                        (1000, 16, 4, 128, 20), (1096, 32, 1, 128, 63), (128, 32, 2, 64, 5), (64, 512, 1, 8, 17),
+                                                        (8, 200, 1, 20, 3), (5120, 40, 1, 128, 31), (8192, 8, 8, 128, 16)])
+def test_few_rows_of_qkv_rotated_and_appended(s, kv_heads, gqa, head_size, b):
+    """Against 64 bits: two roundings of f16 and fp32 sums of s products.  Empty contexts keep their query unrotated; cache rows on and off an 8-byte boundary, the rows around them."""
+    dim, kv_dim = kv_heads * gqa * head_size, kv_heads * head_size
+    shape = Shape(dim=dim, n_layers=1, n_heads=kv_heads * gqa, n_kv_heads=kv_heads, hidden_dim=64, seq_len=64)
+    g = torch.Generator(device="cuda").manual_seed(b)
+    x = torch.randn((b, s), generator=g, device="cuda").half()
+    w = (torch.randn((dim + 2 * kv_dim, s), generator=g, device="cuda") / s ** 0.5).half()
+    pos = torch.randint(0, 64, (b,), generator=g, device="cuda", dtype=torch.int32)
+    angle = torch.rand((64, head_size // 2), generator=g, device="cuda") * 6
+    re, im = torch.cos(angle).half(), torch.sin(angle).half()
+    assert _lib.lib().gh_matmul_qkv_fuses_few_rows(s, kv_heads, gqa, head_size, b, _lib.GH_F16) == 1
+    y = (x.double() @ w.double().t()).half().double()
+    missing = [i for i in range(b) if i % 7 == 5]
+    turn = torch.ones((b, 1, 1), dtype=torch.bool, device="cuda")
+    turn[missing] = False
+    a, c = re[pos.long()].double()[:, None], im[pos.long()].double()[:, None]
+
+    def turned(v):
+        v = v.view(b, -1, head_size // 2, 2)
+        out = torch.stack([v[..., 0] * a - v[..., 1] * c, v[..., 0] * c + v[..., 1] * a], -1).view(b, -1, head_size)
+        return torch.where(turn, out, v.reshape(b, -1, head_size)).reshape(b, -1)
+
+    want_q, want_row = turned(y[:, :dim].contiguous()), torch.cat([turned(y[:, dim: dim + kv_dim].contiguous()), y[:, dim + kv_dim:]], 1)
+    for shift in (0, 1):
+        flat = torch.full((2 * b * 2 * kv_dim + 8,), 5.0, dtype=torch.float16, device="cuda")
+        cache = flat[shift: shift + 2 * b * 2 * kv_dim].view(b, 2, 2 * kv_dim)
+        rows = ops.row_table([0 if i in missing else cache[i].data_ptr() for i in range(b)])
+        got, _ = ops.matmul_qkv_rope_append(x, w, pos, re, im, rows, shape)
+        # a product's sum may round to either side of a tie: one unit of f16 (2^-10) of each of a pair, and the rotation's own rounding
+        assert torch.allclose(got.double(), want_q, rtol=4e-3, atol=4e-3)
+        for i in range(b):
+            assert (cache[i] == 5.0).all() if i in missing else torch.allclose(cache[i, 0].double(), want_row[i], rtol=4e-3, atol=4e-3) and (cache[i, 1] == 5.0).all()
+
+
 # widths and heads of the smallest and the largest the launch takes, groups of query heads, heads that leave rows of lanes idle; more keys than one turn
 @pytest.mark.parametrize("kv_heads,gqa,head_size,batch", [(6, 1, 48, 4), (2, 2, 8, 7), (5, 1, 64, 3), (2, 4, 40, 6), (1, 1, 4, 8), (4, 1, 20, 64), (3, 2, 44, 8)])
 def test_attention_in_the_launch_of_its_projections(kv_heads, gqa, head_size, batch):
