@@ -7,7 +7,8 @@
 //
 // The RMS norm in front of a product is a launch of its own for a few rows that every wave of the product reads anyway.  Where a row is requested in
 // one go (s <= what KU pieces cover) the wave squares what it holds and norms it before it multiplies, which takes a 15M layer from seven launches to
-// five (norm and product as two launches / one, in a graph: 864 x 288 at 4 rows 5.1 / 3.5 us, 32000 x 288 10.4 / 8.8).
+// five (norm and product as two launches / one, in a graph: 864 x 288 at 4 rows 5.1 / 3.2 us, 32000 x 288 10.4 / 9.2, which zeros in the place of what is past a row's end,
+// an instruction an element, made 3.5 and 10.1, 4096 x 512 at 8 rows 5.9 and 7.5).
 #include "gh_common.h"
 
 #include <algorithm>
@@ -225,10 +226,11 @@ __global__ __launch_bounds__( 256 ) void gemm_f32_kernel( Epilogue epi, const fl
           ss[c] = 0.0f;
 #pragma unroll
           for ( int u = 0; u < KU; u++ ) {
-            const bool in = ( u * 64 + lane ) * V < s;
+            if ( ( u * 64 + lane ) * V < s ) {
 #pragma unroll
-            for ( int e = 0; e < V; e++ ) {
-              ss[c] += in ? y[u][c][e] * y[u][c][e] : 0.0f;
+              for ( int e = 0; e < V; e++ ) {
+                ss[c] += y[u][c][e] * y[u][c][e];
+              }
             }
           }
         }
@@ -248,14 +250,31 @@ __global__ __launch_bounds__( 256 ) void gemm_f32_kernel( Epilogue epi, const fl
 #pragma unroll
       for ( int u = 0; u < KU; u++ ) {
         const bool in = !tail.value || k0 + ( u * 64 + lane ) * V < s;
+        // Lanes past the row's end take no part.  With the norm in front everything is here by now and instructions are what counts: they sit a branch out; without it
+        // the first piece's products run while the others are under way, and a branch would end that (4096 x 512 at 4 rows 4.1 us, 4.0 with zeros in their place).
+        if constexpr ( NORM ) {
+          if ( in ) {
 #pragma unroll
-        for ( int e = 0; e < V; e++ ) {
+            for ( int e = 0; e < V; e++ ) {
 #pragma unroll
-          for ( int i = 0; i < ROWS; i++ ) {
-            const float av = in ? a[u][i][e] : 0.0f;
+              for ( int i = 0; i < ROWS; i++ ) {
 #pragma unroll
-            for ( int c = 0; c < COLS; c++ ) {
-              acc[i][c] += av * ( in ? y[u][c][e] : 0.0f );
+                for ( int c = 0; c < COLS; c++ ) {
+                  acc[i][c] += a[u][i][e] * y[u][c][e];
+                }
+              }
+            }
+          }
+        } else {
+#pragma unroll
+          for ( int e = 0; e < V; e++ ) {
+#pragma unroll
+            for ( int i = 0; i < ROWS; i++ ) {
+              const float av = in ? a[u][i][e] : 0.0f;
+#pragma unroll
+              for ( int c = 0; c < COLS; c++ ) {
+                acc[i][c] += av * ( in ? y[u][c][e] : 0.0f );
+              }
             }
           }
         }
