@@ -41,7 +41,22 @@ struct MlstmCols
   uint32_t q, k, v, g, i, f;
 };
 
-// `gates`: (rows, 2 heads) fp32, the log input gates of a token's heads, then its log forget gates (mlstm_gates_kernel)
+// the gates as their product left them
+template<typename E>
+struct MlstmGates
+{
+  ProductView<float> y;
+  MlstmCols col;
+  const E *bias_i, *bias_f;
+  float cap;
+  __device__ __forceinline__ float log_input( float z, uint32_t h ) const { return soft_cap( z + ( bias_i != nullptr ? to_f32( bias_i[h] ) : 0.0f ), cap ); }
+  __device__ __forceinline__ float log_forget( float z, uint32_t h ) const
+  {
+    return log_sigmoid( soft_cap( z + ( bias_f != nullptr ? to_f32( bias_f[h] ) : 0.0f ), cap ) );
+  }
+};
+
+// `gates`: (rows, 2 heads) fp32, the log input gates of a token's heads, then its log forget gates (mlstm_gates_kernel); NULL: the kernel makes them itself
 template<typename E, typename View>
 struct MlstmIn
 {
@@ -52,21 +67,15 @@ struct MlstmIn
 
 template<typename E>
 __global__ __launch_bounds__( 256 ) void mlstm_gates_kernel( float* __restrict__ out,
-                                                             ProductView<float> y,
-                                                             MlstmCols col,
-                                                             const E* __restrict__ bias_i,
-                                                             const E* __restrict__ bias_f,
+                                                             MlstmGates<E> in,
                                                              uint32_t heads,
-                                                             uint64_t rows,
-                                                             float cap )
+                                                             uint64_t rows )
 {
   const uint64_t total = rows * 2 * heads, stride = (uint64_t)gridDim.x * blockDim.x;
   for ( uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride ) {
     const uint64_t row = i / ( 2 * heads );
-    const uint32_t g = (uint32_t)( i % ( 2 * heads ) ), h = g < heads ? g : g - heads;
-    const E* bias = g < heads ? bias_i : bias_f;
-    const float z = soft_cap( y.at( row, ( g < heads ? col.i : col.f ) + h ) + ( bias != nullptr ? to_f32( bias[h] ) : 0.0f ), cap );
-    out[i] = g < heads ? z : log_sigmoid( z );
+    const uint32_t g = (uint32_t)( i % ( 2 * heads ) );
+    out[i] = g < heads ? in.log_input( in.y.at( row, in.col.i + g ), g ) : in.log_forget( in.y.at( row, in.col.f + g - heads ), g - heads );
   }
 }
 
@@ -80,9 +89,10 @@ struct MlstmState
 
 // RPT: rows of S per thread kept in registers (0: S stays in memory, any dim)
 template<typename E, typename View, int RPT>
-__global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ o_out, float* __restrict__ nm_out, MlstmIn<E, View> in, MlstmState st, MlstmShape s )
+__global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ o_out, float* __restrict__ nm_out, MlstmIn<E, View> in, MlstmGates<E> raw, MlstmState st, MlstmShape s )
 {
   extern __shared__ float lds[];
+  __shared__ float g_s[2];        // the gates of one token
   const uint32_t dim4 = ( s.dim + 3 ) / 4 * 4; // v_s and red are read as float4
   float* q_s = lds;               // dim
   float* k_s = q_s + dim4;        // dim
@@ -104,6 +114,16 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
   const uint32_t cl = t & 15, rg = t >> 4;
   const uint32_t c0 = slice * SLICE + cl * 4;
   const bool col_live = c0 < s.vpad;
+  // The gates' sums, a K range a lane (the input gate's in the lower half of the wave), requested in front of the state: one token of a context
+  float gate_part = 0.0f;
+  if ( in.gates == nullptr && t < WAVE ) {
+    const uint32_t k = t & 31;
+    const float* sums = raw.y.data + ctx * raw.y.stride + ( ( t & 32 ) == 0 ? raw.col.i : raw.col.f ) + h;
+    gate_part = k < raw.y.planes() ? sums[k * raw.y.plane] : 0.0f;
+    for ( uint32_t more = k + 32; more < raw.y.planes(); more += 32 ) {
+      gate_part += sums[more * raw.y.plane];
+    }
+  }
   constexpr int R = RPT > 0 ? RPT : 1;
   float4 reg[R];
   if constexpr ( RPT > 0 ) {
@@ -120,6 +140,7 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
       *reinterpret_cast<float4*>( S + (uint64_t)row * s.vpad + c0 ) = make_float4( 0.0f, 0.0f, 0.0f, 0.0f );
     }
   }
+  gate_part = row16_sum( gate_part );
   for ( uint32_t d = t; d < s.dim; d += 256 ) {
     n_s[d] = fresh ? 0.0f : n_in[d];
   }
@@ -136,11 +157,21 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
       const uint32_t c = slice * SLICE + t;
       v_s[t] = c < s.vdim ? in.main.at( row_in, in.col.v + h * s.vdim + c ) : 0.0f;
     }
-    const float gi = in.gates[row_in * 2 * s.heads + h], gf = in.gates[( row_in * 2 + 1 ) * s.heads + h];
+    float gi = 0.0f, gf = 0.0f;
+    if ( in.gates != nullptr ) {
+      gi = in.gates[row_in * 2 * s.heads + h];
+      gf = in.gates[( row_in * 2 + 1 ) * s.heads + h];
+    } else if ( t < WAVE ) { // one wave for all: some 200 instructions
+      g_s[0] = raw.log_input( lane_value( gate_part, 0 ) + lane_value( gate_part, 16 ), h );
+      g_s[1] = raw.log_forget( lane_value( gate_part, 32 ) + lane_value( gate_part, 48 ), h );
+    }
+    __syncthreads();
+    if ( in.gates == nullptr ) {
+      gi = g_s[0], gf = g_s[1];
+    }
     const float m_new = fmaxf( gf + m, gi );
     const float decay = expf( gf + m - m_new ), inp = expf( gi - m_new );
     m = m_new;
-    __syncthreads();
     const float4 v4 = *reinterpret_cast<const float4*>( v_s + cl * 4 );
     float4 acc = make_float4( 0.0f, 0.0f, 0.0f, 0.0f );
     auto row_step = [&]( float4& x, uint32_t row ) {
@@ -817,10 +848,15 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
   return with_product( dt, y, [&]( auto tag, auto view ) -> int {
     using E = decltype( tag );
     using View = decltype( view );
-    mlstm_gates_kernel<E><<<(unsigned)std::min<uint64_t>( ( rows * 2 * s.heads + 255 ) / 256, 4096 ), 256, 0, st>>>(
-      log_gates, ProductView<float>( gates ), col, static_cast<const E*>( bias_i ), static_cast<const E*>( bias_f ), s.heads, rows, s.cap );
-    GH_LAUNCH_CHECK();
-    const MlstmIn<E, View> in { view, log_gates, col };
+    const MlstmGates<E> raw { ProductView<float>( gates ), col, static_cast<const E*>( bias_i ), static_cast<const E*>( bias_f ), s.cap };
+    // One token of a context: every work-group of a head makes the two gates again beside its loads of the state, which is less than a launch in front of it
+    // (32 contexts: 4.6 us).
+    const bool gates_made = n_tokens > 1;
+    if ( gates_made ) {
+      mlstm_gates_kernel<E><<<(unsigned)std::min<uint64_t>( ( rows * 2 * s.heads + 255 ) / 256, 4096 ), 256, 0, st>>>( log_gates, raw, s.heads, rows );
+      GH_LAUNCH_CHECK();
+    }
+    const MlstmIn<E, View> in { view, gates_made ? log_gates : nullptr, col };
     const dim3 grid( ( s.vpad + SLICE - 1 ) / SLICE, s.heads, (unsigned)batch );
     bool walked = false;
     if constexpr ( std::is_same_v<View, ProductView<__bf16>> ) {
@@ -841,13 +877,13 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
     if ( walked ) {
       // the chunk kernel has done it
     } else if ( s.dim <= 64 ) {
-      mlstm_walk_kernel<E, View, 4><<<grid, 256, lds, st>>>( o, nm, in, state, s );
+      mlstm_walk_kernel<E, View, 4><<<grid, 256, lds, st>>>( o, nm, in, raw, state, s );
     } else if ( s.dim <= 128 ) {
-      mlstm_walk_kernel<E, View, 8><<<grid, 256, lds, st>>>( o, nm, in, state, s );
+      mlstm_walk_kernel<E, View, 8><<<grid, 256, lds, st>>>( o, nm, in, raw, state, s );
     } else if ( s.dim <= 256 ) {
-      mlstm_walk_kernel<E, View, 16><<<grid, 256, lds, st>>>( o, nm, in, state, s );
+      mlstm_walk_kernel<E, View, 16><<<grid, 256, lds, st>>>( o, nm, in, raw, state, s );
     } else {
-      mlstm_walk_kernel<E, View, 0><<<grid, 256, lds, st>>>( o, nm, in, state, s );
+      mlstm_walk_kernel<E, View, 0><<<grid, 256, lds, st>>>( o, nm, in, raw, state, s );
     }
     GH_LAUNCH_CHECK();
     const dim3 finish( (unsigned)rows, ( s.heads + 3 ) / 4 );
