@@ -538,6 +538,36 @@ def test_mlstm_extreme_gates(dtype):
             at += c
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,d,dv,batch", [(4, 256, 384, 7), (8, 64, 64, 1), (3, 130, 136, 11), (1, 12, 20, 9), (2, 300, 70, 5)])
+def test_mlstm_walk_of_many_contexts(H, d, dv, batch, dtype):
+    """Work-groups take (context, head) pairs by eights and the rest as they come: every context as in a call of its own, where there are too few pairs for
+    that, bit for bit (small whole numbers: the projections are exact in any order of their sums), and a slot without a context is left alone."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    width, empty = 8, batch // 2 if batch > 1 else None
+    m = GhMlstm(H, d, dv, 15.0, 1e-5)
+    rows, _ = ops.mlstm_weight_rows(m)
+    rng = np.random.default_rng(batch)
+    w = dev(rng.integers(-2, 3, (rows, width)).astype(np.float32), dtype)
+    bias, norm = dev(np.linspace(-3, 3, H), dtype), dev(np.ones(H * dv), dtype)
+    n = ops.mlstm_state_bytes(m) // 4
+    state0 = torch.from_numpy(rng.standard_normal((batch, n)).astype(np.float32)).cuda()
+    start = torch.from_numpy((np.arange(batch) % 3).astype(np.int32)).cuda()  # some start anew
+    for n_tokens in (1, 3):
+        x = dev(rng.integers(-2, 3, (batch * n_tokens, width)).astype(np.float32), dtype)
+        state = state0.clone()
+        got = ops.mlstm_forward(x, w, m, bias, bias, norm, ops.row_table([0 if i == empty else state[i].data_ptr() for i in range(batch)]), start, n_tokens)
+        for i in range(batch):
+            alone = state0[i].clone()
+            if i != empty:
+                one = ops.mlstm_forward(x[i * n_tokens:(i + 1) * n_tokens].contiguous(), w, m, bias, bias, norm, ops.row_table([alone.data_ptr()]), start[i:i + 1].contiguous(),
+                                        n_tokens)
+                assert torch.equal(got[i * n_tokens:(i + 1) * n_tokens], one), i
+            assert torch.equal(state[i], alone), i
+
+
 @pytest.mark.parametrize("d,dv,T", [(64, 64, 320), (128, 192, 257), (256, 512, 512)])
 def test_mlstm_same_bits_twice(d, dv, T):
     """The chunks of a prompt share their LDS tiles: with enough work-groups for the waves of one to drift apart, the same inputs give the
