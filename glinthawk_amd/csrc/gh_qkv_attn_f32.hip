@@ -3,7 +3,8 @@
 // Small models at a handful of contexts are a chain of launches, each bound by being one and by its round trips to memory.  A query head of a context
 // needs 3 x head_size of the weight rows, its own cache rows and nothing of any other, so a work-group that makes q, k and v itself can go on to the
 // attention: a head's weights are read once per context (from L2, but for the first), which costs less than the launch that it saves while a
-// work-group's share is short.  The old keys and values do not depend on the product, so they are requested with the weights, in front of it.
+// work-group's share is short.  The old keys and values do not depend on the product, so they are requested with the weights, in front of it; that no other
+// work-group of the launch writes one of them, i.e. that a context stands in the batch once, is up to the caller.
 //
 //   work-group  8 waves on one (query head, context); 16 lanes share a row of x, of the weights or of a key, four elements a piece
 //   product     a row of lanes takes the weight rows j, j + 32, ... of the head's q | k | v rows, all requested at once

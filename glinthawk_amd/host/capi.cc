@@ -527,6 +527,16 @@ int32_t glint_book_manager_get_context( void* m, uint32_t context_id )
   return ctx ? man.slot_index( ctx ) : -1;
 }
 
+// whether one of these addresses (0: none) stands there twice
+int glint_book_stands_twice( const uint64_t* memory, uint64_t n )
+{
+  std::vector<const void*> all;
+  for ( uint64_t i = 0; i < n; i++ ) {
+    all.push_back( reinterpret_cast<const void*>( memory[i] ) );
+  }
+  return stands_twice( std::move( all ) ) ? 1 : 0;
+}
+
 int glint_book_manager_release( void* m, uint32_t context_id ) { return static_cast<BookManager*>( m )->man.release_context( context_id ) ? 1 : 0; }
 
 // paged context over a counting region: hosts `n_hosted` layers of the 70B-4K shape

@@ -17,6 +17,15 @@
 
 namespace glint {
 
+// Whether a context stands in a batch more than once, by the memory of the rows' contexts (nullptr: none).  The new rows of such a batch are all
+// appended before any of them is attended from, as one of them may be a key of another.
+inline bool stands_twice( std::vector<const void*> memory )
+{
+  std::sort( memory.begin(), memory.end() );
+  const auto first = std::find_if( memory.begin(), memory.end(), []( const void* m ) { return m != nullptr; } );
+  return std::adjacent_find( first, memory.end() ) != memory.end();
+}
+
 // the read interface every context type offers (models/llama2/context.hh:17-45)
 template<typename T, typename DType>
 concept TokenContextConcept = requires( T t ) {

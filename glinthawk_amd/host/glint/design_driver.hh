@@ -153,14 +153,11 @@ public:
   // (a context takes its tokens one after the other).
   bool positions_fit( const ContextVector& contexts, const uint32_t* start_pos, const uint32_t n_tokens ) const
   {
-    std::vector<const void*> seen;
+    std::vector<const void*> memory;
     for ( const auto& c : contexts ) {
-      if ( !c->empty() ) {
-        seen.push_back( c->data() );
-      }
+      memory.push_back( c->empty() ? nullptr : c->data() );
     }
-    std::sort( seen.begin(), seen.end() );
-    if ( std::adjacent_find( seen.begin(), seen.end() ) != seen.end() ) {
+    if ( stands_twice( std::move( memory ) ) ) {
       return false;
     }
     for ( size_t i = 0; i < contexts.size(); i++ ) {

@@ -464,7 +464,7 @@ public:
                                                  Config::n_kv_heads, Config::gqa_size, Config::head_size, gh_type<DType>(), this->stream_ ) );
   }
 
-  // All of a layer up to its attention in one launch; attention_rides( batch_size ): whether there is one
+  // All of a layer up to its attention in one launch, where no context stands twice in the batch; attention_rides( batch_size ): whether there is one
   static bool attention_rides( const uint64_t batch_size )
   {
     const gh_shape s = shape();

@@ -672,7 +672,7 @@ private:
   void normed_layer_ops( const size_t layer, const size_t table_index )
   {
     const auto& w = layers_[layer];
-    if ( !balanced_step_ && LlamaOperations::attention_rides( batch_ ) ) {
+    if ( attention_rides_ ) {
       ops_.rmsnorm_qkv_attention( xb_, x_, w.rms_att_weight, w.wq, batch_, pos_dev(), base_.freq_cis_real, base_.freq_cis_imag, layer_rows_dev( table_index ),
                                   token_rows_dev( table_index ) );
     } else {
@@ -850,6 +850,9 @@ private:
         ptrs[( 2 * k + 1 ) * table_stride() + i] = layer.token( token_positions_[i] ).key();
       }
     }
+    // (a launch that appends and attends reads the old keys while other rows are appended)
+    attention_rides_ = decode && !run.empty() && !balanced_step_ && LlamaOperations::attention_rides( batch_ )
+                       && !stands_twice( std::vector<const void*>( ptrs, ptrs + batch_ ) );
     const size_t bytes = ( ptr_tables( tables_host_ ) - tables_host_ ) + run.size() * 2 * table_stride() * sizeof( void* ); // a multiple of 16
     tables_uploaded_ = true;
     tables_drain_count_ = ops_.drain_count();
@@ -1112,6 +1115,7 @@ private:
   DevicePtr attn_bal_ws_ {};
   uint64_t attn_bal_ws_bytes_ { 0 };
   bool balanced_step_ { false };
+  bool attention_rides_ { false }; // in the launch of its projections, this step
   uint8_t* tables_host_ { nullptr };
   bool tables_uploaded_ { false };
   uint64_t tables_drain_count_ { 0 };

@@ -83,6 +83,7 @@ def host_lib() -> C.CDLL:
             "glint_book_manager_get_contexts": (C.c_int, [vp, vp, vp, u64, u64, u64, vp]),
             "glint_book_manager_get_context": (i32, [vp, u32]),
             "glint_book_manager_release": (C.c_int, [vp, u32]),
+            "glint_book_stands_twice": (C.c_int, [vp, u64]),
             "glint_book_paged_new": (vp, [u32]),
             "glint_book_paged_delete": (None, [vp]),
             "glint_book_paged_prepare": (u64, [vp, u32, u32, C.c_int, C.POINTER(u64)]),
@@ -399,6 +400,12 @@ class BookManager:
 
     def release(self, context_id: int) -> bool:
         return bool(host_lib().glint_book_manager_release(self._m, context_id))
+
+
+def book_stands_twice(memory) -> bool:
+    """Host-only: whether a context, by its address (0: none), stands in a batch more than once."""
+    a = np.ascontiguousarray(np.asarray(memory, dtype=np.uint64))
+    return bool(host_lib().glint_book_stands_twice(a.ctypes.data, len(a)))
 
 
 class BookPagedContext:

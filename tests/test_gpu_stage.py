@@ -246,6 +246,48 @@ def test_inactive_rows_and_slot_reuse():
     st.close()
 
 
+@pytest.mark.parametrize("repeated", [True, False])
+def test_several_tokens_of_a_context_in_one_step(repeated):
+    """Rows of one context at positions p, p + 1 and p + 2 beside other contexts, in one step: as one token after the other, up to the sums of fp32 in another
+    order.  Such a batch is appended before it is attended from, one without a repetition in the launch that also attends: only the first writes q."""
+    name = "stories15m"
+    cfg = SHAPES[name]
+    layers, base = make_weights(cfg, np.float32, seed=41, wcls=False)
+    rng = np.random.default_rng(42)
+    p = 5
+    cids = [10, 11, 10, 12, 10] if repeated else [10, 11, 12, 13, 14]
+    pos = [p, 2, p + 1, 0, p + 2] if repeated else [p, 2, p, 0, p]
+    tokens = rng.integers(0, cfg.vocab_size, len(cids)).tolist()
+    together, single = (S.Stage(name, "f32", 0, cfg.n_layers, len(cids), 8, with_cls=True) for _ in range(2))
+    for st in (together, single):
+        load_weights(st, cfg, layers, base, False)
+        for cid, end in {c: at for c, at in reversed(list(zip(cids, pos)))}.items():     # up to the first position of each context
+            for at in range(end):
+                st.new_state(1)
+                st.set_prompt(0, cid, 100 + cid + at, at)
+                assert st.forward()
+    together.new_state(len(cids))
+    for i, cid in enumerate(cids):
+        together.set_prompt(i, cid, tokens[i], pos[i])
+    mark = np.full((len(cids), cfg.dim), 1e30, np.float32)
+    _lib.check(_lib.lib().gh_memcpy(together.scratch_ptr("q"), mark.ctypes.data, mark.nbytes, _lib.GH_H2D, 0, None), "gh_memcpy")
+    assert together.forward()
+    q = d2h(together.scratch_ptr("q"), mark.shape, np.float32)
+    assert np.array_equal(q, mark) != repeated
+    logits = d2h(together.scratch_ptr("logits"), (len(cids), cfg.vocab_size), np.float32)
+    for i, cid in enumerate(cids):
+        single.new_state(1)
+        single.set_prompt(0, cid, tokens[i], pos[i])
+        assert single.forward()
+        want = d2h(single.scratch_ptr("logits"), (1, cfg.vocab_size), np.float32)[0]
+        assert np.linalg.norm(logits[i] - want) <= 5e-6 * np.linalg.norm(want), i
+        for l in range(cfg.n_layers):
+            have, should = (d2h(st.context_layer_ptr(r, l) + pos[i] * 2 * cfg.kv_dim * 4, (2 * cfg.kv_dim,), np.float32) for st, r in ((together, i), (single, 0)))
+            assert np.linalg.norm(have - should) <= 5e-6 * np.linalg.norm(should), (i, l)
+    together.close()
+    single.close()
+
+
 def test_finish_rule_sets_flag():
     name = "test-tiny"
     cfg = SHAPES[name]

@@ -48,6 +48,15 @@ def test_slot_manager_churn_like_config5():
     assert man.get_contexts([1], [7]) is None     # a new id cannot be served: all slots are owned
 
 
+def test_a_context_that_stands_in_a_batch_twice():
+    man = S.BookManager(4)
+    assert man.get_contexts([1, 1, 1, 0, 0], [7, 9, 7, 7, 7]) == [0, 1, 0, -1, -1]     # accepted, one context for both rows
+    for memory in ([4096, 8192, 4096], [0, 4096, 8192, 0, 4096], [4096] * 2):
+        assert S.book_stands_twice(memory)
+    for memory in ([], [0], [0, 0, 0], [4096], [0, 4096, 0], [3 * 4096, 4096, 0, 8192, 0]):
+        assert not S.book_stands_twice(memory)
+
+
 def test_paged_context_block_accounting():
     n_hosted = 3
     ctx = S.BookPagedContext(n_hosted)
