@@ -344,6 +344,9 @@ static HalfPlan half_plan( uint64_t s, uint64_t r, uint64_t b, bool whole_tiles 
   return best;
 }
 
+// a product runs on the kernel that was asked for, and no other is tried in front of it
+bool gemm_kernel_forced() { return g_force_kernel != 0; }
+
 // Whether a product runs as whole tiles of 256 x 256 (what is left of it once gemm_token_split() has cut it).
 static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout )
 {

@@ -18,6 +18,8 @@
 namespace gh {
 
 uint32_t gemm_ring_splits( uint64_t s, uint64_t r, uint64_t b, double* ns );
+uint64_t gemm_ring_units();
+bool gemm_kernel_forced();
 
 namespace {
 
@@ -226,7 +228,11 @@ __global__ __launch_bounds__( 512, 1 ) void gemm_qkv_kernel( __half* __restrict_
 #endif
 }
 
-uint32_t qkv_share( uint64_t r ) { return (uint32_t)std::max<uint64_t>( 16, ( ( r + cu_count() - 1 ) / cu_count() + 3 ) / 4 * 4 ); }
+uint64_t qkv_share( uint64_t r )
+{
+  const uint64_t units = gemm_ring_units();
+  return ( ( r + units - 1 ) / units + 3 ) / 4 * 4;
+}
 
 } // namespace
 
@@ -242,7 +248,7 @@ constexpr double QKV_START_NS = 4000.0, QKV_EPILOGUE_NS = 4200.0;
 bool gemm_qkv_applicable( uint64_t s, uint64_t b, const void* x, const void* w, const void* q, const QkvRows& rows )
 {
   const uint64_t r = rows.dim + 2ull * rows.kv_dim;
-  const bool takes = b > 0 && b <= 64 && b * s * sizeof( __half ) < QKV_MOST_BYTES && r <= 0x7fffffffull && qkv_share( r ) >= QKV_LEAST && qkv_share( r ) <= QKV_ROWS && s % 8 == 0 && s <= ( 1u << 21 ) // 64 rows of a descriptor are at most 2^28 bytes
+  const bool takes = !gemm_kernel_forced() && b > 0 && b <= 64 && b * s * sizeof( __half ) < QKV_MOST_BYTES && r <= 0x7fffffffull && qkv_share( r ) >= QKV_LEAST && qkv_share( r ) <= QKV_ROWS && s % 8 == 0 && s <= ( 1u << 21 ) // 64 rows of a descriptor are at most 2^28 bytes
          && rows.dim % 4 == 0 && rows.kv_dim % 4 == 0 && rows.head_size % 4 == 0
          && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) | reinterpret_cast<uintptr_t>( q ) ) & 15u ) == 0;
   if ( !takes ) {
@@ -257,7 +263,7 @@ bool gemm_qkv_applicable( uint64_t s, uint64_t b, const void* x, const void* w, 
 int gemm_qkv_launch( void* q, const void* x, const void* w, uint64_t s, uint64_t b, const QkvRows& rows, hipStream_t st )
 {
   const uint64_t r = rows.dim + 2ull * rows.kv_dim;
-  const uint32_t share = qkv_share( r ), units = (uint32_t)( ( r + share - 1 ) / share );
+  const uint32_t share = (uint32_t)qkv_share( r ), units = (uint32_t)( ( r + share - 1 ) / share );
   auto go = [&]( auto width ) {
     gemm_qkv_kernel<decltype( width )::value><<<( units + 7 ) / 8 * 8, 512, 0, st>>>( static_cast<__half*>( q ), static_cast<const __half*>( x ), static_cast<const __half*>( w ),
                                                                                      (uint32_t)s, (uint32_t)r, (uint32_t)b, rows, share, units );

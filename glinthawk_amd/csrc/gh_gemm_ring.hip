@@ -27,6 +27,8 @@
 
 namespace gh {
 
+uint64_t gemm_ring_units();
+
 namespace {
 
 typedef __attribute__( ( address_space( 3 ) ) ) void* lds_ptr;
@@ -382,7 +384,7 @@ RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
     RingPlan plan;
   };
   static thread_local Slot slots[64] {};
-  const uint64_t n_cu = g_ring_cus > 0 ? (uint64_t)g_ring_cus : (uint64_t)cu_count();
+  const uint64_t n_cu = gemm_ring_units();
   const uint64_t mixed = ( ( s * 31 + r ) * 31 + b ) * 2 + ( gate ? 1 : 0 );
   Slot& slot = slots[( mixed * 0x9e3779b97f4a7c15ull ) >> 58];
   if ( slot.s != s || slot.r != r || slot.b != b || slot.n_cu != n_cu || slot.gate != gate ) { // (s > 0: an empty slot is no product's)
@@ -392,6 +394,9 @@ RingPlan ring_plan( uint64_t s, uint64_t r, uint64_t b, bool gate )
 }
 
 } // namespace
+
+// the compute units that plans are balanced for
+uint64_t gemm_ring_units() { return g_ring_cus > 0 ? (uint64_t)g_ring_cus : (uint64_t)cu_count(); }
 
 bool gemm_ring_applicable( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w, const void* xout )
 {

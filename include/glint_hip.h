@@ -171,8 +171,8 @@ int gh_argmax( uint32_t* out_host, uint32_t* out_dev, const void* v, uint64_t n,
 /* Operations::matmul<s,r> / untemplated_matmul  arch/amd64/common/ops.hh:74-93,212-271 :
  * xout(b, r) = sum_p w(r, p) * x(b, p); w row-major (r, s); fp32 accumulate */
 /* tuning hook: kernel 0 auto / 1 small tiled / 2 streaming through registers / 3 128 x 128 tiles (more than 64 rows) / 4 256 x 256 tiles (many rows) / 5 ring; the number of
- * compute units the streaming and the ring kernel's plans are balanced for (<= 0 keeps the current value; the default is the device's own count); `tile_rows` non-zero: a
- * product is never cut in two along the tokens */
+ * compute units that the plans of the streaming and the ring kernel and of q, k and v of few rows in one launch are balanced for (<= 0 keeps the current value; the default
+ * is the device's own count); `tile_rows` non-zero: a product is never cut in two along the tokens */
 int gh_gemm_set_tuning( int kernel, int target_workgroups, int tile_rows );
 /* measurement / test hook: w1 and w3 with the SiLU gate in one launch (gh_matmul_silu_gate) by the streaming kernel in work-groups of 4 or 8
  * waves, at up to 64 rows where that kernel would not split K; 0: the library's choice, the ring kernel */
@@ -193,7 +193,8 @@ int gh_matmul_fuses_many_rows( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt )
 /* host-only query: 1 when gh_matmul_qkv_rope_append (no kv_out, 16-byte aligned operands) rotates and appends the rows of this many tokens, all or all but a
  * rest of them, in the large tile kernel's epilogue: the caller's test for taking the fused call on many rows */
 int gh_matmul_qkv_fuses_many_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt );
-/* host-only query: 1 when it does so for few tokens, in the epilogue of a product whose work-groups take their weight rows over the whole K range */
+/* host-only query of tests and measurements: 1 when it does so for few tokens, in the epilogue of a product whose work-groups take their weight rows over the whole K
+ * range; never under a forced kernel (gh_gemm_set_tuning) */
 int gh_matmul_qkv_fuses_few_rows( uint64_t s, uint32_t n_kv_heads, uint32_t gqa_size, uint32_t head_size, uint64_t b, gh_dtype dt );
 /* host-only query: how the weight-streaming kernel would cut an (r x s) . (b x s)^T product for the initialised device (256 compute
  * units before initialisation): number of K ranges, k per range (a multiple of 256), weight rows per work-group */

@@ -111,3 +111,23 @@ def test_ring_plan_rejects_what_the_kernel_does_not_take():
     out = (C.c_uint32 * 6)()
     for s, r, b, gated in [(100, 64, 1, 0), ((1 << 21) + 8, 64, 1, 0), (64, 0, 1, 0), (64, 64, 0, 0), (64, 66, 1, 1)]:
         assert _lib.lib().gh_gemm_ring_plan(s, r, b, gated, out) != 0 and b"ring" in _lib.lib().gh_last_error()
+
+
+def test_q_k_v_of_few_rows_leave_their_own_kernel_to_a_forced_one():
+    """The fused product has a kernel of its own for 32 to 64 weight rows a compute unit: a forced kernel goes before it, and the units that plans are balanced for are its."""
+    lib = _lib.lib()
+    shapes = [(4096, 32, 1, 128, 32), (8192, 8, 8, 128, 1), (5120, 40, 1, 128, 16)]
+
+    def takes(shape):
+        return lib.gh_matmul_qkv_fuses_few_rows(*shape, _lib.GH_F16)
+
+    assert [takes(c) for c in shapes] == [1, 1, 1]
+    try:
+        for kernel in (1, 2, 3, 4, 5):
+            _lib.check(lib.gh_gemm_set_tuning(kernel, 0, 0))
+            assert [takes(c) for c in shapes] == [0, 0, 0], kernel
+        _lib.check(lib.gh_gemm_set_tuning(0, 64, 0))              # 160 to 240 rows a unit
+        assert [takes(c) for c in shapes] == [0, 0, 0]
+    finally:
+        _lib.check(lib.gh_gemm_set_tuning(0, 256, 0))
+    assert [takes(c) for c in shapes] == [1, 1, 1]
