@@ -141,6 +141,7 @@ SIGNATURES = {
     "gh_rmsnorm_matmul_silu_gate": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _u64, _i, _vp]),
     "gh_rmsnorm_matmul_qkv_rope_append": (_i, [_vp, _vp, _vp, _vp, _u64, _u64, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _i, _vp]),
     "gh_rmsnorm_qkv_attn_rides": (_i, [_u64, _shp, _i]),
+    "gh_rmsnorm_qkv_attn_preferred": (_i, [_u64, _u32, _shp, _i]),
     "gh_rmsnorm_qkv_attn": (_i, [_vp, _vp, _vp, _vp, _u64, _vp, _vp, _vp, _vp, _vp, _shp, _i, _vp]),
     "gh_soft_sample": (_i, [_vp, _vp, _u64, _u64, _u64, _i, _vp]),
     "gh_kv_append": (_i, [_vp, _vp, _u64, _u32, _i, _vp]),

@@ -1651,6 +1651,9 @@ int attn_static_scratch_init( int device )
   return GH_OK;
 }
 
+// a measurement has asked for a kernel or a cut
+bool attn_decode_forced() { return g_chunk_override != 0 || g_auto_variant != GH_ATTN_AUTO; }
+
 } // namespace gh
 
 using namespace gh;

@@ -19,6 +19,9 @@
 #include <type_traits>
 
 namespace gh {
+
+bool attn_decode_forced(); // gh_attn_decode.hip
+
 namespace {
 
 constexpr float LOG2E = 1.4426950408889634f;
@@ -263,6 +266,16 @@ int gh_rmsnorm_qkv_attn_rides( uint64_t b, const gh_shape* shape, gh_dtype dt )
              && (uint64_t)shape->seq_len * shape->kv_dim <= ( 1ull << 28 ) // (offsets of 32 bits)
            ? 1
            : 0;
+}
+
+// The work-group of a (head, context) walks all of its keys, a turn after the other, where the attention by itself cuts them over idle CUs.  Two launches / one, us, in a graph,
+// 512, 768, 1024 and 2048 keys: 6 heads of 48, 2 contexts 11.3 11.5 11.7 11.9 / 9.9 11.5 12.9 19.4, 8 contexts 12.8 13.9 15.0 19.0 / 10.1 11.8 13.6 21.2; 5 of 64, 2 contexts 11.0
+// 11.7 11.6 11.9 / 10.0 11.5 13.4 19.8; 4 of 16, one context 9.0 8.9 8.9 9.8 / 7.6 8.9 10.1 16.8; 8 of 40 over 8, 16 contexts 16.3 18.7 21.2 31.6 / 11.5 13.9 16.8 27.5.  Up to 512 keys
+// one is faster for every shape tried; beyond, it depends on how many CUs the cut would fill.
+constexpr uint32_t QA_KEYS = 512;
+int gh_rmsnorm_qkv_attn_preferred( uint64_t b, uint32_t max_pos, const gh_shape* shape, gh_dtype dt )
+{
+  return max_pos < QA_KEYS && !attn_decode_forced() && gh_rmsnorm_qkv_attn_rides( b, shape, dt ) == 1 ? 1 : 0;
 }
 
 int gh_rmsnorm_qkv_attn( void* xb, const void* x, const void* norm_weight, const void* wqkv, uint64_t b, const uint32_t* pos_dev, const void* freq_real,

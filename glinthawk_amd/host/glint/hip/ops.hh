@@ -464,11 +464,12 @@ public:
                                                  Config::n_kv_heads, Config::gqa_size, Config::head_size, gh_type<DType>(), this->stream_ ) );
   }
 
-  // All of a layer up to its attention in one launch, where no context stands twice in the batch; attention_rides( batch_size ): whether there is one
-  static bool attention_rides( const uint64_t batch_size )
+  // All of a layer up to its attention in one launch, where no context stands twice in the batch; attention_rides(): whether there is one, and it is
+  // the faster way for positions up to max_pos
+  static bool attention_rides( const uint64_t batch_size, const uint32_t max_pos )
   {
     const gh_shape s = shape();
-    return gh_rmsnorm_qkv_attn_rides( batch_size, &s, gh_type<DType>() ) == 1;
+    return gh_rmsnorm_qkv_attn_preferred( batch_size, max_pos, &s, gh_type<DType>() ) == 1;
   }
   void rmsnorm_qkv_attention( DType* xb,
                               const DType* x,

@@ -851,7 +851,7 @@ private:
       }
     }
     // (a launch that appends and attends reads the old keys while other rows are appended)
-    attention_rides_ = decode && !run.empty() && !balanced_step_ && LlamaOperations::attention_rides( batch_ )
+    attention_rides_ = decode && !run.empty() && !balanced_step_ && LlamaOperations::attention_rides( batch_, max_pos_ )
                        && !stands_twice( std::vector<const void*>( ptrs, ptrs + batch_ ) );
     const size_t bytes = ( ptr_tables( tables_host_ ) - tables_host_ ) + run.size() * 2 * table_stride() * sizeof( void* ); // a multiple of 16
     tables_uploaded_ = true;

@@ -240,8 +240,10 @@ int gh_rmsnorm_matmul_qkv_rope_append( void* q, const void* x, const void* norm_
  * (dim <= 320, heads of up to 64) at few contexts: xb(b, dim) = attention of context i over its rows [0, pos_i], of which the last is
  * written here (token_rows_dev[i]).  wqkv as above; empty contexts (NULL) are skipped.  No context may stand in the batch twice: old keys are read while the new
  * ones of other rows are written (gh_rmsnorm_matmul_qkv_rope_append and an attention behind it take such a batch).  gh_rmsnorm_qkv_attn_rides, host-only: 1
- * where the launch takes the shape (it refuses any other) */
+ * where the launch takes the shape (it refuses any other).  gh_rmsnorm_qkv_attn_preferred, host-only: 1 where it is also the faster way for positions of at most max_pos, and
+ * no kernel or cut of the attention is forced (gh_attn_set_auto_variant, gh_attn_set_chunk): the caller's test for taking it */
 int gh_rmsnorm_qkv_attn_rides( uint64_t b, const gh_shape* shape, gh_dtype dt );
+int gh_rmsnorm_qkv_attn_preferred( uint64_t b, uint32_t max_pos, const gh_shape* shape, gh_dtype dt );
 int gh_rmsnorm_qkv_attn( void* xb, const void* x, const void* norm_weight, const void* wqkv, uint64_t b, const uint32_t* pos_dev, const void* freq_real,
                          const void* freq_imag, const void* const* layer_rows_dev, void* const* token_rows_dev, const gh_shape* shape, gh_dtype dt,
                          gh_stream stream );

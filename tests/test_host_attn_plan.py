@@ -76,6 +76,31 @@ def test_workspace_does_not_hang_on_the_kernel_that_auto_stands_for():
             _lib.check(L.gh_attn_set_auto_variant(GH_ATTN_AUTO))
 
 
+def test_attention_in_the_launch_of_its_projections_up_to_a_length():
+    """Where its one work-group a head walks the keys no slower than the attention by itself; a kernel or a cut that is forced is that of the attention by itself."""
+    L, s = _lib.lib(), SHAPES["tiny"].c()
+    s.seq_len = 4096
+
+    def preferred(batch, max_pos):
+        return L.gh_rmsnorm_qkv_attn_preferred(batch, max_pos, C.byref(s), _lib.GH_F32)
+
+    for batch in (2, 16, 42):
+        assert [preferred(batch, p) for p in (0, 255, 511, 512, 4095)] == [1, 1, 1, 0, 0]
+        assert L.gh_rmsnorm_qkv_attn_rides(batch, C.byref(s), _lib.GH_F32) == 1                   # taken all the same
+    assert preferred(1, 0) == 0 and preferred(43, 0) == 0                                         # not taken at all
+    try:
+        L.gh_attn_set_chunk(64)
+        assert preferred(4, 100) == 0
+        L.gh_attn_set_chunk(0)
+        assert preferred(4, 100) == 1
+        _lib.check(L.gh_attn_set_auto_variant(GH_ATTN_GENERIC))
+        assert preferred(4, 100) == 0
+    finally:
+        L.gh_attn_set_chunk(0)
+        _lib.check(L.gh_attn_set_auto_variant(GH_ATTN_AUTO))
+    assert preferred(4, 100) == 1
+
+
 def test_the_case_that_used_to_overflow():
     # 70B shape, limit 64: a batch of 17 rows at the last position is cut into more partials than the full batch
     shape = SHAPES["70B"]
