@@ -1365,27 +1365,56 @@ int merge_splits( const WindowOut<E>& out, const SplitPlan& plan, const WindowRo
 // What counts is the waves on the chip, some 4 to 8 a CU, and that work-groups come out even over the CUs; beyond that neighbouring heads in a work-group, which read
 // neighbouring pieces of a cache row.  So eight waves, on one head while there are no more streams of keys than CUs (cut further where that leaves CUs idle and a stream
 // is long: the merge is a launch), on two heads up to twice as many and on four up to four times.
+struct DotPlan
+{
+  uint32_t waves, heads; // of a work-group
+  uint64_t splits;
+};
+DotPlan plan_dot( const WindowShape& s, uint64_t rows, uint64_t most )
+{
+  const uint64_t streams = rows * s.heads, cus = (uint64_t)cu_count(), weight = most * ( s.values_are_keys ? 1 : 2 );
+  DotPlan p { 8, streams <= cus ? 1u : streams <= 2 * cus ? 2u : streams <= 4 * cus ? 4u : 2u, 1 };
+  // (16 rows of 4097 keys 163 | 84.7 us with four ranges of a head's keys, 158 | 81.1 with two; 48 rows of 64 13.4 | 9.7 and 11.3 | 7.6)
+  if ( p.heads == 2 && ( streams <= 2 * cus ? most > 3072 : most <= 192 ) ) {
+    p.waves = 4;
+  }
+  while ( s.heads % p.heads != 0 ) {
+    p.heads /= 2;
+  }
+  // Many short streams of an odd number of heads: of eight waves on one head most have no keys (120 rows of 5 heads, 33 keys 7.5 | 7.8 us, 5.9 | 5.6 with four).
+  if ( p.heads == 1 && streams > 2 * cus && most <= 192 ) {
+    p.waves = 4;
+  }
+  // Splits of 128 keys, from sixteen of them on of 256 (2 rows of 5 heads, 2500 keys 13.6 | 12.5 us in 27 splits, 11.2 | 10.4 in 16; one of 6 of 96, 16385 keys 20.0 | 15.2 in
+  // 16, 18.1 | 15.1 in 32).
+  if ( const uint64_t idle = cus / streams; idle >= 2 && weight >= ( idle >= 4 ? 1024u : 2048u ) ) {
+    p.splits = std::max<uint64_t>( 1, std::min( { idle, most / 128, std::max<uint64_t>( 16, most / 256 ), (uint64_t)64 } ) );
+  }
+  // Long streams whose work-groups leave a third of the CUs without one, in their only round or in the last: a CU takes in some 35 GB/s, so that is lost.  Four waves on two
+  // heads then, in as many splits as make two a CU; more work-groups than CUs are cut by three.  11 rows of 12 heads, 16385 keys 238 | 118 us, 182 | 96 so (195 | 107 by
+  // window_decode_kernel), 4097 keys 62 | 33 and 51 | 30 (57 | 33); 43 rows of 6 of 96, 16385 keys 476 | 238 and 293 | 150 (451 | 250); 100 of them, values that are keys,
+  // 445 and 352 (413).
+  const uint64_t groups = streams / p.heads, rounds = ( groups + cus - 1 ) / cus;
+  if ( s.heads % 2 == 0 && weight >= 4096 && 8 * groups >= 3 * cus && 100 * groups <= 69 * rounds * cus ) {
+    if ( groups <= cus ) {
+      p.waves = 4;
+      p.heads = streams <= 2 * cus ? 2 : p.heads;
+      p.splits = std::max<uint64_t>( 1, 2 * cus / ( streams / p.heads ) );
+    } else {
+      p.splits = 3;
+    }
+  }
+  return p;
+}
 int attend_dot( const WindowOut<__bf16>& out, const __bf16* q, const float* bias, const WindowRows& wr, const WindowShape& s, uint64_t rows, uint32_t max_pos, hipStream_t st )
 {
   const uint64_t most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
-  const uint64_t streams = rows * s.heads, cus = (uint64_t)cu_count();
-  uint32_t waves = 8, heads = streams <= cus ? 1 : streams <= 2 * cus ? 2 : streams <= 4 * cus ? 4 : 2;
-  // (16 rows of 4097 keys 163 | 84.7 us with four ranges of a head's keys, 158 | 81.1 with two; 48 rows of 64 13.4 | 9.7 and 11.3 | 7.6)
-  if ( heads == 2 && ( streams <= 2 * cus ? most > 3072 : most <= 192 ) ) {
-    waves = 4;
-  }
-  while ( s.heads % heads != 0 ) {
-    heads /= 2;
-  }
-  uint64_t splits = 1;
-  if ( const uint64_t idle = cus / streams; idle >= 2 && most * ( s.values_are_keys ? 1 : 2 ) >= ( idle >= 4 ? 1024u : 2048u ) ) {
-    splits = std::min( { idle, most / 64, (uint64_t)64 } );
-  }
+  const auto [waves, heads, splits] = plan_dot( s, rows, most );
   SplitPlan plan;
   if ( int rc = cut_keys( s, rows, most, splits, st, &plan ) ) {
     return rc;
   }
-  const uint64_t grid = streams / heads * plan.splits;
+  const uint64_t grid = rows * ( s.heads / heads ) * plan.splits;
   GH_REQUIRE( grid < ( 1ull << 31 ), "gh_attn_window: grid too large" );
   auto launch = [&]( auto nw, auto hb ) {
     constexpr int NW = decltype( nw )::value, HB = decltype( hb )::value;
@@ -1400,11 +1429,11 @@ int attend_dot( const WindowOut<__bf16>& out, const __bf16* q, const float* bias
   const std::integral_constant<int, 2> two {};
   const std::integral_constant<int, 1> one {};
   if ( heads == 4 ) {
-    launch( eight, four );
+    waves == 4 ? launch( four, four ) : launch( eight, four );
   } else if ( heads == 2 ) {
     waves == 4 ? launch( four, two ) : launch( eight, two );
   } else {
-    launch( eight, one );
+    waves == 4 ? launch( four, one ) : launch( eight, one );
   }
   GH_LAUNCH_CHECK();
   return merge_splits( out, plan, wr, s, rows, st );

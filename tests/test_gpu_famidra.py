@@ -192,11 +192,12 @@ ATTENTIONS = {
 
 
 # streams of keys (rows x heads) up to the CUs, cut into splits and not; up to two, four times as many and more; short and long; heads that do not divide by
-# two or four; head sizes that leave lanes idle
+# two or four; head sizes that leave lanes idle; long streams whose work-groups are cut because they would leave CUs idle, up to the CUs and beyond
 @pytest.mark.parametrize("shared", [False, True])
 @pytest.mark.parametrize("heads,dim,vdim,rows,keys", [(4, 128, 128, 1, 1500), (2, 72, 128, 40, 2100), (3, 96, 96, 5, 40), (32, 128, 128, 1, 64), (8, 128, 104, 40, 250),
                                                       (4, 72, 72, 70, 3100), (4, 128, 128, 150, 70), (6, 80, 72, 100, 33), (4, 128, 128, 300, 150), (4, 72, 128, 300, 250),
-                                                      (5, 128, 128, 240, 200)])
+                                                      (5, 128, 128, 240, 200), (6, 96, 96, 24, 4200), (6, 72, 72, 52, 4200), (6, 72, 80, 100, 4200), (5, 128, 128, 120, 33),
+                                                      (2, 96, 96, 1, 5000), (12, 72, 72, 50, 8500)])
 def test_decode_of_heads_with_keys_of_their_own(heads, dim, vdim, rows, keys, shared):
     """Against 64 bits: a rounding to bf16 and fp32 sums.  Contexts of all lengths and none, a window with kept keys, a bias by distance, keys whose scores are -inf."""
     import torch
