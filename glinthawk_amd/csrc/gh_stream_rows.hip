@@ -415,7 +415,7 @@ __global__ __launch_bounds__( 256 ) void scale_rows_kernel( float* __restrict__ 
 }
 
 // The same with the index of each row's maximum (the lowest of equal ones; 0 where the row begins with NaN, as in gh_argmax), one work-group a row.
-// Bound by latency; with a launch between the two 32 rows of 4096 took 4.7 + 4.1 us.  r % 4 == 0, 16-byte aligned rows
+// Bound by latency, and by what one CU takes in where a row is long: with a launch between the two 32 rows of 4096 took 4.7 + 4.1 us.  r % 4 == 0, 16-byte aligned rows
 __global__ __launch_bounds__( 1024 ) void scale_rows_argmax_kernel( float* __restrict__ out, uint32_t* __restrict__ best_out, ProductView<float> y, uint32_t r, float scale )
 {
   __shared__ float s_val[1024 / WAVE];
@@ -679,7 +679,11 @@ int gh_matmul_scaled_argmax( float* out, uint32_t* argmax, const void* x, const 
   GH_REQUIRE( out && argmax && x && w, "gh_matmul_scaled_argmax: NULL pointer" );
   GH_REQUIRE( s > 0 && s < ( 1ull << 31 ) && r > 0 && r < ( 1ull << 31 ) && rows < ( 1ull << 31 ), "gh_matmul_scaled_argmax: bad shape" );
   GH_REQUIRE( dt == GH_BF16 || dt == GH_F32, "gh_matmul_scaled_argmax: unsupported dtype %d", (int)dt );
-  if ( r % 4 != 0 || !aligned16( out ) ) {
+  // A few long rows: sums and scale of a row over the whole chip, and a maximum that has more of it under way.  us, 512 k in bf16, two launches / one, at 1, 4, 8 and 32 rows:
+  // 4096 values 10.8 10.9 11.1 11.3 / 9.8 9.9 10.0 10.2, 32000 15.9 16.6 17.4 21.7 / 15.1 15.4 15.6 17.6, 64000 24.4 25.2 26.6 34.9 / 23.6 24.4 25.2 29.0, 128256
+  // 41.2 43.5 46.9 56.5 / 43.0 44.9 45.5 51.0.
+  const bool few_and_long = r > ( 1u << 16 ) && rows < 8;
+  if ( r % 4 != 0 || !aligned16( out ) || few_and_long ) {
     if ( int rc = gh_matmul_scaled( out, x, w, s, r, rows, scale, dt, stream ) ) {
       return rc;
     }

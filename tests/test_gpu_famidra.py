@@ -162,7 +162,8 @@ def test_start_of_a_step(dtype, width, batch, n_tokens, pinned):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("rows,s,r", [(32, 4096, 4096), (1, 64, 4), (3, 100, 36), (5, 256, 8196), (2, 64, 32000), (200, 128, 1000), (4, 64, 30)])
+@pytest.mark.parametrize("rows,s,r", [(32, 4096, 4096), (1, 64, 4), (3, 100, 36), (5, 256, 8196), (2, 64, 32000), (200, 128, 1000), (4, 64, 30), (3, 64, 65536),
+                                      (7, 64, 65540), (8, 64, 65540)])
 def test_scaled_product_with_its_argmax(dtype, rows, s, r):
     """The same bits as the product and the argmax one after the other: ties, NaN first and elsewhere, rows of -inf."""
     import torch
