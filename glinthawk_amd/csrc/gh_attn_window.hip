@@ -1451,13 +1451,14 @@ int attend_decode( const WindowOut<__bf16>& out, const __bf16* q, const float* b
   }
   const uint64_t blocks = s.heads / head_cols, groups = rows * blocks, most = std::min<uint64_t>( (uint64_t)max_pos + 1, (uint64_t)s.window + s.keep_first );
   // Eight waves on the keys of a row where work-groups of four would leave room on the CUs and a row has four tiles or more (below eight tiles some of the
-  // waves have none); with K and V apart a CU holds one such work-group, which pays only while they are few.  us, 32 heads of 128, rows x keys, four waves / eight.  Values that are keys: 1 x 300
-  // 11.0 / 7.6, 8 x 300 13.8 / 9.2, 24 x 300 15.7 / 17.6, 1 x 2048 26 / 18, 32 x 1025 49.4 / 46.9, 48 x 1025 69.2 / 65.0.  Both: 1 x 1025 18.9 / 16.5, 4 x 1025
-  // 24.8 / 26.8, 8 x 300 17.5 / 13.1, 16 x 300 20.3 / 24.0.
+  // waves have none); with K and V apart a CU holds one such work-group, which pays only while they are few.  us, rows x keys, four waves / eight.  32 heads of 64 with keys of
+  // their own, values that are keys: 1 x 300 8.7 / 6.1, 8 x 300 10.0 / 6.6, 24 x 300 10.2 / 12.0, 32 x 1025 29.6 / 28.8, 48 x 1025 41.0 / 39.7; both: 1 x 300 9.9 / 8.0, 8 x 300
+  // 11.8 / 8.8, 8 x 1025 20.2 / 22.0.  32 heads of 128 in groups of four, values that are keys: 24 x 300 12.3 / 8.4, 48 x 300 11.7 / 11.4; both: 8 x 1025 14.8 / 13.5, 8 x 2048 19.0 /
+  // 22.2, 24 x 300 14.9 / 10.9, 48 x 300 17.1 / 20.4.
   const bool wide = s.values_are_keys ? ( groups < 16ull * cu_count() && most >= 16 * STEP_KEYS ) || ( groups <= (uint64_t)cu_count() && most >= 4 * STEP_KEYS )
                                       : most >= 4 * STEP_KEYS && ( 4 * groups <= (uint64_t)cu_count() || ( groups <= (uint64_t)cu_count() && most <= 16 * STEP_KEYS ) );
-  // Two heads a work-group where there are more work-groups than the CUs hold and few keys to each: half as many starts (32 x 64 15.2 -> 12.0, 32 x 300
-  // 36.2 -> 32.8; 32 x 1025 92 -> 93).
+  // Two heads a work-group where there are more work-groups than the CUs hold and few keys to each: half as many starts (32 heads of 64 with keys of their own: 32 x 64
+  // 10.5 -> 7.4, 32 x 300 22.8 -> 18.0; longer rows gain up to a fifth or nothing, 32 x 2048 100 -> 85, 48 x 1025 80 -> 80, and stay as they were).
   const bool pair = !s.values_are_keys && !wide && blocks % 2 == 0 && groups >= 3ull * cu_count() && most <= 16 * STEP_KEYS;
   const uint64_t head_blocks = pair ? blocks / 2 : blocks;
   SplitPlan plan;

@@ -236,11 +236,11 @@ uint64_t qkv_share( uint64_t r )
 
 } // namespace
 
-// Both routes, us in a graph with cold weights, product over K ranges and epilogue / this kernel: 7B (48 rows a CU, 4096 k) at 1 row 21.7 / 18.3, 32 22.4 / 19.0, 64 25.7 / 22.8,
-// 77 29.3 / 25.3; 13B (60, 5120) 29.8 / 27.9, 32.6 / 30.1, 36.8 / 36.3, 39.6 / 39.9; 70B (40, 8192) 31.8 / 30.8, 34.7 / 31.6, 39.0 / 39.1, 44.5 / 45.1; 6144 x 4096 (24 rows a CU)
-// 14.0 / 15.9, 16.0 / 16.2, 19.0 / 20.0, 19.8 / 22.5.  So a step costs its weights at a CU's share of the memory's rate, or weights and activations at what L2 delivers to a CU
-// (50 bytes a ns), but no less than its barrier and its trip through LDS; the other route its estimate and the second launch.  Every work-group reads all activations, and
-// behind the kernels of a layer they come from beyond L2: from some 640 KB on what is left of the gain is lost there (a layer of 70B at 64 rows 3 us slower, of 7B at 77 even).
+// Both routes, us in a graph with cold weights, product over K ranges and epilogue / this kernel, at 1, 32 and 64 rows: 7B (48 rows a CU, 4096 k) 21.7 / 18.3, 22.4 / 19.0,
+// 25.7 / 22.8; 13B (60, 5120) 29.8 / 27.9, 32.6 / 30.1, 36.8 / 36.3; 70B (40, 8192) 31.8 / 30.8, 34.7 / 31.6, 39.0 / 39.1; 6144 x 4096 (24 rows a CU) 14.0 / 15.9, 16.0 / 16.2,
+// 19.0 / 20.0.  So a step costs its weights at a CU's share of the memory's rate, or weights and activations at what L2 delivers to a CU (50 bytes a ns), but no less than its
+// barrier and its trip through LDS; the other route its estimate and the second launch.  Every work-group reads all activations, and behind the kernels of a layer they come from
+// beyond L2: from some 640 KB on what is left of the gain is lost there (a layer of 70B at 64 rows 3 us slower).  A tile of more than 64 activation rows gained nothing in a layer.
 // Fewer than 32 rows a CU: the other route, also where this one would be a microsecond faster (a short K), so that small models sum in the order that wq and wkv alone have.
 constexpr uint32_t QKV_LEAST = 32;
 constexpr uint64_t QKV_MOST_BYTES = 640 << 10;
@@ -248,7 +248,8 @@ constexpr double QKV_START_NS = 4000.0, QKV_EPILOGUE_NS = 4200.0;
 bool gemm_qkv_applicable( uint64_t s, uint64_t b, const void* x, const void* w, const void* q, const QkvRows& rows )
 {
   const uint64_t r = rows.dim + 2ull * rows.kv_dim;
-  const bool takes = !gemm_kernel_forced() && b > 0 && b <= 64 && b * s * sizeof( __half ) < QKV_MOST_BYTES && r <= 0x7fffffffull && qkv_share( r ) >= QKV_LEAST && qkv_share( r ) <= QKV_ROWS && s % 8 == 0 && s <= ( 1u << 21 ) // 64 rows of a descriptor are at most 2^28 bytes
+  const bool takes = !gemm_kernel_forced() && b > 0 && b <= 64 && b * s * sizeof( __half ) < QKV_MOST_BYTES && r <= 0x7fffffffull && qkv_share( r ) >= QKV_LEAST
+         && qkv_share( r ) <= QKV_ROWS && s % 8 == 0 && s <= ( 1u << 21 ) // 64 rows of a descriptor are at most 2^28 bytes
          && rows.dim % 4 == 0 && rows.kv_dim % 4 == 0 && rows.head_size % 4 == 0
          && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) | reinterpret_cast<uintptr_t>( q ) ) & 15u ) == 0;
   if ( !takes ) {

@@ -495,6 +495,51 @@ def test_mlstm(name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,batch", [(4096, 1), (4096, 7), (4096, 32), (1000, 5), (4096, 200), (4104, 200)])
+def test_mlstm_gates_of_many_planes(width, batch, dtype):
+    """Two tokens of each context, one a call: the walk adds up the gates' sums over the K ranges that the product left, a plane a lane (in 16 bits
+    sixteen of them; where the gates of 192 rows and more are a product of their own, one or, by the width, sixteen).  The state's m is made of the gates alone."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    H, d, dv, cap, eps = 2, 16, 24, 15.0, 1e-4
+    m = GhMlstm(H, d, dv, cap, eps)
+    rng = np.random.default_rng(width + batch)
+    rows, gate_row = ops.mlstm_weight_rows(m)
+    hd, hv = H * d, H * dv
+    w = np.zeros((rows, width), np.float32)
+    w[:2 * hd + 2 * hv] = rng.standard_normal((2 * hd + 2 * hv, width)) / np.sqrt(width)
+    w[gate_row:gate_row + 2 * H] = 3 * rng.standard_normal((2 * H, width)) / np.sqrt(width)
+    w = M.to_bf16(w)
+    bi, bf, norm = M.to_bf16(rng.standard_normal(H)), M.to_bf16(np.array([-2.0, 3.0])), M.to_bf16(1 + 0.2 * rng.standard_normal(hv))
+    x = M.to_bf16(rng.standard_normal((2, batch, width)))
+    X, W = x.astype(np.float64), w.astype(np.float64)
+    split = np.split(W[:2 * hd + 2 * hv], [hd, 2 * hd, 2 * hd + hv])
+    q, k = (X @ split[0].T).reshape(2, batch, H, d) * d ** -0.5, (X @ split[1].T).reshape(2, batch, H, d)
+    v, g = (X @ split[2].T).reshape(2, batch, H, dv), X @ split[3].T
+    li = P.soft_cap(X @ W[gate_row:gate_row + H].T + bi, cap)
+    lf = P.log_sigmoid(P.soft_cap(X @ W[gate_row + H:gate_row + 2 * H].T + bf, cap))
+    weights = [dev(a, dtype) for a in (w, bi, bf, norm)]
+    state = torch.full((batch, ops.mlstm_state_bytes(m) // 4), float("nan"), device="cuda")
+    table = ops.row_table([state[i].data_ptr() for i in range(batch)])
+    tol = 5e-5 if dtype == "f32" else 4e-2
+    for t in range(2):
+        got = back(ops.mlstm_forward(dev(x[t], dtype), weights[0], m, *weights[1:], table, torch.full((batch,), t, dtype=torch.int32, device="cuda"), 1))
+        at = state.cpu().numpy().astype(np.float64)
+        for i in range(batch):
+            o, (S, n, mm) = P.mlstm_recurrence(q[:t + 1, i], k[:t + 1, i], v[:t + 1, i], li[:t + 1, i], lf[:t + 1, i])
+            want = P.rms_norm(o, eps).reshape(t + 1, hv) * norm / (1 + np.exp(-g[:t + 1, i]))
+            # the output is divided by n . q and normed, whose rounding, some 2e-6 of |n| |q|, grows by as much as they cancel: up to ten times is looked at
+            if (np.abs((n * q[t, i]).sum(-1)) >= 0.1 * np.linalg.norm(n, axis=-1) * np.linalg.norm(q[t, i], axis=-1)).all():
+                assert_rows(got[i:i + 1], want[t:], tol, f"{t} {i}", 1.0 if dtype == "f32" else 5.0)
+            # at 200 rows of 16 bits k and v are rounded, the gates' sums are not
+            assert_rows(at[i, :hd * dv].reshape(H, -1), S.reshape(H, -1), tol, f"{t} {i}: S")
+            assert_rows(at[i, hd * dv:hd * dv + hd].reshape(1, -1), n.reshape(1, -1), tol, f"{t} {i}: n")
+            # fp32 sums of exact products: a few units of 2^-24 of sqrt(width) terms of size 3 / sqrt(width), through gates whose slopes are at most 1
+            assert np.abs(at[i, -H:] - mm).max() <= 1e-4, f"{t} {i}: m"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_mlstm_extreme_gates(dtype):
     """A far token written once with a strong input gate and kept by open forget gates must still be read, and a closed forget gate
     must wipe it."""
