@@ -558,7 +558,9 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
 // work-group  4 waves on one (context, kv head), 32 query columns a wave; a column is (token, query head) with the query heads of a group side
 //             by side where their number is a power of two, else one query head per work-group
 // keys        64 at a time: the tiles of the kept first tokens in front of the window, then those of the window of the work-group's
-//             tokens.  A tile that every column sees whole takes no mask, one farther away than the bias table is long a constant bias.
+//             tokens.  A wave leaves out a tile that none of its columns sees, takes no mask for one that all of them see whole, and a
+//             constant bias for one farther away than the bias table is long.  Else the table's copy in LDS has entries in front of
+//             distance 0 and behind the last, where they fit: a lane reads the biases of its 32 keys with one address and offsets.
 // scores^T    K Q^T by v_mfma_f32_32x32x16_bf16 (K out of LDS, Q in registers): a lane holds 32 of the tile's 64 scores of ITS column, the
 //             lane 32 further on the others, so maximum and sum stay in the lane but for one exchange
 // values      O^T += V^T P^T: the weights are, as they lie, the right operand; V^T comes out of LDS by transposing reads.  The weights
@@ -567,16 +569,32 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
 //             rows are in registers while this one is multiplied, and two work-groups share a CU.  Where values are keys both products
 //             read one tile: the low four bits of the row, pairs exchanged, keep the plain reads (16 rows, one chunk) and the
 //             transposing ones (4 rows, 4 chunks) apart.
+// order       the longest work-groups of ALL contexts and heads start first.  Those of one pair next to each other, for its keys in L2, left
+//             the last pairs' long ones to the end: 4.9 of 8 waves in flight on average, 6.7 now.  The keys then come out of the Infinity
+//             Cache (600 MB at 8 x 1024 tokens), which is not what bounds it.
+// bound       vector and matrix work of two waves a SIMD, which overlap little.  8 x 1024 tokens, 32 heads of 128, window 1024, 512 distances:
+//             228 us -> 200 with fewer vector instructions (702 -> 510 a tile and wave) -> 155 with the order; 4 x 2048 tokens without a
+//             bias: 305 -> 274 -> 240, keys as values 303 -> 275 -> 221.  The products run at 0.9 PFLOP/s there, both terms counted.
+//             Still fewer vector instructions (430 -> 370), other priorities for the waves in their products: no change.
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY = 8.0f; // the reference point of a column's exponentials moves when its maximum has grown by 2^LAZY
 constexpr uint32_t TILE_KEYS = 64;
 constexpr uint32_t BIAS_LDS = 8192; // floats of bias table a work-group can hold
+// Entries around a head's table, where they fit: from a wave's 32 tokens to the keys of a tile that touches the table the distances reach 94 before its start and behind its end
+constexpr uint32_t BIAS_PAD = 96;
 typedef __attribute__( ( address_space( 3 ) ) ) char lds_char;
 typedef short v4s __attribute__( ( ext_vector_type( 4 ) ) );
 typedef __attribute__( ( address_space( 3 ) ) ) v4s* lds_v4s;
 typedef Mfma<__bf16>::x8 bf16x8;
 
 __device__ __forceinline__ uint32_t shared_swizzle( uint32_t row ) { return ( ( row & 3 ) << 2 ) | ( ( row >> 2 ) & 3 ); }
+
+// two values rounded to bf16, the first in the low half
+__device__ __forceinline__ uint32_t bf16_pair( float a, float b )
+{
+  typedef __bf16 pair_t __attribute__( ( ext_vector_type( 2 ) ) );
+  return __builtin_bit_cast( uint32_t, pair_t { (__bf16)a, (__bf16)b } );
+}
 
 // KS: steps of 16 of the query/key size; VB: blocks of 32 of the value size
 template<int KS, int VB, bool SHARED>
@@ -588,18 +606,20 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
                                                                  uint32_t head_cols,  // query heads side by side in the columns
                                                                  uint32_t col_blocks, // work-groups along the tokens of a pair
                                                                  uint32_t n_pairs,    // contexts x kv heads x (query heads of a group / head_cols)
-                                                                 uint32_t bias_floats )
+                                                                 uint32_t bias_row,   // floats of a head's bias table in LDS; 0: no bias
+                                                                 uint32_t bias_pad )  // its entries in front of distance 0 and behind the last one
 {
   extern __shared__ uint4 lds16[];
   uint4* s_k = lds16;
   uint4* s_v = SHARED ? s_k : s_k + TILE_KEYS * 16;
   float* s_factor = reinterpret_cast<float*>( s_v + TILE_KEYS * 16 );  // SHARED: of the tile's keys, times scale and log2(e)
-  float* s_bias = s_factor + ( SHARED ? TILE_KEYS : 0 );               // (head_cols, n_dist), times log2(e)
+  float* s_bias = s_factor + ( SHARED ? TILE_KEYS : 0 );               // (head_cols, bias_row), times log2(e)
 
-  // all column blocks of a pair on one XCD, next to each other in time: its keys come into one L2 once; the longest first
+  // all column blocks of a pair on one XCD; the longest blocks of all pairs first
   const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const uint32_t cb = col_blocks - 1 - slot % col_blocks;
-  const uint32_t pair = ( slot / col_blocks ) * 8 + xcd;
+  const uint32_t xcd_pairs = ( n_pairs + 7 ) / 8;
+  const uint32_t cb = col_blocks - 1 - slot / xcd_pairs;
+  const uint32_t pair = ( slot % xcd_pairs ) * 8 + xcd;
   if ( pair >= n_pairs ) {
     return;
   }
@@ -621,9 +641,17 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
   const bool col_ok = tok < wr.n_tokens;
   const uint32_t pos = start + ( col_ok ? tok : tok_last ); // a column without a query does as the last one and is not stored
   const uint32_t pos_first = start + tok_wg, pos_last = start + tok_last;
+  // those of the wave's own columns
+  const uint32_t wave_col = __builtin_amdgcn_readfirstlane( wave ) * 32;
+  const uint32_t wave_first = start + min( tok_wg + wave_col / head_cols, tok_last ), wave_last = start + min( tok_wg + ( wave_col + 31 ) / head_cols, tok_last );
 
-  for ( uint32_t i = threadIdx.x; i < bias_floats; i += 256 ) {
-    s_bias[i] = bias[(uint64_t)h0 * s.n_dist + i] * LOG2E;
+  if ( bias_row == 0 && threadIdx.x == 0 ) {
+    s_bias[0] = 0.0f;
+  }
+  for ( uint32_t c = 0; c < ( bias_row > 0 ? head_cols : 0 ); c++ ) {
+    for ( uint32_t i = threadIdx.x; i < bias_row; i += 256 ) { // distances before 0 as 0, those past the table as its last
+      s_bias[c * bias_row + i] = bias[(uint64_t)( h0 + c ) * s.n_dist + min( i - min( i, bias_pad ), s.n_dist - 1 )] * LOG2E;
+    }
   }
 
   bf16x8 qb[KS];
@@ -649,7 +677,10 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
 
   // a thread's four 16-byte pieces of a tile of K and of V: row threadIdx / 16 + 16 i, chunk threadIdx % 16
   const uint32_t ld_chunk = threadIdx.x & 15, ld_row = threadIdx.x >> 4;
-  u32x4_t rk[4], rv[SHARED ? 1 : 4];
+  const uint32_t row_bytes = s.row_elems() * sizeof( __bf16 );
+  const uint32_t at_k = ( g * s.dpad + ld_chunk * 8 ) * sizeof( __bf16 ), at_v = ( s.k_elems() + g * s.vpad + ld_chunk * 8 ) * sizeof( __bf16 );
+  const bool k_chunk = ld_chunk * 8 < s.dpad && ld_chunk < 2 * KS, v_chunk = ld_chunk * 8 < s.vpad && ld_chunk < 4 * VB; // a thread past the head's size keeps its zeros
+  u32x4_t rk[4] = {}, rv[SHARED ? 1 : 4] = {};
   const float* factors = reinterpret_cast<const float*>( base + wr.factors );
   float rf = 0.0f;
   auto load = [&]( uint32_t i ) {
@@ -657,19 +688,26 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
     if ( SHARED && threadIdx.x < TILE_KEYS ) {
       rf = factors[factor_index( min( t0 + threadIdx.x, end - 1 ), g, s.kv_heads )];
     }
-#pragma unroll
-    for ( int k = 0; k < 4; k++ ) {
-      const uint32_t key = t0 + ld_row + 16 * k;
-      rk[k] = u32x4_t { 0, 0, 0, 0 };
-      const __bf16* row = cache + (uint64_t)min( key, end - 1 ) * s.row_elems();
-      if ( key < end && ld_chunk * 8 < s.dpad && ld_chunk < 2 * KS ) {
-        rk[k] = *(global_u32x4_t*)( row + g * s.dpad + ld_chunk * 8 );
+    const char* tile = reinterpret_cast<const char*>( cache ) + (uint64_t)t0 * row_bytes;
+    auto load_row = [&]( int k, const char* at, uint32_t lane_offset ) __attribute__( ( always_inline ) ) {
+      if ( k_chunk ) {
+        rk[k] = *(global_u32x4_t*)( at + ( lane_offset + at_k ) );
       }
       if constexpr ( !SHARED ) {
-        rv[k] = u32x4_t { 0, 0, 0, 0 };
-        if ( key < end && ld_chunk * 8 < s.vpad && ld_chunk < 4 * VB ) {
-          rv[k] = *(global_u32x4_t*)( row + s.k_elems() + g * s.vpad + ld_chunk * 8 );
+        if ( v_chunk ) {
+          rv[k] = *(global_u32x4_t*)( at + ( lane_offset + at_v ) );
         }
+      }
+    };
+    if ( t0 + TILE_KEYS <= end ) { // whole: one address for the wave and the lane's row
+#pragma unroll
+      for ( int k = 0; k < 4; k++ ) {
+        load_row( k, tile + (uint64_t)( 16 * k ) * row_bytes, ld_row * row_bytes );
+      }
+    } else { // (past the last key that key again: no column sees it there)
+#pragma unroll
+      for ( int k = 0; k < 4; k++ ) {
+        load_row( k, tile, min( ld_row + 16 * k, end - 1 - t0 ) * row_bytes );
       }
     }
   };
@@ -699,7 +737,9 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
     }
   }
   float m = NO_KEY, l = 0.0f;
-  const float* my_bias = s_bias + hc * s.n_dist;
+  const float* my_bias = s_bias + hc * bias_row + bias_pad;
+  const uint32_t n_dist = bias_row > 0 ? s.n_dist : 1;
+  auto offset_of = []( int sub, int v ) { return 32 * sub + 8 * ( v / 4 ) + v % 4; }; // of a register's key from key_l
 
   load( 0 );
   for ( uint32_t i = 0; i < tiles; i++ ) {
@@ -710,43 +750,57 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
       load( i + 1 );
     }
     const uint32_t t0 = tile_at( i );
-    mfma_f32x16 st[2];
+    const uint32_t last_key = t0 + TILE_KEYS - 1;
+    const bool in_window = i >= kept_tiles;
+    if ( in_window && ( t0 > wave_last || ( t0 >= s.keep_first && wave_first - min( last_key, wave_first ) >= s.window ) ) ) {
+      continue; // keys that none of the wave's columns sees
+    }
+    const bool far = bias_row == 0 || ( last_key <= wave_first && wave_first - last_key >= n_dist - 1 ); // every distance in the table's last row
+    const bool past_window = in_window && wave_last - t0 >= s.window && last_key >= s.keep_first;
+    const bool edge = in_window ? last_key > wave_first || past_window : last_key >= kept;
+    mfma_f32x16 sx[2];
+#pragma unroll
+    for ( int k = 0; k < KS; k++ ) { // (the two halves in turn: a product that waits for the one before it leaves the matrix unit idle)
+#pragma unroll
+      for ( int sub = 0; sub < 2; sub++ ) {
+        const uint32_t row = 32 * sub + r;
+        const bf16x8 a = __builtin_bit_cast( bf16x8, s_k[row * 16 + ( ( 2 * k + g2 ) ^ ( SHARED ? shared_swizzle( row ) : row & 15 ) )] );
+        const mfma_f32x16 zero = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+        sx[sub] = Mfma<__bf16>::k16( a, qb[k], k == 0 ? zero : sx[sub] );
+      }
+    }
+    float st[2][16];
 #pragma unroll
     for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
       for ( int v = 0; v < 16; v++ ) {
-        st[sub][v] = 0.0f;
-      }
-#pragma unroll
-      for ( int k = 0; k < KS; k++ ) {
-        const uint32_t row = 32 * sub + r;
-        const bf16x8 a = __builtin_bit_cast( bf16x8, s_k[row * 16 + ( ( 2 * k + g2 ) ^ ( SHARED ? shared_swizzle( row ) : row & 15 ) )] );
-        st[sub] = Mfma<__bf16>::k16( a, qb[k], st[sub] );
+        st[sub][v] = sx[sub][v];
       }
     }
-    // what a score is multiplied with: one number, or that of its key
-    float factor[2][16];
+    // ---- scale, bias by distance, mask (log2 domain): a score is st * sc + b
+    const uint32_t key_l = t0 + 4 * g2; // key of register v: key_l + offset_of( sub, v )
+    const int32_t dist_l = (int32_t)( pos - key_l );
+    float sc = 1.0f, b = 0.0f;
+    if constexpr ( SHARED ) { // a factor for each key
 #pragma unroll
-    for ( int sub = 0; sub < 2; sub++ ) {
+      for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
-      for ( int q4 = 0; q4 < 4; q4++ ) {
-        float4 f = make_float4( scale_log2e, scale_log2e, scale_log2e, scale_log2e );
-        if constexpr ( SHARED ) {
-          f = *reinterpret_cast<const float4*>( s_factor + 32 * sub + 8 * q4 + 4 * g2 );
+        for ( int q4 = 0; q4 < 4; q4++ ) {
+          const float4 f = *reinterpret_cast<const float4*>( s_factor + 32 * sub + 8 * q4 + 4 * g2 );
+          st[sub][4 * q4] *= f.x, st[sub][4 * q4 + 1] *= f.y, st[sub][4 * q4 + 2] *= f.z, st[sub][4 * q4 + 3] *= f.w;
         }
-        factor[sub][4 * q4] = f.x, factor[sub][4 * q4 + 1] = f.y, factor[sub][4 * q4 + 2] = f.z, factor[sub][4 * q4 + 3] = f.w;
       }
     }
-    // ---- scale, bias by distance, mask (log2 domain)
-    const uint32_t key_l = t0 + 4 * g2; // key of register v: key_l + 32 sub + 8 (v / 4) + v % 4
-    const uint32_t last_key = t0 + TILE_KEYS - 1;
-    if ( bias_floats == 0 || ( last_key <= pos_first && pos_first - last_key >= s.n_dist - 1 ) ) { // every distance in the table's last row
-      const float b = bias_floats == 0 ? 0.0f : my_bias[s.n_dist - 1];
+    if ( far && ( SHARED || scale_log2e > 0.0f ) ) { // the largest score is that of the largest product, and one instruction scales it and takes its reference point off
+      sc = SHARED ? 1.0f : scale_log2e;
+      b = my_bias[n_dist - 1];
+    } else if ( !far && bias_pad > 0 ) { // from the distance of the last key up, one address for all
+      const float* row = my_bias + dist_l - ( (int)TILE_KEYS - 5 );
 #pragma unroll
       for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
         for ( int v = 0; v < 16; v++ ) {
-          st[sub][v] = st[sub][v] * factor[sub][v] + b;
+          st[sub][v] = __builtin_fmaf( st[sub][v], SHARED ? 1.0f : scale_log2e, row[(int)TILE_KEYS - 5 - offset_of( sub, v )] );
         }
       }
     } else {
@@ -754,23 +808,25 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
       for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
         for ( int v = 0; v < 16; v++ ) {
-          const uint32_t key = key_l + 32 * sub + 8 * ( v / 4 ) + v % 4;
-          st[sub][v] = st[sub][v] * factor[sub][v] + my_bias[min( pos - min( key, pos ), s.n_dist - 1 )];
+          st[sub][v] = __builtin_fmaf( st[sub][v], SHARED ? 1.0f : scale_log2e, my_bias[min( pos - min( key_l + offset_of( sub, v ), pos ), n_dist - 1 )] );
         }
       }
     }
-    const bool in_window = i >= kept_tiles;
-    const bool whole = in_window ? last_key <= pos_first && ( pos_last - t0 < s.window || last_key < s.keep_first ) : last_key < kept;
-    if ( !whole ) {
-      const uint32_t end = in_window ? 0xffffffffu : kept;
+    if ( edge ) { // the hidden keys of a column are those before or behind one offset, which a register's is compared with
+      auto hide = [&]( auto hidden ) __attribute__( ( always_inline ) ) {
 #pragma unroll
-      for ( int sub = 0; sub < 2; sub++ ) {
+        for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
-        for ( int v = 0; v < 16; v++ ) {
-          const uint32_t key = key_l + 32 * sub + 8 * ( v / 4 ) + v % 4;
-          const bool seen = key <= pos && key < end && ( pos - key < s.window || key < s.keep_first );
-          st[sub][v] = seen ? st[sub][v] : -INFINITY;
+          for ( int v = 0; v < 16; v++ ) {
+            st[sub][v] = hidden( (int32_t)offset_of( sub, v ) ) ? -INFINITY : st[sub][v];
+          }
         }
+      };
+      const int32_t end = in_window ? dist_l + 1 : (int32_t)( kept - key_l );
+      hide( [&]( int32_t o ) __attribute__( ( always_inline ) ) { return o >= end; } );
+      if ( in_window && past_window ) {
+        const int32_t outside = dist_l - (int32_t)s.window, keep = (int32_t)( s.keep_first - min( s.keep_first, key_l ) );
+        hide( [&]( int32_t o ) __attribute__( ( always_inline ) ) { return ( o <= outside ) & ( o >= keep ); } );
       }
     }
     // ---- online softmax
@@ -783,7 +839,7 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         mx4[c] = fmaxf( mx4[c], st[c >> 1][8 * ( c & 1 ) + e] );
       }
     }
-    const float mx = half_wave_max( fmaxf( fmaxf( mx4[0], mx4[1] ), fmaxf( mx4[2], mx4[3] ) ) );
+    const float mx = __builtin_fmaf( half_wave_max( fmaxf( fmaxf( mx4[0], mx4[1] ), fmaxf( mx4[2], mx4[3] ) ) ), sc, b );
     if ( __builtin_amdgcn_ballot_w64( mx > m + LAZY ) != 0 ) {
       const float m_new = fmaxf( m, mx );
       const float alpha = __builtin_amdgcn_exp2f( m - m_new );
@@ -797,29 +853,46 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         }
       }
     }
+    const float ref = b - m;
 #pragma unroll
     for ( int kk = 0; kk < 4; kk++ ) { // 16 keys
-      bf16x8 hi, lo;
+      union
+      {
+        uint32_t pair[4];
+        bf16x8 x;
+      } hi, lo;
 #pragma unroll
-      for ( int e = 0; e < 8; e++ ) {
-        const float p = __builtin_amdgcn_exp2f( st[kk >> 1][8 * ( kk & 1 ) + e] - m );
-        l += p;
-        hi[e] = (__bf16)p;
-        lo[e] = (__bf16)( p - (float)hi[e] );
+      for ( int e = 0; e < 4; e++ ) {
+        const float p0 = __builtin_amdgcn_exp2f( __builtin_fmaf( st[kk >> 1][8 * ( kk & 1 ) + 2 * e], sc, ref ) );
+        const float p1 = __builtin_amdgcn_exp2f( __builtin_fmaf( st[kk >> 1][8 * ( kk & 1 ) + 2 * e + 1], sc, ref ) );
+        l += p0;
+        l += p1;
+        hi.pair[e] = bf16_pair( p0, p1 );
+        asm( "" : "+v"( hi.pair[e] ) ); // (taken apart again below: the compiler would convert the two once more instead)
+        lo.pair[e] = bf16_pair( p0 - __builtin_bit_cast( float, hi.pair[e] << 16 ), p1 - __builtin_bit_cast( float, hi.pair[e] & 0xffff0000u ) );
       }
 #pragma unroll
-      for ( int vb = 0; vb < VB; vb++ ) {
+      for ( int vp = 0; vp < VB; vp += 2 ) { // (two blocks in turn: a product that waits for the one before it leaves the matrix unit idle)
         union
         {
           v4s half[2];
           bf16x8 x;
-        } a;
+        } a[2];
 #pragma unroll
-        for ( int hf = 0; hf < 2; hf++ ) {
-          a.half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)s_v + ( v_lane ^ ( 64 * vb ) ^ ( SHARED ? 32 * hf : 0 ) ) + ( 16 * kk + 8 * hf ) * 256 ) );
+        for ( int c = 0; c < min( 2, VB - vp ); c++ ) {
+#pragma unroll
+          for ( int hf = 0; hf < 2; hf++ ) {
+            a[c].half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)s_v + ( v_lane ^ ( 64 * ( vp + c ) ) ^ ( SHARED ? 32 * hf : 0 ) ) + ( 16 * kk + 8 * hf ) * 256 ) );
+          }
         }
-        acc[vb] = Mfma<__bf16>::k16( a.x, lo, acc[vb] );
-        acc[vb] = Mfma<__bf16>::k16( a.x, hi, acc[vb] );
+#pragma unroll
+        for ( int c = 0; c < min( 2, VB - vp ); c++ ) {
+          acc[vp + c] = Mfma<__bf16>::k16( a[c].x, lo.x, acc[vp + c] );
+        }
+#pragma unroll
+        for ( int c = 0; c < min( 2, VB - vp ); c++ ) {
+          acc[vp + c] = Mfma<__bf16>::k16( a[c].x, hi.x, acc[vp + c] );
+        }
       }
     }
   }
@@ -1535,10 +1608,11 @@ int attend_tiles( const WindowOut<__bf16>& out, const __bf16* q, const float* bi
   const uint64_t n_pairs = batch * s.kv_heads * ( s.group / head_cols );
   const uint64_t grid = ( n_pairs + 7 ) / 8 * 8 * col_blocks;
   GH_REQUIRE( grid < ( 1ull << 31 ), "gh_attn_window: grid too large" );
-  const uint32_t bias_floats = bias == nullptr ? 0 : head_cols * s.n_dist;
-  const size_t lds = ( s.values_are_keys ? TILE_KEYS * ( 256 + sizeof( float ) ) : 2 * TILE_KEYS * 256 ) + bias_floats * sizeof( float );
+  const uint32_t bias_pad = bias != nullptr && (uint64_t)head_cols * ( s.n_dist + 2 * BIAS_PAD ) <= BIAS_LDS ? BIAS_PAD : 0;
+  const uint32_t bias_row = bias == nullptr ? 0 : s.n_dist + 2 * bias_pad, bias_floats = head_cols * bias_row;
+  const size_t lds = ( s.values_are_keys ? TILE_KEYS * ( 256 + sizeof( float ) ) : 2 * TILE_KEYS * 256 ) + std::max( bias_floats, 1u ) * sizeof( float );
 #define GH_WINDOW_TILES( KS, VB, SHARED ) \
-  window_tiles_kernel<KS, VB, SHARED><<<(unsigned)grid, 256, lds, st>>>( out, q, bias, wr, s, head_cols, col_blocks, (uint32_t)n_pairs, bias_floats )
+  window_tiles_kernel<KS, VB, SHARED><<<(unsigned)grid, 256, lds, st>>>( out, q, bias, wr, s, head_cols, col_blocks, (uint32_t)n_pairs, bias_row, bias_pad )
   if ( s.values_are_keys ) {
     if ( s.dpad <= 64 ) {
       GH_WINDOW_TILES( 4, 2, true );

@@ -248,6 +248,45 @@ def test_decode_of_heads_with_keys_of_their_own(heads, dim, vdim, rows, keys, sh
         assert ((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 2e-5).all(), i
 
 
+# of a wave's 32 columns and 64 keys at a time: (heads, kv heads, head sizes), (window, kept tokens, distances, scale), (starts, tokens).  Tables of one
+# distance, of fewer than a tile, with room for the entries around it and without, and none; windows that end inside a wave, kept tokens that reach into
+# it; first positions on both sides of a tile's edge, portions past the last full wave; keys that are values too, of a size with an odd number of blocks
+@pytest.mark.parametrize("heads,kv,dim,vdim,shared", [(4, 4, 128, 128, False), (8, 2, 72, 40, False), (6, 2, 128, 64, False), (2, 2, 96, 96, True), (4, 4, 128, 128, True)])
+@pytest.mark.parametrize("window,keep,n_dist,scale", [(0, 0, 0, 1.0), (0, 0, 0, -1.0), (97, 5, 1, 1.0), (64, 70, 17, 1.0), (150, 200, 90, -1.0), (300, 3, 2000, 1.0), (31, 64, 7900, 1.0)])
+@pytest.mark.parametrize("starts,T", [([0, 64], 16), ([1, 257], 131), ([95, 0], 290)])
+def test_tiles_of_keys_by_waves(heads, kv, dim, vdim, shared, window, keep, n_dist, scale, starts, T):
+    """Against 64 bits: a rounding to bf16 and weights in two terms of bf16, whose error is below 2^-17 of the largest value."""
+    import torch
+    from glinthawk_amd import ops
+    a = ops.window_attn(heads, kv, dim, vdim, scale * dim ** -0.5, window, keep, n_dist, shared)
+    g = torch.Generator(device="cuda").manual_seed(T + n_dist)
+    keys = max(starts) + T
+    cache = torch.randn((2, keys, kv * (dim if shared else dim + vdim)), generator=g, device="cuda").bfloat16()
+    groups = -(-keys // 32)
+    factors = torch.rand((2, groups, kv, 32), generator=g, device="cuda") + 0.5
+    memory = torch.cat([cache.view(2, -1).view(torch.uint8), factors.view(2, -1).view(torch.uint8)], 1).contiguous()
+    q = torch.randn((2, T, heads, dim), generator=g, device="cuda").bfloat16()
+    bias = 2.0 * torch.randn((heads, n_dist), generator=g, device="cuda") if n_dist else None
+    got = ops.attn_window(q.view(2 * T, -1), a, ops.row_table([m.data_ptr() for m in memory]), torch.tensor(starts, dtype=torch.int32, device="cuda"), T, max(starts), bias, 0,
+                          cache[0].numel() * 2).double().view(2, T, heads, vdim)
+    for i, start in enumerate(starts):
+        n = start + T
+        k = cache[i, :n, :kv * dim].view(n, kv, dim).double().repeat_interleave(heads // kv, 1)
+        v = k if shared else cache[i, :n, kv * dim:].view(n, kv, vdim).double().repeat_interleave(heads // kv, 1)
+        distance = torch.arange(start, n, device="cuda")[:, None] - torch.arange(n, device="cuda")
+        score = (k.permute(1, 0, 2)[:, None] * q[i].permute(1, 0, 2)[:, :, None].double()).sum(-1) * (scale * dim ** -0.5)     # (heads, tokens, keys)
+        if shared:
+            score = score * factors[i].permute(0, 2, 1).reshape(-1, kv)[:n].double().T.repeat_interleave(heads // kv, 0)[:, None]
+        if n_dist:
+            score = score + bias.double()[:, distance.clamp(0, n_dist - 1)]
+        hidden = distance < 0
+        if window:
+            hidden = hidden | ((distance >= window) & (torch.arange(n, device="cuda") >= keep))
+        weight = score.masked_fill(hidden, -float("inf")).softmax(-1)
+        want = torch.stack([weight[h] @ v[:, h] for h in range(heads)], 1)
+        assert ((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -17 * v.abs().max() + 2e-5).all(), start
+
+
 class Cache:
     """One attention layer's cache rows of a few contexts, filled by hand (heads padded to 8 elements with zeros)."""
 
