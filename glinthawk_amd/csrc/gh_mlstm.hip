@@ -265,20 +265,32 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
 //   S_t = e^(m0 - M_t) S_0 + sum_(s <= t) e^(c_s - M_t) k_s v_s^T                      (n_t likewise)
 //   o_t = (e^(m0 - M_t) S_0^T q_t + sum_(s <= t) e^(c_s - M_t) (k_s . q_t) v_s) / (max(|n_t . q_t|, e^(-m_t)) + 1e-6)
 //
-// work-group  2 waves on one (context, head, 64 columns of v) walk the chunks; a wave owns 32 columns, its part of S (dim x 32, fp32) stays in
-//             accumulator registers from the first chunk to the last.  Two work-groups per CU cover each other's loads.
+// Three kernels:
+//   scan    the gates, b, c and M of every token, a work-group for a (context, head), a wave for a chunk
+//   scores  a work-group for a chunk: the weights of the keys P[t][s] = e^(c_s - M_t) (k_s . q_t), their sums over s, and what the chunk
+//           adds to n.  They do not depend on v: made here once instead of by all the columns of v.
+//   states  4 waves on one (context, head, 64 columns of v) walk the chunks, O = a Q S + P V, then S = decay S + K^T (w V); a wave owns
+//           16 columns, its part of S (dim x 16, fp32) stays in accumulator registers from the first chunk to the last.  Two work-groups
+//           per CU: two waves a SIMD cover each other's reads of LDS and waits.
+//           n is carried by every slice of the columns, a thread an element; each makes the denominators of its share of the tokens.
 // exactness   q, k, v are bf16 already.  What enters the state (the weighted values) meets k as three bf16 terms, 24 bits: the state's sums are
 //             those of fp32 operands at the rate of bf16 matrix instructions.  What is read out of it for the output (S, the weights of
-//             the keys) meets q and v as two terms, 16 bits.  n is carried in fp32, each wave half of it.
-// loads       k of a chunk is requested at its head, once both waves are through with the last one's, q and v of the next one as soon as
-//             both waves have read this one's.
-// operands    an accumulator tile of v_mfma_f32_32x32x16_bf16 (lane = column, registers = rows 8 (v / 4) + 4 (lane / 32) + v % 4) is, as it
-//             lies, an operand of the next product over those rows when the other operand takes its sixteen k in the same order:
+//             the keys) meets q and v as two terms, 16 bits.  n and its products are fp32.
+// loads       k of a chunk is requested at its head and needed behind Q S and P V; q and v of the next one are requested behind those and needed
+//             at the next one's head.
+// operands    an accumulator tile of v_mfma_f32_16x16x32_bf16 (lane = column, registers = rows 4 (lane / 16) + v) is, with the tile below it
+//             and as they lie, an operand of the next product over those 32 rows when the other operand takes its rows in the same order:
 //               scores^T = K Q^T        lane = query, registers = keys   -> left operand of   P V     (V out of LDS transposed)
 //               S                       lane = column of v, registers = dim -> right operand of Q S   (Q out of LDS in pieces of 4)
 //             S += K^T (w V): both operands out of LDS with transposing reads (ds_read_b64_tr_b16).
-// LDS         64 rows each of q, k (16-byte chunks XORed with bits of the row, so that row reads and transposing reads both spread over
-//             the banks) and of v, straight from memory (buffer_load ... lds; rows past the sequence and padding read as zero).
+// LDS         64 rows each of q, k and v, 16-byte chunks XORed with bits of the row so that row reads (16 rows) and transposing reads (8 rows of a
+//             half-wave, two chunks each) both touch every bank once; straight from memory (buffer_load ... lds; rows past the sequence
+//             and padding read as zero).
+// bound       8 contexts of 1024 tokens, 8 heads of 256 x 512: 310 us in one kernel, whose waves, one a SIMD, made gates, weights and n once for every 32
+//             columns; now scan 9, scores 16 and states 118 us (the call 398 -> 257; 1 of 2048 tokens 526 -> 177, 32 of 24 tokens 118 -> 78).  States: the
+//             matrix cores are busy for a third of it, as are the vector units; what is left is waits of four waves for each other, twice a
+//             chunk.  On the way there: requests at the chunk's head instead of where the scheduler put them and stores that the next chunk
+//             doesn't wait for 134 -> 122; Q in reads that are not joined by two 127 (LDS 2.4 x as long active joined).
 constexpr int CHUNK = 64;
 typedef __attribute__( ( address_space( 3 ) ) ) void* lds_ptr;
 typedef __attribute__( ( address_space( 3 ) ) ) char lds_char;
@@ -286,13 +298,12 @@ typedef short v4s __attribute__( ( ext_vector_type( 4 ) ) );
 typedef __attribute__( ( address_space( 3 ) ) ) v4s* lds_v4s;
 typedef Mfma<__bf16>::x8 bf16x8;
 
-// slot of 16-byte chunk `chunk` of row `row` in a tile of DT * 4 chunks a row
-template<int DT>
+// slot of 16-byte chunk `chunk` of row `row` in a tile of `BYTES` a row: 128, 256 or 512
+template<uint32_t BYTES>
 __device__ __forceinline__ uint32_t swizzle( uint32_t row, uint32_t chunk )
 {
-  return DT == 2 ? chunk ^ ( ( ( ( row >> 1 ) & 1 ) << 2 ) | ( ( row >> 2 ) & 3 ) ) : chunk ^ ( ( ( row & 3 ) << 2 ) | ( ( row >> 2 ) & 3 ) );
+  return BYTES == 128 ? chunk ^ ( ( ( ( row >> 1 ) & 3 ) << 1 ) | ( ( row >> 3 ) & 1 ) ) : chunk ^ ( ( ( row & 7 ) << 1 ) | ( ( row >> 3 ) & 1 ) );
 }
-__device__ __forceinline__ uint32_t swizzle_v( uint32_t row, uint32_t chunk ) { return chunk ^ ( 4 * ( ( row >> 1 ) & 1 ) ); }
 
 // Eight fp32 values as N bf16 terms each, 8 bits of mantissa a term; taken two at a time, as the conversion instruction does.
 typedef float f32x2 __attribute__( ( ext_vector_type( 2 ) ) );
@@ -316,24 +327,6 @@ struct Split
     }
   }
 };
-template<int N>
-__device__ __forceinline__ mfma_f32x16 mma( const bf16x8 a, const Split<N>& b, mfma_f32x16 c )
-{
-#pragma unroll
-  for ( int n = N - 1; n >= 0; n-- ) {
-    c = Mfma<__bf16>::k16( a, b.t[n].x, c );
-  }
-  return c;
-}
-template<int N>
-__device__ __forceinline__ mfma_f32x16 mma( const Split<N>& a, const bf16x8 b, mfma_f32x16 c )
-{
-#pragma unroll
-  for ( int n = N - 1; n >= 0; n-- ) {
-    c = Mfma<__bf16>::k16( a.t[n].x, b, c );
-  }
-  return c;
-}
 __device__ __forceinline__ double shfl_up_f64( double v, int by )
 {
   const uint64_t bits = __builtin_bit_cast( uint64_t, v );
@@ -347,20 +340,254 @@ __device__ __forceinline__ double last_lane_f64( double v )
   return __builtin_bit_cast( double, ( (uint64_t)hi << 32 ) | lo );
 }
 
-// DT: 32-row tiles of S, dim <= 32 DT.  dim % 8 == 0, vdim % 8 == 0, 16-byte aligned product rows.
-template<int DT>
-__global__ __launch_bounds__( 128, 1 ) void mlstm_chunk_kernel( float* __restrict__ o_out, float* __restrict__ nm_out, MlstmIn<__bf16, ProductView<__bf16>> in, MlstmState st,
-                                                                MlstmShape s, uint32_t slices, uint32_t n_pairs )
+// What the three kernels and the finishing one hand on, by (context, head) = pair.
+struct MlstmChunks
 {
-  constexpr uint32_t RB = DT * 64; // bytes of a q or k row in LDS
+  float* token;   // planes of (pairs, chunks x 64): see below
+  float* decay;   // (pairs, chunks): factor of the state over a chunk
+  float* n;       // (pairs, chunks, dim): what a chunk adds to n
+  uint4* weights; // (pairs, chunks, WEIGHT_TILES, 2 terms, 64 lanes): P as the left operands of P V
+  uint32_t chunks;
+  uint64_t plane;
+  enum
+  {
+    C,     // c_s - M of the chunk's last token; -inf past the sequence
+    W,     // e to the power of it
+    A,     // factor of the state in front of the chunk
+    M,     // M_t - M of the chunk's last token
+    FLOOR, // e^(-m_t)
+    DEN,   // sum of the weights of the keys
+    OVER,  // 1 / denominator
+    PLANES
+  };
+  __device__ __forceinline__ float* tokens( int which, uint32_t pair, uint32_t chunk ) const { return token + which * plane + ( (uint64_t)pair * chunks + chunk ) * CHUNK; }
+};
+constexpr uint32_t WEIGHT_TILES = 6; // 16 queries x 32 keys; of queries 0 .. 31 the first 32 keys only
+__device__ __forceinline__ constexpr uint32_t weight_tile( uint32_t queries, uint32_t keys ) { return queries < 2 ? queries : 2 * queries - 2 + keys; }
+
+// The tokens of a chunk, lane <-> token: the sums b of the log forget gates, c, and the largest c so far (without what lies in front of the chunk).
+struct ChunkScan
+{
+  double b, c, M;
+  bool live;
+  __device__ __forceinline__ ChunkScan( const MlstmGates<__bf16>& in, const MlstmState& st, uint32_t ctx, uint32_t h, uint32_t tok, uint32_t lane )
+  {
+    live = tok < st.n_tokens;
+    const uint64_t row = (uint64_t)ctx * st.n_tokens + ( live ? tok : 0 );
+    const float gi = in.log_input( in.y.at( row, in.col.i + h ), h ), gf = in.log_forget( in.y.at( row, in.col.f + h ), h );
+    b = live ? (double)gf : 0.0;
+#pragma unroll
+    for ( int by = 1; by < 64; by *= 2 ) {
+      const double up = shfl_up_f64( b, by );
+      b += (int)lane >= by ? up : 0.0;
+    }
+    c = live ? (double)gi - b : -1e300;
+    M = c;
+#pragma unroll
+    for ( int by = 1; by < 64; by *= 2 ) {
+      const double up = shfl_up_f64( M, by );
+      M = (int)lane >= by && up > M ? up : M;
+    }
+  }
+  // what the other kernels take, with the running maximum in front of the chunk
+  __device__ __forceinline__ void finish( const MlstmChunks& out, uint32_t pair, uint32_t chunk, uint32_t lane, double before, float& c_rel, float& w, float& M_rel )
+  {
+    M = before > M ? before : M;
+    const double M_end = last_lane_f64( M );
+    c_rel = live ? (float)( c - M_end ) : -INFINITY;
+    w = expf( c_rel );
+    M_rel = (float)( M - M_end );
+    out.tokens( MlstmChunks::C, pair, chunk )[lane] = c_rel;
+    out.tokens( MlstmChunks::W, pair, chunk )[lane] = w;
+    out.tokens( MlstmChunks::A, pair, chunk )[lane] = expf( (float)( before - M ) );
+    out.tokens( MlstmChunks::M, pair, chunk )[lane] = M_rel;
+    out.tokens( MlstmChunks::FLOOR, pair, chunk )[lane] = expf( -(float)( b + M ) );
+    if ( lane == 0 ) {
+      out.decay[(uint64_t)pair * out.chunks + chunk] = expf( (float)( before - M_end ) );
+    }
+  }
+};
+__device__ __forceinline__ double max_in_front( const uint8_t* base, const MlstmState& st, const MlstmShape& s, uint32_t ctx, uint32_t h )
+{
+  return st.start_pos[ctx] == 0 ? 0.0 : (double)reinterpret_cast<const float*>( base + st.offset )[s.m_off() + h];
+}
+
+// work-group <-> (head, context), wave <-> chunk, lane <-> token
+__global__ __launch_bounds__( 1024 ) void mlstm_scan_kernel( float* __restrict__ nm_out, MlstmGates<__bf16> in, MlstmState st, MlstmShape s, MlstmChunks out )
+{
+  __shared__ double s_b[16], s_M[16]; // of a chunk: sum of its log forget gates, largest c without what lies in front of it
+  const uint32_t h = blockIdx.x, ctx = blockIdx.y, pair = ctx * s.heads + h;
+  const uint8_t* base = static_cast<const uint8_t*>( st.rows[ctx] );
+  if ( base == nullptr ) {
+    return;
+  }
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double m0 = max_in_front( base, st, s, ctx, h );
+  for ( uint32_t c0 = 0; c0 < out.chunks; c0 += 16 ) {
+    const uint32_t chunk = c0 + wave;
+    ChunkScan scan( in, st, ctx, h, chunk * CHUNK + lane, lane );
+    __syncthreads(); // everyone has read the last sixteen chunks'
+    if ( lane == 63 ) {
+      s_b[wave] = scan.b;
+      s_M[wave] = scan.M;
+    }
+    __syncthreads();
+    double before = m0; // running maximum in front of this wave's chunk
+#pragma unroll
+    for ( uint32_t k = 0; k < 16; k++ ) { // (chunks past the last: nothing to add, nothing as large)
+      before = k == wave ? m0 : before;
+      m0 = s_b[k] + ( s_M[k] > m0 ? s_M[k] : m0 );
+    }
+    if ( chunk < out.chunks ) {
+      float c_rel, w, M_rel;
+      scan.finish( out, pair, chunk, lane, before, c_rel, w, M_rel );
+    }
+  }
+  if ( threadIdx.x == 0 ) {
+    nm_out[(uint64_t)pair * ( s.dim + 1 ) + s.dim] = (float)m0;
+  }
+}
+
+// work-group <-> chunk of a (context, head), wave <-> 16 queries.  KS: steps of 32 of dim.  dim % 8 == 0, 16-byte aligned product rows.
+// ALONE: the call has one chunk, whose gates the work-group scans itself beside its loads, without a launch in front (2 contexts of 24 tokens, 4 heads of 64:
+// 27.2 -> 22.5 us for the call; 16 of 64 tokens, 4 heads of 128 x 256: 36.9 -> 31.5).
+template<int KS, bool ALONE>
+__global__ __launch_bounds__( 256 ) void mlstm_scores_kernel( float* __restrict__ nm_out, MlstmIn<__bf16, ProductView<__bf16>> in, MlstmGates<__bf16> raw, MlstmState st, MlstmShape s,
+                                                              MlstmChunks ch, uint32_t n_pairs )
+{
+  constexpr uint32_t PIECES = 4 * KS, SETS = 256 / PIECES; // 8 dims each; threads on the same dims
+  constexpr uint32_t RB = KS * 64;                         // bytes of a row in LDS
+  __shared__ uint4 s_k[CHUNK * RB / 16]; // then the sums for n of the sets
+  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_c[CHUNK], s_w[CHUNK], s_M[CHUNK];
+  // on the XCD that walks the chunks
+  const uint32_t pair = ( blockIdx.x >> 3 ) / ch.chunks * 8 + ( blockIdx.x & 7 ), chunk = ( blockIdx.x >> 3 ) % ch.chunks;
+  if ( pair >= n_pairs ) {
+    return;
+  }
+  const uint32_t h = pair % s.heads, ctx = pair / s.heads;
+  const uint8_t* base = static_cast<const uint8_t*>( st.rows[ctx] );
+  if ( base == nullptr ) {
+    return;
+  }
+  const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 ), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const uint32_t rows = min( (uint32_t)CHUNK, st.n_tokens - chunk * CHUNK );
+  const uint32_t ld_bytes = (uint32_t)( in.main.stride * 2 );
+  const __bf16* first = in.main.data + ( (uint64_t)ctx * st.n_tokens + chunk * CHUNK ) * in.main.stride;
+  const int bytes = (int)( ( rows - 1 ) * ld_bytes + s.dim * 2 ); // rows past the sequence read as zero
+  const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<__bf16*>( first + in.col.q + h * s.dim ), 0, bytes, 0x00020000 );
+  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<__bf16*>( first + in.col.k + h * s.dim ), 0, bytes, 0x00020000 );
+  constexpr uint32_t PAST_THE_END = 0x80000000u; // an offset beyond any descriptor
+  typedef uint32_t u32x4_t __attribute__( ( ext_vector_type( 4 ) ) );
+  bf16x8 qb[KS];
+#pragma unroll
+  for ( int k = 0; k < KS; k++ ) {
+    qb[k] = __builtin_bit_cast( bf16x8, (u32x4_t)__builtin_amdgcn_raw_buffer_load_b128( q_rsrc, ( 4 * k + g ) * 8 < s.dim ? ( 16 * wave + r ) * ld_bytes + ( 4 * k + g ) * 16 : PAST_THE_END, 0, 0 ) );
+  }
+  constexpr uint32_t ROWS = 1024 / RB; // rows of one instruction of one wave
+#pragma unroll
+  for ( uint32_t i = 0; i < CHUNK / ( 4 * ROWS ); i++ ) {
+    const uint32_t row0 = ( 4 * i + wave ) * ROWS, row = row0 + lane / PIECES, piece = swizzle<RB>( row, lane % PIECES );
+    __builtin_amdgcn_raw_ptr_buffer_load_lds( k_rsrc, (lds_ptr)( s_k + row0 * PIECES ), 16, piece * 8 < s.dim ? row * ld_bytes + piece * 16 : PAST_THE_END, 0, 0, 0 );
+  }
+  auto k_at = [&]( uint32_t row, uint32_t piece ) __attribute__( ( always_inline ) ) { return __builtin_bit_cast( bf16x8, s_k[row * PIECES + swizzle<RB>( row, piece )] ); };
+  if ( wave == 0 ) {
+    float c_rel, w, M_rel;
+    if constexpr ( ALONE ) {
+      ChunkScan scan( raw, st, ctx, h, lane, lane );
+      scan.finish( ch, pair, 0, lane, max_in_front( base, st, s, ctx, h ), c_rel, w, M_rel );
+      if ( lane == 63 ) {
+        nm_out[(uint64_t)pair * ( s.dim + 1 ) + s.dim] = (float)( scan.b + scan.M );
+      }
+    } else {
+      c_rel = ch.tokens( MlstmChunks::C, pair, chunk )[lane], w = ch.tokens( MlstmChunks::W, pair, chunk )[lane], M_rel = ch.tokens( MlstmChunks::M, pair, chunk )[lane];
+    }
+    s_c[lane] = c_rel, s_w[lane] = w, s_M[lane] = M_rel;
+  }
+  __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): this wave's part of k has landed
+  __syncthreads();
+  const float Mq = s_M[16 * wave + r];
+  float p[4][4], den = 0.0f;
+#pragma unroll
+  for ( uint32_t kt = 0; kt < 4; kt++ ) {
+#pragma unroll
+    for ( int e = 0; e < 4; e++ ) {
+      p[kt][e] = 0.0f;
+    }
+    if ( kt <= wave ) {
+      mfma_f32x4 sc = { 0, 0, 0, 0 };
+#pragma unroll
+      for ( int k = 0; k < KS; k++ ) {
+        sc = Mfma<__bf16>::k32( k_at( 16 * kt + r, 4 * k + g ), qb[k], sc );
+      }
+      const float4 ck = *reinterpret_cast<const float4*>( &s_c[16 * kt + 4 * g] );
+      const float cks[4] = { ck.x, ck.y, ck.z, ck.w };
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        const bool seen = kt < wave || 4 * g + e <= r;
+        p[kt][e] = seen ? sc[e] * s.q_scale * __expf( cks[e] - Mq ) : 0.0f;
+        den += p[kt][e];
+      }
+    }
+  }
+  den += __shfl_xor( den, 16 );
+  den += __shfl_xor( den, 32 );
+  if ( g == 0 ) {
+    ch.tokens( MlstmChunks::DEN, pair, chunk )[16 * wave + r] = den;
+  }
+  uint4* dst = ch.weights + ( (uint64_t)pair * ch.chunks + chunk ) * ( WEIGHT_TILES * 128 ) + lane;
+#pragma unroll
+  for ( uint32_t j = 0; j < 2; j++ ) {
+    if ( 2 * j <= wave ) {
+      Split<2> f;
+#pragma unroll
+      for ( int k = 0; k < 4; k++ ) {
+        f.set( k, p[2 * j + ( k >> 1 )][2 * ( k & 1 )], p[2 * j + ( k >> 1 )][2 * ( k & 1 ) + 1] );
+      }
+#pragma unroll
+      for ( int n = 0; n < 2; n++ ) {
+        dst[( weight_tile( wave, j ) * 2 + n ) * 64] = __builtin_bit_cast( uint4, f.t[n].x );
+      }
+    }
+  }
+  // what the chunk adds to n
+  const uint32_t piece = threadIdx.x % PIECES, set = threadIdx.x / PIECES;
+  float sum[8] = {};
+#pragma unroll
+  for ( uint32_t i = 0; i < CHUNK / SETS; i++ ) {
+    const float w = s_w[set + SETS * i];
+    const bf16x8 k = k_at( set + SETS * i, piece );
+#pragma unroll
+    for ( int e = 0; e < 8; e++ ) {
+      sum[e] += (float)k[e] * w;
+    }
+  }
+  float* s_n = reinterpret_cast<float*>( s_k );
+  __syncthreads(); // everyone has read k
+#pragma unroll
+  for ( int e = 0; e < 8; e += 4 ) {
+    *reinterpret_cast<float4*>( s_n + set * ( 8 * PIECES ) + piece * 8 + e ) = make_float4( sum[e], sum[e + 1], sum[e + 2], sum[e + 3] );
+  }
+  __syncthreads();
+  if ( threadIdx.x < s.dim ) {
+    float n = 0.0f;
+#pragma unroll
+    for ( uint32_t k = 0; k < SETS; k++ ) {
+      n += s_n[k * ( 8 * PIECES ) + threadIdx.x];
+    }
+    ch.n[( (uint64_t)pair * ch.chunks + chunk ) * s.dim + threadIdx.x] = n;
+  }
+}
+
+// KS: steps of 32 of dim, dim <= 32 KS.  dim % 8 == 0, vdim % 8 == 0, 16-byte aligned product rows.
+template<int KS>
+__global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restrict__ o_out, float* __restrict__ nm_out, MlstmIn<__bf16, ProductView<__bf16>> in, MlstmState st,
+                                                                 MlstmShape s, MlstmChunks ch, uint32_t slices, uint32_t n_pairs )
+{
+  constexpr uint32_t RB = KS * 64; // bytes of a q or k row in LDS
   __shared__ uint4 s_k[CHUNK * RB / 16], s_q[CHUNK * RB / 16];
   __shared__ uint4 s_v[CHUNK * 8];
-  __shared__ float s_n[32 * DT];                                      // a wave reads and writes its half only
-  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_nq[2][CHUNK]; // n . q over each wave's half; everything below: each wave its own copy
-  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_c[2][CHUNK]; // c_s - M of the chunk's last token, s_w: e to the power of it
-  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_w[2][CHUNK];
-  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_a[2][CHUNK];   // factor of the state in front of the chunk, per token
-  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_inv[2][CHUNK]; // one over the denominator
+  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_n[256]; // n in front of the chunk
+  __shared__ __attribute__( ( aligned( 16 ) ) ) float s_a[CHUNK], s_w[2][CHUNK]; // (w is read behind the second barrier of a chunk, when another wave may write the next one's)
 
   // the slices of a (context, head) read the same q and k: all on one XCD, next to each other in time
   const uint32_t pair = ( blockIdx.x >> 3 ) / slices * 8 + ( blockIdx.x & 7 ), slice = ( blockIdx.x >> 3 ) % slices;
@@ -373,85 +600,56 @@ __global__ __launch_bounds__( 128, 1 ) void mlstm_chunk_kernel( float* __restric
     return;
   }
   float* S_mem = reinterpret_cast<float*>( base + st.offset );
-  const float* n_in = S_mem + s.n_off() + (uint64_t)h * s.dim;
-  const float m_mem = S_mem[s.m_off() + h];
-  S_mem += (uint64_t)h * s.dim * s.vpad;
   const bool fresh = st.start_pos[ctx] == 0;
+  float n = !fresh && threadIdx.x < s.dim ? S_mem[s.n_off() + (uint64_t)h * s.dim + threadIdx.x] : 0.0f; // thread <-> element
+  const float* n_chunk = ch.n + (uint64_t)pair * ch.chunks * s.dim + min( threadIdx.x, s.dim - 1 );
+  S_mem += (uint64_t)h * s.dim * s.vpad;
   const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
-  const uint32_t lane = threadIdx.x & 63, r = lane & 31, g2 = lane >> 5;
-  const uint32_t col = slice * 64 + wave * 32 + r; // this lane's column of v
+  const uint32_t lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const uint32_t col = slice * 64 + wave * 16 + r; // this lane's column of v
 
   constexpr uint32_t PAST_THE_END = 0x80000000u; // an offset beyond any descriptor: reads zero, stores nothing
+  const uint64_t S_at = reinterpret_cast<uint64_t>( S_mem ); // (said to be uniform: else every access below becomes a loop over the lanes' addresses)
+  S_mem = reinterpret_cast<float*>( (uint64_t)__builtin_amdgcn_readfirstlane( (uint32_t)( S_at >> 32 ) ) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane( (uint32_t)S_at ) );
   const __amdgpu_buffer_rsrc_t S_rsrc = __builtin_amdgcn_make_buffer_rsrc( S_mem, 0, (int)( s.dim * s.vpad * 4 ), 0x00020000 );
-  const uint32_t S_off = col < s.vpad ? ( 4 * g2 * s.vpad + col ) * 4 : PAST_THE_END;
-  mfma_f32x16 S[DT];
+  const uint32_t S_off = col < s.vpad ? ( 4 * g * s.vpad + col ) * 4 : PAST_THE_END;
+  mfma_f32x4 S[2 * KS]; // rows 16 d + 4 g + v
 #pragma unroll
-  for ( int dt = 0; dt < DT; dt++ ) {
+  for ( int d = 0; d < 2 * KS; d++ ) {
 #pragma unroll
-    for ( int v = 0; v < 16; v++ ) {
-      S[dt][v] = __builtin_bit_cast( float, __builtin_amdgcn_raw_buffer_load_b32( S_rsrc, fresh ? PAST_THE_END : S_off, ( 32 * dt + 8 * ( v / 4 ) + v % 4 ) * s.vpad * 4, 0 ) );
+    for ( int v = 0; v < 4; v++ ) {
+      S[d][v] = __builtin_bit_cast( float, __builtin_amdgcn_raw_buffer_load_b32( S_rsrc, fresh ? PAST_THE_END : S_off, ( 16 * d + v ) * s.vpad * 4, 0 ) );
     }
   }
-  for ( uint32_t d = threadIdx.x; d < 32 * DT; d += 128 ) {
-    s_n[d] = !fresh && d < s.dim ? n_in[d] : 0.0f;
-  }
-  double m0 = fresh ? 0.0 : (double)m_mem;
   const uint64_t row_first = (uint64_t)ctx * st.n_tokens;
   const uint32_t ld_bytes = (uint32_t)( in.main.stride * 2 );
 
-  // LDS byte addresses: a part that depends on the lane, a constant, and a constant XORed with a lane value (the swizzle acts on the
-  // sixteen slots of 256 bytes, or eight of 128).  Computed where they are used: kept in registers over the loop there are too many of them.
-  constexpr uint32_t PERIOD = DT == 2 ? 128 : 256;
-  auto slot_at = [&]( uint32_t constant, uint32_t lane_xor ) __attribute__( ( always_inline ) ) {
-    return constant / PERIOD * PERIOD + ( ( constant % PERIOD ) ^ lane_xor );
-  };
-  auto opaque = []( uint32_t v ) __attribute__( ( always_inline ) ) {
-    asm volatile( "" : "+v"( v ) );
-    return v;
-  };
-  const uint32_t row_swz = swizzle<DT>( r, 0 ) * 16; // of rows r and r + 32
-
-  // rows [0, rows) x `chunks` 16-byte chunks of the product at `p`, LDS rows of 64 DT (or, for v, 128) bytes; the rest reads as zero
-  auto fetch = [&]( uint4* tile, const __bf16* p, uint32_t rows, uint32_t chunks, auto slot_of, auto row_bytes_tag ) {
+  // rows [0, rows) x `chunks` 16-byte chunks of the product at `p`, LDS rows of BYTES; the rest reads as zero
+  auto fetch = [&]( uint4* tile, const __bf16* p, uint32_t rows, uint32_t chunks, auto row_bytes_tag ) __attribute__( ( always_inline ) ) {
     constexpr uint32_t BYTES = decltype( row_bytes_tag )::value;
-    const __amdgpu_buffer_rsrc_t rsrc
-      = __builtin_amdgcn_make_buffer_rsrc( const_cast<__bf16*>( p ), 0, (int)( rows > 0 ? ( rows - 1 ) * ld_bytes + chunks * 16 : 0 ), 0x00020000 );
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<__bf16*>( p ), 0, (int)( ( rows - 1 ) * ld_bytes + chunks * 16 ), 0x00020000 );
     constexpr uint32_t ROWS = 1024 / BYTES; // rows of one instruction of one wave
-    const uint32_t ln = opaque( lane );
 #pragma unroll
-    for ( uint32_t i = 0; i < CHUNK / ( 2 * ROWS ); i++ ) {
-      const uint32_t row0 = ( 2 * i + wave ) * ROWS;
-      const uint32_t row = row0 + ln / ( BYTES / 16 );
-      const uint32_t chunk = slot_of( row, ln % ( BYTES / 16 ) ); // the swizzle is its own inverse
+    for ( uint32_t i = 0; i < CHUNK / ( 4 * ROWS ); i++ ) {
+      const uint32_t row0 = ( 4 * i + wave ) * ROWS;
+      const uint32_t row = row0 + lane / ( BYTES / 16 );
+      const uint32_t chunk = swizzle<BYTES>( row, lane % ( BYTES / 16 ) ); // the swizzle is its own inverse
       const uint32_t off = chunk < chunks ? row * ld_bytes + chunk * 16 : PAST_THE_END;
       __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + row0 * ( BYTES / 16 ) ), 16, off, 0, 0, 0 );
     }
   };
-
-  auto swizzle_row = []( uint32_t row, uint32_t c ) { return swizzle<DT>( row, c ); };
-  auto fetch_qv = [&]( uint32_t t0 ) {
+  auto fetch_qv = [&]( uint32_t t0 ) __attribute__( ( always_inline ) ) {
     const uint32_t rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
     const __bf16* first = in.main.data + ( row_first + t0 ) * in.main.stride;
-    fetch( s_q, first + in.col.q + h * s.dim, rows, s.dim / 8, swizzle_row, std::integral_constant<uint32_t, RB> {} );
-    fetch( s_v, first + in.col.v + h * s.vdim + slice * 64, rows, min( 8u, ( s.vdim - slice * 64 ) / 8 ), swizzle_v, std::integral_constant<uint32_t, 128> {} );
+    fetch( s_q, first + in.col.q + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {} );
+    fetch( s_v, first + in.col.v + h * s.vdim + slice * 64, rows, min( 8u, ( s.vdim - slice * 64 ) / 8 ), std::integral_constant<uint32_t, 128> {} );
   };
 
-  // transposing reads: lane j = 4 e + q of a 16-lane group points at row e (0..3) of its half-wave's four, dims 16 grp + 4 q .. + 3
-  const uint32_t tr_e = ( lane & 15 ) >> 2, tr_q = lane & 3, tr_grp = ( lane >> 4 ) & 1;
-  const uint32_t trk_row = ( 4 * g2 + tr_e ) * RB + ( tr_q & 1 ) * 8, trk_swz = ( swizzle<DT>( 4 * g2 + tr_e, 2 * tr_grp + ( tr_q >> 1 ) ) ) * 16;
-  auto tr_k = [&]( int kk, int dt, uint32_t row, uint32_t swz ) __attribute__( ( always_inline ) ) {
-    union
-    {
-      v4s half[2];
-      bf16x8 x;
-    } u;
-#pragma unroll
-    for ( int hf = 0; hf < 2; hf++ ) { // rows 8 further on: bit 1 of the swizzle's low part
-      u.half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)s_k + row + ( 16 * kk + 8 * hf ) * RB + slot_at( ( 64 * dt ) ^ ( 32 * hf ), swz ) ) );
-    }
-    return u.x;
-  };
-  auto tr_v = [&]( int kk ) __attribute__( ( always_inline ) ) {
+  // 32 rows (keys) x 16 columns from 16-byte chunk `c0` on, transposed: a lane gets its column's rows 4 g + e and 16 + 4 g + e.  Lane 4 e + q of a
+  // 16-lane group points at row e of its four, columns 4 q .. 4 q + 3.
+  const uint32_t tr_row = 4 * g + ( r >> 2 ), tr_q = r & 3;
+  auto transposed = [&]( const uint4* tile, uint32_t row0, uint32_t c0, auto row_bytes_tag ) __attribute__( ( always_inline ) ) {
+    constexpr uint32_t BYTES = decltype( row_bytes_tag )::value;
     union
     {
       v4s half[2];
@@ -459,224 +657,172 @@ __global__ __launch_bounds__( 128, 1 ) void mlstm_chunk_kernel( float* __restric
     } u;
 #pragma unroll
     for ( int hf = 0; hf < 2; hf++ ) {
-      const uint32_t row = 16 * kk + 8 * hf + 4 * g2 + tr_e;
-      u.half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (lds_v4s)( (lds_char*)s_v + row * 128 + swizzle_v( row, 4 * wave + 2 * tr_grp + ( tr_q >> 1 ) ) * 16 + ( tr_q & 1 ) * 8 ) );
+      const uint32_t row = row0 + 16 * hf + tr_row;
+      u.half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)tile + row * BYTES + swizzle<BYTES>( tr_row, c0 + ( tr_q >> 1 ) ) * 16 + ( tr_q & 1 ) * 8 ) );
     }
     return u.x;
   };
 
-  for ( uint32_t t0 = 0; t0 < st.n_tokens; t0 += CHUNK ) {
-    const uint32_t rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
-    const __bf16* first = in.main.data + ( row_first + t0 ) * in.main.stride;
-    if ( t0 > 0 ) {
-      // k of the last chunk is read up to its end, by both waves in whole: neither may have its half replaced before the other is through
-      asm volatile( "s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory" );
-    }
-    fetch( s_k, first + in.col.k + h * s.dim, rows, s.dim / 8, swizzle_row, std::integral_constant<uint32_t, RB> {} );
-    if ( t0 == 0 ) {
-      fetch_qv( 0 );
-    }
+  // Of the four tiles of queries, apart from each other: two reads of 8 bytes at a constant distance would become one instruction whose two halves meet in the
+  // same banks, and whose results have to be moved into their operands' registers.
+  uint32_t q_row[4];
+#pragma unroll
+  for ( int i = 0; i < 4; i++ ) {
+    q_row[i] = ( 16 * i + r ) * RB + ( g & 1 ) * 8;
+    asm( "" : "+v"( q_row[i] ) );
+  }
 
-    // gates: lane = token
-    const bool live = lane < rows;
-    const uint64_t grow = row_first + t0 + ( live ? lane : 0 );
-    const float gi = in.gates[grow * 2 * s.heads + h], gf = in.gates[( grow * 2 + 1 ) * s.heads + h];
-    double b = live ? (double)gf : 0.0;
-#pragma unroll
-    for ( int by = 1; by < 64; by *= 2 ) {
-      const double up = shfl_up_f64( b, by );
-      b += (int)lane >= by ? up : 0.0;
+  float a1 = ch.tokens( MlstmChunks::A, pair, 0 )[lane], w1 = ch.tokens( MlstmChunks::W, pair, 0 )[lane]; // of token `lane`
+  fetch_qv( 0 );
+  __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0)
+  for ( uint32_t c = 0; c < ch.chunks; c++ ) {
+    const uint32_t t0 = c * CHUNK, rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
+    s_n[threadIdx.x] = n;
+    if ( wave == 0 ) {
+      s_a[lane] = a1;
+      s_w[c & 1][lane] = w1;
     }
-    const double c = live ? (double)gi - b : -1e300;
-    double M = c > m0 ? c : m0;
+    // This wave's part of q and v has landed, behind which are no more than the last chunk's 16 stores (memory operations of a wave end in their order).
+    __builtin_amdgcn_s_waitcnt( 0x4F70 ); // vmcnt(16)
+    asm volatile( "s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory" ); // everyone's; and everyone is through with the last chunk's k
+    const uint4* weights = ch.weights + ( (uint64_t)pair * ch.chunks + c ) * ( WEIGHT_TILES * 128 ) + lane;
+    uint4 P[WEIGHT_TILES][2];
 #pragma unroll
-    for ( int by = 1; by < 64; by *= 2 ) {
-      const double up = shfl_up_f64( M, by );
-      M = (int)lane >= by && up > M ? up : M;
+    for ( uint32_t i = 0; i < WEIGHT_TILES; i++ ) {
+      P[i][0] = weights[i * 128];
+      P[i][1] = weights[i * 128 + 64];
     }
-    const double M_end = last_lane_f64( M ), b_end = last_lane_f64( b );
-    const float c_rel = live ? (float)( c - M_end ) : -INFINITY;
-    const float state_decay = expf( (float)( m0 - M_end ) );
-    s_c[wave][lane] = c_rel;
-    s_w[wave][lane] = expf( c_rel );
-    s_a[wave][lane] = expf( (float)( m0 - M ) );
-    const float M_rel = (float)( M - M_end ), floor_den = expf( -(float)( b + M ) ); // of token `lane`
-    m0 = b_end + M_end;
+    const float den1 = ch.tokens( MlstmChunks::DEN, pair, c )[lane], floor1 = ch.tokens( MlstmChunks::FLOOR, pair, c )[lane]; // of token `lane`
+    const float decay = ch.decay[(uint64_t)pair * ch.chunks + c];
+    const float n_more = n_chunk[(uint64_t)c * s.dim];
+    fetch( s_k, in.main.data + ( row_first + t0 ) * in.main.stride + in.col.k + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {} );
+    __builtin_amdgcn_sched_barrier( 0 ); // (else the scheduler moves the requests down to where their results are used)
 
-    __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): this wave's part of the tiles has landed
-    __syncthreads();
-
-    // ---- scores^T and the weights P: query tile tt, key tiles up to it
-    Split<2> P[2][4]; // [query tile][16 keys]
-    float den[2];
+    // ---- Q S (state in front of the chunk): 16 queries a tile
+    mfma_f32x4 O[4];
 #pragma unroll
-    for ( int tt = 0; tt < 2; tt++ ) {
-      const float Mq = __shfl( M_rel, 32 * tt + r ); // of this lane's query
-      den[tt] = 0.0f;
+    for ( int i = 0; i < 4; i++ ) {
+      O[i] = mfma_f32x4 { 0, 0, 0, 0 };
+    }
 #pragma unroll
-      for ( int kt = 0; kt <= tt; kt++ ) {
-        __builtin_amdgcn_sched_barrier( 0 );
-        const uint32_t rb = opaque( r * RB ), swz = opaque( row_swz ^ ( 16 * g2 ) );
-        mfma_f32x16 sc = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+    for ( int j = 0; j < KS; j++ ) {
+      Split<2> sp;
 #pragma unroll
-        for ( int k16 = 0; k16 < 2 * DT; k16++ ) {
-          const uint32_t at = slot_at( 32 * k16, swz );
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>( reinterpret_cast<const char*>( s_k ) + 32 * kt * RB + rb + at );
-          const bf16x8 bq = *reinterpret_cast<const bf16x8*>( reinterpret_cast<const char*>( s_q ) + 32 * tt * RB + rb + at );
-          sc = Mfma<__bf16>::k16( a, bq, sc );
+      for ( int k = 0; k < 4; k++ ) {
+        sp.set( k, S[2 * j + ( k >> 1 )][2 * ( k & 1 )], S[2 * j + ( k >> 1 )][2 * ( k & 1 ) + 1] );
+      }
+      union
+      {
+        uint2 p[2];
+        bf16x8 x;
+      } a[4];
+#pragma unroll
+      for ( int i = 0; i < 4; i++ ) {
+#pragma unroll
+        for ( int hf = 0; hf < 2; hf++ ) {
+          a[i].p[hf] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + q_row[i] + swizzle<RB>( r, 4 * j + 2 * hf + ( g >> 1 ) ) * 16 );
         }
+      }
 #pragma unroll
-        for ( int q4 = 0; q4 < 4; q4++ ) {
-          const uint32_t key0 = opaque( 32 * kt + 8 * q4 + 4 * g2 );
-          const float4 ck = *reinterpret_cast<const float4*>( &s_c[wave][key0] );
-          const float cks[4] = { ck.x, ck.y, ck.z, ck.w };
-          float p[4];
+      for ( int n2 = 1; n2 >= 0; n2-- ) { // (the tiles in turn: a product that waits for the one before it leaves the matrix unit idle)
 #pragma unroll
-          for ( int e = 0; e < 4; e++ ) {
-            const bool seen = kt < tt || key0 + e <= 32 * tt + r;
-            p[e] = seen ? sc[4 * q4 + e] * s.q_scale * __expf( cks[e] - Mq ) : 0.0f;
-            den[tt] += p[e];
-          }
-          P[tt][2 * kt + ( q4 >> 1 )].set( 2 * ( q4 & 1 ), p[0], p[1] );
-          P[tt][2 * kt + ( q4 >> 1 )].set( 2 * ( q4 & 1 ) + 1, p[2], p[3] );
+        for ( int i = 0; i < 4; i++ ) {
+          O[i] = Mfma<__bf16>::k32( a[i].x, sp.t[n2].x, O[i] );
         }
       }
     }
-    // ---- Q S (state in front of the chunk), n . q beside it
-    mfma_f32x16 O[2];
-    float nq[2] = { 0.0f, 0.0f };
+    // ---- denominators of this slice's tokens, a wave each: n . q, four dims a lane
+    for ( uint32_t t0w = slice + wave * 4 * slices; t0w < rows; t0w += 16 * slices ) { // 16 lanes a token
+      const uint32_t t = min( t0w + g * slices, (uint32_t)CHUNK - 1 );
+      float nq = 0.0f;
 #pragma unroll
-    for ( int tt = 0; tt < 2; tt++ ) {
-#pragma unroll
-      for ( int v = 0; v < 16; v++ ) {
-        O[tt][v] = 0.0f;
-      }
-    }
-    __builtin_amdgcn_sched_barrier( 0 ); // (without these fences the scheduler asks for all operands of a phase at once and spills)
-#pragma unroll
-    for ( int dt = 0; dt < DT; dt++ ) {
-#pragma unroll
-      for ( int half = 0; half < 2; half++ ) {
-        __builtin_amdgcn_sched_barrier( 0 );
-        const uint32_t rb = opaque( r * RB + 8 * g2 ), swz = opaque( row_swz );
-        Split<2> sp;
-#pragma unroll
-        for ( int k = 0; k < 4; k++ ) {
-          sp.set( k, S[dt][8 * half + 2 * k], S[dt][8 * half + 2 * k + 1] );
-        }
-#pragma unroll
-        for ( int tt = 0; tt < 2; tt++ ) {
-          union
-          {
-            uint2 p[2];
-            bf16x8 x;
-          } a;
-          a.p[0] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + 32 * tt * RB + rb + slot_at( 64 * dt + 32 * half, swz ) );
-          a.p[1] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + 32 * tt * RB + rb + slot_at( 64 * dt + 32 * half + 16, swz ) );
-          O[tt] = mma( a.x, sp, O[tt] );
-          if ( (uint32_t)( dt / ( DT / 2 ) ) == wave ) { // uniform
-            const float4 n0 = *reinterpret_cast<const float4*>( &s_n[32 * dt + 16 * half + 4 * g2] );
-            const float4 n1 = *reinterpret_cast<const float4*>( &s_n[32 * dt + 16 * half + 8 + 4 * g2] );
-            nq[tt] += (float)a.x[0] * n0.x + (float)a.x[1] * n0.y + (float)a.x[2] * n0.z + (float)a.x[3] * n0.w + (float)a.x[4] * n1.x + (float)a.x[5] * n1.y
-                      + (float)a.x[6] * n1.z + (float)a.x[7] * n1.w;
-          }
+      for ( uint32_t piece = 0; piece < RB / 16; piece += 16 ) { // of 8 dims
+        if ( piece + r < RB / 16 ) {
+          const bf16x8 x = __builtin_bit_cast( bf16x8, s_q[t * ( RB / 16 ) + swizzle<RB>( t, piece + r )] );
+          const float4 n0 = *reinterpret_cast<const float4*>( &s_n[8 * ( piece + r )] ), n1 = *reinterpret_cast<const float4*>( &s_n[8 * ( piece + r ) + 4] ); // (zero past the head's size)
+          nq += (float)x[0] * n0.x + (float)x[1] * n0.y + (float)x[2] * n0.z + (float)x[3] * n0.w + (float)x[4] * n1.x + (float)x[5] * n1.y + (float)x[6] * n1.z + (float)x[7] * n1.w;
         }
       }
-    }
-    bf16x8 V[4];
-#pragma unroll
-    for ( int kk = 0; kk < 4; kk++ ) {
-      V[kk] = tr_v( kk );
-    }
-#pragma unroll
-    for ( int tt = 0; tt < 2; tt++ ) { // the lane 32 further on holds the other half of this query's dims and keys
-      nq[tt] += __shfl_xor( nq[tt], 32 );
-      den[tt] += __shfl_xor( den[tt], 32 );
-      if ( g2 == 0 ) {
-        s_nq[wave][32 * tt + r] = nq[tt];
+      nq = row16_sum( nq );
+      const float over = 1.0f / ( fmaxf( fabsf( nq * s.q_scale * s_a[t] + __shfl( den1, t ) ), __shfl( floor1, t ) ) + 1e-6f );
+      if ( r == 0 && t0w + g * slices < rows ) {
+        ch.tokens( MlstmChunks::OVER, pair, c )[t] = over;
       }
     }
-    __syncthreads(); // both waves have read q and v, and their parts of n . q are there
+    // ---- O = a Q S + P V
+    bf16x8 V[2];
+#pragma unroll
+    for ( int j = 0; j < 2; j++ ) {
+      V[j] = transposed( s_v, 32 * j, 2 * wave, std::integral_constant<uint32_t, 128> {} );
+    }
+#pragma unroll
+    for ( int i = 0; i < 4; i++ ) {
+      const float4 a4 = *reinterpret_cast<const float4*>( &s_a[16 * i + 4 * g] );
+      const float f[4] = { a4.x, a4.y, a4.z, a4.w };
+#pragma unroll
+      for ( int e = 0; e < 4; e++ ) {
+        O[i][e] *= f[e] * s.q_scale;
+      }
+#pragma unroll
+      for ( int j = 0; j <= i / 2; j++ ) {
+#pragma unroll
+        for ( int n2 = 1; n2 >= 0; n2-- ) {
+          O[i] = Mfma<__bf16>::k32( __builtin_bit_cast( bf16x8, P[weight_tile( i, j )][n2] ), V[j], O[i] );
+        }
+      }
+    }
+    __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): this wave's part of k has landed
+    __syncthreads();                      // everyone's; and everyone has read q and v
     if ( t0 + CHUNK < st.n_tokens ) {
+      a1 = ch.tokens( MlstmChunks::A, pair, c + 1 )[lane], w1 = ch.tokens( MlstmChunks::W, pair, c + 1 )[lane];
       fetch_qv( t0 + CHUNK );
     }
-#pragma unroll
-    for ( int tt = 0; tt < 2; tt++ ) {
-      const uint32_t t = 32 * tt + r;
-      const float d = ( s_nq[0][t] + s_nq[1][t] ) * s.q_scale * s_a[wave][t] + den[tt];
-      const float lo = __shfl( floor_den, t );
-      if ( g2 == 0 ) {
-        s_inv[wave][t] = 1.0f / ( fmaxf( fabsf( d ), lo ) + 1e-6f );
-      }
-    }
-    __builtin_amdgcn_sched_barrier( 0 );
-    // ---- O = a Q S + P V, then out
+    __builtin_amdgcn_sched_barrier( 0 ); // the stores stay behind the requests
     const uint32_t hv = s.heads * s.vdim;
     const __amdgpu_buffer_rsrc_t o_rsrc
       = __builtin_amdgcn_make_buffer_rsrc( o_out + ( row_first + t0 ) * hv + h * s.vdim, 0, (int)( ( ( rows - 1 ) * hv + s.vdim ) * 4 ), 0x00020000 );
-    const uint32_t o_off = col < s.vdim ? ( 4 * g2 * hv + col ) * 4 : PAST_THE_END;
+    const uint32_t o_off = col < s.vdim ? ( 4 * g * hv + col ) * 4 : PAST_THE_END;
 #pragma unroll
-    for ( int tt = 0; tt < 2; tt++ ) {
+    for ( int i = 0; i < 4; i++ ) {
 #pragma unroll
-      for ( int q4 = 0; q4 < 4; q4++ ) {
-        const float4 f = *reinterpret_cast<const float4*>( &s_a[wave][32 * tt + 8 * q4 + 4 * g2] );
-        O[tt][4 * q4] *= f.x * s.q_scale;
-        O[tt][4 * q4 + 1] *= f.y * s.q_scale;
-        O[tt][4 * q4 + 2] *= f.z * s.q_scale;
-        O[tt][4 * q4 + 3] *= f.w * s.q_scale;
-      }
-#pragma unroll
-      for ( int kk = 0; kk < 2 * tt + 2; kk++ ) {
-        O[tt] = mma( P[tt][kk], V[kk], O[tt] );
-      }
-#pragma unroll
-      for ( int q4 = 0; q4 < 4; q4++ ) {
-        const uint32_t tok = 32 * tt + 8 * q4 + 4 * g2;
-        const float4 f = *reinterpret_cast<const float4*>( &s_inv[wave][tok] );
-        const float inv[4] = { f.x, f.y, f.z, f.w };
-#pragma unroll
-        for ( int e = 0; e < 4; e++ ) {
-          __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, O[tt][4 * q4 + e] * inv[e] ), o_rsrc, o_off, ( 32 * tt + 8 * q4 + e ) * hv * 4, 0 );
-        }
+      for ( int e = 0; e < 4; e++ ) {
+        __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, (float)O[i][e] ), o_rsrc, o_off, ( 16 * i + e ) * hv * 4, 0 );
       }
     }
-    __builtin_amdgcn_sched_barrier( 0 );
-    // ---- S and n behind the chunk
-    Split<3> wv[4];
+    n = n * decay + n_more;
+    // ---- S behind the chunk
+    Split<3> wv[2];
 #pragma unroll
-    for ( int kk = 0; kk < 4; kk++ ) {
+    for ( int j = 0; j < 2; j++ ) {
 #pragma unroll
       for ( int hf = 0; hf < 2; hf++ ) {
-        const float4 w = *reinterpret_cast<const float4*>( &s_w[wave][16 * kk + 8 * hf + 4 * g2] );
-        wv[kk].set( 2 * hf, (float)V[kk][4 * hf] * w.x, (float)V[kk][4 * hf + 1] * w.y );
-        wv[kk].set( 2 * hf + 1, (float)V[kk][4 * hf + 2] * w.z, (float)V[kk][4 * hf + 3] * w.w );
+        const float4 w = *reinterpret_cast<const float4*>( &s_w[c & 1][32 * j + 16 * hf + 4 * g] );
+        wv[j].set( 2 * hf, (float)V[j][4 * hf] * w.x, (float)V[j][4 * hf + 1] * w.y );
+        wv[j].set( 2 * hf + 1, (float)V[j][4 * hf + 2] * w.z, (float)V[j][4 * hf + 3] * w.w );
       }
     }
 #pragma unroll
-    for ( int dt = 0; dt < DT; dt++ ) {
+    for ( int d0 = 0; d0 < 2 * KS; d0 += 4 ) { // (four tiles in turn, as above)
 #pragma unroll
-      for ( int v = 0; v < 16; v++ ) {
-        S[dt][v] *= state_decay;
-      }
-      float nd = 0.0f;
-      __builtin_amdgcn_sched_barrier( 0 );
-      const uint32_t k_row = opaque( trk_row ), k_swz = opaque( trk_swz );
+      for ( int d = d0; d < d0 + 4; d++ ) {
 #pragma unroll
-      for ( int kk = 0; kk < 4; kk++ ) {
-        const bf16x8 a = tr_k( kk, dt, k_row, k_swz );
-        S[dt] = mma( a, wv[kk], S[dt] );
-        if ( (uint32_t)( dt / ( DT / 2 ) ) == wave ) {
-          const float4 w0 = *reinterpret_cast<const float4*>( &s_w[wave][16 * kk + 4 * g2] );
-          const float4 w1 = *reinterpret_cast<const float4*>( &s_w[wave][16 * kk + 8 + 4 * g2] );
-          nd += (float)a[0] * w0.x + (float)a[1] * w0.y + (float)a[2] * w0.z + (float)a[3] * w0.w + (float)a[4] * w1.x + (float)a[5] * w1.y + (float)a[6] * w1.z
-                + (float)a[7] * w1.w;
+        for ( int v = 0; v < 4; v++ ) {
+          S[d][v] *= decay;
         }
       }
-      if ( (uint32_t)( dt / ( DT / 2 ) ) == wave ) {
-        nd += __shfl_xor( nd, 32 );
-        if ( g2 == 0 ) {
-          s_n[32 * dt + r] = s_n[32 * dt + r] * state_decay + nd;
+#pragma unroll
+      for ( int j = 0; j < 2; j++ ) {
+        bf16x8 a[4];
+#pragma unroll
+        for ( int d = 0; d < 4; d++ ) {
+          a[d] = transposed( s_k, 32 * j, 2 * ( d0 + d ), std::integral_constant<uint32_t, RB> {} );
+        }
+#pragma unroll
+        for ( int n3 = 2; n3 >= 0; n3-- ) {
+#pragma unroll
+          for ( int d = 0; d < 4; d++ ) {
+            S[d0 + d] = Mfma<__bf16>::k32( a[d], wv[j].t[n3].x, S[d0 + d] );
+          }
         }
       }
     }
@@ -685,33 +831,27 @@ __global__ __launch_bounds__( 128, 1 ) void mlstm_chunk_kernel( float* __restric
   uint32_t vpad = s.vpad; // (the row offsets anew: kept from the loads above they would occupy the scalar registers all along)
   asm volatile( "" : "+s"( vpad ) );
 #pragma unroll
-  for ( int dt = 0; dt < DT; dt++ ) {
+  for ( int d = 0; d < 2 * KS; d++ ) {
 #pragma unroll
-    for ( int v = 0; v < 16; v++ ) {
-      __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, (float)S[dt][v] ), S_rsrc, S_off, ( 32 * dt + 8 * ( v / 4 ) + v % 4 ) * vpad * 4, 0 );
+    for ( int v = 0; v < 4; v++ ) {
+      __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, (float)S[d][v] ), S_rsrc, S_off, ( 16 * d + v ) * vpad * 4, 0 );
     }
   }
-  if ( slice == 0 ) {
-    float* dst = nm_out + ( (uint64_t)ctx * s.heads + h ) * ( s.dim + 1 );
-    __syncthreads();
-    for ( uint32_t d = threadIdx.x; d < s.dim; d += 128 ) {
-      dst[d] = s_n[d];
-    }
-    if ( threadIdx.x == 0 ) {
-      dst[s.dim] = (float)m0;
-    }
+  if ( slice == 0 && threadIdx.x < s.dim ) {
+    nm_out[(uint64_t)pair * ( s.dim + 1 ) + threadIdx.x] = n;
   }
 }
 
-// one wave per (token, head); V: columns at a time
-template<typename E, typename View, int V>
+// one wave per (token, head); V: columns at a time; CHUNKED: `o` is not divided by its denominators yet
+template<typename E, typename View, int V, bool CHUNKED>
 __global__ __launch_bounds__( 256 ) void mlstm_finish_kernel( E* __restrict__ out,
                                                               const float* __restrict__ o,
                                                               const float* __restrict__ nm,
                                                               MlstmIn<E, View> in,
                                                               const E* __restrict__ norm,
                                                               MlstmState st,
-                                                              MlstmShape s )
+                                                              MlstmShape s,
+                                                              MlstmChunks ch )
 {
   const uint64_t row = blockIdx.x;
   const uint32_t h = blockIdx.y * 4 + ( threadIdx.x >> 6 ), lane = threadIdx.x & 63;
@@ -722,6 +862,10 @@ __global__ __launch_bounds__( 256 ) void mlstm_finish_kernel( E* __restrict__ ou
   }
   const float* oh = o + row * s.heads * s.vdim + (uint64_t)h * s.vdim;
   E* dst = out + row * s.heads * s.vdim + (uint64_t)h * s.vdim;
+  float over = 1.0f;
+  if constexpr ( CHUNKED ) {
+    over = ch.tokens( MlstmChunks::OVER, ctx * s.heads + h, tok / CHUNK )[tok % CHUNK];
+  }
   if constexpr ( V == 4 ) { // vdim <= 1024, everything in groups of four
     float4 v[4], g[4], w[4];
     float ss = 0.0f;
@@ -731,7 +875,11 @@ __global__ __launch_bounds__( 256 ) void mlstm_finish_kernel( E* __restrict__ ou
       v[k] = *reinterpret_cast<const float4*>( oh + at );
       g[k] = in.main.at4( row, in.col.g + h * s.vdim + at );
       w[k] = ProductView<E>::load4( norm + h * s.vdim + at );
-      ss += c < s.vdim ? v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w : 0.0f;
+    }
+#pragma unroll
+    for ( int k = 0; k < 4; k++ ) {
+      v[k].x *= over, v[k].y *= over, v[k].z *= over, v[k].w *= over;
+      ss += ( k * 64 + lane ) * 4 < s.vdim ? v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w : 0.0f;
     }
     const float inv = 1.0f / sqrtf( wave_sum( ss ) / (float)s.vdim + s.eps );
 #pragma unroll
@@ -758,12 +906,12 @@ __global__ __launch_bounds__( 256 ) void mlstm_finish_kernel( E* __restrict__ ou
   } else {
     float ss = 0.0f;
     for ( uint32_t c = lane; c < s.vdim; c += 64 ) {
-      ss += oh[c] * oh[c];
+      ss += oh[c] * over * ( oh[c] * over );
     }
     const float inv = 1.0f / sqrtf( wave_sum( ss ) / (float)s.vdim + s.eps );
     for ( uint32_t c = lane; c < s.vdim; c += 64 ) {
       const float g = in.main.at( row, in.col.g + h * s.vdim + c );
-      dst[c] = from_f32<E>( oh[c] * inv * to_f32( norm[h * s.vdim + c] ) / ( 1.0f + expf( -g ) ) );
+      dst[c] = from_f32<E>( oh[c] * over * inv * to_f32( norm[h * s.vdim + c] ) / ( 1.0f + expf( -g ) ) );
     }
   }
   if ( tok + 1 == st.n_tokens ) {
@@ -851,12 +999,25 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
   void* scratch = nullptr;
   const uint64_t o_bytes = ( rows * hv * sizeof( float ) + 255 ) / 256 * 256;
   const uint64_t nm_bytes = ( batch * s.heads * ( s.dim + 1ull ) * sizeof( float ) + 255 ) / 256 * 256;
-  if ( int rc = stream_scratch( st, SCRATCH_MIXER, o_bytes + nm_bytes + rows * 2 * s.heads * sizeof( float ), 1ull << 20, &scratch ) ) {
+  const uint64_t n_pairs = batch * s.heads, n_chunks = ( (uint64_t)n_tokens + CHUNK - 1 ) / CHUNK, all_chunks = chunked ? n_pairs * n_chunks : 0;
+  const uint64_t weight_bytes = all_chunks * WEIGHT_TILES * 128 * sizeof( uint4 ), token_bytes = MlstmChunks::PLANES * all_chunks * CHUNK * sizeof( float );
+  const uint64_t more = chunked ? weight_bytes + token_bytes + all_chunks * ( s.dim + 1ull ) * sizeof( float ) : rows * 2 * s.heads * sizeof( float );
+  if ( int rc = stream_scratch( st, SCRATCH_MIXER, o_bytes + nm_bytes + more, 1ull << 20, &scratch ) ) {
     return rc;
   }
   float* o = static_cast<float*>( scratch );
   float* nm = reinterpret_cast<float*>( static_cast<char*>( scratch ) + o_bytes );
-  float* log_gates = reinterpret_cast<float*>( static_cast<char*>( scratch ) + o_bytes + nm_bytes );
+  char* behind = static_cast<char*>( scratch ) + o_bytes + nm_bytes;
+  float* log_gates = reinterpret_cast<float*>( behind );
+  MlstmChunks chunks {};
+  if ( chunked ) {
+    chunks.weights = reinterpret_cast<uint4*>( behind );
+    chunks.token = reinterpret_cast<float*>( behind + weight_bytes );
+    chunks.decay = reinterpret_cast<float*>( behind + weight_bytes + token_bytes );
+    chunks.n = chunks.decay + all_chunks;
+    chunks.chunks = (uint32_t)n_chunks;
+    chunks.plane = all_chunks * CHUNK;
+  }
   const MlstmState state { context_rows_dev, state_offset, start_pos_dev, n_tokens };
   return with_product( dt, y, [&]( auto tag, auto view ) -> int {
     using E = decltype( tag );
@@ -864,7 +1025,7 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
     const MlstmGates<E> raw { ProductView<float>( gates ), col, static_cast<const E*>( bias_i ), static_cast<const E*>( bias_f ), s.cap };
     // One token of a context: every work-group of a head makes the two gates again beside its loads of the state, which is less than a launch in front of it
     // (32 contexts: 4.6 us).
-    const bool gates_made = n_tokens > 1;
+    const bool gates_made = n_tokens > 1 && !chunked;
     if ( gates_made ) {
       mlstm_gates_kernel<E><<<(unsigned)std::min<uint64_t>( ( rows * 2 * s.heads + 255 ) / 256, 4096 ), 256, 0, st>>>( log_gates, raw, s.heads, rows );
       GH_LAUNCH_CHECK();
@@ -874,14 +1035,24 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
     bool walked = false;
     if constexpr ( std::is_same_v<View, ProductView<__bf16>> ) {
       if ( chunked ) {
-        const uint32_t n_pairs = (uint32_t)batch * s.heads;
-        const unsigned groups = ( n_pairs + 7 ) / 8 * 8 * grid.x;
-        if ( s.dim <= 64 ) {
-          mlstm_chunk_kernel<2><<<groups, 128, 0, st>>>( o, nm, in, state, s, grid.x, n_pairs );
-        } else if ( s.dim <= 128 ) {
-          mlstm_chunk_kernel<4><<<groups, 128, 0, st>>>( o, nm, in, state, s, grid.x, n_pairs );
-        } else {
-          mlstm_chunk_kernel<8><<<groups, 128, 0, st>>>( o, nm, in, state, s, grid.x, n_pairs );
+        const unsigned groups = (unsigned)( ( n_pairs + 7 ) / 8 * 8 * grid.x ), score_groups = (unsigned)( ( n_pairs + 7 ) / 8 * 8 * n_chunks );
+        const bool alone = n_chunks == 1;
+        if ( !alone ) {
+          mlstm_scan_kernel<<<dim3( s.heads, (unsigned)batch ), 1024, 0, st>>>( nm, raw, state, s, chunks );
+          GH_LAUNCH_CHECK();
+        }
+        auto walk = [&]( auto steps ) -> int {
+          constexpr int KS = decltype( steps )::value;
+          auto scores = alone ? mlstm_scores_kernel<KS, true> : mlstm_scores_kernel<KS, false>;
+          scores<<<score_groups, 256, 0, st>>>( nm, in, raw, state, s, chunks, (uint32_t)n_pairs );
+          GH_LAUNCH_CHECK();
+          mlstm_states_kernel<KS><<<groups, 256, 0, st>>>( o, nm, in, state, s, chunks, grid.x, (uint32_t)n_pairs );
+          return GH_OK;
+        };
+        const int rc = s.dim <= 64 ? walk( std::integral_constant<int, 2> {} )
+                       : s.dim <= 128 ? walk( std::integral_constant<int, 4> {} ) : walk( std::integral_constant<int, 8> {} );
+        if ( rc ) {
+          return rc;
         }
         walked = true;
       }
@@ -900,11 +1071,21 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
     }
     GH_LAUNCH_CHECK();
     const dim3 finish( (unsigned)rows, ( s.heads + 3 ) / 4 );
+    auto finish_rows = [&]( auto columns ) {
+      constexpr int V = decltype( columns )::value;
+      if constexpr ( std::is_same_v<View, ProductView<__bf16>> ) {
+        if ( walked ) {
+          mlstm_finish_kernel<E, View, V, true><<<finish, 256, 0, st>>>( static_cast<E*>( out ), o, nm, in, static_cast<const E*>( norm ), state, s, chunks );
+          return;
+        }
+      }
+      mlstm_finish_kernel<E, View, V, false><<<finish, 256, 0, st>>>( static_cast<E*>( out ), o, nm, in, static_cast<const E*>( norm ), state, s, chunks );
+    };
     if ( s.vdim % 4 == 0 && s.vdim <= 1024 && view.stride % 4 == 0 && col.g % 4 == 0 && ( reinterpret_cast<uintptr_t>( norm ) & 15u ) == 0
          && ( reinterpret_cast<uintptr_t>( out ) & 15u ) == 0 ) {
-      mlstm_finish_kernel<E, View, 4><<<finish, 256, 0, st>>>( static_cast<E*>( out ), o, nm, in, static_cast<const E*>( norm ), state, s );
+      finish_rows( std::integral_constant<int, 4> {} );
     } else {
-      mlstm_finish_kernel<E, View, 1><<<finish, 256, 0, st>>>( static_cast<E*>( out ), o, nm, in, static_cast<const E*>( norm ), state, s );
+      finish_rows( std::integral_constant<int, 1> {} );
     }
     GH_LAUNCH_CHECK();
     return GH_OK;

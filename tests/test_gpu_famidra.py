@@ -654,6 +654,65 @@ def test_mlstm_walk_of_many_contexts(H, d, dv, batch, dtype):
             assert torch.equal(state[i], alone), i
 
 
+# head sizes below and at each of the kernel's three, that leave part of a step of 32 or of a tile of 64 columns idle; one slice of columns and several;
+# portions of one chunk, of the sixteen that the scan takes at once, of more, all with a last chunk of few tokens
+@pytest.mark.parametrize("H,d,dv", [(3, 40, 8), (2, 64, 136), (1, 72, 64), (4, 128, 72), (2, 232, 200), (1, 256, 64)])
+@pytest.mark.parametrize("cuts", [(24, 65), (1025, 127), (1100,), (33, 1024)])
+def test_mlstm_chunks(H, d, dv, cuts):
+    """Against 64 bits, two contexts and a slot without one.  Weights of the keys and the state meet their partners in two bf16 terms (2^-17); a log gate is
+    off by 2^-22 of itself, and what it is summed over decays with it: weights that matter, above e^-20, are off by 20 x 2^-22 < 2^-17.  Four such errors are
+    allowed to the sums of absolute values, for the numerator and for the denominator; the state is allowed two."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    width, T, B, eps = 8, sum(cuts), 3, 1e-4
+    m = GhMlstm(H, d, dv, 15.0, eps)
+    rows, gate_row = ops.mlstm_weight_rows(m)
+    rng = np.random.default_rng(d + dv)
+    w = rng.integers(-2, 3, (rows, width)).astype(np.float32)             # small whole numbers: the projections are exact
+    w[gate_row:gate_row + 2 * H] *= 0.5
+    bias_i, bias_f, norm = np.linspace(-2, 2, H).astype(np.float32), np.linspace(1, 5, H).astype(np.float32), np.ones(H * dv, np.float32)
+    bias_i, bias_f = M.to_bf16(bias_i), M.to_bf16(bias_f)
+    x = rng.integers(-1, 2, (B, T, width)).astype(np.float32)
+    state = torch.full((B, ops.mlstm_state_bytes(m) // 4), float("nan"), device="cuda")
+    table = ops.row_table([0 if i == 1 else state[i].data_ptr() for i in range(B)])
+    got, at = [], 0
+    for c in cuts:
+        out = ops.mlstm_forward(dev(x[:, at:at + c].reshape(B * c, width), "bf16"), dev(w, "bf16"), m, dev(bias_i, "bf16"), dev(bias_f, "bf16"), dev(norm, "bf16"), table,
+                                torch.full((B,), at, dtype=torch.int32, device="cuda"), c)
+        got.append(back(out).reshape(B, c, H, dv))
+        at += c
+    got = np.concatenate(got, 1)
+    assert (got[1] == 0).all()
+    for b in (0, 2):
+        y = x[b].astype(np.float64) @ w.T
+        q, k, v = (a.reshape(T, H, -1) for a in np.split(y[:, :2 * H * d + H * dv], [H * d, 2 * H * d], 1))
+        q = q * d ** -0.5
+        gate = 1 / (1 + np.exp(-y[:, 2 * H * d + H * dv:2 * H * (d + dv)].reshape(T, H, dv)))
+        li = P.soft_cap(y[:, gate_row:gate_row + H] + bias_i, 15.0)
+        lf = P.log_sigmoid(P.soft_cap(y[:, gate_row + H:gate_row + 2 * H] + bias_f, 15.0))
+        S, n, S_abs, n_abs, top = np.zeros((H, d, dv)), np.zeros((H, d)), np.zeros((H, d, dv)), np.zeros((H, d)), np.zeros(H)
+        for t in range(T):
+            m_new = np.maximum(lf[t] + top, li[t])
+            f, i = np.exp(lf[t] + top - m_new), np.exp(li[t] - m_new)
+            kv = k[t][:, :, None] * v[t][:, None]
+            S, n = f[:, None, None] * S + i[:, None, None] * kv, f[:, None] * n + i[:, None] * k[t]
+            S_abs, n_abs = f[:, None, None] * S_abs + i[:, None, None] * np.abs(kv), f[:, None] * n_abs + i[:, None] * np.abs(k[t])
+            top = m_new
+            den = np.maximum(np.abs((n * q[t]).sum(1)), np.exp(-top))[:, None] + 1e-6
+            o = (S * q[t][:, :, None]).sum(1) / den
+            off = 2.0 ** -15 * ((S_abs * np.abs(q[t])[:, :, None]).sum(1) + np.abs(o) * (n_abs * np.abs(q[t])).sum(1)[:, None]) / den
+            rms = np.sqrt((o ** 2).mean(1) + eps)[:, None]
+            off = (off + np.abs(o) * np.sqrt((off ** 2).mean(1))[:, None] / rms) / rms * gate[t]
+            want = o / rms * gate[t]
+            assert (np.abs(got[b, t] - want) <= 2.0 ** -8 * np.abs(want) + off + 1e-6).all(), (b, t)
+        vp = -(-dv // 4) * 4
+        st = state[b].cpu().numpy().astype(np.float64)
+        assert (np.abs(st[:H * d * vp].reshape(H, d, vp)[:, :, :dv] - S) <= 2.0 ** -16 * S_abs + 1e-9).all(), b
+        assert (np.abs(st[H * d * vp:H * d * (vp + 1)].reshape(H, d) - n) <= 2.0 ** -16 * n_abs + 1e-9).all(), b
+        assert (np.abs(st[-H:] - top) <= 2.0 ** -22 * np.abs(lf).sum(0) + 2.0 ** -20 * 15).all(), b
+
+
 @pytest.mark.parametrize("d,dv,T", [(64, 64, 320), (128, 192, 257), (256, 512, 512)])
 def test_mlstm_same_bits_twice(d, dv, T):
     """The chunks of a prompt share their LDS tiles: with enough work-groups for the waves of one to drift apart, the same inputs give the
