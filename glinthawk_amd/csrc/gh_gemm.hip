@@ -250,44 +250,97 @@ __global__ __launch_bounds__( 256 ) void gemm_reduce_kernel( E* __restrict__ xou
 }
 
 // Few weight rows (r <= 32: the gates of a recurrent mixer) under many activation rows: bound by the activations, which the tile kernels
-// would read with most of their matrix work wasted on rows that are not there.  A work-group takes 32 activation rows, its four waves every
-// fourth 64 of the K range, straight from memory in operand order (eight lanes' pieces make whole 128-byte lines); their sums meet in LDS.
-// fp32 output (b, r).  s % 256 == 0, 16-byte aligned operands.
-constexpr uint32_t SKINNY_ROWS = 32;
-template<typename E>
-__global__ __launch_bounds__( 256 ) void gemm_skinny_kernel( float* __restrict__ out, const E* __restrict__ x, const E* __restrict__ w, uint32_t s, uint32_t r, uint32_t b )
+// would read with most of their matrix work wasted on rows that are not there.  A work-group takes 32 activation rows, its eight waves every
+// eighth 64 of the K range, straight from memory in operand order (a row's 64 bytes an instruction, the rest of the line by the next);
+// their sums meet in LDS.  What counts is how much is asked for at once: two pieces of 64 k a wave, two waves a SIMD.  16 rows of 4096 k
+// at 8192 activation rows: four waves with one piece each, 32 bytes of a row an instruction, 23 to 26 us, so 17.4 (3.9 TB/s; the rest of the
+// time is the launch, the first loads and the sums); 256 rows 16.4 -> 12.5, 32768 78 -> 61.  Four and eight pieces 17.8 and 18.4.
+// fp32 output (b, r).  s % 256 == 0, 16-byte aligned operands.  TILES: of 16 weight rows.
+constexpr uint32_t SKINNY_ROWS = 32, SKINNY_WAVES = 8, SKINNY_AHEAD = 2;
+template<typename E, int TILES>
+__global__ __launch_bounds__( SKINNY_WAVES * 64 ) void gemm_skinny_kernel( float* __restrict__ out, const E* __restrict__ x, const E* __restrict__ w, uint32_t s, uint32_t r, uint32_t b )
 {
-  __shared__ float sums[4][16][64];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, fr = lane & 31, g2 = lane >> 5;
-  const uint32_t token = blockIdx.x * 32 + fr;
-  const E* xp = x + (uint64_t)min( token, b - 1 ) * s + 8 * g2;
-  const E* wp = w + (uint64_t)min( fr, r - 1 ) * s + 8 * g2; // rows past the last repeat it and are not stored
-  mfma_f32x16 acc;
+  typedef typename Mfma<E>::x8 x8;
+  __shared__ float sums[SKINNY_WAVES][8 * TILES][64];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, fr = lane & 15, g = lane >> 4;
+  const uint32_t token0 = blockIdx.x * 32;
+  const E *xp[2], *wp[TILES]; // rows past the last repeat it and are not stored
 #pragma unroll
-  for ( int v = 0; v < 16; v++ ) {
-    acc[v] = 0.0f;
+  for ( uint32_t t = 0; t < 2; t++ ) {
+    xp[t] = x + (uint64_t)min( token0 + 16 * t + fr, b - 1 ) * s + 8 * g;
   }
-  for ( uint32_t k = wave * 64; k < s; k += 256 ) {
 #pragma unroll
-    for ( int i = 0; i < 4; i++ ) {
-      const auto a = *reinterpret_cast<const typename Mfma<E>::x8*>( wp + k + 16 * i );
-      const auto bb = *reinterpret_cast<const typename Mfma<E>::x8*>( xp + k + 16 * i );
-      acc = Mfma<E>::k16( a, bb, acc );
+  for ( uint32_t i = 0; i < TILES; i++ ) {
+    wp[i] = w + (uint64_t)min( 16 * i + fr, r - 1 ) * s + 8 * g;
+  }
+  mfma_f32x4 acc[TILES][2];
+#pragma unroll
+  for ( int i = 0; i < TILES; i++ ) {
+    acc[i][0] = acc[i][1] = mfma_f32x4 { 0.0f, 0.0f, 0.0f, 0.0f };
+  }
+  auto pieces = [&]( uint32_t k, auto count ) __attribute__( ( always_inline ) ) {
+    constexpr int U = decltype( count )::value;
+    x8 xv[U][2][2], wv[U][2][TILES];
+#pragma unroll
+    for ( int u = 0; u < U; u++ ) {
+#pragma unroll
+      for ( int h = 0; h < 2; h++ ) {
+#pragma unroll
+        for ( int t = 0; t < 2; t++ ) {
+          xv[u][h][t] = *reinterpret_cast<const x8*>( xp[t] + k + 64 * SKINNY_WAVES * u + 32 * h );
+        }
+#pragma unroll
+        for ( int i = 0; i < TILES; i++ ) {
+          wv[u][h][i] = *reinterpret_cast<const x8*>( wp[i] + k + 64 * SKINNY_WAVES * u + 32 * h );
+        }
+      }
     }
-  }
-  // acc[v]: weight row 8 * (v / 4) + 4 * g2 + v % 4, token fr
+    __builtin_amdgcn_sched_barrier( 0 ); // (else the scheduler asks for one piece at a time)
 #pragma unroll
-  for ( int v = 0; v < 16; v++ ) {
-    sums[wave][v][lane] = acc[v];
+    for ( int u = 0; u < U; u++ ) {
+#pragma unroll
+      for ( int h = 0; h < 2; h++ ) {
+#pragma unroll
+        for ( int i = 0; i < TILES; i++ ) {
+#pragma unroll
+          for ( int t = 0; t < 2; t++ ) {
+            acc[i][t] = Mfma<E>::k32( wv[u][h][i], xv[u][h][t], acc[i][t] );
+          }
+        }
+      }
+    }
+  };
+  uint32_t k = wave * 64;
+  for ( ; k + 64 * SKINNY_WAVES * ( SKINNY_AHEAD - 1 ) < s; k += 64 * SKINNY_WAVES * SKINNY_AHEAD ) {
+    pieces( k, std::integral_constant<int, SKINNY_AHEAD> {} );
+  }
+  for ( ; k < s; k += 64 * SKINNY_WAVES ) {
+    pieces( k, std::integral_constant<int, 1> {} );
+  }
+  // acc[i][t][v]: weight row 16 i + 4 g + v, token 16 t + fr
+#pragma unroll
+  for ( int i = 0; i < TILES; i++ ) {
+#pragma unroll
+    for ( int t = 0; t < 2; t++ ) {
+#pragma unroll
+      for ( int v = 0; v < 4; v++ ) {
+        sums[wave][8 * i + 4 * t + v][lane] = acc[i][t][v];
+      }
+    }
   }
   __syncthreads();
 #pragma unroll
-  for ( uint32_t i = 0; i < 4; i++ ) {
-    const uint32_t v = wave * 4 + i;
-    const uint32_t row = 8 * ( v / 4 ) + 4 * g2 + v % 4;
-    const float y = ( sums[0][v][lane] + sums[1][v][lane] ) + ( sums[2][v][lane] + sums[3][v][lane] );
+  for ( uint32_t n = 0; n < TILES; n++ ) {
+    const uint32_t at = wave * TILES + n;
+    float y[SKINNY_WAVES];
+#pragma unroll
+    for ( uint32_t o = 0; o < SKINNY_WAVES; o++ ) {
+      y[o] = sums[o][at][lane];
+    }
+    const float sum = ( ( y[0] + y[1] ) + ( y[2] + y[3] ) ) + ( ( y[4] + y[5] ) + ( y[6] + y[7] ) );
+    const uint32_t row = 16 * ( at / 8 ) + 4 * g + at % 4, token = token0 + 16 * ( ( at / 4 ) % 2 ) + fr;
     if ( row < r && token < b ) {
-      out[(uint64_t)token * r + row] = y;
+      out[(uint64_t)token * r + row] = sum;
     }
   }
 }
@@ -357,10 +410,11 @@ static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, c
 }
 
 // Tokens of the first part when a product, `whole_ns` in one, is better run as whole rounds of 256 x 256 tiles and a rest, rest_ns( tokens ); 0 otherwise.
+// `whole_ns` becomes what the choice needs.
 template<typename F>
-static uint64_t cut_tokens( uint64_t s, uint64_t r, uint64_t b, double whole_ns, F&& rest_ns )
+static uint64_t cut_tokens( uint64_t s, uint64_t r, uint64_t b, double& whole_ns, F&& rest_ns )
 {
-  double best = whole_ns;
+  double& best = whole_ns;
   uint64_t best_b1 = 0;
   const uint64_t rounds = gemm_tile256_rounds( r, b );
   for ( uint64_t n = 1; n < 3 && n < rounds; n++ ) { // the first part one round shorter, or two
@@ -383,7 +437,18 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
   if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
     return 0;
   }
-  return cut_tokens( s, r, b, half_plan( s, r, b, true ).ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
+  double ns = half_plan( s, r, b, true ).ns;
+  return cut_tokens( s, r, b, ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
+}
+
+// what a rounded product is estimated to need, aligned operands
+static double product_ns( uint64_t s, uint64_t r, uint64_t b )
+{
+  double ns = half_plan( s, r, b, true ).ns;
+  if ( gemm_tile256_takes( s, b, nullptr, nullptr, nullptr ) ) {
+    cut_tokens( s, r, b, ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
+  }
+  return ns;
 }
 
 // Which kernel takes w1, w3 and the gate in one launch (what is left of it once gemm_token_split() has cut it); none: two launches.
@@ -525,6 +590,23 @@ int gemm_tile_qkv_launch( void* q, const void* x, const void* wqkv, uint64_t s, 
                : GH_OK;
 }
 
+static bool skinny_takes( uint64_t s, uint64_t r, uint64_t b, const void* x, const void* w )
+{
+  return g_force_kernel == 0 && r <= SKINNY_ROWS && b >= 192 && b < ( 1ull << 31 ) && s % 256 == 0
+         && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) ) & 15u ) == 0;
+}
+
+// Whether the last `few` rows of a rounded product of r are better a product of their own: where the others fill rounds of 256 x 256 tiles that all of them
+// overflow.  8192 + 32 rows of 4096 k at 8192 activation rows: 360 us and 39 for the tokens that are left over, against 360 and 20 (the whole prefill of 4 x 2048 tokens 4910 -> 4748 us).
+bool gemm_few_rows_apart( uint64_t s, uint64_t r, uint64_t few, uint64_t b, gh_dtype dt, const void* x, const void* w )
+{
+  if ( !is_half_type( dt ) || few == 0 || few >= r || !gemm_ring_applicable( s, r, b, x, w, x ) || !skinny_takes( s, few, b, x, static_cast<const char*>( w ) + ( r - few ) * s * 2 ) ) {
+    return false;
+  }
+  const double skinny_ns = 5000.0 + (double)( b * s ) * 2.0 / 4500.0;
+  return product_ns( s, r, b ) > product_ns( s, r - few, b ) + skinny_ns;
+}
+
 // The 16-bit part of gemm_partials(): runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums
 // `[splits][b][r]` in the library's workspace (*partial_out, *splits_out) for a fused epilogue; otherwise the kernel may store
 // DType results straight into `xout` (*splits_out == 0 then).
@@ -532,15 +614,15 @@ template<typename E>
 int gemm_half_partials( E* xout, const E* x, const E* w, uint64_t s, uint64_t r, uint64_t b, hipStream_t st, bool want_partials, float** partial_out,
                         uint32_t* splits_out )
 {
-  if ( want_partials && g_force_kernel == 0 && r <= SKINNY_ROWS && b >= 192 && b < ( 1ull << 31 ) && s % 256 == 0
-       && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) ) & 15u ) == 0 ) {
+  if ( want_partials && skinny_takes( s, r, b, x, w ) ) {
     float* ws = nullptr;
     if ( int rc = ensure_workspace( b * r * sizeof( float ), &ws, st ) ) {
       return rc;
     }
     *partial_out = ws;
     *splits_out = 1;
-    gemm_skinny_kernel<E><<<(unsigned)( ( b + 31 ) / 32 ), 256, 0, st>>>( ws, x, w, (uint32_t)s, (uint32_t)r, (uint32_t)b );
+    auto kernel = r <= 16 ? gemm_skinny_kernel<E, 1> : gemm_skinny_kernel<E, 2>;
+    kernel<<<(unsigned)( ( b + 31 ) / 32 ), SKINNY_WAVES * 64, 0, st>>>( ws, x, w, (uint32_t)s, (uint32_t)r, (uint32_t)b );
     GH_LAUNCH_CHECK();
     return GH_OK;
   }

@@ -130,6 +130,38 @@ def test_feed_forward_of_many_rows_with_tanh(n_tokens, ff):
     assert bool((wide[~live] == 5).all()) and bool((wide[:, :40] == 5).all()) and bool((wide[:, 40 + ff:] == 5).all())
 
 
+# rows that fill their rounds of tiles without the gates, all of them and a ragged number of tokens, heads that are not a multiple of eight; few rows
+@pytest.mark.parametrize("heads,kv,n_tokens,width,apart", [(32, 32, 4096, 2048, True), (28, 4, 8150, 2048, True), (32, 32, 100, 2048, False), (28, 4, 4096, 256, False)])
+def test_head_gates_of_many_rows(heads, kv, n_tokens, width, apart):
+    """Gates whose product is one of its own keep fp32 sums (2^-20 of about one, a quarter of it behind the sigmoid, and its fast exponential); as columns of the
+    rounded product they are off by 2^-9 of themselves.  Queries and keys stay as they are, and a context without an entry gets none."""
+    import torch
+    from glinthawk_amd import ops
+    d = 128
+    a = ops.window_attn(heads, kv, d, d, 1.0, values_are_keys=True)
+    rows, _ = ops.parallel_weight_rows(a, True, 0)
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    w = (torch.randn((rows, width), generator=g, device="cuda") * width ** -0.5).bfloat16()
+    x = torch.randn((3 * n_tokens, width), generator=g, device="cuda").bfloat16()
+    keys = -(-n_tokens // 32) * 32
+    at = keys * kv * d * 2
+    regions = [torch.zeros(at + keys * kv * 4, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    q, gates = ops.matmul_parallel(x, w, a, ops.row_table([regions[0].data_ptr(), 0, regions[1].data_ptr()]), positions([0, 0, 0]), n_tokens, 1e-3, 0.0, 0, True, None, factor_offset=at)
+    nq, nk = heads * d, kv * d
+    for i, region in ((0, regions[0]), (2, regions[1])):
+        part = slice(i * n_tokens, (i + 1) * n_tokens)
+        z = x[part].double() @ w[nq + nk:nq + nk + heads].double().T
+        off = (gates[part].double() - torch.sigmoid(z)).abs()
+        assert bool((off <= (1e-5 if apart else 2.0 ** -10 * z.abs() + 1e-5)).all()), float(off.max())
+        y = x[part].float() @ w[:nq + nk].float().T
+        raw = y[:, :nq].view(n_tokens, heads, d)
+        want = raw / (raw.square().mean(-1, keepdim=True) + 1e-3).sqrt()
+        assert bool(((q[part].view(n_tokens, heads, d).float() - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -8).all())
+        got = region[:at].view(torch.bfloat16).view(keys, nk)[:n_tokens].float()
+        assert bool(((got - y[:, nq:]).abs() <= 2.0 ** -8 * y[:, nq:].abs() + 1e-4).all())
+    assert not bool(q[n_tokens:2 * n_tokens].any()) and not bool(gates[n_tokens:2 * n_tokens].any())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("n_tokens", [1, 4, 250, 600])
 @pytest.mark.parametrize("heads,kv,d,ff,gated,every", [(6, 3, 20, 44, True, 7), (4, 1, 64, 0, True, 1), (5, 5, 96, 72, False, 33), (3, 1, 136, 21, True, 64), (2, 2, 300, 40, True, 0),
