@@ -1,6 +1,7 @@
 // Internal helpers shared by the HIP translation units of libglint_hip.so (gfx950 only).
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -259,6 +260,31 @@ template<>
 __device__ __forceinline__ __bf16 from_f32<__bf16>( float v )
 {
   return (__bf16)v; // to nearest even
+}
+
+// two values rounded as one instruction takes them, to nearest even: a in the low half
+template<typename E>
+__device__ __forceinline__ uint32_t rounded_pair( float a, float b )
+{
+  typedef float f32x2 __attribute__( ( ext_vector_type( 2 ) ) );
+  typedef _Float16 f16x2 __attribute__( ( ext_vector_type( 2 ) ) );
+  typedef __bf16 b16x2 __attribute__( ( ext_vector_type( 2 ) ) );
+  if constexpr ( std::is_same_v<E, __half> ) {
+    return __builtin_bit_cast( uint32_t, __builtin_convertvector( ( f32x2 { a, b } ), f16x2 ) );
+  } else {
+    return __builtin_bit_cast( uint32_t, __builtin_convertvector( ( f32x2 { a, b } ), b16x2 ) );
+  }
+}
+
+// y / (1 + exp(-z)), of a gate.  The divisor is at least 1 and, where the quotient does not vanish, below 2^126, so its reciprocal (one Newton step) and the
+// quotient's remainder need no scaling, and the exponential none below the smallest normal number, which leaves 1 as it is: 12 instructions where the
+// general division and exponential take 18.  The quotient is the general one's; -87 and less give 0.
+__device__ __forceinline__ float sigmoid_times( float y, float z )
+{
+  const float d = 1.0f + __builtin_amdgcn_exp2f( z * -1.44269504088896340736f );
+  const float r0 = __builtin_amdgcn_rcpf( d ), r = __builtin_fmaf( __builtin_fmaf( -d, r0, 1.0f ), r0, r0 );
+  const float q = y * r;
+  return __builtin_amdgcn_div_fixupf( __builtin_fmaf( __builtin_fmaf( -d, q, y ), r, q ), d, y ); // (infinities and NaN)
 }
 
 // ---- matrix cores: operands of eight 16-bit elements a lane ------------------------------------

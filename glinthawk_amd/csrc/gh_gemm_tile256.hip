@@ -87,6 +87,9 @@ __device__ __forceinline__ bool tile_of_index( const TileOrder& ord, uint32_t xc
 // again (13B, 16384 tokens: 271 us a layer; the pass of four 36.9 -> 35.5 ms).  With one work-group per CU nothing hides the epilogue, so a
 // gate that takes longer is a variant of its own, bf16: the tanh gate, and biases, kept in LDS since the tile before (8192 rows, 2 x 11008 of
 // 4096 k: 1083 us as a rounded product and a kernel behind it, 984 so; 1024 rows of 2 x 2816 of 1024 k 33.8 and 26.1).
+// The gate's epilogue is 1475 vector instructions a wave with the general division and every factor also rounded for the case that it counts, 738 as it is (bf16;
+// f16, which rounds the factors, 1410 and 933): some 3 of a 64-step tile's 95 us, of which the power budget takes back a part (4 x 2048 tokens of the design whose gate
+// is half of its time 4851 -> 4799 us, 26 x 128 of 70B 17.55 -> 17.47 ms).
 // Or q, k and v as QkvRows says, 16-byte pieces of a token's heads to its query and its cache row: the two kernels that read the product again, append and
 // rotate took 260 us a layer at 13B and 16384 tokens (3 x 5120 rows of 5120), this epilogue 55 of the product's 1785 (1730 with plain stores).
 constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3, EPI_QKV = 4, EPI_BIAS_GATE = 5;
@@ -122,20 +125,21 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
   union Chunk
   {
     uint4 raw;
+    uint32_t pair[4];
     E h[8];
   };
   auto rounded = [&]( int a, int h, int i, int j ) __attribute__( ( always_inline ) ) {
     Chunk y;
 #pragma unroll
-    for ( int e = 0; e < 8; e++ ) {
-      y.h[e] = from_f32<E>( acc[a][h][2 * i + ( e >> 2 )][j][e & 3] );
+    for ( int e = 0; e < 8; e += 2 ) {
+      y.pair[e / 2] = rounded_pair<E>( acc[a][h][2 * i + ( e >> 2 )][j][e & 3], acc[a][h][2 * i + ( e >> 2 )][j][( e & 3 ) + 1] );
     }
     return y;
   };
   auto added = []( Chunk y, const Chunk& old ) __attribute__( ( always_inline ) ) { // the op that follows the product, on the rounded product
 #pragma unroll
-    for ( int e = 0; e < 8; e++ ) {
-      y.h[e] = from_f32<E>( to_f32<E>( old.h[e] ) + to_f32<E>( y.h[e] ) );
+    for ( int e = 0; e < 8; e += 2 ) {
+      y.pair[e / 2] = rounded_pair<E>( to_f32<E>( old.h[e] ) + to_f32<E>( y.h[e] ), to_f32<E>( old.h[e + 1] ) + to_f32<E>( y.h[e + 1] ) );
     }
     return y;
   };
@@ -161,28 +165,37 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
   }
   if constexpr ( EPI == EPI_GATE || EPI == EPI_BIAS_GATE ) { // tile_row0: of the output
     constexpr bool BIAS = EPI == EPI_BIAS_GATE;
-    auto values = [&]( int h, int i, int j, auto act ) __attribute__( ( always_inline ) ) {
-      Chunk y;
+    auto values = [&]( int h, int i, int j, auto act, auto exact ) __attribute__( ( always_inline ) ) {
+      Chunk y, y1, y3; // (the rounded factors)
+      if constexpr ( !BIAS && !exact.value ) {
+        y1 = rounded( 0, h, i, j ), y3 = rounded( 1, h, i, j );
+      }
+      float g[8];
 #pragma unroll
       for ( int e = 0; e < 8; e++ ) {
         const float a1 = acc[0][h][2 * i + ( e >> 2 )][j][e & 3], a3 = acc[1][h][2 * i + ( e >> 2 )][j][e & 3];
         if constexpr ( BIAS ) {
           const float* bias = reinterpret_cast<const float*>( tokens ) + 64 * group + 8 * ( lane >> 4 ) + 32 * i + e;
-          y.h[e] = from_f32<E>( activate<E>( a1 + bias[0], act ) * ( a3 + bias[TM2 / 2] ) );
+          g[e] = activate<E>( a1 + bias[0], act ) * ( a3 + bias[TM2 / 2] );
+        } else if constexpr ( exact.value ) {
+          g[e] = sigmoid_times( a1, a1 ) * a3;
         } else {
-          const float y1 = o.gate.exact ? a1 : to_f32<E>( from_f32<E>( a1 ) ), y3 = o.gate.exact ? a3 : to_f32<E>( from_f32<E>( a3 ) );
-          y.h[e] = from_f32<E>( y1 / ( 1.0f + __expf( -y1 ) ) * y3 );
+          g[e] = sigmoid_times( to_f32<E>( y1.h[e] ), to_f32<E>( y1.h[e] ) ) * to_f32<E>( y3.h[e] );
         }
+      }
+#pragma unroll
+      for ( int e = 0; e < 8; e += 2 ) {
+        y.pair[e / 2] = rounded_pair<E>( g[e], g[e + 1] );
       }
       return y;
     };
     E* base = static_cast<E*>( o.xout ) + (uint64_t)col0 * o.gate.stride + row0;
-    auto store = [&]( auto all, auto act ) __attribute__( ( always_inline ) ) {
+    auto store = [&]( auto all, auto act, auto exact ) __attribute__( ( always_inline ) ) {
 #pragma unroll
       for ( int n = 0; n < 8; n++ ) { // (with biases the four outputs of a row in turn)
         const int h = BIAS ? ( n >> 1 ) & 1 : n >> 2, j = BIAS ? n & 1 : ( n >> 1 ) & 1, i = BIAS ? n >> 2 : n & 1;
         const uint32_t col = col0 + 128 * h + 16 * j;
-        const Chunk y = values( h, i, j, act );
+        const Chunk y = values( h, i, j, act, exact );
         if ( all.value
              || ( row0 + 32 * i < o.r && col < o.b && ( o.gate.context_rows == nullptr || o.gate.context_rows[col / o.gate.n_tokens] != nullptr ) ) ) {
           *reinterpret_cast<uint4*>( base + ( 128 * h + 16 * j ) * o.gate.stride + 32 * i ) = y.raw; // r % 8 == 0: eight rows
@@ -191,13 +204,19 @@ __device__ __forceinline__ bool store_tile( const mfma_f32x4 ( &acc )[2][2][4][2
     };
     if ( ( tile_row0 + TM2 / 2 <= o.r ) & ( tile_col0 + TN2 <= o.b ) & ( o.gate.context_rows == nullptr ) ) {
       if ( BIAS && o.gate.activation == GH_ACT_GELU_TANH ) {
-        store( std::true_type {}, std::integral_constant<int, GH_ACT_GELU_TANH> {} );
+        store( std::true_type {}, std::integral_constant<int, GH_ACT_GELU_TANH> {}, std::true_type {} );
+      } else if ( BIAS || o.gate.exact ) {
+        store( std::true_type {}, std::integral_constant<int, GH_ACT_SILU> {}, std::true_type {} );
       } else {
-        store( std::true_type {}, std::integral_constant<int, GH_ACT_SILU> {} );
+        store( std::true_type {}, std::integral_constant<int, GH_ACT_SILU> {}, std::false_type {} );
       }
       return true;
     }
-    store( std::false_type {}, o.gate.activation );
+    if ( BIAS || o.gate.exact ) {
+      store( std::false_type {}, o.gate.activation, std::true_type {} );
+    } else {
+      store( std::false_type {}, o.gate.activation, std::false_type {} );
+    }
     drain_loads_and_stores();
     return false;
   }

@@ -43,9 +43,9 @@ __device__ __forceinline__ float activate( float z, int act )
   if ( act == GH_ACT_GELU_TANH ) {
     const float u = 0.7978845608028654f * ( z + 0.044715f * z * z * z );
     // 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)); the fp32 build takes the library's tanh
-    return sizeof( E ) == 4 ? 0.5f * z * ( 1.0f + tanhf( u ) ) : z / ( 1.0f + __expf( -2.0f * u ) );
+    return sizeof( E ) == 4 ? 0.5f * z * ( 1.0f + tanhf( u ) ) : sigmoid_times( z, 2.0f * u );
   }
-  return z / ( 1.0f + ( sizeof( E ) == 4 ? expf( -z ) : __expf( -z ) ) );
+  return sizeof( E ) == 4 ? z / ( 1.0f + expf( -z ) ) : sigmoid_times( z, z );
 }
 
 // the stored value of one output, y1 and y3 the fp32 sums of its factors; rows: of each factor

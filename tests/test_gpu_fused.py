@@ -301,6 +301,44 @@ def test_matmul_gate_of_whole_tiles(b, s, hidden, bias, activation):
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * (1.0 + want.abs().sqrt())).all()
 
 
+# 512 rows: the tiles' epilogues whole and with a ragged last tile; 16: the ring kernel
+@pytest.mark.parametrize("b,hidden", [(512, 16384), (500, 16280), (16, 16384)])
+@pytest.mark.parametrize("dt,activation,bias", [(torch.float16, ops.GH_ACT_SILU, False), (torch.bfloat16, ops.GH_ACT_SILU, False), (torch.bfloat16, ops.GH_ACT_SILU, True),
+                                                (torch.bfloat16, ops.GH_ACT_GELU_TANH, False)])
+def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
+    """Factors that are one weight each, so that the sums are exact: over the range of the exponential, signed zeros, the type's smallest and largest,
+    infinities and NaN, against 64 bits.  One rounding to the type, and the exponent's own, 2^-23 of its 127 at most; below 2^-119 (f16: its smallest) nothing is asked
+    but the size: from a divisor of 2^126 on, at factors of -87.3 and less, the reciprocal may be 0, and the quotient is at most 88.8 * 2^-126."""
+    lim = torch.finfo(dt)
+    a = torch.cat([torch.linspace(-130.0, 130.0, 521), torch.tensor([0.0, -0.0, lim.tiny, -lim.tiny, lim.max, lim.min, float("inf"), -float("inf"), float("nan")]),
+                   torch.logspace(-6, 4, 101), -torch.logspace(-6, 4, 101)]).to(dt).cuda()
+    u = torch.tensor([1.0, -0.75, 1.5e-3], device="cuda").to(dt)
+    w = torch.zeros((2 * hidden, 128), device="cuda", dtype=dt)
+    n = torch.arange(hidden, device="cuda")
+    w[:hidden, 0], w[hidden:, 0] = a[n % len(a)], u[n // len(a) % len(u)]
+    x = torch.zeros((b, 128), device="cuda", dtype=dt)
+    x[:, 0] = 1.0
+    lib = _lib.lib()
+    _lib.check(lib.gh_gemm_set_tuning(4 if b > 16 else 5, 0, 0))
+    try:
+        if dt == torch.float16:
+            got = ops.matmul_silu_gate(x, w).double()
+        else:
+            got = ops.matmul_gate(x, w, torch.zeros(2 * hidden, device="cuda", dtype=dt) if bias else None, activation).double()
+    finally:
+        _lib.check(lib.gh_gemm_set_tuning(0, 0, 0))
+    y, f = w[:hidden, 0].double(), w[hidden:, 0].double()
+    z = y if activation == ops.GH_ACT_SILU else 2 * 0.7978845608028654 * (y + 0.044715 * y ** 3)
+    exact = y / (1.0 + torch.exp(-z)) * f
+    for row in (got[0], got[-1]):
+        finite = exact.isfinite() & (exact.abs() <= lim.max)
+        assert torch.equal(row.isnan(), exact.isnan())
+        assert torch.equal(row[exact.isinf()], exact[exact.isinf()])
+        eps = (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 127 * 2.0 ** -23 + (3 * 2.0 ** -23 * z.abs().clamp(max=130.0))
+        small = lim.tiny * 2.0 ** -10 if dt == torch.float16 else 2.0 ** -119
+        assert ((row - exact).abs() <= eps * exact.abs() + small)[finite].all()
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [Shape(dim=32, n_layers=1, n_heads=4, n_kv_heads=2, hidden_dim=48, seq_len=16),
                                    Shape(dim=288, n_layers=1, n_heads=6, n_kv_heads=6, hidden_dim=768, seq_len=256),
