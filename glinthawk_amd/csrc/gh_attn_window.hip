@@ -130,82 +130,160 @@ __global__ __launch_bounds__( 1024 ) void window_append4_kernel( E* __restrict__
   }
 }
 
-// prompts (bias and both norms present): work-group = a token's q, k and v together, the columns of the product in one run; all loads go out
-// together and both sums meet at one barrier
-template<typename E, typename View, int NV>
-__global__ __launch_bounds__( 1024 ) void window_append_row_kernel( E* __restrict__ q_out, View y, const E* __restrict__ bias, AppendPart pq, AppendPart pk, AppendPart pv,
-                                                                    WindowRows wr, WindowShape s, float eps )
+// Prompts (bias and both norms present): a token's q, k and v together, the columns of the product in one run, 4 V of them a group; both sums meet at one barrier.
+// Bound by memory: 403 MB at 8192 tokens of 3 x 4096 columns.  A work-group keeps the tables in registers over its tokens, every gridDim.x-th, and asks for the next
+// token's columns before it reduces this one's, so that reads pass while stores do; 16 bytes a lane: 82 us (4.9 TB/s).  8 bytes a lane 101, a work-group for each
+// token with 8 bytes a lane 112.
+template<typename E, typename View, int NV, int V>
+__global__ __launch_bounds__( 1024 ) __attribute__( ( amdgpu_waves_per_eu( 6, 8 ) ) ) void window_append_row_kernel( E* __restrict__ q_out, View y, const E* __restrict__ bias, AppendPart pq, AppendPart pk, AppendPart pv,
+                                                                    WindowRows wr, WindowShape s, float eps, uint32_t rows )
 {
-  __shared__ float q_sums[16], k_sums[16];
-  const uint64_t row = blockIdx.x;
-  const uint32_t ctx = (uint32_t)( row / wr.n_tokens ), tok = (uint32_t)( row % wr.n_tokens );
-  uint8_t* base = static_cast<uint8_t*>( wr.rows[ctx] );
-  if ( base == nullptr ) {
-    return;
-  }
+  __shared__ float q_sums[2][16], k_sums[2][16];
   const uint32_t cols = pv.first + pv.cols;
   const E *q_norm = static_cast<const E*>( pq.norm ), *k_norm = static_cast<const E*>( pk.norm );
-  float4 v[NV], w[NV];
-  float qq = 0.0f, kk = 0.0f;
+  typedef typename ProductView<E>::Four Four;
+  constexpr bool KEPT = sizeof( E ) == 2;
+  typename View::Four ahead[NV][V];
+  Four w[NV][V], add[NV][V];
+  uint32_t col[NV];
+  auto fours = []( auto ( &to )[V], const auto* from ) __attribute__( ( always_inline ) ) {
+    struct alignas( sizeof( to ) ) Run
+    {
+      std::remove_reference_t<decltype( to[0] )> f[V];
+    };
+    const Run r = *reinterpret_cast<const Run*>( from );
+#pragma unroll
+    for ( int n = 0; n < V; n++ ) {
+      to[n] = r.f[n];
+    }
+  };
+  auto columns = [&]( typename View::Four ( &to )[V], uint64_t row, uint32_t c ) __attribute__( ( always_inline ) ) {
+    if constexpr ( V == 1 ) {
+      to[0] = y.four( row, c );
+    } else { // (one plane)
+      fours( to, y.data + row * y.stride + c );
+    }
+  };
+  auto read = [&]( uint32_t c ) __attribute__( ( always_inline ) ) { return c < cols ? c : 0; }; // past the row's end: its first ones
 #pragma unroll
   for ( int g = 0; g < NV; g++ ) {
-    const uint32_t c = ( g * blockDim.x + threadIdx.x ) * 4, at = c < cols ? c : 0;
-    v[g] = y.at4( row, at );
-    const bool is_q = at < pk.first;
-    w[g] = ProductView<E>::load4( is_q ? q_norm + at : k_norm + ( at < pv.first ? at - pk.first : 0 ) ); // (v: not used)
-    const float4 b = ProductView<E>::load4( bias + at );
-    v[g] = make_float4( v[g].x + b.x, v[g].y + b.y, v[g].z + b.z, v[g].w + b.w );
-    const float sum = c < pv.first ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
-    qq += is_q ? sum : 0.0f;
-    kk += is_q ? 0.0f : sum;
+    col[g] = ( g * blockDim.x + threadIdx.x ) * ( 4 * V );
+    if constexpr ( KEPT ) {
+      columns( ahead[g], blockIdx.x, read( col[g] ) );
+    }
   }
-  qq = wave_sum( qq );
-  kk = wave_sum( kk );
-  if ( ( threadIdx.x & 63 ) == 0 ) {
-    q_sums[threadIdx.x >> 6] = qq;
-    k_sums[threadIdx.x >> 6] = kk;
-  }
-  __syncthreads();
-  qq = kk = 0.0f;
-  for ( uint32_t i = 0; i < blockDim.x / WAVE; i++ ) {
-    qq += q_sums[i];
-    kk += k_sums[i];
-  }
-  const float q_inv = 1.0f / sqrtf( qq / (float)pq.cols + eps );
-  const float k_inv = 1.0f / sqrtf( kk / (float)pk.cols + eps );
-  E* q_dst = q_out + row * s.heads * s.dpad;
-  E* k_dst = reinterpret_cast<E*>( base + wr.offset ) + (uint64_t)( wr.start_pos[ctx] + tok ) * s.row_elems();
-  E* v_dst = k_dst + s.k_elems();
+  auto tables = [&]() __attribute__( ( always_inline ) ) {
 #pragma unroll
-  for ( int g = 0; g < NV; g++ ) {
-    const uint32_t c = ( g * blockDim.x + threadIdx.x ) * 4;
-    if ( c >= cols ) {
+    for ( int g = 0; g < NV; g++ ) {
+      const uint32_t at = read( col[g] );
+      fours( w[g], at < pk.first ? q_norm + at : k_norm + ( at < pv.first ? at - pk.first : 0 ) ); // (v: not used)
+      fours( add[g], bias + at );
+    }
+  };
+  if constexpr ( KEPT ) {
+    tables();
+  }
+  uint32_t turn = 0;
+  for ( uint32_t row = blockIdx.x; row < rows; row += gridDim.x, turn ^= 1 ) {
+    const uint32_t ctx = row / wr.n_tokens, tok = row % wr.n_tokens;
+    uint8_t* const base = static_cast<uint8_t*>( wr.rows[ctx] );
+    const uint32_t pos = wr.start_pos[ctx] + tok;
+    float4 v[NV][V];
+    float qq = 0.0f, kk = 0.0f;
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) { // (nothing that follows from a group's columns is kept from token to token, and the tables as they are, not as the floats that they make)
+      asm volatile( "" : "+v"( col[g] ) );
+    }
+    if constexpr ( KEPT ) {
+#pragma unroll
+      for ( int g = 0; g < NV; g++ ) {
+#pragma unroll
+        for ( int n = 0; n < V; n++ ) {
+          asm volatile( "" : "+v"( w[g][n].x ), "+v"( w[g][n].y ), "+v"( add[g][n].x ), "+v"( add[g][n].y ) );
+        }
+      }
+    } else {
+#pragma unroll
+      for ( int g = 0; g < NV; g++ ) {
+        columns( ahead[g], row, read( col[g] ) );
+      }
+      tables();
+    }
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) {
+#pragma unroll
+      for ( int n = 0; n < V; n++ ) {
+        const float4 x = View::wide( ahead[g][n] ), b = ProductView<E>::wide( add[g][n] );
+        v[g][n] = make_float4( x.x + b.x, x.y + b.y, x.z + b.z, x.w + b.w );
+      }
+    }
+    if constexpr ( KEPT ) {
+      const uint32_t next = min( row + gridDim.x, rows - 1 );
+#pragma unroll
+      for ( int g = 0; g < NV; g++ ) {
+        columns( ahead[g], next, read( col[g] ) );
+      }
+    }
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) {
+      const bool is_q = col[g] < pk.first;
+      float sum = 0.0f;
+#pragma unroll
+      for ( int n = 0; n < V; n++ ) {
+        sum += col[g] < pv.first ? v[g][n].x * v[g][n].x + v[g][n].y * v[g][n].y + v[g][n].z * v[g][n].z + v[g][n].w * v[g][n].w : 0.0f;
+      }
+      qq += is_q ? sum : 0.0f;
+      kk += is_q ? 0.0f : sum;
+    }
+    qq = wave_sum( qq );
+    kk = wave_sum( kk );
+    if ( ( threadIdx.x & 63 ) == 0 ) {
+      q_sums[turn][threadIdx.x >> 6] = qq;
+      k_sums[turn][threadIdx.x >> 6] = kk;
+    }
+    __syncthreads(); // (the sums of the token after next go where these are: everyone is past the barrier between by then)
+    qq = kk = 0.0f;
+    for ( uint32_t i = 0; i < blockDim.x / WAVE; i++ ) {
+      qq += q_sums[turn][i];
+      kk += k_sums[turn][i];
+    }
+    if ( base == nullptr ) {
       continue;
     }
-    const bool is_q = c < pk.first, is_v = c >= pv.first;
-    const float inv = is_q ? q_inv : k_inv;
-    const uint32_t local = c - ( is_q ? 0 : is_v ? pv.first : pk.first );
-    const uint32_t dim = is_v ? pv.dim : pq.dim, pad = is_v ? pv.pad : pq.pad;
-    union
-    {
-      E e[4];
-      uint2 half;
-      uint4 full;
-    } o;
-    o.e[0] = from_f32<E>( is_v ? v[g].x : v[g].x * inv * w[g].x );
-    o.e[1] = from_f32<E>( is_v ? v[g].y : v[g].y * inv * w[g].y );
-    o.e[2] = from_f32<E>( is_v ? v[g].z : v[g].z * inv * w[g].z );
-    o.e[3] = from_f32<E>( is_v ? v[g].w : v[g].w * inv * w[g].w );
-    const uint32_t h = pad != dim ? local / dim : 0, e = local - h * dim;
-    E* at = ( is_q ? q_dst : is_v ? v_dst : k_dst ) + (uint64_t)h * pad + e;
-    if constexpr ( sizeof( E ) == 2 ) {
-      *reinterpret_cast<uint2*>( at ) = o.half;
-    } else {
-      *reinterpret_cast<uint4*>( at ) = o.full;
-    }
-    if ( pad != dim && e + 4 == dim ) {
-      for ( uint32_t z = dim; z < pad; z++ ) {
-        at[z - e] = from_f32<E>( 0.0f );
+    const float q_inv = 1.0f / sqrtf( qq / (float)pq.cols + eps );
+    const float k_inv = 1.0f / sqrtf( kk / (float)pk.cols + eps );
+    E* q_dst = q_out + (uint64_t)row * s.heads * s.dpad;
+    E* k_dst = reinterpret_cast<E*>( base + wr.offset ) + (uint64_t)pos * s.row_elems();
+    E* v_dst = k_dst + s.k_elems();
+#pragma unroll
+    for ( int g = 0; g < NV; g++ ) {
+      const uint32_t c = col[g];
+      if ( c >= cols ) {
+        continue;
+      }
+      const bool is_q = c < pk.first, is_v = c >= pv.first;
+      const float inv = is_q ? q_inv : k_inv;
+      const uint32_t local = c - ( is_q ? 0 : is_v ? pv.first : pk.first );
+      const uint32_t dim = is_v ? pv.dim : pq.dim, pad = is_v ? pv.pad : pq.pad;
+      struct alignas( 4 * V * sizeof( E ) ) Run
+      {
+        E e[4 * V];
+      } o;
+#pragma unroll
+      for ( int n = 0; n < V; n++ ) {
+        const float4 f = ProductView<E>::wide( w[g][n] );
+        o.e[4 * n] = from_f32<E>( is_v ? v[g][n].x : v[g][n].x * inv * f.x );
+        o.e[4 * n + 1] = from_f32<E>( is_v ? v[g][n].y : v[g][n].y * inv * f.y );
+        o.e[4 * n + 2] = from_f32<E>( is_v ? v[g][n].z : v[g][n].z * inv * f.z );
+        o.e[4 * n + 3] = from_f32<E>( is_v ? v[g][n].w : v[g][n].w * inv * f.w );
+      }
+      const uint32_t h = pad != dim ? local / dim : 0, e = local - h * dim;
+      E* at = ( is_q ? q_dst : is_v ? v_dst : k_dst ) + (uint64_t)h * pad + e;
+      *reinterpret_cast<Run*>( at ) = o;
+      if ( pad != dim && e + 4 * V == dim ) {
+        for ( uint32_t z = dim; z < pad; z++ ) {
+          at[z - e] = from_f32<E>( 0.0f );
+        }
       }
     }
   }
@@ -251,7 +329,20 @@ int launch_append( E* q, const View& y, const E* bias, const void* q_norm, const
   if ( s.dim % 4 == 0 && s.vdim % 4 == 0 && y.stride % 4 == 0 && ( tables & 15u ) == 0 && most <= 32768 ) {
     if ( const uint32_t all = ( nq + nk + nv ) / 4; rows >= 1024 && all <= 4096 && bias != nullptr && q_norm != nullptr && k_norm != nullptr ) {
       const uint32_t threads = std::max<uint32_t>( 64, ( ( all + 3 ) / 4 + 63 ) / 64 * 64 );
-      window_append_row_kernel<E, View, 4><<<(unsigned)rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps );
+      // work-groups that run at a time (six waves a SIMD), each as many tokens as the others
+      const uint64_t resident = (uint64_t)cu_count() * std::max( 1u, 1536 / threads ), each = ( rows + resident - 1 ) / resident;
+      const unsigned grid_rows = (unsigned)( ( rows + each - 1 ) / each );
+      const uintptr_t runs = reinterpret_cast<uintptr_t>( y.data ) | reinterpret_cast<uintptr_t>( q );
+      bool wide = false;
+      if constexpr ( std::is_same_v<View, ProductView<__bf16>> ) { // one plane
+        wide = s.dim % 8 == 0 && s.vdim % 8 == 0 && y.stride % 8 == 0 && ( runs & 15u ) == 0;
+        if ( wide ) {
+          window_append_row_kernel<E, View, 2, 2><<<grid_rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps, (uint32_t)rows );
+        }
+      }
+      if ( !wide ) {
+        window_append_row_kernel<E, View, 4, 1><<<grid_rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps, (uint32_t)rows );
+      }
       GH_LAUNCH_CHECK();
       return GH_OK;
     }

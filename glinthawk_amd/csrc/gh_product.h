@@ -5,6 +5,8 @@
 
 #include "gh_common.h"
 
+#include <type_traits>
+
 namespace gh {
 
 bool gemm_few_rows_apart( uint64_t s, uint64_t r, uint64_t few, uint64_t b, gh_dtype dt, const void* x, const void* w );
@@ -147,6 +149,25 @@ struct ProductView
       }
     }
     return sum;
+  }
+  // four neighbouring columns as they lie in memory, where there is one plane: a load that nothing has to wait for before the values are asked for
+  typedef std::conditional_t<sizeof( S ) == 2, uint2, float4> Four;
+  __device__ __forceinline__ Four four( uint64_t row, uint64_t col ) const
+  {
+    if constexpr ( sizeof( S ) == 2 ) {
+      return *reinterpret_cast<const uint2*>( data + row * stride + col );
+    } else {
+      return at4( row, col );
+    }
+  }
+  static __device__ __forceinline__ float4 wide( const Four& f )
+  {
+    if constexpr ( sizeof( S ) == 2 ) {
+      const S* v = reinterpret_cast<const S*>( &f );
+      return make_float4( to_f32( v[0] ), to_f32( v[1] ), to_f32( v[2] ), to_f32( v[3] ) );
+    } else {
+      return f;
+    }
   }
   // eight neighbouring columns; col % 8 == 0, stride % 8 == 0
   __device__ __forceinline__ void at8( float out[8], uint64_t row, uint64_t col ) const

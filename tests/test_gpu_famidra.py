@@ -474,6 +474,48 @@ def test_query_key_norm_and_append(dtype, n_tokens):
         assert (c == 7.0).all(), "rows outside the call were written"
 
 
+# work-groups that take several tokens each, some one less; 16 bytes and 8 at a time, padded heads, more heads than keys have, a row that ends inside a group
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 521), (40, 8, 128, 64, 1111), (60, 20, 52, 36, 1301), (25, 5, 104, 72, 1201)])
+def test_query_key_norm_and_append_of_many_tokens(dtype, heads, kv, d, dv, n_tokens):
+    """Three contexts, the second without one: its tokens are passed over.  Against 64 bits, bound as above."""
+    import torch
+    from glinthawk_amd import ops
+    width, eps = 64, 2e-3
+    g = torch.Generator(device="cuda").manual_seed(heads)
+
+    def draw(*shape):
+        return torch.randn(shape, generator=g, device="cuda").bfloat16().to(torch_dtype(dtype))
+
+    nq, nk, nv = heads * d, kv * d, kv * dv
+    a = ops.window_attn(heads, kv, d, dv, 1.0, 9, 2, 5)
+    x, w, b, qn, kn = draw(3 * n_tokens, width), draw(nq + nk + nv, width) / 8, draw(nq + nk + nv), 1 + draw(nq) / 4, 1 + draw(nk) / 4
+    y = x.double() @ w.double().T + b.double()
+    row = ops.window_row_bytes(a, torch_dtype(dtype)) // (4 if dtype == "f32" else 2)
+    regions = [torch.full((n_tokens + 11, row), 7.0, dtype=torch_dtype(dtype), device="cuda") for _ in range(2)]
+    start = [3, 0, 11]
+    q = ops.matmul_window_append(x, w, a, ops.row_table([regions[0].data_ptr(), 0, regions[1].data_ptr()]), torch.tensor(start, dtype=torch.int32, device="cuda"),
+                                 n_tokens, b, qn, kn, eps)
+
+    def unit(v, weight):
+        return v / torch.sqrt((v * v).mean(-1, keepdim=True) + eps) * weight.double()
+
+    def close(got, want, size, what):
+        got = got.double().reshape(len(want), -1, (size + 7) // 8 * 8)
+        assert got[:, :, size:].abs().sum() == 0, what
+        assert_rows(got[:, :, :size].reshape(len(want), -1).cpu().numpy(), want.cpu().numpy(), 1e-5 if dtype == "f32" else 1e-2, what)
+
+    kp = kv * ((d + 7) // 8 * 8)
+    assert q[n_tokens:2 * n_tokens].abs().sum() == 0
+    for i, region in ((0, regions[0]), (2, regions[1])):
+        at = slice(i * n_tokens, (i + 1) * n_tokens)
+        mine = region[start[i]:start[i] + n_tokens]
+        close(q[at], unit(y[at, :nq], qn), d, "q")
+        close(mine[:, :kp], unit(y[at, nq:nq + nk], kn), d, "k")
+        close(mine[:, kp:], y[at, nq + nk:], dv, "v")
+        assert (region[:start[i]] == 7.0).all() and (region[start[i] + n_tokens:] == 7.0).all(), "rows outside the call were written"
+
+
 MLSTMS = {"small": (3, 12, 20, 9.0), "round": (2, 64, 64, 15.0), "tall": (1, 130, 40, 5.0), "broad": (2, 32, 200, 15.0), "big": (1, 256, 136, 15.0), "huge": (1, 300, 70, 15.0)}
 
 
