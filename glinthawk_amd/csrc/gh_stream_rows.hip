@@ -93,9 +93,44 @@ __device__ __forceinline__ float4 load4_e( const void* p, uint32_t c )
   return ProductView<E>::load4( static_cast<const E*>( p ) + c );
 }
 
-// what a step leaves for the next product: the row, normed where there is a norm
+// Four of a row's weights for each group of a thread, asked for at the kernel's start (EARLY, as they lie in memory, so that nothing waits for them): behind a norm's
+// barrier each table is one more round trip with nothing beside it (8192 rows of 4096: 68 -> 64.5 us, 6.2 TB/s).  Where the registers would cost work-groups in
+// flight, there all the same; and where stores go out before the norm, which the loads would hold up (embeddings of 8192 rows 44.5 us, 48 with early weights).
+template<typename E, int NV, bool EARLY>
+struct StepWeights
+{
+  typedef typename ProductView<E>::Four Four;
+  Four w[EARLY ? NV : 1];
+  const E* p;
+  __device__ __forceinline__ StepWeights( const void* from, const uint32_t ( &col )[NV] )
+    : p( static_cast<const E*>( from ) )
+  {
+    if constexpr ( EARLY ) {
+#pragma unroll
+      for ( int g = 0; g < NV; g++ ) {
+        w[g] = {};
+        if ( p != nullptr ) {
+          w[g] = *reinterpret_cast<const Four*>( p + col[g] );
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ float4 at( int g, uint32_t c ) const
+  {
+    if constexpr ( EARLY ) {
+      return ProductView<E>::wide( w[g] );
+    } else {
+      return load4_e<E>( p, c );
+    }
+  }
+};
 template<typename E, int NV>
-__device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_t ( &col )[NV], const bool ( &live )[NV], uint64_t row, uint32_t width, const StepPtrs& p, float* s_next )
+using NormWeights = StepWeights<E, NV, NV * sizeof( E ) <= 8>;
+
+// what a step leaves for the next product: the row, normed where there is a norm
+template<typename E, int NV, typename Weights>
+__device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_t ( &col )[NV], const bool ( &live )[NV], const Weights& next, uint64_t row, uint32_t width,
+                                          const StepPtrs& p, float* s_next )
 {
   if ( p.out == nullptr ) {
     return;
@@ -114,7 +149,7 @@ __device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_
   for ( int g = 0; g < NV; g++ ) {
     float4 w = make_float4( 1.0f, 1.0f, 1.0f, 1.0f );
     if ( p.next_norm != nullptr ) {
-      w = load4_e<E>( p.next_norm, col[g] );
+      w = next.at( g, col[g] );
       w = make_float4( p.norm_base + w.x, p.norm_base + w.y, p.norm_base + w.z, p.norm_base + w.w );
     }
     union
@@ -154,7 +189,10 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
     col[g] = live[g] ? c : 0;
     old[g] = *reinterpret_cast<const float4*>( xr + col[g] );
   }
+  const NormWeights<E, NV> next( p.next_norm, col );
   if constexpr ( PRODUCT ) {
+    const NormWeights<E, NV> post( p.post_norm, col );
+    const StepWeights<E, NV, NV <= 2> add( p.add, col );
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) {
       v[g] = y.at4( row, col[g] );
@@ -175,7 +213,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
       const float inv = 1.0f / sqrtf( row_sum( ss, s_post ) / (float)width + p.eps );
 #pragma unroll
       for ( int g = 0; g < NV; g++ ) {
-        const float4 w = load4_e<E>( p.post_norm, col[g] );
+        const float4 w = post.at( g, col[g] );
         v[g] = make_float4( v[g].x * inv * ( p.norm_base + w.x ), v[g].y * inv * ( p.norm_base + w.y ), v[g].z * inv * ( p.norm_base + w.z ),
                             v[g].w * inv * ( p.norm_base + w.w ) );
       }
@@ -186,7 +224,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
         v[g] = make_float4( old[g].x + v[g].x, old[g].y + v[g].y, old[g].z + v[g].z, old[g].w + v[g].w );
       }
       if ( p.add != nullptr ) {
-        const float4 a = load4_e<E>( p.add, col[g] );
+        const float4 a = add.at( g, col[g] );
         v[g] = make_float4( v[g].x + a.x, v[g].y + a.y, v[g].z + a.z, v[g].w + a.w );
       }
       if ( live[g] ) {
@@ -199,7 +237,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
       v[g] = old[g];
     }
   }
-  step_out<E, NV>( v, col, live, row, width, p, s_next );
+  step_out<E, NV>( v, col, live, next, row, width, p, s_next );
 }
 
 // any width: the row goes through memory between the passes (each thread re-reads only what it wrote)
@@ -301,7 +339,7 @@ __global__ __launch_bounds__( 1024 ) void embed_step_kernel( float* __restrict__
       }
     }
   }
-  step_out<E, NV>( v, col, live, row, width, p, s_next );
+  step_out<E, NV>( v, col, live, StepWeights<E, NV, false>( p.next_norm, col ), row, width, p, s_next ); // (the stores above go out first)
 }
 
 // Threads to a row of `groups` groups of four columns: many rows, fewer threads with more of the row each; few rows, the row over as many threads as it has groups.
