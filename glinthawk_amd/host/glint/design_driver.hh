@@ -291,7 +291,7 @@ public:
   float* logits() const { return logits_.get(); }
   void copy_logits( float* host, const uint64_t rows )
   {
-    logit_ops_.copy( host, logits_.get(), rows * sizes_.vocab * sizeof( float ), CopyType::DeviceToHost );
+    logit_ops_.rows_out( host, logits_.get(), rows * sizes_.vocab * sizeof( float ) ); // (page-locked memory: written by a kernel, no copy engine to start)
   }
 
 protected:

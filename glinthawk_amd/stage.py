@@ -315,6 +315,42 @@ class Stage:
         return out, nxt
 
 
+class _PinnedResults:
+    """Up to `count` page-locked buffers that result arrays of a stage are laid over; a buffer comes back when its array and every view of it are gone, and
+    all of them are released with the stage and the last array.  A copy from the device into pageable memory goes through a staging buffer and the
+    host's own copy (32 x 4096 logits 40 us, 20 into such a buffer, which a kernel writes)."""
+
+    class _Loan:
+        def __init__(self, pool, ptr, shape):
+            self.pool, self.ptr = pool, ptr
+            self.__array_interface__ = dict(shape=shape, typestr="<f4", data=(ptr, False), strides=None, version=3)
+
+        def __del__(self):
+            self.pool.free.append(self.ptr)
+
+    def __init__(self, n_bytes: int, count: int):
+        from . import _lib
+        self.free, self.n_bytes, self._release = [], n_bytes, _lib.lib().gh_host_free
+        for _ in range(count):
+            ptr = C.c_void_p()
+            if _lib.lib().gh_host_malloc(C.byref(ptr), n_bytes) == 0 and ptr.value:
+                self.free.append(ptr.value)
+
+    def __del__(self):
+        for ptr in self.free:
+            self._release(C.c_void_p(ptr))
+
+    def take(self, rows: int, columns: int) -> Optional[np.ndarray]:
+        """(rows, columns) fp32, or None: too large, or every buffer is in use."""
+        if 4 * rows * columns > self.n_bytes:
+            return None
+        try:
+            ptr = self.free.pop()     # (one thread at a time by the interpreter's lock)
+        except IndexError:
+            return None
+        return np.asarray(self._Loan(self, ptr, (rows, columns)))
+
+
 class DesignStage(Stage):
     """A whole model of a run-time sized design, opened from its model directory (config.json names the architecture,
     model.safetensors holds the weights; random_weights: only config.json is read).  The batched state, the context slots and
@@ -330,6 +366,9 @@ class DesignStage(Stage):
         if not self._h:
             raise GlintError(host_lib().glint_last_error().decode(errors="replace"))
         self.vocab_size, self.max_positions, self.layer_runs = (int(host_lib().glint_stage_size(self._h, k)) for k in range(3))
+        # the logits of a step and those of the one before, where they are not so many that page-locking them would tell
+        step = 4 * concurrency * self.vocab_size
+        self._results = _PinnedResults(step, 2 if step <= 32 << 20 else 0)
 
     def prefill_logits(self, context_ids, start_pos, token_ids, want=(), want_next_tokens: bool = False, residual_width: int = 0):
         """token_ids (batch, n_tokens).  Returns (logits (len(want), vocab), next tokens or None, residual stream (layer runs, rows,
@@ -363,7 +402,9 @@ class DesignStage(Stage):
 
     def logits(self, rows: int) -> np.ndarray:
         """Logits of the first `rows` rows of the last forward()."""
-        out = np.empty((rows, self.vocab_size), dtype=np.float32)
+        out = self._results.take(rows, self.vocab_size) if rows > 0 else None
+        if out is None:
+            out = np.empty((rows, self.vocab_size), dtype=np.float32)
         if host_lib().glint_stage_logits(self._h, out.ctypes.data, rows) != 0:
             raise GlintError("no logits of that many rows")
         return out

@@ -458,6 +458,36 @@ def test_portions_and_decoding(models, name, dtype, cuts):
     st.close()
 
 
+def test_logits_of_earlier_steps_stay(models):
+    """Every array of a step's logits holds its own: more of them at a time than the stage has page-locked memory for, views that outlive their array, arrays that
+    outlive the stage; and memory that came back is used again."""
+    path, _, _, seqs, want, _ = models(NAMES[0])
+    st = open_stage(path, "f32")
+    steps, copies, views = [], [], []
+    for i in range(6):
+        steps.append(decode_step(st, [1, 2], [int(seqs[0][i])] * 2, [i, i]))
+        assert steps[i].shape == (2, st.vocab_size) and steps[i].dtype == np.float32 and steps[i].flags.writeable and steps[i].flags.c_contiguous
+        copies.append(steps[i].copy())
+        views.append(steps[i][1:, ::2])
+    places = {a.ctypes.data for a in steps}
+    assert len(places) == 6
+    del steps[:4]
+    for i in range(6, 9):     # the views of the first ones are still there
+        steps.append(decode_step(st, [1, 2], [int(seqs[0][i])] * 2, [i, i]))
+        copies.append(steps[-1].copy())
+    assert all(np.array_equal(v, c[1:, ::2]) for v, c in zip(views, copies))
+    first = views[0].__array_interface__["data"][0] - 4 * st.vocab_size
+    del views[0]
+    again = decode_step(st, [1, 2], [int(seqs[0][9])] * 2, [9, 9])
+    assert again.ctypes.data == first
+    assert st.logits(1).shape == (1, st.vocab_size) and np.array_equal(st.logits(1), again[:1])
+    kept = again.copy()
+    st.close()
+    del st
+    assert np.array_equal(again, kept) and all(np.array_equal(a, c) for a, c in zip(steps, copies[4:]))
+    assert_logits(np.concatenate([c[:1] for c in copies] + [kept[:1]]), want[0][:10], "f32")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_far_token(tmp_path, dtype):
     """A token that reads one other token, hundreds of positions away: in a prompt, decoded, and behind portions that end next to either."""
