@@ -278,19 +278,22 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
 //             the keys) meets q and v as two terms, 16 bits.  n and its products are fp32.
 // loads       k of a chunk is requested at its head and needed behind Q S and P V; q and v of the next one are requested behind those and needed
 //             at the next one's head.
-// operands    an accumulator tile of v_mfma_f32_16x16x32_bf16 (lane = column, registers = rows 4 (lane / 16) + v) is, with the tile below it
-//             and as they lie, an operand of the next product over those 32 rows when the other operand takes its rows in the same order:
+// order       of the sums: terms of 16 keys or dims at a time, the lower term first, as v_mfma_f32_32x32x16_bf16 takes them (eight of a lane, lanes 0 .. 31 in
+//             front).  v_mfma_f32_16x16x32_bf16 is two of those in turn, bit for bit, so its lanes 32 .. 63 hold the next term of the same 16, or the first of the
+//             next, instead of 16 others: permlane32_swap brings a lane's terms there.  Models depend on the last bits (behind a thousand tokens and two
+//             layers they are more than a tenth of the logits of one token in 5000, in either order as far off 64 bits), so the order is kept whatever the tile.
+// operands    an accumulator tile of v_mfma_f32_16x16x32_bf16 (lane = column, registers = rows 4 (lane / 16) + v) is, with the tile of the next quads,
+//             an operand of the next product over those rows when the other operand takes its rows in the same order:
 //               scores^T = K Q^T        lane = query, registers = keys   -> left operand of   P V     (V out of LDS transposed)
 //               S                       lane = column of v, registers = dim -> right operand of Q S   (Q out of LDS in pieces of 4)
 //             S += K^T (w V): both operands out of LDS with transposing reads (ds_read_b64_tr_b16).
-// LDS         64 rows each of q, k and v, 16-byte chunks XORed with bits of the row so that row reads (16 rows) and transposing reads (8 rows of a
-//             half-wave, two chunks each) both touch every bank once; straight from memory (buffer_load ... lds; rows past the sequence
-//             and padding read as zero).
+// LDS         64 rows each of q, k and v, 16-byte chunks XORed with bits of the row so that row reads (16 rows) and transposing reads (8 rows, two chunks
+//             each) both touch every bank once; straight from memory (buffer_load ... lds; rows past the sequence and padding read as zero).
 // bound       8 contexts of 1024 tokens, 8 heads of 256 x 512: 310 us in one kernel, whose waves, one a SIMD, made gates, weights and n once for every 32
-//             columns; now scan 9, scores 16 and states 118 us (the call 398 -> 257; 1 of 2048 tokens 526 -> 177, 32 of 24 tokens 118 -> 78).  States: the
-//             matrix cores are busy for a third of it, as are the vector units; what is left is waits of four waves for each other, twice a
-//             chunk.  On the way there: requests at the chunk's head instead of where the scheduler put them and stores that the next chunk
-//             doesn't wait for 134 -> 122; Q in reads that are not joined by two 127 (LDS 2.4 x as long active joined).
+//             columns; now scan 11, scores 15 and states 164 us (the call 391 -> 293; 1 of 2048 tokens 528 -> 230, 32 of 24 tokens 117 -> 83).  States: waits of
+//             four waves for each other, twice a chunk, and for LDS, 330 reads a chunk and wave, with two waves a SIMD; the matrix cores are busy for a quarter of it.
+//             With 32 keys or dims of one term in a product, whose bits differ: 200 reads fewer and 129 us.  A third operand of k out of LDS instead of one
+//             selected from two: 235 us at 1 x 2048 tokens instead of 230, 8 x 1024 even.
 constexpr int CHUNK = 64;
 typedef __attribute__( ( address_space( 3 ) ) ) void* lds_ptr;
 typedef __attribute__( ( address_space( 3 ) ) ) char lds_char;
@@ -298,11 +301,17 @@ typedef short v4s __attribute__( ( ext_vector_type( 4 ) ) );
 typedef __attribute__( ( address_space( 3 ) ) ) v4s* lds_v4s;
 typedef Mfma<__bf16>::x8 bf16x8;
 
-// slot of 16-byte chunk `chunk` of row `row` in a tile of `BYTES` a row: 128, 256 or 512
-template<uint32_t BYTES>
+// slot of 16-byte chunk `chunk` of row `row` in a tile of `BYTES` a row, 128, 256 or 512: eight rows in a row and those `FAR` further on apart
+template<uint32_t BYTES, uint32_t FAR = 8>
 __device__ __forceinline__ uint32_t swizzle( uint32_t row, uint32_t chunk )
 {
-  return BYTES == 128 ? chunk ^ ( ( ( ( row >> 1 ) & 3 ) << 1 ) | ( ( row >> 3 ) & 1 ) ) : chunk ^ ( ( ( row & 7 ) << 1 ) | ( ( row >> 3 ) & 1 ) );
+  return BYTES == 128 ? chunk ^ ( ( ( ( row >> 1 ) & 3 ) << 1 ) | ( ( row / FAR ) & 1 ) ) : chunk ^ ( ( ( row & 7 ) << 1 ) | ( ( row / FAR ) & 1 ) );
+}
+// eight rows in a row and a chunk and the next but one apart
+template<uint32_t BYTES>
+__device__ __forceinline__ uint32_t swizzle_pair( uint32_t row, uint32_t chunk )
+{
+  return BYTES == 128 ? chunk ^ ( ( ( row >> 1 ) & 1 ) | ( row & 4 ) ) : chunk ^ ( ( row & 1 ) | ( ( row & 6 ) << 1 ) );
 }
 
 // Eight fp32 values as N bf16 terms each, 8 bits of mantissa a term; taken two at a time, as the conversion instruction does.
@@ -346,7 +355,7 @@ struct MlstmChunks
   float* token;   // planes of (pairs, chunks x 64): see below
   float* decay;   // (pairs, chunks): factor of the state over a chunk
   float* n;       // (pairs, chunks, dim): what a chunk adds to n
-  uint4* weights; // (pairs, chunks, WEIGHT_TILES, 2 terms, 64 lanes): P as the left operands of P V
+  uint4* weights; // (pairs, chunks, WEIGHT_TILES, 64 lanes): P as the left operands of P V
   uint32_t chunks;
   uint64_t plane;
   enum
@@ -362,8 +371,21 @@ struct MlstmChunks
   };
   __device__ __forceinline__ float* tokens( int which, uint32_t pair, uint32_t chunk ) const { return token + which * plane + ( (uint64_t)pair * chunks + chunk ) * CHUNK; }
 };
-constexpr uint32_t WEIGHT_TILES = 6; // 16 queries x 32 keys; of queries 0 .. 31 the first 32 keys only
-__device__ __forceinline__ constexpr uint32_t weight_tile( uint32_t queries, uint32_t keys ) { return queries < 2 ? queries : 2 * queries - 2 + keys; }
+constexpr uint32_t WEIGHT_TILES = 10; // 16 queries x 16 keys, both terms, up to the queries' own
+__device__ __forceinline__ constexpr uint32_t weight_tile( uint32_t queries, uint32_t keys ) { return queries * ( queries + 1 ) / 2 + keys; }
+
+// Lanes 0 .. 31 of both operands in the first, lanes 32 .. 63 of both in the second: [a | A], [b | B] -> [a | b], [A | B]
+__device__ __forceinline__ void swap_halves( bf16x8& first, bf16x8& second )
+{
+  typedef uint32_t u32x4_t __attribute__( ( ext_vector_type( 4 ) ) );
+  u32x4_t a = __builtin_bit_cast( u32x4_t, first ), b = __builtin_bit_cast( u32x4_t, second );
+#pragma unroll
+  for ( int k = 0; k < 4; k++ ) {
+    const auto ab = __builtin_amdgcn_permlane32_swap( a[k], b[k], false, false );
+    a[k] = ab[0], b[k] = ab[1];
+  }
+  first = __builtin_bit_cast( bf16x8, a ), second = __builtin_bit_cast( bf16x8, b );
+}
 
 // The tokens of a chunk, lane <-> token: the sums b of the log forget gates, c, and the largest c so far (without what lies in front of the chunk).
 struct ChunkScan
@@ -455,9 +477,9 @@ template<int KS, bool ALONE>
 __global__ __launch_bounds__( 256 ) void mlstm_scores_kernel( float* __restrict__ nm_out, MlstmIn<__bf16, ProductView<__bf16>> in, MlstmGates<__bf16> raw, MlstmState st, MlstmShape s,
                                                               MlstmChunks ch, uint32_t n_pairs )
 {
-  constexpr uint32_t PIECES = 4 * KS, SETS = 256 / PIECES; // 8 dims each; threads on the same dims
+  constexpr uint32_t PIECES = 4 * KS; // 8 dims each
   constexpr uint32_t RB = KS * 64;                         // bytes of a row in LDS
-  __shared__ uint4 s_k[CHUNK * RB / 16]; // then the sums for n of the sets
+  __shared__ uint4 s_k[CHUNK * RB / 16]; // then the sums for n of eight keys each
   __shared__ __attribute__( ( aligned( 16 ) ) ) float s_c[CHUNK], s_w[CHUNK], s_M[CHUNK];
   // on the XCD that walks the chunks
   const uint32_t pair = ( blockIdx.x >> 3 ) / ch.chunks * 8 + ( blockIdx.x & 7 ), chunk = ( blockIdx.x >> 3 ) % ch.chunks;
@@ -486,10 +508,10 @@ __global__ __launch_bounds__( 256 ) void mlstm_scores_kernel( float* __restrict_
   constexpr uint32_t ROWS = 1024 / RB; // rows of one instruction of one wave
 #pragma unroll
   for ( uint32_t i = 0; i < CHUNK / ( 4 * ROWS ); i++ ) {
-    const uint32_t row0 = ( 4 * i + wave ) * ROWS, row = row0 + lane / PIECES, piece = swizzle<RB>( row, lane % PIECES );
+    const uint32_t row0 = ( 4 * i + wave ) * ROWS, row = row0 + lane / PIECES, piece = swizzle<RB, 32>( row, lane % PIECES );
     __builtin_amdgcn_raw_ptr_buffer_load_lds( k_rsrc, (lds_ptr)( s_k + row0 * PIECES ), 16, piece * 8 < s.dim ? row * ld_bytes + piece * 16 : PAST_THE_END, 0, 0, 0 );
   }
-  auto k_at = [&]( uint32_t row, uint32_t piece ) __attribute__( ( always_inline ) ) { return __builtin_bit_cast( bf16x8, s_k[row * PIECES + swizzle<RB>( row, piece )] ); };
+  auto k_at = [&]( uint32_t row, uint32_t piece ) __attribute__( ( always_inline ) ) { return __builtin_bit_cast( bf16x8, s_k[row * PIECES + swizzle<RB, 32>( row, piece )] ); };
   if ( wave == 0 ) {
     float c_rel, w, M_rel;
     if constexpr ( ALONE ) {
@@ -506,75 +528,95 @@ __global__ __launch_bounds__( 256 ) void mlstm_scores_kernel( float* __restrict_
   __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): this wave's part of k has landed
   __syncthreads();
   const float Mq = s_M[16 * wave + r];
-  float p[4][4], den = 0.0f;
+  // lane group g: keys 32 (g / 2) + 8 kt + 4 (g % 2) + e
+  const uint32_t key_l = 32 * ( g >> 1 ) + 4 * ( g & 1 ), key_r = 32 * ( r >> 3 ) + 4 * ( ( r >> 2 ) & 1 ) + ( r & 3 ), query = 16 * wave + r;
+  float dot[4][4], weight[4][4], p[4][4];
 #pragma unroll
   for ( uint32_t kt = 0; kt < 4; kt++ ) {
 #pragma unroll
     for ( int e = 0; e < 4; e++ ) {
-      p[kt][e] = 0.0f;
+      dot[kt][e] = weight[kt][e] = p[kt][e] = 0.0f;
     }
-    if ( kt <= wave ) {
+    if ( wave > 0 || kt < 2 ) { // (the first 16 queries see none of the others' keys)
       mfma_f32x4 sc = { 0, 0, 0, 0 };
 #pragma unroll
       for ( int k = 0; k < KS; k++ ) {
-        sc = Mfma<__bf16>::k32( k_at( 16 * kt + r, 4 * k + g ), qb[k], sc );
+        sc = Mfma<__bf16>::k32( k_at( key_r + 8 * kt, 4 * k + g ), qb[k], sc );
       }
-      const float4 ck = *reinterpret_cast<const float4*>( &s_c[16 * kt + 4 * g] );
+      const float4 ck = *reinterpret_cast<const float4*>( &s_c[key_l + 8 * kt] );
       const float cks[4] = { ck.x, ck.y, ck.z, ck.w };
 #pragma unroll
       for ( int e = 0; e < 4; e++ ) {
-        const bool seen = kt < wave || 4 * g + e <= r;
-        p[kt][e] = seen ? sc[e] * s.q_scale * __expf( cks[e] - Mq ) : 0.0f;
-        den += p[kt][e];
+        dot[kt][e] = sc[e] * s.q_scale, weight[kt][e] = __expf( cks[e] - Mq );
+        p[kt][e] = key_l + 8 * kt + e <= query ? dot[kt][e] * weight[kt][e] : 0.0f;
       }
     }
+  }
+  // their sum, the quads of keys of an even number and those of an odd one each in their order: lanes 32 further on go on from where these end
+  float den = 0.0f;
+#pragma unroll
+  for ( int k = 0; k < 16; k++ ) { // (the last 32 queries see all of the first 32 keys)
+    den = wave >= 2 ? __builtin_fmaf( dot[k / 4][k % 4], weight[k / 4][k % 4], den ) : den + p[k / 4][k % 4];
+  }
+  den = __shfl_xor( den, 32 );
+#pragma unroll
+  for ( int k = 0; k < 16; k++ ) {
+    den += p[k / 4][k % 4];
   }
   den += __shfl_xor( den, 16 );
-  den += __shfl_xor( den, 32 );
-  if ( g == 0 ) {
-    ch.tokens( MlstmChunks::DEN, pair, chunk )[16 * wave + r] = den;
+  if ( g == 2 ) {
+    ch.tokens( MlstmChunks::DEN, pair, chunk )[query] = den;
   }
-  uint4* dst = ch.weights + ( (uint64_t)pair * ch.chunks + chunk ) * ( WEIGHT_TILES * 128 ) + lane;
+  // as operands: the lower term of 16 keys in lanes 0 .. 31, the upper one of the same keys in the others
+  uint4* dst = ch.weights + ( (uint64_t)pair * ch.chunks + chunk ) * ( WEIGHT_TILES * 64 ) + lane;
 #pragma unroll
   for ( uint32_t j = 0; j < 2; j++ ) {
-    if ( 2 * j <= wave ) {
-      Split<2> f;
+    Split<2> f;
 #pragma unroll
-      for ( int k = 0; k < 4; k++ ) {
-        f.set( k, p[2 * j + ( k >> 1 )][2 * ( k & 1 )], p[2 * j + ( k >> 1 )][2 * ( k & 1 ) + 1] );
-      }
+    for ( int k = 0; k < 4; k++ ) {
+      f.set( k, p[2 * j + ( k >> 1 )][2 * ( k & 1 )], p[2 * j + ( k >> 1 )][2 * ( k & 1 ) + 1] );
+    }
+    swap_halves( f.t[1].x, f.t[0].x );
 #pragma unroll
-      for ( int n = 0; n < 2; n++ ) {
-        dst[( weight_tile( wave, j ) * 2 + n ) * 64] = __builtin_bit_cast( uint4, f.t[n].x );
+    for ( uint32_t n = 0; n < 2; n++ ) { // keys 32 n + 16 j ..
+      if ( 2 * n + j <= wave ) {
+        dst[weight_tile( wave, 2 * n + j ) * 64] = __builtin_bit_cast( uint4, f.t[1 - n].x );
       }
     }
   }
-  // what the chunk adds to n
+  // what the chunk adds to n: eight keys and eight dims a thread
   const uint32_t piece = threadIdx.x % PIECES, set = threadIdx.x / PIECES;
-  float sum[8] = {};
+  float sum[8];
+  if ( set < 8 ) { // of the quads 4 (set / 2) + set % 2 and the next but one
+    const uint32_t key0 = 16 * ( set >> 1 ) + 4 * ( set & 1 );
+    bf16x8 k[8];
 #pragma unroll
-  for ( uint32_t i = 0; i < CHUNK / SETS; i++ ) {
-    const float w = s_w[set + SETS * i];
-    const bf16x8 k = k_at( set + SETS * i, piece );
+    for ( int i = 0; i < 8; i++ ) {
+      k[i] = k_at( key0 + i + 4 * ( i / 4 ), piece );
+    }
+    const float4 w0 = *reinterpret_cast<const float4*>( &s_w[key0] ), w1 = *reinterpret_cast<const float4*>( &s_w[key0 + 8] );
 #pragma unroll
     for ( int e = 0; e < 8; e++ ) {
-      sum[e] += (float)k[e] * w;
+      sum[e] = (float)k[0][e] * w0.x + (float)k[1][e] * w0.y + (float)k[2][e] * w0.z + (float)k[3][e] * w0.w + (float)k[4][e] * w1.x + (float)k[5][e] * w1.y + (float)k[6][e] * w1.z
+               + (float)k[7][e] * w1.w;
     }
   }
   float* s_n = reinterpret_cast<float*>( s_k );
   __syncthreads(); // everyone has read k
+  if ( set < 8 ) {
 #pragma unroll
-  for ( int e = 0; e < 8; e += 4 ) {
-    *reinterpret_cast<float4*>( s_n + set * ( 8 * PIECES ) + piece * 8 + e ) = make_float4( sum[e], sum[e + 1], sum[e + 2], sum[e + 3] );
+    for ( int e = 0; e < 8; e += 4 ) {
+      *reinterpret_cast<float4*>( s_n + set * ( 8 * PIECES ) + piece * 8 + e ) = make_float4( sum[e], sum[e + 1], sum[e + 2], sum[e + 3] );
+    }
   }
   __syncthreads();
   if ( threadIdx.x < s.dim ) {
-    float n = 0.0f;
+    float n[2] = { 0.0f, 0.0f };
 #pragma unroll
-    for ( uint32_t k = 0; k < SETS; k++ ) {
-      n += s_n[k * ( 8 * PIECES ) + threadIdx.x];
+    for ( uint32_t k = 0; k < 8; k++ ) {
+      n[k & 1] += s_n[k * ( 8 * PIECES ) + threadIdx.x];
     }
-    ch.n[( (uint64_t)pair * ch.chunks + chunk ) * s.dim + threadIdx.x] = n;
+    ch.n[( (uint64_t)pair * ch.chunks + chunk ) * s.dim + threadIdx.x] = n[0] + n[1];
   }
 }
 
@@ -602,7 +644,7 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
   float* S_mem = reinterpret_cast<float*>( base + st.offset );
   const bool fresh = st.start_pos[ctx] == 0;
   float n = !fresh && threadIdx.x < s.dim ? S_mem[s.n_off() + (uint64_t)h * s.dim + threadIdx.x] : 0.0f; // thread <-> element
-  const float* n_chunk = ch.n + (uint64_t)pair * ch.chunks * s.dim + min( threadIdx.x, s.dim - 1 );
+  const float* n_chunk = ch.n + (uint64_t)pair * ch.chunks * s.dim + threadIdx.x;
   S_mem += (uint64_t)h * s.dim * s.vpad;
   const uint32_t wave = __builtin_amdgcn_readfirstlane( threadIdx.x >> 6 );
   const uint32_t lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -612,69 +654,77 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
   const uint64_t S_at = reinterpret_cast<uint64_t>( S_mem ); // (said to be uniform: else every access below becomes a loop over the lanes' addresses)
   S_mem = reinterpret_cast<float*>( (uint64_t)__builtin_amdgcn_readfirstlane( (uint32_t)( S_at >> 32 ) ) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane( (uint32_t)S_at ) );
   const __amdgpu_buffer_rsrc_t S_rsrc = __builtin_amdgcn_make_buffer_rsrc( S_mem, 0, (int)( s.dim * s.vpad * 4 ), 0x00020000 );
-  const uint32_t S_off = col < s.vpad ? ( 4 * g * s.vpad + col ) * 4 : PAST_THE_END;
-  mfma_f32x4 S[2 * KS]; // rows 16 d + 4 g + v
+  // tile d: rows 32 (d / 2) + 8 (d % 2) + 16 (g / 2) + 4 (g % 2) + v, so that a lane holds both quads of eight rows apart, lanes 32 further on those of 16 rows further on
+  const uint32_t S_off = col < s.vpad ? ( ( 16 * ( g >> 1 ) + 4 * ( g & 1 ) ) * s.vpad + col ) * 4 : PAST_THE_END;
+  mfma_f32x4 S[2 * KS];
 #pragma unroll
   for ( int d = 0; d < 2 * KS; d++ ) {
 #pragma unroll
     for ( int v = 0; v < 4; v++ ) {
-      S[d][v] = __builtin_bit_cast( float, __builtin_amdgcn_raw_buffer_load_b32( S_rsrc, fresh ? PAST_THE_END : S_off, ( 16 * d + v ) * s.vpad * 4, 0 ) );
+      S[d][v] = __builtin_bit_cast( float, __builtin_amdgcn_raw_buffer_load_b32( S_rsrc, fresh ? PAST_THE_END : S_off, ( 32 * ( d / 2 ) + 8 * ( d % 2 ) + v ) * s.vpad * 4, 0 ) );
     }
   }
   const uint64_t row_first = (uint64_t)ctx * st.n_tokens;
   const uint32_t ld_bytes = (uint32_t)( in.main.stride * 2 );
 
   // rows [0, rows) x `chunks` 16-byte chunks of the product at `p`, LDS rows of BYTES; the rest reads as zero
-  auto fetch = [&]( uint4* tile, const __bf16* p, uint32_t rows, uint32_t chunks, auto row_bytes_tag ) __attribute__( ( always_inline ) ) {
+  auto fetch = [&]( uint4* tile, const __bf16* p, uint32_t rows, uint32_t chunks, auto row_bytes_tag, auto slot ) __attribute__( ( always_inline ) ) {
     constexpr uint32_t BYTES = decltype( row_bytes_tag )::value;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc( const_cast<__bf16*>( p ), 0, (int)( ( rows - 1 ) * ld_bytes + chunks * 16 ), 0x00020000 );
     constexpr uint32_t ROWS = 1024 / BYTES; // rows of one instruction of one wave
+    constexpr uint32_t FORMS = BYTES == 512 ? 2 : 1; // 16 rows on a lane's chunk is the same again, so those are an offset of the wave's
 #pragma unroll
-    for ( uint32_t i = 0; i < CHUNK / ( 4 * ROWS ); i++ ) {
-      const uint32_t row0 = ( 4 * i + wave ) * ROWS;
-      const uint32_t row = row0 + lane / ( BYTES / 16 );
-      const uint32_t chunk = swizzle<BYTES>( row, lane % ( BYTES / 16 ) ); // the swizzle is its own inverse
+    for ( uint32_t form = 0; form < FORMS; form++ ) {
+      const uint32_t row = ( 4 * form + wave ) * ROWS + lane / ( BYTES / 16 );
+      const uint32_t chunk = slot( row, lane % ( BYTES / 16 ) ); // the swizzle is its own inverse
       const uint32_t off = chunk < chunks ? row * ld_bytes + chunk * 16 : PAST_THE_END;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + row0 * ( BYTES / 16 ) ), 16, off, 0, 0, 0 );
+#pragma unroll
+      for ( uint32_t i = 0; i < CHUNK / ( 4 * ROWS * FORMS ); i++ ) {
+        const uint32_t on = 4 * ROWS * FORMS * i; // rows
+        __builtin_amdgcn_raw_ptr_buffer_load_lds( rsrc, (lds_ptr)( tile + ( ( 4 * form + wave ) * ROWS + on ) * ( BYTES / 16 ) ), 16, off, on * ld_bytes, 0, 0 );
+      }
     }
   };
   auto fetch_qv = [&]( uint32_t t0 ) __attribute__( ( always_inline ) ) {
     const uint32_t rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
     const __bf16* first = in.main.data + ( row_first + t0 ) * in.main.stride;
-    fetch( s_q, first + in.col.q + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {} );
-    fetch( s_v, first + in.col.v + h * s.vdim + slice * 64, rows, min( 8u, ( s.vdim - slice * 64 ) / 8 ), std::integral_constant<uint32_t, 128> {} );
+    fetch( s_q, first + in.col.q + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {}, swizzle<RB> );
+    fetch( s_v, first + in.col.v + h * s.vdim + slice * 64, rows, min( 8u, ( s.vdim - slice * 64 ) / 8 ), std::integral_constant<uint32_t, 128> {}, swizzle<128> );
   };
 
-  // 32 rows (keys) x 16 columns from 16-byte chunk `c0` on, transposed: a lane gets its column's rows 4 g + e and 16 + 4 g + e.  Lane 4 e + q of a
-  // 16-lane group points at row e of its four, columns 4 q .. 4 q + 3.
-  const uint32_t tr_row = 4 * g + ( r >> 2 ), tr_q = r & 3;
-  auto transposed = [&]( const uint4* tile, uint32_t row0, uint32_t c0, auto row_bytes_tag ) __attribute__( ( always_inline ) ) {
-    constexpr uint32_t BYTES = decltype( row_bytes_tag )::value;
+  // 16 columns of keys, transposed: a lane gets its column's rows 4 (g % 2) + e and 8 + 4 (g % 2) + e.  Lane 4 e + q of a 16-lane group points at row e of
+  // its four, columns 4 q .. 4 q + 3: of the 16 of this wave (v), or of the rows of a tile of S (k).
+  const uint32_t tr_row = 4 * ( g & 1 ) + ( r >> 2 ), tr_q = r & 3;
+  const uint32_t upper = 16 * ( g >> 1 ); // rows further on for lanes 32 .. 63, where an operand is of 32 keys
+  auto transposed = [&]( const uint4* tile, uint32_t first, uint32_t second ) __attribute__( ( always_inline ) ) {
     union
     {
       v4s half[2];
       bf16x8 x;
     } u;
-#pragma unroll
-    for ( int hf = 0; hf < 2; hf++ ) {
-      const uint32_t row = row0 + 16 * hf + tr_row;
-      u.half[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)tile + row * BYTES + swizzle<BYTES>( tr_row, c0 + ( tr_q >> 1 ) ) * 16 + ( tr_q & 1 ) * 8 ) );
-    }
+    u.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)tile + first ) );
+    u.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16( (lds_v4s)( (lds_char*)tile + second ) );
     return u.x;
   };
-
-  // Of the four tiles of queries, apart from each other: two reads of 8 bytes at a constant distance would become one instruction whose two halves meet in the
-  // same banks, and whose results have to be moved into their operands' registers.
-  uint32_t q_row[4];
-#pragma unroll
-  for ( int i = 0; i < 4; i++ ) {
-    q_row[i] = ( 16 * i + r ) * RB + ( g & 1 ) * 8;
-    asm( "" : "+v"( q_row[i] ) );
-  }
+  // Byte addresses: a part of the lane, its low bits XORed with a constant, and a constant.  Computed where they are used: kept in registers over the loop there
+  // are too many of them.
+  auto opaque = []( uint32_t v ) __attribute__( ( always_inline ) ) {
+    asm volatile( "" : "+v"( v ) );
+    return v;
+  };
+  const uint32_t v_lane = tr_row * 128 + swizzle<128>( tr_row, 2 * wave + ( tr_q >> 1 ) ) * 16 + ( tr_q & 1 ) * 8;
+  auto v_at = [&]( uint32_t lane_part ) __attribute__( ( always_inline ) ) { return transposed( s_v, lane_part, ( lane_part ^ 16 ) + 8 * 128 ); }; // (eight rows on: the swizzle's low bit)
+  const uint32_t k_lane = tr_row * RB + swizzle_pair<RB>( tr_row, 2 * ( tr_q >> 1 ) ) * 16 + ( tr_q & 1 ) * 8;
+  // a query's quads g % 2 of 16 dims.  The four tiles of queries apart from each other: two reads of 8 bytes at a constant distance would become one instruction
+  // whose two halves meet in the same banks, and whose results have to be moved into their operands' registers.
+  const uint32_t q_lane = r * RB + swizzle<RB>( r, 0 ) * 16 + ( g & 1 ) * 8;
+  constexpr uint32_t PERIOD = RB == 128 ? 128 : 256; // bytes that the swizzles act on
+  auto slot = [&]( uint32_t lane_part, uint32_t chunk ) __attribute__( ( always_inline ) ) { return ( lane_part ^ ( 16 * chunk % PERIOD ) ) + 16 * chunk / PERIOD * PERIOD; };
 
   float a1 = ch.tokens( MlstmChunks::A, pair, 0 )[lane], w1 = ch.tokens( MlstmChunks::W, pair, 0 )[lane]; // of token `lane`
   fetch_qv( 0 );
   __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0)
+  constexpr int STORES = 16; // of O, each an instruction of its own: the rows of a tile are whole rows of the output apart
   for ( uint32_t c = 0; c < ch.chunks; c++ ) {
     const uint32_t t0 = c * CHUNK, rows = min( (uint32_t)CHUNK, st.n_tokens - t0 );
     s_n[threadIdx.x] = n;
@@ -682,81 +732,101 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
       s_a[lane] = a1;
       s_w[c & 1][lane] = w1;
     }
-    // This wave's part of q and v has landed, behind which are no more than the last chunk's 16 stores (memory operations of a wave end in their order).
-    __builtin_amdgcn_s_waitcnt( 0x4F70 ); // vmcnt(16)
+    // This wave's part of q and v has landed: behind its requests are AT LEAST the last chunk's STORES (memory operations of a wave end in their order).
+    __builtin_amdgcn_s_waitcnt( ( STORES & 15 ) | ( STORES >> 4 ) << 14 | 0x0F70 );
     asm volatile( "s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory" ); // everyone's; and everyone is through with the last chunk's k
-    const uint4* weights = ch.weights + ( (uint64_t)pair * ch.chunks + c ) * ( WEIGHT_TILES * 128 ) + lane;
-    uint4 P[WEIGHT_TILES][2];
+    const uint4* weights = ch.weights + ( (uint64_t)pair * ch.chunks + c ) * ( WEIGHT_TILES * 64 ) + lane;
+    uint4 P[WEIGHT_TILES];
 #pragma unroll
     for ( uint32_t i = 0; i < WEIGHT_TILES; i++ ) {
-      P[i][0] = weights[i * 128];
-      P[i][1] = weights[i * 128 + 64];
+      P[i] = weights[i * 64];
     }
     const float den1 = ch.tokens( MlstmChunks::DEN, pair, c )[lane], floor1 = ch.tokens( MlstmChunks::FLOOR, pair, c )[lane]; // of token `lane`
     const float decay = ch.decay[(uint64_t)pair * ch.chunks + c];
-    const float n_more = n_chunk[(uint64_t)c * s.dim];
-    fetch( s_k, in.main.data + ( row_first + t0 ) * in.main.stride + in.col.k + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {} );
+    const float n_more = threadIdx.x < s.dim ? n_chunk[(uint64_t)c * s.dim] : 0.0f;
+    fetch( s_k, in.main.data + ( row_first + t0 ) * in.main.stride + in.col.k + h * s.dim, rows, s.dim / 8, std::integral_constant<uint32_t, RB> {}, swizzle_pair<RB> );
     __builtin_amdgcn_sched_barrier( 0 ); // (else the scheduler moves the requests down to where their results are used)
 
     // ---- Q S (state in front of the chunk): 16 queries a tile
     mfma_f32x4 O[4];
+    uint32_t q_row[4];
 #pragma unroll
     for ( int i = 0; i < 4; i++ ) {
       O[i] = mfma_f32x4 { 0, 0, 0, 0 };
+      q_row[i] = opaque( 16 * i * RB + q_lane );
     }
 #pragma unroll
     for ( int j = 0; j < KS; j++ ) {
+      if ( j % 2 == 0 ) {
+        __builtin_amdgcn_sched_barrier( 0 ); // (without these fences the scheduler asks for all operands of a phase at once and spills)
+      }
       Split<2> sp;
 #pragma unroll
       for ( int k = 0; k < 4; k++ ) {
         sp.set( k, S[2 * j + ( k >> 1 )][2 * ( k & 1 )], S[2 * j + ( k >> 1 )][2 * ( k & 1 ) + 1] );
       }
-      union
-      {
-        uint2 p[2];
-        bf16x8 x;
-      } a[4];
+      swap_halves( sp.t[1].x, sp.t[0].x ); // both terms of the lower 16 rows, the lower term in front; both of the upper 16
 #pragma unroll
-      for ( int i = 0; i < 4; i++ ) {
-#pragma unroll
-        for ( int hf = 0; hf < 2; hf++ ) {
-          a[i].p[hf] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + q_row[i] + swizzle<RB>( r, 4 * j + 2 * hf + ( g >> 1 ) ) * 16 );
-        }
-      }
-#pragma unroll
-      for ( int n2 = 1; n2 >= 0; n2-- ) { // (the tiles in turn: a product that waits for the one before it leaves the matrix unit idle)
+      for ( int n2 = 1; n2 >= 0; n2-- ) {
+        union
+        {
+          uint2 p[2];
+          bf16x8 x;
+        } a[4];
 #pragma unroll
         for ( int i = 0; i < 4; i++ ) {
+#pragma unroll
+          for ( int hf = 0; hf < 2; hf++ ) {
+            a[i].p[hf] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + slot( q_row[i], 4 * j + 2 * ( 1 - n2 ) + hf ) );
+          }
+        }
+#pragma unroll
+        for ( int i = 0; i < 4; i++ ) { // (the tiles in turn: a product that waits for the one before it leaves the matrix unit idle)
           O[i] = Mfma<__bf16>::k32( a[i].x, sp.t[n2].x, O[i] );
         }
       }
     }
-    // ---- denominators of this slice's tokens, a wave each: n . q, four dims a lane
-    for ( uint32_t t0w = slice + wave * 4 * slices; t0w < rows; t0w += 16 * slices ) { // 16 lanes a token
-      const uint32_t t = min( t0w + g * slices, (uint32_t)CHUNK - 1 );
+    // ---- denominators of this slice's tokens: n . q, four lanes a token, a quarter of the dims each
+    if ( slice + slices * wave < rows ) {
+      const uint32_t ln = opaque( lane );
+      const uint32_t token = slice + slices * ( wave + ( ln & ~3u ) ), t = min( token, (uint32_t)CHUNK - 1 );
+      const uint32_t half = ( ln >> 1 ) & 1, quad = ln & 1; // of the head's dims, of eight
+      const uint32_t q_token = t * RB + swizzle<RB>( t, 2 * KS * half ) * 16 + quad * 8;
+      const float* nk = s_n + 16 * KS * half + 4 * quad;
       float nq = 0.0f;
 #pragma unroll
-      for ( uint32_t piece = 0; piece < RB / 16; piece += 16 ) { // of 8 dims
-        if ( piece + r < RB / 16 ) {
-          const bf16x8 x = __builtin_bit_cast( bf16x8, s_q[t * ( RB / 16 ) + swizzle<RB>( t, piece + r )] );
-          const float4 n0 = *reinterpret_cast<const float4*>( &s_n[8 * ( piece + r )] ), n1 = *reinterpret_cast<const float4*>( &s_n[8 * ( piece + r ) + 4] ); // (zero past the head's size)
-          nq += (float)x[0] * n0.x + (float)x[1] * n0.y + (float)x[2] * n0.z + (float)x[3] * n0.w + (float)x[4] * n1.x + (float)x[5] * n1.y + (float)x[6] * n1.z + (float)x[7] * n1.w;
+      for ( uint32_t k = 0; k < KS; k++ ) { // 16 dims
+        if ( k % 4 == 0 ) {
+          __builtin_amdgcn_sched_barrier( 0 );
         }
+        union
+        {
+          uint2 p[2];
+          bf16x8 x;
+        } a;
+        const float4 n0 = *reinterpret_cast<const float4*>( nk + 16 * k ), n1 = *reinterpret_cast<const float4*>( nk + 16 * k + 8 );
+#pragma unroll
+        for ( uint32_t hf = 0; hf < 2; hf++ ) {
+          a.p[hf] = *reinterpret_cast<const uint2*>( reinterpret_cast<const char*>( s_q ) + slot( q_token, 2 * k + hf ) );
+        }
+        nq += (float)a.x[0] * n0.x + (float)a.x[1] * n0.y + (float)a.x[2] * n0.z + (float)a.x[3] * n0.w + (float)a.x[4] * n1.x + (float)a.x[5] * n1.y + (float)a.x[6] * n1.z
+              + (float)a.x[7] * n1.w;
       }
-      nq = row16_sum( nq );
+      nq += __shfl_xor( nq, 1 );
+      nq += __shfl_xor( nq, 2 );
       const float over = 1.0f / ( fmaxf( fabsf( nq * s.q_scale * s_a[t] + __shfl( den1, t ) ), __shfl( floor1, t ) ) + 1e-6f );
-      if ( r == 0 && t0w + g * slices < rows ) {
+      if ( ( ln & 3 ) == 0 && token < rows ) {
         ch.tokens( MlstmChunks::OVER, pair, c )[t] = over;
       }
     }
     // ---- O = a Q S + P V
-    bf16x8 V[2];
+    bf16x8 V[4];
 #pragma unroll
-    for ( int j = 0; j < 2; j++ ) {
-      V[j] = transposed( s_v, 32 * j, 2 * wave, std::integral_constant<uint32_t, 128> {} );
+    for ( int k = 0; k < 4; k++ ) {
+      V[k] = v_at( v_lane + 16 * k * 128 );
     }
 #pragma unroll
-    for ( int i = 0; i < 4; i++ ) {
+    for ( uint32_t i = 0; i < 4; i++ ) {
       const float4 a4 = *reinterpret_cast<const float4*>( &s_a[16 * i + 4 * g] );
       const float f[4] = { a4.x, a4.y, a4.z, a4.w };
 #pragma unroll
@@ -764,12 +834,14 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
         O[i][e] *= f[e] * s.q_scale;
       }
 #pragma unroll
-      for ( int j = 0; j <= i / 2; j++ ) {
-#pragma unroll
-        for ( int n2 = 1; n2 >= 0; n2-- ) {
-          O[i] = Mfma<__bf16>::k32( __builtin_bit_cast( bf16x8, P[weight_tile( i, j )][n2] ), V[j], O[i] );
-        }
+      for ( uint32_t k = 0; k <= i; k++ ) {
+        O[i] = Mfma<__bf16>::k32( __builtin_bit_cast( bf16x8, P[weight_tile( i, k )] ), V[k], O[i] );
       }
+    }
+    bf16x8 V2[2]; // the keys of 32 over the lanes: a half's terms are made in it, and change places with the other's
+#pragma unroll
+    for ( int k = 0; k < 2; k++ ) {
+      V2[k] = v_at( v_lane + ( 32 * k + upper ) * 128 );
     }
     __builtin_amdgcn_s_waitcnt( 0x0F70 ); // vmcnt(0): this wave's part of k has landed
     __syncthreads();                      // everyone's; and everyone has read q and v
@@ -782,6 +854,7 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
     const __amdgpu_buffer_rsrc_t o_rsrc
       = __builtin_amdgcn_make_buffer_rsrc( o_out + ( row_first + t0 ) * hv + h * s.vdim, 0, (int)( ( ( rows - 1 ) * hv + s.vdim ) * 4 ), 0x00020000 );
     const uint32_t o_off = col < s.vdim ? ( 4 * g * hv + col ) * 4 : PAST_THE_END;
+    static_assert( sizeof( O ) == STORES * sizeof( float ), "the wait at a chunk's head counts on one store for each element" );
 #pragma unroll
     for ( int i = 0; i < 4; i++ ) {
 #pragma unroll
@@ -791,18 +864,27 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
     }
     n = n * decay + n_more;
     // ---- S behind the chunk
-    Split<3> wv[2];
+    // 32 keys are three products: lower and middle term of the first 16; their upper term and the lower one of the others; the others' middle and upper term
+    bf16x8 wv[2][3];
 #pragma unroll
     for ( int j = 0; j < 2; j++ ) {
+      Split<3> terms;
 #pragma unroll
       for ( int hf = 0; hf < 2; hf++ ) {
-        const float4 w = *reinterpret_cast<const float4*>( &s_w[c & 1][32 * j + 16 * hf + 4 * g] );
-        wv[j].set( 2 * hf, (float)V[j][4 * hf] * w.x, (float)V[j][4 * hf + 1] * w.y );
-        wv[j].set( 2 * hf + 1, (float)V[j][4 * hf + 2] * w.z, (float)V[j][4 * hf + 3] * w.w );
+        const float4 w = *reinterpret_cast<const float4*>( &s_w[c & 1][32 * j + upper + 8 * hf + 4 * ( g & 1 )] );
+        terms.set( 2 * hf, (float)V2[j][4 * hf] * w.x, (float)V2[j][4 * hf + 1] * w.y );
+        terms.set( 2 * hf + 1, (float)V2[j][4 * hf + 2] * w.z, (float)V2[j][4 * hf + 3] * w.w );
       }
+      bf16x8 lower = terms.t[1].x, others = terms.t[1].x; // the middle terms of either, in all lanes
+      swap_halves( lower, others );
+      const bool first = lane < 32;
+      wv[j][0] = first ? terms.t[2].x : lower;
+      wv[j][1] = first ? terms.t[0].x : terms.t[2].x;
+      wv[j][2] = first ? others : terms.t[0].x;
     }
 #pragma unroll
     for ( int d0 = 0; d0 < 2 * KS; d0 += 4 ) { // (four tiles in turn, as above)
+      __builtin_amdgcn_sched_barrier( 0 );
 #pragma unroll
       for ( int d = d0; d < d0 + 4; d++ ) {
 #pragma unroll
@@ -810,18 +892,22 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
           S[d][v] *= decay;
         }
       }
+      const uint32_t k_both = opaque( k_lane );
 #pragma unroll
       for ( int j = 0; j < 2; j++ ) {
-        bf16x8 a[4];
+        bf16x8 a[3][4];
 #pragma unroll
         for ( int d = 0; d < 4; d++ ) {
-          a[d] = transposed( s_k, 32 * j, 2 * ( d0 + d ), std::integral_constant<uint32_t, RB> {} );
+          const uint32_t at = slot( k_both, 4 * ( ( d0 + d ) / 2 ) + d % 2 ) + 32 * j * RB;
+          a[0][d] = transposed( s_k, at, at + 8 * RB );
+          a[2][d] = transposed( s_k, at + 16 * RB, at + 24 * RB );
+          a[1][d] = lane < 32 ? a[0][d] : a[2][d];
         }
 #pragma unroll
-        for ( int n3 = 2; n3 >= 0; n3-- ) {
+        for ( int n3 = 0; n3 < 3; n3++ ) {
 #pragma unroll
           for ( int d = 0; d < 4; d++ ) {
-            S[d0 + d] = Mfma<__bf16>::k32( a[d], wv[j].t[n3].x, S[d0 + d] );
+            S[d0 + d] = Mfma<__bf16>::k32( a[n3][d], wv[j][n3], S[d0 + d] );
           }
         }
       }
@@ -834,7 +920,7 @@ __global__ __launch_bounds__( 256, 2 ) void mlstm_states_kernel( float* __restri
   for ( int d = 0; d < 2 * KS; d++ ) {
 #pragma unroll
     for ( int v = 0; v < 4; v++ ) {
-      __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, (float)S[d][v] ), S_rsrc, S_off, ( 16 * d + v ) * vpad * 4, 0 );
+      __builtin_amdgcn_raw_buffer_store_b32( __builtin_bit_cast( unsigned, (float)S[d][v] ), S_rsrc, S_off, ( 32 * ( d / 2 ) + 8 * ( d % 2 ) + v ) * vpad * 4, 0 );
     }
   }
   if ( slice == 0 && threadIdx.x < s.dim ) {
@@ -1001,6 +1087,7 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
   const uint64_t nm_bytes = ( batch * s.heads * ( s.dim + 1ull ) * sizeof( float ) + 255 ) / 256 * 256;
   const uint64_t n_pairs = batch * s.heads, n_chunks = ( (uint64_t)n_tokens + CHUNK - 1 ) / CHUNK, all_chunks = chunked ? n_pairs * n_chunks : 0;
   const uint64_t weight_bytes = all_chunks * WEIGHT_TILES * 128 * sizeof( uint4 ), token_bytes = MlstmChunks::PLANES * all_chunks * CHUNK * sizeof( float );
+  // chunks: 12 KB and a head's n, whatever the size of its values (a tenth of the call's workspace at 512 columns of v, two fifths at 64)
   const uint64_t more = chunked ? weight_bytes + token_bytes + all_chunks * ( s.dim + 1ull ) * sizeof( float ) : rows * 2 * s.heads * sizeof( float );
   if ( int rc = stream_scratch( st, SCRATCH_MIXER, o_bytes + nm_bytes + more, 1ull << 20, &scratch ) ) {
     return rc;
@@ -1059,7 +1146,7 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
     }
     const size_t lds = ( 3 * ( ( s.dim + 3 ) / 4 * 4 ) + SLICE + 16 + 16 * SLICE ) * sizeof( float );
     if ( walked ) {
-      // the chunk kernel has done it
+      // the chunks' kernels have done it
     } else if ( s.dim <= 64 ) {
       mlstm_walk_kernel<E, View, 4><<<grid, 256, lds, st>>>( o, nm, in, raw, state, s );
     } else if ( s.dim <= 128 ) {

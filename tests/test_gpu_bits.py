@@ -1,0 +1,56 @@
+"""Bits of kernels whose order of sums models depend on.  A design whose layers feed each other for a thousand tokens turns a last bit into a difference of a
+token's logits that can be far larger than that of any of its parts, so a faster kernel here keeps the order of its sums, and what is pinned are checksums of whole
+outputs.  Inputs are whole numbers over powers of two from a generator of numpy's, and products in front of the kernel are exact in any order."""
+import zlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def draw(rng, shape, spread=0, dtype="bfloat16"):
+    """Up to seven significant bits, over `spread` + 1 powers of two."""
+    import torch
+    v = rng.integers(-127, 128, shape).astype(np.float32) / 64.0
+    if spread:
+        v = np.ldexp(v, -rng.integers(0, spread + 1, shape))
+    return torch.from_numpy(v.astype(np.float32)).cuda().to(getattr(torch, dtype))
+
+
+def checksum(*tensors):
+    import torch
+    c = 0
+    for t in tensors:
+        c = zlib.crc32(t.contiguous().view(torch.uint8).cpu().numpy().tobytes(), c)
+    return c
+
+
+MLSTM = {(3, 40, 8, 24, 65): 3122385930, (2, 64, 136, 33, 256): 1821903039, (4, 128, 72, 64, 300): 579374656, (2, 232, 200, 130, 127): 3581533614,
+         (8, 256, 512, 1025, 64): 3581607802}
+
+
+def mlstm_bits(H, d, dv, *cuts):
+    """Two contexts and a slot without one, in two portions: outputs, then the state."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    rng = np.random.default_rng(d + dv)
+    m, width, B = GhMlstm(H, d, dv, 15.0, 1e-4), 8, 3
+    rows, gate_row = ops.mlstm_weight_rows(m)
+    w = rng.integers(-2, 3, (rows, width)) * np.where(np.arange(rows) >= gate_row, 0.5, 1.0)[:, None]
+    w = torch.from_numpy(w.astype(np.float32)).cuda().bfloat16()
+    x = torch.from_numpy(rng.integers(-1, 2, (B, sum(cuts), width)).astype(np.float32)).cuda().bfloat16()
+    bias_i, bias_f, norm = draw(rng, H), draw(rng, H) + 3, draw(rng, H * dv) / 8 + 1
+    state = torch.zeros((B, ops.mlstm_state_bytes(m) // 4), device="cuda")
+    table, out, at = ops.row_table([0 if i == 1 else state[i].data_ptr() for i in range(B)]), [], 0
+    for c in cuts:
+        start = torch.full((B,), at, dtype=torch.int32, device="cuda")
+        out.append(ops.mlstm_forward(x[:, at:at + c].reshape(B * c, width).contiguous(), w, m, bias_i, bias_f, norm, table, start, c))
+        at += c
+    return checksum(*out, state)
+
+
+@pytest.mark.parametrize("shape", MLSTM)
+def test_mlstm(shape):
+    assert mlstm_bits(*shape) == MLSTM[shape]
