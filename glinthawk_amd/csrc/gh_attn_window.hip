@@ -663,10 +663,12 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
 // order       the longest work-groups of ALL contexts and heads start first.  Those of one pair next to each other, for its keys in L2, left
 //             the last pairs' long ones to the end: 4.9 of 8 waves in flight on average, 6.7 now.  The keys then come out of the Infinity
 //             Cache (600 MB at 8 x 1024 tokens), which is not what bounds it.
+// rounding    scale and bias are one fused multiplication in every tile, the reference point is taken off behind it.  Both in one for tiles with a constant bias
+//             saves 32 of a tile's instructions and no time (8 x 1024 tokens 166 us against 165), and bits differ from one form of tile to the other.
 // bound       vector and matrix work of two waves a SIMD, which overlap little.  8 x 1024 tokens, 32 heads of 128, window 1024, 512 distances:
 //             228 us -> 200 with fewer vector instructions (702 -> 510 a tile and wave) -> 155 with the order; 4 x 2048 tokens without a
 //             bias: 305 -> 274 -> 240, keys as values 303 -> 275 -> 221.  The products run at 0.9 PFLOP/s there, both terms counted.
-//             Still fewer vector instructions (430 -> 370), other priorities for the waves in their products: no change.
+//             Other priorities for the waves in their products: no change.
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY = 8.0f; // the reference point of a column's exponentials moves when its maximum has grown by 2^LAZY
 constexpr uint32_t TILE_KEYS = 64;
@@ -868,40 +870,34 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         st[sub][v] = sx[sub][v];
       }
     }
-    // ---- scale, bias by distance, mask (log2 domain): a score is st * sc + b
+    // ---- scale, bias by distance, mask (log2 domain)
     const uint32_t key_l = t0 + 4 * g2; // key of register v: key_l + offset_of( sub, v )
     const int32_t dist_l = (int32_t)( pos - key_l );
-    float sc = 1.0f, b = 0.0f;
-    if constexpr ( SHARED ) { // a factor for each key
+    auto scores = [&]( auto bias_of ) __attribute__( ( always_inline ) ) {
 #pragma unroll
       for ( int sub = 0; sub < 2; sub++ ) {
 #pragma unroll
         for ( int q4 = 0; q4 < 4; q4++ ) {
-          const float4 f = *reinterpret_cast<const float4*>( s_factor + 32 * sub + 8 * q4 + 4 * g2 );
-          st[sub][4 * q4] *= f.x, st[sub][4 * q4 + 1] *= f.y, st[sub][4 * q4 + 2] *= f.z, st[sub][4 * q4 + 3] *= f.w;
+          float4 f = make_float4( scale_log2e, scale_log2e, scale_log2e, scale_log2e );
+          if constexpr ( SHARED ) { // a factor for each key
+            f = *reinterpret_cast<const float4*>( s_factor + 32 * sub + 8 * q4 + 4 * g2 );
+          }
+          const float factor[4] = { f.x, f.y, f.z, f.w };
+#pragma unroll
+          for ( int e = 0; e < 4; e++ ) {
+            st[sub][4 * q4 + e] = __builtin_fmaf( st[sub][4 * q4 + e], factor[e], bias_of( offset_of( sub, 4 * q4 + e ) ) );
+          }
         }
       }
-    }
-    if ( far && ( SHARED || scale_log2e > 0.0f ) ) { // the largest score is that of the largest product, and one instruction scales it and takes its reference point off
-      sc = SHARED ? 1.0f : scale_log2e;
-      b = my_bias[n_dist - 1];
-    } else if ( !far && bias_pad > 0 ) { // from the distance of the last key up, one address for all
+    };
+    if ( far ) {
+      const float b = my_bias[n_dist - 1];
+      scores( [&]( int ) __attribute__( ( always_inline ) ) { return b; } );
+    } else if ( bias_pad > 0 ) { // from the distance of the last key up, one address for all
       const float* row = my_bias + dist_l - ( (int)TILE_KEYS - 5 );
-#pragma unroll
-      for ( int sub = 0; sub < 2; sub++ ) {
-#pragma unroll
-        for ( int v = 0; v < 16; v++ ) {
-          st[sub][v] = __builtin_fmaf( st[sub][v], SHARED ? 1.0f : scale_log2e, row[(int)TILE_KEYS - 5 - offset_of( sub, v )] );
-        }
-      }
+      scores( [&]( int o ) __attribute__( ( always_inline ) ) { return row[(int)TILE_KEYS - 5 - o]; } );
     } else {
-#pragma unroll
-      for ( int sub = 0; sub < 2; sub++ ) {
-#pragma unroll
-        for ( int v = 0; v < 16; v++ ) {
-          st[sub][v] = __builtin_fmaf( st[sub][v], SHARED ? 1.0f : scale_log2e, my_bias[min( pos - min( key_l + offset_of( sub, v ), pos ), n_dist - 1 )] );
-        }
-      }
+      scores( [&]( int o ) __attribute__( ( always_inline ) ) { return my_bias[min( pos - min( key_l + o, pos ), n_dist - 1 )]; } );
     }
     if ( edge ) { // the hidden keys of a column are those before or behind one offset, which a register's is compared with
       auto hide = [&]( auto hidden ) __attribute__( ( always_inline ) ) {
@@ -930,7 +926,7 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         mx4[c] = fmaxf( mx4[c], st[c >> 1][8 * ( c & 1 ) + e] );
       }
     }
-    const float mx = __builtin_fmaf( half_wave_max( fmaxf( fmaxf( mx4[0], mx4[1] ), fmaxf( mx4[2], mx4[3] ) ) ), sc, b );
+    const float mx = half_wave_max( fmaxf( fmaxf( mx4[0], mx4[1] ), fmaxf( mx4[2], mx4[3] ) ) );
     if ( __builtin_amdgcn_ballot_w64( mx > m + LAZY ) != 0 ) {
       const float m_new = fmaxf( m, mx );
       const float alpha = __builtin_amdgcn_exp2f( m - m_new );
@@ -944,7 +940,6 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         }
       }
     }
-    const float ref = b - m;
 #pragma unroll
     for ( int kk = 0; kk < 4; kk++ ) { // 16 keys
       union
@@ -954,8 +949,8 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
       } hi, lo;
 #pragma unroll
       for ( int e = 0; e < 4; e++ ) {
-        const float p0 = __builtin_amdgcn_exp2f( __builtin_fmaf( st[kk >> 1][8 * ( kk & 1 ) + 2 * e], sc, ref ) );
-        const float p1 = __builtin_amdgcn_exp2f( __builtin_fmaf( st[kk >> 1][8 * ( kk & 1 ) + 2 * e + 1], sc, ref ) );
+        const float p0 = __builtin_amdgcn_exp2f( st[kk >> 1][8 * ( kk & 1 ) + 2 * e] - m );
+        const float p1 = __builtin_amdgcn_exp2f( st[kk >> 1][8 * ( kk & 1 ) + 2 * e + 1] - m );
         l += p0;
         l += p1;
         hi.pair[e] = bf16_pair( p0, p1 );

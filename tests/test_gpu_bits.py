@@ -54,3 +54,27 @@ def mlstm_bits(H, d, dv, *cuts):
 @pytest.mark.parametrize("shape", MLSTM)
 def test_mlstm(shape):
     assert mlstm_bits(*shape) == MLSTM[shape]
+
+
+# (heads, kv heads, head sizes, values are keys), (window, kept tokens, distances), tokens: no bias, one that ends before the keys do, one too long for room around it
+WINDOW = {(4, 4, 128, 128, False, 0, 0, 0, 290): 322941296, (8, 2, 72, 40, False, 97, 5, 1, 131): 2589682963, (4, 4, 128, 128, False, 300, 4, 64, 700): 43964091,
+          (4, 4, 128, 128, True, 0, 0, 90, 290): 2409675448, (2, 2, 96, 96, True, 64, 70, 17, 131): 4132586507, (6, 2, 128, 64, False, 31, 64, 7900, 131): 382486082}
+
+
+def window_bits(heads, kv, dim, vdim, shared, window, keep, n_dist, T):
+    """Two contexts, one of them with keys in front."""
+    import torch
+    from glinthawk_amd import ops
+    rng = np.random.default_rng(dim + T)
+    a, starts = ops.window_attn(heads, kv, dim, vdim, dim ** -0.5, window, keep, n_dist, shared), [0, 77]
+    keys = max(starts) + T
+    cache, factors = draw(rng, (2, keys, kv * (dim if shared else dim + vdim)), 2), draw(rng, (2, -(-keys // 32) * kv * 32), 0, "float32") / 4 + 1
+    memory = torch.cat([cache.view(2, -1).view(torch.uint8), factors.view(torch.uint8)], 1).contiguous()
+    bias = draw(rng, (heads, n_dist), 2, "float32") if n_dist else None
+    return checksum(ops.attn_window(draw(rng, (2 * T, heads * dim), 2), a, ops.row_table([m.data_ptr() for m in memory]), torch.tensor(starts, dtype=torch.int32, device="cuda"), T,
+                                    max(starts), bias, 0, cache[0].numel() * 2))
+
+
+@pytest.mark.parametrize("shape", WINDOW)
+def test_window_attention(shape):
+    assert window_bits(*shape) == WINDOW[shape]
