@@ -660,18 +660,21 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
 //             rows are in registers while this one is multiplied, and two work-groups share a CU.  Where values are keys both products
 //             read one tile: the low four bits of the row, pairs exchanged, keep the plain reads (16 rows, one chunk) and the
 //             transposing ones (4 rows, 4 chunks) apart.
-// order       the longest work-groups of ALL contexts and heads start first.  Those of one pair next to each other, for its keys in L2, left
-//             the last pairs' long ones to the end: 4.9 of 8 waves in flight on average, 6.7 now.  The keys then come out of the Infinity
-//             Cache (600 MB at 8 x 1024 tokens), which is not what bounds it.
+// order       the longest work-groups of up to eight pairs of an XCD start first, then those of the next eight.  Those of one pair next to each other leave
+//             the last pairs' long ones to the end, 4.9 of 8 waves in flight on average where there are few; those of all pairs at once need all keys at a
+//             time, which come out of HBM again for every block once they are more than the Infinity Cache holds.  Heads of 128, us: pair by pair, eight, all:
+//             8 x 1024 tokens of window 1024 198, 149, 153; 32 x 1024 of it 783, 642, 775; 16 x 2048 1131, 1020, 1294; 8 x 4096 1970, 1818, 2107; 64 heads, 16 x
+//             2048 of window 1024 1884, 1791, 2238; 2 x 8192 1812, 1751, 1755; keys as values 16 x 2048 979, 898, 933.  Groups of 4 to 16 are within 4 %, of 2 and 48 behind.
 // rounding    scale and bias are one fused multiplication in every tile, the reference point is taken off behind it.  Both in one for tiles with a constant bias
 //             saves 32 of a tile's instructions and no time (8 x 1024 tokens 166 us against 165), and bits differ from one form of tile to the other.
 // bound       vector and matrix work of two waves a SIMD, which overlap little.  8 x 1024 tokens, 32 heads of 128, window 1024, 512 distances:
-//             228 us -> 200 with fewer vector instructions (702 -> 510 a tile and wave) -> 155 with the order; 4 x 2048 tokens without a
-//             bias: 305 -> 274 -> 240, keys as values 303 -> 275 -> 221.  The products run at 0.9 PFLOP/s there, both terms counted.
+//             221 us -> 200 with fewer vector instructions (702 -> 540 a tile and wave) -> 161 with the order; 4 x 2048 tokens without a
+//             bias: 309 -> 239, keys as values 293 -> 222 (calls in a row, their keys in the Infinity Cache).  The products run at 0.9 PFLOP/s there, both terms counted.
 //             Other priorities for the waves in their products: no change.
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY = 8.0f; // the reference point of a column's exponentials moves when its maximum has grown by 2^LAZY
 constexpr uint32_t TILE_KEYS = 64;
+constexpr uint32_t GROUP_PAIRS = 8;
 constexpr uint32_t BIAS_LDS = 8192; // floats of bias table a work-group can hold
 // Entries around a head's table, where they fit: from a wave's 32 tokens to the keys of a tile that touches the table the distances reach 94 before its start and behind its end
 constexpr uint32_t BIAS_PAD = 96;
@@ -699,6 +702,7 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
                                                                  uint32_t head_cols,  // query heads side by side in the columns
                                                                  uint32_t col_blocks, // work-groups along the tokens of a pair
                                                                  uint32_t n_pairs,    // contexts x kv heads x (query heads of a group / head_cols)
+                                                                 uint32_t group_pairs, // pairs of an XCD whose blocks are in one order
                                                                  uint32_t bias_row,   // floats of a head's bias table in LDS; 0: no bias
                                                                  uint32_t bias_pad )  // its entries in front of distance 0 and behind the last one
 {
@@ -708,11 +712,12 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
   float* s_factor = reinterpret_cast<float*>( s_v + TILE_KEYS * 16 );  // SHARED: of the tile's keys, times scale and log2(e)
   float* s_bias = s_factor + ( SHARED ? TILE_KEYS : 0 );               // (head_cols, bias_row), times log2(e)
 
-  // all column blocks of a pair on one XCD; the longest blocks of all pairs first
+  // all column blocks of a pair on one XCD; the longest blocks of a group of pairs first
   const uint32_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const uint32_t xcd_pairs = ( n_pairs + 7 ) / 8;
-  const uint32_t cb = col_blocks - 1 - slot / xcd_pairs;
-  const uint32_t pair = ( slot % xcd_pairs ) * 8 + xcd;
+  const uint32_t group = slot / ( group_pairs * col_blocks ), in_group = slot % ( group_pairs * col_blocks );
+  const uint32_t pairs = min( group_pairs, ( n_pairs + 7 ) / 8 - group * group_pairs );
+  const uint32_t cb = col_blocks - 1 - in_group / pairs;
+  const uint32_t pair = ( group * group_pairs + in_group % pairs ) * 8 + xcd;
   if ( pair >= n_pairs ) {
     return;
   }
@@ -1694,11 +1699,13 @@ int attend_tiles( const WindowOut<__bf16>& out, const __bf16* q, const float* bi
   const uint64_t n_pairs = batch * s.kv_heads * ( s.group / head_cols );
   const uint64_t grid = ( n_pairs + 7 ) / 8 * 8 * col_blocks;
   GH_REQUIRE( grid < ( 1ull << 31 ), "gh_attn_window: grid too large" );
+  const uint64_t xcd_pairs = ( n_pairs + 7 ) / 8, groups = ( xcd_pairs + GROUP_PAIRS - 1 ) / GROUP_PAIRS;
+  const uint32_t group_pairs = (uint32_t)( ( xcd_pairs + groups - 1 ) / groups ); // as many in each
   const uint32_t bias_pad = bias != nullptr && (uint64_t)head_cols * ( s.n_dist + 2 * BIAS_PAD ) <= BIAS_LDS ? BIAS_PAD : 0;
   const uint32_t bias_row = bias == nullptr ? 0 : s.n_dist + 2 * bias_pad, bias_floats = head_cols * bias_row;
   const size_t lds = ( s.values_are_keys ? TILE_KEYS * ( 256 + sizeof( float ) ) : 2 * TILE_KEYS * 256 ) + std::max( bias_floats, 1u ) * sizeof( float );
 #define GH_WINDOW_TILES( KS, VB, SHARED ) \
-  window_tiles_kernel<KS, VB, SHARED><<<(unsigned)grid, 256, lds, st>>>( out, q, bias, wr, s, head_cols, col_blocks, (uint32_t)n_pairs, bias_row, bias_pad )
+  window_tiles_kernel<KS, VB, SHARED><<<(unsigned)grid, 256, lds, st>>>( out, q, bias, wr, s, head_cols, col_blocks, (uint32_t)n_pairs, group_pairs, bias_row, bias_pad )
   if ( s.values_are_keys ) {
     if ( s.dpad <= 64 ) {
       GH_WINDOW_TILES( 4, 2, true );

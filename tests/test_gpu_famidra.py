@@ -250,8 +250,9 @@ def test_decode_of_heads_with_keys_of_their_own(heads, dim, vdim, rows, keys, sh
 
 # of a wave's 32 columns and 64 keys at a time: (heads, kv heads, head sizes), (window, kept tokens, distances, scale), (starts, tokens).  Tables of one
 # distance, of fewer than a tile, with room for the entries around it and without, and none; windows that end inside a wave, kept tokens that reach into
-# it; first positions on both sides of a tile's edge, portions past the last full wave; keys that are values too, of a size with an odd number of blocks
-@pytest.mark.parametrize("heads,kv,dim,vdim,shared", [(4, 4, 128, 128, False), (8, 2, 72, 40, False), (6, 2, 128, 64, False), (2, 2, 96, 96, True), (4, 4, 128, 128, True)])
+# it; first positions on both sides of a tile's edge, portions past the last full wave; keys that are values too, of a size with an odd number of blocks; 33 heads:
+# two groups of work-groups an XCD, the second one smaller, of which some have no head
+@pytest.mark.parametrize("heads,kv,dim,vdim,shared", [(4, 4, 128, 128, False), (8, 2, 72, 40, False), (6, 2, 128, 64, False), (2, 2, 96, 96, True), (4, 4, 128, 128, True), (33, 33, 64, 64, False)])
 @pytest.mark.parametrize("window,keep,n_dist,scale", [(0, 0, 0, 1.0), (0, 0, 0, -1.0), (97, 5, 1, 1.0), (64, 70, 17, 1.0), (150, 200, 90, -1.0), (300, 3, 2000, 1.0), (31, 64, 7900, 1.0)])
 @pytest.mark.parametrize("starts,T", [([0, 64], 16), ([1, 257], 131), ([95, 0], 290)])
 def test_tiles_of_keys_by_waves(heads, kv, dim, vdim, shared, window, keep, n_dist, scale, starts, T):
