@@ -250,13 +250,14 @@ __global__ __launch_bounds__( 256 ) void gemm_reduce_kernel( E* __restrict__ xou
 }
 
 // Few weight rows (r <= 32: the gates of a recurrent mixer) under many activation rows: bound by the activations, which the tile kernels
-// would read with most of their matrix work wasted on rows that are not there.  A work-group takes 32 activation rows, its eight waves every
-// eighth 64 of the K range, straight from memory in operand order (a row's 64 bytes an instruction, the rest of the line by the next);
-// their sums meet in LDS.  What counts is how much is asked for at once: two pieces of 64 k a wave, two waves a SIMD.  16 rows of 4096 k
-// at 8192 activation rows: four waves with one piece each, 32 bytes of a row an instruction, 23 to 26 us, so 17.4 (3.9 TB/s; the rest of the
-// time is the launch, the first loads and the sums); 256 rows 16.4 -> 12.5, 32768 78 -> 61.  Four and eight pieces 17.8 and 18.4.
+// would read with most of their matrix work wasted on rows that are not there.  A work-group takes 32 activation rows, its four waves every
+// fourth 64 of the K range, straight from memory in operand order (a row's 64 bytes an instruction, the rest of the line by the next);
+// their sums meet in LDS.  What counts is how much is asked for at once: two pieces of 64 k a wave, the next as soon as one is multiplied.  16 rows of 4096 k,
+// calls in a row: 8192 activation rows, one piece at a time and 32 bytes of a row an instruction 25.0 us, so 21.7 (3.1 TB/s; the rest of the time is the launch,
+// the first loads and the sums); 256 rows 15.2 -> 14.3, 32768 71 -> 63.  Four and eight pieces 21.4 and 22.3, 65 and 68.  The order of the sums is that of
+// v_mfma_f32_32x32x16_bf16, two of which in turn are one of the instructions here, bit for bit.  Eight waves with every eighth 64 each (19.8, 14.3 and 57 us) give other bits.
 // fp32 output (b, r).  s % 256 == 0, 16-byte aligned operands.  TILES: of 16 weight rows.
-constexpr uint32_t SKINNY_ROWS = 32, SKINNY_WAVES = 8, SKINNY_AHEAD = 2;
+constexpr uint32_t SKINNY_ROWS = 32, SKINNY_WAVES = 4, SKINNY_AHEAD = 2;
 template<typename E, int TILES>
 __global__ __launch_bounds__( SKINNY_WAVES * 64 ) void gemm_skinny_kernel( float* __restrict__ out, const E* __restrict__ x, const E* __restrict__ w, uint32_t s, uint32_t r, uint32_t b )
 {
@@ -267,55 +268,70 @@ __global__ __launch_bounds__( SKINNY_WAVES * 64 ) void gemm_skinny_kernel( float
   const E *xp[2], *wp[TILES]; // rows past the last repeat it and are not stored
 #pragma unroll
   for ( uint32_t t = 0; t < 2; t++ ) {
-    xp[t] = x + (uint64_t)min( token0 + 16 * t + fr, b - 1 ) * s + 8 * g;
+    xp[t] = x + (uint64_t)min( token0 + 16 * t + fr, b - 1 ) * s + 64 * wave + 8 * g;
   }
 #pragma unroll
   for ( uint32_t i = 0; i < TILES; i++ ) {
-    wp[i] = w + (uint64_t)min( 16 * i + fr, r - 1 ) * s + 8 * g;
+    wp[i] = w + (uint64_t)min( 16 * i + fr, r - 1 ) * s + 64 * wave + 8 * g;
   }
   mfma_f32x4 acc[TILES][2];
 #pragma unroll
   for ( int i = 0; i < TILES; i++ ) {
     acc[i][0] = acc[i][1] = mfma_f32x4 { 0.0f, 0.0f, 0.0f, 0.0f };
   }
-  auto pieces = [&]( uint32_t k, auto count ) __attribute__( ( always_inline ) ) {
-    constexpr int U = decltype( count )::value;
-    x8 xv[U][2][2], wv[U][2][TILES];
+  x8 xv[SKINNY_AHEAD][2][2], wv[SKINNY_AHEAD][2][TILES];
+  auto ask = [&]( int u, uint32_t k ) __attribute__( ( always_inline ) ) { // 64 k
 #pragma unroll
-    for ( int u = 0; u < U; u++ ) {
+    for ( int h = 0; h < 2; h++ ) {
 #pragma unroll
-      for ( int h = 0; h < 2; h++ ) {
+      for ( int t = 0; t < 2; t++ ) {
+        xv[u][h][t] = *reinterpret_cast<const x8*>( xp[t] + k + 32 * h );
+      }
 #pragma unroll
-        for ( int t = 0; t < 2; t++ ) {
-          xv[u][h][t] = *reinterpret_cast<const x8*>( xp[t] + k + 64 * SKINNY_WAVES * u + 32 * h );
-        }
-#pragma unroll
-        for ( int i = 0; i < TILES; i++ ) {
-          wv[u][h][i] = *reinterpret_cast<const x8*>( wp[i] + k + 64 * SKINNY_WAVES * u + 32 * h );
-        }
+      for ( int i = 0; i < TILES; i++ ) {
+        wv[u][h][i] = *reinterpret_cast<const x8*>( wp[i] + k + 32 * h );
       }
     }
-    __builtin_amdgcn_sched_barrier( 0 ); // (else the scheduler asks for one piece at a time)
+  };
+  auto multiply = [&]( int u ) __attribute__( ( always_inline ) ) {
 #pragma unroll
-    for ( int u = 0; u < U; u++ ) {
+    for ( int h = 0; h < 2; h++ ) {
 #pragma unroll
-      for ( int h = 0; h < 2; h++ ) {
+      for ( int i = 0; i < TILES; i++ ) {
 #pragma unroll
-        for ( int i = 0; i < TILES; i++ ) {
-#pragma unroll
-          for ( int t = 0; t < 2; t++ ) {
-            acc[i][t] = Mfma<E>::k32( wv[u][h][i], xv[u][h][t], acc[i][t] );
-          }
+        for ( int t = 0; t < 2; t++ ) {
+          acc[i][t] = Mfma<E>::k32( wv[u][h][i], xv[u][h][t], acc[i][t] );
         }
       }
     }
   };
-  uint32_t k = wave * 64;
-  for ( ; k + 64 * SKINNY_WAVES * ( SKINNY_AHEAD - 1 ) < s; k += 64 * SKINNY_WAVES * SKINNY_AHEAD ) {
-    pieces( k, std::integral_constant<int, SKINNY_AHEAD> {} );
+  constexpr uint32_t STEP = 64 * SKINNY_WAVES;
+#pragma unroll
+  for ( int u = 0; u < (int)SKINNY_AHEAD; u++ ) {
+    if ( u * STEP < s ) {
+      ask( u, u * STEP );
+    }
   }
-  for ( ; k < s; k += 64 * SKINNY_WAVES ) {
-    pieces( k, std::integral_constant<int, 1> {} );
+  uint32_t k = 0; // (of wave 0; the others' pieces lie behind its)
+  for ( ; k + ( 2 * SKINNY_AHEAD - 1 ) * STEP < s; k += SKINNY_AHEAD * STEP ) {
+#pragma unroll
+    for ( int u = 0; u < (int)SKINNY_AHEAD; u++ ) {
+      multiply( u );
+      __builtin_amdgcn_sched_barrier( 0 );
+      ask( u, k + ( SKINNY_AHEAD + u ) * STEP );
+      __builtin_amdgcn_sched_barrier( 0 );
+    }
+  }
+  for ( ; k < s; k += SKINNY_AHEAD * STEP ) {
+#pragma unroll
+    for ( int u = 0; u < (int)SKINNY_AHEAD; u++ ) {
+      if ( k + u * STEP < s ) {
+        multiply( u );
+      }
+      if ( k + ( SKINNY_AHEAD + u ) * STEP < s ) {
+        ask( u, k + ( SKINNY_AHEAD + u ) * STEP );
+      }
+    }
   }
   // acc[i][t][v]: weight row 16 i + 4 g + v, token 16 t + fr
 #pragma unroll
@@ -330,14 +346,14 @@ __global__ __launch_bounds__( SKINNY_WAVES * 64 ) void gemm_skinny_kernel( float
   }
   __syncthreads();
 #pragma unroll
-  for ( uint32_t n = 0; n < TILES; n++ ) {
-    const uint32_t at = wave * TILES + n;
+  for ( uint32_t n = 0; n < 8 * TILES / SKINNY_WAVES; n++ ) {
+    const uint32_t at = wave * ( 8 * TILES / SKINNY_WAVES ) + n;
     float y[SKINNY_WAVES];
 #pragma unroll
     for ( uint32_t o = 0; o < SKINNY_WAVES; o++ ) {
       y[o] = sums[o][at][lane];
     }
-    const float sum = ( ( y[0] + y[1] ) + ( y[2] + y[3] ) ) + ( ( y[4] + y[5] ) + ( y[6] + y[7] ) );
+    const float sum = ( y[0] + y[1] ) + ( y[2] + y[3] );
     const uint32_t row = 16 * ( at / 8 ) + 4 * g + at % 4, token = token0 + 16 * ( ( at / 4 ) % 2 ) + fr;
     if ( row < r && token < b ) {
       out[(uint64_t)token * r + row] = sum;
@@ -603,7 +619,7 @@ bool gemm_few_rows_apart( uint64_t s, uint64_t r, uint64_t few, uint64_t b, gh_d
   if ( !is_half_type( dt ) || few == 0 || few >= r || !gemm_ring_applicable( s, r, b, x, w, x ) || !skinny_takes( s, few, b, x, static_cast<const char*>( w ) + ( r - few ) * s * 2 ) ) {
     return false;
   }
-  const double skinny_ns = 5000.0 + (double)( b * s ) * 2.0 / 4500.0;
+  const double skinny_ns = 5000.0 + (double)( b * s ) * 2.0 / 4000.0;
   return product_ns( s, r, b ) > product_ns( s, r - few, b ) + skinny_ns;
 }
 

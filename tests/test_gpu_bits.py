@@ -78,3 +78,18 @@ def window_bits(heads, kv, dim, vdim, shared, window, keep, n_dist, T):
 @pytest.mark.parametrize("shape", WINDOW)
 def test_window_attention(shape):
     assert window_bits(*shape) == WINDOW[shape]
+
+
+# (k, activation rows, weight rows): work-groups whose waves get one piece of 64 k or two, some of them one more or none; one tile of weight rows and two
+FEW_ROWS = {(256, 200, 8): 1210123369, (768, 225, 17): 3488112410, (1280, 333, 32): 1850897936, (512, 193, 1): 827850632, (4096, 1000, 16): 916273720}
+
+
+def few_rows_bits(s, b, r):
+    from glinthawk_amd import ops
+    rng = np.random.default_rng(s + b)
+    return checksum(ops.matmul_scaled(draw(rng, (b, s), 6), draw(rng, (r, s), 6), 0.5))
+
+
+@pytest.mark.parametrize("shape", FEW_ROWS)
+def test_product_of_few_weight_rows(shape):
+    assert few_rows_bits(*shape) == FEW_ROWS[shape]
