@@ -130,131 +130,168 @@ __global__ __launch_bounds__( 1024 ) void window_append4_kernel( E* __restrict__
   }
 }
 
-// Prompts (bias and both norms present): a token's q, k and v together, the columns of the product in one run, 4 V of them a group; both sums meet at one barrier.
-// Bound by memory: 403 MB at 8192 tokens of 3 x 4096 columns.  A work-group keeps the tables in registers over its tokens, every gridDim.x-th, and asks for the next
-// token's columns before it reduces this one's, so that reads pass while stores do; 16 bytes a lane: 82 us (4.9 TB/s).  8 bytes a lane 101, a work-group for each
-// token with 8 bytes a lane 112.
-template<typename E, typename View, int NV, int V>
-__global__ __launch_bounds__( 1024 ) __attribute__( ( amdgpu_waves_per_eu( 6, 8 ) ) ) void window_append_row_kernel( E* __restrict__ q_out, View y, const E* __restrict__ bias, AppendPart pq, AppendPart pk, AppendPart pv,
-                                                                    WindowRows wr, WindowShape s, float eps, uint32_t rows )
+// prompts (bias and both norms present): work-group = a token's q, k and v together, the columns of the product in one run; all loads go out
+// together and both sums meet at one barrier
+template<typename E, typename View, int NV>
+__global__ __launch_bounds__( 1024 ) void window_append_row_kernel( E* __restrict__ q_out, View y, const E* __restrict__ bias, AppendPart pq, AppendPart pk, AppendPart pv,
+                                                                    WindowRows wr, WindowShape s, float eps )
 {
-  __shared__ float q_sums[2][16], k_sums[2][16];
+  __shared__ float q_sums[16], k_sums[16];
+  const uint64_t row = blockIdx.x;
+  const uint32_t ctx = (uint32_t)( row / wr.n_tokens ), tok = (uint32_t)( row % wr.n_tokens );
+  uint8_t* base = static_cast<uint8_t*>( wr.rows[ctx] );
+  if ( base == nullptr ) {
+    return;
+  }
   const uint32_t cols = pv.first + pv.cols;
   const E *q_norm = static_cast<const E*>( pq.norm ), *k_norm = static_cast<const E*>( pk.norm );
-  typedef typename ProductView<E>::Four Four;
-  constexpr bool KEPT = sizeof( E ) == 2;
-  typename View::Four ahead[NV][V];
-  Four w[NV][V], add[NV][V];
-  uint32_t col[NV];
-  auto fours = []( auto ( &to )[V], const auto* from ) __attribute__( ( always_inline ) ) {
-    struct alignas( sizeof( to ) ) Run
-    {
-      std::remove_reference_t<decltype( to[0] )> f[V];
-    };
-    const Run r = *reinterpret_cast<const Run*>( from );
-#pragma unroll
-    for ( int n = 0; n < V; n++ ) {
-      to[n] = r.f[n];
-    }
-  };
-  auto columns = [&]( typename View::Four ( &to )[V], uint64_t row, uint32_t c ) __attribute__( ( always_inline ) ) {
-    if constexpr ( V == 1 ) {
-      to[0] = y.four( row, c );
-    } else { // (one plane)
-      fours( to, y.data + row * y.stride + c );
-    }
-  };
-  auto read = [&]( uint32_t c ) __attribute__( ( always_inline ) ) { return c < cols ? c : 0; }; // past the row's end: its first ones
+  float4 v[NV], w[NV];
+  float qq = 0.0f, kk = 0.0f;
 #pragma unroll
   for ( int g = 0; g < NV; g++ ) {
-    col[g] = ( g * blockDim.x + threadIdx.x ) * ( 4 * V );
-    if constexpr ( KEPT ) {
-      columns( ahead[g], blockIdx.x, read( col[g] ) );
-    }
+    const uint32_t c = ( g * blockDim.x + threadIdx.x ) * 4, at = c < cols ? c : 0;
+    v[g] = y.at4( row, at );
+    const bool is_q = at < pk.first;
+    w[g] = ProductView<E>::load4( is_q ? q_norm + at : k_norm + ( at < pv.first ? at - pk.first : 0 ) ); // (v: not used)
+    const float4 b = ProductView<E>::load4( bias + at );
+    v[g] = make_float4( v[g].x + b.x, v[g].y + b.y, v[g].z + b.z, v[g].w + b.w );
+    const float sum = c < pv.first ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
+    qq += is_q ? sum : 0.0f;
+    kk += is_q ? 0.0f : sum;
   }
-  auto tables = [&]() __attribute__( ( always_inline ) ) {
+  qq = wave_sum( qq );
+  kk = wave_sum( kk );
+  if ( ( threadIdx.x & 63 ) == 0 ) {
+    q_sums[threadIdx.x >> 6] = qq;
+    k_sums[threadIdx.x >> 6] = kk;
+  }
+  __syncthreads();
+  qq = kk = 0.0f;
+  for ( uint32_t i = 0; i < blockDim.x / WAVE; i++ ) {
+    qq += q_sums[i];
+    kk += k_sums[i];
+  }
+  const float q_inv = 1.0f / sqrtf( qq / (float)pq.cols + eps );
+  const float k_inv = 1.0f / sqrtf( kk / (float)pk.cols + eps );
+  E* q_dst = q_out + row * s.heads * s.dpad;
+  E* k_dst = reinterpret_cast<E*>( base + wr.offset ) + (uint64_t)( wr.start_pos[ctx] + tok ) * s.row_elems();
+  E* v_dst = k_dst + s.k_elems();
 #pragma unroll
-    for ( int g = 0; g < NV; g++ ) {
-      const uint32_t at = read( col[g] );
-      fours( w[g], at < pk.first ? q_norm + at : k_norm + ( at < pv.first ? at - pk.first : 0 ) ); // (v: not used)
-      fours( add[g], bias + at );
+  for ( int g = 0; g < NV; g++ ) {
+    const uint32_t c = ( g * blockDim.x + threadIdx.x ) * 4;
+    if ( c >= cols ) {
+      continue;
     }
-  };
-  if constexpr ( KEPT ) {
-    tables();
+    const bool is_q = c < pk.first, is_v = c >= pv.first;
+    const float inv = is_q ? q_inv : k_inv;
+    const uint32_t local = c - ( is_q ? 0 : is_v ? pv.first : pk.first );
+    const uint32_t dim = is_v ? pv.dim : pq.dim, pad = is_v ? pv.pad : pq.pad;
+    union
+    {
+      E e[4];
+      uint2 half;
+      uint4 full;
+    } o;
+    o.e[0] = from_f32<E>( is_v ? v[g].x : v[g].x * inv * w[g].x );
+    o.e[1] = from_f32<E>( is_v ? v[g].y : v[g].y * inv * w[g].y );
+    o.e[2] = from_f32<E>( is_v ? v[g].z : v[g].z * inv * w[g].z );
+    o.e[3] = from_f32<E>( is_v ? v[g].w : v[g].w * inv * w[g].w );
+    const uint32_t h = pad != dim ? local / dim : 0, e = local - h * dim;
+    E* at = ( is_q ? q_dst : is_v ? v_dst : k_dst ) + (uint64_t)h * pad + e;
+    if constexpr ( sizeof( E ) == 2 ) {
+      *reinterpret_cast<uint2*>( at ) = o.half;
+    } else {
+      *reinterpret_cast<uint4*>( at ) = o.full;
+    }
+    if ( pad != dim && e + 4 == dim ) {
+      for ( uint32_t z = dim; z < pad; z++ ) {
+        at[z - e] = from_f32<E>( 0.0f );
+      }
+    }
   }
-  uint32_t turn = 0;
-  for ( uint32_t row = blockIdx.x; row < rows; row += gridDim.x, turn ^= 1 ) {
+}
+
+// Many tokens of long rows, bf16 in one plane: 16 bytes a lane, 4 V columns a group, and a work-group keeps the tables in registers over its tokens, every gridDim.x-th,
+// and asks for the next token's columns before it reduces this one's, so that reads pass while stores do.  Bound by memory: 403 MB at 8192 tokens of 3 x 4096 columns,
+// 112 us with a work-group for each, 84 so (4.8 TB/s; 82 without the sums' way through LDS, which keeps the order and so the bits of that kernel); 8 bytes a lane and
+// tokens in turn 101.
+__global__ __launch_bounds__( 1024 ) __attribute__( ( amdgpu_waves_per_eu( 6, 8 ) ) ) void window_append_rows_kernel( __bf16* __restrict__ q_out, ProductView<__bf16> y, const __bf16* __restrict__ bias,
+                                                                    AppendPart pq, AppendPart pk, AppendPart pv, WindowRows wr, WindowShape s, float eps, uint32_t rows )
+{
+  constexpr int NV = 2; // groups of eight columns a thread
+  extern __shared__ float fours_sums[]; // of squares, two a group
+  __shared__ float q_sums[16], k_sums[16];
+  const uint32_t cols = pv.first + pv.cols;
+  const __bf16 *q_norm = static_cast<const __bf16*>( pq.norm ), *k_norm = static_cast<const __bf16*>( pk.norm );
+  auto run_at = []( const __bf16* p ) __attribute__( ( always_inline ) ) { return *reinterpret_cast<const uint4*>( p ); };
+  auto wide = []( const uint4& run, int e ) __attribute__( ( always_inline ) ) { return to_f32( reinterpret_cast<const __bf16*>( &run )[e] ); };
+  auto read = [&]( uint32_t c ) __attribute__( ( always_inline ) ) { return c < cols ? c : 0; }; // past the row's end: its first ones
+  uint4 ahead[NV], w[NV], add[NV];
+  uint32_t col[NV];
+#pragma unroll
+  for ( int g = 0; g < NV; g++ ) {
+    col[g] = ( g * blockDim.x + threadIdx.x ) * 8;
+    const uint32_t at = read( col[g] );
+    ahead[g] = run_at( y.data + (uint64_t)blockIdx.x * y.stride + at );
+    w[g] = run_at( at < pk.first ? q_norm + at : k_norm + ( at < pv.first ? at - pk.first : 0 ) ); // (v: not used)
+    add[g] = run_at( bias + at );
+  }
+  for ( uint32_t row = blockIdx.x; row < rows; row += gridDim.x ) {
     const uint32_t ctx = row / wr.n_tokens, tok = row % wr.n_tokens;
     uint8_t* const base = static_cast<uint8_t*>( wr.rows[ctx] );
     const uint32_t pos = wr.start_pos[ctx] + tok;
-    float4 v[NV][V];
-    float qq = 0.0f, kk = 0.0f;
+    const uint32_t next = min( row + gridDim.x, rows - 1 );
+    float v[NV][8];
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) { // (nothing that follows from a group's columns is kept from token to token, and the tables as they are, not as the floats that they make)
       asm volatile( "" : "+v"( col[g] ) );
-    }
-    if constexpr ( KEPT ) {
+      asm volatile( "" : "+v"( w[g].x ), "+v"( w[g].y ), "+v"( w[g].z ), "+v"( w[g].w ), "+v"( add[g].x ), "+v"( add[g].y ), "+v"( add[g].z ), "+v"( add[g].w ) );
 #pragma unroll
-      for ( int g = 0; g < NV; g++ ) {
-#pragma unroll
-        for ( int n = 0; n < V; n++ ) {
-          asm volatile( "" : "+v"( w[g][n].x ), "+v"( w[g][n].y ), "+v"( add[g][n].x ), "+v"( add[g][n].y ) );
-        }
-      }
-    } else {
-#pragma unroll
-      for ( int g = 0; g < NV; g++ ) {
-        columns( ahead[g], row, read( col[g] ) );
-      }
-      tables();
-    }
-#pragma unroll
-    for ( int g = 0; g < NV; g++ ) {
-#pragma unroll
-      for ( int n = 0; n < V; n++ ) {
-        const float4 x = View::wide( ahead[g][n] ), b = ProductView<E>::wide( add[g][n] );
-        v[g][n] = make_float4( x.x + b.x, x.y + b.y, x.z + b.z, x.w + b.w );
-      }
-    }
-    if constexpr ( KEPT ) {
-      const uint32_t next = min( row + gridDim.x, rows - 1 );
-#pragma unroll
-      for ( int g = 0; g < NV; g++ ) {
-        columns( ahead[g], next, read( col[g] ) );
+      for ( int e = 0; e < 8; e++ ) {
+        v[g][e] = wide( ahead[g], e ) + wide( add[g], e );
       }
     }
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) {
-      const bool is_q = col[g] < pk.first;
-      float sum = 0.0f;
+      ahead[g] = run_at( y.data + (uint64_t)next * y.stride + read( col[g] ) );
+    }
 #pragma unroll
-      for ( int n = 0; n < V; n++ ) {
-        sum += col[g] < pv.first ? v[g][n].x * v[g][n].x + v[g][n].y * v[g][n].y + v[g][n].z * v[g][n].z + v[g][n].w * v[g][n].w : 0.0f;
+    for ( int g = 0; g < NV; g++ ) {
+#pragma unroll
+      for ( int e = 0; e < 8; e += 4 ) {
+        const float sum = v[g][e] * v[g][e] + v[g][e + 1] * v[g][e + 1] + v[g][e + 2] * v[g][e + 2] + v[g][e + 3] * v[g][e + 3];
+        fours_sums[( col[g] + e ) / 4] = col[g] < pv.first ? sum : 0.0f;
       }
-      qq += is_q ? sum : 0.0f;
-      kk += is_q ? 0.0f : sum;
+    }
+    __syncthreads();
+    float qq = 0.0f, kk = 0.0f;
+#pragma unroll
+    for ( int g = 0; g < 2 * NV; g++ ) { // in the order of a thread with four columns at a time
+      const uint32_t f = g * blockDim.x + threadIdx.x;
+      const float sum = fours_sums[f];
+      qq += 4 * f < pk.first ? sum : 0.0f;
+      kk += 4 * f < pk.first ? 0.0f : sum;
     }
     qq = wave_sum( qq );
     kk = wave_sum( kk );
     if ( ( threadIdx.x & 63 ) == 0 ) {
-      q_sums[turn][threadIdx.x >> 6] = qq;
-      k_sums[turn][threadIdx.x >> 6] = kk;
+      q_sums[threadIdx.x >> 6] = qq;
+      k_sums[threadIdx.x >> 6] = kk;
     }
-    __syncthreads(); // (the sums of the token after next go where these are: everyone is past the barrier between by then)
+    __syncthreads(); // (and everyone has read the sums of fours; those of the waves are written again behind the next token's first barrier)
     qq = kk = 0.0f;
     for ( uint32_t i = 0; i < blockDim.x / WAVE; i++ ) {
-      qq += q_sums[turn][i];
-      kk += k_sums[turn][i];
+      qq += q_sums[i];
+      kk += k_sums[i];
     }
     if ( base == nullptr ) {
       continue;
     }
     const float q_inv = 1.0f / sqrtf( qq / (float)pq.cols + eps );
     const float k_inv = 1.0f / sqrtf( kk / (float)pk.cols + eps );
-    E* q_dst = q_out + (uint64_t)row * s.heads * s.dpad;
-    E* k_dst = reinterpret_cast<E*>( base + wr.offset ) + (uint64_t)pos * s.row_elems();
-    E* v_dst = k_dst + s.k_elems();
+    __bf16* q_dst = q_out + (uint64_t)row * s.heads * s.dpad;
+    __bf16* k_dst = reinterpret_cast<__bf16*>( base + wr.offset ) + (uint64_t)pos * s.row_elems();
+    __bf16* v_dst = k_dst + s.k_elems();
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) {
       const uint32_t c = col[g];
@@ -263,28 +300,17 @@ __global__ __launch_bounds__( 1024 ) __attribute__( ( amdgpu_waves_per_eu( 6, 8 
       }
       const bool is_q = c < pk.first, is_v = c >= pv.first;
       const float inv = is_q ? q_inv : k_inv;
-      const uint32_t local = c - ( is_q ? 0 : is_v ? pv.first : pk.first );
-      const uint32_t dim = is_v ? pv.dim : pq.dim, pad = is_v ? pv.pad : pq.pad;
-      struct alignas( 4 * V * sizeof( E ) ) Run
+      union
       {
-        E e[4 * V];
+        __bf16 e[8];
+        uint4 run;
       } o;
 #pragma unroll
-      for ( int n = 0; n < V; n++ ) {
-        const float4 f = ProductView<E>::wide( w[g][n] );
-        o.e[4 * n] = from_f32<E>( is_v ? v[g][n].x : v[g][n].x * inv * f.x );
-        o.e[4 * n + 1] = from_f32<E>( is_v ? v[g][n].y : v[g][n].y * inv * f.y );
-        o.e[4 * n + 2] = from_f32<E>( is_v ? v[g][n].z : v[g][n].z * inv * f.z );
-        o.e[4 * n + 3] = from_f32<E>( is_v ? v[g][n].w : v[g][n].w * inv * f.w );
+      for ( int e = 0; e < 8; e++ ) {
+        o.e[e] = from_f32<__bf16>( is_v ? v[g][e] : v[g][e] * inv * wide( w[g], e ) );
       }
-      const uint32_t h = pad != dim ? local / dim : 0, e = local - h * dim;
-      E* at = ( is_q ? q_dst : is_v ? v_dst : k_dst ) + (uint64_t)h * pad + e;
-      *reinterpret_cast<Run*>( at ) = o;
-      if ( pad != dim && e + 4 * V == dim ) {
-        for ( uint32_t z = dim; z < pad; z++ ) {
-          at[z - e] = from_f32<E>( 0.0f );
-        }
-      }
+      // (heads are not padded, as they are a multiple of eight)
+      *reinterpret_cast<uint4*>( ( is_q ? q_dst : is_v ? v_dst : k_dst ) + ( c - ( is_q ? 0 : is_v ? pv.first : pk.first ) ) ) = o.run;
     }
   }
 }
@@ -329,19 +355,20 @@ int launch_append( E* q, const View& y, const E* bias, const void* q_norm, const
   if ( s.dim % 4 == 0 && s.vdim % 4 == 0 && y.stride % 4 == 0 && ( tables & 15u ) == 0 && most <= 32768 ) {
     if ( const uint32_t all = ( nq + nk + nv ) / 4; rows >= 1024 && all <= 4096 && bias != nullptr && q_norm != nullptr && k_norm != nullptr ) {
       const uint32_t threads = std::max<uint32_t>( 64, ( ( all + 3 ) / 4 + 63 ) / 64 * 64 );
-      // work-groups that run at a time (six waves a SIMD), each as many tokens as the others
-      const uint64_t resident = (uint64_t)cu_count() * std::max( 1u, 1536 / threads ), each = ( rows + resident - 1 ) / resident;
-      const unsigned grid_rows = (unsigned)( ( rows + each - 1 ) / each );
-      const uintptr_t runs = reinterpret_cast<uintptr_t>( y.data ) | reinterpret_cast<uintptr_t>( q );
-      bool wide = false;
+      bool in_turn = false;
       if constexpr ( std::is_same_v<View, ProductView<__bf16>> ) { // one plane
-        wide = s.dim % 8 == 0 && s.vdim % 8 == 0 && y.stride % 8 == 0 && ( runs & 15u ) == 0;
-        if ( wide ) {
-          window_append_row_kernel<E, View, 2, 2><<<grid_rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps, (uint32_t)rows );
+        // Work-groups that run at a time (six waves a SIMD), each as many tokens as the others: at least six, and long rows.  One token a work-group and several, the call:
+        // 3 x 4096 columns at 2048, 3072 and 8192 tokens 44.2, 57.1 and 172 us and 44.2, 56.7 and 146; 10240 at 3072 and 8192 56.5 and 164, 55.9 and 141; 9216 at 8192
+        // 108.8 and 110; 6144 at 4096 and 32768 47.2 and 321, 49.9 and 347.
+        const uint64_t resident = (uint64_t)cu_count() * std::max( 1u, 1536 / threads ), each = ( rows + resident - 1 ) / resident;
+        const uintptr_t runs = reinterpret_cast<uintptr_t>( y.data ) | reinterpret_cast<uintptr_t>( q );
+        in_turn = all >= 2560 && each >= 6 && s.dim % 8 == 0 && s.vdim % 8 == 0 && y.stride % 8 == 0 && ( runs & 15u ) == 0;
+        if ( in_turn ) {
+          window_append_rows_kernel<<<(unsigned)( ( rows + each - 1 ) / each ), threads, 4 * threads * sizeof( float ), st>>>( q, y, bias, pq, pk, pv, wr, s, eps, (uint32_t)rows );
         }
       }
-      if ( !wide ) {
-        window_append_row_kernel<E, View, 4, 1><<<grid_rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps, (uint32_t)rows );
+      if ( !in_turn ) {
+        window_append_row_kernel<E, View, 4><<<(unsigned)rows, threads, 0, st>>>( q, y, bias, pq, pk, pv, wr, s, eps );
       }
       GH_LAUNCH_CHECK();
       return GH_OK;

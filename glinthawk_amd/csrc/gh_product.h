@@ -150,16 +150,8 @@ struct ProductView
     }
     return sum;
   }
-  // four neighbouring columns as they lie in memory, where there is one plane: a load that nothing has to wait for before the values are asked for
+  // four neighbouring columns as they lie in memory: a load that nothing has to wait for before the values are asked for
   typedef std::conditional_t<sizeof( S ) == 2, uint2, float4> Four;
-  __device__ __forceinline__ Four four( uint64_t row, uint64_t col ) const
-  {
-    if constexpr ( sizeof( S ) == 2 ) {
-      return *reinterpret_cast<const uint2*>( data + row * stride + col );
-    } else {
-      return at4( row, col );
-    }
-  }
   static __device__ __forceinline__ float4 wide( const Four& f )
   {
     if constexpr ( sizeof( S ) == 2 ) {

@@ -93,3 +93,26 @@ def few_rows_bits(s, b, r):
 @pytest.mark.parametrize("shape", FEW_ROWS)
 def test_product_of_few_weight_rows(shape):
     assert few_rows_bits(*shape) == FEW_ROWS[shape]
+
+
+# (heads, kv heads, head sizes), tokens: a work-group for each, rows that end inside a group of threads, padded heads; long rows of many tokens, several a work-group
+APPEND = {(32, 32, 128, 128, 521): 3915238599, (40, 8, 128, 64, 700): 3069143961, (25, 5, 104, 72, 900): 2630354648, (60, 20, 52, 36, 611): 3883644428,
+          (4, 4, 64, 64, 1000): 1073606430, (32, 32, 128, 128, 1100): 1240766657, (64, 16, 128, 40, 1301): 2555571595}
+
+
+def append_bits(heads, kv, d, dv, T):
+    """q, then what two contexts were appended; the tokens of a third one are passed over."""
+    import torch
+    from glinthawk_amd import ops
+    rng = np.random.default_rng(heads + T)
+    a, n = ops.window_attn(heads, kv, d, dv, 1.0, 9, 2, 5), heads * d + kv * (d + dv)
+    x, w = (torch.from_numpy(rng.integers(-3, 4, s).astype(np.float32)).cuda().bfloat16() for s in ((3 * T, 16), (n, 16)))     # products below 256: exact
+    b, qn, kn = draw(rng, n, 3), draw(rng, heads * d, 2) / 4 + 1, draw(rng, kv * d, 2) / 4 + 1
+    region = [torch.zeros((T + 11, ops.window_row_bytes(a, torch.bfloat16) // 2), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    table, start = ops.row_table([region[0].data_ptr(), 0, region[1].data_ptr()]), torch.tensor([3, 0, 11], dtype=torch.int32, device="cuda")
+    return checksum(ops.matmul_window_append(x, w, a, table, start, T, b, qn, kn, 2e-3), *region)
+
+
+@pytest.mark.parametrize("shape", APPEND)
+def test_query_key_norm_and_append(shape):
+    assert append_bits(*shape) == APPEND[shape]

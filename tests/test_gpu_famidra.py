@@ -476,9 +476,10 @@ def test_query_key_norm_and_append(dtype, n_tokens):
         assert (c == 7.0).all(), "rows outside the call were written"
 
 
-# work-groups that take several tokens each, some one less; 16 bytes and 8 at a time, padded heads, more heads than keys have, a row that ends inside a group
+# padded heads, more heads than keys have, a row that ends inside a group; long rows of many tokens, which work-groups take in turn, some one less
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 521), (40, 8, 128, 64, 1111), (60, 20, 52, 36, 1301), (25, 5, 104, 72, 1201)])
+@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 521), (40, 8, 128, 64, 1111), (60, 20, 52, 36, 1301), (25, 5, 104, 72, 1201), (32, 32, 128, 128, 1100),
+                                                    (64, 16, 128, 40, 1301)])
 def test_query_key_norm_and_append_of_many_tokens(dtype, heads, kv, d, dv, n_tokens):
     """Three contexts, the second without one: its tokens are passed over.  Against 64 bits, bound as above."""
     import torch
