@@ -276,13 +276,13 @@ __device__ __forceinline__ uint32_t rounded_pair( float a, float b )
   }
 }
 
-// y / (1 + exp(-z)), of a gate.  The divisor is at least 1 and, where the quotient does not vanish, below 2^126, so its reciprocal (one Newton step) and the
-// quotient's remainder need no scaling, and the exponential none below the smallest normal number, which leaves 1 as it is: 12 instructions where the
-// general division and exponential take 18.  The quotient is the general one's; -87 and less give 0.
+// y / (1 + exp(-z)), of a gate.  The divisor is at least 1, so the quotient needs no scaling but for the reciprocal of a divisor of 2^126 and more (z below -126 ln 2 =
+// -87.34), which would be subnormal and given as 0; and the exponential needs none below the smallest normal number, which leaves 1 as it is: 14 instructions where the
+// general division and exponential take 18.  The quotient is the general one's.
 __device__ __forceinline__ float sigmoid_times( float y, float z )
 {
   const float d = 1.0f + __builtin_amdgcn_exp2f( z * -1.44269504088896340736f );
-  const float r0 = __builtin_amdgcn_rcpf( d ), r = __builtin_fmaf( __builtin_fmaf( -d, r0, 1.0f ), r0, r0 );
+  const float r0 = 0.25f * __builtin_amdgcn_rcpf( 0.25f * d ), r = __builtin_fmaf( __builtin_fmaf( -d, r0, 1.0f ), r0, r0 );
   const float q = y * r;
   return __builtin_amdgcn_div_fixupf( __builtin_fmaf( __builtin_fmaf( -d, q, y ), r, q ), d, y ); // (infinities and NaN)
 }

@@ -307,8 +307,8 @@ def test_matmul_gate_of_whole_tiles(b, s, hidden, bias, activation):
                                                 (torch.bfloat16, ops.GH_ACT_GELU_TANH, False)])
 def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
     """Factors that are one weight each, so that the sums are exact: over the range of the exponential, signed zeros, the type's smallest and largest,
-    infinities and NaN, against 64 bits.  One rounding to the type, and the exponent's own, 2^-23 of its 127 at most; below 2^-119 (f16: its smallest) nothing is asked
-    but the size: from a divisor of 2^126 on, at factors of -87.3 and less, the reciprocal may be 0, and the quotient is at most 88.8 * 2^-126."""
+    infinities and NaN, against 64 bits.  One rounding to the type, and the exponent's own, 2^-23 of its 127 at most; from factors of -128 ln 2 on, where the divisor
+    overflows, and below f16's smallest nothing is asked but the size."""
     lim = torch.finfo(dt)
     a = torch.cat([torch.linspace(-130.0, 130.0, 521), torch.tensor([0.0, -0.0, lim.tiny, -lim.tiny, lim.max, lim.min, float("inf"), -float("inf"), float("nan")]),
                    torch.logspace(-6, 4, 101), -torch.logspace(-6, 4, 101)]).to(dt).cuda()
@@ -335,7 +335,7 @@ def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
         assert torch.equal(row.isnan(), exact.isnan())
         assert torch.equal(row[exact.isinf()], exact[exact.isinf()])
         eps = (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 127 * 2.0 ** -23 + (3 * 2.0 ** -23 * z.abs().clamp(max=130.0))
-        small = lim.tiny * 2.0 ** -10 if dt == torch.float16 else 2.0 ** -119
+        small = lim.tiny * 2.0 ** -10 if dt == torch.float16 else 128 * 0.6932 * 2.0 ** -128
         assert ((row - exact).abs() <= eps * exact.abs() + small)[finite].all()
 
 
