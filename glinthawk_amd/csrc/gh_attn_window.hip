@@ -712,13 +712,6 @@ typedef Mfma<__bf16>::x8 bf16x8;
 
 __device__ __forceinline__ uint32_t shared_swizzle( uint32_t row ) { return ( ( row & 3 ) << 2 ) | ( ( row >> 2 ) & 3 ); }
 
-// two values rounded to bf16, the first in the low half
-__device__ __forceinline__ uint32_t bf16_pair( float a, float b )
-{
-  typedef __bf16 pair_t __attribute__( ( ext_vector_type( 2 ) ) );
-  return __builtin_bit_cast( uint32_t, pair_t { (__bf16)a, (__bf16)b } );
-}
-
 // KS: steps of 16 of the query/key size; VB: blocks of 32 of the value size
 template<int KS, int VB, bool SHARED>
 __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf16> out,
@@ -985,9 +978,9 @@ __global__ __launch_bounds__( 256, 2 ) void window_tiles_kernel( WindowOut<__bf1
         const float p1 = __builtin_amdgcn_exp2f( st[kk >> 1][8 * ( kk & 1 ) + 2 * e + 1] - m );
         l += p0;
         l += p1;
-        hi.pair[e] = bf16_pair( p0, p1 );
+        hi.pair[e] = rounded_pair<__bf16>( p0, p1 );
         asm( "" : "+v"( hi.pair[e] ) ); // (taken apart again below: the compiler would convert the two once more instead)
-        lo.pair[e] = bf16_pair( p0 - __builtin_bit_cast( float, hi.pair[e] << 16 ), p1 - __builtin_bit_cast( float, hi.pair[e] & 0xffff0000u ) );
+        lo.pair[e] = rounded_pair<__bf16>( p0 - __builtin_bit_cast( float, hi.pair[e] << 16 ), p1 - __builtin_bit_cast( float, hi.pair[e] & 0xffff0000u ) );
       }
 #pragma unroll
       for ( int vp = 0; vp < VB; vp += 2 ) { // (two blocks in turn: a product that waits for the one before it leaves the matrix unit idle)

@@ -339,6 +339,25 @@ def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
         assert ((row - exact).abs() <= eps * exact.abs() + small)[finite].all()
 
 
+@pytest.mark.parametrize("b,hidden", [(512, 16384), (500, 16280)])
+def test_gate_of_tiles_and_of_stored_factors(b, hidden):
+    """f16: the product of gate and factor is rounded as every other route rounds it, to the bit.  A sum is one product of two values here, so the factors are known.  Of
+    these outputs 6.4e-5 are not the correctly rounded ones, with v_fma_mixlo_f16 in the place of a multiplication and a conversion 8.4e-5."""
+    g = torch.Generator(device="cuda").manual_seed(b)
+    w, x = torch.zeros((2 * hidden, 128), device="cuda", dtype=torch.float16), torch.zeros((b, 128), device="cuda", dtype=torch.float16)
+    w[:, 0], x[:, 0] = torch.randn(2 * hidden, generator=g, device="cuda").half(), torch.randn(b, generator=g, device="cuda").half() * 2
+    factors = (x[:, :1].float() * w[:, 0].float()).half()
+    want = factors[:, :hidden].contiguous()
+    ops.silu(want, factors[:, hidden:].contiguous())
+    lib = _lib.lib()
+    _lib.check(lib.gh_gemm_set_tuning(4, 0, 0))
+    try:
+        got = ops.matmul_silu_gate(x, w)
+    finally:
+        _lib.check(lib.gh_gemm_set_tuning(0, 0, 0))
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dt", [torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [Shape(dim=32, n_layers=1, n_heads=4, n_kv_heads=2, hidden_dim=48, seq_len=16),
                                    Shape(dim=288, n_layers=1, n_heads=6, n_kv_heads=6, hidden_dim=768, seq_len=256),
