@@ -94,8 +94,8 @@ __device__ __forceinline__ float4 load4_e( const void* p, uint32_t c )
 }
 
 // Four of a row's weights for each group of a thread, asked for at the kernel's start (EARLY, as they lie in memory, so that nothing waits for them): behind a norm's
-// barrier each table is one more round trip with nothing beside it (8192 rows of 4096: 68 -> 64.5 us, 6.2 TB/s).  Where the registers would cost work-groups in
-// flight, there all the same; and where stores go out before the norm, which the loads would hold up (embeddings of 8192 rows 44.5 us, 48 with early weights).
+// barrier each table is one more round trip with nothing beside it (8192 rows of 4096: 68 -> 64.5 us, 6.2 TB/s).  Not where stores go out before the norm, which the
+// loads would hold up (embeddings of 8192 rows 44.5 us, 48 with early weights), and not in fp32 (32 rows of 4096 16.2 us, 16.5).
 template<typename E, int NV, bool EARLY>
 struct StepWeights
 {
@@ -124,8 +124,6 @@ struct StepWeights
     }
   }
 };
-template<typename E, int NV>
-using NormWeights = StepWeights<E, NV, NV * sizeof( E ) <= 8>;
 
 // what a step leaves for the next product: the row, normed where there is a norm
 template<typename E, int NV, typename Weights>
@@ -173,7 +171,7 @@ __device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_
 }
 
 // A thread owns NV groups of four columns.  A group past the row's end reads group 0 and stores nothing: no load sits under a branch.
-template<typename E, typename View, bool PRODUCT, int NV>
+template<typename E, typename View, bool PRODUCT, int NV, bool EARLY>
 __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict__ x, View y, uint32_t width, StepPtrs p )
 {
   __shared__ float s_post[16], s_next[16];
@@ -189,10 +187,10 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
     col[g] = live[g] ? c : 0;
     old[g] = *reinterpret_cast<const float4*>( xr + col[g] );
   }
-  const NormWeights<E, NV> next( p.next_norm, col );
+  const StepWeights<E, NV, EARLY> next( p.next_norm, col );
   if constexpr ( PRODUCT ) {
-    const NormWeights<E, NV> post( p.post_norm, col );
-    const StepWeights<E, NV, NV <= 2> add( p.add, col );
+    const StepWeights<E, NV, EARLY> post( p.post_norm, col );
+    const StepWeights<E, NV, EARLY && NV <= 2> add( p.add, col );
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) {
       v[g] = y.at4( row, col[g] );
@@ -377,7 +375,18 @@ int launch_step( float* x, const View& y, uint64_t width, uint64_t rows, const S
   const uint32_t groups = w / 4;
   const uint32_t threads = step_threads( groups, rows );
   with_groups( ( groups + threads - 1 ) / threads, [&]( auto nv ) {
-    stream_step_kernel<E, View, PRODUCT, decltype( nv )::value><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
+    constexpr int NV = decltype( nv )::value;
+    // Weights asked for early take registers: six waves a SIMD instead of eight.  Where eight hold all of a call, but six no longer do, or hardly, that is slower: without a
+    // norm behind the product 2000 rows of 4096 22.9 us, 24.1 with early weights, 6000 of 1024 18.3 and 19.2; 4000 of 1024 15.1 and 14.5, 3000 of 4096 34.6 and 33.4;
+    // and with a thread for each group of columns, 1000 rows of 4096 17.1 and 17.5.
+    const uint64_t waves = rows * ( threads / WAVE ), cus = cu_count();
+    if constexpr ( sizeof( E ) == 2 && NV <= 4 ) {
+      if ( waves <= 20 * cus || ( NV > 1 && waves > 32 * cus ) ) {
+        stream_step_kernel<E, View, PRODUCT, NV, true><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
+        return;
+      }
+    }
+    stream_step_kernel<E, View, PRODUCT, NV, false><<<(unsigned)rows, threads, 0, st>>>( x, y, w, p );
   } );
   GH_LAUNCH_CHECK();
   return GH_OK;
