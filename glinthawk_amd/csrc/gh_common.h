@@ -262,6 +262,15 @@ __device__ __forceinline__ __bf16 from_f32<__bf16>( float v )
   return (__bf16)v; // to nearest even
 }
 
+// Sum of the squares of four columns.  The order is written out: left to the compiler it begins with the first or the second column, as the code around it happens to be,
+// and the last bits of a norm move with it, of which a model's later layers make far more.  FIRST: it begins with the first.
+template<bool FIRST>
+__device__ __forceinline__ float squares( const float4 v )
+{
+  const float two = FIRST ? __builtin_fmaf( v.y, v.y, v.x * v.x ) : __builtin_fmaf( v.x, v.x, v.y * v.y );
+  return __builtin_fmaf( v.w, v.w, __builtin_fmaf( v.z, v.z, two ) );
+}
+
 // two values rounded as one instruction takes them, to nearest even: a in the low half
 template<typename E>
 __device__ __forceinline__ uint32_t rounded_pair( float a, float b )

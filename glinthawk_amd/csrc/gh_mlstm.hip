@@ -965,7 +965,7 @@ __global__ __launch_bounds__( 256 ) void mlstm_finish_kernel( E* __restrict__ ou
 #pragma unroll
     for ( int k = 0; k < 4; k++ ) {
       v[k].x *= over, v[k].y *= over, v[k].z *= over, v[k].w *= over;
-      ss += ( k * 64 + lane ) * 4 < s.vdim ? v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w : 0.0f;
+      ss += ( k * 64 + lane ) * 4 < s.vdim ? squares<false>( v[k] ) : 0.0f;
     }
     const float inv = 1.0f / sqrtf( wave_sum( ss ) / (float)s.vdim + s.eps );
 #pragma unroll

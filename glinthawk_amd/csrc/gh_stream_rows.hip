@@ -125,8 +125,8 @@ struct StepWeights
   }
 };
 
-// what a step leaves for the next product: the row, normed where there is a norm
-template<typename E, int NV, typename Weights>
+// what a step leaves for the next product: the row, normed where there is a norm; FIRST: order of the squares
+template<typename E, int NV, bool FIRST, typename Weights>
 __device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_t ( &col )[NV], const bool ( &live )[NV], const Weights& next, uint64_t row, uint32_t width,
                                           const StepPtrs& p, float* s_next )
 {
@@ -138,7 +138,7 @@ __device__ __forceinline__ void step_out( const float4 ( &v )[NV], const uint32_
     float ss = 0.0f;
 #pragma unroll
     for ( int g = 0; g < NV; g++ ) {
-      ss += live[g] ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
+      ss += live[g] ? squares<FIRST>( v[g] ) : 0.0f;
     }
     inv = 1.0f / sqrtf( row_sum( ss, s_next ) / (float)width + p.eps );
   }
@@ -206,7 +206,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
       float ss = 0.0f;
 #pragma unroll
       for ( int g = 0; g < NV; g++ ) {
-        ss += live[g] ? v[g].x * v[g].x + v[g].y * v[g].y + v[g].z * v[g].z + v[g].w * v[g].w : 0.0f;
+        ss += live[g] ? squares<NV == 1>( v[g] ) : 0.0f;
       }
       const float inv = 1.0f / sqrtf( row_sum( ss, s_post ) / (float)width + p.eps );
 #pragma unroll
@@ -235,7 +235,7 @@ __global__ __launch_bounds__( 1024 ) void stream_step_kernel( float* __restrict_
       v[g] = old[g];
     }
   }
-  step_out<E, NV>( v, col, live, next, row, width, p, s_next );
+  step_out<E, NV, PRODUCT && NV == 1>( v, col, live, next, row, width, p, s_next );
 }
 
 // any width: the row goes through memory between the passes (each thread re-reads only what it wrote)
@@ -337,7 +337,7 @@ __global__ __launch_bounds__( 1024 ) void embed_step_kernel( float* __restrict__
       }
     }
   }
-  step_out<E, NV>( v, col, live, StepWeights<E, NV, false>( p.next_norm, col ), row, width, p, s_next ); // (the stores above go out first)
+  step_out<E, NV, NV == 1>( v, col, live, StepWeights<E, NV, false>( p.next_norm, col ), row, width, p, s_next ); // (the stores above go out first)
 }
 
 // Threads to a row of `groups` groups of four columns: many rows, fewer threads with more of the row each; few rows, the row over as many threads as it has groups.

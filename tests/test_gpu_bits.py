@@ -116,3 +116,51 @@ def append_bits(heads, kv, d, dv, T):
 @pytest.mark.parametrize("shape", APPEND)
 def test_query_key_norm_and_append(shape):
     assert append_bits(*shape) == APPEND[shape]
+
+
+# rows, width, dtype, a norm behind the product: a thread for each group of columns with work-groups beyond those in flight, and few rows; more groups a thread
+STEP = {(700, 4096, "bfloat16", True): 3824987965, (999, 4096, "bfloat16", False): 2599642962, (33, 4096, "bfloat16", True): 1377173294,
+        (1300, 2048, "bfloat16", True): 3409561444, (600, 1024, "float32", True): 706433486, (1100, 4096, "float32", True): 3856038900}
+
+
+def step_bits(rows, width, dtype, post):
+    """The residual stream, then the normed rows."""
+    import torch
+    from glinthawk_amd import ops
+    rng = np.random.default_rng(rows)
+    inp, w = (torch.from_numpy(rng.integers(-3, 4, s).astype(np.float32)).cuda().to(getattr(torch, dtype)) for s in ((rows, 16), (width, 16)))
+    x, bias, norms = draw(rng, (rows, width), 9, "float32"), draw(rng, width, 3, dtype), [draw(rng, width, 2, dtype) / 4 + 1 for _ in range(2)]
+    out = torch.empty((rows, width), dtype=inp.dtype, device="cuda")
+    ops.matmul_stream(x, inp, w, 1e-4, bias=bias, post_norm=norms[0] if post else None, next_norm=norms[1], out=out)
+    return checksum(x, out)
+
+
+@pytest.mark.parametrize("shape", STEP)
+def test_residual_step(shape):
+    assert step_bits(*shape) == STEP[shape]
+
+
+# heads, head sizes, contexts, dtype: tokens one after the other
+MLSTM_STEP = {(4, 16, 512, 300, "bfloat16"): 9421239, (4, 16, 512, 300, "float32"): 2747313704, (2, 24, 1024, 150, "bfloat16"): 2003180597, (3, 16, 40, 500, "float32"): 1522406068}
+
+
+def mlstm_step_bits(H, d, dv, B, dtype):
+    """Three tokens of every context: outputs, then the state."""
+    import torch
+    from glinthawk_amd import ops
+    from glinthawk_amd._lib import GhMlstm
+    rng, dt = np.random.default_rng(d + dv), getattr(torch, dtype)
+    m, width = GhMlstm(H, d, dv, 15.0, 1e-4), 8
+    rows, gate_row = ops.mlstm_weight_rows(m)
+    w = rng.integers(-2, 3, (rows, width)) * np.where(np.arange(rows) >= gate_row, 0.5, 1.0)[:, None]
+    w, x = torch.from_numpy(w.astype(np.float32)).cuda().to(dt), torch.from_numpy(rng.integers(-1, 2, (3, B, width)).astype(np.float32)).cuda().to(dt)
+    bias_i, bias_f, norm = draw(rng, H, 0, dtype), draw(rng, H, 0, dtype) + 3, draw(rng, H * dv, 0, dtype) / 8 + 1
+    state = torch.zeros((B, ops.mlstm_state_bytes(m) // 4), device="cuda")
+    table = ops.row_table([s.data_ptr() for s in state])
+    out = [ops.mlstm_forward(x[t], w, m, bias_i, bias_f, norm, table, torch.full((B,), t, dtype=torch.int32, device="cuda"), 1) for t in range(3)]
+    return checksum(*out, state)
+
+
+@pytest.mark.parametrize("shape", MLSTM_STEP)
+def test_mlstm_step(shape):
+    assert mlstm_step_bits(*shape) == MLSTM_STEP[shape]
