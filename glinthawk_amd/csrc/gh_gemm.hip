@@ -426,11 +426,10 @@ static bool tile256_wanted( uint64_t s, uint64_t r, uint64_t b, const void* x, c
 }
 
 // Tokens of the first part when a product, `whole_ns` in one, is better run as whole rounds of 256 x 256 tiles and a rest, rest_ns( tokens ); 0 otherwise.
-// `whole_ns` becomes what the choice needs.
 template<typename F>
-static uint64_t cut_tokens( uint64_t s, uint64_t r, uint64_t b, double& whole_ns, F&& rest_ns )
+static uint64_t cut_tokens( uint64_t s, uint64_t r, uint64_t b, double whole_ns, F&& rest_ns )
 {
-  double& best = whole_ns;
+  double best = whole_ns;
   uint64_t best_b1 = 0;
   const uint64_t rounds = gemm_tile256_rounds( r, b );
   for ( uint64_t n = 1; n < 3 && n < rounds; n++ ) { // the first part one round shorter, or two
@@ -453,18 +452,7 @@ uint64_t gemm_token_split( uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, cons
   if ( !is_half_type( dt ) || g_force_kernel != 0 || !gemm_tile256_takes( s, b, x, w, xout ) ) {
     return 0;
   }
-  double ns = half_plan( s, r, b, true ).ns;
-  return cut_tokens( s, r, b, ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
-}
-
-// what a rounded product is estimated to need, aligned operands
-static double product_ns( uint64_t s, uint64_t r, uint64_t b )
-{
-  double ns = half_plan( s, r, b, true ).ns;
-  if ( gemm_tile256_takes( s, b, nullptr, nullptr, nullptr ) ) {
-    cut_tokens( s, r, b, ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
-  }
-  return ns;
+  return cut_tokens( s, r, b, half_plan( s, r, b, true ).ns, [&]( uint64_t rest ) { return half_plan( s, r, rest, false ).ns; } );
 }
 
 // Which kernel takes w1, w3 and the gate in one launch (what is left of it once gemm_token_split() has cut it); none: two launches.
@@ -610,17 +598,6 @@ static bool skinny_takes( uint64_t s, uint64_t r, uint64_t b, const void* x, con
 {
   return g_force_kernel == 0 && r <= SKINNY_ROWS && b >= 192 && b < ( 1ull << 31 ) && s % 256 == 0
          && ( ( reinterpret_cast<uintptr_t>( x ) | reinterpret_cast<uintptr_t>( w ) ) & 15u ) == 0;
-}
-
-// Whether the last `few` rows of a rounded product of r are better a product of their own: where the others fill rounds of 256 x 256 tiles that all of them
-// overflow.  8192 + 32 rows of 4096 k at 8192 activation rows: 360 us and 39 for the tokens that are left over, against 360 and 20 (the whole prefill of 4 x 2048 tokens 4910 -> 4748 us).
-bool gemm_few_rows_apart( uint64_t s, uint64_t r, uint64_t few, uint64_t b, gh_dtype dt, const void* x, const void* w )
-{
-  if ( !is_half_type( dt ) || few == 0 || few >= r || !gemm_ring_applicable( s, r, b, x, w, x ) || !skinny_takes( s, few, b, x, static_cast<const char*>( w ) + ( r - few ) * s * 2 ) ) {
-    return false;
-  }
-  const double skinny_ns = 5000.0 + (double)( b * s ) * 2.0 / 4000.0;
-  return product_ns( s, r, b ) > product_ns( s, r - few, b ) + skinny_ns;
 }
 
 // The 16-bit part of gemm_partials(): runs the GEMM proper.  With `want_partials` the result is always left as fp32 partial sums

@@ -41,7 +41,6 @@ struct ParallelOut
   uint64_t hidden_stride;
   uint32_t ff;
   int act;
-  const float* gates; // (rows, heads), the product of the head gates where it is one of its own; NULL: columns of `y`
 };
 
 template<typename E>
@@ -162,7 +161,7 @@ __global__ __launch_bounds__( 256 ) void parallel_rows_kernel( ParallelOut<E> o,
       factor *= 1.0f + u.temp_coef * logf( (float)( ( pos + 1 ) / u.temp_every ) + 1.0f );
     }
     if ( o.head_gates != nullptr && lane == 0 ) {
-      o.head_gates[row * s.heads + unit] = sigmoid<E>( o.gates != nullptr ? o.gates[row * s.heads + unit] : y.at( row, cols.g + unit ) );
+      o.head_gates[row * s.heads + unit] = sigmoid<E>( y.at( row, cols.g + unit ) );
     }
   } else {
     const uint32_t g = unit - s.heads;
@@ -263,25 +262,14 @@ int gh_matmul_parallel( void* q, float* head_gates, void* hidden, uint64_t hidde
       cols.r = cols.ff;
     }
   }
-  // many rows with the heads alone: the gates apart where they are too much for the others' rounds of tiles
-  const uint64_t apart = head_gates != nullptr && ff == 0 && cols.r > cols.g && rows >= PRODUCT_ROUNDED_ROWS
-                             && gemm_few_rows_apart( width, cols.r, cols.r - cols.g, rows, dt, x, w )
-                           ? s.heads
-                           : 0;
-  Product y, gates;
-  if ( int rc = make_product( x, w, width, apart ? cols.g : cols.r, rows, dt, false, st, &y ) ) {
+  Product y;
+  if ( int rc = make_product( x, w, width, cols.r, rows, dt, false, st, &y ) ) {
     return rc;
   }
-  if ( apart ) { // (one plane of fp32 sums)
-    if ( int rc = make_product( x, static_cast<const char*>( w ) + (uint64_t)cols.g * width * dtype_size( dt ), width, apart, rows, dt, true, st, &gates ) ) {
-      return rc;
-    }
-  }
-  const float* gate_sums = apart ? static_cast<const float*>( gates.data ) : nullptr;
   const WindowRows wr { context_rows_dev, cache_offset, factor_offset, start_pos_dev, n_tokens };
   return with_product( dt, y, [&]( auto tag, auto view ) -> int {
     using E = decltype( tag );
-    const ParallelOut<E> o { static_cast<E*>( q ), head_gates, static_cast<E*>( hidden ), hidden_stride, (uint32_t)ff, activation, gate_sums };
+    const ParallelOut<E> o { static_cast<E*>( q ), head_gates, static_cast<E*>( hidden ), hidden_stride, (uint32_t)ff, activation };
     return launch_parallel<E>( o, view, wr, s, *u, cols, rows, st );
   } );
 }

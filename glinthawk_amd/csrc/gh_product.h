@@ -9,7 +9,6 @@
 
 namespace gh {
 
-bool gemm_few_rows_apart( uint64_t s, uint64_t r, uint64_t few, uint64_t b, gh_dtype dt, const void* x, const void* w );
 int gemm_partials( void* xout, const void* x, const void* w, uint64_t s, uint64_t r, uint64_t b, gh_dtype dt, hipStream_t st, bool want_partials,
                    float** partial_out, uint32_t* splits_out );
 

@@ -164,3 +164,27 @@ def mlstm_step_bits(H, d, dv, B, dtype):
 @pytest.mark.parametrize("shape", MLSTM_STEP)
 def test_mlstm_step(shape):
     assert mlstm_step_bits(*shape) == MLSTM_STEP[shape]
+
+
+# heads, key heads, tokens of a context, width: columns that overflow whole rounds of tiles by the heads' gates, with a ragged last tile; few rows
+PARALLEL = {(32, 32, 4096, 2048): 1705321414, (32, 32, 667, 4096): 3510089885, (28, 4, 8150, 512): 498023561, (5, 5, 40, 256): 483779571}
+
+
+def parallel_bits(heads, kv, T, width):
+    """Queries, gates and what two contexts were appended, the tokens of a third one passed over; products are exact in any order."""
+    import torch
+    from glinthawk_amd import ops
+    rng, d, keys = np.random.default_rng(heads + T), 128, -(-T // 32) * 32
+    a = ops.window_attn(heads, kv, d, d, 1.0, values_are_keys=True)
+    n, _ = ops.parallel_weight_rows(a, True, 0)
+    x, w = (torch.from_numpy(rng.integers(-3, 4, s).astype(np.float32)).cuda().bfloat16() for s in ((3 * T, width), (n, width)))
+    at = keys * kv * d * 2
+    region = [torch.zeros(at + keys * kv * 4, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    start = torch.zeros(3, dtype=torch.int32, device="cuda")
+    q, gates = ops.matmul_parallel(x, w / 64, a, ops.row_table([region[0].data_ptr(), 0, region[1].data_ptr()]), start, T, 1e-3, 0.1, 512, True, None, factor_offset=at)
+    return checksum(q, gates, *region)
+
+
+@pytest.mark.parametrize("shape", PARALLEL)
+def test_heads_of_a_parallel_layer(shape):
+    assert parallel_bits(*shape) == PARALLEL[shape]
