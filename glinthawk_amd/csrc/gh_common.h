@@ -21,6 +21,7 @@ int fail( int status, const char* fmt, ... ) __attribute__( ( format( printf, 2,
   do {                                                                                                                 \
     hipError_t gh_err_ = ( expr );                                                                                     \
     if ( gh_err_ != hipSuccess ) {                                                                                     \
+      (void)hipGetLastError(); /* reported here, and not by the next launch's check as well */                         \
       return ::gh::fail( gh_err_ == hipErrorOutOfMemory ? GH_ERR_OOM : GH_ERR_DEVICE,                                  \
                          "%s failed: %s (%s:%d)",                                                                      \
                          #expr,                                                                                        \

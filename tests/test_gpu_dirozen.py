@@ -488,6 +488,30 @@ def test_logits_of_earlier_steps_stay(models):
     assert_logits(np.concatenate([c[:1] for c in copies] + [kept[:1]]), want[0][:10], "f32")
 
 
+def test_logits_without_page_locked_memory(models, monkeypatch):
+    """Memory that cannot be had is an error of that call alone, and a stage whose page-locked arrays are refused takes pageable ones."""
+    import torch
+    from glinthawk_amd import ops, stage
+    from glinthawk_amd._lib import GlintError
+
+    class Refused(stage._PinnedResults):
+        def __init__(self, n_bytes, count):
+            super().__init__(1 << 60, count)
+
+    with pytest.raises(GlintError):
+        ops.pinned_empty((1 << 60,), np.uint8)
+    x, out = torch.ones((2, 8), device="cuda"), torch.zeros((2, 8), device="cuda")
+    ops.stream_out(x, out)
+    assert torch.equal(x, out)
+    monkeypatch.setattr(stage, "_PinnedResults", Refused)
+    path, _, _, seqs, want, _ = models(NAMES[0])
+    st = open_stage(path, "f32")
+    assert st._results.take(1, 1) is None
+    got = [decode_step(st, [1], [int(seqs[0][i])], [i]) for i in range(4)]
+    assert_logits(np.concatenate(got), want[0][:4], "f32")
+    st.close()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_far_token(tmp_path, dtype):
     """A token that reads one other token, hundreds of positions away: in a prompt, decoded, and behind portions that end next to either."""
