@@ -60,8 +60,7 @@ def assert_logits(got, want, dtype, what=""):
 
 
 # ---- mechanisms alone ----------------------------------------------------------------------------
-@pytest.mark.parametrize("b,s,r", [(1, 64, 40), (3, 52, 17), (7, 256, 512), (70, 136, 200), (200, 256, 384), (300, 512, 2048), (200, 512, 8), (333, 1024, 24), (1030, 2048, 32), (2048, 1024, 8192),
-                                   (200, 256, 8), (225, 768, 17), (333, 1280, 32)])
+@pytest.mark.parametrize("b,s,r", [(1, 64, 40), (3, 52, 17), (7, 256, 512), (70, 136, 200), (200, 256, 384), (300, 512, 2048), (200, 512, 8), (333, 1024, 24), (1030, 2048, 32), (2048, 1024, 8192)])
 def test_bf16_products(b, s, r):
     import torch
     from glinthawk_amd import ops
@@ -72,6 +71,12 @@ def test_bf16_products(b, s, r):
     got = ops.matmul(x, w).float()
     assert (got - want).abs().max() <= 2 ** -8 * want.abs().max() + 1e-6
     assert (ops.matmul_scaled(x, w, 0.5) - 0.5 * want).abs().max() <= 1e-5 * want.abs().max()
+
+
+# K ranges that leave a wave of the few weight rows' kernel one piece of 64, three and five
+@pytest.mark.parametrize("b,s,r", [(200, 256, 8), (225, 768, 17), (333, 1280, 32)])
+def test_bf16_products_of_few_weight_rows(b, s, r):
+    test_bf16_products(b, s, r)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -251,9 +256,8 @@ def test_decode_of_heads_with_keys_of_their_own(heads, dim, vdim, rows, keys, sh
 
 # of a wave's 32 columns and 64 keys at a time: (heads, kv heads, head sizes), (window, kept tokens, distances, scale), (starts, tokens).  Tables of one
 # distance, of fewer than a tile, with room for the entries around it and without, and none; windows that end inside a wave, kept tokens that reach into
-# it; first positions on both sides of a tile's edge, portions past the last full wave; keys that are values too, of a size with an odd number of blocks; 33 heads:
-# two groups of work-groups an XCD, the second one smaller, of which some have no head
-@pytest.mark.parametrize("heads,kv,dim,vdim,shared", [(4, 4, 128, 128, False), (8, 2, 72, 40, False), (6, 2, 128, 64, False), (2, 2, 96, 96, True), (4, 4, 128, 128, True), (33, 33, 64, 64, False)])
+# it; first positions on both sides of a tile's edge, portions past the last full wave; keys that are values too, of a size with an odd number of blocks
+@pytest.mark.parametrize("heads,kv,dim,vdim,shared", [(4, 4, 128, 128, False), (8, 2, 72, 40, False), (6, 2, 128, 64, False), (2, 2, 96, 96, True), (4, 4, 128, 128, True)])
 @pytest.mark.parametrize("window,keep,n_dist,scale", [(0, 0, 0, 1.0), (0, 0, 0, -1.0), (97, 5, 1, 1.0), (64, 70, 17, 1.0), (150, 200, 90, -1.0), (300, 3, 2000, 1.0), (31, 64, 7900, 1.0)])
 @pytest.mark.parametrize("starts,T", [([0, 64], 16), ([1, 257], 131), ([95, 0], 290)])
 def test_tiles_of_keys_by_waves(heads, kv, dim, vdim, shared, window, keep, n_dist, scale, starts, T):
@@ -287,6 +291,13 @@ def test_tiles_of_keys_by_waves(heads, kv, dim, vdim, shared, window, keep, n_di
         weight = score.masked_fill(hidden, -float("inf")).softmax(-1)
         want = torch.stack([weight[h] @ v[:, h] for h in range(heads)], 1)
         assert ((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -17 * v.abs().max() + 2e-5).all(), start
+
+
+# two groups of work-groups an XCD, the second one smaller, of which some have no head
+@pytest.mark.parametrize("window,keep,n_dist,scale", [(0, 0, 0, 1.0), (0, 0, 0, -1.0), (97, 5, 1, 1.0), (64, 70, 17, 1.0), (150, 200, 90, -1.0), (300, 3, 2000, 1.0), (31, 64, 7900, 1.0)])
+@pytest.mark.parametrize("starts,T", [([0, 64], 16), ([1, 257], 131), ([95, 0], 290)])
+def test_tiles_of_keys_of_many_heads(window, keep, n_dist, scale, starts, T):
+    test_tiles_of_keys_by_waves(33, 33, 64, 64, False, window, keep, n_dist, scale, starts, T)
 
 
 class Cache:
@@ -476,10 +487,9 @@ def test_query_key_norm_and_append(dtype, n_tokens):
         assert (c == 7.0).all(), "rows outside the call were written"
 
 
-# padded heads, more heads than keys have, a row that ends inside a group; long rows of many tokens, which work-groups take in turn, some one less
+# work-groups that take several tokens each, some one less; 16 bytes and 8 at a time, padded heads, more heads than keys have, a row that ends inside a group
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 521), (40, 8, 128, 64, 1111), (60, 20, 52, 36, 1301), (25, 5, 104, 72, 1201), (32, 32, 128, 128, 1100),
-                                                    (64, 16, 128, 40, 1301)])
+@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 521), (40, 8, 128, 64, 1111), (60, 20, 52, 36, 1301), (25, 5, 104, 72, 1201)])
 def test_query_key_norm_and_append_of_many_tokens(dtype, heads, kv, d, dv, n_tokens):
     """Three contexts, the second without one: its tokens are passed over.  Against 64 bits, bound as above."""
     import torch
@@ -517,6 +527,13 @@ def test_query_key_norm_and_append_of_many_tokens(dtype, heads, kv, d, dv, n_tok
         close(mine[:, :kp], unit(y[at, nq:nq + nk], kn), d, "k")
         close(mine[:, kp:], y[at, nq + nk:], dv, "v")
         assert (region[:start[i]] == 7.0).all() and (region[start[i] + n_tokens:] == 7.0).all(), "rows outside the call were written"
+
+
+# long rows of many tokens, which work-groups take in turn, some one less
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,kv,d,dv,n_tokens", [(32, 32, 128, 128, 1100), (64, 16, 128, 40, 1301)])
+def test_query_key_norm_and_append_of_long_rows(dtype, heads, kv, d, dv, n_tokens):
+    test_query_key_norm_and_append_of_many_tokens(dtype, heads, kv, d, dv, n_tokens)
 
 
 MLSTMS = {"small": (3, 12, 20, 9.0), "round": (2, 64, 64, 15.0), "tall": (1, 130, 40, 5.0), "broad": (2, 32, 200, 15.0), "big": (1, 256, 136, 15.0), "huge": (1, 300, 70, 15.0)}

@@ -307,8 +307,8 @@ def test_matmul_gate_of_whole_tiles(b, s, hidden, bias, activation):
                                                 (torch.bfloat16, ops.GH_ACT_GELU_TANH, False)])
 def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
     """Factors that are one weight each, so that the sums are exact: over the range of the exponential, signed zeros, the type's smallest and largest,
-    infinities and NaN, against 64 bits.  One rounding to the type, and the exponent's own, 2^-23 of its 127 at most; from factors of -128 ln 2 on, where the divisor
-    overflows, and below f16's smallest nothing is asked but the size."""
+    infinities and NaN, against 64 bits.  One rounding to the type, and the exponent's own, 2^-23 of its 127 at most; below 2^-119 (f16: its smallest) nothing is asked
+    but the size: from a divisor of 2^126 on, at factors of -87.3 and less, the reciprocal may be 0, and the quotient is at most 88.8 * 2^-126."""
     lim = torch.finfo(dt)
     a = torch.cat([torch.linspace(-130.0, 130.0, 521), torch.tensor([0.0, -0.0, lim.tiny, -lim.tiny, lim.max, lim.min, float("inf"), -float("inf"), float("nan")]),
                    torch.logspace(-6, 4, 101), -torch.logspace(-6, 4, 101)]).to(dt).cuda()
@@ -335,8 +335,28 @@ def test_gate_of_large_and_small_factors(dt, activation, bias, b, hidden):
         assert torch.equal(row.isnan(), exact.isnan())
         assert torch.equal(row[exact.isinf()], exact[exact.isinf()])
         eps = (2.0 ** -11 if dt == torch.float16 else 2.0 ** -8) + 127 * 2.0 ** -23 + (3 * 2.0 ** -23 * z.abs().clamp(max=130.0))
-        small = lim.tiny * 2.0 ** -10 if dt == torch.float16 else 128 * 0.6932 * 2.0 ** -128
+        small = lim.tiny * 2.0 ** -10 if dt == torch.float16 else 2.0 ** -119
         assert ((row - exact).abs() <= eps * exact.abs() + small)[finite].all()
+
+
+# whole tiles and a ragged last one; the ring kernel
+@pytest.mark.parametrize("b,hidden,kernel", [(512, 16384, 4), (500, 16280, 4), (16, 16384, 5)])
+def test_gate_of_vanishing_factors(b, hidden, kernel):
+    """bf16, factors between -128 ln 2, where the divisor overflows, and -126 ln 2, from where on it has no normal reciprocal: against 64 bits, one rounding to the type
+    and the exponent's own."""
+    w, x = torch.zeros((2 * hidden, 128), device="cuda", dtype=torch.bfloat16), torch.zeros((b, 128), device="cuda", dtype=torch.bfloat16)
+    y, f = torch.tensor([-87.0, -87.5, -88.0, -88.5], device="cuda"), torch.tensor([1.0, -0.75, 4.0], device="cuda")
+    n = torch.arange(hidden, device="cuda")
+    w[:hidden, 0], w[hidden:, 0], x[:, 0] = y[n % 4].bfloat16(), f[n // 4 % 3].bfloat16(), 1.0
+    lib = _lib.lib()
+    _lib.check(lib.gh_gemm_set_tuning(kernel, 0, 0))
+    try:
+        got = ops.matmul_gate(x, w, None, ops.GH_ACT_SILU).double()
+    finally:
+        _lib.check(lib.gh_gemm_set_tuning(0, 0, 0))
+    y, f = w[:hidden, 0].double(), w[hidden:, 0].double()
+    want = y / (1.0 + torch.exp(-y)) * f
+    assert ((got - want).abs() <= (2.0 ** -8 + 2.0 ** -14) * want.abs()).all()
 
 
 @pytest.mark.parametrize("b,hidden", [(512, 16384), (500, 16280)])
