@@ -317,8 +317,9 @@ class Stage:
 
 class _PinnedResults:
     """Up to `count` page-locked buffers that result arrays of a stage are laid over; a buffer comes back when its array and every view of it are gone, and
-    all of them are released with the stage and the last array.  A copy from the device into pageable memory goes through a staging buffer and the
-    host's own copy (32 x 4096 logits 40 us, 20 into such a buffer, which a kernel writes)."""
+    is released then where the stage is closed, which releases the others (35 us each: not when a caller drops the last array, but for that array's own).
+    A copy from the device into pageable memory goes through a staging buffer and the host's own copy (32 x 4096 logits 40 us, 20 into such a buffer,
+    which a kernel writes)."""
 
     class _Loan:
         def __init__(self, pool, ptr, shape):
@@ -326,19 +327,29 @@ class _PinnedResults:
             self.__array_interface__ = dict(shape=shape, typestr="<f4", data=(ptr, False), strides=None, version=3)
 
         def __del__(self):
-            self.pool.free.append(self.ptr)
+            if self.pool.closed:
+                self.pool.release(self.ptr)
+            else:
+                self.pool.free.append(self.ptr)
 
     def __init__(self, n_bytes: int, count: int):
         from . import _lib
-        self.free, self.n_bytes, self._release = [], n_bytes, _lib.lib().gh_host_free
+        self.free, self.n_bytes, self.release, self.closed = [], n_bytes, _lib.lib().gh_host_free, False
         for _ in range(count):
             ptr = C.c_void_p()
             if _lib.lib().gh_host_malloc(C.byref(ptr), n_bytes) == 0 and ptr.value:
                 self.free.append(ptr.value)
 
-    def __del__(self):
-        for ptr in self.free:
-            self._release(C.c_void_p(ptr))
+    def close(self) -> None:
+        self.closed = True
+        while self.free:
+            try:
+                self.release(self.free.pop())
+            except IndexError:     # (taken by another thread)
+                break
+
+    def __del__(self):     # (also when the interpreter ends, where this module's names may be gone)
+        self.close()
 
     def take(self, rows: int, columns: int) -> Optional[np.ndarray]:
         """(rows, columns) fp32, or None: too large, or every buffer is in use."""
@@ -369,6 +380,11 @@ class DesignStage(Stage):
         # the logits of a step and those of the one before, where they are not so many that page-locking them would tell
         step = 4 * concurrency * self.vocab_size
         self._results = _PinnedResults(step, 2 if step <= 32 << 20 else 0)
+
+    def close(self) -> None:
+        if getattr(self, "_results", None) is not None:
+            self._results.close()
+        super().close()
 
     def prefill_logits(self, context_ids, start_pos, token_ids, want=(), want_next_tokens: bool = False, residual_width: int = 0):
         """token_ids (batch, n_tokens).  Returns (logits (len(want), vocab), next tokens or None, residual stream (layer runs, rows,
