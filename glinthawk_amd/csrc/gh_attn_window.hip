@@ -213,7 +213,7 @@ __global__ __launch_bounds__( 1024 ) void window_append_row_kernel( E* __restric
 
 // Many tokens of long rows, bf16 in one plane: 16 bytes a lane, 4 V columns a group, and a work-group keeps the tables in registers over its tokens, every gridDim.x-th,
 // and asks for the next token's columns before it reduces this one's, so that reads pass while stores do.  Bound by memory: 403 MB at 8192 tokens of 3 x 4096 columns,
-// 112 us with a work-group for each, 84 so (4.8 TB/s; 82 without the sums' way through LDS, which keeps the order and so the bits of that kernel); 8 bytes a lane and
+// 112 us with a work-group for each, 84 so (4.8 TB/s; 87 in a prefill; 82 without the sums' way through LDS, which keeps the order and so the bits of that kernel); 8 bytes a lane and
 // tokens in turn 101.
 __global__ __launch_bounds__( 1024 ) __attribute__( ( amdgpu_waves_per_eu( 6, 8 ) ) ) void window_append_rows_kernel( __bf16* __restrict__ q_out, ProductView<__bf16> y, const __bf16* __restrict__ bias,
                                                                     AppendPart pq, AppendPart pk, AppendPart pv, WindowRows wr, WindowShape s, float eps, uint32_t rows )
@@ -696,7 +696,7 @@ __global__ __launch_bounds__( 256 ) void window_merge_kernel( WindowOut<E> out, 
 //             saves 32 of a tile's instructions and no time (8 x 1024 tokens 166 us against 165), and bits differ from one form of tile to the other.
 // bound       vector and matrix work of two waves a SIMD, which overlap little.  8 x 1024 tokens, 32 heads of 128, window 1024, 512 distances:
 //             221 us -> 200 with fewer vector instructions (702 -> 540 a tile and wave) -> 161 with the order; 4 x 2048 tokens without a
-//             bias: 309 -> 239, keys as values 293 -> 222 (calls in a row, their keys in the Infinity Cache).  The products run at 0.9 PFLOP/s there, both terms counted.
+//             bias: 309 -> 239, keys as values 293 -> 222 (calls in a row, their keys in the Infinity Cache; in prefills 182 and, keys as values, 270).  The products run at 0.9 PFLOP/s there, both terms counted.
 //             Other priorities for the waves in their products: no change.
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LAZY = 8.0f; // the reference point of a column's exponentials moves when its maximum has grown by 2^LAZY

@@ -87,9 +87,9 @@ __device__ __forceinline__ bool tile_of_index( const TileOrder& ord, uint32_t xc
 // again (13B, 16384 tokens: 271 us a layer; the pass of four 36.9 -> 35.5 ms).  With one work-group per CU nothing hides the epilogue, so a
 // gate that takes longer is a variant of its own, bf16: the tanh gate, and biases, kept in LDS since the tile before (8192 rows, 2 x 11008 of
 // 4096 k: 1083 us as a rounded product and a kernel behind it, 984 so; 1024 rows of 2 x 2816 of 1024 k 33.8 and 26.1).
-// The gate's epilogue is 1475 vector instructions a wave with the general division and every factor also rounded for the case that it counts, 738 as it is (bf16;
-// f16, which rounds the factors, 1410 and 933): some 3 of a 64-step tile's 95 us, of which the power budget takes back a part (4 x 2048 tokens of the design whose gate
-// is half of its time 4851 -> 4799 us, 26 x 128 of 70B 17.55 -> 17.47 ms).
+// The gate's epilogue is 1475 vector instructions a wave with the general division and every factor also rounded for the case that it counts, 866 as it is (bf16;
+// f16, which rounds the factors, 1410 and 1061): some 3 of a 64-step tile's 95 us, of which the power budget takes back a part (4 x 2048 tokens of the design whose gate
+// is half of its time 4851 -> 4799 us, 26 x 128 of 70B 17.55 -> 17.47 ms, both with two instructions an output fewer, whose gates of factors below -87.3 were 0).
 // Or q, k and v as QkvRows says, 16-byte pieces of a token's heads to its query and its cache row: the two kernels that read the product again, append and
 // rotate took 260 us a layer at 13B and 16384 tokens (3 x 5120 rows of 5120), this epilogue 55 of the product's 1785 (1730 with plain stores).
 constexpr int EPI_STORE = 0, EPI_ACCUM = 1, EPI_GATE = 2, EPI_PARTIAL = 3, EPI_QKV = 4, EPI_BIAS_GATE = 5;

@@ -281,7 +281,7 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
 // order       of the sums: terms of 16 keys or dims at a time, the lower term first, as v_mfma_f32_32x32x16_bf16 takes them (eight of a lane, lanes 0 .. 31 in
 //             front).  v_mfma_f32_16x16x32_bf16 is two of those in turn, bit for bit, so its lanes 32 .. 63 hold the next term of the same 16, or the first of the
 //             next, instead of 16 others: permlane32_swap brings a lane's terms there.  Models depend on the last bits (behind a thousand tokens and two
-//             layers they are more than a tenth of the logits of one token in 5000, in either order as far off 64 bits), so the order is kept whatever the tile.
+//             layers they are more than a tenth of the logits of 3 tokens in 960, in either order as far off 64 bits), so the order is kept whatever the tile.
 // operands    an accumulator tile of v_mfma_f32_16x16x32_bf16 (lane = column, registers = rows 4 (lane / 16) + v) is, with the tile of the next quads,
 //             an operand of the next product over those rows when the other operand takes its rows in the same order:
 //               scores^T = K Q^T        lane = query, registers = keys   -> left operand of   P V     (V out of LDS transposed)
@@ -290,8 +290,8 @@ __global__ __launch_bounds__( 256 ) void mlstm_walk_kernel( float* __restrict__ 
 // LDS         64 rows each of q, k and v, 16-byte chunks XORed with bits of the row so that row reads (16 rows) and transposing reads (8 rows, two chunks
 //             each) both touch every bank once; straight from memory (buffer_load ... lds; rows past the sequence and padding read as zero).
 // bound       8 contexts of 1024 tokens, 8 heads of 256 x 512: 310 us in one kernel, whose waves, one a SIMD, made gates, weights and n once for every 32
-//             columns; now scan 11, scores 15 and states 164 us (the call 391 -> 293; 1 of 2048 tokens 528 -> 230, 32 of 24 tokens 117 -> 83).  States: waits of
-//             four waves for each other, twice a chunk, and for LDS, 330 reads a chunk and wave, with two waves a SIMD; the matrix cores are busy for a quarter of it.
+//             columns; now, in a prefill, scan 10, scores 24 and states 162 us (calls in a row 391 -> 293, with scores of 15, whose q and k the last call left in
+//             the caches; 1 of 2048 tokens 528 -> 230, 32 of 24 tokens 117 -> 83).  States: waits of four waves for each other, twice a chunk, and for LDS, 330 reads a chunk and wave, with two waves a SIMD; the matrix cores are busy for a quarter of it.
 //             With 32 keys or dims of one term in a product, whose bits differ: 200 reads fewer and 129 us.  A third operand of k out of LDS instead of one
 //             selected from two: 235 us at 1 x 2048 tokens instead of 230, 8 x 1024 even.
 constexpr int CHUNK = 64;
