@@ -1086,7 +1086,7 @@ int gh_mlstm_forward( void* out, const void* x, const void* w, uint64_t width, c
   const uint64_t o_bytes = ( rows * hv * sizeof( float ) + 255 ) / 256 * 256;
   const uint64_t nm_bytes = ( batch * s.heads * ( s.dim + 1ull ) * sizeof( float ) + 255 ) / 256 * 256;
   const uint64_t n_pairs = batch * s.heads, n_chunks = ( (uint64_t)n_tokens + CHUNK - 1 ) / CHUNK, all_chunks = chunked ? n_pairs * n_chunks : 0;
-  const uint64_t weight_bytes = all_chunks * WEIGHT_TILES * 128 * sizeof( uint4 ), token_bytes = MlstmChunks::PLANES * all_chunks * CHUNK * sizeof( float );
+  const uint64_t weight_bytes = all_chunks * WEIGHT_TILES * 64 * sizeof( uint4 ), token_bytes = MlstmChunks::PLANES * all_chunks * CHUNK * sizeof( float );
   // chunks: 12 KB and a head's n, whatever the size of its values (a tenth of the call's workspace at 512 columns of v, two fifths at 64)
   const uint64_t more = chunked ? weight_bytes + token_bytes + all_chunks * ( s.dim + 1ull ) * sizeof( float ) : rows * 2 * s.heads * sizeof( float );
   if ( int rc = stream_scratch( st, SCRATCH_MIXER, o_bytes + nm_bytes + more, 1ull << 20, &scratch ) ) {
